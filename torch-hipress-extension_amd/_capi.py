@@ -4,6 +4,8 @@ The library is the product: if it has not been built this module raises, it
 never falls back to another implementation.
 """
 import ctypes as C
+import glob
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -128,6 +130,17 @@ def load():
         getattr(L, name)  # AttributeError if the build lost an entry point
     _lib = L
     return L
+
+
+def load_extension(name):
+    """A torch extension built into ext/ (csrc/Makefile), imported from there; raises if it is missing."""
+    found = glob.glob(os.path.join(_HERE, "ext", name + ".*.so"))
+    if not found:
+        raise RuntimeError(f"ext/{name} is missing: build it first (python -c 'import __graft_entry__ as g; g.build()' or make -C csrc)")
+    spec = importlib.util.spec_from_file_location(name, found[0])
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
 
 
 def last_error():
