@@ -7,6 +7,8 @@
 // after tensor.  Here every phase is ONE launch for all tensors of a call (a
 // table of tensors in the kernel arguments, as in the TBQ and TernGrad paths):
 //
+//   pick        for samples of up to 65536: the exact threshold by one workgroup per
+//               tensor (which gathers small samples itself), in place of select
 //   sample      |G[i]+R[i]| at the reference's LCG index stream, gathered
 //               BEFORE the update (the same fp32 sum the update will store)
 //   select      exact k-th largest of the sample by three radix-histogram
@@ -29,7 +31,10 @@
 // radix sort by |r| (ties keep ascending index) over as many byte digits as the
 // largest key has, whose last pass writes the message.  The expand launch has
 // by then left the candidates and their keys where the sort wants them.
+#include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <unordered_map>
 #include <vector>
 
 #include <immintrin.h>
@@ -54,13 +59,17 @@ struct GdState {
   uint32_t hits;      // provisional path: samples found above the provisional threshold so far
   uint32_t thr_bits;  // threshold as fp32 bits (provisional path: the provisional one until the exact one is known)
   uint32_t fallback;  // provisional path: 1 when the provisional threshold turned out to lie above the exact one
-  uint32_t pad[61];
+  uint32_t total;     // candidates, left by the expand launch for the cut launch
+  uint32_t pad[60];
 };
 constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold
 constexpr uint32_t kPreSamples = 16384;  // samples the provisional threshold is taken from
 constexpr uint32_t kFallback = 0xFFFFFFFEu;  // reported in place of a count: this tensor has to take the other path
 constexpr int kScanChunk = 4096;   // per-tile counts scanned by one workgroup
 constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
+constexpr uint32_t kPickGather = 3072;   // a sample up to this size is gathered by the one workgroup that takes its threshold
+constexpr uint32_t kPickMax = 65536;     // ... and up to this size its threshold is taken by one workgroup
+constexpr uint32_t kCutLds = 8192;       // candidates one workgroup sorts and cuts in LDS
 
 __host__ __device__ constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 __host__ __device__ constexpr uint32_t cdiv(uint64_t a, uint64_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
@@ -270,7 +279,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_select_kernel(const GdArgs<CAP
 // One workgroup per tensor.
 template <int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<CAP> a) {
-  const GdSeg& sg = a.seg[blockIdx.x];
+  const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   const uint32_t* hist = reinterpret_cast<const uint32_t*>(sg.ws + l.hist);
   uint32_t d1, d2, d3, rank;
@@ -315,6 +324,138 @@ __device__ __forceinline__ uint32_t select_rank(const uint32_t* __restrict__ key
     prefix = pass == 1 ? d : pass == 2 ? ((prefix << 11) | d) : ((prefix << 10) | d);
   }
   return prefix;
+}
+
+// The largest t whose bits below LO are zero and which more than `rank` of the wave's keys (R per lane) reach: with
+// LO = 0 the key of that rank (0-based from the top), else a lower bound of it.  Keys are bit patterns of
+// non-negative floats.  One wave, no barrier: a bit costs R compares and R counts on the scalar unit.
+template <int R, int LO>
+__device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t rank) {
+  uint32_t t = 0;
+#pragma unroll 1
+  for (int b = 30; b >= LO; b--) {
+    const uint32_t c = t | (1u << b);
+    uint32_t reach = 0;
+#pragma unroll
+    for (int j = 0; j < R; j++) reach += uint32_t(__popcll(__ballot(key[j] >= c)));
+    if (reach > rank) t = c;
+  }
+  return t;
+}
+
+// The threshold of a tensor whose sample has at most kPickMax entries, by ONE workgroup in one launch; up to kPickGather
+// of them it gathers itself (two lines per sample, about 1 us per 1000 samples; beyond that one CU's gathers take longer
+// than the extra launch that spreads them over the chip).  The rank wanted is low, a thousandth of the sample, so
+// no histogram of the whole sample is needed: of the lanes' largest keys the one of that rank, cut off below its top
+// bits, is a lower bound of the threshold that hardly more keys reach than have to; those are listed in LDS and
+// one wave finds the exact one among them, bit by bit.  Where the bound does not help (a rank beyond the lanes, a
+// list that overflows: many equal keys) the workgroup takes the three histogram passes instead.
+// Replaces three histogram launches and a rank search: 1 M elements 15 us in four launches -> 8.4 us in one; ResNet-50's
+// 161 tensors 20 -> 19.8 us, and 6 us less in the gather launch before it.
+constexpr uint32_t kPickList = 1024;
+template <int CAP>
+__global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> a) {
+  __shared__ uint32_t s_hist[kBins1];              // the lanes' largest keys; the histogram of the other way
+  __shared__ __align__(16) uint32_t s_list[kPickList];
+  __shared__ uint32_t s_n, s_key;
+  const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
+  const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
+  uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
+  const uint32_t count = sg.sample_cnt, t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  constexpr int kOwn = int(kPickGather) / kSelThreads;
+  uint32_t own[kOwn] = {};   // this lane's keys where they are gathered here
+  uint32_t big = 0;
+  if (count <= kPickGather) {
+    float gv[kOwn], rv[kOwn];
+#pragma unroll
+    for (int j = 0; j < kOwn; j++) {
+      const uint32_t x = uint32_t(j) * kSelThreads + t;
+      const uint32_t i = x < count ? sample_index(sg.seed, x, sg.n) : 0u;
+      gv[j] = x < count ? sg.g[i] : 0.0f;
+      rv[j] = x < count && a.residual ? sg.r[i] : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < kOwn; j++) {
+      const uint32_t x = uint32_t(j) * kSelThreads + t;
+      own[j] = __float_as_uint(__builtin_fabsf(a.residual ? gv[j] + rv[j] : gv[j]));
+      if (x < count) samples[x] = own[j];
+      big = own[j] > big ? own[j] : big;
+    }
+  } else {
+    for (uint32_t x = t; x < count; x += 8 * kSelThreads) {
+      uint32_t k[8];
+#pragma unroll
+      for (uint32_t j = 0; j < 8; j++) k[j] = x + j * kSelThreads < count ? samples[x + j * kSelThreads] : 0u;
+#pragma unroll
+      for (uint32_t j = 0; j < 8; j++) big = k[j] > big ? k[j] : big;
+    }
+  }
+  s_hist[t] = big;
+  if (t == 0) s_n = 0;
+  __syncthreads();
+  if (wave == 0) {
+    uint32_t k[kSelThreads / kWave];
+#pragma unroll
+    for (uint32_t j = 0; j < kSelThreads / kWave; j++) k[j] = s_hist[j * kWave + lane];
+    // with one key per lane at most, the lanes' keys are the sample
+    const uint32_t b = count <= uint32_t(kSelThreads) ? wave_rank<kSelThreads / kWave, 0>(k, sg.thr_index)
+                                                      : wave_rank<kSelThreads / kWave, 19>(k, sg.thr_index);
+    if (lane == 0) s_key = b;
+  }
+  __syncthreads();
+  const uint32_t bound = s_key;
+  if (count <= uint32_t(kSelThreads)) {
+    if (t == 0) seg_state(sg)->thr_bits = bound;
+    return;
+  }
+  bool listed = sg.thr_index < uint32_t(kSelThreads) && bound != 0u;   // workgroup-uniform
+  if (listed) {
+    auto append = [&](uint32_t key, bool live) {
+      const bool in = live && key >= bound;
+      const uint64_t m = __ballot(in);
+      if (m == 0) return;
+      uint32_t base = 0;
+      if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(&s_n, uint32_t(__popcll(m)));
+      base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+      if (in && base < kPickList) s_list[base] = key;
+    };
+    if (count <= kPickGather) {
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) append(own[j], uint32_t(j) * kSelThreads + t < count);
+    } else {
+      for (uint32_t x = t; x - t < count; x += 8 * kSelThreads) {
+        uint32_t k[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) k[j] = x + j * kSelThreads < count ? samples[x + j * kSelThreads] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) append(k[j], x + j * kSelThreads < count);
+      }
+    }
+    __syncthreads();
+    const uint32_t n = s_n;
+    listed = n <= kPickList;
+    if (listed) {
+      if (wave == 0) {
+        uint32_t key;
+        if (n <= 256) {
+          uint32_t k[4];
+#pragma unroll
+          for (uint32_t j = 0; j < 4; j++) k[j] = j * kWave + lane < n ? s_list[j * kWave + lane] : 0u;
+          key = wave_rank<4, 0>(k, sg.thr_index);
+        } else {
+          uint32_t k[kPickList / kWave];
+#pragma unroll
+          for (uint32_t j = 0; j < kPickList / kWave; j++) k[j] = j * kWave + lane < n ? s_list[j * kWave + lane] : 0u;
+          key = wave_rank<kPickList / kWave, 0>(k, sg.thr_index);
+        }
+        if (lane == 0) seg_state(sg)->thr_bits = key;
+      }
+      return;
+    }
+  }
+  __syncthreads();
+  const uint32_t key = select_rank(samples, count, sg.thr_index, s_hist);
+  if (t == 0) seg_state(sg)->thr_bits = key;
 }
 
 // The first kPreSamples samples, one per lane over many workgroups (one workgroup's gathers into arrays of
@@ -611,6 +752,10 @@ __global__ __launch_bounds__(kSelThreads) void gd_scan_kernel(const GdArgs<CAP> 
   }
 }
 
+// Tensors of at most kScanChunk tiles (16.7 M elements) take no part in the scan launch: the expand launch's
+// workgroups add up the counts before their tiles for themselves (at most 16 KB out of the L2), which saves
+// a launch of 3-5 us.
+//
 // Turns the per-tile bit masks into the ascending index list, kExpandTiles consecutive tiles
 // per wave (their mask words, and then the values of their first candidates, are loaded
 // together: a wave with one tile spent its time waiting for one load after the other, and
@@ -650,18 +795,90 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
 #pragma unroll
   for (int j = 0; j < kExpandTiles; j++) m[j] = tile0 + j < ntiles ? masks[size_t(tile0 + j) * kWave + lane] : 0ull;
 
-  // chunk totals, two per lane: inclusive prefix over the lanes
-  const uint32_t a0 = 2 * lane < nchunks ? chunk_tot[2 * lane] : 0u, a1 = 2 * lane + 1 < nchunks ? chunk_tot[2 * lane + 1] : 0u;
-  uint32_t inc2 = a0 + a1;
+  __shared__ uint32_t s_sum[3][kThreads / kWave];
+  uint32_t total, mm = 0;      // the tensor's candidates; its largest |r| (only the wave that reports needs it)
+  uint32_t ex0 = 0, ex1 = 0;   // scanned tensors: exclusive prefixes of chunks 2 * lane and 2 * lane + 1
+  uint32_t own_off = 0;        // the others: lane j's tile tile0 + j starts here
+  const bool scanned = nchunks > 1;
+  if (scanned) {
+    // chunk totals, two per lane: inclusive prefix over the lanes
+    const uint32_t* __restrict__ chunk_max = reinterpret_cast<const uint32_t*>(sg.ws + l.cmax);
+    const uint32_t a0 = 2 * lane < nchunks ? chunk_tot[2 * lane] : 0u, a1 = 2 * lane + 1 < nchunks ? chunk_tot[2 * lane + 1] : 0u;
+    uint32_t inc2 = a0 + a1;
 #pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t v = __shfl_up(inc2, o, kWave);
-    if (lane >= uint32_t(o)) inc2 += v;
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t v = __shfl_up(inc2, o, kWave);
+      if (lane >= uint32_t(o)) inc2 += v;
+    }
+    total = __builtin_amdgcn_readlane(inc2, kWave - 1);
+    ex0 = inc2 - a0 - a1;
+    ex1 = ex0 + a0;
+    if (tile0 == 0) {
+      const uint32_t m0 = 2 * lane < nchunks ? chunk_max[2 * lane] : 0u, m1 = 2 * lane + 1 < nchunks ? chunk_max[2 * lane + 1] : 0u;
+      mm = m0 > m1 ? m0 : m1;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(mm, o, kWave); mm = v > mm ? v : mm; }
+    }
+  } else {
+    // The counts of all tiles, four per lane and load (the array's padding may be read, not used): the total, and
+    // what lies before this workgroup's first tile.
+    const uint32_t first = uint32_t(blk - a.tile_start[s]) * kExpandPerBlock;
+    const uint4* __restrict__ cnt4 = reinterpret_cast<const uint4*>(sg.ws + l.cnt);
+    const uint4* __restrict__ mx4 = reinterpret_cast<const uint4*>(sg.ws + l.mx);
+    constexpr uint32_t kSteps = kScanChunk / (4 * kThreads);
+    uint4 c[kSteps], big[kSteps];
+#pragma unroll
+    for (uint32_t q = 0; q < kSteps; q++) {
+      const uint32_t i = q * kThreads + threadIdx.x;
+      const bool any = 4 * i < ntiles;
+      c[q] = any ? cnt4[i] : make_uint4(0, 0, 0, 0);
+      big[q] = any && first == 0 ? mx4[i] : make_uint4(0, 0, 0, 0);
+    }
+    const uint32_t j = tile0 + lane;
+    const uint32_t mine = lane < uint32_t(kExpandTiles) && j < ntiles ? reinterpret_cast<const uint32_t*>(cnt4)[j] : 0u;
+    uint32_t all = 0, before = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kSteps; q++) {
+      const uint32_t i = 4 * (q * kThreads + threadIdx.x);
+      const uint32_t v[4] = {c[q].x, c[q].y, c[q].z, c[q].w}, b[4] = {big[q].x, big[q].y, big[q].z, big[q].w};
+#pragma unroll
+      for (uint32_t k = 0; k < 4; k++) {
+        const uint32_t x = i + k < ntiles ? v[k] : 0u, y = i + k < ntiles ? b[k] : 0u;
+        all += x;
+        before += i + k < first ? x : 0u;
+        mm = y > mm ? y : mm;
+      }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      all += __shfl_xor(all, o, kWave);
+      before += __shfl_xor(before, o, kWave);
+      const uint32_t v = __shfl_xor(mm, o, kWave);
+      mm = v > mm ? v : mm;
+    }
+    uint32_t incl = mine;
+#pragma unroll
+    for (int o = 1; o < kExpandTiles; o <<= 1) {
+      const uint32_t v = __shfl_up(incl, o, kWave);
+      if (lane >= uint32_t(o)) incl += v;
+    }
+    const uint32_t own = __builtin_amdgcn_readlane(incl, kExpandTiles - 1);  // this wave's candidates
+    __shared__ uint32_t s_own[kThreads / kWave];
+    if (lane == 0) { s_sum[0][wave] = all; s_sum[1][wave] = before; s_sum[2][wave] = mm; s_own[wave] = own; }
+    __syncthreads();
+    total = 0;
+    own_off = incl - mine;
+    mm = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kThreads / kWave; w++) {
+      total += s_sum[0][w];
+      own_off += s_sum[1][w] + (w < wave ? s_own[w] : 0u);
+      mm = s_sum[2][w] > mm ? s_sum[2][w] : mm;
+    }
   }
-  const uint32_t total = __builtin_amdgcn_readlane(inc2, kWave - 1);
-  const uint32_t ex0 = inc2 - a0 - a1, ex1 = ex0 + a0;  // exclusive prefixes of chunks 2 * lane and 2 * lane + 1
   if (a.margin >= 0 && st->fallback) {
     // the provisional threshold was not below the exact one: nothing of what the masks hold may be used
+    if (tile0 == 0 && lane == 0) seg_state(sg)->total = 0;
     if (tile0 == 0 && a.report != nullptr && lane == 0) {
       uint32_t* rep = a.report + size_t(s) * kReportWords;
       __hip_atomic_store(rep + 0, kFallback, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -670,14 +887,10 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     }
     return;
   }
+  if (tile0 == 0 && lane == 0) seg_state(sg)->total = total;
   if (tile0 == 0 && a.report != nullptr) {
     // Pinned host words the host polls (no copy command, no wait for the stream).  The host waits for each
     // of the three words to change, so plain system-scope stores do (a release would write the whole L2 back).
-    const uint32_t* __restrict__ chunk_max = reinterpret_cast<const uint32_t*>(sg.ws + l.cmax);
-    const uint32_t m0 = 2 * lane < nchunks ? chunk_max[2 * lane] : 0u, m1 = 2 * lane + 1 < nchunks ? chunk_max[2 * lane + 1] : 0u;
-    uint32_t mm = m0 > m1 ? m0 : m1;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(mm, o, kWave); mm = v > mm ? v : mm; }
     if (lane == 0) {
       uint32_t* rep = a.report + size_t(s) * kReportWords;
       __hip_atomic_store(rep + 0, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -696,7 +909,8 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   for (int j = 0; j < kExpandTiles; j++) {
     const uint32_t tile = tile0 + j < ntiles ? tile0 + j : ntiles - 1;
     const uint32_t chunk = tile / kScanChunk;
-    const uint32_t coff = __shfl((chunk & 1u) ? ex1 : ex0, int(chunk >> 1), kWave);
+    const uint32_t start = scanned ? __shfl((chunk & 1u) ? ex1 : ex0, int(chunk >> 1), kWave) + tile_off[tile]
+                                   : uint32_t(__builtin_amdgcn_readlane(own_off, j));
     const uint32_t c = __popcll(m[j]);
     uint32_t incl = c;
 #pragma unroll
@@ -704,7 +918,7 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
       const uint32_t v = __shfl_up(incl, o, kWave);
       if (lane >= uint32_t(o)) incl += v;
     }
-    pos[j] = coff + tile_off[tile] + incl - c;
+    pos[j] = start + incl - c;
   }
   // The first candidate of each of the lane's 64-element groups: their values are loaded together.
   uint32_t e1[kExpandTiles];
@@ -1017,28 +1231,228 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
   }
 }
 
-// ---- decode -----------------------------------------------------------------
-// The fill of a written tensor is a pure write stream: streaming stores, three workgroups per CU (hpx_common.h;
-// 138 M elements: 119 -> 95 us for the whole call, 103 without the limit on the workgroups).
-__global__ __launch_bounds__(kThreads) void gd_zero_kernel(float* __restrict__ out, uint32_t n) {
-  const uint32_t stride = gridDim.x * kThreads * 4;
-  for (uint32_t e = (blockIdx.x * kThreads + threadIdx.x) * 4; e < n; e += stride) {
-    if (n - e >= 4) {
-      st4_stream(out + e, make_float4(0.f, 0.f, 0.f, 0.f));
-    } else {
-      for (uint32_t i = e; i < n; i++) out[i] = 0.f;
+// The cut of a tensor with at most kCutLds candidates, by one workgroup in one launch: the same stable LSD sort
+// by byte digits, pairs in registers between the passes and in LDS for the exchange, then the message.  It is
+// queued behind the expand launch before the host knows any count and leaves at once where nothing has to be cut,
+// so a call of such tensors needs no work of the host's in the middle: the seven launches of the three-pass sort and the
+// host's turn-around (45-50 us for the 161 tensors of ResNet-50) became one launch of 18 us.
+template <int CAP>
+__global__ __launch_bounds__(kSortThreads) void gd_cut_kernel(const GdArgs<CAP> a) {
+  constexpr uint32_t BINS = 256, kBinWaves = BINS / kWave;
+  constexpr int kPer = int(kCutLds) / kSortThreads;
+  extern __shared__ uint32_t s_stage[];          // [kCutLds] keys, then [kCutLds] indices
+  __shared__ uint32_t s_cnt[kSortWaves][BINS];
+  __shared__ uint32_t s_part[kBinWaves], s_max[kSortWaves];
+  uint32_t* s_key = s_stage;
+  uint32_t* s_id = s_stage + kCutLds;
+  const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
+  const uint32_t n = seg_state(sg)->total, keep = sg.limit;
+  if (n <= keep || n > sg.cap || n > kCutLds) return;
+  const CutLayout cl = cut_layout(sg.cap);
+  const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(sg.cut + cl.ka);
+  const int32_t* __restrict__ cand = reinterpret_cast<const int32_t*>(sg.cut + cl.ia);
+  const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const uint32_t per = cdiv(n, kSortThreads);    // rounds of 64 pairs per wave, the same for every wave
+  const uint32_t x0 = wave * per * kWave + lane;
+  uint32_t key[kPer], id[kPer], big = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const uint32_t x = x0 + uint32_t(j) * kWave;
+    const bool live = uint32_t(j) < per && x < n;
+    key[j] = live ? keys[x] : 0u;
+    id[j] = live ? uint32_t(cand[x]) : 0u;
+    big = key[j] > big ? key[j] : big;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(big, o, kWave); big = v > big ? v : big; }
+  if (lane == 0) s_max[wave] = big;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSortWaves; w++) big = s_max[w] > big ? s_max[w] : big;
+  const int passes = big ? (39 - __builtin_clz(big)) / 8 : 1;
+#pragma unroll 1
+  for (int pass = 0; pass < passes; pass++) {
+    const int shift = pass * 8;
+#pragma unroll
+    for (uint32_t q = 0; q < kBinWaves; q++) s_cnt[wave][q * kWave + lane] = 0;  // own row
+    uint32_t place[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+      if (uint32_t(j) < per) {
+        const bool live = x0 + uint32_t(j) * kWave < n;
+        const uint32_t bin = (BINS - 1) - ((key[j] >> shift) & (BINS - 1));
+        const uint64_t same = match_bin<8>(bin, live);
+        const uint32_t rank = uint32_t(__popcll(same & ((uint64_t(1) << lane) - 1)));
+        uint32_t base = 0;
+        if (live && rank == 0) {
+          base = s_cnt[wave][bin];
+          s_cnt[wave][bin] = base + uint32_t(__popcll(same));
+        }
+        base = __shfl(base, live ? __builtin_ctzll(same) : int(lane), kWave);
+        place[j] = base + rank;
+      }
+    }
+    __syncthreads();
+    // bin t: the tile's total, an exclusive scan of the totals, then every wave's first place
+    uint32_t c[kSortWaves], mine = 0;
+    if (t < BINS) {
+#pragma unroll
+      for (int w = 0; w < kSortWaves; w++) { c[w] = s_cnt[w][t]; mine += c[w]; }
+    }
+    uint32_t incl = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t v = __shfl_up(incl, o, kWave);
+      if (lane >= uint32_t(o)) incl += v;
+    }
+    if (t < BINS && lane == kWave - 1) s_part[wave] = incl;
+    __syncthreads();
+    if (t < BINS) {
+      uint32_t run = incl - mine;
+      for (uint32_t w = 0; w < wave; w++) run += s_part[w];
+#pragma unroll
+      for (int w = 0; w < kSortWaves; w++) { s_cnt[w][t] = run; run += c[w]; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+      if (uint32_t(j) < per && x0 + uint32_t(j) * kWave < n) {
+        const uint32_t p = s_cnt[wave][(BINS - 1) - ((key[j] >> shift) & (BINS - 1))] + place[j];
+        s_key[p] = key[j];
+        s_id[p] = id[j];
+      }
+    }
+    __syncthreads();
+    if (pass + 1 < passes) {
+#pragma unroll
+      for (int j = 0; j < kPer; j++) {
+        const uint32_t x = x0 + uint32_t(j) * kWave;
+        if (uint32_t(j) < per && x < n) { key[j] = s_key[x]; id[j] = s_id[x]; }
+      }
+    }
+  }
+  int32_t* __restrict__ idx = reinterpret_cast<int32_t*>(sg.out + 4);
+  float* __restrict__ val = reinterpret_cast<float*>(sg.out + 4 + size_t(keep) * 4);
+  float* __restrict__ r = sg.r;
+  if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + keep * 8);
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const uint32_t p = uint32_t(j) * kSortThreads + t;
+    if (p < keep) {
+      const uint32_t i = s_id[p];
+      idx[p] = int32_t(i);
+      val[p] = r[i];
+      r[i] = 0.0f;
     }
   }
 }
 
-template <bool ADD>
-__global__ __launch_bounds__(kThreads) void gd_scatter_kernel(const int32_t* __restrict__ idx, const float* __restrict__ val,
-                                                              uint32_t k, float* __restrict__ out) {
-  const uint32_t x = blockIdx.x * kThreads + threadIdx.x;
-  if (x < k) {
-    const int32_t i = idx[x];
-    if (ADD) out[i] += val[x]; else out[i] = val[x];  // gd_body.h:250, :280
+// ---- decode -----------------------------------------------------------------
+// A call's messages travel as a table in the kernel arguments.  The reference reads every header on the host before
+// it touches an output (gd_body.h:301-325).  Here the check runs on the device: a launch either checks all headers of
+// its table itself (every workgroup reads them, one per lane - a few hundred bytes out of the L2) and leaves
+// everything alone if one is bad, or has been queued after the host has seen the verdict.  The verdict is one
+// 64-bit pinned word, written as soon as the first launch runs; the host polls it.
+// Before, every header was a copy of its own and every message a launch or two: decoding 161 messages cost 600 us of
+// an encode + decode pass of 864, now one launch of 5.
+struct GdMsg {   // 32 bytes
+  const uint8_t* in;
+  float* out;
+  uint32_t out_n;
+  int32_t in_size;
+  int32_t add;
+  int32_t pad;
+};
+template <int CAP>
+struct GdDecArgs {
+  int32_t nseg;
+  int32_t check;                // 1: check the headers of this table before anything is written
+  int32_t tile_start[CAP + 1];
+  GdMsg seg[CAP];
+  unsigned long long* report;   // pinned: the verdict of this table's check goes here (null: nobody waits for it)
+};
+static_assert(sizeof(GdDecArgs<kCapLarge>) <= 18000, "kernel-argument budget");
+// verdict << 48 | first offending message << 32 | its header
+constexpr unsigned long long kVerdictGood = 1ull, kVerdictLong = 2ull, kVerdictShort = 3ull;
+
+// Whether every header of the table fits its message (the same answer in all lanes of the workgroup, all of which
+// must call).  `tell`: this workgroup reports.
+template <int CAP>
+__device__ __forceinline__ bool headers_fit(const GdDecArgs<CAP>& a, bool tell) {
+  static_assert(CAP <= kThreads, "a message per lane");
+  __shared__ uint32_t s_bad;
+  if (threadIdx.x == 0) s_bad = 0xFFFFFFFFu;
+  __syncthreads();
+  const uint32_t t = threadIdx.x;
+  int32_t M = 4, room = 4;
+  if (t < uint32_t(a.nseg)) {
+    M = *reinterpret_cast<const int32_t*>(a.seg[t].in);
+    room = a.seg[t].in_size;
+    if (room < M || M < 4) atomicMin(&s_bad, t);
   }
+  __syncthreads();
+  const uint32_t bad = s_bad;
+  if (tell && a.report != nullptr && t == (bad == 0xFFFFFFFFu ? 0u : bad)) {
+    const unsigned long long verdict = bad == 0xFFFFFFFFu ? kVerdictGood : room < M ? kVerdictLong : kVerdictShort;
+    __hip_atomic_store(a.report, verdict << 48 | (unsigned long long)(bad & 0xFFFFu) << 32 | (unsigned long long)(uint32_t(M)),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  return bad == 0xFFFFFFFFu;
+}
+
+template <int CAP>
+__global__ __launch_bounds__(kThreads) void gd_check_kernel(const GdDecArgs<CAP> a) {
+  (void)headers_fit<CAP>(a, true);
+}
+
+// The fill of a written tensor is a pure write stream: streaming stores, three workgroups per CU (hpx_common.h;
+// 138 M elements: 119 -> 95 us for the whole call, 103 without the limit on the workgroups), 4 KB per workgroup.
+constexpr uint32_t kZeroTile = kThreads * 4;
+template <int CAP>
+__global__ __launch_bounds__(kThreads) void gd_zero_kernel(const GdDecArgs<CAP> a) {
+  if (a.check && !headers_fit<CAP>(a, blockIdx.x == 0)) return;
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x);
+  float* __restrict__ out = a.seg[s].out;
+  const uint32_t n = a.seg[s].out_n;
+  const uint32_t e = uint32_t(int(blockIdx.x) - a.tile_start[s]) * kZeroTile + threadIdx.x * 4;
+  if (e >= n) return;
+  if (n - e >= 4) {
+    st4_stream(out + e, make_float4(0.f, 0.f, 0.f, 0.f));
+  } else {
+    for (uint32_t i = e; i < n; i++) out[i] = 0.f;
+  }
+}
+
+constexpr uint32_t kScatterBlocks = 4096;  // workgroups of one message at most; they stride over the rest
+template <int CAP>
+__global__ __launch_bounds__(kThreads) void gd_scatter_kernel(const GdDecArgs<CAP> a) {
+  if (a.check && !headers_fit<CAP>(a, blockIdx.x == 0)) return;
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x);
+  const uint8_t* __restrict__ in = a.seg[s].in;
+  float* __restrict__ out = a.seg[s].out;
+  const uint32_t n = a.seg[s].out_n;
+  const bool add = a.seg[s].add != 0;
+  const uint32_t k = uint32_t(*reinterpret_cast<const int32_t*>(in) - 4) / 8u;
+  const int32_t* __restrict__ idx = reinterpret_cast<const int32_t*>(in + 4);
+  const float* __restrict__ val = reinterpret_cast<const float*>(in + 4 + size_t(k) * 4);
+  const uint32_t stride = uint32_t(a.tile_start[s + 1] - a.tile_start[s]) * kThreads;
+  for (uint32_t x = uint32_t(int(blockIdx.x) - a.tile_start[s]) * kThreads + threadIdx.x; x < k; x += stride) {
+    const uint32_t i = uint32_t(idx[x]);
+    const float v = val[x];
+    if (i >= n) continue;  // not an index an encoder writes
+    if (add) out[i] += v; else out[i] = v;  // gd_body.h:250, :280
+  }
+}
+
+// The dynamic-LDS limit is a property of the function on one device: raised once per device (bit d of `done`:
+// done on device d; devices beyond 63 set it on every call).
+int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+  int dev = 0;
+  HPX_HIP(hipGetDevice(&dev));
+  if (dev < 64 && (done.load(std::memory_order_acquire) >> dev & 1)) return HPX_OK;
+  HPX_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  if (dev < 64) done.fetch_or(uint64_t(1) << dev, std::memory_order_release);
+  return HPX_OK;
 }
 
 // One tensor of the cut path as the host sees it.
@@ -1052,19 +1466,8 @@ struct CutJob {
 template <int CAP, int BITS>
 int sort_passes(SortArgs<CAP>& a, int passes, hipStream_t st) {
   constexpr int kStageBytes = 2 * kSortTile * int(sizeof(uint32_t));
-  // The dynamic-LDS limit is a property of the function on one device: raise it once per device.
-  static std::mutex attr_mu;
-  static uint64_t attr_done = 0;  // bit d: done on device d (devices beyond 63 set it on every call)
-  {
-    int dev = 0;
-    HPX_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> g(attr_mu);
-    if (dev >= 64 || !(attr_done >> dev & 1)) {
-      HPX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gd_sort_pass_kernel<CAP, BITS>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kStageBytes));
-      if (dev < 64) attr_done |= uint64_t(1) << dev;
-    }
-  }
+  static std::atomic<uint64_t> attr_done{0};
+  if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_sort_pass_kernel<CAP, BITS>), kStageBytes, attr_done)) return rc;
   const dim3 grid(uint32_t(a.tile_start[a.nseg]));
   for (int pass = 0; pass < passes; pass++) {
     a.shift = pass * BITS;
@@ -1111,8 +1514,13 @@ struct Plan {
   int index;  // position in the call
 };
 
+// Whether the device alone settles a tensor's cut (gd_cut_kernel) as long as it has `found` candidates.
+bool cut_on_device(const GdSeg& sg, uint64_t found) { return sg.limit < kCutLds && found <= sg.cap && found <= kCutLds; }
+
 // The phases for up to CAP tensors, no host wait.  margin < 0: the threshold from the full gathered sample
-// (sample, three histogram passes, rank search), then the pass, scan and expand.  margin >= 0: the provisional
+// (for samples of up to kPickMax one workgroup each, behind a gather launch where a sample exceeds kPickGather; for
+// larger ones gather, three histogram passes, rank search), then the pass, scan, expand and the cut of the tensors
+// whose candidates fit a workgroup.  A launch that no tensor of the table takes part in is left out.  margin >= 0: the provisional
 // path (above): provisional threshold, the pass, the samples against the mask, exact threshold, recount, scan, expand.
 template <int CAP>
 int launch_phases(const Plan* plans, int count, bool residual, int margin, uint32_t* report, hipStream_t st) {
@@ -1128,6 +1536,7 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     return dim3(uint32_t(a.tile_start[count]));
   };
   auto sel_blocks = [](const GdSeg& sg) {
+    if (sg.sample_cnt <= kPickMax) return 0u;
     const uint32_t b = cdiv(sg.sample_cnt, kSelThreads * 8);
     return b > uint32_t(kSelBlocksMax) ? uint32_t(kSelBlocksMax) : b;
   };
@@ -1140,13 +1549,21 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   };
   dim3 grid;
   if (margin < 0) {
-    grid = tiles([](const GdSeg& sg) { return cdiv(sg.sample_cnt > uint32_t(kHistWords) ? sg.sample_cnt : uint32_t(kHistWords), kThreads); });
-    HPX_LAUNCH("gd_sample_kernel", gd_sample_kernel<CAP>, grid, dim3(kThreads), st, a);
+    grid = tiles([](const GdSeg& sg) {
+      if (sg.sample_cnt <= kPickGather) return 0u;
+      return cdiv(sg.sample_cnt, kThreads);   // more than enough lanes to clear the histograms where they are used
+    });
+    if (grid.x) HPX_LAUNCH("gd_sample_kernel", gd_sample_kernel<CAP>, grid, dim3(kThreads), st, a);
+    grid = tiles([](const GdSeg& sg) { return sg.sample_cnt <= kPickMax ? 1u : 0u; });
+    if (grid.x) HPX_LAUNCH("gd_pick_kernel", gd_pick_kernel<CAP>, grid, dim3(kSelThreads), st, a);
     grid = tiles(sel_blocks);
-    HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<1, CAP>), grid, dim3(kSelThreads), st, a);
-    HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<2, CAP>), grid, dim3(kSelThreads), st, a);
-    HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<3, CAP>), grid, dim3(kSelThreads), st, a);
-    HPX_LAUNCH("gd_threshold_kernel", gd_threshold_kernel<CAP>, dim3(uint32_t(count)), dim3(kSelThreads), st, a);
+    if (grid.x) {
+      HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<1, CAP>), grid, dim3(kSelThreads), st, a);
+      HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<2, CAP>), grid, dim3(kSelThreads), st, a);
+      HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<3, CAP>), grid, dim3(kSelThreads), st, a);
+      grid = tiles([](const GdSeg& sg) { return sg.sample_cnt <= kPickMax ? 0u : 1u; });
+      HPX_LAUNCH("gd_threshold_kernel", gd_threshold_kernel<CAP>, grid, dim3(kSelThreads), st, a);
+    }
     stream_pass();
   } else {
     grid = tiles([](const GdSeg& sg) { return cdiv(sg.sample_cnt < kPreSamples ? sg.sample_cnt : kPreSamples, kThreads); });
@@ -1159,13 +1576,23 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kThreads / kWave); });
     HPX_LAUNCH("gd_recount_kernel", gd_recount_kernel<CAP>, grid, dim3(kThreads), st, a);
   }
-  grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kScanChunk); });
-  HPX_LAUNCH("gd_scan_kernel", gd_scan_kernel<CAP>, grid, dim3(kSelThreads), st, a);
+  grid = tiles([](const GdSeg& sg) {
+    const uint32_t chunks = cdiv(cdiv(sg.n, kTile), kScanChunk);
+    return chunks > 1 ? chunks : 0u;
+  });
+  if (grid.x) HPX_LAUNCH("gd_scan_kernel", gd_scan_kernel<CAP>, grid, dim3(kSelThreads), st, a);
   HPX_HIP(hipGetLastError());
   // Queued before the host knows the counts: the finish where nothing has to be cut,
   // else the candidate list and keys of the cut path.
   grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
   HPX_LAUNCH("gd_expand_kernel", gd_expand_kernel<CAP>, grid, dim3(kThreads), st, a);
+  grid = tiles([](const GdSeg& sg) { return sg.limit < kCutLds && sg.limit < sg.n ? 1u : 0u; });
+  if (grid.x) {
+    constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));
+    static std::atomic<uint64_t> attr_done{0};
+    if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_cut_kernel<CAP>), kStageBytes, attr_done)) return rc;
+    HPX_LAUNCH_LDS("gd_cut_kernel", hpx::g_prof_on, gd_cut_kernel<CAP>, grid, dim3(kSortThreads), kStageBytes, st, a);
+  }
   HPX_HIP(hipGetLastError());
   return HPX_OK;
 }
@@ -1192,6 +1619,24 @@ int wait_reports(volatile uint32_t* report, int count, hipStream_t st) {
           hpx::set_error("sparsifier encode: tensor %d was not reported by the scan launch", t);
           return HPX_ERR_HIP;
         }
+      }
+    }
+  }
+  __atomic_thread_fence(__ATOMIC_ACQUIRE);
+  return HPX_OK;
+}
+
+// The same for one 64-bit word that is zero until a kernel writes it.
+int wait_word(volatile unsigned long long* word, hipStream_t st) {
+  uint32_t spins = 0;
+  while (*word == 0) {
+    _mm_pause();
+    if ((++spins & 511u) == 0) {
+      const hipError_t e = hipStreamQuery(st);
+      if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+      if (e != hipSuccess || *word == 0) {
+        hpx::set_error("sparsifier decode: %s", e != hipSuccess ? hipGetErrorString(e) : "the headers were not reported");
+        return HPX_ERR_HIP;
       }
     }
   }
@@ -1270,16 +1715,20 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
       for (int w = 0; w < 3; w++) report[size_t(t) * kReportWords + w] = kNotReported;
     __atomic_thread_fence(__ATOMIC_RELEASE);
   };
+  // Tensors whose every possible count the device settles by itself: nothing to report, nothing to wait for.
+  bool unattended = margin < 0;
+  for (const Plan& p : plans) unattended = unattended && (cut_on_device(p.seg, p.seg.n) || p.seg.limit >= p.seg.n);
   for (int first = 0; first < total; first += kMaxPerWait) {
     const int batch = total - first < kMaxPerWait ? total - first : kMaxPerWait;
-    reset_reports(batch);
+    if (!unattended) reset_reports(batch);
     for (int k = 0; k < batch; k += kCapLarge) {
       const int m = batch - k < kCapLarge ? batch - k : kCapLarge;
-      uint32_t* rep = const_cast<uint32_t*>(report) + size_t(k) * kReportWords;
+      uint32_t* rep = unattended ? nullptr : const_cast<uint32_t*>(report) + size_t(k) * kReportWords;
       rc = m <= kCapSmall ? launch_phases<kCapSmall>(&plans[first + k], m, residuals != nullptr, margin, rep, st)
                           : launch_phases<kCapLarge>(&plans[first + k], m, residuals != nullptr, margin, rep, st);
       if (rc != HPX_OK) return rc;
     }
+    if (unattended) continue;
     rc = wait_reports(report, batch, st);
     if (rc != HPX_OK) return rc;
     // What the tensors reported, kept on the host: the pinned words serve again below.
@@ -1321,7 +1770,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
     for (int t = 0; t < batch; t++) {
       const GdSeg& sg = plans[first + t].seg;
       const uint32_t found = rep_host[size_t(t) * kReportWords];
-      if (found <= sg.limit) continue;
+      if (found <= sg.limit || cut_on_device(sg, found)) continue;
       const uint32_t thr_bits = rep_host[size_t(t) * kReportWords + 1], max_bits = rep_host[size_t(t) * kReportWords + 2];
       // keys are |r| bits minus threshold bits: the largest tells how many byte digits are in use
       const uint32_t max_key = max_bits > thr_bits ? max_bits - thr_bits : 0u;
@@ -1419,6 +1868,47 @@ HPX_API int64_t hpx_gd_fallbacks(hpx_stream_t stream) {
 }
 
 namespace {
+// A table of messages, none of which names another's output.
+template <int CAP>
+void decode_table(GdDecArgs<CAP>& a, const GdMsg* msgs, int count, bool check, unsigned long long* report) {
+  a.nseg = count;
+  a.check = check ? 1 : 0;
+  a.report = report;
+  for (int i = 0; i < count; i++) a.seg[i] = msgs[i];
+}
+template <int CAP>
+int launch_check(const GdMsg* msgs, int count, unsigned long long* report, hipStream_t st) {
+  GdDecArgs<CAP> a;
+  decode_table(a, msgs, count, true, report);
+  a.tile_start[0] = 0;
+  for (int i = 0; i < count; i++) a.tile_start[i + 1] = 0;
+  HPX_LAUNCH("gd_check_kernel", gd_check_kernel<CAP>, dim3(1), dim3(kThreads), st, a);
+  HPX_HIP(hipGetLastError());
+  return HPX_OK;
+}
+// The fill of the tensors that are written (zero_fill), then all values to their places.
+template <int CAP>
+int launch_decode(const GdMsg* msgs, int count, bool zero_fill, bool check, unsigned long long* report, hipStream_t st) {
+  GdDecArgs<CAP> a;
+  decode_table(a, msgs, count, check, report);
+  a.tile_start[0] = 0;
+  for (int i = 0; i < count; i++)
+    a.tile_start[i + 1] = a.tile_start[i] + (zero_fill && !msgs[i].add ? int32_t(cdiv(msgs[i].out_n, kZeroTile)) : 0);
+  if (a.tile_start[count] > 0) {
+    HPX_LAUNCH_LDS("gd_zero_kernel", hpx::g_prof_on, gd_zero_kernel<CAP>, dim3(uint32_t(a.tile_start[count])), dim3(kThreads),
+                   hpx::kWriteStreamPadLds3, st, a);
+    a.report = nullptr;  // that launch reports
+  }
+  for (int i = 0; i < count; i++) {
+    // by the room the message has: its header is on the device
+    const uint32_t most = cdiv(msgs[i].in_size > 4 ? uint32_t(msgs[i].in_size - 4) / 8u : 0u, kThreads);
+    a.tile_start[i + 1] = a.tile_start[i] + int32_t(most < 1 ? 1 : most > kScatterBlocks ? kScatterBlocks : most);
+  }
+  HPX_LAUNCH("gd_scatter_kernel", gd_scatter_kernel<CAP>, dim3(uint32_t(a.tile_start[count])), dim3(kThreads), st, a);
+  HPX_HIP(hipGetLastError());
+  return HPX_OK;
+}
+
 // gd_r_body (zero_fill: write mode clears the whole output first, gd_body.h:335-347)
 // and dgc_r_body (no clearing, dgc_body.h:283-289).
 int decode_messages(int count, const uint8_t* const* ins, const int32_t* in_sizes, float* const* outs,
@@ -1441,33 +1931,82 @@ int decode_messages(int count, const uint8_t* const* ins, const int32_t* in_size
   std::lock_guard<std::mutex> lock(ws->mu);
   int rc = hpx::ensure_workspace(ws, 0);
   if (rc != HPX_OK) return rc;
-  // headers first, one wait (gd_body.h:301-309)
-  int32_t* Ms = reinterpret_cast<int32_t*>(ws->pinned);
-  for (int i = 0; i < count; i++) HPX_HIP(hipMemcpyAsync(&Ms[i], ins[i], sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  HPX_HIP(hipStreamSynchronize(st));
-  for (int i = 0; i < count; i++) {
-    if (in_sizes[i] < Ms[i]) {  // gd_body.h:317-325
-      hpx::set_error("input space provided is not enough! in_uint8_t_size=%d\tM=%d (message %d, is_add_to %d)", in_sizes[i],
-                     Ms[i], i, is_add_tos[i]);
-      return HPX_ERR_BODY;
+
+  // Messages that name one output are applied in call order: round j takes the j-th message of every output, all of a
+  // round together; outputs that overlap otherwise take a round per message.
+  std::vector<int> order(count), round_of(count, 0);
+  for (int i = 0; i < count; i++) order[i] = i;
+  int rounds = 1;
+  if (const int cls = hpx::classify_outputs(count, outs, out_sizes)) {
+    std::unordered_map<const float*, int> seen;
+    for (int i = 0; i < count; i++) {
+      round_of[i] = cls == 1 ? seen[outs[i]]++ : i;
+      rounds = round_of[i] + 1 > rounds ? round_of[i] + 1 : rounds;
     }
-    HPX_ARG(Ms[i] >= 4, "hpx_gd_decode: message %d has header %d", i, Ms[i]);
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return round_of[x] < round_of[y]; });
   }
-  for (int i = 0; i < count; i++) {
-    const uint32_t k = static_cast<uint32_t>((Ms[i] - 4) / 8);
-    const int32_t* idx = reinterpret_cast<const int32_t*>(ins[i] + 4);
-    const float* val = reinterpret_cast<const float*>(ins[i] + 4 + size_t(k) * 4);
-    if (!is_add_tos[i]) {
-      const uint32_t n = static_cast<uint32_t>(out_sizes[i]);
-      if (n && zero_fill) {
-        uint32_t blocks = cdiv(n, kThreads * 4);
-        HPX_LAUNCH_LDS("gd_zero_kernel", hpx::g_prof_on, gd_zero_kernel, dim3(blocks), dim3(kThreads), hpx::kWriteStreamPadLds3, st, outs[i], n);
+  uint64_t zero_tiles = 0;
+  for (int i = 0; i < count; i++)
+    if (zero_fill && !is_add_tos[i]) zero_tiles += cdiv(uint32_t(out_sizes[i]), kZeroTile);
+
+  std::vector<GdMsg> msgs(count);
+  for (int i = 0; i < count; i++) msgs[i] = {ins[i], outs[i], static_cast<uint32_t>(out_sizes[i]), in_sizes[i], is_add_tos[i], 0};
+
+  volatile unsigned long long* report = reinterpret_cast<volatile unsigned long long*>(ws->pinned);
+  // One table and hardly anything to clear: everything is queued at once and checks for itself.  Else the host
+  // hears the verdict first (about 6 us): a fill of many short workgroups is slowed by reading headers in each
+  // (from about a thousand workgroups on, more than the wait costs), and several tables must all be good before any is applied.
+  const bool at_once = rounds == 1 && count <= kCapLarge && zero_tiles <= 1024;
+  const int tables = at_once ? 1 : (count + kCapLarge - 1) / kCapLarge;
+  for (int k = 0; k < tables; k++) report[k] = 0;
+  __atomic_thread_fence(__ATOMIC_RELEASE);
+  auto verdict = [&]() {
+    for (int k = 0; k < tables; k++) {
+      const int rcw = wait_word(&report[k], st);
+      if (rcw != HPX_OK) return rcw;
+      const unsigned long long w = report[k];
+      if ((w >> 48) == kVerdictGood) continue;
+      const int i = k * kCapLarge + int(w >> 32 & 0xFFFFu);
+      const int32_t M = static_cast<int32_t>(uint32_t(w));
+      if ((w >> 48) == kVerdictLong) {  // gd_body.h:317-325
+        hpx::set_error("input space provided is not enough! in_uint8_t_size=%d\tM=%d (message %d, is_add_to %d)", in_sizes[i], M, i,
+                       is_add_tos[i]);
+        return int(HPX_ERR_BODY);
       }
-      if (k) HPX_LAUNCH("gd_scatter_kernel", gd_scatter_kernel<false>, dim3(cdiv(k, kThreads)), dim3(kThreads), st, idx, val, k, outs[i]);
-    } else if (k) {
-      HPX_LAUNCH("gd_scatter_kernel", gd_scatter_kernel<true>, dim3(cdiv(k, kThreads)), dim3(kThreads), st, idx, val, k, outs[i]);
+      hpx::set_error("hpx_gd_decode: message %d has header %d", i, M);
+      return int(HPX_ERR_ARG);
     }
-    HPX_HIP(hipGetLastError());
+    return int(HPX_OK);
+  };
+  unsigned long long* word = reinterpret_cast<unsigned long long*>(ws->pinned);
+  if (at_once) {
+    rc = count <= kCapSmall ? launch_decode<kCapSmall>(msgs.data(), count, zero_fill, true, word, st)
+                            : launch_decode<kCapLarge>(msgs.data(), count, zero_fill, true, word, st);
+    return rc != HPX_OK ? rc : verdict();
+  }
+  for (int k = 0; k < count; k += kCapLarge) {
+    const int m = count - k < kCapLarge ? count - k : kCapLarge;
+    rc = m <= kCapSmall ? launch_check<kCapSmall>(&msgs[k], m, word + k / kCapLarge, st)
+                        : launch_check<kCapLarge>(&msgs[k], m, word + k / kCapLarge, st);
+    if (rc != HPX_OK) return rc;
+  }
+  rc = verdict();
+  if (rc != HPX_OK) return rc;
+  std::vector<GdMsg> sorted(count);
+  for (int i = 0; i < count; i++) sorted[i] = msgs[order[i]];
+  for (int first = 0; first < count;) {
+    // a round at most, and no more workgroups than a launch takes
+    int last = first;
+    uint64_t tiles = 0;
+    while (last < count && last - first < kCapLarge && round_of[order[last]] == round_of[order[first]]) {
+      tiles += cdiv(sorted[last].out_n, kZeroTile) + kScatterBlocks;
+      if (last > first && tiles > (1u << 23)) break;
+      last++;
+    }
+    rc = last - first <= kCapSmall ? launch_decode<kCapSmall>(&sorted[first], last - first, zero_fill, false, nullptr, st)
+                                   : launch_decode<kCapLarge>(&sorted[first], last - first, zero_fill, false, nullptr, st);
+    if (rc != HPX_OK) return rc;
+    first = last;
   }
   return HPX_OK;
 }
