@@ -16,15 +16,18 @@
 //   stream      ONE pass over the tensor: r = g + r, store r, compare with the
 //               threshold, wave64 ballot -> one 64-bit word per 64 elements
 //               (bit i = element i), a popcount and the largest |r| per workgroup
-//   scan        exclusive prefix of the per-workgroup counts within chunks of 4096,
-//               the chunks' totals and largest |r|
-//   expand      folds the chunk totals (each wave for itself), reports count,
+//   finish      tensors that keep up to 2560 entries: one workgroup lists the candidates, cuts
+//               them if they are too many, writes the message and clears the residual
+//   scan        larger tensors of more than 4096 workgroups: exclusive prefix of the
+//               per-workgroup counts within chunks of 4096, the chunks' totals and largest |r|
+//   expand      larger tensors: folds the totals (each workgroup for itself), reports count,
 //               threshold and largest |r| of each tensor to the host; bit words ->
-//               ascending indices at the scanned offsets, values out, residual
+//               ascending indices at their offsets, values out, residual
 //               entries zeroed, header written
 //
 // The stream pass moves 12 bytes per element (g, r in; r out) plus 1/8 byte of
-// mask; everything else touches O(sample + selected) data.  The host learns the
+// mask; everything else touches O(sample + selected) data.  For tensors
+// that keep fewer than 8192 entries that is all: their cut is the device's own business.  For the others the host learns the
 // candidate counts from pinned memory while the expand launch is still running
 // (it polls the words the expand launch writes first; no wait for the stream), and only
 // for tensors with more than `expected` candidates queues the cut: a stable LSD
@@ -59,7 +62,7 @@ struct GdState {
   uint32_t hits;      // provisional path: samples found above the provisional threshold so far
   uint32_t thr_bits;  // threshold as fp32 bits (provisional path: the provisional one until the exact one is known)
   uint32_t fallback;  // provisional path: 1 when the provisional threshold turned out to lie above the exact one
-  uint32_t total;     // candidates, left by the expand launch for the cut launch
+  uint32_t total;     // candidates of a tensor whose cut follows on the device, left by the expand launch
   uint32_t pad[60];
 };
 constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold
@@ -67,7 +70,8 @@ constexpr uint32_t kPreSamples = 16384;  // samples the provisional threshold is
 constexpr uint32_t kFallback = 0xFFFFFFFEu;  // reported in place of a count: this tensor has to take the other path
 constexpr int kScanChunk = 4096;   // per-tile counts scanned by one workgroup
 constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
-constexpr uint32_t kPickGather = 3072;   // a sample up to this size is gathered by the one workgroup that takes its threshold
+constexpr uint32_t kPickGather = 1536;   // a sample up to this size is gathered by the one workgroup that takes its threshold
+constexpr uint32_t kPickGatherBeside = 256;  // ... where the call has larger ones, and with them a gather launch, anyway
 constexpr uint32_t kPickMax = 65536;     // ... and up to this size its threshold is taken by one workgroup
 constexpr uint32_t kCutLds = 8192;       // candidates one workgroup sorts and cuts in LDS
 
@@ -142,6 +146,8 @@ struct GdArgs {
   int32_t residual;             // 0: the sparsifier without residual (dgc_body.h)
   int32_t margin;               // provisional path: how many times the expected number of entries the provisional
                                 // threshold lets through
+  uint32_t gather;              // the pick launch gathers samples of up to this size itself
+  int32_t device_cut;           // 1: tensors that keep fewer than kCutLds entries are cut on the device and report nothing
   int32_t tile_start[CAP + 1];  // exclusive prefix of this launch's workgroups per tensor
   GdSeg seg[CAP];
   uint32_t* report;             // pinned host memory, kReportWords per tensor of this table
@@ -328,12 +334,23 @@ __device__ __forceinline__ uint32_t select_rank(const uint32_t* __restrict__ key
 
 // The largest t whose bits below LO are zero and which more than `rank` of the wave's keys (R per lane) reach: with
 // LO = 0 the key of that rank (0-based from the top), else a lower bound of it.  Keys are bit patterns of
-// non-negative floats.  One wave, no barrier: a bit costs R compares and R counts on the scalar unit.
+// non-negative floats, zeros stand for no key; `floor` is a value the key of that rank is known to reach.  One wave, no
+// barrier: a bit costs R compares and R counts on the scalar unit, and the bits that the largest key shares with
+// the floor cost nothing.
 template <int R, int LO>
-__device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t rank) {
-  uint32_t t = 0;
+__device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor) {
+  uint32_t top = 0;
+#pragma unroll
+  for (int j = 0; j < R; j++) top = key[j] > top ? key[j] : top;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
+  top = __builtin_amdgcn_readfirstlane(top);
+  floor = __builtin_amdgcn_readfirstlane(floor);
+  const int first = 31 - __builtin_clz((top ^ floor) | 1u);   // bits above it are common to every candidate
+  uint32_t t = first < 31 ? (floor >> (first + 1)) << (first + 1) : 0u;
+  t = LO > 0 ? (t >> LO) << LO : t;
 #pragma unroll 1
-  for (int b = 30; b >= LO; b--) {
+  for (int b = first < 30 ? first : 30; b >= LO; b--) {
     const uint32_t c = t | (1u << b);
     uint32_t reach = 0;
 #pragma unroll
@@ -344,14 +361,16 @@ __device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t
 }
 
 // The threshold of a tensor whose sample has at most kPickMax entries, by ONE workgroup in one launch; up to kPickGather
-// of them it gathers itself (two lines per sample, about 1 us per 1000 samples; beyond that one CU's gathers take longer
-// than the extra launch that spreads them over the chip).  The rank wanted is low, a thousandth of the sample, so
+// of them it gathers itself (two lines per sample at about 700 random lines a microsecond for one CU: beyond that the
+// launch that spreads them over the chip is the quicker one).  The rank wanted is low, a thousandth of the sample, so
 // no histogram of the whole sample is needed: of the lanes' largest keys the one of that rank, cut off below its top
-// bits, is a lower bound of the threshold that hardly more keys reach than have to; those are listed in LDS and
-// one wave finds the exact one among them, bit by bit.  Where the bound does not help (a rank beyond the lanes, a
-// list that overflows: many equal keys) the workgroup takes the three histogram passes instead.
-// Replaces three histogram launches and a rank search: 1 M elements 15 us in four launches -> 8.4 us in one; ResNet-50's
-// 161 tensors 20 -> 19.8 us, and 6 us less in the gather launch before it.
+// bits, is a lower bound of the threshold that hardly more keys reach than have to; those are listed in LDS (from the three largest that every lane keeps)
+// and one wave finds the exact one among them, bit by bit.  Where the bound does not help (a rank beyond the lanes, a
+// list that overflows or a lane with more than it keeps: many equal keys) the workgroup takes the three histogram
+// passes instead.  The code is kept short on purpose: a launch of one workgroup per tensor meets a cold instruction cache,
+// and with the keys in 64 registers and every step unrolled over them this kernel took 9 and 20 us.
+// Replaces three histogram launches and a rank search: 1 M elements 15 us in four launches -> 5.2 us in one; ResNet-50's
+// 161 tensors 20 -> 7 us, and 4 us less in the gather launch before it.
 constexpr uint32_t kPickList = 1024;
 template <int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> a) {
@@ -362,10 +381,16 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
   const uint32_t count = sg.sample_cnt, t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  constexpr int kOwn = int(kPickGather) / kSelThreads;
-  uint32_t own[kOwn] = {};   // this lane's keys where they are gathered here
-  uint32_t big = 0;
-  if (count <= kPickGather) {
+  // the lane's three largest keys
+  uint32_t m1 = 0, m2 = 0, m3 = 0;
+  auto take = [&](uint32_t k) {
+    const uint32_t u = m1 < k ? m1 : k, v = m2 < u ? m2 : u;
+    m1 = m1 > k ? m1 : k;
+    m2 = m2 > u ? m2 : u;
+    m3 = m3 > v ? m3 : v;
+  };
+  if (count <= a.gather) {
+    constexpr int kOwn = (int(kPickGather) + kSelThreads - 1) / kSelThreads;
     float gv[kOwn], rv[kOwn];
 #pragma unroll
     for (int j = 0; j < kOwn; j++) {
@@ -377,58 +402,80 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
 #pragma unroll
     for (int j = 0; j < kOwn; j++) {
       const uint32_t x = uint32_t(j) * kSelThreads + t;
-      own[j] = __float_as_uint(__builtin_fabsf(a.residual ? gv[j] + rv[j] : gv[j]));
-      if (x < count) samples[x] = own[j];
-      big = own[j] > big ? own[j] : big;
+      const uint32_t k = __float_as_uint(__builtin_fabsf(a.residual ? gv[j] + rv[j] : gv[j]));
+      if (x < count) samples[x] = k;
+      take(k);
     }
   } else {
-    for (uint32_t x = t; x < count; x += 8 * kSelThreads) {
-      uint32_t k[8];
+    // four keys per load, four loads in flight (what lies beyond the sample counts as zero)
+    const uint4* __restrict__ quads = reinterpret_cast<const uint4*>(samples);
+    const uint32_t last = (count - 1) / 4;
+#pragma unroll 1
+    for (uint32_t q0 = 0; 4 * q0 < count; q0 += 4 * kSelThreads) {
+      uint4 k[4];
 #pragma unroll
-      for (uint32_t j = 0; j < 8; j++) k[j] = x + j * kSelThreads < count ? samples[x + j * kSelThreads] : 0u;
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t q = q0 + j * kSelThreads + t;
+        k[j] = quads[q < last ? q : last];
+      }
 #pragma unroll
-      for (uint32_t j = 0; j < 8; j++) big = k[j] > big ? k[j] : big;
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t x = 4 * (q0 + j * kSelThreads + t);
+        take(x + 0 < count ? k[j].x : 0u);
+        take(x + 1 < count ? k[j].y : 0u);
+        take(x + 2 < count ? k[j].z : 0u);
+        take(x + 3 < count ? k[j].w : 0u);
+      }
     }
   }
-  s_hist[t] = big;
+  s_hist[t] = m1;
   if (t == 0) s_n = 0;
   __syncthreads();
+  // The bound, from the largest keys of groups of lanes: with at least twice as many groups as keys wanted, few groups
+  // hide a second one, and a search over 64 keys takes a tenth of the time of one over 1024.  It is cut off at 12
+  // mantissa bits (with 4, a sample whose largest values crowd just under one value, as residuals do that are cleared
+  // when they pass a threshold, overflowed the list).
   if (wave == 0) {
-    uint32_t k[kSelThreads / kWave];
+    constexpr uint32_t kRows = kSelThreads / kWave;
+    uint32_t k[kRows];
 #pragma unroll
-    for (uint32_t j = 0; j < kSelThreads / kWave; j++) k[j] = s_hist[j * kWave + lane];
-    // with one key per lane at most, the lanes' keys are the sample
-    const uint32_t b = count <= uint32_t(kSelThreads) ? wave_rank<kSelThreads / kWave, 0>(k, sg.thr_index)
-                                                      : wave_rank<kSelThreads / kWave, 19>(k, sg.thr_index);
+    for (uint32_t j = 0; j < kRows; j++) k[j] = s_hist[j * kWave + lane];
+    uint32_t q[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+      q[j] = k[j];
+#pragma unroll
+      for (uint32_t i = j + 4; i < kRows; i += 4) q[j] = k[i] > q[j] ? k[i] : q[j];
+    }
+    uint32_t one[1] = {q[0]};
+#pragma unroll
+    for (uint32_t j = 1; j < 4; j++) one[0] = q[j] > one[0] ? q[j] : one[0];
+    const uint32_t b = count <= uint32_t(kWave) ? wave_rank<1, 0>(one, sg.thr_index, 0u)   // the sample itself
+                       : sg.thr_index < 32      ? wave_rank<1, 11>(one, sg.thr_index, 0u)
+                       : sg.thr_index < 128     ? wave_rank<4, 11>(q, sg.thr_index, 0u)
+                                                : wave_rank<kRows, 11>(k, sg.thr_index, 0u);
     if (lane == 0) s_key = b;
   }
   __syncthreads();
   const uint32_t bound = s_key;
-  if (count <= uint32_t(kSelThreads)) {
+  if (count <= uint32_t(kWave)) {
     if (t == 0) seg_state(sg)->thr_bits = bound;
     return;
   }
   bool listed = sg.thr_index < uint32_t(kSelThreads) && bound != 0u;   // workgroup-uniform
   if (listed) {
-    auto append = [&](uint32_t key, bool live) {
-      const bool in = live && key >= bound;
-      const uint64_t m = __ballot(in);
-      if (m == 0) return;
-      uint32_t base = 0;
-      if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(&s_n, uint32_t(__popcll(m)));
-      base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
-      if (in && base < kPickList) s_list[base] = key;
-    };
-    if (count <= kPickGather) {
-#pragma unroll
-      for (int j = 0; j < kOwn; j++) append(own[j], uint32_t(j) * kSelThreads + t < count);
-    } else {
-      for (uint32_t x = t; x - t < count; x += 8 * kSelThreads) {
-        uint32_t k[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) k[j] = x + j * kSelThreads < count ? samples[x + j * kSelThreads] : 0u;
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) append(k[j], x + j * kSelThreads < count);
+    if (__ballot(m1 >= bound) != 0) {   // most waves hold none
+#pragma unroll 1
+      for (int j = 0; j < 3; j++) {
+        const bool in = m1 >= bound;
+        const uint64_t m = __ballot(in);
+        if (m == 0) break;
+        uint32_t base = 0;
+        if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(&s_n, uint32_t(__popcll(m)));
+        base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+        if (in && base < kPickList) s_list[base] = m1;
+        m1 = m2; m2 = m3;
+        if (j == 2 && __ballot(in) != 0 && lane == 0) atomicAdd(&s_n, kPickList);   // a lane may hold a fourth: not all are listed
       }
     }
     __syncthreads();
@@ -436,26 +483,29 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
     listed = n <= kPickList;
     if (listed) {
       if (wave == 0) {
-        uint32_t key;
-        if (n <= 256) {
+        uint32_t found;
+        if (n <= kWave) {
+          const uint32_t k[1] = {lane < n ? s_list[lane] : 0u};
+          found = wave_rank<1, 0>(k, sg.thr_index, bound);
+        } else if (n <= 256) {
           uint32_t k[4];
 #pragma unroll
           for (uint32_t j = 0; j < 4; j++) k[j] = j * kWave + lane < n ? s_list[j * kWave + lane] : 0u;
-          key = wave_rank<4, 0>(k, sg.thr_index);
+          found = wave_rank<4, 0>(k, sg.thr_index, bound);
         } else {
           uint32_t k[kPickList / kWave];
 #pragma unroll
           for (uint32_t j = 0; j < kPickList / kWave; j++) k[j] = j * kWave + lane < n ? s_list[j * kWave + lane] : 0u;
-          key = wave_rank<kPickList / kWave, 0>(k, sg.thr_index);
+          found = wave_rank<kPickList / kWave, 0>(k, sg.thr_index, bound);
         }
-        if (lane == 0) seg_state(sg)->thr_bits = key;
+        if (lane == 0) seg_state(sg)->thr_bits = found;
       }
       return;
     }
   }
   __syncthreads();
-  const uint32_t key = select_rank(samples, count, sg.thr_index, s_hist);
-  if (t == 0) seg_state(sg)->thr_bits = key;
+  const uint32_t exact = select_rank(samples, count, sg.thr_index, s_hist);
+  if (t == 0) seg_state(sg)->thr_bits = exact;
 }
 
 // The first kPreSamples samples, one per lane over many workgroups (one workgroup's gathers into arrays of
@@ -878,7 +928,6 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   }
   if (a.margin >= 0 && st->fallback) {
     // the provisional threshold was not below the exact one: nothing of what the masks hold may be used
-    if (tile0 == 0 && lane == 0) seg_state(sg)->total = 0;
     if (tile0 == 0 && a.report != nullptr && lane == 0) {
       uint32_t* rep = a.report + size_t(s) * kReportWords;
       __hip_atomic_store(rep + 0, kFallback, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -887,8 +936,9 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     }
     return;
   }
+  const bool cut_here = a.device_cut != 0 && sg.limit < kCutLds;
   if (tile0 == 0 && lane == 0) seg_state(sg)->total = total;
-  if (tile0 == 0 && a.report != nullptr) {
+  if (tile0 == 0 && a.report != nullptr && !cut_here) {
     // Pinned host words the host polls (no copy command, no wait for the stream).  The host waits for each
     // of the three words to change, so plain system-scope stores do (a release would write the whole L2 back).
     if (lane == 0) {
@@ -932,12 +982,14 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     int32_t* __restrict__ cand = reinterpret_cast<int32_t*>(sg.cut + cl.ia);
     uint32_t* __restrict__ keys = reinterpret_cast<uint32_t*>(sg.cut + cl.ka);
     const uint32_t thr_bits = st->thr_bits;
+    // For the cut launch the sign travels in the index's top bit: it then never has to read the values again.
+    const uint32_t sign = cut_here ? 0x80000000u : 0u;
     // Sort key: distance of |r| above the threshold in fp32 bit patterns (same order as |r|;
     // the high digits of such keys are mostly zero, which lets the sort skip its last passes).
 #pragma unroll
     for (int j = 0; j < kExpandTiles; j++) {
       if (m[j]) {
-        cand[pos[j]] = int32_t(e1[j]);
+        cand[pos[j]] = int32_t(e1[j] | (__float_as_uint(v1[j]) & sign));
         keys[pos[j]] = __float_as_uint(__builtin_fabsf(v1[j])) - thr_bits;
         pos[j]++;
         m[j] &= m[j] - 1;
@@ -946,8 +998,9 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
       while (m[j]) {  // further candidates of the same group: rare
         const uint32_t e = e0 + uint32_t(__builtin_ctzll(m[j]));
         m[j] &= m[j] - 1;
-        cand[pos[j]] = int32_t(e);
-        keys[pos[j]] = __float_as_uint(__builtin_fabsf(r[e])) - thr_bits;
+        const float v = r[e];
+        cand[pos[j]] = int32_t(e | (__float_as_uint(v) & sign));
+        keys[pos[j]] = __float_as_uint(__builtin_fabsf(v)) - thr_bits;
         pos[j]++;
       }
     }
@@ -1231,42 +1284,192 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
   }
 }
 
-// The cut of a tensor with at most kCutLds candidates, by one workgroup in one launch: the same stable LSD sort
-// by byte digits, pairs in registers between the passes and in LDS for the exchange, then the message.  It is
-// queued behind the expand launch before the host knows any count and leaves at once where nothing has to be cut,
-// so a call of such tensors needs no work of the host's in the middle: the seven launches of the three-pass sort and the
-// host's turn-around (45-50 us for the 161 tensors of ResNet-50) became one launch of 18 us.
-template <int CAP>
-__global__ __launch_bounds__(kSortThreads) void gd_cut_kernel(const GdArgs<CAP> a) {
+// Exclusive prefix of `v` over the workgroup's lanes in order; `total` is the sum.  s_wave: a word per wave.
+__device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+  const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  uint32_t incl = v;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t u = __shfl_up(incl, o, kWave);
+    if (lane >= uint32_t(o)) incl += u;
+  }
+  if (lane == kWave - 1) s_wave[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < uint32_t(kSortWaves); w++) {
+    const uint32_t c = s_wave[w];
+    before += w < wave ? c : 0u;
+    total += c;
+  }
+  __syncthreads();
+  return before + incl - v;
+}
+
+// The `keep` largest |r| among the elements whose mask bit is set, in ascending index order, to LDS (keys as
+// distances from the threshold, the sign in the index's top bit): for a tensor with more candidates than fit.  A rank search over the candidates, then
+// one walk that lists those above the value found and the first ones equal to it.  Slow (one workgroup, four
+// walks over the mask) and all but never needed: a sampled threshold lets a few times the expected number
+// through only where the sample is a handful of values.
+__device__ __forceinline__ void top_of_masks(const uint64_t* __restrict__ masks, const float* __restrict__ r, uint32_t n, uint32_t keep,
+                                             uint32_t thr_bits, uint32_t* s_hist, uint32_t* s_wave, uint32_t* s_key, uint32_t* s_id) {
+  const uint32_t words = cdiv(n, kWave), t = threadIdx.x;
+  uint32_t prefix = 0, rank = keep - 1;
+#pragma unroll 1
+  for (int pass = 1; pass <= 3; pass++) {
+    for (int i = t; i < kBins1; i += kSortThreads) s_hist[i] = 0;
+    __syncthreads();
+    for (uint32_t w = t; w < words; w += kSortThreads) {
+      for (uint64_t m = masks[w]; m; m &= m - 1) {
+        const uint32_t v = __float_as_uint(__builtin_fabsf(r[w * kWave + uint32_t(__builtin_ctzll(m))]));
+        if (pass == 1) atomicAdd(&s_hist[v >> 21], 1u);
+        else if (pass == 2) { if ((v >> 21) == prefix) atomicAdd(&s_hist[(v >> 10) & 2047u], 1u); }
+        else if ((v >> 10) == prefix) atomicAdd(&s_hist[v & 1023u], 1u);
+      }
+    }
+    __syncthreads();
+    uint32_t d;
+    if (pass == 3) find_digit<kBins3>(s_hist, rank, d, rank); else find_digit<kBins1>(s_hist, rank, d, rank);
+    prefix = pass == 1 ? d : pass == 2 ? ((prefix << 11) | d) : ((prefix << 10) | d);
+  }
+  uint32_t at = 0, ties = rank + 1;  // of the elements equal to the value found, the first `ties` stay
+#pragma unroll 1
+  for (uint32_t w0 = 0; w0 < words; w0 += kSortThreads) {
+    const uint32_t w = w0 + t;
+    uint64_t above = 0, equal = 0;
+    for (uint64_t m = w < words ? masks[w] : 0ull; m; m &= m - 1) {
+      const uint64_t bit = m & (~m + 1);
+      const uint32_t v = __float_as_uint(__builtin_fabsf(r[w * kWave + uint32_t(__builtin_ctzll(m))]));
+      above |= v > prefix ? bit : 0ull;
+      equal |= v == prefix ? bit : 0ull;
+    }
+    uint32_t all_equal, all_listed;
+    const uint32_t equal_before = block_prefix(uint32_t(__popcll(equal)), s_wave, all_equal);
+    uint32_t room = ties > equal_before ? ties - equal_before : 0u;
+    uint64_t list = above;
+    for (; equal && room; equal &= equal - 1, room--) list |= equal & (~equal + 1);
+    uint32_t pos = at + block_prefix(uint32_t(__popcll(list)), s_wave, all_listed);
+    for (; list; list &= list - 1, pos++) {
+      const uint32_t e = w * kWave + uint32_t(__builtin_ctzll(list));
+      const uint32_t v = __float_as_uint(r[e]);
+      s_key[pos] = (v & 0x7FFFFFFFu) - thr_bits;
+      s_id[pos] = e | (v & 0x80000000u);
+    }
+    at += all_listed;
+    ties -= all_equal < ties ? all_equal : ties;
+  }
+  __syncthreads();
+}
+
+// The cut by one workgroup, of up to kCutLds candidates.  What bounds it is the chain of workgroup-wide steps, so the sort
+// has as few as possible: the keys (distance of |r| above the threshold in bit patterns) go into 4096 bins by exponent
+// and seven further bits of the distance as a float - fine where keys crowd just above the threshold, however far the
+// largest lies - the bins are laid out one after the other, and a key's place is its bin's first place plus the number
+// of keys of the bin that come before it (larger, or equal with a smaller index).  Where a bin is crowded all the same
+// (many equal values) the keys take a stable LSD sort by byte digits, pairs in registers between the passes and in
+// LDS for the exchange.  The code is instantiated for the number of pairs per lane: unrolled for the
+// most a workgroup can hold it was three times as long, and a launch of one workgroup per tensor meets a cold
+// instruction cache.
+constexpr uint32_t kCutBins = 4096;
+constexpr uint32_t kCutCrowd = 128;   // keys of one bin from which the digit sort is the quicker one
+struct CutArgs {
+  uint32_t* stage;   // LDS: 2 * kCutLds words
+  uint32_t* bins;    // LDS: kCutBins + 4 words, the first kCutBins zero
+  uint32_t* wave;    // LDS: a word per wave
+  float* r;
+  uint8_t* out;
+  uint32_t n, keep, thr_bits;
+  __device__ __forceinline__ void put(uint32_t place, uint32_t key, uint32_t id) const {   // an entry of the message
+    const uint32_t i = id & 0x7FFFFFFFu;
+    reinterpret_cast<int32_t*>(out + 4)[place] = int32_t(i);
+    reinterpret_cast<uint32_t*>(out + 4 + size_t(keep) * 4)[place] = (key + thr_bits) | (id & 0x80000000u);
+    r[i] = 0.0f;
+  }
+};
+
+// n pairs, lane t with those at t, t + 1024 ... (in ascending index order; the sign in the index's top bit).  False: some
+// bin is crowded, nothing has been written, and the pairs are in LDS, [kCutLds] keys and then [kCutLds] indices.
+template <int PER>
+__device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER]) {
+  const uint32_t t = threadIdx.x, n = f.n;
+  uint2* s_pair = reinterpret_cast<uint2*>(f.stage);
+  uint32_t* s_bins = f.bins;
+  uint32_t bin[PER], slot[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const bool live = uint32_t(j) * kSortThreads + t < n;
+    bin[j] = live ? kCutBins - 1 - ((__float_as_uint(float(key[j])) >> 16) - (127u << 7)) : 0u;
+    slot[j] = live ? atomicAdd(&s_bins[bin[j]], 1u) : 0u;
+  }
+  __syncthreads();
+  const uint4 c = reinterpret_cast<const uint4*>(s_bins)[t];
+  const uint32_t c01 = c.x > c.y ? c.x : c.y, c23 = c.z > c.w ? c.z : c.w;
+  uint32_t total;
+  const uint32_t first = block_prefix(c.x + c.y + c.z + c.w, f.wave, total);
+  if (__syncthreads_or((c01 > c23 ? c01 : c23) > kCutCrowd)) {
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const uint32_t x = uint32_t(j) * kSortThreads + t;
+      if (x < n) { f.stage[x] = key[j]; f.stage[kCutLds + x] = id[j]; }
+    }
+    __syncthreads();
+    return false;
+  }
+  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
+  if (t == 0) s_bins[kCutBins] = total;
+  __syncthreads();
+  uint32_t lo[PER], hi[PER], place[PER], longest = 0;
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const bool live = uint32_t(j) * kSortThreads + t < n;
+    place[j] = lo[j] = live ? s_bins[bin[j]] : 0u;
+    hi[j] = live ? s_bins[bin[j] + 1] : 0u;
+    longest = hi[j] - lo[j] > longest ? hi[j] - lo[j] : longest;
+    if (live) s_pair[lo[j] + slot[j]] = make_uint2(key[j], id[j]);
+  }
+  __syncthreads();
+  for (uint32_t q = 0; q < longest; q++) {   // the lane's pairs side by side: their LDS reads overlap
+    uint2 k[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) k[j] = s_pair[lo[j] + q < hi[j] ? lo[j] + q : lo[j]];
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+      place[j] += lo[j] + q < hi[j] && (k[j].x > key[j] || (k[j].x == key[j] && (k[j].y << 1) < (id[j] << 1))) ? 1u : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < PER; j++)
+    if (lo[j] < hi[j] && place[j] < f.keep) f.put(place[j], key[j], id[j]);
+  return true;
+}
+
+// The same for many equal or nearly equal keys: the digit sort.
+__device__ __forceinline__ void cut_crowded(const CutArgs& f) {
   constexpr uint32_t BINS = 256, kBinWaves = BINS / kWave;
   constexpr int kPer = int(kCutLds) / kSortThreads;
-  extern __shared__ uint32_t s_stage[];          // [kCutLds] keys, then [kCutLds] indices
-  __shared__ uint32_t s_cnt[kSortWaves][BINS];
   __shared__ uint32_t s_part[kBinWaves], s_max[kSortWaves];
-  uint32_t* s_key = s_stage;
-  uint32_t* s_id = s_stage + kCutLds;
-  const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
-  const uint32_t n = seg_state(sg)->total, keep = sg.limit;
-  if (n <= keep || n > sg.cap || n > kCutLds) return;
-  const CutLayout cl = cut_layout(sg.cap);
-  const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(sg.cut + cl.ka);
-  const int32_t* __restrict__ cand = reinterpret_cast<const int32_t*>(sg.cut + cl.ia);
+  static_assert(kCutBins >= kSortWaves * BINS, "one block for both");
+  uint32_t (*s_cnt)[BINS] = reinterpret_cast<uint32_t (*)[BINS]>(f.bins);
+  uint32_t* s_key = f.stage;
+  uint32_t* s_id = f.stage + kCutLds;
   const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t / kWave);
-  const uint32_t per = cdiv(n, kSortThreads);    // rounds of 64 pairs per wave, the same for every wave
+  const uint32_t n = f.n, keep = f.keep;
+  // pairs in order, the same number of rounds of 64 per wave for every wave
+  const uint32_t per = cdiv(n, kSortThreads);
   const uint32_t x0 = wave * per * kWave + lane;
   uint32_t key[kPer], id[kPer], big = 0;
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
     const uint32_t x = x0 + uint32_t(j) * kWave;
     const bool live = uint32_t(j) < per && x < n;
-    key[j] = live ? keys[x] : 0u;
-    id[j] = live ? uint32_t(cand[x]) : 0u;
+    id[j] = live ? s_id[x] : 0u;
+    key[j] = live ? s_key[x] : 0u;
     big = key[j] > big ? key[j] : big;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(big, o, kWave); big = v > big ? v : big; }
   if (lane == 0) s_max[wave] = big;
-  __syncthreads();
+  __syncthreads();   // also: every pair has been read
 #pragma unroll
   for (int w = 0; w < kSortWaves; w++) big = s_max[w] > big ? s_max[w] : big;
   const int passes = big ? (39 - __builtin_clz(big)) / 8 : 1;
@@ -1331,20 +1534,172 @@ __global__ __launch_bounds__(kSortThreads) void gd_cut_kernel(const GdArgs<CAP> 
       }
     }
   }
-  int32_t* __restrict__ idx = reinterpret_cast<int32_t*>(sg.out + 4);
-  float* __restrict__ val = reinterpret_cast<float*>(sg.out + 4 + size_t(keep) * 4);
-  float* __restrict__ r = sg.r;
-  if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + keep * 8);
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
     const uint32_t p = uint32_t(j) * kSortThreads + t;
-    if (p < keep) {
-      const uint32_t i = s_id[p];
-      idx[p] = int32_t(i);
-      val[p] = r[i];
-      r[i] = 0.0f;
-    }
+    if (p < keep) f.put(p, s_key[p], s_id[p]);
   }
+}
+// Pairs from wherever `pair(x, key, id)` finds them.
+template <int PER, typename F>
+__device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
+  uint32_t key[PER], id[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++) {   // (a pair beyond the last is read as the last and not used: no branch between the loads)
+    const uint32_t x = uint32_t(j) * kSortThreads + threadIdx.x;
+    pair(x < f.n ? x : f.n - 1, key[j], id[j]);
+  }
+  return cut_by_bins<PER>(f, key, id);
+}
+
+// What is left to do for a tensor that keeps at most kFinishKeep entries once the pass has marked its candidates,
+// by one workgroup in one launch: list them, cut them if there are too many, write the message and clear the
+// residual.  (Beyond that the values' random reads and the clearing's random writes, at about 700 lines a
+// microsecond for one CU, take longer than the expand launch that spreads them.)  A group of lanes looks after a tile
+// (as many as give every lane something to do), a lane after a run of the tile's mask words, of which the tile's coarse
+// word names the few that have a bit set; lanes in order, so one prefix over the workgroup's counts puts the indices
+// in ascending order in LDS.
+// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 6-9 us; ResNet-50's 161
+// tensors 58 -> 23 us.
+// Larger ones that still fit are only cut here, behind the expand launch.  All of it is queued before the host knows any
+// count.
+constexpr uint32_t kFinishKeep = 2560;
+constexpr uint32_t kFinishTiles = kScanChunk;
+// The cut of the tensors that keep between kFinishKeep and kCutLds entries, whose candidates and keys the expand
+// launch has listed (or, where they are too many for the list or for LDS, are found again in the mask).
+__device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, uint32_t* s_bins, uint32_t* s_wave) {
+  const uint32_t found = seg_state(sg)->total, keep = sg.limit, thr_bits = seg_state(sg)->thr_bits;
+  if (found <= keep) return;
+  const uint32_t t = threadIdx.x;
+  if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + keep * 8);
+  if (keep == 0) return;
+  const bool listed = found <= sg.cap && found <= kCutLds;
+  if (!listed) {
+    const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
+    top_of_masks(reinterpret_cast<const uint64_t*>(sg.ws + l.masks), sg.r, sg.n, keep, thr_bits, s_bins, s_wave, s_stage, s_stage + kCutLds);
+  }
+  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
+  const CutArgs f{s_stage, s_bins, s_wave, sg.r, sg.out, listed ? found : keep, keep, thr_bits};
+  bool done;
+  if (listed) {
+    const CutLayout cl = cut_layout(sg.cap);
+    const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(sg.cut + cl.ka);
+    const uint32_t* __restrict__ cand = reinterpret_cast<const uint32_t*>(sg.cut + cl.ia);
+    auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) { key = keys[x]; id = cand[x]; };
+    done = f.n <= 2 * kSortThreads ? cut_loaded<2>(f, pair) : f.n <= 4 * kSortThreads ? cut_loaded<4>(f, pair) : cut_loaded<8>(f, pair);
+  } else {
+    done = cut_loaded<8>(f, [=](uint32_t x, uint32_t& key, uint32_t& id) { key = f.stage[x]; id = f.stage[kCutLds + x]; });
+  }
+  if (!done) cut_crowded(f);
+}
+
+template <int CAP>
+__global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CAP> a) {
+  extern __shared__ uint32_t s_stage[];          // [kCutLds] keys, then [kCutLds] indices; or pairs of them
+  __shared__ __align__(16) uint32_t s_bins[kCutBins + 4];   // counts, then first places; the rank search's histogram; the digit sort's counts
+  __shared__ uint32_t s_wave[kSortWaves];
+  static_assert(kCutBins >= uint32_t(kBins1), "one block for both");
+  uint32_t* s_key = s_stage;
+  uint32_t* s_id = s_stage + kCutLds;
+  const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
+  if (sg.limit > kFinishKeep || cdiv(sg.n, kTile) > kFinishTiles) {
+    cut_listed(sg, s_stage, s_bins, s_wave);
+    return;
+  }
+  const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
+  const uint64_t* __restrict__ masks = reinterpret_cast<const uint64_t*>(sg.ws + l.masks);
+  const uint64_t* __restrict__ coarse = reinterpret_cast<const uint64_t*>(sg.ws + l.coarse);
+  const uint32_t thr_bits = seg_state(sg)->thr_bits, keep = sg.limit;
+  const uint32_t t = threadIdx.x;
+  const uint32_t ntiles = cdiv(sg.n, kTile);
+  float* __restrict__ r = sg.r;
+
+  // lanes per tile (a power of two, at most one per mask word), or tiles per lane
+  int group = 0;   // log2
+  while (group < 6 && (ntiles << (group + 1)) <= uint32_t(kSortThreads)) group++;
+  const uint32_t per_lane = cdiv(ntiles, kSortThreads);   // 1 unless there are more tiles than lanes
+  const uint32_t tile0 = group ? t >> group : t * per_lane;
+  const uint32_t words = kWave >> group, word0 = (t & ((1u << group) - 1)) * words;
+  const uint64_t range = words == 64 ? ~0ull : ((1ull << words) - 1) << word0;
+  // The lane's words of its first tile, the first four of them in registers.
+  auto four = [&](uint32_t tile, uint64_t& c, uint32_t (&e)[4], uint64_t (&m)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t w = c ? uint32_t(__builtin_ctzll(c)) : 0u;
+      e[k] = tile * uint32_t(kTile) + w * kWave;
+      m[k] = c ? masks[size_t(tile) * kWave + w] : 0ull;
+      c &= c - 1;   // 0 stays 0
+    }
+  };
+  uint64_t c0 = tile0 < ntiles ? coarse[tile0] & range : 0ull, m0[4];
+  uint32_t e0[4];
+  four(tile0, c0, e0, m0);
+  uint32_t mine = 0, n;
+  if (group == 0) {   // whole tiles: the pass has left their counts
+    for (uint32_t q = 0; q < per_lane && tile0 + q < ntiles; q++) mine += reinterpret_cast<const uint32_t*>(sg.ws + l.cnt)[tile0 + q];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++) mine += uint32_t(__popcll(m0[k]));
+    for (uint64_t c = c0; c; c &= c - 1) mine += uint32_t(__popcll(masks[size_t(tile0) * kWave + uint32_t(__builtin_ctzll(c))]));
+  }
+  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
+  uint32_t pos = block_prefix(mine, s_wave, n);
+  const bool cut = n > keep;
+  if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + (cut ? keep : n) * 8);
+  if (n == 0 || keep == 0) return;
+  if (n <= kCutLds) {
+    auto list = [&](const uint32_t (&e)[4], const uint64_t (&m)[4]) {
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        for (uint64_t x = m[k]; x; x &= x - 1, pos++) s_id[pos] = e[k] + uint32_t(__builtin_ctzll(x));
+    };
+    list(e0, m0);
+    for (uint32_t q = 0;;) {
+      while (c0) {
+        four(tile0 + q, c0, e0, m0);
+        list(e0, m0);
+      }
+      if (++q >= per_lane || tile0 + q >= ntiles) break;
+      c0 = coarse[tile0 + q];
+    }
+    __syncthreads();
+  } else {
+    top_of_masks(masks, r, sg.n, keep, thr_bits, s_bins, s_wave, s_key, s_id);
+    reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
+    n = keep;
+  }
+  if (!cut) {   // gd_body.h:193-229
+    int32_t* __restrict__ idx = reinterpret_cast<int32_t*>(sg.out + 4);
+    float* __restrict__ val = reinterpret_cast<float*>(sg.out + 4 + size_t(n) * 4);
+    for (uint32_t x0 = t; x0 < n; x0 += 3 * kSortThreads) {   // three values in flight per lane
+      uint32_t i[3];
+      float v[3];
+#pragma unroll
+      for (uint32_t j = 0; j < 3; j++) i[j] = s_id[x0 + j * kSortThreads < n ? x0 + j * kSortThreads : x0];
+#pragma unroll
+      for (uint32_t j = 0; j < 3; j++) v[j] = r[i[j]];
+#pragma unroll
+      for (uint32_t j = 0; j < 3; j++) {
+        const uint32_t x = x0 + j * kSortThreads;
+        if (x < n) {
+          idx[x] = int32_t(i[j]);
+          val[x] = v[j];
+          r[i[j]] = 0.0f;
+        }
+      }
+    }
+    return;
+  }
+  const CutArgs f{s_stage, s_bins, s_wave, r, sg.out, n, keep, thr_bits};
+  auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
+    id = s_id[x];
+    const uint32_t v = __float_as_uint(r[id & 0x7FFFFFFFu]);
+    key = (v & 0x7FFFFFFFu) - thr_bits;
+    id |= v & 0x80000000u;
+  };
+  const bool done = n <= kSortThreads ? cut_loaded<1>(f, pair) : n <= 3 * kSortThreads ? cut_loaded<3>(f, pair) : cut_loaded<8>(f, pair);
+  if (!done) cut_crowded(f);
 }
 
 // ---- decode -----------------------------------------------------------------
@@ -1514,13 +1869,15 @@ struct Plan {
   int index;  // position in the call
 };
 
-// Whether the device alone settles a tensor's cut (gd_cut_kernel) as long as it has `found` candidates.
-bool cut_on_device(const GdSeg& sg, uint64_t found) { return sg.limit < kCutLds && found <= sg.cap && found <= kCutLds; }
+// Who settles a tensor behind the pass: one workgroup (gd_finish_kernel); the expand launch and, if it has to be cut, one
+// workgroup (the same launch: its LDS holds what is kept); or the expand launch and the host, which queues the sort of
+// many workgroups once it has heard the count.  The provisional path keeps to the last: it may have to fall back.
+bool finishes(const GdSeg& sg, int margin) { return margin < 0 && sg.limit <= kFinishKeep && cdiv(sg.n, kTile) <= kFinishTiles; }
+bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutLds; }
 
 // The phases for up to CAP tensors, no host wait.  margin < 0: the threshold from the full gathered sample
 // (for samples of up to kPickMax one workgroup each, behind a gather launch where a sample exceeds kPickGather; for
-// larger ones gather, three histogram passes, rank search), then the pass, scan, expand and the cut of the tensors
-// whose candidates fit a workgroup.  A launch that no tensor of the table takes part in is left out.  margin >= 0: the provisional
+// larger ones gather, three histogram passes, rank search), then the pass, and the finish or scan and expand.  A launch that no tensor of the table takes part in is left out.  margin >= 0: the provisional
 // path (above): provisional threshold, the pass, the samples against the mask, exact threshold, recount, scan, expand.
 template <int CAP>
 int launch_phases(const Plan* plans, int count, bool residual, int margin, uint32_t* report, hipStream_t st) {
@@ -1528,6 +1885,8 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   a.nseg = count;
   a.residual = residual ? 1 : 0;
   a.margin = margin;
+  a.gather = 0;
+  a.device_cut = margin < 0 ? 1 : 0;
   a.report = report;
   for (int i = 0; i < count; i++) a.seg[i] = plans[i].seg;
   auto tiles = [&](auto per_tensor) {
@@ -1549,8 +1908,14 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   };
   dim3 grid;
   if (margin < 0) {
-    grid = tiles([](const GdSeg& sg) {
-      if (sg.sample_cnt <= kPickGather) return 0u;
+    // One workgroup's gathers of a sample take as long as a launch that spreads them at about kPickGather samples;
+    // beside larger samples that launch is there anyway.
+    a.gather = kPickGather;
+    for (int i = 0; i < count; i++)
+      if (a.seg[i].sample_cnt > kPickGather) a.gather = kPickGatherBeside;
+    const uint32_t gather = a.gather;
+    grid = tiles([gather](const GdSeg& sg) {
+      if (sg.sample_cnt <= gather) return 0u;
       return cdiv(sg.sample_cnt, kThreads);   // more than enough lanes to clear the histograms where they are used
     });
     if (grid.x) HPX_LAUNCH("gd_sample_kernel", gd_sample_kernel<CAP>, grid, dim3(kThreads), st, a);
@@ -1584,14 +1949,14 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   HPX_HIP(hipGetLastError());
   // Queued before the host knows the counts: the finish where nothing has to be cut,
   // else the candidate list and keys of the cut path.
-  grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
-  HPX_LAUNCH("gd_expand_kernel", gd_expand_kernel<CAP>, grid, dim3(kThreads), st, a);
-  grid = tiles([](const GdSeg& sg) { return sg.limit < kCutLds && sg.limit < sg.n ? 1u : 0u; });
+  grid = tiles([margin](const GdSeg& sg) { return finishes(sg, margin) ? 0u : cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
+  if (grid.x) HPX_LAUNCH("gd_expand_kernel", gd_expand_kernel<CAP>, grid, dim3(kThreads), st, a);
+  grid = tiles([margin](const GdSeg& sg) { return finishes(sg, margin) || cut_on_device(sg, margin) ? 1u : 0u; });
   if (grid.x) {
     constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));
     static std::atomic<uint64_t> attr_done{0};
-    if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_cut_kernel<CAP>), kStageBytes, attr_done)) return rc;
-    HPX_LAUNCH_LDS("gd_cut_kernel", hpx::g_prof_on, gd_cut_kernel<CAP>, grid, dim3(kSortThreads), kStageBytes, st, a);
+    if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_finish_kernel<CAP>), kStageBytes, attr_done)) return rc;
+    HPX_LAUNCH_LDS("gd_finish_kernel", hpx::g_prof_on, gd_finish_kernel<CAP>, grid, dim3(kSortThreads), kStageBytes, st, a);
   }
   HPX_HIP(hipGetLastError());
   return HPX_OK;
@@ -1601,8 +1966,10 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
 // the kernel writes them with system-scope stores as the first thing it does, so they arrive while the stream
 // is still busy with that launch).  Polls memory; every 20 us or so it also asks whether the stream has drained, which ends the
 // wait if the words can only be seen once the kernels have finished, or if a launch failed.
-int wait_reports(volatile uint32_t* report, int count, hipStream_t st) {
+// A tensor that is settled on the device is not waited for.
+int wait_reports(volatile uint32_t* report, const Plan* plans, int count, int margin, hipStream_t st) {
   for (int t = 0; t < count; t++) {
+    if (cut_on_device(plans[t].seg, margin)) continue;
     volatile uint32_t* word = report + size_t(t) * kReportWords;
     uint32_t spins = 0;
     auto pending = [word]() { return word[0] == kNotReported || word[1] == kNotReported || word[2] == kNotReported; };
@@ -1715,21 +2082,17 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
       for (int w = 0; w < 3; w++) report[size_t(t) * kReportWords + w] = kNotReported;
     __atomic_thread_fence(__ATOMIC_RELEASE);
   };
-  // Tensors whose every possible count the device settles by itself: nothing to report, nothing to wait for.
-  bool unattended = margin < 0;
-  for (const Plan& p : plans) unattended = unattended && (cut_on_device(p.seg, p.seg.n) || p.seg.limit >= p.seg.n);
   for (int first = 0; first < total; first += kMaxPerWait) {
     const int batch = total - first < kMaxPerWait ? total - first : kMaxPerWait;
-    if (!unattended) reset_reports(batch);
+    reset_reports(batch);
     for (int k = 0; k < batch; k += kCapLarge) {
       const int m = batch - k < kCapLarge ? batch - k : kCapLarge;
-      uint32_t* rep = unattended ? nullptr : const_cast<uint32_t*>(report) + size_t(k) * kReportWords;
+      uint32_t* rep = const_cast<uint32_t*>(report) + size_t(k) * kReportWords;
       rc = m <= kCapSmall ? launch_phases<kCapSmall>(&plans[first + k], m, residuals != nullptr, margin, rep, st)
                           : launch_phases<kCapLarge>(&plans[first + k], m, residuals != nullptr, margin, rep, st);
       if (rc != HPX_OK) return rc;
     }
-    if (unattended) continue;
-    rc = wait_reports(report, batch, st);
+    rc = wait_reports(report, &plans[first], batch, margin, st);
     if (rc != HPX_OK) return rc;
     // What the tensors reported, kept on the host: the pinned words serve again below.
     std::vector<uint32_t> rep_host(size_t(batch) * kReportWords);
@@ -1756,10 +2119,12 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
                               : launch_phases<kCapLarge>(&again[k], m, false, -1, rep, st);
           if (rc != HPX_OK) return rc;
         }
-        rc = wait_reports(report, int(again.size()), st);
+        rc = wait_reports(report, again.data(), int(again.size()), -1, st);
         if (rc != HPX_OK) return rc;
-        for (size_t j = 0; j < fb.size(); j++)
+        for (size_t j = 0; j < fb.size(); j++) {
           for (int w = 0; w < kReportWords; w++) rep_host[size_t(fb[j]) * kReportWords + w] = report[j * kReportWords + w];
+          if (cut_on_device(again[j].seg, -1)) rep_host[size_t(fb[j]) * kReportWords] = 0;   // nothing left to cut
+        }
       }
     }
     // More candidates than `expected`: order them by |r| descending and keep the first `expected`
@@ -1770,7 +2135,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
     for (int t = 0; t < batch; t++) {
       const GdSeg& sg = plans[first + t].seg;
       const uint32_t found = rep_host[size_t(t) * kReportWords];
-      if (found <= sg.limit || cut_on_device(sg, found)) continue;
+      if (cut_on_device(sg, margin) || found <= sg.limit) continue;
       const uint32_t thr_bits = rep_host[size_t(t) * kReportWords + 1], max_bits = rep_host[size_t(t) * kReportWords + 2];
       // keys are |r| bits minus threshold bits: the largest tells how many byte digits are in use
       const uint32_t max_key = max_bits > thr_bits ? max_bits - thr_bits : 0u;
@@ -1815,6 +2180,8 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         a.nseg = 1;
         a.residual = residuals != nullptr;
         a.margin = -1;
+        a.gather = 0;
+        a.device_cut = 0;
         a.report = nullptr;  // the host has its report
         a.seg[0] = plan.seg;
         a.seg[0].cut = cut;
