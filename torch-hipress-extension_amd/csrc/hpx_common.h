@@ -149,7 +149,9 @@ int copy_ranges(int count, uint8_t* const* dst, const uint8_t* const* src, const
 // How the outputs of a decode call relate: 0 = pairwise disjoint, 1 = some are
 // named more than once but every overlap is an exact duplicate (same pointer,
 // same size: several messages accumulate into one tensor), 2 = partial overlaps.
-int classify_outputs(int count, float* const* outs, const int32_t* sizes);
+// Where the list is a first run of distinct tensors repeated in the same order (the usual hand-over of several gathered
+// messages per tensor) *period is the length of that run, else 0.
+int classify_outputs(int count, float* const* outs, const int32_t* sizes, int* period = nullptr);
 
 // ---- device helpers --------------------------------------------------------
 constexpr int kWave = 64;

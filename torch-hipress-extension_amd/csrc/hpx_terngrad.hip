@@ -81,6 +81,9 @@ struct EncArgs {
 struct __attribute__((packed, aligned(1))) u32u {
   uint32_t v;
 };
+struct __attribute__((packed, aligned(1))) u16u {
+  uint16_t v;
+};
 struct DecSeg {
   float* out;
   const uint8_t* in;
@@ -428,6 +431,15 @@ __device__ __forceinline__ void quant_unit_ragged(const EncSeg& sg, float mn, fl
   }
 }
 
+// The BYTES packed bytes of a unit, at an address that is only known to be a byte's (the payload starts at byte 10).
+template <int BYTES>
+__device__ __forceinline__ void store_codes(uint8_t* p, uint32_t packed) {
+  static_assert(BYTES == 1 || BYTES == 2 || BYTES == 4, "bytes of a unit");
+  if constexpr (BYTES == 4) reinterpret_cast<u32u*>(p)->v = packed;
+  else if constexpr (BYTES == 2) reinterpret_cast<u16u*>(p)->v = uint16_t(packed);
+  else *p = uint8_t(packed);
+}
+
 // One tile of the quantise stream.  A unit is UNIT = max(4, 8/B) consecutive
 // elements owned by one lane per step; it packs into BPU = UNIT*B/8 bytes.
 template <int B, bool RANDOM>
@@ -462,21 +474,27 @@ __device__ __forceinline__ void quant_tile(const EncSeg& sg, const float mn, con
       for (int h = 0; h < UNIT / 4; h++)
         v[k][h] = ld4_stream(xp + size_t(u0 + k * kThreads) * UNIT + h * 4);
 #pragma unroll
-    for (int k = 0; k < kQIters; k++) {
-      const uint32_t packed = quant_unit<B, RANDOM>(v[k], mn, gi, draw, kStrideBytes);
-#pragma unroll
-      for (int jb = 0; jb < BPU; jb++) pay[size_t(u0 + k * kThreads) * BPU + jb] = uint8_t(packed >> (8 * jb));
-    }
+    for (int k = 0; k < kQIters; k++)
+      store_codes<BPU>(pay + size_t(u0 + k * kThreads) * BPU, quant_unit<B, RANDOM>(v[k], mn, gi, draw, kStrideBytes));
     return;
   }
-  // Tile holding the end of the tensor.
+  // Tile holding the end of the tensor: its whole units like those above, all loads first (a lane without one reads
+  // the tile's first and stores nothing); the partial unit, if there is one, from memory element by element.  (Done
+  // element by element throughout, this workgroup waited for memory sixteen times in a row behind all others.)
+  const uint32_t whole = n / UNIT;
+  float4 v[kQIters][UNIT / 4];
+#pragma unroll
   for (int k = 0; k < kQIters; k++) {
     const uint32_t u = u0 + k * kThreads;
-    if (u < units_total) quant_unit_ragged<B, RANDOM>(sg, mn, gi, u, draw);
-    if (RANDOM) {
 #pragma unroll
-      for (int q = 0; q < UNIT; q++) draw[q] += lcg_mul(q % DPB + 2) * kStrideBytes;
-    }
+    for (int h = 0; h < UNIT / 4; h++) v[k][h] = whole ? ld4(xp + size_t(u < whole ? u : 0u) * UNIT + h * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+#pragma unroll
+  for (int k = 0; k < kQIters; k++) {
+    const uint32_t u = u0 + k * kThreads;
+    if (u == whole && u < units_total) quant_unit_ragged<B, RANDOM>(sg, mn, gi, u, draw);
+    const uint32_t packed = quant_unit<B, RANDOM>(v[k], mn, gi, draw, kStrideBytes);
+    if (u < whole) store_codes<BPU>(pay + size_t(u) * BPU, packed);
   }
 }
 
@@ -498,6 +516,106 @@ __global__ __launch_bounds__(kThreads) void terngrad_quant_kernel(const EncArgs<
     case 2: quant_dispatch<2>(a.seg[s], mn, gi, t); break;
     case 4: quant_dispatch<4>(a.seg[s], mn, gi, t); break;
     default: quant_dispatch<8>(a.seg[s], mn, gi, t); break;
+  }
+}
+
+// ---- small tensors ----------------------------------------------------------------
+// A tensor of at most kSmallMax elements, start to finish by one workgroup: extremes, then codes, the second time out
+// of the L2 (or, up to 16384 elements, out of the registers).  What bounds such a call is launches and
+// latencies: one launch instead of two, and no slots to fold and read back.  One tensor of 2048 elements, encode +
+// decode back to back: 9.0 -> 6.7 us; one CU reads 256 KB in about 3 us, which is where the second launch of the tiled pair
+// becomes the cheaper way.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallRows = 4;      // units per lane and step
+constexpr int32_t kSmallMax = 65536;
+template <int B, bool RANDOM>
+__device__ __forceinline__ void small_tensor(const EncSeg& sg) {
+  constexpr int DPB = 8 / B;
+  constexpr int UNIT = DPB > 4 ? DPB : 4;
+  constexpr int BPU = UNIT / DPB;
+  constexpr int kWaves = kSmallThreads / kWave;
+  __shared__ float s_mn[kWaves], s_mx[kWaves], s_am[kWaves];
+  __shared__ uint32_t s_first;
+  const float* __restrict__ xp = sg.x;
+  const uint32_t n = static_cast<uint32_t>(sg.n), whole = n / UNIT, t = threadIdx.x;
+  const uint32_t steps = ((n + UNIT - 1) / UNIT - 1) / (kSmallThreads * kSmallRows) + 1;   // a partial last unit included
+  float4 v[kSmallRows][UNIT / 4];
+  auto load = [&](uint32_t step) {   // (a lane past the end reads the tensor's first unit again)
+#pragma unroll
+    for (int k = 0; k < kSmallRows; k++) {
+      const uint32_t u = (step * kSmallRows + k) * kSmallThreads + t;
+#pragma unroll
+      for (int h = 0; h < UNIT / 4; h++)
+        v[k][h] = whole ? ld4(xp + size_t(u < whole ? u : 0u) * UNIT + h * 4) : make_float4(xp[0], xp[0], xp[0], xp[0]);
+    }
+  };
+  float mn = __builtin_inff(), mx = -__builtin_inff(), am = __builtin_inff();
+  if (whole * UNIT + t < n) acc3(xp[whole * UNIT + t], mn, mx, am);
+#pragma unroll 1
+  for (uint32_t i = 0; i < steps; i++) {
+    load(i);
+#pragma unroll
+    for (int k = 0; k < kSmallRows; k++)
+#pragma unroll
+      for (int h = 0; h < UNIT / 4; h++) acc3x4(v[k][h], mn, mx, am);
+  }
+  mn = wave_min(mn);
+  mx = wave_max(mx);
+  am = wave_min(am);
+  if ((t & (kWave - 1)) == 0) { s_mn[t / kWave] = mn; s_mx[t / kWave] = mx; s_am[t / kWave] = am; }
+  if (t == 0) s_first = 0xFFFFFFFFu;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) {
+    mn = s_mn[w] < mn ? s_mn[w] : mn;
+    mx = s_mx[w] > mx ? s_mx[w] : mx;
+    am = s_am[w] < am ? s_am[w] : am;
+  }
+  if (am == 0.0f && (mn == 0.0f || mx == 0.0f)) {   // a zero extreme takes the sign of the first zero
+    uint32_t first = 0xFFFFFFFFu;
+    for (uint32_t e = t; e < n; e += kSmallThreads)
+      if (xp[e] == 0.0f) { first = e; break; }
+    first = wave_min_u32(first);
+    if ((t & (kWave - 1)) == 0) atomicMin(&s_first, first);
+    __syncthreads();
+    const float zv = xp[s_first];
+    if (mn == 0.0f) mn = zv;
+    if (mx == 0.0f) mx = zv;
+  }
+  const float gi = inverse_gap(mn, mx, B);
+  if (t == 0) write_header(sg.out, B, n, mn, mx);
+  uint8_t* __restrict__ pay = sg.out + 10;
+#pragma unroll 1
+  for (uint32_t i = steps; i-- > 0;) {   // the last step's units are still in registers
+    if (i + 1 < steps) load(i);
+    const uint32_t u0 = i * kSmallRows * kSmallThreads + t;
+    uint32_t draw[UNIT];
+    if (RANDOM) {
+#pragma unroll
+      for (int q = 0; q < UNIT; q++) draw[q] = lcg_mul(q % DPB + 2) * (sg.seed + u0 * BPU + q / DPB) + lcg_add(q % DPB + 2);
+    }
+#pragma unroll
+    for (int k = 0; k < kSmallRows; k++) {
+      const uint32_t u = u0 + k * kSmallThreads;
+      if (u == whole && whole * UNIT < n) quant_unit_ragged<B, RANDOM>(sg, mn, gi, u, draw);
+      const uint32_t packed = quant_unit<B, RANDOM>(v[k], mn, gi, draw, uint32_t(kSmallThreads) * BPU);
+      if (u < whole) store_codes<BPU>(pay + size_t(u) * BPU, packed);
+    }
+  }
+}
+
+template <int CAP>
+__global__ __launch_bounds__(kSmallThreads) void terngrad_small_kernel(const EncArgs<CAP> a) {
+  const EncSeg& sg = a.seg[blockIdx.x];
+  switch (sg.bits * 2 + (sg.random ? 1 : 0)) {
+    case 2: small_tensor<1, false>(sg); break;
+    case 3: small_tensor<1, true>(sg); break;
+    case 4: small_tensor<2, false>(sg); break;
+    case 5: small_tensor<2, true>(sg); break;
+    case 8: small_tensor<4, false>(sg); break;
+    case 9: small_tensor<4, true>(sg); break;
+    case 16: small_tensor<8, false>(sg); break;
+    default: small_tensor<8, true>(sg); break;
   }
 }
 
@@ -1329,8 +1447,8 @@ template <int B>
 __device__ __forceinline__ uint32_t group_bits(const uint8_t* __restrict__ pay, size_t e) {
   if (B == 1) return (uint32_t(pay[e >> 3]) >> (e & 4)) & 0xFu;
   if (B == 2) return pay[e >> 2];
-  if (B == 4) return uint32_t(pay[e >> 1]) | (uint32_t(pay[(e >> 1) + 1]) << 8);
-  return uint32_t(pay[e]) | (uint32_t(pay[e + 1]) << 8) | (uint32_t(pay[e + 2]) << 16) | (uint32_t(pay[e + 3]) << 24);
+  if (B == 4) return as_global(reinterpret_cast<const u16u*>(pay + (e >> 1)))->v;
+  return as_global(reinterpret_cast<const u32u*>(pay + e))->v;
 }
 
 template <int B>
@@ -1373,19 +1491,33 @@ __device__ __forceinline__ void decode_tile(const DecSeg& sg, float mn, float ga
     }
     return;
   }
-  for (int k = 0; k < kDIters; k++) {
-    const size_t e = size_t(g0 + k * kThreads) * 4;
-    if (e + 4 <= cnt) {
-      float4 v = group_values<B>(group_bits<B>(pay, e), gap, mn);
-      if (ADD) {
-        const float4 o = ld4(op + e);
-        v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
+  // The tile that holds the end: its whole groups as above, all loads first (a lane without one reads the tensor's
+  // first and stores nothing), then the 1..3 elements that are left.
+  const uint32_t whole = cnt / 4;
+  uint32_t q[kDIters];
+  float4 o[kDIters];
+  if (whole) {
+#pragma unroll
+    for (int k = 0; k < kDIters; k++) {
+      const size_t e = g0 + k * kThreads < whole ? size_t(g0 + k * kThreads) * 4 : 0;
+      q[k] = group_bits<B>(pay, e);
+      o[k] = ADD ? ld4(op + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int k = 0; k < kDIters; k++) {
+      if (g0 + k * kThreads < whole) {
+        float4 v = group_values<B>(q[k], gap, mn);
+        if (ADD) { v.x += o[k].x; v.y += o[k].y; v.z += o[k].z; v.w += o[k].w; }
+        st4(op + size_t(g0 + k * kThreads) * 4, v);
       }
-      st4(op + e, v);
-    } else {
-      for (size_t i = e; i < cnt && i < e + 4; i++) {
-        const uint32_t q = (pay[i / DPB] >> ((i % DPB) * B)) & MASK;
-        const float v = float(int(q)) * gap + mn;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kDIters; k++) {
+    if (g0 + k * kThreads == whole) {
+      for (size_t i = size_t(whole) * 4; i < cnt; i++) {
+        const uint32_t c = (pay[i / DPB] >> ((i % DPB) * B)) & MASK;
+        const float v = float(int(c)) * gap + mn;
         op[i] = ADD ? v + op[i] : v;
       }
     }
@@ -1440,7 +1572,8 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_kernel(const DecArgs
 constexpr int kMultiSegs = 64;
 constexpr int kMultiSlots = 448;
 constexpr int kMultiSlotsPerSeg = 32;  // header fields of one tensor's messages are staged in LDS
-constexpr int kMultiRep = 4;            // sub-tiles of kDecTile elements per workgroup of the multi-message decode
+constexpr int kMultiRep = 4;            // sub-tiles of kDecTile elements per workgroup of the multi-message decode (headers parsed once) ...
+constexpr int64_t kMultiFull = 1024;    // ... as long as that leaves this many workgroups (4 per CU); fewer sub-tiles each below that
 struct MSeg {
   float* out;
   int32_t out_size;
@@ -1455,6 +1588,7 @@ struct MSlot {
 };
 struct MArgs {
   int32_t nseg;
+  int32_t reps;         // sub-tiles per workgroup
   int32_t tile_start[kMultiSegs + 1];
   MSeg seg[kMultiSegs];
   MSlot slot[kMultiSlots];
@@ -1479,6 +1613,7 @@ struct SSeg {
 };
 struct SArgs {
   int32_t nseg;
+  int32_t reps;         // sub-tiles per workgroup
   int32_t tile_start[kStrideSegs + 1];
   SSeg seg[kStrideSegs];
   uint32_t* status;
@@ -1508,7 +1643,7 @@ __device__ __forceinline__ uint32_t code_at(const uint8_t* __restrict__ pay, siz
 }
 
 // The common case of the multi-message decoder (NS complete 2-bit messages, 2 <= NS <= 8), for the sub-tiles of
-// the workgroup that lie wholly inside the tensor; returns how many of its kMultiRep sub-tiles it has done.
+// the workgroup that lie wholly inside the tensor; returns how many of its sub-tiles it has done.
 // A wave owns kDIters * 64 consecutive groups, i.e. that many consecutive payload bytes of every message: each
 // message costs the wave ONE load (a dword per lane) and the lanes pick their bytes out of it with cross-lane
 // reads.  NS is a compile-time constant and the loads are unconditional: under per-message branches the
@@ -1516,13 +1651,13 @@ __device__ __forceinline__ uint32_t code_at(const uint8_t* __restrict__ pay, siz
 // latency (7 messages into 25.5 M elements: 75 us; now 65, of which about 30 are the 22 operations per group
 // and message).
 template <int NS>
-__device__ __forceinline__ uint32_t decode_two_bit_whole(float* __restrict__ op, uint32_t n, bool need_old, uint32_t sub0,
+__device__ __forceinline__ uint32_t decode_two_bit_whole(float* __restrict__ op, uint32_t n, bool need_old, uint32_t sub0, uint32_t reps,
                                                              const uint8_t* const* s_pay, const float* s_gap,
                                                              const float* s_mn, const int32_t* s_add) {
   static_assert(kDIters * 4 <= kWave, "a wave's bytes of one message must fit one dword per lane");
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t whole = n / uint32_t(kThreads * kDIters * 4);  // sub-tiles wholly inside the tensor
-  const uint32_t nfull = whole > sub0 ? (whole - sub0 < uint32_t(kMultiRep) ? whole - sub0 : uint32_t(kMultiRep)) : 0u;
+  const uint32_t nfull = whole > sub0 ? (whole - sub0 < reps ? whole - sub0 : reps) : 0u;
   // per-message constants as wave-uniform values in scalar registers
   const uint8_t* pay[NS];
   float gap[NS], mn[NS];
@@ -1595,6 +1730,56 @@ __device__ __forceinline__ uint32_t decode_two_bit_whole(float* __restrict__ op,
   return nfull;
 }
 
+// NS (at most 4) messages of one width other than 2 bits folded into the groups of a whole sub-tile: the loads of all
+// of them and of the lane's groups in flight together.
+template <int B, int NS>
+__device__ __forceinline__ void fold_messages(float4 (&acc)[kDIters], uint32_t g0, int j0, const uint8_t* const* s_pay, const float* s_gap,
+                                              const float* s_mn, const int32_t* s_add) {
+  uint32_t raw[NS][kDIters];
+#pragma unroll
+  for (int j = 0; j < NS; j++)
+#pragma unroll
+    for (int k = 0; k < kDIters; k++) {
+      const size_t e = size_t(g0 + k * kThreads) * 4;
+      global_ptr<uint8_t> pay = as_global(s_pay[j0 + j]);
+      if (B == 1) raw[j][k] = (uint32_t(pay[e >> 3]) >> (e & 4)) & 0xFu;
+      else if (B == 4) raw[j][k] = reinterpret_cast<global_ptr<u16u>>(pay + (e >> 1))->v;
+      else raw[j][k] = reinterpret_cast<global_ptr<u32u>>(pay + e)->v;
+    }
+#pragma unroll
+  for (int j = 0; j < NS; j++) {
+    const float gap = s_gap[j0 + j], mn = s_mn[j0 + j];
+    const bool add = s_add[j0 + j] != 0;
+#pragma unroll
+    for (int k = 0; k < kDIters; k++) {
+      const float4 v = group_values<B>(raw[j][k], gap, mn);
+      acc[k].x = add ? v.x + acc[k].x : v.x; acc[k].y = add ? v.y + acc[k].y : v.y;
+      acc[k].z = add ? v.z + acc[k].z : v.z; acc[k].w = add ? v.w + acc[k].w : v.w;
+    }
+  }
+}
+// A whole sub-tile of complete messages of one width other than 2 bits.
+template <int B>
+__device__ __forceinline__ void decode_whole(float* __restrict__ op, bool need_old, uint32_t g0, int ns, const uint8_t* const* s_pay,
+                                             const float* s_gap, const float* s_mn, const int32_t* s_add) {
+  float4 acc[kDIters];
+#pragma unroll
+  for (int k = 0; k < kDIters; k++) acc[k] = need_old ? ld4_stream(op + size_t(g0 + k * kThreads) * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int j0 = 0; j0 < ns; j0 += 4) {
+    switch (ns - j0) {
+      case 1: fold_messages<B, 1>(acc, g0, j0, s_pay, s_gap, s_mn, s_add); break;
+      case 2: fold_messages<B, 2>(acc, g0, j0, s_pay, s_gap, s_mn, s_add); break;
+      case 3: fold_messages<B, 3>(acc, g0, j0, s_pay, s_gap, s_mn, s_add); break;
+      default: fold_messages<B, 4>(acc, g0, j0, s_pay, s_gap, s_mn, s_add); break;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kDIters; k++) {
+    st4_stream(op + size_t(g0 + k * kThreads) * 4, acc[k]);
+    __asm__ volatile("" ::: "memory");
+  }
+}
+
 template <typename Args>
 __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const Args a) {
   __shared__ float s_mn[kMultiSlotsPerSeg], s_gap[kMultiSlotsPerSeg];
@@ -1639,23 +1824,27 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const A
   for (int j = 0; j < ns; j++) all_cover = all_cover && s_cnt[j] == n;
   bool all_two_bit = true;  // ... and is a 2-bit message (the configuration the reference ships with)
   for (int j = 0; j < ns; j++) all_two_bit = all_two_bit && s_bits[j] == 2u;
-  // The headers are parsed once per workgroup and serve kMultiRep consecutive sub-tiles.
+  const uint32_t width = s_bits[0];
+  bool one_width = true;    // ... or of one width, whichever it is
+  for (int j = 1; j < ns; j++) one_width = one_width && s_bits[j] == width;
+  // The headers are parsed once per workgroup and serve `reps` consecutive sub-tiles.
+  const uint32_t reps = static_cast<uint32_t>(a.reps);
   uint32_t rep_begin = 0;
   if (all_cover && all_two_bit && ns <= 8) {
-    const uint32_t sub0 = static_cast<uint32_t>(tile - a.tile_start[s]) * kMultiRep;
+    const uint32_t sub0 = static_cast<uint32_t>(tile - a.tile_start[s]) * reps;
     switch (ns) {  // the number of messages as a compile-time constant: straight-line code, all loads of a sub-tile in flight together
-      case 2: rep_begin = decode_two_bit_whole<2>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
-      case 3: rep_begin = decode_two_bit_whole<3>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
-      case 4: rep_begin = decode_two_bit_whole<4>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
-      case 5: rep_begin = decode_two_bit_whole<5>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
-      case 6: rep_begin = decode_two_bit_whole<6>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
-      case 7: rep_begin = decode_two_bit_whole<7>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
-      case 8: rep_begin = decode_two_bit_whole<8>(op, n, need_old, sub0, s_pay, s_gap, s_mn, s_add); break;
+      case 2: rep_begin = decode_two_bit_whole<2>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
+      case 3: rep_begin = decode_two_bit_whole<3>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
+      case 4: rep_begin = decode_two_bit_whole<4>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
+      case 5: rep_begin = decode_two_bit_whole<5>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
+      case 6: rep_begin = decode_two_bit_whole<6>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
+      case 7: rep_begin = decode_two_bit_whole<7>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
+      case 8: rep_begin = decode_two_bit_whole<8>(op, n, need_old, sub0, reps, s_pay, s_gap, s_mn, s_add); break;
       default: break;
     }
   }
-  for (uint32_t rep = rep_begin; rep < uint32_t(kMultiRep); rep++) {
-  const uint32_t g0 = (static_cast<uint32_t>(tile - a.tile_start[s]) * kMultiRep + rep) * uint32_t(kThreads * kDIters) + threadIdx.x;
+  for (uint32_t rep = rep_begin; rep < reps; rep++) {
+  const uint32_t g0 = (static_cast<uint32_t>(tile - a.tile_start[s]) * reps + rep) * uint32_t(kThreads * kDIters) + threadIdx.x;
   if (uint64_t(g0 - threadIdx.x) * 4 >= n) break;
   if (all_cover && all_two_bit && uint64_t(g0 - threadIdx.x + kThreads * kDIters) * 4 <= n) {
     // Whole tile of complete 2-bit messages.  A wave owns kDIters * 64 consecutive groups, i.e. that many
@@ -1702,8 +1891,14 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const A
     }
     continue;
   }
+  if (all_cover && one_width && uint64_t(g0 - threadIdx.x + kThreads * kDIters) * 4 <= n) {
+    if (width == 1) decode_whole<1>(op, need_old, g0, ns, s_pay, s_gap, s_mn, s_add);
+    else if (width == 4) decode_whole<4>(op, need_old, g0, ns, s_pay, s_gap, s_mn, s_add);
+    else decode_whole<8>(op, need_old, g0, ns, s_pay, s_gap, s_mn, s_add);
+    continue;
+  }
   if (all_cover && uint64_t(g0 - threadIdx.x + kThreads * kDIters) * 4 <= n) {
-    // Whole tile, every message complete, other widths: old values and the code bytes of up to 4 messages x 4
+    // Whole tile, every message complete, mixed widths: old values and the code bytes of up to 4 messages x 4
     // groups are requested together, then folded in message order.
     float4 acc[kDIters];
 #pragma unroll
@@ -2096,6 +2291,14 @@ int launch_resident(const ResArgs& ra, int num_cus, hipStream_t st) {
   }
 }
 
+// Whether every tensor of a call is one workgroup's work.  (Beside a larger tensor small ones go through its two
+// launches: a third would cost more than it saves.)
+bool all_small(int count, const int32_t* in_sizes) {
+  for (int i = 0; i < count; i++)
+    if (in_sizes[i] > kSmallMax) return false;
+  return true;
+}
+
 template <int CAP>
 int launch_encode(int count, const float* const* ins, const int32_t* in_sizes, uint8_t* const* outs,
                   const int32_t* out_sizes, const uint8_t* bitwidths, const int32_t* enable_randoms,
@@ -2104,6 +2307,19 @@ int launch_encode(int count, const float* const* ins, const int32_t* in_sizes, u
   const bool prof = timed && hpx::g_prof_on;
   EncArgs<CAP> a;
   int i = 0;
+  if (all_small(count, in_sizes)) {
+    while (i < count) {
+      a.nseg = 0;
+      for (; i < count && a.nseg < CAP; i++) {
+        const uint64_t seed = seeds ? seeds[i] : hpx::clock_seed();
+        a.seg[a.nseg++] = EncSeg{ins[i], outs[i], in_sizes[i], out_sizes[i], static_cast<uint32_t>(seed), bitwidths[i],
+                                 static_cast<uint8_t>(enable_randoms[i] != 0), 0};
+      }
+      HPX_LAUNCH_LDS("terngrad_small_kernel", prof, terngrad_small_kernel<CAP>, dim3(a.nseg), dim3(kSmallThreads), 0, st, a);
+      HPX_HIP(hipGetLastError());
+    }
+    return HPX_OK;
+  }
   while (i < count) {
     const int first = i;
     a.nseg = 0;
@@ -2213,18 +2429,22 @@ std::vector<MultiGroup> plan_multi_launch(int count, float* const* outs, const i
 }
 
 int launch_decode_multi(int count, float* const* outs, const int32_t* out_sizes, const uint8_t* const* ins,
-                        const int32_t* in_sizes, const int32_t* is_add_tos, uint32_t* status, hipStream_t st) {
+                        const int32_t* in_sizes, const int32_t* is_add_tos, int period, uint32_t* status, hipStream_t st) {
+  // period > 0: message j is for the tensor of message j - period (classify_outputs)
   std::vector<char> done(count, 0);
   int left = 0;
   for (int j = 0; j < count; j++) {
     HPX_ARG(out_sizes[j] >= 0 && in_sizes[j] >= 10, "hpx_terngrad_decode: message %d: out_size %d, in_size %d", j,
             out_sizes[j], in_sizes[j]);
-    if (out_sizes[j] == 0) { done[j] = 1; continue; }
+    if (out_sizes[j] == 0) { done[j] = 1; period = 0; continue; }
     HPX_ARG(outs[j] && ins[j], "hpx_terngrad_decode: message %d has a null pointer", j);
     left++;
   }
   if (left == 0) return HPX_OK;
-  auto tiles_of = [](int32_t n) { return ceil_div(n, kDecTile * kMultiRep); };
+  // A workgroup takes several sub-tiles where there are plenty: 3 M elements in 24 tensors (732 sub-tiles) left most of the
+  // chip idle at four each.
+  auto reps_for = [](int64_t sub_tiles) { return sub_tiles >= kMultiFull * kMultiRep ? kMultiRep : sub_tiles >= kMultiFull * 2 ? 2 : 1; };
+  auto tiles_of = [](int32_t n, int reps) { return ceil_div(n, int64_t(kDecTile) * reps); };
   {
     // The fixed-distance form when the whole call fits it: at most kStrideSegs tensors, every tensor's messages (in
     // call order) at one distance from each other, of one size, and all but the first added.
@@ -2236,30 +2456,39 @@ int launch_decode_multi(int count, float* const* outs, const int32_t* out_sizes,
     bool fits = true;
     for (int j = 0; j < count && fits; j++) {
       if (out_sizes[j] == 0) continue;
-      auto it = index.find(outs[j]);
-      if (it == index.end()) {
+      int at = -1;   // the tensor's place in the table
+      if (period > 0) {
+        at = j < period ? -1 : j % period;
+      } else {
+        auto it = index.find(outs[j]);
+        if (it != index.end()) at = it->second;
+      }
+      if (at < 0) {
         if (sa.nseg == kStrideSegs) { fits = false; break; }
-        index[outs[j]] = sa.nseg;
+        if (period == 0) index[outs[j]] = sa.nseg;
         sa.seg[sa.nseg] = SSeg{outs[j], ins[j], 0, out_sizes[j], in_sizes[j], 1, int16_t(is_add_tos[j] != 0), -1, 0};
         last[sa.nseg] = ins[j];
         sa.nseg++;
         continue;
       }
-      SSeg& g = sa.seg[it->second];
-      const int64_t step = static_cast<int64_t>(reinterpret_cast<intptr_t>(ins[j]) - reinterpret_cast<intptr_t>(last[it->second]));  // addresses, not elements of one array
+      SSeg& g = sa.seg[at];
+      const int64_t step = static_cast<int64_t>(reinterpret_cast<intptr_t>(ins[j]) - reinterpret_cast<intptr_t>(last[at]));  // addresses, not elements of one array
       if (g.nslots == kMultiSlotsPerSeg || is_add_tos[j] == 0 || in_sizes[j] != g.in_size || out_sizes[j] != g.out_size) fits = false;
       else if (g.nslots == 1) g.stride = step;
       else if (step == g.stride) {}
       else if (g.skip < 0 && step == 2 * g.stride) g.skip = g.nslots;                                   // the gap
       else if (g.skip < 0 && g.nslots == 2 && 2 * step == g.stride) { g.stride = step; g.skip = 1; }    // the gap came first
       else fits = false;
-      last[it->second] = ins[j];
+      last[at] = ins[j];
       g.nslots++;
     }
     int64_t tiles = 0;
+    for (int k = 0; k < sa.nseg; k++) tiles += tiles_of(sa.seg[k].out_size, 1);
+    sa.reps = reps_for(tiles);
+    tiles = 0;
     sa.tile_start[0] = 0;
     for (int k = 0; k < sa.nseg && fits; k++) {
-      tiles += tiles_of(sa.seg[k].out_size);
+      tiles += tiles_of(sa.seg[k].out_size, sa.reps);
       if (tiles > INT32_MAX) fits = false;
       sa.tile_start[k + 1] = int32_t(tiles);
     }
@@ -2272,14 +2501,17 @@ int launch_decode_multi(int count, float* const* outs, const int32_t* out_sizes,
   MArgs a;
   a.status = status;
   while (left > 0) {
-    const std::vector<MultiGroup> groups = plan_multi_launch(count, outs, out_sizes, done, tiles_of);
+    const std::vector<MultiGroup> groups = plan_multi_launch(count, outs, out_sizes, done, [&](int32_t n) { return tiles_of(n, 1); });
+    int64_t sub_tiles = 0;
+    for (const MultiGroup& g : groups) sub_tiles += tiles_of(g.n, 1);
+    a.reps = reps_for(sub_tiles);
     a.nseg = 0;
     a.tile_start[0] = 0;
     int nslots = 0;
     for (const MultiGroup& g : groups) {
       a.seg[a.nseg] = MSeg{g.out, g.n, nslots, static_cast<int32_t>(g.msgs.size()), 0};
       for (int m : g.msgs) a.slot[nslots++] = MSlot{ins[m], in_sizes[m], is_add_tos[m] != 0};
-      a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + tiles_of(g.n);
+      a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + tiles_of(g.n, a.reps);
       a.nseg++;
     }
     if (nslots == 0) { hpx::set_error("hpx_terngrad_decode: could not place the remaining messages"); return HPX_ERR_ARG; }
@@ -2585,7 +2817,8 @@ HPX_API int hpx_terngrad_encode_noalloc(int count, const float* const* ins, cons
   // kernel, not a memset node, so that the sequence can be recorded into a graph), and the epoch tag is
   // a constant.
   const uint32_t words = uint32_t(count) * kSlotsPerTensor;
-  hipLaunchKernelGGL(terngrad_scratch_clear_kernel, dim3((words + kThreads - 1) / kThreads), dim3(kThreads), 0, st, slots, words);
+  if (!all_small(count, in_sizes))   // those use no slots
+    hipLaunchKernelGGL(terngrad_scratch_clear_kernel, dim3((words + kThreads - 1) / kThreads), dim3(kThreads), 0, st, slots, words);
   HPX_HIP(hipGetLastError());
   if (count <= kCapSmall)
     return launch_encode<kCapSmall>(count, ins, in_sizes, outs, out_sizes, bitwidths, enable_randoms, seeds,
@@ -2637,10 +2870,11 @@ HPX_API int hpx_terngrad_decode(int count, float* const* outs, const int32_t* ou
   int rc = hpx::ensure_workspace(ws, 0);
   if (rc != HPX_OK) return rc;
   uint32_t* status = ws->state + hpx::kStatusWord;
-  switch (hpx::classify_outputs(count, outs, out_sizes)) {
+  int period = 0;
+  switch (hpx::classify_outputs(count, outs, out_sizes, &period)) {
     case 0: break;
     case 1:  // several messages accumulate into the same tensor(s): one pass per tensor
-      return launch_decode_multi(count, outs, out_sizes, ins, in_sizes, is_add_tos, status, st);
+      return launch_decode_multi(count, outs, out_sizes, ins, in_sizes, is_add_tos, period, status, st);
     default: {  // partially overlapping outputs: keep the reference's one-message-at-a-time order
       for (int i = 0; i < count; i++) {
         const int rc1 = launch_decode<kCapSmall>(1, outs + i, out_sizes + i, ins + i, in_sizes + i, is_add_tos + i, status, st);
