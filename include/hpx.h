@@ -114,6 +114,19 @@ int hpx_release_stream(hpx_stream_t stream);
 int hpx_set_option(const char* name, int64_t value);
 int hpx_get_option(const char* name, int64_t* value);
 
+/* ---- waiting for a call -----------------------------------------------------
+ * No counterpart in the reference, whose drivers end with cudaStreamSynchronize.
+ * A caller that waits for the calls it makes brackets them: kernels the calling
+ * thread launches through this library after hpx_completion_begin carry an event
+ * of their own, and hpx_completion_wait returns when the last of them - and with
+ * it all that was queued before it on its stream - has finished (waits for the
+ * whole stream where none was launched).  Same meaning as waiting for the stream,
+ * without the marker that hipStreamSynchronize queues behind the kernels: 2 us
+ * less per call.  All calls in between go to one stream, the one handed to
+ * hpx_completion_wait. */
+int hpx_completion_begin(void);
+int hpx_completion_wait(hpx_stream_t stream);
+
 /* ---- measurement aid ------------------------------------------------------
  * No counterpart in the reference.  While enabled, every kernel the library
  * launches carries a pair of HIP events that take the kernel's own begin and

@@ -19,6 +19,8 @@ SYMBOLS = (
     "hpx_release_stream",
     "hpx_set_option",
     "hpx_get_option",
+    "hpx_completion_begin",
+    "hpx_completion_wait",
     "hpx_profile_enable",
     "hpx_profile_reset",
     "hpx_profile_query",
@@ -91,6 +93,7 @@ def load():
     L.hpx_version.restype = C.c_int
     L.hpx_last_error.restype = C.c_char_p
     L.hpx_release_workspaces.restype = C.c_int
+    L.hpx_completion_wait.argtypes = [p]
     L.hpx_profile_enable.argtypes = [C.c_int]
     L.hpx_profile_query.argtypes = [C.c_char_p, C.POINTER(C.c_double), C.POINTER(C.c_int64)]
     L.hpx_set_option.argtypes = [C.c_char_p, C.c_int64]

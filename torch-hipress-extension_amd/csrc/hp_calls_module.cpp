@@ -135,14 +135,14 @@ PyObject* released(F&& call) {
 // The call, then a wait for the stream (hp_cuda_kernel.cu:157, :197).
 template <typename F>
 PyObject* released_and_waited(hipStream_t st, F&& call) {
-  int rc;
-  hipError_t e;
+  int rc, waited;
   Py_BEGIN_ALLOW_THREADS
+  const int begun = hpx_completion_begin();
   rc = call();
-  e = hipStreamSynchronize(st);
+  waited = begun == HPX_OK ? hpx_completion_wait(st) : begun;
   Py_END_ALLOW_THREADS
-  if (e != hipSuccess) {
-    PyErr_Format(PyExc_RuntimeError, "HIP error: %s", hipGetErrorString(e));
+  if (waited != HPX_OK) {
+    PyErr_Format(PyExc_RuntimeError, "HIP error: %s", hpx_last_error());
     throw PyError{};
   }
   return PyLong_FromLong(rc);

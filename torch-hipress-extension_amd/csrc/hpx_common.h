@@ -40,6 +40,11 @@ extern bool g_prof_on;
 // A new record under `name` and its two events, not yet recorded.
 void prof_events(const char* name, hipEvent_t* start, hipEvent_t* stop);
 
+// What a caller waits for between hpx_completion_begin and hpx_completion_wait: while `t_stop` is set every launch of
+// this thread carries that event, so the last of them leaves it.
+extern thread_local hipEvent_t t_stop;
+extern thread_local bool t_stop_used;
+
 // Every kernel goes out through these macros.  With hpx_profile_enable(1) a launch carries two HIP events that
 // take the kernel's own begin and end times (hipExtLaunchKernelGGL), so hpx_profile_query reports the durations a
 // kernel trace shows; events recorded on the stream around a launch would add the hand-over between launches
@@ -50,6 +55,9 @@ void prof_events(const char* name, hipEvent_t* start, hipEvent_t* stop);
       hipEvent_t hpx_e0_ = nullptr, hpx_e1_ = nullptr;                                           \
       hpx::prof_events(NAME, &hpx_e0_, &hpx_e1_);                                                \
       hipExtLaunchKernelGGL(KERNEL, GRID, BLOCK, LDS, STREAM, hpx_e0_, hpx_e1_, 0, __VA_ARGS__); \
+    } else if (hpx::t_stop) {                                                                    \
+      hpx::t_stop_used = true;                                                                   \
+      hipExtLaunchKernelGGL(KERNEL, GRID, BLOCK, LDS, STREAM, nullptr, hpx::t_stop, 0, __VA_ARGS__); \
     } else {                                                                                     \
       hipLaunchKernelGGL(KERNEL, GRID, BLOCK, LDS, STREAM, __VA_ARGS__);                         \
     }                                                                                            \

@@ -81,6 +81,14 @@ int ensure_aux(Workspace* ws, size_t bytes) {
 
 // ---- per-kernel timing --------------------------------------------------------
 bool g_prof_on = false;
+thread_local hipEvent_t t_stop = nullptr;
+thread_local bool t_stop_used = false;
+namespace {
+// Events not in use, per device; as many exist as threads have waited at once.
+std::mutex g_stop_mu;
+std::map<int, std::vector<hipEvent_t>> g_stop_pool;
+thread_local int t_stop_device = 0;
+}  // namespace
 namespace {
 struct ProfRec {
   const char* name;
@@ -396,6 +404,40 @@ HPX_API int hpx_get_option(const char* name, int64_t* value) {
   HPX_ARG(i >= 0, "hpx_get_option: unknown option '%s'", name);
   *value = hpx::g_opt[i].load();
   return HPX_OK;
+}
+
+HPX_API int hpx_completion_begin(void) {
+  hpx::clear_error();
+  HPX_ARG(hpx::t_stop == nullptr, "hpx_completion_begin: the thread has not waited for its last one");
+  int device = 0;
+  HPX_HIP(hipGetDevice(&device));
+  hipEvent_t e = nullptr;
+  {
+    std::lock_guard<std::mutex> g(hpx::g_stop_mu);
+    auto& pool = hpx::g_stop_pool[device];
+    if (!pool.empty()) {
+      e = pool.back();
+      pool.pop_back();
+    }
+  }
+  if (!e) HPX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  hpx::t_stop = e;
+  hpx::t_stop_used = false;
+  hpx::t_stop_device = device;
+  return HPX_OK;
+}
+
+HPX_API int hpx_completion_wait(hpx_stream_t stream) {
+  const hipEvent_t e = hpx::t_stop;
+  hpx::t_stop = nullptr;
+  const hipError_t rc = e && hpx::t_stop_used ? hipEventSynchronize(e) : hipStreamSynchronize(static_cast<hipStream_t>(stream));
+  if (e) {
+    std::lock_guard<std::mutex> g(hpx::g_stop_mu);
+    hpx::g_stop_pool[hpx::t_stop_device].push_back(e);
+  }
+  if (rc == hipSuccess) return HPX_OK;
+  hpx::set_error("hpx_completion_wait: %s", hipGetErrorString(rc));
+  return HPX_ERR_HIP;
 }
 
 HPX_API int hpx_profile_enable(int on) {

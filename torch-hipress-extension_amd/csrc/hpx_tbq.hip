@@ -592,30 +592,36 @@ std::vector<MultiGroup> plan_multi_launch(int count, float* const* outs, const i
 // tensor's messages (in call order) at one distance from each other, with one threshold, and all but the first
 // added.  Arguments have been checked.
 bool plan_strided(int count, float* const* outs, const int32_t* sizes, const uint8_t* const* ins, const float* thresholds,
-                  const int32_t* is_add_tos, SArgs& a) {
-  std::unordered_map<float*, int> index;
+                  const int32_t* is_add_tos, int period, SArgs& a) {
+  std::unordered_map<float*, int> index;   // unused where the list repeats its first `period` tensors (classify_outputs)
   std::vector<const uint8_t*> last(kStrideSegs, nullptr);
   a.nseg = 0;
   for (int j = 0; j < count; j++) {
     if (sizes[j] == 0) continue;
-    auto it = index.find(outs[j]);
-    if (it == index.end()) {
+    int at = -1;   // the tensor's place in the table
+    if (period > 0) {
+      at = j < period ? -1 : j % period;
+    } else {
+      auto it = index.find(outs[j]);
+      if (it != index.end()) at = it->second;
+    }
+    if (at < 0) {
       if (a.nseg == kStrideSegs) return false;
-      index[outs[j]] = a.nseg;
+      if (period == 0) index[outs[j]] = a.nseg;
       a.seg[a.nseg] = SSeg{outs[j], ins[j], 0, sizes[j], thresholds[j], 1, int16_t(is_add_tos[j] != 0), -1, 0};
       last[a.nseg] = ins[j];
       a.nseg++;
       continue;
     }
-    SSeg& g = a.seg[it->second];
-    const int64_t step = static_cast<int64_t>(reinterpret_cast<intptr_t>(ins[j]) - reinterpret_cast<intptr_t>(last[it->second]));  // addresses, not elements of one array
+    SSeg& g = a.seg[at];
+    const int64_t step = static_cast<int64_t>(reinterpret_cast<intptr_t>(ins[j]) - reinterpret_cast<intptr_t>(last[at]));  // addresses, not elements of one array
     if (g.nslots == kMultiSlotsPerSeg || is_add_tos[j] == 0 || thresholds[j] != g.thr || sizes[j] != g.n) return false;
     if (g.nslots == 1) g.stride = step;
     else if (step == g.stride) {}
     else if (g.skip < 0 && step == 2 * g.stride) g.skip = g.nslots;                                   // the gap
     else if (g.skip < 0 && g.nslots == 2 && 2 * step == g.stride) { g.stride = step; g.skip = 1; }    // the gap came first
     else return false;
-    last[it->second] = ins[j];
+    last[at] = ins[j];
     g.nslots++;
   }
   int64_t tiles = 0;
@@ -629,19 +635,19 @@ bool plan_strided(int count, float* const* outs, const int32_t* sizes, const uin
 }
 
 int launch_decode_multi(int count, float* const* outs, const int32_t* sizes, const uint8_t* const* ins,
-                        const float* thresholds, const int32_t* is_add_tos, hipStream_t st) {
+                        const float* thresholds, const int32_t* is_add_tos, int period, hipStream_t st) {
   std::vector<char> done(count, 0);
   int left = 0;
   for (int j = 0; j < count; j++) {
     HPX_ARG(sizes[j] >= 0, "hpx_tbq_decode: tensor %d has negative size %d", j, sizes[j]);
-    if (sizes[j] == 0) { done[j] = 1; continue; }
+    if (sizes[j] == 0) { done[j] = 1; period = 0; continue; }
     HPX_ARG(outs[j] && ins[j], "hpx_tbq_decode: tensor %d has a null pointer", j);
     left++;
   }
   if (left == 0) return HPX_OK;
   {
     SArgs sa;
-    if (plan_strided(count, outs, sizes, ins, thresholds, is_add_tos, sa)) {
+    if (plan_strided(count, outs, sizes, ins, thresholds, is_add_tos, period, sa)) {
       HPX_LAUNCH("tbq_decode_multi_kernel", tbq_decode_multi_kernel<SArgs>, dim3(sa.tile_start[sa.nseg]), dim3(kThreads), st, sa);
       HPX_HIP(hipGetLastError());
       return HPX_OK;
@@ -689,10 +695,11 @@ HPX_API int hpx_tbq_decode(int count, float* const* outs, const int32_t* sizes,
   if (count == 0) return HPX_OK;
   HPX_ARG(outs && sizes && ins && thresholds && is_add_tos, "hpx_tbq_decode: null argument array");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  switch (hpx::classify_outputs(count, outs, sizes)) {
+  int period = 0;
+  switch (hpx::classify_outputs(count, outs, sizes, &period)) {
     case 0: break;
     case 1:  // several messages accumulate into the same tensor(s): one pass per tensor
-      return launch_decode_multi(count, outs, sizes, ins, thresholds, is_add_tos, st);
+      return launch_decode_multi(count, outs, sizes, ins, thresholds, is_add_tos, period, st);
     default: {  // partially overlapping outputs: keep the reference's one-message-at-a-time order
       for (int i = 0; i < count; i++) {
         const int rc = launch_decode<kCapSmall>(1, outs + i, sizes + i, ins + i, thresholds + i, is_add_tos + i, st);
