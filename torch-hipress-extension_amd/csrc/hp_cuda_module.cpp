@@ -19,6 +19,9 @@
 // its streams; here tensors are only checked and turned into pointers.
 #include <torch/extension.h>
 
+#include <array>
+#include <atomic>
+#include <climits>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -28,8 +31,9 @@
 
 namespace {
 
+using Kept = std::array<torch::Tensor, 5>;
 std::mutex g_mu;
-std::unordered_map<uint64_t, std::vector<torch::Tensor>> g_in_flight;  // serial -> tensors of a task
+std::unordered_map<uint64_t, Kept> g_in_flight;  // serial -> tensors of a task
 
 void check_device_input(const torch::Tensor& x, const char* what) {
   TORCH_CHECK(x.is_cuda(), what, " must be a CUDA tensor");
@@ -53,9 +57,13 @@ void release_done() {
   }
 }
 
-bool submit(const std::string& name, hpx_task_t& t, std::vector<torch::Tensor> keep) {
-  release_done();
-  t.name = name.c_str();
+// Finished tasks are looked for once in so many submissions, and whenever results are asked for.
+constexpr unsigned kReleaseEvery = 64;
+
+bool submit(const char* name, hpx_task_t& t, Kept keep) {
+  static std::atomic<unsigned> submitted{0};
+  if (++submitted % kReleaseEvery == 0) release_done();
+  t.name = name;
   uint64_t serial = 0;
   if (hpx_sched_submit(&t, &serial) != 0) {
     const std::string text = hpx_sched_error();
@@ -89,70 +97,113 @@ bool end() {
   return true;
 }
 
-bool submit_task_without_residual(const std::string& name, torch::Tensor tensor, torch::Tensor B, torch::Tensor C,
-                                  int is_root, int task_id) {
-  check_device_input(tensor, "tensor");
-  check_device_input(B, "B");
-  check_host_input(C, "C");
-  hpx_task_t t{};
-  t.task_id = task_id;
-  t.is_root = is_root;
-  t.tensor = static_cast<float*>(tensor.data_ptr());
-  t.tensor_numel = tensor.numel();
-  t.B = static_cast<uint8_t*>(B.data_ptr());
-  t.B_bytes = B.numel() * B.element_size();
-  t.C = static_cast<uint8_t*>(C.data_ptr());
-  t.C_bytes = C.numel() * C.element_size();
-  return submit(name, t, {tensor, B, C});
+// submit_task, all three forms.  A caller hands over a model's tensors one by one, so what a call costs is what decides
+// when the last of them can start: read from the argument vector directly it is about 0.3 us, through an overload
+// set with converted copies of every argument it was 0.9, more than the link needs for the average message.
+struct PyError {};
+
+const torch::Tensor& tensor_arg(PyObject* o, const char* what) {
+  if (THPVariable_Check(o)) return THPVariable_Unpack(o);
+  PyErr_Format(PyExc_TypeError, "submit_task(): incompatible function arguments: %s must be a tensor", what);
+  throw PyError{};
+}
+int int_arg(PyObject* o, const char* what) {
+  PyObject* i = PyNumber_Index(o);
+  if (!i) {
+    PyErr_Format(PyExc_TypeError, "submit_task(): incompatible function arguments: %s must be an integer", what);
+    throw PyError{};
+  }
+  int overflow = 0;
+  const long v = PyLong_AsLongAndOverflow(i, &overflow);
+  Py_DECREF(i);
+  if (overflow || v < INT_MIN || v > INT_MAX) {
+    PyErr_Format(PyExc_TypeError, "submit_task(): incompatible function arguments: %s is out of range", what);
+    throw PyError{};
+  }
+  return static_cast<int>(v);
 }
 
-bool submit_task_with_residual(const std::string& name, torch::Tensor tensor, torch::Tensor residual, torch::Tensor B,
-                               torch::Tensor C, int is_root, int task_id) {
+void set_tensor(hpx_task_t& t, const torch::Tensor& tensor) {
   check_device_input(tensor, "tensor");
-  check_device_input(residual, "residual");
-  check_device_input(B, "B");
-  check_host_input(C, "C");
-  hpx_task_t t{};
-  t.task_id = task_id;
-  t.is_root = is_root;
   t.tensor = static_cast<float*>(tensor.data_ptr());
   t.tensor_numel = tensor.numel();
+}
+void set_residual(hpx_task_t& t, const torch::Tensor& residual) {
+  check_device_input(residual, "residual");
   t.residual = static_cast<float*>(residual.data_ptr());
   t.residual_numel = residual.numel();
+}
+void set_message(hpx_task_t& t, const torch::Tensor& B, const torch::Tensor& C) {
+  check_device_input(B, "B");
+  check_host_input(C, "C");
   t.B = static_cast<uint8_t*>(B.data_ptr());
   t.B_bytes = B.numel() * B.element_size();
   t.C = static_cast<uint8_t*>(C.data_ptr());
   t.C_bytes = C.numel() * C.element_size();
+}
+
+bool submit_args(PyObject* const* a, Py_ssize_t n) {
+  if (n != 6 && n != 7) {
+    PyErr_SetString(PyExc_TypeError, "submit_task(): incompatible function arguments");
+    throw PyError{};
+  }
+  const char* name = PyUnicode_Check(a[0]) ? PyUnicode_AsUTF8(a[0]) : nullptr;
+  if (!name) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "submit_task(): incompatible function arguments: the name must be a string");
+    throw PyError{};
+  }
+  hpx_task_t t{};
+  if (n == 7 && THPVariable_Check(a[5])) {  // (name, tensor, residual, M, P, Q, task_id)
+    const torch::Tensor &tensor = tensor_arg(a[1], "tensor"), &residual = tensor_arg(a[2], "residual"), &M = tensor_arg(a[3], "M"),
+                        &P = tensor_arg(a[4], "P"), &Q = tensor_arg(a[5], "Q");
+    t.task_id = int_arg(a[6], "task_id");
+    set_tensor(t, tensor);
+    set_residual(t, residual);
+    check_device_input(M, "M");
+    check_device_input(P, "P");
+    check_device_input(Q, "Q");
+    TORCH_CHECK(M.dim() == 2 && P.dim() == 2 && Q.dim() == 2, "M, P and Q must be matrices");
+    t.M = static_cast<float*>(M.data_ptr());
+    t.P = static_cast<float*>(P.data_ptr());
+    t.Q = static_cast<float*>(Q.data_ptr());
+    t.n = static_cast<int32_t>(M.size(0));
+    t.m = static_cast<int32_t>(M.size(1));
+    t.r = static_cast<int32_t>(P.size(1));
+    return submit(name, t, {tensor, residual, M, P, Q});
+  }
+  const bool has_residual = n == 7;  // (name, tensor, [residual,] B, C, is_root, task_id)
+  PyObject* const* b = a + (has_residual ? 3 : 2);
+  const torch::Tensor &tensor = tensor_arg(a[1], "tensor"), &B = tensor_arg(b[0], "B"), &C = tensor_arg(b[1], "C");
+  t.is_root = int_arg(b[2], "is_root");
+  t.task_id = int_arg(b[3], "task_id");
+  set_tensor(t, tensor);
+  if (!has_residual) {
+    set_message(t, B, C);
+    return submit(name, t, {tensor, B, C});
+  }
+  const torch::Tensor& residual = tensor_arg(a[2], "residual");
+  set_residual(t, residual);
+  set_message(t, B, C);
   return submit(name, t, {tensor, residual, B, C});
 }
 
-bool submit_task_for_powersgd(const std::string& name, torch::Tensor tensor, torch::Tensor residual, torch::Tensor M,
-                              torch::Tensor P, torch::Tensor Q, int task_id) {
-  check_device_input(tensor, "tensor");
-  check_device_input(residual, "residual");
-  check_device_input(M, "M");
-  check_device_input(P, "P");
-  check_device_input(Q, "Q");
-  TORCH_CHECK(M.dim() == 2 && P.dim() == 2 && Q.dim() == 2, "M, P and Q must be matrices");
-  hpx_task_t t{};
-  t.task_id = task_id;
-  t.is_root = 0;
-  t.tensor = static_cast<float*>(tensor.data_ptr());
-  t.tensor_numel = tensor.numel();
-  t.residual = static_cast<float*>(residual.data_ptr());
-  t.residual_numel = residual.numel();
-  t.M = static_cast<float*>(M.data_ptr());
-  t.P = static_cast<float*>(P.data_ptr());
-  t.Q = static_cast<float*>(Q.data_ptr());
-  t.n = static_cast<int32_t>(M.size(0));
-  t.m = static_cast<int32_t>(M.size(1));
-  t.r = static_cast<int32_t>(P.size(1));
-  return submit(name, t, {tensor, residual, M, P, Q});
+PyObject* submit_task(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  try {
+    return PyBool_FromLong(submit_args(args, nargs));
+  } catch (const PyError&) {
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+  }
+  return nullptr;
 }
+PyMethodDef g_submit_task = {"submit_task", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&submit_task)), METH_FASTCALL,
+                             "submit_task(name, tensor, B, C, is_root, task_id)\n"
+                             "submit_task(name, tensor, residual, B, C, is_root, task_id)\n"
+                             "submit_task(name, tensor, residual, M, P, Q, task_id)\n\nFalse, with the reason printed, if the task is refused."};
 
 std::vector<std::string> get_results(int task_id) {
   std::vector<std::string> out;
-  std::vector<char> buf(1 << 16);
+  static thread_local std::vector<char> buf(1 << 16);
   for (;;) {
     const int64_t n = hpx_sched_get_results(task_id, buf.data(), static_cast<int64_t>(buf.size()));
     if (n <= 0) break;  // negative: the library has printed the reference's message
@@ -178,9 +229,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("init", &init, "init");
   m.def("end", &end, "end");
   m.def("getResults", &get_results, "get results");
-  m.def("submit_task", &submit_task_without_residual, "submit task without residual");
-  m.def("submit_task", &submit_task_with_residual, "submit task with residual");
-  m.def("submit_task", &submit_task_for_powersgd, "submit task for powersgd");
+  m.add_object("submit_task", pybind11::reinterpret_steal<pybind11::object>(PyCFunction_NewEx(&g_submit_task, nullptr, m.attr("__name__").ptr())));
   m.def("wait", &wait_for, pybind11::arg("task_id"), pybind11::arg("timeout_ms") = 1000,
         "block until getResults(task_id) would return something (True) or the time is up (False)");
   m.def("error_count", []() { return hpx_sched_error_count(); });

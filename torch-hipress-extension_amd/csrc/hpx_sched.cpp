@@ -1,17 +1,26 @@
 // Task scheduler over the codecs of hpx.h (see include/hpx_sched.h for what it
 // replaces and what it does differently).
 //
-// One worker thread owns a compute stream and a data stream.  It sleeps on a
+// One worker thread owns two streams, the lanes.  It sleeps on a
 // condition variable, takes everything that is queued as one batch (like
 // TaskQueue::GetTasksFromQueue, hp_cuda.cpp:122-133) and turns the batch into a
 // few multi-tensor codec calls.  Transfers and codec calls are cut into runs of
-// growing size (1 MB of messages, then 2, 4 ... 16 MB) so that the link and the
-// kernels work at the same time:
+// growing size (1 MB of messages, then 2, 4 ... 16 MB), and the runs are dealt out to the
+// lanes in turn, so that the link and the kernels work at the same time:
 //
-//   data stream     H2D run 1 ── a_1 ── H2D run 2 ── a_2 ...      D2H run 1 ── d_1 ── D2H run 2 ── d_2 ...
-//   compute stream  (waits a_1) decode run 1, (waits a_2) decode run 2 ... encode run 1 ── e_1 ── encode run 2 ── e_2 ...
-//                                                                  (D2H run k waits e_k)
-//   worker          between runs, and at the end: publishes every run whose event has passed
+//   lane 0   encode run 1 ── D2H run 1 ── e_1      H2D run 3 ── decode run 3 ── e_3 ...
+//   lane 1         encode run 2 ── D2H run 2 ── e_2      H2D run 4 ── decode run 4 ── e_4 ...
+//   worker   between runs, and while it has nothing else to do: publishes every run whose event has passed
+//
+// A run's kernels follow each other on one stream, so no stream ever waits for another (with a compute and a data stream
+// the two event calls per run cost the worker 20 us, more than its launches).  Runs are independent of each other
+// because no tensor, residual, B or C is in two of them: a batch in which one is (a root task's tensor is decoded and then
+// encoded) stays on one lane, and a batch that names one still in use by an earlier batch waits for that.
+//
+// Batches follow each other without waiting for the one before: a caller that submits 161 tasks one after the other
+// hands over the first few long before the last, and with every batch drained before the next was looked at the
+// link stood idle for most of the time (ResNet-50's messages out and back: 700 us, of which 240 on the link).  Up to
+// kSlots batches are under way at once, each with its own staging memory and events.
 //
 // A transfer run is one launch of the range-copy kernel over all its messages (the GPU reads or
 // writes the pinned host buffers itself): with a copy call per message the host spent longer
@@ -27,6 +36,7 @@
 // multi-message decoders) and then re-encodes it.
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -38,6 +48,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <unordered_set>
 #include <vector>
 
 #include "hpx.h"
@@ -48,6 +59,10 @@
 namespace hpx {
 // hpx_runtime.hip: all ranges in one kernel launch (device memory or pinned host memory on either side)
 int copy_ranges(int count, uint8_t* const* dst, const uint8_t* const* src, const int64_t* bytes, hipStream_t st);
+// hpx_terngrad.hip: hpx_terngrad_encode, with or without the launches that meet at a grid-wide barrier
+int terngrad_encode(bool barriers, int count, const float* const* ins, const int32_t* in_sizes, uint8_t* const* outs,
+                    const int32_t* out_sizes, const uint8_t* bitwidths, const int32_t* enable_randoms, const uint64_t* seeds,
+                    hipStream_t st);
 }
 
 namespace {
@@ -70,20 +85,22 @@ struct Task {
   std::string name;
   uint64_t serial = 0;
   hpx_task_t t{};
-  mutable bool published = false;
+  mutable bool grouped = false;   // some group publishes it
 };
 
 struct Sched {
   std::mutex mu;                  // queue, params, running flags
   std::condition_variable cv;     // work arrived / shutdown
-  std::deque<Task> queue;
+  std::vector<Task> queue;        // swapped out whole: a submitting thread never waits for the worker to move tasks
   Params params;
   bool running = false, stop = false, ready = false;
   int init_rc = 0;
   std::thread worker;
   uint64_t next_serial = 1;
 
-  std::mutex fmu;                 // finished queues, done serials
+  alignas(64) std::atomic<int> queued{0};  // length of the queue, for a look without the lock
+
+  alignas(64) std::mutex fmu;     // finished queues, done serials
   std::condition_variable fcv;
   std::deque<std::string> finished[3];  // COMP, DECOMP, ROOT (FinishedQueues, hp_cuda.h:128-132)
   std::deque<uint64_t> done;
@@ -144,12 +161,24 @@ struct Arena {  // grow-only block, re-used from offset 0 by every batch
   }
 };
 
-struct Worker {
-  hipStream_t compute = nullptr, data = nullptr;
+struct Pending { uint8_t* dst; const uint8_t* src; size_t bytes; };
+
+struct Group {  // tasks published together once `landed` has passed
+  std::vector<const Task*> tasks;
+  int queue = 0;
+  hipEvent_t landed = nullptr;
+  std::vector<Pending> host_copies;  // pinned bounce buffer -> pageable C
+};
+
+constexpr int kSlots = 4;
+// A batch under way: its tasks, staging memory, events, and the groups that are still to be published.
+struct Slot {
+  std::vector<Task> tasks;
   Arena pinned_arena, device_arena;
   std::vector<hipEvent_t> events;
   size_t next_event = 0;
-  struct Pending { uint8_t* dst; const uint8_t* src; size_t bytes; };
+  std::deque<Group> groups;
+  size_t next_pub = 0;
   hipEvent_t event() {
     if (next_event == events.size()) {
       hipEvent_t e = nullptr;
@@ -158,6 +187,15 @@ struct Worker {
     }
     return events[next_event++];
   }
+};
+
+struct Worker {
+  hipStream_t lane[2] = {nullptr, nullptr};
+  unsigned turn = 0;
+  Slot slots[kSlots];
+  std::deque<Slot*> in_flight, free_slots;
+  std::unordered_set<const void*> held;       // every tensor, residual, B and C of the batches in flight
+  Slot* cur = nullptr;                        // the batch being queued
 };
 
 // The address under which the GPU can reach host memory `p` (pinned and mapped), or null for
@@ -195,36 +233,29 @@ int64_t message_bytes(const Params& p, const hpx_task_t& t) {
 constexpr int64_t kPipeFirstBytes = int64_t(1) << 20;
 constexpr int64_t kPipeMaxBytes = int64_t(16) << 20;
 
-struct Group {  // tasks published together once `landed` has passed
-  std::vector<const Task*> tasks;
-  int queue = 0;
-  hipEvent_t landed = nullptr;
-  std::vector<Worker::Pending> host_copies;  // pinned bounce buffer -> pageable C
-};
-
-// Copies gathered for one phase and issued as one kernel launch on the data stream.
+// Copies gathered for one run and issued as one kernel launch.
 struct CopyList {
   std::vector<uint8_t*> dst;
   std::vector<const uint8_t*> src;
   std::vector<int64_t> bytes;
   void add(uint8_t* d, const uint8_t* s, int64_t b) { dst.push_back(d); src.push_back(s); bytes.push_back(b); }
-  void issue(Worker& w) {
+  void issue(hipStream_t st) {
     if (dst.empty()) return;
-    const int rc = hpx::copy_ranges(int(dst.size()), dst.data(), src.data(), bytes.data(), w.data);
+    const int rc = hpx::copy_ranges(int(dst.size()), dst.data(), src.data(), bytes.data(), st);
     if (rc != HPX_OK) fail("scheduler: staging copy failed, ret = %d. %s", rc, hpx_last_error());
     dst.clear(); src.clear(); bytes.clear();
   }
 };
 
 // Device -> host of one message: straight into C when it is pinned, else into the pinned bounce
-// buffer, from where the worker copies it to C once the data stream has passed.
+// buffer, from where the worker copies it to C once the run has passed.
 void copy_out(Worker& w, CopyList& cl, Group& grp, const hpx_task_t& t, int64_t bytes) {
   if (bytes <= 0) return;
   if (bytes > t.C_bytes || bytes > t.B_bytes) { fail("scheduler: task buffers too small for a %lld-byte message (B %lld, C %lld)", (long long)bytes, (long long)t.B_bytes, (long long)t.C_bytes); return; }
   if (uint8_t* c = device_alias(t.C)) {
     cl.add(c, t.B, bytes);
   } else {
-    uint8_t* bounce = w.pinned_arena.take(size_t(bytes));
+    uint8_t* bounce = w.cur->pinned_arena.take(size_t(bytes));
     cl.add(bounce, t.B, bytes);
     grp.host_copies.push_back({t.C, bounce, size_t(bytes)});
   }
@@ -236,38 +267,63 @@ void copy_in(Worker& w, CopyList& cl, uint8_t* dst, const uint8_t* src, int64_t 
   if (const uint8_t* c = device_alias(src)) {
     cl.add(dst, c, bytes);
   } else {
-    uint8_t* bounce = w.pinned_arena.take(size_t(bytes));
+    uint8_t* bounce = w.cur->pinned_arena.take(size_t(bytes));
     std::memcpy(bounce, src, size_t(bytes));
     cl.add(dst, bounce, bytes);
   }
 }
 
 void publish(Group& grp) {
-  if (grp.tasks.empty()) return;
   if (grp.landed) SCHED_HIP(hipEventSynchronize(grp.landed));
   for (const auto& c : grp.host_copies) std::memcpy(c.dst, c.src, c.bytes);
   {
     std::lock_guard<std::mutex> l(g.fmu);
     for (const Task* t : grp.tasks) {
-      g.finished[grp.queue].push_back(t->name);
+      if (grp.queue >= 0) g.finished[grp.queue].push_back(t->name);
       g.done.push_back(t->serial);
-      t->published = true;
     }
   }
   g.fcv.notify_all();
 }
 
-// after `producer` has reached this point, `consumer` may go on
-hipEvent_t chain(Worker& w, hipStream_t producer, hipStream_t consumer) {
-  hipEvent_t e = w.event();
-  if (!e) return nullptr;
-  SCHED_HIP(hipEventRecord(e, producer));
-  if (consumer) SCHED_HIP(hipStreamWaitEvent(consumer, e, 0));
+// What a task reads or writes; no two batches in flight name the same.
+std::array<const void*, 7> named(const hpx_task_t& t) { return {t.tensor, t.residual, t.B, t.C, t.M, t.P, t.Q}; }
+
+// Publishes, in the order they were queued, the groups whose events have passed; with `wait` at least everything of the
+// oldest batch.
+void publish_landed(Worker& w, bool wait) {
+  while (!w.in_flight.empty()) {
+    Slot& s = *w.in_flight.front();
+    for (; s.next_pub < s.groups.size(); s.next_pub++) {
+      Group& grp = s.groups[s.next_pub];
+      if (!wait && grp.landed && hipEventQuery(grp.landed) == hipErrorNotReady) {
+        (void)hipGetLastError();  // "not ready" must not be taken for a failed launch later on
+        return;
+      }
+      publish(grp);
+    }
+    if (&s == w.cur) return;  // still being queued
+    for (const Task& t : s.tasks)
+      for (const void* p : named(t.t)) w.held.erase(p);
+    s.tasks.clear();
+    s.groups.clear();
+    w.in_flight.pop_front();
+    w.free_slots.push_back(&s);
+    wait = false;
+  }
+}
+
+// An event behind everything queued on `st` so far.
+hipEvent_t mark(Worker& w, hipStream_t st) {
+  hipEvent_t e = w.cur->event();
+  if (e) SCHED_HIP(hipEventRecord(e, st));
   return e;
 }
 
 // ---- the three quantiser / sparsifier algorithms ---------------------------------
-void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch) {
+void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch, bool one_lane) {
+  auto next_lane = [&]() { return one_lane ? w.lane[0] : w.lane[w.turn++ & 1u]; };
+  std::deque<Group>& sent = w.cur->groups;
   std::vector<const Task*> comp, decomp, root;
   for (const Task& t : batch) {
     switch (t.t.task_id) {
@@ -287,8 +343,7 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
     pinned_need += pad(slots) + pad(message_bytes(p, t->t));
     device_need += pad(slots);
   }
-  if (!w.pinned_arena.reserve(pinned_need) || !w.device_arena.reserve(device_need)) return;
-  w.next_event = 0;
+  if (!w.cur->pinned_arena.reserve(pinned_need) || !w.cur->device_arena.reserve(device_need)) return;
 
   // Transfers and codec calls are cut into runs so that the PCIe transfer of one run overlaps the kernels of
   // the next (a 200-tensor TBQ bucket spends 2.5 times as long on the link as in its encode kernel).
@@ -300,25 +355,22 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
     return b == 0 ? kPipeFirstBytes : (b * 2 < kPipeMaxBytes ? b * 2 : kPipeMaxBytes);
   };
 
-  // ---- messages in (data stream): every run's copy is queued now, its decode later ----
+  // ---- messages in ----
   struct DecodeRun {
     std::vector<float*> out;           // decode argument lists (hp_cuda.cpp:420-461)
     std::vector<int32_t> out_size, in_size, add;
     std::vector<const uint8_t*> in;
     std::vector<const Task*> decomp;   // the DECOMP tasks among them: published once the decode has run
-    hipEvent_t arrived = nullptr;
+    CopyList copies;
     int64_t bytes = 0;
   };
   std::vector<DecodeRun> dec_runs;
   std::vector<const Task*> root_ok;
   {
-    CopyList cl_in;
     DecodeRun run;
     int64_t pipe_bytes = next_run_bytes(0);
     auto close_run = [&]() {
       if (run.out.empty()) return;
-      cl_in.issue(w);
-      run.arrived = chain(w, w.data, nullptr);
       dec_runs.push_back(std::move(run));
       run = DecodeRun();
       pipe_bytes = next_run_bytes(pipe_bytes);
@@ -326,7 +378,7 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
     for (const Task* t : decomp) {
       const int64_t bytes = message_bytes(p, t->t);
       if (bytes > t->t.C_bytes || bytes > t->t.B_bytes) { fail("scheduler: decode task '%s': message of %lld bytes does not fit B (%lld) / C (%lld)", t->name.c_str(), (long long)bytes, (long long)t->t.B_bytes, (long long)t->t.C_bytes); continue; }
-      copy_in(w, cl_in, t->t.B, t->t.C, bytes);  // t.B->copy_(t.C->slice(0,0,compressed_size,1), true)
+      copy_in(w, run.copies, t->t.B, t->t.C, bytes);  // t.B->copy_(t.C->slice(0,0,compressed_size,1), true)
       run.out.push_back(t->t.tensor); run.out_size.push_back(int32_t(t->t.tensor_numel));
       run.in.push_back(t->t.B); run.in_size.push_back(int32_t(bytes)); run.add.push_back(t->t.is_root);
       run.decomp.push_back(t);
@@ -337,8 +389,8 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
       const int64_t bytes = message_bytes(p, t->t);
       const int64_t slots = int64_t(p.size) * bytes;
       if (slots > t->t.C_bytes) { fail("scheduler: root task '%s': C holds %lld bytes, %d slots of %lld needed", t->name.c_str(), (long long)t->t.C_bytes, p.size, (long long)bytes); continue; }
-      uint8_t* tmp = w.device_arena.take(size_t(slots));  // temp_cuda_tensors_for_c, hp_cuda.cpp:149-158
-      copy_in(w, cl_in, tmp, t->t.C, slots);
+      uint8_t* tmp = w.cur->device_arena.take(size_t(slots));  // temp_cuda_tensors_for_c, hp_cuda.cpp:149-158
+      copy_in(w, run.copies, tmp, t->t.C, slots);
       for (int i = 0; i < p.size; i++) {
         if (i == p.rank) continue;
         run.out.push_back(t->t.tensor); run.out_size.push_back(int32_t(t->t.tensor_numel));
@@ -352,22 +404,8 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
   }
   root = root_ok;
 
-  // Groups in the order they were queued; names go out as their events pass.
-  std::deque<Group> sent;
-  size_t next_pub = 0;
-  auto publish_landed = [&](bool wait) {
-    for (; next_pub < sent.size(); next_pub++) {
-      Group& grp = sent[next_pub];
-      if (!wait && grp.landed && hipEventQuery(grp.landed) != hipSuccess) {
-        (void)hipGetLastError();  // "not ready" must not be taken for a failed launch later on
-        return;
-      }
-      publish(grp);
-    }
-  };
-
   // ---- compute ----
-  auto encode = [&](const std::vector<const Task*>& ts, const char* what) {
+  auto encode = [&](const std::vector<const Task*>& ts, bool alone, hipStream_t st, const char* what) {
     if (ts.empty()) return;
     const int n = int(ts.size());
     std::vector<const float*> in(n);
@@ -382,41 +420,44 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
     if (p.alg == kTerngrad) {
       std::vector<uint8_t> bw(n, uint8_t(p.bitwidth));
       std::vector<int32_t> rnd(n, p.enable_random);
-      codec(hpx_terngrad_encode(n, in.data(), in_size.data(), out.data(), out_size.data(), bw.data(), rnd.data(),
-                                p.has_seed ? seeds.data() : nullptr, w.compute), what);
-      // Before the messages leave B: a launch that waits at a grid barrier is the one kind that can fail to
-      // write its message.  Returns at once when the run took none; otherwise waits for the compute stream
-      // and encodes again what an expired barrier left unwritten.
-      codec(hpx_terngrad_encode_status(w.compute), "hpx_terngrad_encode_status");
+      // A launch that meets at a grid barrier occupies every CU, so it would wait for the copies of earlier runs to end and
+      // keep those of later ones from starting: only a run that has the GPU to itself takes one.
+      codec(hpx::terngrad_encode(alone, n, in.data(), in_size.data(), out.data(), out_size.data(), bw.data(), rnd.data(),
+                                 p.has_seed ? seeds.data() : nullptr, st), what);
+      // Before the messages leave B: such a launch is the one kind that can fail to write its message.  Waits for the
+      // stream and encodes again what an expired barrier left unwritten.
+      if (alone) codec(hpx_terngrad_encode_status(st), "hpx_terngrad_encode_status");
     } else if (p.alg == kTbq) {
       std::vector<float> thr(n, p.threshold);
-      codec(hpx_tbq_encode(n, in.data(), in_size.data(), res.data(), out.data(), thr.data(), w.compute), what);
+      codec(hpx_tbq_encode(n, in.data(), in_size.data(), res.data(), out.data(), thr.data(), st), what);
     } else {
       std::vector<double> sr(n, p.sample_rate), dr(n, p.drop_ratio);
       codec(hpx_gd_encode(n, in.data(), in_size.data(), res.data(), out.data(), sr.data(), dr.data(),
-                          p.has_seed ? seeds.data() : nullptr, w.compute), what);
+                          p.has_seed ? seeds.data() : nullptr, st), what);
     }
   };
   auto decode = [&]() {
     for (DecodeRun& r : dec_runs) {
-      if (r.arrived) SCHED_HIP(hipStreamWaitEvent(w.compute, r.arrived, 0));
+      const hipStream_t st = next_lane();
+      r.copies.issue(st);
       const int n = int(r.out.size());
       if (p.alg == kTerngrad) {
-        codec(hpx_terngrad_decode(n, r.out.data(), r.out_size.data(), r.in.data(), r.in_size.data(), r.add.data(), w.compute), "hp_cuda_terngradr");
+        codec(hpx_terngrad_decode(n, r.out.data(), r.out_size.data(), r.in.data(), r.in_size.data(), r.add.data(), st), "hp_cuda_terngradr");
       } else if (p.alg == kTbq) {
         std::vector<float> thr(n, p.threshold);
-        codec(hpx_tbq_decode(n, r.out.data(), r.out_size.data(), r.in.data(), thr.data(), r.add.data(), w.compute), "hp_cuda_tbqr");
+        codec(hpx_tbq_decode(n, r.out.data(), r.out_size.data(), r.in.data(), thr.data(), r.add.data(), st), "hp_cuda_tbqr");
       } else {
-        codec(hpx_gd_decode(n, r.in.data(), r.in_size.data(), r.out.data(), r.out_size.data(), r.add.data(), w.compute), "hp_cuda_gdr");
+        codec(hpx_gd_decode(n, r.in.data(), r.in_size.data(), r.out.data(), r.out_size.data(), r.add.data(), st), "hp_cuda_gdr");
       }
       if (!r.decomp.empty()) {
         sent.emplace_back();
         Group& grp = sent.back();
         grp.queue = 1;
         grp.tasks = std::move(r.decomp);
-        grp.landed = chain(w, w.compute, nullptr);
+        for (const Task* t : grp.tasks) t->grouped = true;
+        grp.landed = mark(w, st);
       }
-      publish_landed(false);
+      publish_landed(w, false);
     }
   };
   // Encodes `ts` run by run; each run's messages go out behind it:
@@ -432,8 +473,9 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
         bytes += message_bytes(p, ts[i]->t);
         run.push_back(ts[i++]);
       }
-      encode(run, what);
-      chain(w, w.compute, w.data);
+      const bool alone = i == ts.size() && run.size() == ts.size() && w.in_flight.size() == 1;
+      const hipStream_t st = alone ? w.lane[0] : next_lane();   // one stream per device may launch barrier kernels
+      encode(run, alone, st, what);
       CopyList cl;
       const size_t first_group = sent.size();
       for (const Task* t : run) {
@@ -443,12 +485,13 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
           sent.back().queue = q;
         }
         sent.back().tasks.push_back(t);
+        t->grouped = true;
         copy_out(w, cl, sent.back(), t->t, message_bytes(p, t->t));
       }
-      cl.issue(w);
-      hipEvent_t landed = chain(w, w.data, nullptr);
+      cl.issue(st);
+      hipEvent_t landed = mark(w, st);
       for (size_t k = first_group; k < sent.size(); k++) sent[k].landed = landed;
-      publish_landed(false);
+      publish_landed(w, false);
     }
   };
 
@@ -462,11 +505,11 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch)
     both.insert(both.end(), comp.begin(), comp.end());
     encode_and_send(both, p.alg == kTbq ? "hp_cuda_tbq" : "hp_cuda_gd");
   }
-  publish_landed(true);
 }
 
 // ---- PowerSGD --------------------------------------------------------------------
 void run_powersgd_batch(Worker& w, const Params&, const std::vector<Task>& batch) {
+  const hipStream_t st = w.lane[0];   // the three phases of a matrix follow each other
   std::vector<const Task*> e1, e2, dec;
   for (const Task& t : batch) {
     switch (t.t.task_id) {
@@ -476,7 +519,6 @@ void run_powersgd_batch(Worker& w, const Params&, const std::vector<Task>& batch
       default: fail("error find task_id != 40 50 60 where task_id is %d", t.t.task_id); break;
     }
   }
-  w.next_event = 0;
   auto lists = [](const std::vector<const Task*>& ts, std::vector<float*>& G, std::vector<float*>& R, std::vector<float*>& M,
                   std::vector<float*>& P, std::vector<float*>& Q, std::vector<int64_t>& numel, std::vector<int32_t>& n,
                   std::vector<int32_t>& m, std::vector<int32_t>& r) {
@@ -493,41 +535,86 @@ void run_powersgd_batch(Worker& w, const Params&, const std::vector<Task>& batch
     lists(e1, G, R, M, P, Q, numel, n, m, r);
     if (!e1.empty())
       codec(hpx_powersgd_encode1(int(e1.size()), G.data(), numel.data(), R.data(), Q.data(), M.data(), P.data(), n.data(),
-                                 m.data(), r.data(), w.compute), "hp_cuda_powersgd_encode1");
-    g1.landed = chain(w, w.compute, nullptr);
+                                 m.data(), r.data(), st), "hp_cuda_powersgd_encode1");
+    if (!g1.tasks.empty()) g1.landed = mark(w, st);
   }
   {
     std::vector<float*> G, R, M, P, Q; std::vector<int64_t> numel; std::vector<int32_t> n, m, r;
     lists(e2, G, R, M, P, Q, numel, n, m, r);
     if (!e2.empty())
-      codec(hpx_powersgd_encode2(int(e2.size()), P.data(), M.data(), Q.data(), n.data(), m.data(), r.data(), w.compute),
+      codec(hpx_powersgd_encode2(int(e2.size()), P.data(), M.data(), Q.data(), n.data(), m.data(), r.data(), st),
             "hp_cuda_powersgd_encode2");
-    g2.landed = chain(w, w.compute, nullptr);
+    if (!g2.tasks.empty()) g2.landed = mark(w, st);
   }
   {
     std::vector<float*> G, R, M, P, Q; std::vector<int64_t> numel; std::vector<int32_t> n, m, r;
     lists(dec, G, R, M, P, Q, numel, n, m, r);
     if (!dec.empty())
       codec(hpx_powersgd_decode(int(dec.size()), P.data(), Q.data(), M.data(), R.data(), G.data(), numel.data(), n.data(),
-                                m.data(), r.data(), w.compute), "hp_cuda_powersgd_decode");
-    g3.landed = chain(w, w.compute, nullptr);
+                                m.data(), r.data(), st), "hp_cuda_powersgd_decode");
+    if (!g3.tasks.empty()) g3.landed = mark(w, st);
   }
-  publish(g3);  // decode, encode1, encode2: the reference's publication order
-  publish(g1);
-  publish(g2);
+  for (Group* grp : {&g3, &g1, &g2}) {  // decode, encode1, encode2: the reference's publication order
+    for (const Task* t : grp->tasks) t->grouped = true;
+    if (!grp->tasks.empty()) w.cur->groups.push_back(std::move(*grp));
+  }
+}
+
+// Queues a batch behind those under way.
+void run_batch(Worker& w, const Params& p, std::vector<Task>& batch) {
+  bool clash = false, twice = false;
+  std::vector<const void*> mine;
+  mine.reserve(batch.size() * 4);
+  for (const Task& t : batch) {
+    twice = twice || t.t.task_id == HPX_ROOT_DECOMP_COMP_TASK;
+    for (const void* x : named(t.t))
+      if (x) mine.push_back(x);
+  }
+  for (const void* x : mine) clash = clash || (!w.held.empty() && w.held.count(x));
+  while (!w.in_flight.empty() && (clash || w.free_slots.empty())) publish_landed(w, true);
+  Slot& s = *w.free_slots.front();
+  w.free_slots.pop_front();
+  s.tasks.swap(batch);   // (the slot's empty list goes back: lists keep their room)
+  s.next_event = 0;
+  s.next_pub = 0;
+  for (Task& t : s.tasks) t.t.name = t.name.c_str();
+  for (const void* x : mine) twice = !w.held.insert(x).second || twice;
+  w.cur = &s;
+  w.in_flight.push_back(&s);
+  if (p.alg == kPowersgd) run_powersgd_batch(w, p, s.tasks); else run_codec_batch(w, p, s.tasks, twice);
+  // A task that failed its checks was skipped (the failure is counted and kept for hpx_sched_error); its
+  // name is published all the same, once the batch has drained, so that a caller polling for it does not
+  // wait for ever: the reference publishes every task of a batch (hp_cuda.cpp:626-636).
+  hipEvent_t drained = nullptr;
+  for (const Task& t : s.tasks) {
+    if (t.grouped) continue;
+    if (!drained) {
+      if (hipEvent_t other = mark(w, w.lane[1])) SCHED_HIP(hipStreamWaitEvent(w.lane[0], other, 0));
+      drained = mark(w, w.lane[0]);
+    }
+    Group grp;
+    grp.tasks.push_back(&t);
+    grp.queue = queue_of(t.t.task_id);
+    grp.landed = drained;
+    s.groups.push_back(std::move(grp));
+  }
+  w.cur = nullptr;
 }
 
 void worker_main() {
   Worker w;
-  w.pinned_arena.pinned = true;
+  for (Slot& s : w.slots) {
+    s.pinned_arena.pinned = true;
+    w.free_slots.push_back(&s);
+  }
   int rc = 0;
   Params p0;
   {
     std::lock_guard<std::mutex> l(g.mu);
     p0 = g.params;
   }
-  if (hipSetDevice(p0.device) != hipSuccess || hipStreamCreateWithFlags(&w.compute, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&w.data, hipStreamNonBlocking) != hipSuccess) {
+  if (hipSetDevice(p0.device) != hipSuccess || hipStreamCreateWithFlags(&w.lane[0], hipStreamNonBlocking) != hipSuccess ||
+      hipStreamCreateWithFlags(&w.lane[1], hipStreamNonBlocking) != hipSuccess) {
     fail("scheduler: cannot set up device %d: %s", p0.device, hipGetErrorString(hipGetLastError()));
     rc = HPX_ERR_HIP;
   }
@@ -539,47 +626,43 @@ void worker_main() {
   g.cv.notify_all();
   if (rc != 0) return;
 
+  // With nothing under way the worker sleeps until a task is queued.  With batches under way it looks for landed groups
+  // and new tasks in turn: without a pause at first (a run takes some tens of microseconds), every 20 us once nothing has
+  // happened for a while (the streams may be waiting behind a long kernel of the caller's).
+  uint32_t idle = 0;
+  std::vector<Task> batch;
   for (;;) {
-    std::vector<Task> batch;
+    batch.clear();
     Params p;
-    {
+    if (w.in_flight.empty() || g.queued.load(std::memory_order_acquire) > 0 || idle > 2000) {
       std::unique_lock<std::mutex> l(g.mu);
-      g.cv.wait(l, [] { return g.stop || !g.queue.empty(); });
-      if (g.queue.empty() && g.stop) break;
-      batch.assign(std::make_move_iterator(g.queue.begin()), std::make_move_iterator(g.queue.end()));
-      g.queue.clear();
+      auto woken = [] { return g.stop || !g.queue.empty(); };
+      if (w.in_flight.empty()) g.cv.wait(l, woken);
+      else if (idle > 2000 && g.queue.empty()) g.cv.wait_for(l, std::chrono::microseconds(20));
+      if (g.queue.empty() && g.stop && w.in_flight.empty()) break;
+      batch.swap(g.queue);
+      g.queued.store(0, std::memory_order_release);
       p = g.params;
     }
-    for (Task& t : batch) t.t.name = t.name.c_str();
-    if (p.alg == kPowersgd) run_powersgd_batch(w, p, batch); else run_codec_batch(w, p, batch);
-    // A task that failed its checks was skipped (the failure is counted and kept for hpx_sched_error); its
-    // name is published all the same, once the batch has drained, so that a caller polling for it does not
-    // wait for ever: the reference publishes every task of a batch (hp_cuda.cpp:626-636).
-    SCHED_HIP(hipStreamSynchronize(w.compute));
-    SCHED_HIP(hipStreamSynchronize(w.data));
-    {
-      bool any = false;
-      std::lock_guard<std::mutex> l(g.fmu);
-      for (const Task& t : batch) {
-        if (t.published) continue;
-        const int q = queue_of(t.t.task_id);
-        if (q >= 0) { g.finished[q].push_back(t.name); any = true; }
-        g.done.push_back(t.serial);
-      }
-      if (any) g.fcv.notify_all();
-    }
+    const Slot* oldest = w.in_flight.empty() ? nullptr : w.in_flight.front();
+    const size_t published = oldest ? oldest->next_pub : 0;
+    if (!batch.empty()) run_batch(w, p, batch);
+    publish_landed(w, false);
+    const bool moved = oldest == nullptr || w.in_flight.empty() || w.in_flight.front() != oldest || oldest->next_pub != published;
+    idle = moved ? 0 : idle + 1;
   }
-  (void)hipStreamSynchronize(w.compute);
-  (void)hipStreamSynchronize(w.data);
-  for (hipEvent_t e : w.events) (void)hipEventDestroy(e);
-  w.pinned_arena.release();
-  w.device_arena.release();
-  // The codec workspaces of the two streams go with them, and with the compute stream's its claim on the
+  for (hipStream_t st : w.lane) (void)hipStreamSynchronize(st);
+  for (Slot& s : w.slots) {
+    for (hipEvent_t e : s.events) (void)hipEventDestroy(e);
+    s.pinned_arena.release();
+    s.device_arena.release();
+  }
+  // The codec workspaces of the two streams go with them, and with them the claim on the
   // grid-barrier kernels: the worker of a later init() gets the resident TernGrad encode again.
-  (void)hpx_release_stream(w.compute);
-  (void)hpx_release_stream(w.data);
-  (void)hipStreamDestroy(w.compute);
-  (void)hipStreamDestroy(w.data);
+  for (hipStream_t st : w.lane) {
+    (void)hpx_release_stream(st);
+    (void)hipStreamDestroy(st);
+  }
 }
 
 }  // namespace
@@ -681,6 +764,7 @@ HPX_API int hpx_sched_submit(const hpx_task_t* task, uint64_t* serial) {
   t.serial = g.next_serial++;
   if (serial) *serial = t.serial;
   g.queue.push_back(std::move(t));
+  g.queued.fetch_add(1, std::memory_order_release);
   g.cv.notify_one();
   return HPX_OK;
 }

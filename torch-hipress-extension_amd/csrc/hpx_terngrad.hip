@@ -2642,10 +2642,12 @@ constexpr size_t kResidentLogMax = 4096;  // records kept before hpx_terngrad_en
 
 }  // namespace
 
-HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_t* in_sizes,
-                                uint8_t* const* outs, const int32_t* out_sizes,
-                                const uint8_t* bitwidths, const int32_t* enable_randoms,
-                                const uint64_t* seeds, hpx_stream_t stream) {
+// barriers = false: without the launches that meet at a grid-wide barrier, for a caller that has other work on the GPU
+// which they would wait for and hold up.
+namespace hpx {
+int terngrad_encode(bool barriers, int count, const float* const* ins, const int32_t* in_sizes, uint8_t* const* outs,
+                    const int32_t* out_sizes, const uint8_t* bitwidths, const int32_t* enable_randoms, const uint64_t* seeds,
+                    hipStream_t stream) {
   hpx::clear_error();
   HPX_ARG(count >= 0, "hpx_terngrad_encode: negative count");
   if (count == 0) return HPX_OK;
@@ -2663,7 +2665,7 @@ HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_
     HPX_ARG(out_sizes[i] >= need, "hpx_terngrad_encode: tensor %d needs %lld output bytes, got %d", i,
             static_cast<long long>(need), out_sizes[i]);
   }
-  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipStream_t st = stream;
   int rc = hpx::reject_capture(st, "hpx_terngrad_encode");
   if (rc != HPX_OK) return rc;
   hpx::Workspace* ws = hpx::workspace_record(st);
@@ -2673,8 +2675,10 @@ HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_
   if (rc != HPX_OK) return rc;
   rc = hpx::ensure_slots(ws, size_t(count) * kSlotsPerTensor);
   if (rc != HPX_OK) return rc;
-  rc = hpx::ensure_barrier(ws);
-  if (rc != HPX_OK) return rc;
+  if (barriers) {
+    rc = hpx::ensure_barrier(ws);
+    if (rc != HPX_OK) return rc;
+  }
 
   // A barrier kernel of an earlier call on this stream gave up waiting: its messages are queued again
   // through the tiled kernels before this call's work, and this call takes the tiled kernels too.  (The
@@ -2695,7 +2699,7 @@ HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_
   // takes the single-tensor resident kernel; the rest goes to the tiled pair of kernels.
   std::vector<int> tiled;
   tiled.reserve(count);
-  const bool buckets = count >= 2 && hpx::option(hpx::kOptTerngradResidentBucket) != 0 &&
+  const bool buckets = barriers && count >= 2 && hpx::option(hpx::kOptTerngradResidentBucket) != 0 &&
                        hpx::option(hpx::kOptTerngradResidentMin) >= 0;
   auto log_resident = [&](const EncSeg& sg, uint64_t seed) {
     ws->resident_log.add(hpx::Workspace::ResidentRec{sg.x, sg.out, sg.n, sg.out_size, seed, sg.bits, sg.random});
@@ -2738,7 +2742,7 @@ HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_
     const int stop = j > i ? j : i + 1;
     for (; i < stop; i++) {
       ResArgs ra;
-      if (ws->barrier_broken || !resident_plan(in_sizes[i], bitwidths[i], enable_randoms[i] != 0, ws, ra) ||
+      if (!barriers || ws->barrier_broken || !resident_plan(in_sizes[i], bitwidths[i], enable_randoms[i] != 0, ws, ra) ||
           !hpx::claim_barrier_kernels(ws)) {
         tiled.push_back(i);
         continue;
@@ -2777,6 +2781,15 @@ HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_
   }
   return encode_tiled(ws, st, m, t_in.data(), t_isz.data(), t_out.data(), t_osz.data(), t_bits.data(), t_rnd.data(),
                       t_seed.data());
+}
+}  // namespace hpx
+
+HPX_API int hpx_terngrad_encode(int count, const float* const* ins, const int32_t* in_sizes,
+                                uint8_t* const* outs, const int32_t* out_sizes,
+                                const uint8_t* bitwidths, const int32_t* enable_randoms,
+                                const uint64_t* seeds, hpx_stream_t stream) {
+  return hpx::terngrad_encode(true, count, ins, in_sizes, outs, out_sizes, bitwidths, enable_randoms, seeds,
+                              static_cast<hipStream_t>(stream));
 }
 
 HPX_API int hpx_terngrad_encode_noalloc(int count, const float* const* ins, const int32_t* in_sizes,
