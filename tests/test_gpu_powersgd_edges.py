@@ -1,0 +1,96 @@
+"""GPU: PowerSGD where its launches and its orthonormalisation change ways.
+
+Oracle: float64 products of the very P, Q and M that the device was given.  Tolerances: P and Q are sums of at most
+4100 products of fp32 values in fp32, in parts of a few hundred: 1e-5 of the Frobenius norm; orthonormal columns rounded
+to fp32 once: every product of two columns within 2^-23 of its value, times at most 8 columns.
+"""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import assert_bits_equal, dev, host
+from oracle import powersgd as ps
+from test_gpu_powersgd import Psgd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def psgd(capi):
+    return Psgd(capi)
+
+
+def _phases(psgd, shapes, seed):
+    rng = np.random.default_rng(seed)
+    G = [rng.normal(0, 1e-2, n * m).astype(np.float32) for n, m, r in shapes]
+    R = [rng.normal(0, 1e-3, n * m).astype(np.float32) for n, m, r in shapes]
+    Q = [rng.normal(0, 1, (m, r)).astype(np.float32) for n, m, r in shapes]
+    dG, dR, dQ = [dev(x) for x in G], [dev(x) for x in R], [dev(x) for x in Q]
+    dM = [torch.full((n, m), 7.0, device="cuda") for n, m, r in shapes]
+    dP = [torch.full((n, r), 7.0, device="cuda") for n, m, r in shapes]
+    psgd.encode1(dG, dR, dQ, dM, dP)
+    for i, s in enumerate(shapes):
+        Mref, Pref = ps.encode1(G[i], R[i], Q[i], np.zeros(s[:2], np.float32))
+        assert_bits_equal(host(dM[i]), Mref, f"M {s}")
+        assert ps.rel_fro(host(dP[i]), Pref) < 1e-5, s
+    before = [host(p).copy() for p in dP]
+    psgd.encode2(dP, dM, dQ)
+    for i, s in enumerate(shapes):
+        P, Qn, Mh = host(dP[i]).astype(np.float64), host(dQ[i]), host(dM[i]).astype(np.float64)
+        assert ps.rel_fro(P, ps.orthogonalize(before[i])) < 1e-5, s
+        assert np.abs(P.T @ P - np.eye(s[2])).max() < 8 * 2.0 ** -23, s
+        assert ps.rel_fro(Qn, Mh.T @ P) < 1e-5, s
+    psgd.decode(dP, dQ, dM, dR, dG)
+    for i, s in enumerate(shapes):
+        P, Qn = host(dP[i]).astype(np.float64), host(dQ[i]).astype(np.float64)
+        assert ps.rel_fro(host(dM[i]), P @ Qn.T) < 1e-6, s
+        assert_bits_equal(host(dG[i]), host(dM[i]).reshape(-1), f"grad {s}")
+        assert_bits_equal(host(dR[i]), G[i] - host(dM[i]).reshape(-1), f"residual {s}")
+
+
+@pytest.mark.parametrize("m", [1, 3, 4, 61, 64, 65, 127, 129, 191, 205, 257, 511, 767, 768, 1023, 1535, 1537, 2049])
+def test_widths_around_the_strips(psgd, m):
+    # n above and below what a strip's tile holds, alone (rows spread out) and beside enough rows to fill the chip
+    _phases(psgd, [(n, m, min(4, n, m)) for n in (4, 17, 33, 515)], m)
+    _phases(psgd, [(n, m, min(2, m)) for n in (8201, 129)], m + 1)
+
+
+@pytest.mark.parametrize("count", [1, 16, 17, 64, 65, 161])
+def test_tables_of_every_size(psgd, count):
+    _phases(psgd, [(5 + 3 * (i % 11), 9 + 7 * (i % 13), 1 + i % 4) for i in range(count)], count)
+
+
+@pytest.mark.parametrize("r", [1, 2, 3, 4, 5, 7, 8, 9])
+def test_ranks_around_the_gram_matrix(psgd, r):
+    _phases(psgd, [(n, 70, r) for n in (r, 63, 1025, 4100)], r)
+
+
+@pytest.mark.parametrize("r", [2, 4, 8])
+def test_columns_that_depend_on_each_other(psgd, r):
+    # The last column is the first plus `eps` of something else: with eps 1e-2 (squared far above 2^-20) the Gram matrix
+    # decides, with 1e-5 Gram-Schmidt does; either way the columns are orthonormal and span what they spanned.  A column
+    # of zeros stays one and leaves the others alone; a NaN reaches the columns from its own on.
+    rng = np.random.default_rng(r)
+    n, m = 3000, 40
+    M = rng.normal(0, 1, (n, m)).astype(np.float32)
+    for eps in (1e-2, 1e-5):
+        P = rng.normal(0, 1, (n, r)).astype(np.float32)
+        P[:, -1] = P[:, 0] + np.float32(eps) * rng.normal(0, 1, n).astype(np.float32)
+        dP, dQ = dev(P), torch.zeros(m, r, device="cuda")
+        psgd.encode2([dP], [dev(M)], [dQ])
+        got = host(dP).astype(np.float64)
+        assert np.abs(got.T @ got - np.eye(r)).max() < 1e-5, eps
+        inside = got.T @ P.astype(np.float64)
+        # what is left of P outside the span: fp32 rounding of unit columns, and with Gram-Schmidt of its steps too
+        assert np.linalg.norm(P - got @ inside) / np.linalg.norm(P) < 1e-6, eps
+    P = rng.normal(0, 1, (n, r)).astype(np.float32)
+    P[:, 0] = 0
+    dP, dQ = dev(P), torch.zeros(m, r, device="cuda")
+    psgd.encode2([dP], [dev(M)], [dQ])
+    got = host(dP).astype(np.float64)
+    assert not got[:, 0].any() and np.abs(got[:, 1:].T @ got[:, 1:] - np.eye(r - 1)).max() < 8 * 2.0 ** -23
+    P[5, r - 1] = np.nan
+    dP = dev(P)
+    psgd.encode2([dP], [dev(M)], [dQ])
+    got = host(dP)
+    assert np.isnan(got[:, r - 1]).all() and not np.isnan(got[:, :r - 1]).any()

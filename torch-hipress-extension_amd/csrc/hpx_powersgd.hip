@@ -28,13 +28,32 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kMaxSeg = 40;
+// Matrices per launch.  A launch that follows another waits for the last workgroup of it: ResNet-50's 54 matrices in
+// two launches a phase (tables of 40) took 73 + 34 + 73 us for encode1, encode2's product and decode, in one 62 + 25 + 65.
+// A smaller table is searched faster: up to 16 entries by the scalar unit, up to 64 with one load per lane.
+constexpr int kSegSmall = 16, kSegMiddle = 64, kSegLarge = 160;
+#define PSGD_BY_COUNT(LAUNCHES, ...)                               \
+  (count <= kSegSmall    ? LAUNCHES<kSegSmall>(count, __VA_ARGS__)  \
+   : count <= kSegMiddle ? LAUNCHES<kSegMiddle>(count, __VA_ARGS__) \
+                         : LAUNCHES<kSegLarge>(count, __VA_ARGS__))
 constexpr int kMaxCG = 4;                 // column groups of 4 -> rank <= 16
-constexpr int kStrip = 256;               // columns per wave step in encode2 / decode
-constexpr int kE2RowsPerBlock = 128;      // rows folded into one partial of Q
 // Decode is three write streams against one read stream; with 8 rows per wave instead of 32 the
 // stores of a workgroup stay close together in time and address and the pass runs 10 % faster.
-constexpr int kDecRowsPerBlock = 32;
+constexpr int kQRowsMin = 32, kQRowsMax = 512;  // rows folded into one partial of Q (of a strip 256 columns wide)
+constexpr int64_t kQTiles = 1024;
+constexpr int kDecRowsPerBlock = 32;      // rows of a decode tile 256 columns wide (narrower tiles are as much taller)
+
+// encode2 and decode cut a matrix into strips of 4 * lanes columns; a wave lays kWave / lanes row groups of a strip
+// side by side.  256 columns unless the lanes past the last column would be more than a quarter of those before it, then
+// 128, then 64.  30 ragged matrices of up to 1500 x 1001: 163 us a pass at a quarter, 170 at an eighth, 181 at a
+// sixteenth: narrow strips touch more lines per byte; wide ones leave lanes idle.
+inline int strip_lanes(int m) {
+  for (int lanes = kWave; lanes > 16; lanes /= 2) {
+    const int64_t w = 4 * lanes;
+    if ((m + w - 1) / w * w - m <= m / 4) return lanes;
+  }
+  return 16;
+}
 
 struct Seg {
   const float* grad;   // encode1: in.  decode: in/out (as float*)
@@ -48,30 +67,35 @@ struct Seg {
   int32_t part_off;    // encode2: offset (in floats / 4) of this matrix's partials
   int32_t ld;          // row stride of P and Q (the full rank; r is the width of the block of columns at hand)
   int32_t mode;        // kFromM | kOntoM | kKeepGrad, for the passes of a rank above 16
+  int32_t split;       // encode1: waves that share four rows.  encode2, decode: strip_lanes
 };
 constexpr int32_t kFromM = 1;    // encode1: M has been stored by an earlier pass: read it instead of grad + residual
 constexpr int32_t kOntoM = 2;    // decode: add this block's P Q^T to what M holds instead of starting from zero
 constexpr int32_t kKeepGrad = 4; // decode: more blocks follow: write M only, leave residual and gradient alone
+template <int CAP>
 struct Args {
   int32_t nseg;
-  int32_t tile_start[kMaxSeg + 1];
-  Seg seg[kMaxSeg];
+  int32_t rows;        // encode2: rows folded into one partial of Q, of a strip 256 columns wide
+  int32_t tile_start[CAP + 1];
+  Seg seg[CAP];
   float* partials;
 };
-static_assert(sizeof(Args) <= 4096, "kernarg limit");
+static_assert(sizeof(Args<kSegLarge>) <= 18000, "kernel-argument budget");
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
 
 // ---- encode1: M = G + R (flat prefix), P = M Q -------------------------------
-// One workgroup per group of 4 rows; its 4 waves share out the columns and meet in
-// LDS.  Lane 4b+i of a wave owns row i and the 4 columns k0+4b..k0+4b+3 of each
-// 64-column step, which is one 128-bit load of G and of R and one store of M.
-template <int CG>
-__global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args a) {
+// Lane 4b+i of a wave owns row i of four and the 4 columns k0+4b..k0+4b+3 of each 64-column step, which is one
+// 128-bit load of G and of R and one store of M.  Bound by HBM (12 bytes an element).  A workgroup takes four rows
+// with all its waves where rows are long; of shorter rows it takes eight or sixteen, two or one wave to four rows
+// (split_rows below): otherwise the waves past the end of the row idle and a workgroup is gone before the next
+// has started.
+template <int CG, int CAP>
+__global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> a) {
   const int tile = blockIdx.x;
-  const int s = find_segment<kMaxSeg>(a.tile_start, a.nseg, tile);
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
   const Seg& sg = a.seg[s];
   const float* __restrict__ G = sg.grad;
   const float* __restrict__ R = sg.res;
@@ -80,12 +104,15 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args a) {
   const int n = sg.n, m = sg.m, r = sg.r, ld = sg.ld;
   const bool from_m = (sg.mode & kFromM) != 0;
   const int64_t N = sg.numel;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int row0 = (tile - a.tile_start[s]) * 4;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int split = sg.split, groups = kWaves / split;
+  const int part = wave % split;  // of the waves that share four rows
+  const int64_t tile_row = int64_t(tile - a.tile_start[s]) * 4 * groups;
+  const int64_t row0 = tile_row + wave / split * 4;
   const int i = lane & 3, b = lane >> 2;
-  const int row = row0 + i;
-  // Columns: the workgroup walks the rows in chunks of kWaves * 256 columns, wave w taking the w-th 256 of each
-  // chunk, so that at any time the four waves read neighbouring pieces of the same four rows (a contiguous
+  const int64_t row = row0 + i;
+  // Columns: the waves walk the rows in chunks of split * 256 columns, wave w taking the w-th 256 of each
+  // chunk, so that at any time they read neighbouring pieces of the same four rows (a contiguous
   // quarter of the row per wave ran 9 % slower); what is left past the last whole 256 goes round the waves in
   // 64-column steps.
   constexpr int kUnroll = 4;
@@ -96,15 +123,15 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args a) {
 #pragma unroll
   for (int c = 0; c < CG; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const bool rows_full = (row0 + 3 < n) && (int64_t(row0 + 4) * m <= N);
+  const bool rows_full = (row0 + 3 < n) && ((row0 + 4) * m <= N);
   if (rows_full) {
     // Main loop: kUnroll 64-column steps at a time, every load issued before the first use.
-    for (int k0 = wave * kChunk; k0 < mfull; k0 += kWaves * kChunk) {
+    for (int k0 = part * kChunk; k0 < mfull; k0 += split * kChunk) {
       float4 g4[kUnroll], r4[kUnroll];
       float q[kUnroll][4][CG];
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
-        const int64_t f = int64_t(row) * m + k0 + 64 * u + 4 * b;
+        const int64_t f = row * m + k0 + 64 * u + 4 * b;
         g4[u] = from_m ? ld4_stream(M + f) : ld4_stream(G + f);
         r4[u] = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_stream(R + f);
       }
@@ -119,7 +146,7 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args a) {
           }
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
-        const int64_t f = int64_t(row) * m + k0 + 64 * u + 4 * b;
+        const int64_t f = row * m + k0 + 64 * u + 4 * b;
         const float4 m4 = make_float4(g4[u].x + r4[u].x, g4[u].y + r4[u].y, g4[u].z + r4[u].z, g4[u].w + r4[u].w);
         if (!from_m) st4_stream(M + f, m4);  // the set of M matrices is far larger than the caches: do not allocate
         const float v[4] = {m4.x, m4.y, m4.z, m4.w};
@@ -130,23 +157,22 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args a) {
       }
     }
   }
-  for (int k0 = (rows_full ? mfull : 0) + wave * 64; k0 < m; k0 += kWaves * 64) {
+  for (int k0 = (rows_full ? mfull : 0) + part * 64; k0 < m; k0 += split * 64) {
     const int kk = k0 + 4 * b;
+    const int64_t f0 = row * m + kk;
     float v[4];
-    if (rows_full && k0 + 64 <= m) {
-      const int64_t f = int64_t(row) * m + kk;
-      const float4 g4 = from_m ? ld4_stream(M + f) : ld4_stream(G + f);
-      const float4 r4 = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_stream(R + f);
+    if (row < n && kk + 4 <= m && f0 + 4 <= N) {
+      const float4 g4 = from_m ? ld4_stream(M + f0) : ld4_stream(G + f0);
+      const float4 r4 = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_stream(R + f0);
       const float4 m4 = make_float4(g4.x + r4.x, g4.y + r4.y, g4.z + r4.z, g4.w + r4.w);
-      if (!from_m) st4(M + f, m4);
+      if (!from_m) st4(M + f0, m4);
       v[0] = m4.x; v[1] = m4.y; v[2] = m4.z; v[3] = m4.w;
     } else {
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        const int k = kk + t;
+        const int64_t f = f0 + t;
         float x = 0.f;
-        if (row < n && k < m) {
-          const int64_t f = int64_t(row) * m + k;
+        if (row < n && kk + t < m) {
           if (f < N && !from_m) {
             x = G[f] + R[f];
             M[f] = x;
@@ -180,22 +206,27 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args a) {
       if (lane < 4) s_p[wave][c][ii][lane] = x;
     }
   __syncthreads();
-  if (threadIdx.x < CG * 16) {
-    const int c = threadIdx.x / 16, ii = (threadIdx.x / 4) & 3, j = threadIdx.x & 3;
+  if (threadIdx.x < groups * CG * 16) {
+    const int grp = threadIdx.x / (CG * 16), e = threadIdx.x % (CG * 16);
+    const int c = e / 16, ii = (e / 4) & 3, j = e & 3;
+    const int64_t prow = tile_row + grp * 4 + ii;
     const int col = c * 4 + j;
-    if (row0 + ii < n && col < r) {
-      float x = s_p[0][c][ii][j];
-#pragma unroll
-      for (int w = 1; w < kWaves; w++) x += s_p[w][c][ii][j];
-      sg.P[int64_t(row0 + ii) * ld + col] = x;
+    if (prow < n && col < r) {
+      float x = s_p[grp * split][c][ii][j];
+      for (int w = 1; w < split; w++) x += s_p[grp * split + w][c][ii][j];
+      sg.P[prow * ld + col] = x;
     }
   }
 }
 
 // ---- encode2, step 1: orthonormalise the columns of P -------------------------
-// Modified Gram-Schmidt, two sweeps (the second restores orthogonality lost to
-// cancellation), reductions in fp64.  One workgroup per matrix; P is n x r <= 16.
+// One workgroup per matrix.  The factor is small (64 KB at 4096 x 4) and the launch is a chain of workgroup-wide
+// reductions, so what counts is how many there are: up to kGramCols columns need ONE, of all products of two columns
+// at once (gram_orth below); modified Gram-Schmidt, r + r(r-1)/2 reductions a sweep and two sweeps, is for wider
+// factors and for columns that nearly depend on each other.
 constexpr int kOrthThreads = 1024;
+constexpr int kOrthWaves = kOrthThreads / kWave;
+constexpr int kGramCols = 8;
 
 __device__ __forceinline__ double block_sum(double v, double* s_red) {
 #pragma unroll
@@ -244,53 +275,193 @@ __device__ __forceinline__ void gram_schmidt(const PView<LDS> P, double* s_red) 
   }
 }
 
-// Global-memory variant: any n x r.
-__global__ __launch_bounds__(kOrthThreads) void psgd_orth_kernel(const Args a) {
-  __shared__ double s_red[kOrthThreads / kWave];
-  const Seg& sg = a.seg[blockIdx.x];
-  gram_schmidt(PView<false>{sg.P, sg.n, sg.r}, s_red);
+// Sums of v[0 ... V-1] over the lanes of a wave, V a power of two up to 64: at every step a lane hands on the half of
+// its values that the lanes on the other side look after, so the wave exchanges about V values in all instead of 6 V.
+// Returns the sum of v[fold_index<V>(lane)].
+template <int V, int O = kWave / 2>
+__device__ __forceinline__ double wave_fold(const double (&v)[V], int lane) {
+  if constexpr (V > 1) {
+    const bool up = (lane & O) != 0;
+    double h[V / 2];
+#pragma unroll
+    for (int k = 0; k < V / 2; k++) {
+      const double send = up ? v[k] : v[k + V / 2], keep = up ? v[k + V / 2] : v[k];
+      h[k] = keep + __shfl_xor(send, O, kWave);
+    }
+    return wave_fold<V / 2, O / 2>(h, lane);
+  } else {
+    double x = v[0];
+#pragma unroll
+    for (int o = O; o >= 1; o /= 2) x += __shfl_xor(x, o, kWave);
+    return x;
+  }
+}
+template <int V>
+__device__ __forceinline__ int fold_index(int lane) { return lane / (kWave / V); }
+
+template <int C>
+__device__ __forceinline__ void load_row(float (&x)[C], const float* P, int64_t row, int n, int r) {
+  if (C == 4 && r == 4) {
+    const float4 v = row < n ? ld4(P + row * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+  } else {
+#pragma unroll
+    for (int c = 0; c < C; c++) x[c] = c < r && row < n ? P[row * r + c] : 0.f;
+  }
 }
 
-// LDS variant: the whole n x r factor (at most kOrthLdsFloats values) is staged in
-// dynamic shared memory, orthonormalised there and written back.
+// Orthonormalises the columns by way of their Gram matrix: G = P^T P in fp64 (the products of fp32 values are exact
+// there), G = R^T R, P <- P R^-1 in fp64 with one rounding to fp32 at the end.  What Gram-Schmidt computes, in other
+// words, from one pass over P for the sums and one for the result.  The columns come out orthonormal to about
+// n 2^-53 / (smallest R_cc^2 / G_cc); where that ratio is below 2^-20, so that this would come near fp32's own
+// rounding, or is no number, nothing is written and the answer is false.  A column of zeros stays zero.
+// us for 36 factors of 4096 or 1024 rows and 4 columns: 38 with Gram-Schmidt, now 12; 54 factors of 64 ... 2048 rows
+// and 2 columns: 2 x 10.7, now 7.3.
+template <int C>
+__device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
+  constexpr int kPairs = C * (C + 1) / 2;
+  constexpr int V = C <= 4 ? 16 : 64;
+  static_assert(kPairs <= V && C <= kGramCols, "pairs of columns");
+  __shared__ double s_part[kOrthWaves][V];
+  __shared__ double s_gram[V];
+  __shared__ double s_T[C][C];
+  __shared__ bool s_ok;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  double g[V];
+#pragma unroll
+  for (int k = 0; k < V; k++) g[k] = 0;
+  constexpr int kRows = 16 / C;  // loaded together: one row at a time the loop is a chain of memory latencies
+  for (int64_t row0 = threadIdx.x; row0 < n; row0 += kRows * kOrthThreads) {
+    float x[kRows][C];
+#pragma unroll
+    for (int u = 0; u < kRows; u++) load_row<C>(x[u], P, row0 + u * kOrthThreads, n, r);
+#pragma unroll
+    for (int u = 0; u < kRows; u++)
+#pragma unroll
+      for (int c = 0; c < C; c++)
+#pragma unroll
+        for (int d = 0; d <= c; d++) g[c * (c + 1) / 2 + d] = fma(double(x[u][c]), double(x[u][d]), g[c * (c + 1) / 2 + d]);
+  }
+  const double sum = wave_fold<V>(g, lane);
+  if (lane % (kWave / V) == 0) s_part[wave][fold_index<V>(lane)] = sum;
+  __syncthreads();
+  if (threadIdx.x < V) {
+    double x = 0;
+#pragma unroll
+    for (int w = 0; w < kOrthWaves; w++) x += s_part[w][threadIdx.x];
+    s_gram[threadIdx.x] = x;
+  }
+  __syncthreads();
+  // T = R^-1, upper triangular, column by column: with u = the first c columns of T applied to G's column c,
+  // R_kc = u_k, R_cc^2 = G_cc - sum u_k^2 and T's column c = (e_c - sum u_k T_k) / R_cc.  Every lane of the first wave
+  // computes (and reads back) the same T; it lies in LDS because 8 x 8 of them in registers spill.
+  if (wave == 0) {
+    bool ok = true;
+#pragma unroll 1
+    for (int c = 0; c < C; c++) {
+      const double gcc = s_gram[c * (c + 1) / 2 + c];
+      double d = gcc, t[C];
+#pragma unroll
+      for (int k = 0; k < C; k++) t[k] = k == c ? 1.0 : 0.0;
+#pragma unroll 1
+      for (int k = 0; k < c; k++) {
+        double u = 0;
+#pragma unroll
+        for (int l = 0; l < C; l++)
+          if (l <= k) u = fma(s_T[l][k], s_gram[c * (c + 1) / 2 + l], u);
+        d = fma(-u, u, d);
+#pragma unroll
+        for (int l = 0; l < C; l++)
+          if (l <= k) t[l] = fma(-u, s_T[l][k], t[l]);
+      }
+      double inv = 0;
+      if (gcc != 0) {
+        if (!(d >= gcc * 0x1p-20) || !(gcc < 0x1p300)) ok = false;
+        inv = 1.0 / sqrt(d);
+      }
+#pragma unroll
+      for (int l = 0; l < C; l++) s_T[l][c] = t[l] * inv;
+    }
+    s_ok = ok;
+  }
+  __syncthreads();
+  if (!s_ok) return false;
+  double T[kPairs];
+#pragma unroll
+  for (int c = 0; c < C; c++)
+#pragma unroll
+    for (int l = 0; l <= c; l++) T[c * (c + 1) / 2 + l] = s_T[l][c];
+  for (int64_t row0 = threadIdx.x; row0 < n; row0 += kRows * kOrthThreads) {
+    float x[kRows][C];
+#pragma unroll
+    for (int u = 0; u < kRows; u++) load_row<C>(x[u], P, row0 + u * kOrthThreads, n, r);
+#pragma unroll
+    for (int u = 0; u < kRows; u++) {
+      const int64_t row = row0 + u * kOrthThreads;
+#pragma unroll
+      for (int c = 0; c < C; c++) {
+        double y = 0;
+#pragma unroll
+        for (int l = 0; l <= c; l++) y = fma(double(x[u][l]), T[c * (c + 1) / 2 + l], y);
+        if (c < r && row < n) P[row * r + c] = float(y);
+      }
+    }
+  }
+  return true;
+}
+
+// WIDE: the call has factors of more than four columns that gram_orth takes.  LDS: every factor of the call (at most
+// kOrthLdsFloats values) fits dynamic shared memory, where Gram-Schmidt then works.
 constexpr int kOrthLdsFloats = 36 * 1024;  // 144 KiB of the 160 KiB LDS
-__global__ __launch_bounds__(kOrthThreads) void psgd_orth_lds_kernel(const Args a) {
-  __shared__ double s_red[kOrthThreads / kWave];
+template <bool WIDE, bool LDS, int CAP>
+__global__ __launch_bounds__(kOrthThreads) void psgd_orth_kernel(const Args<CAP> a) {
+  __shared__ double s_red[kOrthWaves];
   extern __shared__ float s_p[];
   const Seg& sg = a.seg[blockIdx.x];
   float* __restrict__ Pg = sg.P;
   const int n = sg.n, r = sg.r;
-  for (int e = threadIdx.x; e < n * r; e += kOrthThreads) s_p[(e % r) * n + e / r] = Pg[e];
-  __syncthreads();
-  gram_schmidt(PView<true>{s_p, n, r}, s_red);
-  __syncthreads();
-  for (int e = threadIdx.x; e < n * r; e += kOrthThreads) Pg[e] = s_p[(e % r) * n + e / r];
+  if (r <= 4) {
+    if (gram_orth<4>(Pg, n, r)) return;
+  } else if (WIDE && r <= kGramCols) {
+    if (gram_orth<kGramCols>(Pg, n, r)) return;
+  }
+  if constexpr (LDS) {
+    for (int e = threadIdx.x; e < n * r; e += kOrthThreads) s_p[(e % r) * n + e / r] = Pg[e];
+    __syncthreads();
+    gram_schmidt(PView<true>{s_p, n, r}, s_red);
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * r; e += kOrthThreads) Pg[e] = s_p[(e % r) * n + e / r];
+  } else {
+    gram_schmidt(PView<false>{Pg, n, r}, s_red);
+  }
 }
 
 // ---- encode2, step 2: Q = M^T P ------------------------------------------------
-// A workgroup takes a strip of 256 columns and 128 rows (32 per wave).  Per row a
+// A workgroup takes a strip of columns (256, or 128 or 64 with two or four rows side by side in a wave: strip_lanes)
+// and a.rows rows of it (two or four times that), the rows going round its waves.  Per row a
 // lane loads its 4 columns of M with one 128-bit load; register t of that load
 // is the A operand of MFMA t, whose block b / row-of-block i' is column
-// k0 + 16b + 4i' + t; the B operand is P[row][j] in every block.  The waves meet
+// k0 + 16b + 4i' + t; the B operand is P[row][j] in every block.  The waves (and the rows side by side) meet
 // in LDS and the workgroup writes one partial of Q; a second kernel adds the
 // partials in a fixed order.
-template <int CG>
-__global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args a) {
+template <int CG, int CAP>
+__global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
   const int tile = blockIdx.x;
-  const int s = find_segment<kMaxSeg>(a.tile_start, a.nseg, tile);
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
   const Seg& sg = a.seg[s];
   const float* __restrict__ M = sg.M;
   const float* __restrict__ P = sg.P;
   const int n = sg.n, m = sg.m, r = sg.r, ld = sg.ld;
-  const int strips = (m + kStrip - 1) / kStrip;
+  const int lanes = sg.split, side = kWave / lanes, width = 4 * lanes;
+  const int strips = (m + width - 1) / width;
   const int t_in = tile - a.tile_start[s];
   const int strip = t_in % strips, rblk = t_in / strips;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int k0 = strip * kStrip;
-  const int kk = k0 + 4 * lane;
-  const int rbeg = rblk * kE2RowsPerBlock + wave * (kE2RowsPerBlock / kWaves);
-  int rend = rbeg + kE2RowsPerBlock / kWaves;
-  if (rend > n) rend = n;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int k0 = strip * width;
+  const int kk = k0 + 4 * (lane & (lanes - 1));
+  const int step = kWaves * side;  // rows of the workgroup per round
+  const int64_t last = int64_t(rblk + 1) * a.rows * side;
+  const int64_t rend = last < n ? last : n;
 
   f32x4 acc[CG][4];
 #pragma unroll
@@ -298,50 +469,62 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args a) {
 #pragma unroll
     for (int t = 0; t < 4; t++) acc[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const bool cols_full = k0 + kStrip <= m;
   const int j = lane & 3;
-  int row = rbeg;
-  if (cols_full) {
-    // Main loop: 8 rows at a time, every load issued before the first use.
-    constexpr int kRows = 8;
-    for (; row + kRows <= rend; row += kRows) {
-      float4 m4[kRows];
-      float p[kRows][CG];
+  const int mine = lane / lanes;  // which of the rows side by side
+  int64_t row0 = int64_t(rblk) * a.rows * side + wave * side;  // the first of the wave's rows in a round
+  // Main loop: 8 rounds at a time, every load issued before the first use.  Only the lane that holds the row's end
+  // and those past it take the element-wise way.
+  constexpr int kRows = 8;
+  for (; row0 + (kRows - 1) * step + side <= rend; row0 += kRows * step) {
+    float4 m4[kRows];
+    float p[kRows][CG];
+    const float* Mp = M + (row0 + mine) * m + kk;
+    if (kk + 4 <= m) {
 #pragma unroll
-      for (int u = 0; u < kRows; u++) m4[u] = ld4_stream(M + int64_t(row + u) * m + kk);
-#pragma unroll
-      for (int u = 0; u < kRows; u++)
-#pragma unroll
-        for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[int64_t(row + u) * ld + c * 4 + j] : 0.f;
-#pragma unroll
-      for (int u = 0; u < kRows; u++) {
-        const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-#pragma unroll
-          for (int t = 0; t < 4; t++) acc[c][t] = mfma4(v[t], p[u][c], acc[c][t]);
-      }
-    }
-  }
-  for (; row < rend; row++) {
-    float v[4];
-    if (cols_full) {
-      const float4 m4 = ld4_stream(M + int64_t(row) * m + kk);
-      v[0] = m4.x; v[1] = m4.y; v[2] = m4.z; v[3] = m4.w;
+      for (int u = 0; u < kRows; u++) m4[u] = ld4_stream(Mp + int64_t(u) * step * m);
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; t++) v[t] = (kk + t < m) ? M[int64_t(row) * m + kk + t] : 0.f;
+      for (int u = 0; u < kRows; u++) {
+        const float* q = Mp + int64_t(u) * step * m;
+        m4[u] = make_float4(kk < m ? q[0] : 0.f, kk + 1 < m ? q[1] : 0.f, kk + 2 < m ? q[2] : 0.f, 0.f);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kRows; u++)
+#pragma unroll
+      for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[(row0 + u * step + mine) * ld + c * 4 + j] : 0.f;
+#pragma unroll
+    for (int u = 0; u < kRows; u++) {
+      const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
+#pragma unroll
+      for (int c = 0; c < CG; c++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc[c][t] = mfma4(v[t], p[u][c], acc[c][t]);
+    }
+  }
+  for (; row0 < rend; row0 += step) {
+    const int64_t row = row0 + mine;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (row < rend) {
+      const float* q = M + row * m + kk;
+      if (kk + 4 <= m) {
+        const float4 m4 = ld4_stream(q);
+        v[0] = m4.x; v[1] = m4.y; v[2] = m4.z; v[3] = m4.w;
+      } else {
+#pragma unroll
+        for (int t = 0; t < 3; t++) v[t] = kk + t < m ? q[t] : 0.f;
+      }
     }
 #pragma unroll
     for (int c = 0; c < CG; c++) {
       const int col = c * 4 + j;
-      const float p = col < r ? P[int64_t(row) * ld + col] : 0.f;
+      const float p = row < rend && col < r ? P[row * ld + col] : 0.f;
 #pragma unroll
       for (int t = 0; t < 4; t++) acc[c][t] = mfma4(v[t], p, acc[c][t]);
     }
   }
-  // acc[c][t][i'] in lane 4b+j  ->  Q[k0 + 16b + 4i' + t][4c + j]
-  __shared__ float s_q[kWaves][CG][kStrip][4];
+  // acc[c][t][i'] in lane 4b+j  ->  Q[k0 + (16b + 4i' + t) % width][4c + j], part (16b + 4i' + t) / width of the wave
+  __shared__ float s_q[kWaves][CG][4 * kWave][4];
 #pragma unroll
   for (int c = 0; c < CG; c++)
 #pragma unroll
@@ -350,43 +533,55 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args a) {
       for (int ii = 0; ii < 4; ii++) s_q[wave][c][16 * (lane >> 2) + 4 * ii + t][j] = acc[c][t][ii];
   __syncthreads();
   float* part = a.partials + (int64_t(sg.part_off) * 4) + int64_t(rblk) * m * r;
-  for (int e = threadIdx.x; e < CG * kStrip * 4; e += kThreads) {
-    const int c = e / (kStrip * 4), kl = (e / 4) % kStrip, jj = e & 3;
+  for (int e = threadIdx.x; e < CG * width * 4; e += kThreads) {
+    const int c = e / (width * 4), kl = (e / 4) & (width - 1), jj = e & 3;
     const int k = k0 + kl, col = c * 4 + jj;
     if (k < m && col < r) {
-      float x = s_q[0][c][kl][jj];
+      float x = 0.f;
+      for (int h = 0; h < side; h++)
 #pragma unroll
-      for (int w = 1; w < kWaves; w++) x += s_q[w][c][kl][jj];
+        for (int w = 0; w < kWaves; w++) x += s_q[w][c][h * width + kl][jj];
       part[int64_t(k) * r + col] = x;
     }
   }
 }
 
-__global__ __launch_bounds__(kThreads) void psgd_qreduce_kernel(const Args a) {
+template <int CAP>
+__global__ __launch_bounds__(kThreads) void psgd_qreduce_kernel(const Args<CAP> a) {
   const int tile = blockIdx.x;
-  const int s = find_segment<kMaxSeg>(a.tile_start, a.nseg, tile);
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
   const Seg& sg = a.seg[s];
   const int64_t mr = int64_t(sg.m) * sg.r;
-  const int nparts = (sg.n + kE2RowsPerBlock - 1) / kE2RowsPerBlock;
+  const int64_t per = int64_t(a.rows) * (kWave / sg.split);
+  const int nparts = int((sg.n + per - 1) / per);
   const float* part = a.partials + int64_t(sg.part_off) * 4;
   const int64_t e = int64_t(tile - a.tile_start[s]) * kThreads + threadIdx.x;
   if (e < mr) {
     float x = 0.f;
-    for (int p = 0; p < nparts; p++) x += part[int64_t(p) * mr + e];
+    int p = 0;
+    for (; p + 8 <= nparts; p += 8) {  // eight loads under way, added in their order
+      float y[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) y[u] = part[int64_t(p + u) * mr + e];
+#pragma unroll
+      for (int u = 0; u < 8; u++) x += y[u];
+    }
+    for (; p < nparts; p++) x += part[int64_t(p) * mr + e];
     sg.Qout[(e / sg.r) * sg.ld + e % sg.r] = x;
   }
 }
 
 // ---- decode: M = P Q^T, residual = grad - M, grad = M ---------------------------
-// A workgroup takes a strip of 256 columns and kDecRowsPerBlock rows (8 per wave).  MFMA
+// A workgroup takes a strip of 256 columns and kDecRowsPerBlock rows (8 per wave), or 128 or 64 columns and two or
+// four times the rows, two or four groups of four rows side by side in a wave (strip_lanes).  MFMA
 // (t, j) has A = P[row0+i'][j] and B = Q[k0+4*lane+t][j], so after the sum over
 // j register i' of accumulator t is M[row0+i'][k0+4*lane+t]: the four
 // accumulators give each lane 4 consecutive columns of 4 rows, i.e. 128-bit
 // loads of grad and 128-bit stores of M, residual and grad.
-template <int CG>
-__global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args a) {
+template <int CG, int CAP>
+__global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a) {
   const int tile = blockIdx.x;
-  const int s = find_segment<kMaxSeg>(a.tile_start, a.nseg, tile);
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
   const Seg& sg = a.seg[s];
   const float* __restrict__ P = sg.P;
   const float* __restrict__ Q = sg.Q;
@@ -396,15 +591,15 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args a) {
   const int n = sg.n, m = sg.m, r = sg.r, ld = sg.ld;
   const bool onto_m = (sg.mode & kOntoM) != 0, keep_grad = (sg.mode & kKeepGrad) != 0;
   const int64_t N = sg.numel;
-  const int strips = (m + kStrip - 1) / kStrip;
+  const int lanes = sg.split, side = kWave / lanes, width = 4 * lanes;
+  const int strips = (m + width - 1) / width;
   const int t_in = tile - a.tile_start[s];
   const int strip = t_in % strips, rblk = t_in / strips;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int k0 = strip * kStrip;
-  const int kk = k0 + 4 * lane;
-  const int rbeg = rblk * kDecRowsPerBlock + wave * (kDecRowsPerBlock / kWaves);
-  int rend = rbeg + kDecRowsPerBlock / kWaves;
-  if (rend > n) rend = n;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int kk = strip * width + 4 * (lane & (lanes - 1));
+  const int per_wave = kDecRowsPerBlock / kWaves * side;
+  const int64_t rbeg = (int64_t(rblk) * kWaves + wave) * per_wave;
+  const int64_t rend = rbeg + per_wave < n ? rbeg + per_wave : n;
   const int i = lane & 3;
 
   float q[4][CG * 4];  // Q[kk+t][col]
@@ -413,13 +608,13 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args a) {
 #pragma unroll
     for (int col = 0; col < CG * 4; col++) q[t][col] = (kk + t < m && col < r) ? Q[int64_t(kk + t) * ld + col] : 0.f;
 
-  const bool cols_full = k0 + kStrip <= m;
-  for (int row0 = rbeg; row0 < rend; row0 += 4) {
-    const bool full4 = cols_full && row0 + 4 <= rend && int64_t(row0 + 3) * m + kk + 4 <= N;
+  for (int64_t at = rbeg; at < rend; at += 4 * side) {
+    const int64_t row0 = at + 4 * (lane / lanes);
+    const bool full4 = kk + 4 <= m && row0 + 4 <= rend && (row0 + 3) * m + kk + 4 <= N;
     float4 g4[4];
     if (full4) {
 #pragma unroll
-      for (int ii = 0; ii < 4; ii++) g4[ii] = ld4_stream(G + int64_t(row0 + ii) * m + kk);
+      for (int ii = 0; ii < 4; ii++) g4[ii] = ld4_stream(G + (row0 + ii) * m + kk);
     }
     f32x4 acc[4];
 #pragma unroll
@@ -429,18 +624,18 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args a) {
       for (int ii = 0; ii < 4; ii++)
 #pragma unroll
         for (int t = 0; t < 4; t++)
-          if (row0 + ii < rend && kk + t < m) acc[t][ii] = M[int64_t(row0 + ii) * m + kk + t];
+          if (row0 + ii < rend && kk + t < m) acc[t][ii] = M[(row0 + ii) * m + kk + t];
     }
 #pragma unroll
     for (int col = 0; col < CG * 4; col++) {
-      const float p = (row0 + i < n && col < r) ? P[int64_t(row0 + i) * ld + col] : 0.f;
+      const float p = (row0 + i < n && col < r) ? P[(row0 + i) * ld + col] : 0.f;
 #pragma unroll
       for (int t = 0; t < 4; t++) acc[t] = mfma4(p, q[t][col], acc[t]);
     }
     if (full4) {
 #pragma unroll
       for (int ii = 0; ii < 4; ii++) {
-        const int64_t f = int64_t(row0 + ii) * m + kk;
+        const int64_t f = (row0 + ii) * m + kk;
         const float4 m4 = make_float4(acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]);
         const float4 r4 = make_float4(g4[ii].x - m4.x, g4[ii].y - m4.y, g4[ii].z - m4.z, g4[ii].w - m4.w);
         if (!keep_grad) {
@@ -453,9 +648,9 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args a) {
     }
 #pragma unroll
     for (int ii = 0; ii < 4; ii++) {
-      const int row = row0 + ii;
+      const int64_t row = row0 + ii;
       if (row >= rend) break;
-      const int64_t f = int64_t(row) * m + kk;
+      const int64_t f = row * m + kk;
       const float mv[4] = {acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]};
 #pragma unroll
       for (int t = 0; t < 4; t++) {
@@ -493,14 +688,173 @@ int check_dims(const char* who, const Batch& b, int* max_rank) {
 // the column groups of four it needs.
 inline int block_cols(int r, int c0) { return r <= c0 ? 0 : (r - c0 < kPassCols ? r - c0 : kPassCols); }
 
-#define PSGD_LAUNCH_CG_LDS(KERNEL, cg, grid, lds, st, args)                                                         \
-  switch (cg) {                                                                                                     \
-    case 1: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, KERNEL<1>, dim3(grid), dim3(kThreads), lds, st, args); break;  \
-    case 2: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, KERNEL<2>, dim3(grid), dim3(kThreads), lds, st, args); break;  \
-    case 3: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, KERNEL<3>, dim3(grid), dim3(kThreads), lds, st, args); break;  \
-    default: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, KERNEL<4>, dim3(grid), dim3(kThreads), lds, st, args); break; \
+// encode1: waves that share four rows of m columns.  A wave keeps 256 columns in flight, so a row of fewer than
+// 768 is one wave's work and one of fewer than 1536 two waves' (ResNet-50's matrices: 61 us with this rule; all
+// rows to four waves 64, to one or two 73); calls too small to
+// fill the chip spread their rows over as many workgroups as they can.
+inline int split_rows(int m, bool fills) { return !fills || m >= 1536 ? kWaves : m >= 768 ? kWaves / 2 : 1; }
+constexpr int64_t kFillGroups = 2048;  // groups of four rows that fill the chip: eight workgroups on each of 256 CUs
+
+#define PSGD_LAUNCH_CG_LDS(KERNEL, cg, grid, lds, st, args)                                                             \
+  switch (cg) {                                                                                                         \
+    case 1: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, (KERNEL<1, CAP>), dim3(grid), dim3(kThreads), lds, st, args); break;  \
+    case 2: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, (KERNEL<2, CAP>), dim3(grid), dim3(kThreads), lds, st, args); break;  \
+    case 3: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, (KERNEL<3, CAP>), dim3(grid), dim3(kThreads), lds, st, args); break;  \
+    default: HPX_LAUNCH_LDS(#KERNEL, hpx::g_prof_on, (KERNEL<4, CAP>), dim3(grid), dim3(kThreads), lds, st, args); break; \
   }
 #define PSGD_LAUNCH_CG(KERNEL, cg, grid, st, args) PSGD_LAUNCH_CG_LDS(KERNEL, cg, grid, 0, st, args)
+
+template <int CAP>
+int encode1_launches(int count, int max_rank, const float* const* grads, const int64_t* numels, const float* const* residuals,
+                     const float* const* Qs, float* const* Ms, float* const* Ps, const int32_t* ns, const int32_t* ms,
+                     const int32_t* rs, hipStream_t st) {
+  int64_t row_groups = 0;
+  for (int i = 0; i < count; i++) row_groups += cdiv(ns[i], 4);
+  const bool fills = row_groups >= kFillGroups;
+  Args<CAP> a;
+  a.partials = nullptr;
+  for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
+    int i = 0;
+    while (i < count) {
+      a.nseg = 0;
+      a.tile_start[0] = 0;
+      int cg = 1;
+      while (i < count && a.nseg < CAP) {
+        const int rb = block_cols(rs[i], c0);
+        if (rb == 0) { i++; continue; }
+        const int split = split_rows(ms[i], fills);
+        const int32_t t = cdiv(ns[i], 4 * (kWaves / split));
+        if (int64_t(a.tile_start[a.nseg]) + t > INT32_MAX) break;
+        a.seg[a.nseg] = Seg{grads[i], residuals[i], Qs[i] + c0, Ms[i], Ps[i] + c0, nullptr, numels[i], ns[i], ms[i], rb, 0,
+                            rs[i], c0 ? kFromM : 0, split};
+        if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
+        a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + t;
+        a.nseg++;
+        i++;
+      }
+      if (a.nseg == 0) continue;
+      // Two read streams and a write stream: held to four workgroups per CU (LDS the kernel never touches), 36 matrices
+      // of the layer set 598 us instead of 618 (five per CU: 607, three: 599), ResNet-50's 54 61.6 instead of 64.0.
+      PSGD_LAUNCH_CG_LDS(psgd_encode1_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds4, st, a);
+      HPX_HIP(hipGetLastError());
+    }
+  }
+  return HPX_OK;
+}
+
+template <bool WIDE, bool LDS, int CAP>
+int orth_launch(const Args<CAP>& a, size_t lds, hipStream_t st) {
+  if (lds)
+    HPX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(psgd_orth_kernel<WIDE, LDS, CAP>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+  HPX_LAUNCH_LDS("psgd_orth_kernel", hpx::g_prof_on, (psgd_orth_kernel<WIDE, LDS, CAP>), dim3(a.nseg), dim3(kOrthThreads), lds, st, a);
+  HPX_HIP(hipGetLastError());
+  return HPX_OK;
+}
+
+// Partials of a matrix: of `rows` rows each, as many times more as strips side by side in a wave.
+inline int32_t q_parts(int n, int m, int rows) { return cdiv(n, int64_t(rows) * (kWave / strip_lanes(m))); }
+
+template <int CAP>
+int encode2_launches(int count, int max_rank, int rows, float* partials, float* const* Ps, const float* const* Ms, float* const* Qs,
+                     const int32_t* ns, const int32_t* ms, const int32_t* rs, hipStream_t st) {
+  Args<CAP> a;
+  a.rows = rows;
+  a.partials = partials;
+  // step 1: orthonormalise every P over all of its columns
+  for (int i = 0; i < count;) {
+    a.nseg = 0;
+    int64_t max_nr = 0;
+    bool wide = false;
+    for (; i < count && a.nseg < CAP; i++) {
+      a.seg[a.nseg++] = Seg{nullptr, nullptr, nullptr, nullptr, Ps[i], nullptr, 0, ns[i], ms[i], rs[i], 0, rs[i], 0, 0};
+      if (int64_t(ns[i]) * rs[i] > max_nr) max_nr = int64_t(ns[i]) * rs[i];
+      wide = wide || (rs[i] > 4 && rs[i] <= kGramCols);
+    }
+    const bool fits = max_nr <= kOrthLdsFloats;
+    const size_t lds = fits ? size_t(max_nr) * sizeof(float) : 0;
+    const int rc = wide ? (fits ? orth_launch<true, true>(a, lds, st) : orth_launch<true, false>(a, lds, st))
+                        : (fits ? orth_launch<false, true>(a, lds, st) : orth_launch<false, false>(a, lds, st));
+    if (rc != HPX_OK) return rc;
+  }
+  // step 2: Q = M^T P, sixteen columns per pass over M
+  for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
+    int i = 0;
+    int64_t poff = 0;
+    while (i < count) {
+      a.nseg = 0;
+      a.tile_start[0] = 0;
+      int32_t red_start[CAP + 1];
+      red_start[0] = 0;
+      int cg = 1;
+      while (i < count && a.nseg < CAP) {
+        const int rb = block_cols(rs[i], c0);
+        if (rb == 0) { i++; continue; }
+        const int lanes = strip_lanes(ms[i]);
+        const int32_t parts = q_parts(ns[i], ms[i], rows);
+        const int64_t t = int64_t(cdiv(ms[i], 4 * lanes)) * parts;
+        const int32_t tr = cdiv(int64_t(ms[i]) * rb, kThreads);
+        if (a.tile_start[a.nseg] + t > INT32_MAX || int64_t(red_start[a.nseg]) + tr > INT32_MAX) {
+          HPX_ARG(a.nseg > 0, "hpx_powersgd_encode2: matrix %d is too large", i);
+          break;
+        }
+        a.seg[a.nseg] = Seg{nullptr, nullptr, nullptr, const_cast<float*>(Ms[i]), Ps[i] + c0, Qs[i] + c0, 0, ns[i], ms[i], rb,
+                            static_cast<int32_t>(poff), rs[i], 0, lanes};
+        poff += (int64_t(parts) * ms[i] * rb + 3) / 4;
+        if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
+        a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + int32_t(t);
+        red_start[a.nseg + 1] = red_start[a.nseg] + tr;
+        a.nseg++;
+        i++;
+      }
+      if (a.nseg == 0) continue;
+      PSGD_LAUNCH_CG(psgd_mtp_kernel, cg, a.tile_start[a.nseg], st, a);
+      HPX_HIP(hipGetLastError());
+      for (int k = 0; k <= a.nseg; k++) a.tile_start[k] = red_start[k];
+      HPX_LAUNCH("psgd_qreduce_kernel", psgd_qreduce_kernel<CAP>, dim3(a.tile_start[a.nseg]), dim3(kThreads), st, a);
+      HPX_HIP(hipGetLastError());
+    }
+  }
+  return HPX_OK;
+}
+
+template <int CAP>
+int decode_launches(int count, int max_rank, const float* const* Ps, const float* const* Qs, float* const* Ms, float* const* residuals,
+                    float* const* grads, const int64_t* numels, const int32_t* ns, const int32_t* ms, const int32_t* rs, hipStream_t st) {
+  Args<CAP> a;
+  a.partials = nullptr;
+  for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
+    int i = 0;
+    while (i < count) {
+      a.nseg = 0;
+      a.tile_start[0] = 0;
+      int cg = 1;
+      while (i < count && a.nseg < CAP) {
+        const int rb = block_cols(rs[i], c0);
+        if (rb == 0) { i++; continue; }
+        const int lanes = strip_lanes(ms[i]);
+        const int64_t t = int64_t(cdiv(ms[i], 4 * lanes)) * cdiv(ns[i], int64_t(kDecRowsPerBlock) * (kWave / lanes));
+        if (a.tile_start[a.nseg] + t > INT32_MAX) {
+          HPX_ARG(a.nseg > 0, "hpx_powersgd_decode: matrix %d is too large", i);
+          break;
+        }
+        const int32_t mode = (c0 ? kOntoM : 0) | (c0 + kPassCols < rs[i] ? kKeepGrad : 0);
+        a.seg[a.nseg] = Seg{grads[i], residuals[i], Qs[i] + c0, Ms[i], const_cast<float*>(Ps[i]) + c0, nullptr, numels[i], ns[i],
+                            ms[i], rb, 0, rs[i], mode, lanes};
+        if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
+        a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + int32_t(t);
+        a.nseg++;
+        i++;
+      }
+      if (a.nseg == 0) continue;
+      // One read and three writes per element: held to two workgroups per CU (LDS the kernel never touches,
+      // hpx_common.h), the 36 matrices of the configuration decode in 755 us instead of 792 (three per CU: 776).
+      PSGD_LAUNCH_CG_LDS(psgd_decode_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds2, st, a);
+      HPX_HIP(hipGetLastError());
+    }
+  }
+  return HPX_OK;
+}
 
 }  // namespace
 
@@ -521,32 +875,7 @@ HPX_API int hpx_powersgd_encode1(int count, const float* const* grads, const int
             static_cast<long long>(numels[i]));
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  Args a;
-  a.partials = nullptr;
-  for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
-    int i = 0;
-    while (i < count) {
-      a.nseg = 0;
-      a.tile_start[0] = 0;
-      int cg = 1;
-      while (i < count && a.nseg < kMaxSeg) {
-        const int rb = block_cols(rs[i], c0);
-        if (rb == 0) { i++; continue; }
-        const int32_t t = cdiv(ns[i], 4);
-        if (int64_t(a.tile_start[a.nseg]) + t > INT32_MAX) break;
-        a.seg[a.nseg] = Seg{grads[i], residuals[i], Qs[i] + c0, Ms[i], Ps[i] + c0, nullptr, numels[i], ns[i], ms[i], rb, 0,
-                            rs[i], c0 ? kFromM : 0};
-        if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
-        a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + t;
-        a.nseg++;
-        i++;
-      }
-      if (a.nseg == 0) continue;
-      PSGD_LAUNCH_CG(psgd_encode1_kernel, cg, a.tile_start[a.nseg], st, a);
-      HPX_HIP(hipGetLastError());
-    }
-  }
-  return HPX_OK;
+  return PSGD_BY_COUNT(encode1_launches, max_rank, grads, numels, residuals, Qs, Ms, Ps, ns, ms, rs, st);
 }
 
 HPX_API int hpx_powersgd_encode2(int count, float* const* Ps, const float* const* Ms, float* const* Qs,
@@ -558,11 +887,18 @@ HPX_API int hpx_powersgd_encode2(int count, float* const* Ps, const float* const
   int max_rank = 1;
   int rc = check_dims("hpx_powersgd_encode2", Batch{count, ns, ms, rs}, &max_rank);
   if (rc != HPX_OK) return rc;
-  int64_t part_quads = 0;  // partial storage in units of 4 floats (one pass at a time uses it)
-  for (int i = 0; i < count; i++) {
-    HPX_ARG(Ps[i] && Ms[i] && Qs[i], "hpx_powersgd_encode2: matrix %d has a null pointer", i);
-    part_quads += (int64_t(cdiv(ns[i], kE2RowsPerBlock)) * ms[i] * block_cols(rs[i], 0) + 3) / 4;
+  for (int i = 0; i < count; i++) HPX_ARG(Ps[i] && Ms[i] && Qs[i], "hpx_powersgd_encode2: matrix %d has a null pointer", i);
+  // Rows per partial: as many as leave four workgroups for each CU, since every partial is written and read back
+  // (36 matrices of the layer set: 5.0 us for adding them up instead of 12.7 with 128 rows; ResNet-50's 54 a pass 166 us,
+  // 170 with the line at eight workgroups per CU); few rows where the call is small, so that it spreads out.
+  int rows = kQRowsMax;
+  for (; rows > kQRowsMin; rows /= 2) {
+    int64_t tiles = 0;
+    for (int i = 0; i < count; i++) tiles += int64_t(cdiv(ms[i], 4 * strip_lanes(ms[i]))) * q_parts(ns[i], ms[i], rows);
+    if (tiles >= kQTiles) break;
   }
+  int64_t part_quads = 0;  // partial storage in units of 4 floats (one pass at a time uses it)
+  for (int i = 0; i < count; i++) part_quads += (int64_t(q_parts(ns[i], ms[i], rows)) * ms[i] * block_cols(rs[i], 0) + 3) / 4;
   HPX_ARG(part_quads <= INT32_MAX, "hpx_powersgd_encode2: batch too large for one call");
   hipStream_t st = static_cast<hipStream_t>(stream);
   hpx::Workspace* ws = hpx::workspace_record(st);
@@ -570,60 +906,8 @@ HPX_API int hpx_powersgd_encode2(int count, float* const* Ps, const float* const
   std::lock_guard<std::mutex> lock(ws->mu);
   rc = hpx::ensure_workspace(ws, size_t(part_quads) * 16);
   if (rc != HPX_OK) return rc;
-  Args a;
-  a.partials = reinterpret_cast<float*>(ws->dev);
-  // step 1: orthonormalise every P over all of its columns
-  for (int i = 0; i < count;) {
-    a.nseg = 0;
-    int64_t max_nr = 0;
-    for (; i < count && a.nseg < kMaxSeg; i++) {
-      a.seg[a.nseg++] = Seg{nullptr, nullptr, nullptr, nullptr, Ps[i], nullptr, 0, ns[i], ms[i], rs[i], 0, rs[i], 0};
-      if (int64_t(ns[i]) * rs[i] > max_nr) max_nr = int64_t(ns[i]) * rs[i];
-    }
-    if (max_nr <= kOrthLdsFloats) {
-      const size_t lds = size_t(max_nr) * sizeof(float);
-      HPX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(psgd_orth_lds_kernel),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-      HPX_LAUNCH_LDS("psgd_orth_kernel", hpx::g_prof_on, psgd_orth_lds_kernel, dim3(a.nseg), dim3(kOrthThreads), lds, st, a);
-    } else {
-      HPX_LAUNCH("psgd_orth_kernel", psgd_orth_kernel, dim3(a.nseg), dim3(kOrthThreads), st, a);
-    }
-    HPX_HIP(hipGetLastError());
-  }
-  // step 2: Q = M^T P, sixteen columns per pass over M
-  for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
-    int i = 0;
-    int64_t poff = 0;
-    while (i < count) {
-      a.nseg = 0;
-      a.tile_start[0] = 0;
-      int32_t red_start[kMaxSeg + 1];
-      red_start[0] = 0;
-      int cg = 1;
-      while (i < count && a.nseg < kMaxSeg) {
-        const int rb = block_cols(rs[i], c0);
-        if (rb == 0) { i++; continue; }
-        const int32_t t = cdiv(ms[i], kStrip) * cdiv(ns[i], kE2RowsPerBlock);
-        const int32_t tr = cdiv(int64_t(ms[i]) * rb, kThreads);
-        if (int64_t(a.tile_start[a.nseg]) + t > INT32_MAX || int64_t(red_start[a.nseg]) + tr > INT32_MAX) break;
-        a.seg[a.nseg] = Seg{nullptr, nullptr, nullptr, const_cast<float*>(Ms[i]), Ps[i] + c0, Qs[i] + c0, 0, ns[i], ms[i], rb,
-                            static_cast<int32_t>(poff), rs[i], 0};
-        poff += (int64_t(cdiv(ns[i], kE2RowsPerBlock)) * ms[i] * rb + 3) / 4;
-        if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
-        a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + t;
-        red_start[a.nseg + 1] = red_start[a.nseg] + tr;
-        a.nseg++;
-        i++;
-      }
-      if (a.nseg == 0) continue;
-      PSGD_LAUNCH_CG(psgd_mtp_kernel, cg, a.tile_start[a.nseg], st, a);
-      HPX_HIP(hipGetLastError());
-      for (int k = 0; k <= a.nseg; k++) a.tile_start[k] = red_start[k];
-      HPX_LAUNCH("psgd_qreduce_kernel", psgd_qreduce_kernel, dim3(a.tile_start[a.nseg]), dim3(kThreads), st, a);
-      HPX_HIP(hipGetLastError());
-    }
-  }
-  return HPX_OK;
+  float* partials = reinterpret_cast<float*>(ws->dev);
+  return PSGD_BY_COUNT(encode2_launches, max_rank, rows, partials, Ps, Ms, Qs, ns, ms, rs, st);
 }
 
 HPX_API int hpx_powersgd_decode(int count, const float* const* Ps, const float* const* Qs, float* const* Ms,
@@ -642,33 +926,5 @@ HPX_API int hpx_powersgd_decode(int count, const float* const* Ps, const float* 
             static_cast<long long>(numels[i]));
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  Args a;
-  a.partials = nullptr;
-  for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
-    int i = 0;
-    while (i < count) {
-      a.nseg = 0;
-      a.tile_start[0] = 0;
-      int cg = 1;
-      while (i < count && a.nseg < kMaxSeg) {
-        const int rb = block_cols(rs[i], c0);
-        if (rb == 0) { i++; continue; }
-        const int32_t t = cdiv(ms[i], kStrip) * cdiv(ns[i], kDecRowsPerBlock);
-        if (int64_t(a.tile_start[a.nseg]) + t > INT32_MAX) break;
-        const int32_t mode = (c0 ? kOntoM : 0) | (c0 + kPassCols < rs[i] ? kKeepGrad : 0);
-        a.seg[a.nseg] = Seg{grads[i], residuals[i], Qs[i] + c0, Ms[i], const_cast<float*>(Ps[i]) + c0, nullptr, numels[i], ns[i],
-                            ms[i], rb, 0, rs[i], mode};
-        if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
-        a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + t;
-        a.nseg++;
-        i++;
-      }
-      if (a.nseg == 0) continue;
-      // One read and three writes per element: held to two workgroups per CU (LDS the kernel never touches,
-      // hpx_common.h), the 36 matrices of the configuration decode in 755 us instead of 792 (three per CU: 776).
-      PSGD_LAUNCH_CG_LDS(psgd_decode_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds2, st, a);
-      HPX_HIP(hipGetLastError());
-    }
-  }
-  return HPX_OK;
+  return PSGD_BY_COUNT(decode_launches, max_rank, Ps, Qs, Ms, residuals, grads, numels, ns, ms, rs, st);
 }
