@@ -73,7 +73,9 @@ constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
 constexpr uint32_t kPickGather = 1536;   // a sample up to this size is gathered by the one workgroup that takes its threshold
 constexpr uint32_t kPickGatherBeside = 256;  // ... where the call has larger ones, and with them a gather launch, anyway
 constexpr uint32_t kPickMax = 65536;     // ... and up to this size its threshold is taken by one workgroup
-constexpr uint32_t kCutLds = 8192;       // candidates one workgroup sorts and cuts in LDS
+constexpr uint32_t kCutKeep = 8192;      // tensors that keep fewer entries than this are cut on the device ...
+constexpr uint32_t kCutLds = 16384;      // ... by one workgroup, which sorts up to this many candidates in LDS: a threshold taken
+                                         // from the 80th largest of a sample lets a tenth more or less through
 
 __host__ __device__ constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 __host__ __device__ constexpr uint32_t cdiv(uint64_t a, uint64_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
@@ -147,7 +149,7 @@ struct GdArgs {
   int32_t margin;               // provisional path: how many times the expected number of entries the provisional
                                 // threshold lets through
   uint32_t gather;              // the pick launch gathers samples of up to this size itself
-  int32_t device_cut;           // 1: tensors that keep fewer than kCutLds entries are cut on the device and report nothing
+  int32_t device_cut;           // 1: tensors that keep fewer than kCutKeep entries are cut on the device and report nothing
   int32_t tile_start[CAP + 1];  // exclusive prefix of this launch's workgroups per tensor
   GdSeg seg[CAP];
   uint32_t* report;             // pinned host memory, kReportWords per tensor of this table
@@ -372,10 +374,45 @@ __device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t
 // Replaces three histogram launches and a rank search: 1 M elements 15 us in four launches -> 5.2 us in one; ResNet-50's
 // 161 tensors 20 -> 7 us, and 4 us less in the gather launch before it.
 constexpr uint32_t kPickList = 1024;
+constexpr uint32_t kPickAll = 4096;   // listed by a second walk over the sample where the lanes' three largest do not do
+// wave_rank over keys of the whole workgroup, four a lane: a barrier a bit.  s_part: two rows of a word per wave.
+__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[4], uint32_t rank, uint32_t floor, uint32_t (*s_part)[kSelThreads / kWave]) {
+  constexpr int kWaves = kSelThreads / kWave;
+  const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  uint32_t top = 0;
+#pragma unroll
+  for (int j = 0; j < 4; j++) top = key[j] > top ? key[j] : top;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
+  if (lane == 0) s_part[0][wave] = top;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) top = s_part[0][w] > top ? s_part[0][w] : top;
+  top = __builtin_amdgcn_readfirstlane(top);
+  floor = __builtin_amdgcn_readfirstlane(floor);
+  const int first = 31 - __builtin_clz((top ^ floor) | 1u);   // bits above it are common to every candidate
+  uint32_t t = first < 31 ? (floor >> (first + 1)) << (first + 1) : 0u;
+  int row = 1;
+#pragma unroll 1
+  for (int b = first < 30 ? first : 30; b >= 0; b--, row ^= 1) {
+    const uint32_t c = t | (1u << b);
+    uint32_t reach = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) reach += uint32_t(__popcll(__ballot(key[j] >= c)));
+    if (lane == 0) s_part[row][wave] = reach;
+    __syncthreads();   // the row before it is not written again before everyone is past this one
+    reach = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) reach += s_part[row][w];
+    if (reach > rank) t = c;
+  }
+  return t;
+}
 template <int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> a) {
   __shared__ uint32_t s_hist[kBins1];              // the lanes' largest keys; the histogram of the other way
-  __shared__ __align__(16) uint32_t s_list[kPickList];
+  __shared__ __align__(16) uint32_t s_list[kPickAll];
+  __shared__ uint32_t s_part[2][kSelThreads / kWave];
   __shared__ uint32_t s_n, s_key;
   const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
@@ -462,8 +499,9 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
     if (t == 0) seg_state(sg)->thr_bits = bound;
     return;
   }
-  bool listed = sg.thr_index < uint32_t(kSelThreads) && bound != 0u;   // workgroup-uniform
-  if (listed) {
+  const bool bounded = sg.thr_index < uint32_t(kSelThreads) && bound != 0u;   // workgroup-uniform
+  // (from 256 keys above the bound on, some lane all but certainly holds four)
+  if (bounded && sg.thr_index < 256u) {
     if (__ballot(m1 >= bound) != 0) {   // most waves hold none
 #pragma unroll 1
       for (int j = 0; j < 3; j++) {
@@ -480,8 +518,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
     }
     __syncthreads();
     const uint32_t n = s_n;
-    listed = n <= kPickList;
-    if (listed) {
+    if (n <= kPickList) {
       if (wave == 0) {
         uint32_t found;
         if (n <= kWave) {
@@ -500,6 +537,57 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
         }
         if (lane == 0) seg_state(sg)->thr_bits = found;
       }
+      return;
+    }
+  }
+  if (bounded) {
+    // Every key from the bound on, by a second walk over the sample (out of the L2).  The histogram passes below would
+    // walk it three times, with most keys of a wave in the same few bins: samples of 8000 to 41000 for one entry in a
+    // hundred took this launch 35 us, now 23.
+    __syncthreads();
+    if (t == 0) s_n = 0;
+    __syncthreads();
+    const uint4* __restrict__ quads = reinterpret_cast<const uint4*>(samples);
+    const uint32_t last = (count - 1) / 4;
+#pragma unroll 1
+    for (uint32_t q0 = 0; 4 * q0 < count; q0 += 4 * kSelThreads) {
+      uint4 k[4];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t q = q0 + j * kSelThreads + t;
+        k[j] = quads[q < last ? q : last];
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t x = 4 * (q0 + j * kSelThreads + t);
+        const uint32_t v[4] = {k[j].x, k[j].y, k[j].z, k[j].w};
+        uint64_t in[4];
+        uint32_t all = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+          in[i] = __ballot(x + i < count && v[i] >= bound);
+          all += uint32_t(__popcll(in[i]));
+        }
+        if (all == 0) continue;
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(&s_n, all);
+        base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+          const uint32_t at = base + uint32_t(__popcll(in[i] & ((1ull << lane) - 1ull)));
+          if ((in[i] >> lane & 1u) && at < kPickAll) s_list[at] = v[i];
+          base += uint32_t(__popcll(in[i]));
+        }
+      }
+    }
+    __syncthreads();
+    const uint32_t n = s_n;
+    if (n <= kPickAll) {
+      uint32_t k[4];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) k[j] = j * kSelThreads + t < n ? s_list[j * kSelThreads + t] : 0u;
+      const uint32_t found = workgroup_rank(k, sg.thr_index, bound, s_part);
+      if (t == 0) seg_state(sg)->thr_bits = found;
       return;
     }
   }
@@ -936,7 +1024,7 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     }
     return;
   }
-  const bool cut_here = a.device_cut != 0 && sg.limit < kCutLds;
+  const bool cut_here = a.device_cut != 0 && sg.limit < kCutKeep;
   if (tile0 == 0 && lane == 0) seg_state(sg)->total = total;
   if (tile0 == 0 && a.report != nullptr && !cut_here) {
     // Pinned host words the host polls (no copy command, no wait for the stream).  The host waits for each
@@ -1181,25 +1269,51 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
     id[j] = x < n ? idx_in[x] : 0;
   }
   // bin t (first BINS lanes): pairs in all tiles, in the tiles before this one, in this one.
-  // The first 40 tiles (163,840 pairs) are read with independent loads.
+  // Up to 40 tiles (163,840 pairs) are read with independent loads.
   uint32_t total = 0, before = 0, mine = 0;
-  if (t < BINS) {
-    constexpr uint32_t kFlat = 40;
-    uint32_t c[kFlat];
+  constexpr uint32_t kFlat = 40;
+  if (nblk <= kFlat) {
+    if (t < BINS) {
+      uint32_t c[kFlat];
 #pragma unroll
-    for (uint32_t q = 0; q < kFlat; q++) c[q] = q < nblk ? counts[size_t(q) * BINS + t] : 0u;
+      for (uint32_t q = 0; q < kFlat; q++) c[q] = q < nblk ? counts[size_t(q) * BINS + t] : 0u;
 #pragma unroll
-    for (uint32_t q = 0; q < kFlat; q++) {
-      total += c[q];
-      before += q < blk ? c[q] : 0u;
-      mine += q == blk ? c[q] : 0u;
+      for (uint32_t q = 0; q < kFlat; q++) {
+        total += c[q];
+        before += q < blk ? c[q] : 0u;
+        mine += q == blk ? c[q] : 0u;
+      }
     }
-    for (uint32_t q = kFlat; q < nblk; q++) {
-      const uint32_t v = counts[size_t(q) * BINS + t];
-      total += v;
-      before += q < blk ? v : 0u;
-      mine += q == blk ? v : 0u;
+  } else {
+    // More tiles: shared out over all lanes, sixteen loads in flight in each (one bin's lane on its own, load after load,
+    // made a pass over 760 K pairs 43 us long; now 13).
+    constexpr uint32_t kShare = uint32_t(kSortThreads) / BINS, kRound = 16;
+    const uint32_t b = t % BINS, g = t / BINS;
+    for (uint32_t q0 = g; q0 < nblk; q0 += kShare * kRound) {
+      uint32_t c[kRound];
+#pragma unroll
+      for (uint32_t k = 0; k < kRound; k++) c[k] = q0 + k * kShare < nblk ? counts[size_t(q0 + k * kShare) * BINS + b] : 0u;
+#pragma unroll
+      for (uint32_t k = 0; k < kRound; k++) {
+        total += c[k];
+        before += q0 + k * kShare < blk ? c[k] : 0u;
+        mine += q0 + k * kShare == blk ? c[k] : 0u;
+      }
     }
+    s_stage[t] = total;
+    s_stage[kSortThreads + t] = before;
+    s_stage[2 * kSortThreads + t] = mine;
+    __syncthreads();
+    total = before = mine = 0;
+    if (t < BINS) {
+#pragma unroll
+      for (uint32_t k = 0; k < kShare; k++) {
+        total += s_stage[k * BINS + t];
+        before += s_stage[kSortThreads + k * BINS + t];
+        mine += s_stage[2 * kSortThreads + k * BINS + t];
+      }
+    }
+    __syncthreads();
   }
   if (msg) {
     // Last pass: if every key has the same digit the input is already in order.
@@ -1310,8 +1424,9 @@ __device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* s_wave, u
 // The `keep` largest |r| among the elements whose mask bit is set, in ascending index order, to LDS (keys as
 // distances from the threshold, the sign in the index's top bit): for a tensor with more candidates than fit.  A rank search over the candidates, then
 // one walk that lists those above the value found and the first ones equal to it.  Slow (one workgroup, four
-// walks over the mask) and all but never needed: a sampled threshold lets a few times the expected number
-// through only where the sample is a handful of values.
+// walks over the mask) and all but never needed: a sampled threshold lets twice the expected number
+// through only where the sample is a handful of values.  (While the workgroup held 8192 pairs, every other cut of a
+// tensor that keeps nearly as many came here: 23 tensors of 16.5 M, one in a hundred kept, 122-137 us; now 50-64.)
 __device__ __forceinline__ void top_of_masks(const uint64_t* __restrict__ masks, const float* __restrict__ r, uint32_t n, uint32_t keep,
                                              uint32_t thr_bits, uint32_t* s_hist, uint32_t* s_wave, uint32_t* s_key, uint32_t* s_id) {
   const uint32_t words = cdiv(n, kWave), t = threadIdx.x;
@@ -1362,7 +1477,7 @@ __device__ __forceinline__ void top_of_masks(const uint64_t* __restrict__ masks,
   __syncthreads();
 }
 
-// The cut by one workgroup, of up to kCutLds candidates.  What bounds it is the chain of workgroup-wide steps, so the sort
+// The cut by one workgroup, of up to kCutKeep candidates (listed ones: kCutLds, cut_wide).  What bounds it is the chain of workgroup-wide steps, so the sort
 // has as few as possible: the keys (distance of |r| above the threshold in bit patterns) go into 4096 bins by exponent
 // and seven further bits of the distance as a float - fine where keys crowd just above the threshold, however far the
 // largest lies - the bins are laid out one after the other, and a key's place is its bin's first place plus the number
@@ -1388,6 +1503,31 @@ struct CutArgs {
   }
 };
 
+__device__ __forceinline__ uint32_t cut_bin(uint32_t key) { return kCutBins - 1 - ((__float_as_uint(float(key)) >> 16) - (127u << 7)); }
+// From the counts of the bins to their first places, in place (all lanes, behind the barrier that follows the counting).
+// False: some bin is crowded, and the counts are still there.
+__device__ __forceinline__ bool bins_laid_out(const CutArgs& f) {
+  const uint32_t t = threadIdx.x;
+  const uint4 c = reinterpret_cast<const uint4*>(f.bins)[t];
+  const uint32_t c01 = c.x > c.y ? c.x : c.y, c23 = c.z > c.w ? c.z : c.w;
+  uint32_t total;
+  const uint32_t first = block_prefix(c.x + c.y + c.z + c.w, f.wave, total);
+  if (__syncthreads_or((c01 > c23 ? c01 : c23) > kCutCrowd)) return false;
+  reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
+  if (t == 0) f.bins[kCutBins] = total;
+  __syncthreads();
+  return true;
+}
+template <int PER>
+__device__ __forceinline__ void stage_pairs(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER]) {
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const uint32_t x = uint32_t(j) * kSortThreads + threadIdx.x;
+    if (x < f.n) { f.stage[x] = key[j]; f.stage[kCutLds + x] = id[j]; }
+  }
+  __syncthreads();
+}
+
 // n pairs, lane t with those at t, t + 1024 ... (in ascending index order; the sign in the index's top bit).  False: some
 // bin is crowded, nothing has been written, and the pairs are in LDS, [kCutLds] keys and then [kCutLds] indices.
 template <int PER>
@@ -1399,26 +1539,14 @@ __device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&k
 #pragma unroll
   for (int j = 0; j < PER; j++) {
     const bool live = uint32_t(j) * kSortThreads + t < n;
-    bin[j] = live ? kCutBins - 1 - ((__float_as_uint(float(key[j])) >> 16) - (127u << 7)) : 0u;
+    bin[j] = live ? cut_bin(key[j]) : 0u;
     slot[j] = live ? atomicAdd(&s_bins[bin[j]], 1u) : 0u;
   }
   __syncthreads();
-  const uint4 c = reinterpret_cast<const uint4*>(s_bins)[t];
-  const uint32_t c01 = c.x > c.y ? c.x : c.y, c23 = c.z > c.w ? c.z : c.w;
-  uint32_t total;
-  const uint32_t first = block_prefix(c.x + c.y + c.z + c.w, f.wave, total);
-  if (__syncthreads_or((c01 > c23 ? c01 : c23) > kCutCrowd)) {
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-      const uint32_t x = uint32_t(j) * kSortThreads + t;
-      if (x < n) { f.stage[x] = key[j]; f.stage[kCutLds + x] = id[j]; }
-    }
-    __syncthreads();
+  if (!bins_laid_out(f)) {
+    stage_pairs<PER>(f, key, id);
     return false;
   }
-  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
-  if (t == 0) s_bins[kCutBins] = total;
-  __syncthreads();
   uint32_t lo[PER], hi[PER], place[PER], longest = 0;
 #pragma unroll
   for (int j = 0; j < PER; j++) {
@@ -1443,10 +1571,56 @@ __device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&k
   return true;
 }
 
+// The same for up to kCutLds pairs that lie in memory, keys and indices: walked twice, once for the counts and once into
+// their bins, and then bin by bin (sixteen pairs a lane in registers, as above, spill).  Crowded bins: false, and nothing
+// is left in LDS.
+__device__ __forceinline__ bool cut_wide(const CutArgs& f, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cand) {
+  constexpr uint32_t kAtOnce = 4;
+  const uint32_t t = threadIdx.x, n = f.n;
+  uint2* s_pair = reinterpret_cast<uint2*>(f.stage);
+#pragma unroll 1
+  for (uint32_t x0 = t; x0 < n; x0 += kAtOnce * kSortThreads) {
+    uint32_t key[kAtOnce];
+#pragma unroll
+    for (uint32_t j = 0; j < kAtOnce; j++) key[j] = x0 + j * kSortThreads < n ? keys[x0 + j * kSortThreads] : 0u;
+#pragma unroll
+    for (uint32_t j = 0; j < kAtOnce; j++)
+      if (x0 + j * kSortThreads < n) atomicAdd(&f.bins[cut_bin(key[j])], 1u);
+  }
+  __syncthreads();
+  if (!bins_laid_out(f)) return false;
+#pragma unroll 1
+  for (uint32_t x0 = t; x0 < n; x0 += kAtOnce * kSortThreads) {
+    uint2 pair[kAtOnce];
+#pragma unroll
+    for (uint32_t j = 0; j < kAtOnce; j++) {
+      const uint32_t x = x0 + j * kSortThreads;
+      pair[j] = x < n ? make_uint2(keys[x], cand[x]) : make_uint2(0u, 0u);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kAtOnce; j++)
+      if (x0 + j * kSortThreads < n) s_pair[atomicAdd(&f.bins[cut_bin(pair[j].x)], 1u)] = pair[j];
+  }
+  __syncthreads();   // a bin's word is now the place behind its last pair
+#pragma unroll 1
+  for (uint32_t x = t; x < n; x += kSortThreads) {
+    const uint2 own = s_pair[x];
+    const uint32_t b = cut_bin(own.x), lo = b ? f.bins[b - 1] : 0u, hi = f.bins[b];
+    uint32_t place = lo;
+#pragma unroll 4
+    for (uint32_t q = lo; q < hi; q++) {
+      const uint2 k = s_pair[q];
+      place += k.x > own.x || (k.x == own.x && (k.y << 1) < (own.y << 1)) ? 1u : 0u;
+    }
+    if (place < f.keep) f.put(place, own.x, own.y);
+  }
+  return true;
+}
+
 // The same for many equal or nearly equal keys: the digit sort.
 __device__ __forceinline__ void cut_crowded(const CutArgs& f) {
   constexpr uint32_t BINS = 256, kBinWaves = BINS / kWave;
-  constexpr int kPer = int(kCutLds) / kSortThreads;
+  constexpr int kPer = int(kCutKeep) / kSortThreads;
   __shared__ uint32_t s_part[kBinWaves], s_max[kSortWaves];
   static_assert(kCutBins >= kSortWaves * BINS, "one block for both");
   uint32_t (*s_cnt)[BINS] = reinterpret_cast<uint32_t (*)[BINS]>(f.bins);
@@ -1565,7 +1739,7 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // count.
 constexpr uint32_t kFinishKeep = 2560;
 constexpr uint32_t kFinishTiles = kScanChunk;
-// The cut of the tensors that keep between kFinishKeep and kCutLds entries, whose candidates and keys the expand
+// The cut of the tensors that keep between kFinishKeep and kCutKeep entries, whose candidates and keys the expand
 // launch has listed (or, where they are too many for the list or for LDS, are found again in the mask).
 __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, uint32_t* s_bins, uint32_t* s_wave) {
   const uint32_t found = seg_state(sg)->total, keep = sg.limit, thr_bits = seg_state(sg)->thr_bits;
@@ -1573,19 +1747,27 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
   const uint32_t t = threadIdx.x;
   if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + keep * 8);
   if (keep == 0) return;
-  const bool listed = found <= sg.cap && found <= kCutLds;
+  const CutLayout cl = cut_layout(sg.cap);
+  const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(sg.cut + cl.ka);
+  const uint32_t* __restrict__ cand = reinterpret_cast<const uint32_t*>(sg.cut + cl.ia);
+  auto clear_bins = [&]() {
+    reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+  };
+  if (found <= sg.cap && found > kCutKeep && found <= kCutLds) {
+    clear_bins();
+    if (cut_wide(CutArgs{s_stage, s_bins, s_wave, sg.r, sg.out, found, keep, thr_bits}, keys, cand)) return;
+    __syncthreads();
+  }
+  const bool listed = found <= sg.cap && found <= kCutKeep;
   if (!listed) {
     const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
     top_of_masks(reinterpret_cast<const uint64_t*>(sg.ws + l.masks), sg.r, sg.n, keep, thr_bits, s_bins, s_wave, s_stage, s_stage + kCutLds);
   }
-  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
-  __syncthreads();
+  clear_bins();
   const CutArgs f{s_stage, s_bins, s_wave, sg.r, sg.out, listed ? found : keep, keep, thr_bits};
   bool done;
   if (listed) {
-    const CutLayout cl = cut_layout(sg.cap);
-    const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(sg.cut + cl.ka);
-    const uint32_t* __restrict__ cand = reinterpret_cast<const uint32_t*>(sg.cut + cl.ia);
     auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) { key = keys[x]; id = cand[x]; };
     done = f.n <= 2 * kSortThreads ? cut_loaded<2>(f, pair) : f.n <= 4 * kSortThreads ? cut_loaded<4>(f, pair) : cut_loaded<8>(f, pair);
   } else {
@@ -1648,7 +1830,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
   const bool cut = n > keep;
   if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + (cut ? keep : n) * 8);
   if (n == 0 || keep == 0) return;
-  if (n <= kCutLds) {
+  if (n <= kCutKeep) {
     auto list = [&](const uint32_t (&e)[4], const uint64_t (&m)[4]) {
 #pragma unroll
       for (int k = 0; k < 4; k++)
@@ -1873,7 +2055,7 @@ struct Plan {
 // workgroup (the same launch: its LDS holds what is kept); or the expand launch and the host, which queues the sort of
 // many workgroups once it has heard the count.  The provisional path keeps to the last: it may have to fall back.
 bool finishes(const GdSeg& sg, int margin) { return margin < 0 && sg.limit <= kFinishKeep && cdiv(sg.n, kTile) <= kFinishTiles; }
-bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutLds; }
+bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutKeep; }
 
 // The phases for up to CAP tensors, no host wait.  margin < 0: the threshold from the full gathered sample
 // (for samples of up to kPickMax one workgroup each, behind a gather launch where a sample exceeds kPickGather; for
