@@ -41,6 +41,7 @@ constexpr int kMaxCG = 4;                 // column groups of 4 -> rank <= 16
 // stores of a workgroup stay close together in time and address and the pass runs 10 % faster.
 constexpr int kQRowsMin = 32, kQRowsMax = 512;  // rows folded into one partial of Q (of a strip 256 columns wide)
 constexpr int64_t kQTiles = 1024;
+constexpr int64_t kDecTiles = 256;
 constexpr int kDecRowsPerBlock = 32;      // rows of a decode tile 256 columns wide (narrower tiles are as much taller)
 
 // encode2 and decode cut a matrix into strips of 4 * lanes columns; a wave lays kWave / lanes row groups of a strip
@@ -75,7 +76,7 @@ constexpr int32_t kKeepGrad = 4; // decode: more blocks follow: write M only, le
 template <int CAP>
 struct Args {
   int32_t nseg;
-  int32_t rows;        // encode2: rows folded into one partial of Q, of a strip 256 columns wide
+  int32_t rows;        // encode2: rows folded into one partial of Q, decode: rows of a tile (of a strip 256 columns wide)
   int32_t tile_start[CAP + 1];
   Seg seg[CAP];
   float* partials;
@@ -342,45 +343,49 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
 #pragma unroll
         for (int d = 0; d <= c; d++) g[c * (c + 1) / 2 + d] = fma(double(x[u][c]), double(x[u][d]), g[c * (c + 1) / 2 + d]);
   }
-  const double sum = wave_fold<V>(g, lane);
-  if (lane % (kWave / V) == 0) s_part[wave][fold_index<V>(lane)] = sum;
+  const int busy = n < kOrthThreads ? (n + kWave - 1) / kWave : kOrthWaves;  // waves that have a row
+  if (wave < busy) {
+    const double sum = wave_fold<V>(g, lane);
+    if (lane % (kWave / V) == 0) s_part[wave][fold_index<V>(lane)] = sum;
+  }
   __syncthreads();
   if (threadIdx.x < V) {
     double x = 0;
-#pragma unroll
-    for (int w = 0; w < kOrthWaves; w++) x += s_part[w][threadIdx.x];
+    for (int w = 0; w < busy; w++) x += s_part[w][threadIdx.x];
     s_gram[threadIdx.x] = x;
   }
   __syncthreads();
-  // T = R^-1, upper triangular, column by column: with u = the first c columns of T applied to G's column c,
-  // R_kc = u_k, R_cc^2 = G_cc - sum u_k^2 and T's column c = (e_c - sum u_k T_k) / R_cc.  Every lane of the first wave
-  // computes (and reads back) the same T; it lies in LDS because 8 x 8 of them in registers spill.
+  // Cholesky's factor of G and the inverse of it by elimination on [G | I], lane j of the first wave with column j of both
+  // halves.  Row k of the left half ends as R's, column l of the right half as R^-1's row l.
   if (wave == 0) {
     bool ok = true;
-#pragma unroll 1
-    for (int c = 0; c < C; c++) {
-      const double gcc = s_gram[c * (c + 1) / 2 + c];
-      double d = gcc, t[C];
+    const int col = lane < C ? lane : C - 1;
+    double A[C], Y[C];
 #pragma unroll
-      for (int k = 0; k < C; k++) t[k] = k == c ? 1.0 : 0.0;
-#pragma unroll 1
-      for (int k = 0; k < c; k++) {
-        double u = 0;
+    for (int k = 0; k < C; k++) {
+      A[k] = s_gram[k >= col ? k * (k + 1) / 2 + col : col * (col + 1) / 2 + k];
+      Y[k] = k == col ? 1.0 : 0.0;
+    }
 #pragma unroll
-        for (int l = 0; l < C; l++)
-          if (l <= k) u = fma(s_T[l][k], s_gram[c * (c + 1) / 2 + l], u);
-        d = fma(-u, u, d);
-#pragma unroll
-        for (int l = 0; l < C; l++)
-          if (l <= k) t[l] = fma(-u, s_T[l][k], t[l]);
-      }
+    for (int k = 0; k < C; k++) {
+      const double gkk = s_gram[k * (k + 1) / 2 + k], d = __shfl(A[k], k, kWave);
       double inv = 0;
-      if (gcc != 0) {
-        if (!(d >= gcc * 0x1p-20) || !(gcc < 0x1p300)) ok = false;
-        inv = 1.0 / sqrt(d);
+      if (gkk != 0) {
+        if (!(d >= gkk * 0x1p-20) || !(gkk < 0x1p300)) ok = false;
+        inv = rsqrt(d);
       }
+      A[k] *= inv;
+      Y[k] *= inv;
 #pragma unroll
-      for (int l = 0; l < C; l++) s_T[l][c] = t[l] * inv;
+      for (int i = k + 1; i < C; i++) {
+        const double f = __shfl(A[k], i, kWave);
+        A[i] = fma(-f, A[k], A[i]);
+        Y[i] = fma(-f, Y[k], Y[i]);
+      }
+    }
+    if (lane < C) {
+#pragma unroll
+      for (int k = 0; k < C; k++) s_T[lane][k] = Y[k];
     }
     s_ok = ok;
   }
@@ -532,7 +537,10 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
 #pragma unroll
       for (int ii = 0; ii < 4; ii++) s_q[wave][c][16 * (lane >> 2) + 4 * ii + t][j] = acc[c][t][ii];
   __syncthreads();
-  float* part = a.partials + (int64_t(sg.part_off) * 4) + int64_t(rblk) * m * r;
+  // the one partial of a matrix of few rows is Q itself
+  const bool whole = int64_t(a.rows) * side >= n;
+  float* part = whole ? sg.Qout : a.partials + (int64_t(sg.part_off) * 4) + int64_t(rblk) * m * r;
+  const int stride = whole ? ld : r;
   for (int e = threadIdx.x; e < CG * width * 4; e += kThreads) {
     const int c = e / (width * 4), kl = (e / 4) & (width - 1), jj = e & 3;
     const int k = k0 + kl, col = c * 4 + jj;
@@ -541,7 +549,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
       for (int h = 0; h < side; h++)
 #pragma unroll
         for (int w = 0; w < kWaves; w++) x += s_q[w][c][h * width + kl][jj];
-      part[int64_t(k) * r + col] = x;
+      part[int64_t(k) * stride + col] = x;
     }
   }
 }
@@ -597,7 +605,7 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
   const int strip = t_in % strips, rblk = t_in / strips;
   const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int kk = strip * width + 4 * (lane & (lanes - 1));
-  const int per_wave = kDecRowsPerBlock / kWaves * side;
+  const int per_wave = a.rows / kWaves * side;
   const int64_t rbeg = (int64_t(rblk) * kWaves + wave) * per_wave;
   const int64_t rend = rbeg + per_wave < n ? rbeg + per_wave : n;
   const int i = lane & 3;
@@ -793,7 +801,7 @@ int encode2_launches(int count, int max_rank, int rows, float* partials, float* 
         const int lanes = strip_lanes(ms[i]);
         const int32_t parts = q_parts(ns[i], ms[i], rows);
         const int64_t t = int64_t(cdiv(ms[i], 4 * lanes)) * parts;
-        const int32_t tr = cdiv(int64_t(ms[i]) * rb, kThreads);
+        const int32_t tr = parts > 1 ? cdiv(int64_t(ms[i]) * rb, kThreads) : 0;
         if (a.tile_start[a.nseg] + t > INT32_MAX || int64_t(red_start[a.nseg]) + tr > INT32_MAX) {
           HPX_ARG(a.nseg > 0, "hpx_powersgd_encode2: matrix %d is too large", i);
           break;
@@ -811,6 +819,7 @@ int encode2_launches(int count, int max_rank, int rows, float* partials, float* 
       PSGD_LAUNCH_CG(psgd_mtp_kernel, cg, a.tile_start[a.nseg], st, a);
       HPX_HIP(hipGetLastError());
       for (int k = 0; k <= a.nseg; k++) a.tile_start[k] = red_start[k];
+      if (a.tile_start[a.nseg] == 0) continue;
       HPX_LAUNCH("psgd_qreduce_kernel", psgd_qreduce_kernel<CAP>, dim3(a.tile_start[a.nseg]), dim3(kThreads), st, a);
       HPX_HIP(hipGetLastError());
     }
@@ -821,8 +830,16 @@ int encode2_launches(int count, int max_rank, int rows, float* partials, float* 
 template <int CAP>
 int decode_launches(int count, int max_rank, const float* const* Ps, const float* const* Qs, float* const* Ms, float* const* residuals,
                     float* const* grads, const int64_t* numels, const int32_t* ns, const int32_t* ms, const int32_t* rs, hipStream_t st) {
+  auto tiles_of = [&](int i, int rows) {
+    const int lanes = strip_lanes(ms[i]);
+    return int64_t(cdiv(ms[i], 4 * lanes)) * cdiv(ns[i], int64_t(rows) * (kWave / lanes));
+  };
+  int64_t tiles = 0;
+  for (int i = 0; i < count; i++) tiles += tiles_of(i, kDecRowsPerBlock);
   Args<CAP> a;
   a.partials = nullptr;
+  // Where the chip takes the whole call at once a wave has one group of rows, not one after the other.
+  a.rows = tiles < kDecTiles ? kDecRowsPerBlock / 2 : kDecRowsPerBlock;
   for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
     int i = 0;
     while (i < count) {
@@ -833,7 +850,7 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
         const int rb = block_cols(rs[i], c0);
         if (rb == 0) { i++; continue; }
         const int lanes = strip_lanes(ms[i]);
-        const int64_t t = int64_t(cdiv(ms[i], 4 * lanes)) * cdiv(ns[i], int64_t(kDecRowsPerBlock) * (kWave / lanes));
+        const int64_t t = tiles_of(i, a.rows);
         if (a.tile_start[a.nseg] + t > INT32_MAX) {
           HPX_ARG(a.nseg > 0, "hpx_powersgd_decode: matrix %d is too large", i);
           break;
