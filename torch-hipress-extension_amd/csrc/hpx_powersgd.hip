@@ -19,6 +19,8 @@
 // of columns of P and Q by an offset pointer, the block's width `r` and the factors' row stride `ld`; encode1
 // stores M in its first pass and reads it back in the others, decode builds M up over its passes and writes the
 // residual and the gradient in the last.
+#include <type_traits>
+
 #include "hpx_common.h"
 
 namespace {
@@ -83,6 +85,20 @@ struct Args {
 };
 static_assert(sizeof(Args<kSegLarge>) <= 18000, "kernel-argument budget");
 
+template <bool STREAM>
+__device__ __forceinline__ float4 ld4_as(const float* p) { return STREAM ? ld4_stream(p) : ld4(p); }
+template <bool STREAM>
+__device__ __forceinline__ void st4_as(float* p, float4 v) {
+  if (STREAM) st4_stream(p, v); else st4(p, v);
+}
+// Whether rows of m elements from these addresses on all start on a cache line.  Where they do not, the pieces of a row that
+// successive instructions move share lines: streaming accesses, which keep nothing in the caches, then fetch and write such a
+// line twice, and plain ones are the faster.  encode1 / decode of 1200 x 601 matrices 30.8 / 36.1 us streaming, 26.4 / 29.9
+// plain, of 2049 columns 25.4 / 28.1 and 20.4 / 23.0.
+__device__ __forceinline__ bool rows_on_lines(int m, const void* a, const void* b, const void* c) {
+  return ((uintptr_t(a) | uintptr_t(b) | uintptr_t(c) | uintptr_t(uint32_t(m)) * 4) & 127) == 0;
+}
+
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
@@ -125,7 +141,8 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
   for (int c = 0; c < CG; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const bool rows_full = (row0 + 3 < n) && ((row0 + 4) * m <= N);
-  if (rows_full) {
+  auto chunks = [&](auto stream) {
+    constexpr bool STREAM = decltype(stream)::value;
     // Main loop: kUnroll 64-column steps at a time, every load issued before the first use.
     for (int k0 = part * kChunk; k0 < mfull; k0 += split * kChunk) {
       float4 g4[kUnroll], r4[kUnroll];
@@ -133,8 +150,8 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
         const int64_t f = row * m + k0 + 64 * u + 4 * b;
-        g4[u] = from_m ? ld4_stream(M + f) : ld4_stream(G + f);
-        r4[u] = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_stream(R + f);
+        g4[u] = from_m ? ld4_as<STREAM>(M + f) : ld4_as<STREAM>(G + f);
+        r4[u] = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_as<STREAM>(R + f);
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; u++)
@@ -149,7 +166,7 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
       for (int u = 0; u < kUnroll; u++) {
         const int64_t f = row * m + k0 + 64 * u + 4 * b;
         const float4 m4 = make_float4(g4[u].x + r4[u].x, g4[u].y + r4[u].y, g4[u].z + r4[u].z, g4[u].w + r4[u].w);
-        if (!from_m) st4_stream(M + f, m4);  // the set of M matrices is far larger than the caches: do not allocate
+        if (!from_m) st4_as<STREAM>(M + f, m4);  // the set of M matrices is far larger than the caches: do not allocate
         const float v[4] = {m4.x, m4.y, m4.z, m4.w};
 #pragma unroll
         for (int t = 0; t < 4; t++)
@@ -157,44 +174,68 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
           for (int c = 0; c < CG; c++) acc[c] = mfma4(v[t], q[u][t][c], acc[c]);
       }
     }
+  };
+  if (rows_full) {
+    if (rows_on_lines(m, G, R, M)) chunks(std::true_type{}); else chunks(std::false_type{});
   }
-  for (int k0 = (rows_full ? mfull : 0) + part * 64; k0 < m; k0 += split * 64) {
-    const int kk = k0 + 4 * b;
-    const int64_t f0 = row * m + kk;
-    float v[4];
-    if (row < n && kk + 4 <= m && f0 + 4 <= N) {
-      const float4 g4 = from_m ? ld4_stream(M + f0) : ld4_stream(G + f0);
-      const float4 r4 = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_stream(R + f0);
-      const float4 m4 = make_float4(g4.x + r4.x, g4.y + r4.y, g4.z + r4.z, g4.w + r4.w);
-      if (!from_m) st4(M + f0, m4);
-      v[0] = m4.x; v[1] = m4.y; v[2] = m4.z; v[3] = m4.w;
-    } else {
+  // What is left of the columns (or everything, of rows that are not full), two steps' loads in flight together
+  // where the wave has several (four: as fast, but the registers they take slow the loop above): one step after the other, each waits for memory (encode1 of 1200 x 147 matrices
+  // 44 us, now 32).
+  const int rest = (rows_full ? mfull : 0) + part * 64;
+  auto steps = [&](auto unroll) {
+    constexpr int kSteps = decltype(unroll)::value;
+    for (int k0 = rest; k0 < m; k0 += split * 64 * kSteps) {
+      float4 g4[kSteps], r4[kSteps];
+      float q[kSteps][4][CG];
+      bool whole[kSteps];
 #pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int64_t f = f0 + t;
-        float x = 0.f;
-        if (row < n && kk + t < m) {
-          if (f < N && !from_m) {
-            x = G[f] + R[f];
-            M[f] = x;
-          } else {
-            x = M[f];  // beyond the gradient: whatever the caller left in M takes part in P = M Q
+      for (int u = 0; u < kSteps; u++) {
+        const int64_t kk = int64_t(k0) + u * split * 64 + 4 * b, f0 = row * m + kk;
+        whole[u] = row < n && kk + 4 <= m && f0 + 4 <= N;
+        if (whole[u]) {
+          g4[u] = from_m ? ld4(M + f0) : ld4(G + f0);
+          r4[u] = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4(R + f0);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+          for (int c = 0; c < CG; c++) {
+            const int col = c * 4 + i;  // B operand: lane 4b+j holds Q[k][j]
+            q[u][t][c] = (kk + t < m && col < r) ? Q[(kk + t) * ld + col] : 0.f;
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < kSteps; u++) {
+        const int64_t kk = int64_t(k0) + u * split * 64 + 4 * b, f0 = row * m + kk;
+        float v[4];
+        if (whole[u]) {
+          const float4 m4 = make_float4(g4[u].x + r4[u].x, g4[u].y + r4[u].y, g4[u].z + r4[u].z, g4[u].w + r4[u].w);
+          if (!from_m) st4(M + f0, m4);
+          v[0] = m4.x; v[1] = m4.y; v[2] = m4.z; v[3] = m4.w;
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            const int64_t f = f0 + t;
+            float x = 0.f;
+            if (row < n && kk + t < m) {
+              if (f < N && !from_m) {
+                x = G[f] + R[f];
+                M[f] = x;
+              } else {
+                x = M[f];  // beyond the gradient: whatever the caller left in M takes part in P = M Q
+              }
+            }
+            v[t] = x;
           }
         }
-        v[t] = x;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+          for (int c = 0; c < CG; c++) acc[c] = mfma4(v[t], q[u][t][c], acc[c]);
       }
     }
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      const int k = kk + t;
-#pragma unroll
-      for (int c = 0; c < CG; c++) {
-        const int col = c * 4 + i;  // B operand: lane 4b+j holds Q[k][j]
-        const float q = (k < m && col < r) ? Q[int64_t(k) * ld + col] : 0.f;
-        acc[c] = mfma4(v[t], q, acc[c]);
-      }
-    }
-  }
+  };
+  if (rest + split * 64 >= m) steps(std::integral_constant<int, 1>{}); else steps(std::integral_constant<int, 2>{});
   // acc[c][ii] in lane 4b+j is the part of P[row0+ii][4c+j] from this lane's columns: fold the 16 blocks
   __shared__ float s_p[kWaves][CG][4][4];
 #pragma unroll
@@ -616,62 +657,67 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
 #pragma unroll
     for (int col = 0; col < CG * 4; col++) q[t][col] = (kk + t < m && col < r) ? Q[int64_t(kk + t) * ld + col] : 0.f;
 
-  for (int64_t at = rbeg; at < rend; at += 4 * side) {
-    const int64_t row0 = at + 4 * (lane / lanes);
-    const bool full4 = kk + 4 <= m && row0 + 4 <= rend && (row0 + 3) * m + kk + 4 <= N;
-    float4 g4[4];
-    if (full4) {
+  // (two loops: of one loop with a choice at each store the compiler makes plain stores)
+  auto rows = [&](auto stream) {
+    constexpr bool STREAM = decltype(stream)::value;
+    for (int64_t at = rbeg; at < rend; at += 4 * side) {
+      const int64_t row0 = at + 4 * (lane / lanes);
+      const bool full4 = kk + 4 <= m && row0 + 4 <= rend && (row0 + 3) * m + kk + 4 <= N;
+      float4 g4[4];
+      if (full4) {
 #pragma unroll
-      for (int ii = 0; ii < 4; ii++) g4[ii] = ld4_stream(G + (row0 + ii) * m + kk);
-    }
-    f32x4 acc[4];
+        for (int ii = 0; ii < 4; ii++) g4[ii] = ld4_as<STREAM>(G + (row0 + ii) * m + kk);
+      }
+      f32x4 acc[4];
 #pragma unroll
-    for (int t = 0; t < 4; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (onto_m) {  // a later block of columns of a rank above 16: go on from what the earlier blocks left in M
+      for (int t = 0; t < 4; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (onto_m) {  // a later block of columns of a rank above 16: go on from what the earlier blocks left in M
 #pragma unroll
-      for (int ii = 0; ii < 4; ii++)
+        for (int ii = 0; ii < 4; ii++)
 #pragma unroll
-        for (int t = 0; t < 4; t++)
-          if (row0 + ii < rend && kk + t < m) acc[t][ii] = M[(row0 + ii) * m + kk + t];
-    }
+          for (int t = 0; t < 4; t++)
+            if (row0 + ii < rend && kk + t < m) acc[t][ii] = M[(row0 + ii) * m + kk + t];
+      }
 #pragma unroll
-    for (int col = 0; col < CG * 4; col++) {
-      const float p = (row0 + i < n && col < r) ? P[(row0 + i) * ld + col] : 0.f;
+      for (int col = 0; col < CG * 4; col++) {
+        const float p = (row0 + i < n && col < r) ? P[(row0 + i) * ld + col] : 0.f;
 #pragma unroll
-      for (int t = 0; t < 4; t++) acc[t] = mfma4(p, q[t][col], acc[t]);
-    }
-    if (full4) {
+        for (int t = 0; t < 4; t++) acc[t] = mfma4(p, q[t][col], acc[t]);
+      }
+      if (full4) {
+#pragma unroll
+        for (int ii = 0; ii < 4; ii++) {
+          const int64_t f = (row0 + ii) * m + kk;
+          const float4 m4 = make_float4(acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]);
+          const float4 r4 = make_float4(g4[ii].x - m4.x, g4[ii].y - m4.y, g4[ii].z - m4.z, g4[ii].w - m4.w);
+          if (!keep_grad) {
+            st4_as<STREAM>(R + f, r4);
+            st4_as<STREAM>(G + f, m4);  // in place over the line just read
+          }
+          st4(M + f, m4);  // plain: streaming this third store was measurably slower
+        }
+        continue;
+      }
 #pragma unroll
       for (int ii = 0; ii < 4; ii++) {
-        const int64_t f = (row0 + ii) * m + kk;
-        const float4 m4 = make_float4(acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]);
-        const float4 r4 = make_float4(g4[ii].x - m4.x, g4[ii].y - m4.y, g4[ii].z - m4.z, g4[ii].w - m4.w);
-        if (!keep_grad) {
-          st4_stream(R + f, r4);
-          st4_stream(G + f, m4);  // in place over the line just read
-        }
-        st4(M + f, m4);  // plain: streaming this third store was measurably slower
-      }
-      continue;
-    }
+        const int64_t row = row0 + ii;
+        if (row >= rend) break;
+        const int64_t f = row * m + kk;
+        const float mv[4] = {acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]};
 #pragma unroll
-    for (int ii = 0; ii < 4; ii++) {
-      const int64_t row = row0 + ii;
-      if (row >= rend) break;
-      const int64_t f = row * m + kk;
-      const float mv[4] = {acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]};
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        if (kk + t < m) {
-          if (f + t < N && !keep_grad) {
-            R[f + t] = G[f + t] - mv[t];
-            G[f + t] = mv[t];
+        for (int t = 0; t < 4; t++) {
+          if (kk + t < m) {
+            if (f + t < N && !keep_grad) {
+              R[f + t] = G[f + t] - mv[t];
+              G[f + t] = mv[t];
+            }
+            M[f + t] = mv[t];
           }
-          M[f + t] = mv[t];
         }
       }
     }
-  }
+  };
+  if (rows_on_lines(m, G, R, M)) rows(std::true_type{}); else rows(std::false_type{});
 }
 
 inline int32_t cdiv(int64_t x, int64_t y) { return static_cast<int32_t>((x + y - 1) / y); }
