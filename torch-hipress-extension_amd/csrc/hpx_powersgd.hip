@@ -162,6 +162,9 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
             const int col = c * 4 + i;  // B operand: lane 4b+j holds Q[k][j]
             q[u][t][c] = col < r ? Q[int64_t(k0 + 64 * u + 4 * b + t) * ld + col] : 0.f;
           }
+      f32x4 sum[CG];  // of this chunk, added to the rest afterwards: shorter chains of fp32 sums
+#pragma unroll
+      for (int c = 0; c < CG; c++) sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
         const int64_t f = row * m + k0 + 64 * u + 4 * b;
@@ -171,16 +174,18 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
-          for (int c = 0; c < CG; c++) acc[c] = mfma4(v[t], q[u][t][c], acc[c]);
+          for (int c = 0; c < CG; c++) sum[c] = mfma4(v[t], q[u][t][c], sum[c]);
       }
+#pragma unroll
+      for (int c = 0; c < CG; c++) acc[c] += sum[c];
     }
   };
   if (rows_full) {
     if (rows_on_lines(m, G, R, M)) chunks(std::true_type{}); else chunks(std::false_type{});
   }
-  // What is left of the columns (or everything, of rows that are not full), two steps' loads in flight together
-  // where the wave has several (four: as fast, but the registers they take slow the loop above): one step after the other, each waits for memory (encode1 of 1200 x 147 matrices
-  // 44 us, now 32).
+  // What is left of the columns (or everything, of rows that are not full), two steps' loads in flight together where the
+  // wave has several (four: as fast, but the registers they take slow the loop above): one step after the other, each
+  // waits for memory (encode1 of 1200 x 147 matrices 44 us, now 33).
   const int rest = (rows_full ? mfull : 0) + part * 64;
   auto steps = [&](auto unroll) {
     constexpr int kSteps = decltype(unroll)::value;
@@ -518,7 +523,8 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
   const int j = lane & 3;
   const int mine = lane / lanes;  // which of the rows side by side
   int64_t row0 = int64_t(rblk) * a.rows * side + wave * side;  // the first of the wave's rows in a round
-  // Main loop: 8 rounds at a time, every load issued before the first use.  Only the lane that holds the row's end
+  // Main loop: 8 rounds at a time, every load issued before the first use, summed on their own and added to what there is
+  // (one chain of fp32 sums down all rows of a partial of 512 left Q half as far again from the exact product).  Only the lane that holds the row's end
   // and those past it take the element-wise way.
   constexpr int kRows = 8;
   for (; row0 + (kRows - 1) * step + side <= rend; row0 += kRows * step) {
@@ -539,14 +545,23 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
     for (int u = 0; u < kRows; u++)
 #pragma unroll
       for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[(row0 + u * step + mine) * ld + c * 4 + j] : 0.f;
+    f32x4 sum[CG][4];
+#pragma unroll
+    for (int c = 0; c < CG; c++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) sum[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < kRows; u++) {
       const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
 #pragma unroll
       for (int c = 0; c < CG; c++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) acc[c][t] = mfma4(v[t], p[u][c], acc[c][t]);
+        for (int t = 0; t < 4; t++) sum[c][t] = mfma4(v[t], p[u][c], sum[c][t]);
     }
+#pragma unroll
+    for (int c = 0; c < CG; c++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) acc[c][t] += sum[c][t];
   }
   for (; row0 < rend; row0 += step) {
     const int64_t row = row0 + mine;
@@ -587,9 +602,11 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
     const int k = k0 + kl, col = c * 4 + jj;
     if (k < m && col < r) {
       float x = 0.f;
-      for (int h = 0; h < side; h++)
-#pragma unroll
-        for (int w = 0; w < kWaves; w++) x += s_q[w][c][h * width + kl][jj];
+      static_assert(kWaves == 4, "summed in pairs");
+      for (int h = 0; h < side; h++) {
+        const int l = h * width + kl;
+        x += (s_q[0][c][l][jj] + s_q[1][c][l][jj]) + (s_q[2][c][l][jj] + s_q[3][c][l][jj]);
+      }
       part[int64_t(k) * stride + col] = x;
     }
   }
@@ -608,12 +625,11 @@ __global__ __launch_bounds__(kThreads) void psgd_qreduce_kernel(const Args<CAP> 
   if (e < mr) {
     float x = 0.f;
     int p = 0;
-    for (; p + 8 <= nparts; p += 8) {  // eight loads under way, added in their order
+    for (; p + 8 <= nparts; p += 8) {  // eight loads under way, added in pairs (a chain over all partials is less exact)
       float y[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) y[u] = part[int64_t(p + u) * mr + e];
-#pragma unroll
-      for (int u = 0; u < 8; u++) x += y[u];
+      x += ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
     }
     for (; p < nparts; p++) x += part[int64_t(p) * mr + e];
     sg.Qout[(e / sg.r) * sg.ld + e % sg.r] = x;
