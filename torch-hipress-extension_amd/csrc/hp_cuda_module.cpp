@@ -147,7 +147,10 @@ bool submit_args(PyObject* const* a, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "submit_task(): incompatible function arguments");
     throw PyError{};
   }
-  const char* name = PyUnicode_Check(a[0]) ? PyUnicode_AsUTF8(a[0]) : nullptr;
+  const char* name = PyUnicode_Check(a[0]) ? PyUnicode_AsUTF8(a[0])
+                     : PyBytes_Check(a[0]) ? PyBytes_AS_STRING(a[0])
+                     : PyByteArray_Check(a[0]) ? PyByteArray_AS_STRING(a[0])
+                                               : nullptr;
   if (!name) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "submit_task(): incompatible function arguments: the name must be a string");
     throw PyError{};
@@ -197,9 +200,12 @@ PyObject* submit_task(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return nullptr;
 }
 PyMethodDef g_submit_task = {"submit_task", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&submit_task)), METH_FASTCALL,
-                             "submit_task(name, tensor, B, C, is_root, task_id)\n"
-                             "submit_task(name, tensor, residual, B, C, is_root, task_id)\n"
-                             "submit_task(name, tensor, residual, M, P, Q, task_id)\n\nFalse, with the reason printed, if the task is refused."};
+                             "submit_task(*args)\nOverloaded function.  False, with the reason printed, if the task is refused.\n\n"
+                             "1. submit_task(name: str, tensor: torch.Tensor, B: torch.Tensor, C: torch.Tensor, is_root: int, task_id: int) -> bool\n\n"
+                             "2. submit_task(name: str, tensor: torch.Tensor, residual: torch.Tensor, B: torch.Tensor, C: torch.Tensor, "
+                             "is_root: int, task_id: int) -> bool\n\n"
+                             "3. submit_task(name: str, tensor: torch.Tensor, residual: torch.Tensor, M: torch.Tensor, P: torch.Tensor, "
+                             "Q: torch.Tensor, task_id: int) -> bool\n"};
 
 std::vector<std::string> get_results(int task_id) {
   std::vector<std::string> out;
