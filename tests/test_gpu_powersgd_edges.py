@@ -67,7 +67,7 @@ def test_ranks_around_the_gram_matrix(psgd, r):
 
 @pytest.mark.parametrize("r", [2, 4, 8])
 def test_columns_that_depend_on_each_other(psgd, r):
-    # The last column is the first plus `eps` of something else: with eps 1e-2 (squared far above 2^-20) the Gram matrix
+    # The last column is the first plus `eps` of something else: with eps 1e-2 the Gram matrix
     # decides, with 1e-5 Gram-Schmidt does; either way the columns are orthonormal and span what they spanned.  A column
     # of zeros stays one and leaves the others alone; a NaN reaches the columns from its own on.
     rng = np.random.default_rng(r)
@@ -94,3 +94,23 @@ def test_columns_that_depend_on_each_other(psgd, r):
     psgd.encode2([dP], [dev(M)], [dQ])
     got = host(dP)
     assert np.isnan(got[:, r - 1]).all() and not np.isnan(got[:, :r - 1]).any()
+
+
+@pytest.mark.parametrize("r,delta", [(4, 2.0 ** -7), (4, 0.01), (4, 0.1), (6, 2.0 ** -5), (8, 2.0 ** -3), (8, 0.05), (8, 0.3)])
+@pytest.mark.parametrize("n", [1000, 4100, 100_003])
+def test_chain_of_columns(psgd, n, r, delta):
+    # c_1 = u_1, c_k+1 = u_k + delta u_k+1 of independent u: no column loses much to those before it, the inverse of R grows
+    # with the product of all losses.  Either way of orthonormalising has to leave the columns orthonormal to fp32:
+    # Gram-Schmidt's two sweeps in fp32 leave at most about 2 r roundings of 2^-24.
+    rng = np.random.default_rng(int(1 / delta) * r + n)
+    u = rng.normal(0, 1, (n, r))
+    P = u.copy()
+    P[:, 1:] = u[:, :-1] + delta * u[:, 1:]
+    P = P.astype(np.float32)
+    M = rng.normal(0, 1, (n, 12)).astype(np.float32)
+    dP, dQ = dev(P), torch.zeros(12, r, device="cuda")
+    psgd.encode2([dP], [dev(M)], [dQ])
+    got = host(dP).astype(np.float64)
+    assert np.abs(got.T @ got - np.eye(r)).max() < 2 * r * 2.0 ** -24
+    assert np.linalg.norm(P - got @ (got.T @ P.astype(np.float64))) / np.linalg.norm(P) < 1e-6
+    assert ps.rel_fro(host(dQ), M.astype(np.float64).T @ got) < 1e-5

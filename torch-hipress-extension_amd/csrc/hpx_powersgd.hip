@@ -358,10 +358,15 @@ __device__ __forceinline__ void load_row(float (&x)[C], const float* P, int64_t 
 }
 
 // Orthonormalises the columns by way of their Gram matrix: G = P^T P in fp64 (the products of fp32 values are exact
-// there), G = R^T R, P <- P R^-1 in fp64 with one rounding to fp32 at the end.  What Gram-Schmidt computes, in other
-// words, from one pass over P for the sums and one for the result.  The columns come out orthonormal to about
-// n 2^-53 / (smallest R_cc^2 / G_cc); where that ratio is below 2^-20, so that this would come near fp32's own
-// rounding, or is no number, nothing is written and the answer is false.  A column of zeros stays zero.
+// there), G = R^T R, P <- P R^-1 in fp64 with one rounding to fp32 at the end: one pass over P for the sums and one for
+// the result.  What the sums, the elimination and the product round away is at most k 2^-53 sqrt(G_ii G_jj) in the entries
+// of G and comes out multiplied by R^-1 from both sides: with s_c = sum over l of |R^-1_lc| sqrt(G_ll) the columns are
+// orthonormal to k 2^-53 s_c^2, k the length of the longest chain of sums (the n / 1024 rows of a lane, the fold over lanes
+// and waves, the elimination: 32 for all but the first).  s_c is about 1 for columns that have little to do with each other
+// and grows with the product of what the columns before lose to each other, not only with each one's own loss: a chain
+// c_1 = u_1, c_k+1 = u_k + 0.05 u_k+1 of eight columns keeps every R_cc^2 above 2^-10 G_cc, and its P R^-1 is no
+// orthonormal matrix at all.  Where k s_c^2 exceeds 2^27 (2^-26 in the products of columns, a quarter of fp32's own rounding), or is no number,
+// nothing is written and the answer is false.  A column of zeros stays zero.
 // us for 36 factors of 4096 or 1024 rows and 4 columns: 38 with Gram-Schmidt, now 12; 54 factors of 64 ... 2048 rows
 // and 2 columns: 2 x 10.7, now 7.3.
 template <int C>
@@ -372,7 +377,7 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
   __shared__ double s_part[kOrthWaves][V];
   __shared__ double s_gram[V];
   __shared__ double s_T[C][C];
-  __shared__ bool s_ok;
+  __shared__ double s_norm[C];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   double g[V];
 #pragma unroll
@@ -404,7 +409,6 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
   // Cholesky's factor of G and the inverse of it by elimination on [G | I], lane j of the first wave with column j of both
   // halves.  Row k of the left half ends as R's, column l of the right half as R^-1's row l.
   if (wave == 0) {
-    bool ok = true;
     const int col = lane < C ? lane : C - 1;
     double A[C], Y[C];
 #pragma unroll
@@ -414,12 +418,8 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
     }
 #pragma unroll
     for (int k = 0; k < C; k++) {
-      const double gkk = s_gram[k * (k + 1) / 2 + k], d = __shfl(A[k], k, kWave);
-      double inv = 0;
-      if (gkk != 0) {
-        if (!(d >= gkk * 0x1p-20) || !(gkk < 0x1p300)) ok = false;
-        inv = rsqrt(d);
-      }
+      const double d = __shfl(A[k], k, kWave);
+      const double inv = s_gram[k * (k + 1) / 2 + k] != 0 ? rsqrt(d) : 0;  // of what is not above zero: no number, or infinite
       A[k] *= inv;
       Y[k] *= inv;
 #pragma unroll
@@ -432,16 +432,24 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
     if (lane < C) {
 #pragma unroll
       for (int k = 0; k < C; k++) s_T[lane][k] = Y[k];
+      s_norm[lane] = sqrt(s_gram[lane * (lane + 1) / 2 + lane]);
     }
-    s_ok = ok;
   }
   __syncthreads();
-  if (!s_ok) return false;
   double T[kPairs];
+  bool ok = true;
+  const double limit = 0x1p27 / (32 + (n - 1) / kOrthThreads + 1);
 #pragma unroll
-  for (int c = 0; c < C; c++)
+  for (int c = 0; c < C; c++) {
+    double s = 0;
 #pragma unroll
-    for (int l = 0; l <= c; l++) T[c * (c + 1) / 2 + l] = s_T[l][c];
+    for (int l = 0; l <= c; l++) {
+      T[c * (c + 1) / 2 + l] = s_T[l][c];
+      s = fma(fabs(T[c * (c + 1) / 2 + l]), s_norm[l], s);
+    }
+    ok = ok && s * s <= limit;
+  }
+  if (!ok) return false;  // the same in every thread
   for (int64_t row0 = threadIdx.x; row0 < n; row0 += kRows * kOrthThreads) {
     float x[kRows][C];
 #pragma unroll
