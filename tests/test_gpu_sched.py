@@ -381,3 +381,60 @@ def test_task_with_too_small_buffers_is_skipped_counted_and_still_named(hp):
     _collect(hp, 20, ["tiny"])
     assert hp.error_count() == before + 1 and "does not fit" in hp.last_error()
     assert float(g.abs().max()) > 0 and int(Cc.sum()) == 0           # nothing was decoded, nothing written
+
+
+def test_tasks_on_views_that_overlap(hp, oracle_cpu):
+    # Messages of more than 1 MB, so that every task is a run of its own; all submitted in one go.  What a task sees must
+    # not depend on how the worker's batches and runs fall, also where the memory two tasks share starts at different
+    # addresses.  The threshold is a power of two and the tensors hold few multiples of it: sums are exact in any order.
+    rng = np.random.default_rng(17)
+    n, thr, size, rank = (4 << 20) + 40, 2.0 ** -7, 3, 1
+    assert hp.init("tbq", {"threshold": thr}, 0, rank, size)
+    mb = oracle_cpu.tbq_packed_size(n)
+    message = lambda: oracle_cpu.tbq_encode(rng.normal(0, 2 * thr, n).astype(np.float32), np.zeros(n, np.float32), thr)
+    dev_bytes = lambda: torch.zeros(mb, dtype=torch.uint8, device="cuda")
+    msgs = [message() for _ in range(6)]
+    Cs = [_host_buf(mb, 1) for _ in msgs]
+    for C, m in zip(Cs, msgs):
+        C.numpy()[:] = m
+    Bs = [dev_bytes() for _ in msgs]
+    slots = np.concatenate([message() for _ in range(size)])
+    Cg = _host_buf(size * mb, 1); Cg.numpy()[:] = slots
+
+    # six windows, each on half of the one before, added into one bucket
+    flat = torch.zeros(n // 2 * 7, device="cuda")
+    windows = [flat[n // 2 * k:n // 2 * k + n] for k in range(6)]
+    # then a slice of the bucket as a gradient: it holds the sums
+    at, ln = n // 4 + 3, n * 3
+    lmb = oracle_cpu.tbq_packed_size(ln)
+    res, Bl, Cl = torch.zeros(ln, device="cuda"), torch.zeros(lmb, dtype=torch.uint8, device="cuda"), _host_buf(lmb, 1)
+    # a slot of a gathered buffer, then the aggregation that overwrites it
+    one, grad, gres = torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda")
+    B1, B2 = dev_bytes(), dev_bytes()
+    torch.cuda.synchronize()
+    for k in range(6):
+        assert hp.submit_task(f"add{k}", windows[k], Bs[k], Cs[k], 1, 20)
+    assert hp.submit_task("slice", flat[at:at + ln], res, Bl, Cl, 0, 10)
+    assert hp.submit_task("slot", one, B1, Cg[:mb], 0, 20)
+    assert hp.submit_task("root", grad, gres, B2, Cg, 1, 30)
+    _collect(hp, 20, [f"add{k}" for k in range(6)] + ["slot"])
+    _collect(hp, 10, ["slice"])
+    _collect(hp, 30, ["root"])
+
+    want = np.zeros(flat.numel(), np.float32)
+    for k, m in enumerate(msgs):
+        want[n // 2 * k:n // 2 * k + n] += oracle_cpu.tbq_decode(m, n, thr)
+    assert_bits_equal(host(flat), want, "windows added into one bucket")
+    rr = np.zeros(ln, np.float32)
+    assert_bits_equal(Cl.numpy(), oracle_cpu.tbq_encode(want[at:at + ln], rr, thr), "message of the slice")
+    assert_bits_equal(host(res), rr, "residual of the slice")
+    assert_bits_equal(host(one), oracle_cpu.tbq_decode(slots[:mb], n, thr), "slot of the gathered buffer as it was received")
+    total = np.zeros(n, np.float32)
+    for i in range(size):
+        if i != rank:
+            total = oracle_cpu.tbq_decode(slots[i * mb:(i + 1) * mb], n, thr, total, 1)
+    rr = np.zeros(n, np.float32)
+    msg = oracle_cpu.tbq_encode(total, rr, thr)
+    assert_bits_equal(host(grad), total, "aggregated gradient"); assert_bits_equal(host(gres), rr, "its residual")
+    assert_bits_equal(Cg.numpy(), np.concatenate([msg, slots[mb:]]), "gathered buffer afterwards")
+    assert hp.error_count() == 0, hp.last_error()

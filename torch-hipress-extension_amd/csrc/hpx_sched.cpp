@@ -14,8 +14,9 @@
 //
 // A run's kernels follow each other on one stream, so no stream ever waits for another (with a compute and a data stream
 // the two event calls per run cost the worker 20 us, more than its launches).  Runs are independent of each other
-// because no tensor, residual, B or C is in two of them: a batch in which one is (a root task's tensor is decoded and then
-// encoded) stays on one lane, and a batch that names one still in use by an earlier batch waits for that.
+// because no byte of a tensor, residual, B or C is in two of them (hpx_task_ranges.h): a batch in which one is (a root task's
+// tensor is decoded and then encoded) stays on one lane, and a batch that names one still in use by an earlier batch waits
+// for that.
 //
 // Batches follow each other without waiting for the one before: a caller that submits 161 tasks one after the other
 // hands over the first few long before the last, and with every batch drained before the next was looked at the
@@ -36,7 +37,6 @@
 // multi-message decoders) and then re-encodes it.
 #include <hip/hip_runtime.h>
 
-#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -48,11 +48,11 @@
 #include <mutex>
 #include <string>
 #include <thread>
-#include <unordered_set>
 #include <vector>
 
 #include "hpx.h"
 #include "hpx_sched.h"
+#include "hpx_task_ranges.h"
 
 #define HPX_API extern "C" __attribute__((visibility("default")))
 
@@ -174,6 +174,7 @@ constexpr int kSlots = 4;
 // A batch under way: its tasks, staging memory, events, and the groups that are still to be published.
 struct Slot {
   std::vector<Task> tasks;
+  hpx::Ranges named;              // every tensor, residual, B and C of them
   Arena pinned_arena, device_arena;
   std::vector<hipEvent_t> events;
   size_t next_event = 0;
@@ -194,7 +195,6 @@ struct Worker {
   unsigned turn = 0;
   Slot slots[kSlots];
   std::deque<Slot*> in_flight, free_slots;
-  std::unordered_set<const void*> held;       // every tensor, residual, B and C of the batches in flight
   Slot* cur = nullptr;                        // the batch being queued
 };
 
@@ -286,9 +286,6 @@ void publish(Group& grp) {
   g.fcv.notify_all();
 }
 
-// What a task reads or writes; no two batches in flight name the same.
-std::array<const void*, 7> named(const hpx_task_t& t) { return {t.tensor, t.residual, t.B, t.C, t.M, t.P, t.Q}; }
-
 // Publishes, in the order they were queued, the groups whose events have passed; with `wait` at least everything of the
 // oldest batch.
 void publish_landed(Worker& w, bool wait) {
@@ -303,9 +300,8 @@ void publish_landed(Worker& w, bool wait) {
       publish(grp);
     }
     if (&s == w.cur) return;  // still being queued
-    for (const Task& t : s.tasks)
-      for (const void* p : named(t.t)) w.held.erase(p);
     s.tasks.clear();
+    s.named.clear();
     s.groups.clear();
     w.in_flight.pop_front();
     w.free_slots.push_back(&s);
@@ -562,26 +558,29 @@ void run_powersgd_batch(Worker& w, const Params&, const std::vector<Task>& batch
 
 // Queues a batch behind those under way.
 void run_batch(Worker& w, const Params& p, std::vector<Task>& batch) {
-  bool clash = false, twice = false;
-  std::vector<const void*> mine;
-  mine.reserve(batch.size() * 4);
+  bool one_lane = false;
+  hpx::Ranges named;
   for (const Task& t : batch) {
-    twice = twice || t.t.task_id == HPX_ROOT_DECOMP_COMP_TASK;
-    for (const void* x : named(t.t))
-      if (x) mine.push_back(x);
+    one_lane = one_lane || t.t.task_id == HPX_ROOT_DECOMP_COMP_TASK;
+    named.add(t.t);
   }
-  for (const void* x : mine) clash = clash || (!w.held.empty() && w.held.count(x));
-  while (!w.in_flight.empty() && (clash || w.free_slots.empty())) publish_landed(w, true);
+  one_lane = named.close() || one_lane;
+  auto clash = [&] {
+    for (const Slot* s : w.in_flight)
+      if (s->named.meets(named)) return true;
+    return false;
+  };
+  while (!w.in_flight.empty() && (w.free_slots.empty() || clash())) publish_landed(w, true);
   Slot& s = *w.free_slots.front();
   w.free_slots.pop_front();
   s.tasks.swap(batch);   // (the slot's empty list goes back: lists keep their room)
   s.next_event = 0;
   s.next_pub = 0;
   for (Task& t : s.tasks) t.t.name = t.name.c_str();
-  for (const void* x : mine) twice = !w.held.insert(x).second || twice;
+  s.named.swap(named);
   w.cur = &s;
   w.in_flight.push_back(&s);
-  if (p.alg == kPowersgd) run_powersgd_batch(w, p, s.tasks); else run_codec_batch(w, p, s.tasks, twice);
+  if (p.alg == kPowersgd) run_powersgd_batch(w, p, s.tasks); else run_codec_batch(w, p, s.tasks, one_lane);
   // A task that failed its checks was skipped (the failure is counted and kept for hpx_sched_error); its
   // name is published all the same, once the batch has drained, so that a caller polling for it does not
   // wait for ever: the reference publishes every task of a batch (hp_cuda.cpp:626-636).
