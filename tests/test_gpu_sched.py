@@ -438,3 +438,40 @@ def test_tasks_on_views_that_overlap(hp, oracle_cpu):
     assert_bits_equal(host(grad), total, "aggregated gradient"); assert_bits_equal(host(gres), rr, "its residual")
     assert_bits_equal(Cg.numpy(), np.concatenate([msg, slots[mb:]]), "gathered buffer afterwards")
     assert hp.error_count() == 0, hp.last_error()
+
+
+@pytest.mark.parametrize("pinned", [0, 1])
+@pytest.mark.parametrize("shared", ["C", "B"])
+def test_terngrad_received_message_before_an_encoded_one(hp, oracle_cpu, shared, pinned):
+    # A DECOMP task and a later COMP task that share their host buffer, or their device buffer: whether they land in one
+    # batch (behind a task whose pageable message keeps the worker busy) or in two, what was received is decoded and
+    # what was encoded is left in C.
+    rng = np.random.default_rng(23)
+    b, seed, big, n = 2, 3, 40_000_000, 70_001
+    assert hp.init("terngrad", {"enable_random": 1, "bitwidth": b, "seed": seed}, 0, 0, 2)
+    mb = oracle_cpu.terngrad_packed_size(n, b)
+    dev_bytes = lambda k: torch.zeros(k, dtype=torch.uint8, device="cuda")
+    rc, busy = oracle_cpu.terngrad_encode(np.full(big, 0.5, np.float32), b, 0, seed)
+    busy_C = torch.from_numpy(busy)
+    busy_t, busy_B = torch.zeros(big, device="cuda"), dev_bytes(busy.size)
+    pairs = []
+    for k in range(6):
+        x = rng.normal(0, 1e-2, n).astype(np.float32)
+        rc, received = oracle_cpu.terngrad_encode(rng.normal(0, 1e-2, n).astype(np.float32), b, 1, 50 + k)
+        C = _host_buf(mb, pinned); C.numpy()[:] = received
+        B = dev_bytes(mb)
+        pairs.append((x, received, torch.zeros(n, device="cuda"), dev(x), B, C, B if shared == "B" else dev_bytes(mb),
+                      C if shared == "C" else _host_buf(mb, pinned)))
+    torch.cuda.synchronize()
+    assert hp.submit_task("busy", busy_t, busy_B, busy_C, 0, 20)
+    for k, (x, received, out, dx, B, C, B2, C2) in enumerate(pairs):
+        assert hp.submit_task(f"d{k}", out, B, C, 0, 20)
+        assert hp.submit_task(f"c{k}", dx, B2, C2, 0, 10)
+    _collect(hp, 20, ["busy"] + [f"d{k}" for k in range(6)])
+    _collect(hp, 10, [f"c{k}" for k in range(6)])
+    for k, (x, received, out, dx, B, C, B2, C2) in enumerate(pairs):
+        rc, want = oracle_cpu.terngrad_decode(received, n)
+        assert_bits_equal(host(out), want, f"d{k}: the message received")
+        rc, ref = oracle_cpu.terngrad_encode(x, b, 1, seed)
+        assert_bits_equal(C2.numpy(), ref, f"c{k}: the message encoded")
+    assert hp.error_count() == 0, hp.last_error()

@@ -362,6 +362,22 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
   };
   std::vector<DecodeRun> dec_runs;
   std::vector<const Task*> root_ok;
+  // TernGrad encodes before it decodes.  A task that shares its C with a COMP task of the batch (one lane: they share
+  // memory) decodes what was received and not what the batch sends: the messages in are copied before the first encoded one
+  // goes out, from pinned memory as from pageable.  Not into a B that a COMP task encodes into: there the message
+  // follows the encode, as the decode does.
+  const bool in_first = one_lane && p.alg == kTerngrad && !comp.empty();
+  CopyList first;
+  hpx::Ranges encoded;
+  if (in_first)
+    for (const Task* t : comp) encoded.add(t->t.B, t->t.B_bytes);
+  encoded.close();
+  auto list_for = [&](CopyList& later, const uint8_t* to, int64_t bytes) -> CopyList& {
+    if (!in_first) return later;
+    hpx::Ranges r;
+    r.add(to, bytes);
+    return encoded.meets(r) ? later : first;
+  };
   {
     DecodeRun run;
     int64_t pipe_bytes = next_run_bytes(0);
@@ -374,7 +390,7 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
     for (const Task* t : decomp) {
       const int64_t bytes = message_bytes(p, t->t);
       if (bytes > t->t.C_bytes || bytes > t->t.B_bytes) { fail("scheduler: decode task '%s': message of %lld bytes does not fit B (%lld) / C (%lld)", t->name.c_str(), (long long)bytes, (long long)t->t.B_bytes, (long long)t->t.C_bytes); continue; }
-      copy_in(w, run.copies, t->t.B, t->t.C, bytes);  // t.B->copy_(t.C->slice(0,0,compressed_size,1), true)
+      copy_in(w, list_for(run.copies, t->t.B, bytes), t->t.B, t->t.C, bytes);  // t.B->copy_(t.C->slice(0,0,compressed_size,1), true)
       run.out.push_back(t->t.tensor); run.out_size.push_back(int32_t(t->t.tensor_numel));
       run.in.push_back(t->t.B); run.in_size.push_back(int32_t(bytes)); run.add.push_back(t->t.is_root);
       run.decomp.push_back(t);
@@ -386,7 +402,7 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
       const int64_t slots = int64_t(p.size) * bytes;
       if (slots > t->t.C_bytes) { fail("scheduler: root task '%s': C holds %lld bytes, %d slots of %lld needed", t->name.c_str(), (long long)t->t.C_bytes, p.size, (long long)bytes); continue; }
       uint8_t* tmp = w.cur->device_arena.take(size_t(slots));  // temp_cuda_tensors_for_c, hp_cuda.cpp:149-158
-      copy_in(w, run.copies, tmp, t->t.C, slots);
+      copy_in(w, list_for(run.copies, tmp, slots), tmp, t->t.C, slots);
       for (int i = 0; i < p.size; i++) {
         if (i == p.rank) continue;
         run.out.push_back(t->t.tensor); run.out_size.push_back(int32_t(t->t.tensor_numel));
@@ -399,6 +415,7 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
     close_run();
   }
   root = root_ok;
+  first.issue(w.lane[0]);
 
   // ---- compute ----
   auto encode = [&](const std::vector<const Task*>& ts, bool alone, hipStream_t st, const char* what) {
