@@ -114,3 +114,29 @@ def test_chain_of_columns(psgd, n, r, delta):
     assert np.abs(got.T @ got - np.eye(r)).max() < 2 * r * 2.0 ** -24
     assert np.linalg.norm(P - got @ (got.T @ P.astype(np.float64))) / np.linalg.norm(P) < 1e-6
     assert ps.rel_fro(host(dQ), M.astype(np.float64).T @ got) < 1e-5
+
+
+def test_a_matrix_alone_and_among_others(psgd):
+    # The order in which the entries of P and Q are summed is the matrix's own: the same bits in a call of one and in a
+    # call of many, on either side of every width and height at which the way of summing changes.
+    shapes = [(n, m, r) for n, r in ((64, 2), (127, 4), (129, 4), (515, 20), (2100, 4)) for m in (80, 300, 767, 900, 1537)]
+    shapes += [(4096, 2048, 4), (1024, 4096, 4)]
+    rng = np.random.default_rng(0)
+    G = [dev(rng.normal(0, 1e-2, n * m).astype(np.float32)) for n, m, r in shapes]
+    R = [dev(rng.normal(0, 1e-3, n * m).astype(np.float32)) for n, m, r in shapes]
+    Q0 = [dev(rng.normal(0, 1, (m, r)).astype(np.float32)) for n, m, r in shapes]
+    results = []
+    for groups in ([[i] for i in range(len(shapes))], [list(range(len(shapes)))]):
+        Q = [q.clone() for q in Q0]
+        M = [torch.zeros(n, m, device="cuda") for n, m, r in shapes]
+        P = [torch.zeros(n, r, device="cuda") for n, m, r in shapes]
+        for idx in groups:
+            of = lambda ts: [ts[i] for i in idx]
+            psgd.encode1(of(G), of(R), of(Q), of(M), of(P))
+        first = [host(p).copy() for p in P]
+        for idx in groups:
+            psgd.encode2([P[i] for i in idx], [M[i] for i in idx], [Q[i] for i in idx])
+        results.append([(a, host(b), host(c)) for a, b, c in zip(first, P, Q)])
+    for s, alone, among in zip(shapes, *results):
+        for a, b, what in zip(alone, among, ("P", "P orthonormal", "Q")):
+            assert_bits_equal(a, b, f"{s} {what}")

@@ -41,8 +41,6 @@ constexpr int kSegSmall = 16, kSegMiddle = 64, kSegLarge = 160;
 constexpr int kMaxCG = 4;                 // column groups of 4 -> rank <= 16
 // Decode is three write streams against one read stream; with 8 rows per wave instead of 32 the
 // stores of a workgroup stay close together in time and address and the pass runs 10 % faster.
-constexpr int kQRowsMin = 32, kQRowsMax = 512;  // rows folded into one partial of Q (of a strip 256 columns wide)
-constexpr int64_t kQTiles = 1024;
 constexpr int64_t kDecTiles = 256;
 constexpr int kDecRowsPerBlock = 32;      // rows of a decode tile 256 columns wide (narrower tiles are as much taller)
 
@@ -71,6 +69,7 @@ struct Seg {
   int32_t ld;          // row stride of P and Q (the full rank; r is the width of the block of columns at hand)
   int32_t mode;        // kFromM | kOntoM | kKeepGrad, for the passes of a rank above 16
   int32_t split;       // encode1: waves that share four rows.  encode2, decode: strip_lanes
+  int32_t rows;        // encode2: rows folded into one partial of Q (of a strip 256 columns wide)
 };
 constexpr int32_t kFromM = 1;    // encode1: M has been stored by an earlier pass: read it instead of grad + residual
 constexpr int32_t kOntoM = 2;    // decode: add this block's P Q^T to what M holds instead of starting from zero
@@ -78,7 +77,7 @@ constexpr int32_t kKeepGrad = 4; // decode: more blocks follow: write M only, le
 template <int CAP>
 struct Args {
   int32_t nseg;
-  int32_t rows;        // encode2: rows folded into one partial of Q, decode: rows of a tile (of a strip 256 columns wide)
+  int32_t rows;        // decode: rows of a tile (of a strip 256 columns wide)
   int32_t tile_start[CAP + 1];
   Seg seg[CAP];
   float* partials;
@@ -162,9 +161,11 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
             const int col = c * 4 + i;  // B operand: lane 4b+j holds Q[k][j]
             q[u][t][c] = col < r ? Q[int64_t(k0 + 64 * u + 4 * b + t) * ld + col] : 0.f;
           }
-      f32x4 sum[CG];  // of this chunk, added to the rest afterwards: shorter chains of fp32 sums
+      // Of each half of this chunk, added to the rest afterwards: shorter chains of fp32 sums.  (P's distance from the exact
+      // product 1.00e-7 of its norm for 4096 x 4096, 9.1e-8 for 200 x 600; in one chain 1.09e-7 and 1.11e-7; time alike.)
+      f32x4 sum[2][CG];
 #pragma unroll
-      for (int c = 0; c < CG; c++) sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < CG; c++) sum[0][c] = sum[1][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
         const int64_t f = row * m + k0 + 64 * u + 4 * b;
@@ -174,10 +175,10 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
-          for (int c = 0; c < CG; c++) sum[c] = mfma4(v[t], q[u][t][c], sum[c]);
+          for (int c = 0; c < CG; c++) sum[u & 1][c] = mfma4(v[t], q[u][t][c], sum[u & 1][c]);
       }
 #pragma unroll
-      for (int c = 0; c < CG; c++) acc[c] += sum[c];
+      for (int c = 0; c < CG; c++) acc[c] += sum[0][c] + sum[1][c];
     }
   };
   if (rows_full) {
@@ -213,6 +214,9 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
       for (int u = 0; u < kSteps; u++) {
         const int64_t kk = int64_t(k0) + u * split * 64 + 4 * b, f0 = row * m + kk;
         float v[4];
+        f32x4 sum[CG];
+#pragma unroll
+        for (int c = 0; c < CG; c++) sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (whole[u]) {
           const float4 m4 = make_float4(g4[u].x + r4[u].x, g4[u].y + r4[u].y, g4[u].z + r4[u].z, g4[u].w + r4[u].w);
           if (!from_m) st4(M + f0, m4);
@@ -236,7 +240,9 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
-          for (int c = 0; c < CG; c++) acc[c] = mfma4(v[t], q[u][t][c], acc[c]);
+          for (int c = 0; c < CG; c++) sum[c] = mfma4(v[t], q[u][t][c], sum[c]);
+#pragma unroll
+        for (int c = 0; c < CG; c++) acc[c] += sum[c];
       }
     }
   };
@@ -497,7 +503,7 @@ __global__ __launch_bounds__(kOrthThreads) void psgd_orth_kernel(const Args<CAP>
 
 // ---- encode2, step 2: Q = M^T P ------------------------------------------------
 // A workgroup takes a strip of columns (256, or 128 or 64 with two or four rows side by side in a wave: strip_lanes)
-// and a.rows rows of it (two or four times that), the rows going round its waves.  Per row a
+// and sg.rows rows of it (two or four times that), the rows going round its waves.  Per row a
 // lane loads its 4 columns of M with one 128-bit load; register t of that load
 // is the A operand of MFMA t, whose block b / row-of-block i' is column
 // k0 + 16b + 4i' + t; the B operand is P[row][j] in every block.  The waves (and the rows side by side) meet
@@ -519,7 +525,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
   const int k0 = strip * width;
   const int kk = k0 + 4 * (lane & (lanes - 1));
   const int step = kWaves * side;  // rows of the workgroup per round
-  const int64_t last = int64_t(rblk + 1) * a.rows * side;
+  const int64_t last = int64_t(rblk + 1) * sg.rows * side;
   const int64_t rend = last < n ? last : n;
 
   f32x4 acc[CG][4];
@@ -530,10 +536,11 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
 
   const int j = lane & 3;
   const int mine = lane / lanes;  // which of the rows side by side
-  int64_t row0 = int64_t(rblk) * a.rows * side + wave * side;  // the first of the wave's rows in a round
-  // Main loop: 8 rounds at a time, every load issued before the first use, summed on their own and added to what there is
-  // (one chain of fp32 sums down all rows of a partial of 512 left Q half as far again from the exact product).  Only the lane that holds the row's end
-  // and those past it take the element-wise way.
+  int64_t row0 = int64_t(rblk) * sg.rows * side + wave * side;  // the first of the wave's rows in a round
+  // Main loop: 8 rounds at a time, every load issued before the first use, summed on their own in two chains and added to
+  // what there is (one chain of fp32 sums down all rows of a partial of 512 left Q half as far again from the exact product;
+  // two chains of four instead of one of eight 8.24e-8 of its norm for 4096 x 4096 and 7.5e-8 for 200 x 600, from
+  // 8.46e-8 and 7.7e-8).  Only the lane that holds the row's end and those past it take the element-wise way.
   constexpr int kRows = 8;
   for (; row0 + (kRows - 1) * step + side <= rend; row0 += kRows * step) {
     float4 m4[kRows];
@@ -553,23 +560,20 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
     for (int u = 0; u < kRows; u++)
 #pragma unroll
       for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[(row0 + u * step + mine) * ld + c * 4 + j] : 0.f;
-    f32x4 sum[CG][4];
 #pragma unroll
-    for (int c = 0; c < CG; c++)
+    for (int c = 0; c < CG; c++) {
+      f32x4 sum[2][4];
 #pragma unroll
-      for (int t = 0; t < 4; t++) sum[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < 4; t++) sum[0][t] = sum[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < kRows; u++) {
-      const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
+      for (int u = 0; u < kRows; u++) {
+        const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
 #pragma unroll
-      for (int c = 0; c < CG; c++)
+        for (int t = 0; t < 4; t++) sum[u & 1][t] = mfma4(v[t], p[u][c], sum[u & 1][t]);
+      }
 #pragma unroll
-        for (int t = 0; t < 4; t++) sum[c][t] = mfma4(v[t], p[u][c], sum[c][t]);
+      for (int t = 0; t < 4; t++) acc[c][t] += sum[0][t] + sum[1][t];
     }
-#pragma unroll
-    for (int c = 0; c < CG; c++)
-#pragma unroll
-      for (int t = 0; t < 4; t++) acc[c][t] += sum[c][t];
   }
   for (; row0 < rend; row0 += step) {
     const int64_t row = row0 + mine;
@@ -602,7 +606,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
       for (int ii = 0; ii < 4; ii++) s_q[wave][c][16 * (lane >> 2) + 4 * ii + t][j] = acc[c][t][ii];
   __syncthreads();
   // the one partial of a matrix of few rows is Q itself
-  const bool whole = int64_t(a.rows) * side >= n;
+  const bool whole = int64_t(sg.rows) * side >= n;
   float* part = whole ? sg.Qout : a.partials + (int64_t(sg.part_off) * 4) + int64_t(rblk) * m * r;
   const int stride = whole ? ld : r;
   for (int e = threadIdx.x; e < CG * width * 4; e += kThreads) {
@@ -626,7 +630,7 @@ __global__ __launch_bounds__(kThreads) void psgd_qreduce_kernel(const Args<CAP> 
   const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
   const Seg& sg = a.seg[s];
   const int64_t mr = int64_t(sg.m) * sg.r;
-  const int64_t per = int64_t(a.rows) * (kWave / sg.split);
+  const int64_t per = int64_t(sg.rows) * (kWave / sg.split);
   const int nparts = int((sg.n + per - 1) / per);
   const float* part = a.partials + int64_t(sg.part_off) * 4;
   const int64_t e = int64_t(tile - a.tile_start[s]) * kThreads + threadIdx.x;
@@ -766,12 +770,12 @@ int check_dims(const char* who, const Batch& b, int* max_rank) {
 // the column groups of four it needs.
 inline int block_cols(int r, int c0) { return r <= c0 ? 0 : (r - c0 < kPassCols ? r - c0 : kPassCols); }
 
-// encode1: waves that share four rows of m columns.  A wave keeps 256 columns in flight, so a row of fewer than
+// encode1: waves that share four rows of an n x m matrix.  A wave keeps 256 columns in flight, so a row of fewer than
 // 768 is one wave's work and one of fewer than 1536 two waves' (ResNet-50's matrices: 61 us with this rule; all
-// rows to four waves 64, to one or two 73); calls too small to
-// fill the chip spread their rows over as many workgroups as they can.
-inline int split_rows(int m, bool fills) { return !fills || m >= 1536 ? kWaves : m >= 768 ? kWaves / 2 : 1; }
-constexpr int64_t kFillGroups = 2048;  // groups of four rows that fill the chip: eight workgroups on each of 256 CUs
+// rows to four waves 64, to one or two 73).  A matrix of fewer than 128 rows spreads them over as many workgroups as it can
+// (64 x 147, all three phases: 21.9 us, 22.9 by the other rule).  The sums that make up an entry of P are cut at the waves,
+// so the choice rests on the matrix alone and not on what else is in the call: a matrix has one P.
+inline int split_rows(int n, int m) { return n < 128 || m >= 1536 ? kWaves : m >= 768 ? kWaves / 2 : 1; }
 
 #define PSGD_LAUNCH_CG_LDS(KERNEL, cg, grid, lds, st, args)                                                             \
   switch (cg) {                                                                                                         \
@@ -786,9 +790,6 @@ template <int CAP>
 int encode1_launches(int count, int max_rank, const float* const* grads, const int64_t* numels, const float* const* residuals,
                      const float* const* Qs, float* const* Ms, float* const* Ps, const int32_t* ns, const int32_t* ms,
                      const int32_t* rs, hipStream_t st) {
-  int64_t row_groups = 0;
-  for (int i = 0; i < count; i++) row_groups += cdiv(ns[i], 4);
-  const bool fills = row_groups >= kFillGroups;
   Args<CAP> a;
   a.partials = nullptr;
   for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
@@ -800,11 +801,11 @@ int encode1_launches(int count, int max_rank, const float* const* grads, const i
       while (i < count && a.nseg < CAP) {
         const int rb = block_cols(rs[i], c0);
         if (rb == 0) { i++; continue; }
-        const int split = split_rows(ms[i], fills);
+        const int split = split_rows(ns[i], ms[i]);
         const int32_t t = cdiv(ns[i], 4 * (kWaves / split));
         if (int64_t(a.tile_start[a.nseg]) + t > INT32_MAX) break;
         a.seg[a.nseg] = Seg{grads[i], residuals[i], Qs[i] + c0, Ms[i], Ps[i] + c0, nullptr, numels[i], ns[i], ms[i], rb, 0,
-                            rs[i], c0 ? kFromM : 0, split};
+                            rs[i], c0 ? kFromM : 0, split, 0};
         if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
         a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + t;
         a.nseg++;
@@ -833,11 +834,26 @@ int orth_launch(const Args<CAP>& a, size_t lds, hipStream_t st) {
 // Partials of a matrix: of `rows` rows each, as many times more as strips side by side in a wave.
 inline int32_t q_parts(int n, int m, int rows) { return cdiv(n, int64_t(rows) * (kWave / strip_lanes(m))); }
 
+// Rows per partial: as many as leave the matrix kQTiles workgroups, since every partial is written and read back; 64 at
+// least, or 32 where 64 would leave fewer than kQTilesSmall.  Like split_rows by the matrix alone: Q is the sum of the
+// partials, and what a matrix's Q is must not depend on what else is in the call.  A pass over all three phases in us, with the rows
+// chosen so that the call had 1024 workgroups / with this rule / with at most 256 rows: layer set of 36 matrices 1566 /
+// 1574 / 1588, 4096 x 4096 alone 116 / 127 / 119, 4 of 2000 x 1000 74 / 70 / 70, ResNet-50's 54 157.6 / 157.5 / 157.5
+// (with 32 rows for all of those 160.5); with kQTiles 64 and 32 4096 x 1024 alone is at 59 and 68 instead of 56.
+constexpr int kQRowsMin = 32, kQRowsMax = 512;
+constexpr int64_t kQTiles = 128, kQTilesSmall = 32;
+inline int q_rows(int n, int m) {
+  auto tiles = [=](int rows) { return int64_t(cdiv(m, 4 * strip_lanes(m))) * q_parts(n, m, rows); };
+  int rows = kQRowsMax;
+  while (rows > 2 * kQRowsMin && tiles(rows) < kQTiles) rows /= 2;
+  return rows == 2 * kQRowsMin && tiles(rows) < kQTilesSmall ? kQRowsMin : rows;
+}
+
 template <int CAP>
-int encode2_launches(int count, int max_rank, int rows, float* partials, float* const* Ps, const float* const* Ms, float* const* Qs,
+int encode2_launches(int count, int max_rank, float* partials, float* const* Ps, const float* const* Ms, float* const* Qs,
                      const int32_t* ns, const int32_t* ms, const int32_t* rs, hipStream_t st) {
   Args<CAP> a;
-  a.rows = rows;
+  a.rows = 0;
   a.partials = partials;
   // step 1: orthonormalise every P over all of its columns
   for (int i = 0; i < count;) {
@@ -845,7 +861,7 @@ int encode2_launches(int count, int max_rank, int rows, float* partials, float* 
     int64_t max_nr = 0;
     bool wide = false;
     for (; i < count && a.nseg < CAP; i++) {
-      a.seg[a.nseg++] = Seg{nullptr, nullptr, nullptr, nullptr, Ps[i], nullptr, 0, ns[i], ms[i], rs[i], 0, rs[i], 0, 0};
+      a.seg[a.nseg++] = Seg{nullptr, nullptr, nullptr, nullptr, Ps[i], nullptr, 0, ns[i], ms[i], rs[i], 0, rs[i], 0, 0, 0};
       if (int64_t(ns[i]) * rs[i] > max_nr) max_nr = int64_t(ns[i]) * rs[i];
       wide = wide || (rs[i] > 4 && rs[i] <= kGramCols);
     }
@@ -869,6 +885,7 @@ int encode2_launches(int count, int max_rank, int rows, float* partials, float* 
         const int rb = block_cols(rs[i], c0);
         if (rb == 0) { i++; continue; }
         const int lanes = strip_lanes(ms[i]);
+        const int rows = q_rows(ns[i], ms[i]);
         const int32_t parts = q_parts(ns[i], ms[i], rows);
         const int64_t t = int64_t(cdiv(ms[i], 4 * lanes)) * parts;
         const int32_t tr = parts > 1 ? cdiv(int64_t(ms[i]) * rb, kThreads) : 0;
@@ -877,7 +894,7 @@ int encode2_launches(int count, int max_rank, int rows, float* partials, float* 
           break;
         }
         a.seg[a.nseg] = Seg{nullptr, nullptr, nullptr, const_cast<float*>(Ms[i]), Ps[i] + c0, Qs[i] + c0, 0, ns[i], ms[i], rb,
-                            static_cast<int32_t>(poff), rs[i], 0, lanes};
+                            static_cast<int32_t>(poff), rs[i], 0, lanes, rows};
         poff += (int64_t(parts) * ms[i] * rb + 3) / 4;
         if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
         a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + int32_t(t);
@@ -927,7 +944,7 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
         }
         const int32_t mode = (c0 ? kOntoM : 0) | (c0 + kPassCols < rs[i] ? kKeepGrad : 0);
         a.seg[a.nseg] = Seg{grads[i], residuals[i], Qs[i] + c0, Ms[i], const_cast<float*>(Ps[i]) + c0, nullptr, numels[i], ns[i],
-                            ms[i], rb, 0, rs[i], mode, lanes};
+                            ms[i], rb, 0, rs[i], mode, lanes, 0};
         if ((rb + 3) / 4 > cg) cg = (rb + 3) / 4;
         a.tile_start[a.nseg + 1] = a.tile_start[a.nseg] + int32_t(t);
         a.nseg++;
@@ -975,17 +992,8 @@ HPX_API int hpx_powersgd_encode2(int count, float* const* Ps, const float* const
   int rc = check_dims("hpx_powersgd_encode2", Batch{count, ns, ms, rs}, &max_rank);
   if (rc != HPX_OK) return rc;
   for (int i = 0; i < count; i++) HPX_ARG(Ps[i] && Ms[i] && Qs[i], "hpx_powersgd_encode2: matrix %d has a null pointer", i);
-  // Rows per partial: as many as leave four workgroups for each CU, since every partial is written and read back
-  // (36 matrices of the layer set: 5.0 us for adding them up instead of 12.7 with 128 rows; ResNet-50's 54 a pass 166 us,
-  // 170 with the line at eight workgroups per CU); few rows where the call is small, so that it spreads out.
-  int rows = kQRowsMax;
-  for (; rows > kQRowsMin; rows /= 2) {
-    int64_t tiles = 0;
-    for (int i = 0; i < count; i++) tiles += int64_t(cdiv(ms[i], 4 * strip_lanes(ms[i]))) * q_parts(ns[i], ms[i], rows);
-    if (tiles >= kQTiles) break;
-  }
   int64_t part_quads = 0;  // partial storage in units of 4 floats (one pass at a time uses it)
-  for (int i = 0; i < count; i++) part_quads += (int64_t(q_parts(ns[i], ms[i], rows)) * ms[i] * block_cols(rs[i], 0) + 3) / 4;
+  for (int i = 0; i < count; i++) part_quads += (int64_t(q_parts(ns[i], ms[i], q_rows(ns[i], ms[i]))) * ms[i] * block_cols(rs[i], 0) + 3) / 4;
   HPX_ARG(part_quads <= INT32_MAX, "hpx_powersgd_encode2: batch too large for one call");
   hipStream_t st = static_cast<hipStream_t>(stream);
   hpx::Workspace* ws = hpx::workspace_record(st);
@@ -994,7 +1002,7 @@ HPX_API int hpx_powersgd_encode2(int count, float* const* Ps, const float* const
   rc = hpx::ensure_workspace(ws, size_t(part_quads) * 16);
   if (rc != HPX_OK) return rc;
   float* partials = reinterpret_cast<float*>(ws->dev);
-  return PSGD_BY_COUNT(encode2_launches, max_rank, rows, partials, Ps, Ms, Qs, ns, ms, rs, st);
+  return PSGD_BY_COUNT(encode2_launches, max_rank, partials, Ps, Ms, Qs, ns, ms, rs, st);
 }
 
 HPX_API int hpx_powersgd_decode(int count, const float* const* Ps, const float* const* Qs, float* const* Ms,
