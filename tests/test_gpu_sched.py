@@ -475,3 +475,22 @@ def test_terngrad_received_message_before_an_encoded_one(hp, oracle_cpu, shared,
         rc, ref = oracle_cpu.terngrad_encode(x, b, 1, seed)
         assert_bits_equal(C2.numpy(), ref, f"c{k}: the message encoded")
     assert hp.error_count() == 0, hp.last_error()
+
+
+def test_tensors_of_finished_tasks_are_given_back_at_the_next_submission(hp):
+    # A caller that submits task after task and asks for results only now and then does not pay for it in memory.
+    assert hp.init("tbq", {"threshold": 1e-3}, 0, 0, 2)
+    n = 8 << 20
+    for k in range(3):
+        before = torch.cuda.memory_allocated()
+        big = [torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda"), torch.zeros(n // 4, dtype=torch.uint8, device="cuda")]
+        small = [torch.zeros(8, device="cuda"), torch.zeros(8, device="cuda"), torch.zeros(2, dtype=torch.uint8, device="cuda")]
+        torch.cuda.synchronize()
+        assert hp.submit_task(f"big{k}", *big, _host_buf(n // 4, 1), 0, 10)
+        assert hp.wait(10, 20000)
+        del big
+        assert torch.cuda.memory_allocated() >= before + 8 * n            # the task's own until somebody looks
+        assert hp.submit_task(f"small{k}", *small, _host_buf(2, 1), 0, 10)
+        assert torch.cuda.memory_allocated() < before + n
+        _collect(hp, 10, [f"big{k}", f"small{k}"])
+    assert hp.error_count() == 0, hp.last_error()

@@ -20,7 +20,6 @@
 #include <torch/extension.h>
 
 #include <array>
-#include <atomic>
 #include <climits>
 #include <mutex>
 #include <string>
@@ -57,12 +56,8 @@ void release_done() {
   }
 }
 
-// Finished tasks are looked for once in so many submissions, and whenever results are asked for.
-constexpr unsigned kReleaseEvery = 64;
-
 bool submit(const char* name, hpx_task_t& t, Kept keep) {
-  static std::atomic<unsigned> submitted{0};
-  if (++submitted % kReleaseEvery == 0) release_done();
+  release_done();
   t.name = name;
   uint64_t serial = 0;
   if (hpx_sched_submit(&t, &serial) != 0) {

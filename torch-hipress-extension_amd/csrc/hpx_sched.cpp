@@ -104,6 +104,7 @@ struct Sched {
   std::condition_variable fcv;
   std::deque<std::string> finished[3];  // COMP, DECOMP, ROOT (FinishedQueues, hp_cuda.h:128-132)
   std::deque<uint64_t> done;
+  std::atomic<bool> any_done{false};    // for a look without the lock
 
   std::mutex emu;
   std::string last_error;
@@ -282,6 +283,7 @@ void publish(Group& grp) {
       if (grp.queue >= 0) g.finished[grp.queue].push_back(t->name);
       g.done.push_back(t->serial);
     }
+    g.any_done.store(true, std::memory_order_relaxed);
   }
   g.fcv.notify_all();
 }
@@ -811,13 +813,14 @@ HPX_API int hpx_sched_wait(int task_id, int timeout_ms) {
 }
 
 HPX_API int64_t hpx_sched_take_done(uint64_t* serials, int64_t cap) {
-  if (!serials || cap <= 0) return 0;
+  if (!serials || cap <= 0 || !g.any_done.load(std::memory_order_relaxed)) return 0;
   std::lock_guard<std::mutex> l(g.fmu);
   int64_t n = 0;
   while (n < cap && !g.done.empty()) {
     serials[n++] = g.done.front();
     g.done.pop_front();
   }
+  g.any_done.store(!g.done.empty(), std::memory_order_relaxed);
   return n;
 }
 
