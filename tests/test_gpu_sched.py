@@ -494,3 +494,25 @@ def test_tensors_of_finished_tasks_are_given_back_at_the_next_submission(hp):
         assert torch.cuda.memory_allocated() < before + n
         _collect(hp, 10, [f"big{k}", f"small{k}"])
     assert hp.error_count() == 0, hp.last_error()
+
+
+def test_graddrop_batches_share_one_workspace(hp):
+    # Batches under way together: the second and later ones take no more device memory than the first alone did.
+    n, sr, dr_ = 60_000_000, 0.01, 0.999
+    fixed = 4 + int(2 * np.ceil(n * (1 - dr_))) * 4
+    items = [(f"w{k}", torch.randn(n, device="cuda") * 1e-3, torch.zeros(n, device="cuda"),
+              torch.zeros(fixed, dtype=torch.uint8, device="cuda"), _host_buf(fixed, 1), 0, 10) for k in range(3)]
+    torch.cuda.synchronize()
+    assert hp.init("graddrop", {"sample_rate": sr, "drop_ratio": dr_, "seed": 1}, 0, 0, 2)
+    free = torch.cuda.mem_get_info()[0]
+    assert hp.submit_task(*items[0])
+    _collect(hp, 10, ["w0"])
+    one = free - torch.cuda.mem_get_info()[0]
+    import time
+    for _ in range(10):
+        for it in items:
+            assert hp.submit_task(*it)
+            time.sleep(1e-4)                 # the encode takes some 200 us: the next task is a batch of its own, behind it
+        _collect(hp, 10, [it[0] for it in items])
+    assert one > 0 and free - torch.cuda.mem_get_info()[0] <= one + (2 << 20), one
+    assert hp.error_count() == 0, hp.last_error()

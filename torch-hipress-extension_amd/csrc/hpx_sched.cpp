@@ -320,7 +320,9 @@ hipEvent_t mark(Worker& w, hipStream_t st) {
 
 // ---- the three quantiser / sparsifier algorithms ---------------------------------
 void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch, bool one_lane) {
-  auto next_lane = [&]() { return one_lane ? w.lane[0] : w.lane[w.turn++ & 1u]; };
+  // GradDrop stays on one lane too: its encode's workspace grows with the tensors (20 MB for 60 M elements), and a second
+  // one would buy little, with messages a thousandth of the tensor.
+  auto next_lane = [&]() { return one_lane || p.alg == kGraddrop ? w.lane[0] : w.lane[w.turn++ & 1u]; };
   std::deque<Group>& sent = w.cur->groups;
   std::vector<const Task*> comp, decomp, root;
   for (const Task& t : batch) {
