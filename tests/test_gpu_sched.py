@@ -516,3 +516,19 @@ def test_graddrop_batches_share_one_workspace(hp):
         _collect(hp, 10, [it[0] for it in items])
     assert one > 0 and free - torch.cuda.mem_get_info()[0] <= one + (2 << 20), one
     assert hp.error_count() == 0, hp.last_error()
+
+
+def test_batches_one_after_the_other_share_their_staging_memory(hp):
+    # A root task's gathered messages are staged in device memory, here 40 MB.  Batches that do not overlap use one block.
+    n, size = 20_000_000, 8
+    assert hp.init("tbq", {"threshold": 1e-3}, 0, 0, size)
+    t, r, B = torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda"), torch.zeros(n // 4, dtype=torch.uint8, device="cuda")
+    Cc = _host_buf(size * n // 4, 1)
+    torch.cuda.synchronize()
+    used = []
+    for k in range(6):
+        assert hp.submit_task("root", t, r, B, Cc, 0, 30)
+        _collect(hp, 30, ["root"])
+        used.append(torch.cuda.mem_get_info()[0])
+    assert used[0] - used[-1] <= 2 << 20, used
+    assert hp.error_count() == 0, hp.last_error()

@@ -306,7 +306,7 @@ void publish_landed(Worker& w, bool wait) {
     s.named.clear();
     s.groups.clear();
     w.in_flight.pop_front();
-    w.free_slots.push_back(&s);
+    w.free_slots.push_front(&s);  // the next batch takes it again: only batches that overlap hold staging memory side by side
     wait = false;
   }
 }
