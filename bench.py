@@ -844,7 +844,7 @@ def x_scheduler(torch, np, capi, L, stream, gen, res):
             "errors": hp.error_count()}
 
     # 200 COMP tasks at once (the TBQ bucket, 110 M elements): the worker batches what is queued into
-    # multi-tensor encodes; 27.5 MB of messages go to pinned C buffers on the data stream
+    # multi-tensor encodes; 27.5 MB of messages go to pinned C buffers run by run, each on the stream of its encode
     if hp.init("tbq", {"threshold": 1e-2}, torch.cuda.current_device(), 0, 2):
         sizes = bucket_sizes(np)
         gs = [torch.randn(int(n_), device="cuda", generator=gen) * 5e-3 for n_ in sizes]

@@ -16,10 +16,14 @@
  * 4 + 8*ceil(N*(1-drop_ratio)) (hp_cuda.cpp:230), root tasks decoding every
  * gathered slot but their own rank's and then re-encoding.
  * What is different: one worker thread that sleeps on a condition variable
- * (the reference polls five queues every 500 us, one for TBQ); staging copies
- * run on a data stream ordered against the compute stream by events; a batch's
+ * while nothing is under way (the reference polls five queues every 500 us, one
+ * for TBQ) and otherwise asks for finished events, without a pause until some
+ * 2000 questions have found nothing, then every 20 us; up to four batches under
+ * way, each with its own staging memory; a batch's
  * transfers and codec calls are cut into runs (1 MB of messages, then 2, 4 ...
- * 16 MB; GradDrop: one run) so that one run's transfer overlaps the next run's
+ * 16 MB; GradDrop: one run), and a run's staging copy and codec call follow each
+ * other on one of two streams that runs take in turn (GradDrop and PowerSGD:
+ * one), so that one run's transfer overlaps the next run's
  * kernels, all messages of a run in ONE kernel launch that reads or writes the
  * pinned host buffers directly (through a pinned bounce buffer when the caller's
  * host tensor is pageable) instead of one copy call per message; a name is
@@ -27,6 +31,12 @@
  * the batch; HIP errors are counted and kept (hpx_sched_error) instead of ignored;
  * a task whose buffers are too small for its message is skipped and counted as
  * a failure (the reference overruns them), and its name is still published.
+ *
+ * Tasks may share memory.  What counts is the bytes of the buffers as declared
+ * in hpx_task_t, not where they start: views into one tensor, a slot of a
+ * gathered buffer.  Tasks of one batch that share any run on one stream in the
+ * order above, the messages received copied in before the first encoded one
+ * goes out; a batch that shares any with one under way waits for that.
  */
 #ifndef HPX_SCHED_H_
 #define HPX_SCHED_H_

@@ -50,7 +50,7 @@ def _phases(psgd, shapes, seed):
 
 @pytest.mark.parametrize("m", [1, 3, 4, 61, 64, 65, 127, 129, 191, 205, 257, 511, 767, 768, 1023, 1535, 1537, 2049])
 def test_widths_around_the_strips(psgd, m):
-    # n above and below what a strip's tile holds, alone (rows spread out) and beside enough rows to fill the chip
+    # n above and below what a strip's tile holds, and on either side of the height below which rows are spread out
     _phases(psgd, [(n, m, min(4, n, m)) for n in (4, 17, 33, 515)], m)
     _phases(psgd, [(n, m, min(2, m)) for n in (8201, 129)], m + 1)
 

@@ -1733,8 +1733,8 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // (as many as give every lane something to do), a lane after a run of the tile's mask words, of which the tile's coarse
 // word names the few that have a bit set; lanes in order, so one prefix over the workgroup's counts puts the indices
 // in ascending order in LDS.
-// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 6-9 us; ResNet-50's 161
-// tensors 58 -> 23 us.
+// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 6.5-16 us, 10.8 on average;
+// ResNet-50's 161 tensors 58 -> 23 us, 16-36.
 // Larger ones that still fit are only cut here, behind the expand launch.  All of it is queued before the host knows any
 // count.
 constexpr uint32_t kFinishKeep = 2560;

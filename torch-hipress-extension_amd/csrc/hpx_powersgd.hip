@@ -41,7 +41,7 @@ constexpr int kSegSmall = 16, kSegMiddle = 64, kSegLarge = 160;
 constexpr int kMaxCG = 4;                 // column groups of 4 -> rank <= 16
 // Decode is three write streams against one read stream; with 8 rows per wave instead of 32 the
 // stores of a workgroup stay close together in time and address and the pass runs 10 % faster.
-constexpr int64_t kDecTiles = 256;
+constexpr int64_t kDecTiles = 256;        // fewer than this many tiles are halved
 constexpr int kDecRowsPerBlock = 32;      // rows of a decode tile 256 columns wide (narrower tiles are as much taller)
 
 // encode2 and decode cut a matrix into strips of 4 * lanes columns; a wave lays kWave / lanes row groups of a strip
@@ -952,7 +952,9 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
       }
       if (a.nseg == 0) continue;
       // One read and three writes per element: held to two workgroups per CU (LDS the kernel never touches,
-      // hpx_common.h), the 36 matrices of the configuration decode in 755 us instead of 792 (three per CU: 776).
+      // hpx_common.h), the 36 matrices of the configuration decode in 755 us instead of 792 (three per CU: 776).  Between the
+      // other phases of a pass it has been 750 in one process and 813 in another, for the same kernel and matrices at
+      // other addresses.
       PSGD_LAUNCH_CG_LDS(psgd_decode_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds2, st, a);
       HPX_HIP(hipGetLastError());
     }
