@@ -140,3 +140,29 @@ def test_a_matrix_alone_and_among_others(psgd):
     for s, alone, among in zip(shapes, *results):
         for a, b, what in zip(alone, among, ("P", "P orthonormal", "Q")):
             assert_bits_equal(a, b, f"{s} {what}")
+
+
+@pytest.mark.parametrize("big", [(7679, 4096), (7680, 4096), (7683, 4100), (8001, 4160)])
+def test_decode_of_calls_that_store_m_streaming(psgd, big):
+    # 120 MiB of M and more, whole tiles and ragged ones, a gradient that ends within M, ranks of one and two passes: the bits
+    # of every matrix decoded by a call of its own, and of the big one in row blocks that are far from the line.
+    g = torch.Generator(device="cuda").manual_seed(big[0])
+    shapes = [big + (4, 0), (65, 4096, 4, 3000), (33, 512, 18, 0), (130, 147, 2, 1)]
+    rand = lambda *s: torch.empty(*s, device="cuda").normal_(generator=g)
+    P = [rand(n, r) for n, m, r, cut in shapes]
+    Q = [rand(m, r) for n, m, r, cut in shapes]
+    G0 = [rand(n * m - cut) for n, m, r, cut in shapes]
+    empty = lambda: ([torch.full((n, m), 7.0, device="cuda") for n, m, r, cut in shapes], [torch.full_like(x, 7.0) for x in G0], [x.clone() for x in G0])
+    M, R, G = empty()
+    psgd.decode(P, Q, M, R, G)
+    wM, wR, wG = empty()
+    n, m = big
+    step = 3840  # rows of the big matrix at a time: whole tiles of 32 rows
+    for a in range(0, n, step):
+        b = min(n, a + step)
+        psgd.decode([P[0][a:b]], [Q[0]], [wM[0][a:b]], [wR[0][a * m:b * m]], [wG[0][a * m:b * m]])
+    for i in range(1, len(shapes)):
+        psgd.decode([P[i]], [Q[i]], [wM[i]], [wR[i]], [wG[i]])
+    for i, s in enumerate(shapes):
+        for got, want, what in ((M, wM, "M"), (R, wR, "residual"), (G, wG, "gradient")):
+            assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), (s, what)

@@ -78,12 +78,20 @@ template <int CAP>
 struct Args {
   int32_t nseg;
   int32_t rows;        // decode: rows of a tile (of a strip 256 columns wide)
+  int32_t stream_m;    // decode: M is stored streaming too (kDecStreamedBytes)
   int32_t tile_start[CAP + 1];
   Seg seg[CAP];
   float* partials;
 };
 static_assert(sizeof(Args<kSegLarge>) <= 18000, "kernel-argument budget");
 
+// Decode: bytes of M in a call from which M is stored streaming as the residual and the gradient are.  One array of less
+// than half the 256 MB Infinity Cache stays there when the launch ends and reaches memory beside the launches that follow,
+// which read; a larger one is written out within the launch, line by line between the two streams.  us of a decode with M
+// plain / streaming (a call of one matrix of 4096 columns): 84 MB 56.6 / 61.1, 109 MB 72.4 / 77.7, 126 MB 88.2 / 87.7, 134 MB
+// 97.1 / 91.9, 185 MB 130.9 / 122.9; ResNet-50's 94 MB 64 / 76, the layer set's 1208 MB 813 / 765.  Two arrays plain, or all
+// three, are slower than one at every size.
+constexpr int64_t kDecStreamedBytes = int64_t(120) << 20;
 template <bool STREAM>
 __device__ __forceinline__ float4 ld4_as(const float* p) { return STREAM ? ld4_stream(p) : ld4(p); }
 template <bool STREAM>
@@ -685,9 +693,9 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
 #pragma unroll
     for (int col = 0; col < CG * 4; col++) q[t][col] = (kk + t < m && col < r) ? Q[int64_t(kk + t) * ld + col] : 0.f;
 
-  // (two loops: of one loop with a choice at each store the compiler makes plain stores)
-  auto rows = [&](auto stream) {
-    constexpr bool STREAM = decltype(stream)::value;
+  // (a loop for each choice: of one loop with a choice at each store the compiler makes plain stores)
+  auto rows = [&](auto stream, auto stream_m) {
+    constexpr bool STREAM = decltype(stream)::value, STREAM_M = decltype(stream_m)::value;
     for (int64_t at = rbeg; at < rend; at += 4 * side) {
       const int64_t row0 = at + 4 * (lane / lanes);
       const bool full4 = kk + 4 <= m && row0 + 4 <= rend && (row0 + 3) * m + kk + 4 <= N;
@@ -713,16 +721,32 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
         for (int t = 0; t < 4; t++) acc[t] = mfma4(p, q[t][col], acc[t]);
       }
       if (full4) {
+        float4 m4[4], r4[4];
 #pragma unroll
         for (int ii = 0; ii < 4; ii++) {
-          const int64_t f = (row0 + ii) * m + kk;
-          const float4 m4 = make_float4(acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]);
-          const float4 r4 = make_float4(g4[ii].x - m4.x, g4[ii].y - m4.y, g4[ii].z - m4.z, g4[ii].w - m4.w);
+          m4[ii] = make_float4(acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]);
+          r4[ii] = make_float4(g4[ii].x - m4[ii].x, g4[ii].y - m4[ii].y, g4[ii].z - m4[ii].z, g4[ii].w - m4[ii].w);
+        }
+        if constexpr (STREAM_M) {
+          // array after array (the layer set: 763 us; row after row 794)
           if (!keep_grad) {
-            st4_as<STREAM>(R + f, r4);
-            st4_as<STREAM>(G + f, m4);  // in place over the line just read
+#pragma unroll
+            for (int ii = 0; ii < 4; ii++) st4_stream(R + (row0 + ii) * m + kk, r4[ii]);
+#pragma unroll
+            for (int ii = 0; ii < 4; ii++) st4_stream(G + (row0 + ii) * m + kk, m4[ii]);  // in place over the line just read
           }
-          st4(M + f, m4);  // plain: streaming this third store was measurably slower
+#pragma unroll
+          for (int ii = 0; ii < 4; ii++) st4_stream(M + (row0 + ii) * m + kk, m4[ii]);
+        } else {
+#pragma unroll
+          for (int ii = 0; ii < 4; ii++) {
+            const int64_t f = (row0 + ii) * m + kk;
+            if (!keep_grad) {
+              st4_as<STREAM>(R + f, r4[ii]);
+              st4_as<STREAM>(G + f, m4[ii]);
+            }
+            st4(M + f, m4[ii]);
+          }
         }
         continue;
       }
@@ -745,7 +769,9 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
       }
     }
   };
-  if (rows_on_lines(m, G, R, M)) rows(std::true_type{}); else rows(std::false_type{});
+  if (!rows_on_lines(m, G, R, M)) rows(std::false_type{}, std::false_type{});
+  else if (a.stream_m) rows(std::true_type{}, std::true_type{});
+  else rows(std::true_type{}, std::false_type{});
 }
 
 inline int32_t cdiv(int64_t x, int64_t y) { return static_cast<int32_t>((x + y - 1) / y); }
@@ -922,9 +948,14 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
     return int64_t(cdiv(ms[i], 4 * lanes)) * cdiv(ns[i], int64_t(rows) * (kWave / lanes));
   };
   int64_t tiles = 0;
-  for (int i = 0; i < count; i++) tiles += tiles_of(i, kDecRowsPerBlock);
+  int64_t bytes = 0;
+  for (int i = 0; i < count; i++) {
+    tiles += tiles_of(i, kDecRowsPerBlock);
+    bytes += int64_t(ns[i]) * ms[i] * int64_t(sizeof(float));
+  }
   Args<CAP> a;
   a.partials = nullptr;
+  a.stream_m = bytes >= kDecStreamedBytes;
   // Where the chip takes the whole call at once a wave has one group of rows, not one after the other.
   a.rows = tiles < kDecTiles ? kDecRowsPerBlock / 2 : kDecRowsPerBlock;
   for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
@@ -952,9 +983,8 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
       }
       if (a.nseg == 0) continue;
       // One read and three writes per element: held to two workgroups per CU (LDS the kernel never touches,
-      // hpx_common.h), the 36 matrices of the configuration decode in 755 us instead of 792 (three per CU: 776).  Between the
-      // other phases of a pass it has been 750 in one process and 813 in another, for the same kernel and matrices at
-      // other addresses.
+      // hpx_common.h), the 36 matrices of the configuration decode in 765 us instead of 784 with three or four (a
+      // pass over three such sets of buffers in turn).
       PSGD_LAUNCH_CG_LDS(psgd_decode_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds2, st, a);
       HPX_HIP(hipGetLastError());
     }
