@@ -55,6 +55,17 @@ def test_widths_around_the_strips(psgd, m):
     _phases(psgd, [(n, m, min(2, m)) for n in (8201, 129)], m + 1)
 
 
+@pytest.mark.parametrize("n", [31, 32, 33, 255, 256, 257, 1055, 2081])
+def test_heights_around_the_blocks_of_rows(psgd, n):
+    # blocks of 32, 64 and 128 rows dealt out to the partials of a strip, the last one not whole
+    _phases(psgd, [(n, m, min(4, n)) for m in (1024, 384, 192, 70)], n)
+
+
+@pytest.mark.parametrize("n,m", [(4095, 4096), (4097, 4096), (5001, 3500)])
+def test_matrices_around_the_larger_number_of_partials(psgd, n, m):
+    _phases(psgd, [(n, m, 4)], n + m)
+
+
 @pytest.mark.parametrize("count", [1, 16, 17, 64, 65, 161])
 def test_tables_of_every_size(psgd, count):
     _phases(psgd, [(5 + 3 * (i % 11), 9 + 7 * (i % 13), 1 + i % 4) for i in range(count)], count)

@@ -511,7 +511,9 @@ __global__ __launch_bounds__(kOrthThreads) void psgd_orth_kernel(const Args<CAP>
 
 // ---- encode2, step 2: Q = M^T P ------------------------------------------------
 // A workgroup takes a strip of columns (256, or 128 or 64 with two or four rows side by side in a wave: strip_lanes)
-// and sg.rows rows of it (two or four times that), the rows going round its waves.  Per row a
+// and sg.rows rows of it (two or four times that), in blocks of 32 rows (64, 128) that the workgroups of a strip take in
+// turn: what is being read at any time is one stretch of the matrix, not a place every sg.rows rows (the layer set 210 us
+// with each workgroup's rows in one piece, 188 so).  The rows of a block go round the waves.  Per row a
 // lane loads its 4 columns of M with one 128-bit load; register t of that load
 // is the A operand of MFMA t, whose block b / row-of-block i' is column
 // k0 + 16b + 4i' + t; the B operand is P[row][j] in every block.  The waves (and the rows side by side) meet
@@ -533,8 +535,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
   const int k0 = strip * width;
   const int kk = k0 + 4 * (lane & (lanes - 1));
   const int step = kWaves * side;  // rows of the workgroup per round
-  const int64_t last = int64_t(rblk + 1) * sg.rows * side;
-  const int64_t rend = last < n ? last : n;
+  const int64_t per = int64_t(sg.rows) * side, parts = (n + per - 1) / per;
 
   f32x4 acc[CG][4];
 #pragma unroll
@@ -544,13 +545,14 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
 
   const int j = lane & 3;
   const int mine = lane / lanes;  // which of the rows side by side
-  int64_t row0 = int64_t(rblk) * sg.rows * side + wave * side;  // the first of the wave's rows in a round
-  // Main loop: 8 rounds at a time, every load issued before the first use, summed on their own in two chains and added to
+  constexpr int kRows = 8;
+  const int64_t block = kRows * step;
+  int64_t row0 = rblk * block + wave * side;  // the first of the wave's rows in a round
+  // Main loop: a block at a time, every load issued before the first use, summed on their own in two chains and added to
   // what there is (one chain of fp32 sums down all rows of a partial of 512 left Q half as far again from the exact product;
   // two chains of four instead of one of eight 8.24e-8 of its norm for 4096 x 4096 and 7.5e-8 for 200 x 600, from
   // 8.46e-8 and 7.7e-8).  Only the lane that holds the row's end and those past it take the element-wise way.
-  constexpr int kRows = 8;
-  for (; row0 + (kRows - 1) * step + side <= rend; row0 += kRows * step) {
+  for (; row0 + (kRows - 1) * step + side <= n; row0 += parts * block) {
     float4 m4[kRows];
     float p[kRows][CG];
     const float* Mp = M + (row0 + mine) * m + kk;
@@ -583,10 +585,12 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
       for (int t = 0; t < 4; t++) acc[c][t] += sum[0][t] + sum[1][t];
     }
   }
-  for (; row0 < rend; row0 += step) {
+  // the matrix's last block, where this wave's rows of it are not whole
+  const int64_t after = row0 - wave * side + block;
+  for (const int64_t rend = after < n ? after : n; row0 < rend; row0 += step) {
     const int64_t row = row0 + mine;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
-    if (row < rend) {
+    if (row < n) {
       const float* q = M + row * m + kk;
       if (kk + 4 <= m) {
         const float4 m4 = ld4_stream(q);
@@ -599,7 +603,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
 #pragma unroll
     for (int c = 0; c < CG; c++) {
       const int col = c * 4 + j;
-      const float p = row < rend && col < r ? P[row * ld + col] : 0.f;
+      const float p = row < n && col < r ? P[row * ld + col] : 0.f;
 #pragma unroll
       for (int t = 0; t < 4; t++) acc[c][t] = mfma4(v[t], p, acc[c][t]);
     }
@@ -614,7 +618,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
       for (int ii = 0; ii < 4; ii++) s_q[wave][c][16 * (lane >> 2) + 4 * ii + t][j] = acc[c][t][ii];
   __syncthreads();
   // the one partial of a matrix of few rows is Q itself
-  const bool whole = int64_t(sg.rows) * side >= n;
+  const bool whole = parts == 1;
   float* part = whole ? sg.Qout : a.partials + (int64_t(sg.part_off) * 4) + int64_t(rblk) * m * r;
   const int stride = whole ? ld : r;
   for (int e = threadIdx.x; e < CG * width * 4; e += kThreads) {
@@ -867,11 +871,14 @@ inline int32_t q_parts(int n, int m, int rows) { return cdiv(n, int64_t(rows) * 
 // 1574 / 1588, 4096 x 4096 alone 116 / 127 / 119, 4 of 2000 x 1000 74 / 70 / 70, ResNet-50's 54 157.6 / 157.5 / 157.5
 // (with 32 rows for all of those 160.5); with kQTiles 64 and 32 4096 x 1024 alone is at 59 and 68 instead of 56.
 constexpr int kQRowsMin = 32, kQRowsMax = 512;
-constexpr int64_t kQTiles = 128, kQTilesSmall = 32;
+// A matrix of 2^24 elements and more is given kQTilesLarge: 4096 x 4096 alone 127 us with 128 workgroups, 119 with 256; the
+// layer set, which twelve such matrices are part of, pays 4 of 1565 for their partials, and 8 if all 36 have as many.
+constexpr int64_t kQTiles = 128, kQTilesSmall = 32, kQTilesLarge = 256;
 inline int q_rows(int n, int m) {
   auto tiles = [=](int rows) { return int64_t(cdiv(m, 4 * strip_lanes(m))) * q_parts(n, m, rows); };
   int rows = kQRowsMax;
-  while (rows > 2 * kQRowsMin && tiles(rows) < kQTiles) rows /= 2;
+  const int64_t enough = int64_t(n) * m >= (1 << 24) ? kQTilesLarge : kQTiles;
+  while (rows > 2 * kQRowsMin && tiles(rows) < enough) rows /= 2;
   return rows == 2 * kQRowsMin && tiles(rows) < kQTilesSmall ? kQRowsMin : rows;
 }
 
