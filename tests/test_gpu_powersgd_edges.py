@@ -153,27 +153,42 @@ def test_a_matrix_alone_and_among_others(psgd):
             assert_bits_equal(a, b, f"{s} {what}")
 
 
-@pytest.mark.parametrize("big", [(7679, 4096), (7680, 4096), (7683, 4100), (8001, 4160)])
-def test_decode_of_calls_that_store_m_streaming(psgd, big):
-    # 120 MiB of M and more, whole tiles and ragged ones, a gradient that ends within M, ranks of one and two passes: the bits
-    # of every matrix decoded by a call of its own, and of the big one in row blocks that are far from the line.
-    g = torch.Generator(device="cuda").manual_seed(big[0])
-    shapes = [big + (4, 0), (65, 4096, 4, 3000), (33, 512, 18, 0), (130, 147, 2, 1)]
+@pytest.mark.parametrize("elements", [5 << 19, 3 << 24])
+@pytest.mark.parametrize("more", [-1, 0, 700])
+def test_calls_around_what_stays_in_the_caches(psgd, elements, more):
+    # 10 and 192 MiB of M are where encode1 changes what it leaves in the caches: the bits of every matrix are those of a call
+    # of its own (a few rows at a time: far below the line), whole and ragged rows, a gradient that ends within M, ranks of
+    # one and two passes.
+    g = torch.Generator(device="cuda").manual_seed(elements + more)
+    shapes = [(elements // 2048 + more, 2048, 4, 0), (65, 2048, 4, 3000), (33, 512, 18, 0), (130, 147, 2, 1)]
     rand = lambda *s: torch.empty(*s, device="cuda").normal_(generator=g)
-    P = [rand(n, r) for n, m, r, cut in shapes]
+    G0, R0 = [rand(n * m - cut) for n, m, r, cut in shapes], [rand(n * m - cut) for n, m, r, cut in shapes]
     Q = [rand(m, r) for n, m, r, cut in shapes]
-    G0 = [rand(n * m - cut) for n, m, r, cut in shapes]
-    empty = lambda: ([torch.full((n, m), 7.0, device="cuda") for n, m, r, cut in shapes], [torch.full_like(x, 7.0) for x in G0], [x.clone() for x in G0])
-    M, R, G = empty()
-    psgd.decode(P, Q, M, R, G)
-    wM, wR, wG = empty()
-    n, m = big
-    step = 3840  # rows of the big matrix at a time: whole tiles of 32 rows
-    for a in range(0, n, step):
-        b = min(n, a + step)
-        psgd.decode([P[0][a:b]], [Q[0]], [wM[0][a:b]], [wR[0][a * m:b * m]], [wG[0][a * m:b * m]])
-    for i in range(1, len(shapes)):
-        psgd.decode([P[i]], [Q[i]], [wM[i]], [wR[i]], [wG[i]])
-    for i, s in enumerate(shapes):
-        for got, want, what in ((M, wM, "M"), (R, wR, "residual"), (G, wG, "gradient")):
-            assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), (s, what)
+    results = []
+    for split in (False, True):
+        M = [torch.full((n, m), 7.0, device="cuda") for n, m, r, cut in shapes]
+        P = [torch.full((n, r), 7.0, device="cuda") for n, m, r, cut in shapes]
+        G, R = [x.clone() for x in G0], [x.clone() for x in R0]
+        if not split:
+            psgd.encode1(G, R, Q, M, P)
+            factors = [p.clone() for p in P]
+            psgd.decode(P, Q, M, R, G)
+        else:
+            n, m = shapes[0][:2]
+            for a in range(0, n, 1024):   # whole groups of four rows
+                b = min(n, a + 1024)
+                part = lambda x: [x[0][a * m:b * m]]
+                psgd.encode1(part(G), part(R), [Q[0]], [M[0][a:b]], [P[0][a:b]])
+            for i in range(1, len(shapes)):
+                psgd.encode1([G[i]], [R[i]], [Q[i]], [M[i]], [P[i]])
+            factors = [p.clone() for p in P]
+            for a in range(0, n, 1024):
+                b = min(n, a + 1024)
+                part = lambda x: [x[0][a * m:b * m]]
+                psgd.decode([P[0][a:b]], [Q[0]], [M[0][a:b]], part(R), part(G))
+            for i in range(1, len(shapes)):
+                psgd.decode([P[i]], [Q[i]], [M[i]], [R[i]], [G[i]])
+        results.append((factors, M, R, G))
+    for one, other, what in zip(*results, ("P", "M", "residual", "gradient")):
+        for x, y, s in zip(one, other, shapes):
+            assert torch.equal(x.view(torch.int32), y.view(torch.int32)), (s, what)

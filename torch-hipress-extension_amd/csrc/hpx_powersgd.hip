@@ -78,20 +78,24 @@ template <int CAP>
 struct Args {
   int32_t nseg;
   int32_t rows;        // decode: rows of a tile (of a strip 256 columns wide)
-  int32_t stream_m;    // decode: M is stored streaming too (kDecStreamedBytes)
+  int32_t keep;        // encode1: a Keep
   int32_t tile_start[CAP + 1];
   Seg seg[CAP];
   float* partials;
 };
 static_assert(sizeof(Args<kSegLarge>) <= 18000, "kernel-argument budget");
 
-// Decode: bytes of M in a call from which M is stored streaming as the residual and the gradient are.  One array of less
-// than half the 256 MB Infinity Cache stays there when the launch ends and reaches memory beside the launches that follow,
-// which read; a larger one is written out within the launch, line by line between the two streams.  us of a decode with M
-// plain / streaming (a call of one matrix of 4096 columns): 84 MB 56.6 / 61.1, 109 MB 72.4 / 77.7, 126 MB 88.2 / 87.7, 134 MB
-// 97.1 / 91.9, 185 MB 130.9 / 122.9; ResNet-50's 94 MB 64 / 76, the layer set's 1208 MB 813 / 765.  Two arrays plain, or all
-// three, are slower than one at every size.
-constexpr int64_t kDecStreamedBytes = int64_t(120) << 20;
+// What a pass keeps in the 256 MB Infinity Cache from one phase to the next, by the bytes of M in the call.  Streaming
+// accesses leave nothing there, plain ones do.  encode1 reads the gradient, which decode reads again, and writes M, which
+// encode2 reads and decode writes; decode's three outputs are streamed, array after array.  us of a pass (encode1, encode2
+// and decode of matrices of 4096 columns, three sets of buffers in turn) with encode1 streaming everything / keeping the
+// gradient and M / keeping the gradient: 8 MB 36.9 / 38.0 / 38.6, 17 MB 49.1 / 48.4 / 52.5, 34 MB 82.4 / 76.7 / 79.5, 67 MB
+// 123 / 112 / 117, 117 MB 191 / 177 / 182, 168 MB 263 / 251 / 251, 201 MB 306 / 294 / 291, 235 MB 351 / 339 / 335; ResNet-50's
+// 94 MB 168 / 151 / 153, the layer set's 1208 MB 1562 / 1581 / 1556.
+constexpr int64_t kKeepFrom = 10 << 20;        // below, everything stays in the caches anyway
+constexpr int64_t kKeepBothTo = 192 << 20;     // gradient and M together 384 MB: the first third of each is lost
+enum Keep : int32_t { kKeepNone, kKeepGradM, kKeepGradOnly };
+inline Keep keep_rule(int64_t m_bytes) { return m_bytes < kKeepFrom ? kKeepNone : m_bytes < kKeepBothTo ? kKeepGradM : kKeepGradOnly; }
 template <bool STREAM>
 __device__ __forceinline__ float4 ld4_as(const float* p) { return STREAM ? ld4_stream(p) : ld4(p); }
 template <bool STREAM>
@@ -148,17 +152,17 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
   for (int c = 0; c < CG; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const bool rows_full = (row0 + 3 < n) && ((row0 + 4) * m <= N);
-  auto chunks = [&](auto stream) {
-    constexpr bool STREAM = decltype(stream)::value;
-    // Main loop: kUnroll 64-column steps at a time, every load issued before the first use.
-    for (int k0 = part * kChunk; k0 < mfull; k0 += split * kChunk) {
-      float4 g4[kUnroll], r4[kUnroll];
-      float q[kUnroll][4][CG];
+  const float* __restrict__ A = from_m ? M : G;
+  const int64_t lane_at = row * m + 4 * b;
+  struct Chunk { float4 g[kUnroll], r[kUnroll]; float q[kUnroll][4][CG]; };
+  auto chunks = [&](auto stream_g, auto stream_r, auto stream_m) {
+    constexpr bool G_STREAM = decltype(stream_g)::value, R_STREAM = decltype(stream_r)::value, M_STREAM = decltype(stream_m)::value;
+    // kUnroll 64-column steps at a time, every load issued before the first use
+    auto load = [&](Chunk& h, int k0) {
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
-        const int64_t f = row * m + k0 + 64 * u + 4 * b;
-        g4[u] = from_m ? ld4_as<STREAM>(M + f) : ld4_as<STREAM>(G + f);
-        r4[u] = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_as<STREAM>(R + f);
+        h.g[u] = ld4_as<G_STREAM>(A + lane_at + k0 + 64 * u);
+        h.r[u] = from_m ? make_float4(0.f, 0.f, 0.f, 0.f) : ld4_as<R_STREAM>(R + lane_at + k0 + 64 * u);
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; u++)
@@ -167,30 +171,62 @@ __global__ __launch_bounds__(kThreads) void psgd_encode1_kernel(const Args<CAP> 
 #pragma unroll
           for (int c = 0; c < CG; c++) {
             const int col = c * 4 + i;  // B operand: lane 4b+j holds Q[k][j]
-            q[u][t][c] = col < r ? Q[int64_t(k0 + 64 * u + 4 * b + t) * ld + col] : 0.f;
+            h.q[u][t][c] = col < r ? Q[int64_t(k0 + 64 * u + 4 * b + t) * ld + col] : 0.f;
           }
-      // Of each half of this chunk, added to the rest afterwards: shorter chains of fp32 sums.  (P's distance from the exact
-      // product 1.00e-7 of its norm for 4096 x 4096, 9.1e-8 for 200 x 600; in one chain 1.09e-7 and 1.11e-7; time alike.)
+    };
+    // Of each half of a chunk, added to the rest afterwards: shorter chains of fp32 sums.  (P's distance from the exact
+    // product 1.00e-7 of its norm for 4096 x 4096, 9.1e-8 for 200 x 600; in one chain 1.09e-7 and 1.11e-7; time alike.)
+    auto use = [&](const Chunk& h, int k0) {
       f32x4 sum[2][CG];
 #pragma unroll
       for (int c = 0; c < CG; c++) sum[0][c] = sum[1][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
-        const int64_t f = row * m + k0 + 64 * u + 4 * b;
-        const float4 m4 = make_float4(g4[u].x + r4[u].x, g4[u].y + r4[u].y, g4[u].z + r4[u].z, g4[u].w + r4[u].w);
-        if (!from_m) st4_as<STREAM>(M + f, m4);  // the set of M matrices is far larger than the caches: do not allocate
+        const float4 m4 = make_float4(h.g[u].x + h.r[u].x, h.g[u].y + h.r[u].y, h.g[u].z + h.r[u].z, h.g[u].w + h.r[u].w);
+        if (!from_m) st4_as<M_STREAM>(M + lane_at + k0 + 64 * u, m4);
         const float v[4] = {m4.x, m4.y, m4.z, m4.w};
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
-          for (int c = 0; c < CG; c++) sum[u & 1][c] = mfma4(v[t], q[u][t][c], sum[u & 1][c]);
+          for (int c = 0; c < CG; c++) sum[u & 1][c] = mfma4(v[t], h.q[u][t][c], sum[u & 1][c]);
       }
 #pragma unroll
       for (int c = 0; c < CG; c++) acc[c] += sum[0][c] + sum[1][c];
+    };
+    // Two chunks in turn, the next one's loads under way while one is used: 2048 x 1024 alone 37.7 us for all three phases
+    // (one chunk after the other 38.8), the layer set 1563 (1572).
+    const int step = split * kChunk;
+    int k0 = part * kChunk;
+    if (k0 >= mfull) return;
+    Chunk x, y;
+    if constexpr (CG > 1) {  // (their Q takes the registers: rank 8 with two chunks in turn 36 matrices 566, so 560)
+#pragma unroll 1
+      for (; k0 < mfull; k0 += step) {
+        load(x, k0);
+        use(x, k0);
+      }
+      return;
+    }
+    load(x, k0);
+#pragma unroll 1
+    for (;;) {
+      const int k1 = k0 + step;
+      if (k1 < mfull) load(y, k1);
+      use(x, k0);
+      if (k1 >= mfull) return;
+      k0 = k1 + step;
+      if (k0 < mfull) load(x, k0);
+      use(y, k1);
+      if (k0 >= mfull) return;
     }
   };
-  if (rows_full) {
-    if (rows_on_lines(m, G, R, M)) chunks(std::true_type{}); else chunks(std::false_type{});
+  if (rows_full) {  // (a loop for each choice: of one loop with a choice at each access the compiler makes plain ones)
+    constexpr auto kPlain = std::false_type{};
+    constexpr auto kStream = std::true_type{};
+    if (!rows_on_lines(m, G, R, M)) chunks(kPlain, kPlain, kPlain);
+    else if (a.keep == kKeepNone) chunks(kStream, kStream, kStream);
+    else if (a.keep == kKeepGradM) chunks(kPlain, kStream, kPlain);
+    else chunks(kPlain, kStream, kStream);
   }
   // What is left of the columns (or everything, of rows that are not full), two steps' loads in flight together where the
   // wave has several (four: as fast, but the registers they take slow the loop above): one step after the other, each
@@ -697,9 +733,9 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
 #pragma unroll
     for (int col = 0; col < CG * 4; col++) q[t][col] = (kk + t < m && col < r) ? Q[int64_t(kk + t) * ld + col] : 0.f;
 
-  // (a loop for each choice: of one loop with a choice at each store the compiler makes plain stores)
-  auto rows = [&](auto stream, auto stream_m) {
-    constexpr bool STREAM = decltype(stream)::value, STREAM_M = decltype(stream_m)::value;
+  // (two loops: of one loop with a choice at each store the compiler makes plain stores)
+  auto rows = [&](auto stream) {
+    constexpr bool STREAM = decltype(stream)::value;
     for (int64_t at = rbeg; at < rend; at += 4 * side) {
       const int64_t row0 = at + 4 * (lane / lanes);
       const bool full4 = kk + 4 <= m && row0 + 4 <= rend && (row0 + 3) * m + kk + 4 <= N;
@@ -731,27 +767,15 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
           m4[ii] = make_float4(acc[0][ii], acc[1][ii], acc[2][ii], acc[3][ii]);
           r4[ii] = make_float4(g4[ii].x - m4[ii].x, g4[ii].y - m4[ii].y, g4[ii].z - m4[ii].z, g4[ii].w - m4[ii].w);
         }
-        if constexpr (STREAM_M) {
-          // array after array (the layer set: 763 us; row after row 794)
-          if (!keep_grad) {
+        // array after array (the layer set: 765 us; row after row 794)
+        if (!keep_grad) {
 #pragma unroll
-            for (int ii = 0; ii < 4; ii++) st4_stream(R + (row0 + ii) * m + kk, r4[ii]);
+          for (int ii = 0; ii < 4; ii++) st4_as<STREAM>(R + (row0 + ii) * m + kk, r4[ii]);
 #pragma unroll
-            for (int ii = 0; ii < 4; ii++) st4_stream(G + (row0 + ii) * m + kk, m4[ii]);  // in place over the line just read
-          }
-#pragma unroll
-          for (int ii = 0; ii < 4; ii++) st4_stream(M + (row0 + ii) * m + kk, m4[ii]);
-        } else {
-#pragma unroll
-          for (int ii = 0; ii < 4; ii++) {
-            const int64_t f = (row0 + ii) * m + kk;
-            if (!keep_grad) {
-              st4_as<STREAM>(R + f, r4[ii]);
-              st4_as<STREAM>(G + f, m4[ii]);
-            }
-            st4(M + f, m4[ii]);
-          }
+          for (int ii = 0; ii < 4; ii++) st4_as<STREAM>(G + (row0 + ii) * m + kk, m4[ii]);  // in place over the line just read
         }
+#pragma unroll
+        for (int ii = 0; ii < 4; ii++) st4_as<STREAM>(M + (row0 + ii) * m + kk, m4[ii]);
         continue;
       }
 #pragma unroll
@@ -773,9 +797,7 @@ __global__ __launch_bounds__(kThreads) void psgd_decode_kernel(const Args<CAP> a
       }
     }
   };
-  if (!rows_on_lines(m, G, R, M)) rows(std::false_type{}, std::false_type{});
-  else if (a.stream_m) rows(std::true_type{}, std::true_type{});
-  else rows(std::true_type{}, std::false_type{});
+  if (rows_on_lines(m, G, R, M)) rows(std::true_type{}); else rows(std::false_type{});
 }
 
 inline int32_t cdiv(int64_t x, int64_t y) { return static_cast<int32_t>((x + y - 1) / y); }
@@ -821,6 +843,9 @@ int encode1_launches(int count, int max_rank, const float* const* grads, const i
                      const float* const* Qs, float* const* Ms, float* const* Ps, const int32_t* ns, const int32_t* ms,
                      const int32_t* rs, hipStream_t st) {
   Args<CAP> a;
+  int64_t m_bytes = 0;
+  for (int k = 0; k < count; k++) m_bytes += int64_t(ns[k]) * ms[k] * int64_t(sizeof(float));
+  a.keep = keep_rule(m_bytes);
   a.partials = nullptr;
   for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
     int i = 0;
@@ -842,8 +867,8 @@ int encode1_launches(int count, int max_rank, const float* const* grads, const i
         i++;
       }
       if (a.nseg == 0) continue;
-      // Two read streams and a write stream: held to four workgroups per CU (LDS the kernel never touches), 36 matrices
-      // of the layer set 598 us instead of 618 (five per CU: 607, three: 599), ResNet-50's 54 61.6 instead of 64.0.
+      // Two read streams and a write stream: held to four workgroups per CU (LDS the kernel never touches).  Ranks up to
+      // four are held to three by their registers; without either limit the layer set's 36 matrices took 618 us, at four 598.
       PSGD_LAUNCH_CG_LDS(psgd_encode1_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds4, st, a);
       HPX_HIP(hipGetLastError());
     }
@@ -955,14 +980,9 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
     return int64_t(cdiv(ms[i], 4 * lanes)) * cdiv(ns[i], int64_t(rows) * (kWave / lanes));
   };
   int64_t tiles = 0;
-  int64_t bytes = 0;
-  for (int i = 0; i < count; i++) {
-    tiles += tiles_of(i, kDecRowsPerBlock);
-    bytes += int64_t(ns[i]) * ms[i] * int64_t(sizeof(float));
-  }
+  for (int i = 0; i < count; i++) tiles += tiles_of(i, kDecRowsPerBlock);
   Args<CAP> a;
   a.partials = nullptr;
-  a.stream_m = bytes >= kDecStreamedBytes;
   // Where the chip takes the whole call at once a wave has one group of rows, not one after the other.
   a.rows = tiles < kDecTiles ? kDecRowsPerBlock / 2 : kDecRowsPerBlock;
   for (int c0 = 0; c0 < max_rank; c0 += kPassCols) {
