@@ -148,10 +148,17 @@ __global__ __launch_bounds__(kThreads) void tbq_encode_kernel(const EncArgs<CAP>
     reinterpret_cast<u32u*>(op + gw + 4 * lane)->v = dw;  // messages start at any byte
     return;
   }
-  // First (short) or last tile of the tensor: bounds-checked, and the lane owning the
-  // partial group leaves the fields past the end at code 1.  All loads first: the last
-  // tile of the last tensor is the tail of the launch.
+  // First (short) or last tile of the tensor: bounds-checked; the partial group goes an element to a lane (one lane that
+  // took them in turn waited for memory up to six times in a row).  All loads first: the last tile of the last tensor is
+  // the tail of the launch.
   const uint32_t lim = glim < full ? glim : full;  // complete groups of this tile end here
+  const bool one = full >= gbeg && full < glim && threadIdx.x < (n & 3);  // this lane's one of the partial group's elements
+  const size_t e1 = size_t(full) * 4 + threadIdx.x;
+  float g1 = 0.f, r1 = 0.f;
+  if (one) {
+    g1 = gp[e1];
+    r1 = rp[e1];
+  }
   float4 gt[kIters], rt[kIters];
 #pragma unroll
   for (int k = 0; k < kIters; k++) {
@@ -170,16 +177,17 @@ __global__ __launch_bounds__(kThreads) void tbq_encode_kernel(const EncArgs<CAP>
       const uint32_t q = tbq_code4(gv, rv, thr);
       st4(rp + e, rv);
       op[grp] = static_cast<uint8_t>(q);
-    } else if (grp == full && grp < glim && (n & 3)) {
-      uint32_t q = 85;
-      for (uint32_t j = 0; j < (n & 3); j++) {
-        float r = rp[e + j];
-        const uint32_t c = tbq_code(gp[e + j], r, thr);
-        rp[e + j] = r;
-        q = (q & ~(3u << (2 * j))) | (c << (2 * j));
-      }
-      op[grp] = static_cast<uint8_t>(q);
     }
+  }
+  if (threadIdx.x < kWave) {
+    uint32_t q = 1u << (2 * (threadIdx.x & 3));  // the fields past the end stay at code 1
+    if (one) {
+      q = tbq_code(g1, r1, thr) << (2 * threadIdx.x);
+      rp[e1] = r1;
+    }
+    q |= __shfl_xor(q, 1, kWave);
+    q |= __shfl_xor(q, 2, kWave);
+    if (one && threadIdx.x == 0) op[full] = static_cast<uint8_t>(q);
   }
 }
 
@@ -229,6 +237,14 @@ __device__ __forceinline__ void tbq_decode_tile(const DecSeg& sg, uint32_t t) {
     return;
   }
   const uint32_t lim = glim < full ? glim : full;  // complete groups of this (first or last) tile end here
+  const bool one = full >= gbeg && full < glim && threadIdx.x < (n & 3);  // this lane's one of the partial group's elements
+  const size_t e1 = size_t(full) * 4 + threadIdx.x;
+  uint32_t q1 = 0;
+  float o1 = 0.f;
+  if (one) {
+    q1 = ip[full];
+    if (ADD) o1 = op[e1];
+  }
   uint32_t qt[kIters];
   float4 ot[kIters];
 #pragma unroll
@@ -250,13 +266,11 @@ __device__ __forceinline__ void tbq_decode_tile(const DecSeg& sg, uint32_t t) {
         v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
       }
       st4(op + e, v);
-    } else if (grp == full && grp < glim && (n & 3)) {
-      const uint32_t q = ip[grp];
-      for (uint32_t j = 0; j < (n & 3); j++) {
-        const float v = (static_cast<float>((q >> (2 * j)) & 3) - 1) * thr;
-        op[e + j] = ADD ? v + op[e + j] : v;
-      }
     }
+  }
+  if (one) {
+    const float v = (static_cast<float>((q1 >> (2 * threadIdx.x)) & 3) - 1) * thr;
+    op[e1] = ADD ? v + o1 : v;
   }
 }
 
@@ -417,9 +431,13 @@ __global__ __launch_bounds__(kThreads) void tbq_decode_multi_kernel(const Args a
   }
   // The tile that holds the end of the tensor.  Its whole groups are handled like the ones above, one byte
   // load per group and message, with the loads of all of a lane's groups and of up to 8 messages in flight
-  // together; only the last, partial group goes element by element.  (Done element by element for the whole
+  // together, and with them the last, partial group, an element to a lane.  (Done element by element for the whole
   // tile, every element waited for its own loads, message after message: up to 16 x (1 + messages) memory
   // latencies in a row in ONE workgroup, tens of microseconds that the rest of the grid could not hide.)
+  const uint32_t first = g0 - threadIdx.x;
+  const bool one = full >= first && full - first < uint32_t(kTileGroups) && threadIdx.x < (n & 3u);  // this lane's one of the last, partial group
+  const size_t e1 = size_t(full) * 4 + threadIdx.x;
+  float sum = one && need_old ? op[e1] : 0.f;
   float4 acc[kIters];
   bool live[kIters];
 #pragma unroll
@@ -437,11 +455,19 @@ __global__ __launch_bounds__(kThreads) void tbq_decode_multi_kernel(const Args a
         q[jj][k] = 85u;
         if (j0 + jj < ns && live[k]) q[jj][k] = as_global(s_in[j0 + jj])[g0 + k * kThreads];
       }
+    uint32_t q1[8];
+#pragma unroll
+    for (int jj = 0; jj < 8; jj++) {
+      q1[jj] = 85u;
+      if (j0 + jj < ns && one) q1[jj] = as_global(s_in[j0 + jj])[full];
+    }
 #pragma unroll
     for (int jj = 0; jj < 8; jj++) {
       if (j0 + jj < ns) {
         const float thr = s_thr[j0 + jj];
         const bool add = s_add[j0 + jj] != 0;
+        const float x = (static_cast<float>((q1[jj] >> (2 * (threadIdx.x & 3))) & 3) - 1) * thr;
+        sum = add ? x + sum : x;
 #pragma unroll
         for (int k = 0; k < kIters; k++) {
           const float4 v = tbq_values(q[jj][k], thr);
@@ -457,23 +483,7 @@ __global__ __launch_bounds__(kThreads) void tbq_decode_multi_kernel(const Args a
 #pragma unroll
   for (int k = 0; k < kIters; k++)
     if (live[k]) st4(op + size_t(g0 + k * kThreads) * 4, acc[k]);
-  // the partial group, if the tensor has one and it belongs to this lane
-  const uint32_t rest = n & 3u;
-  if (rest && full >= g0 && (full - g0) % kThreads == 0 && (full - g0) / kThreads < uint32_t(kIters)) {
-    const size_t e = size_t(full) * 4;
-    float tail[3];
-    for (uint32_t i = 0; i < rest; i++) tail[i] = need_old ? op[e + i] : 0.f;
-    for (int j = 0; j < ns; j++) {
-      const uint32_t q = as_global(s_in[j])[full];
-      const float thr = s_thr[j];
-      const bool add = s_add[j] != 0;
-      for (uint32_t i = 0; i < rest; i++) {
-        const float v = (static_cast<float>((q >> (2 * i)) & 3) - 1) * thr;
-        tail[i] = add ? v + tail[i] : v;
-      }
-    }
-    for (uint32_t i = 0; i < rest; i++) op[e + i] = tail[i];
-  }
+  if (one) op[e1] = sum;
 }
 
 inline int32_t tiles_for(int32_t n) {

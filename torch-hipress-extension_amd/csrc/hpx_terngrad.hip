@@ -261,7 +261,21 @@ __global__ __launch_bounds__(kThreads) void terngrad_minmax_kernel(const EncArgs
 #pragma unroll
     for (int k = 0; k < kRedIters; k++) acc3x4(v[k], mn, mx, am);
   } else {
-    for (uint32_t e = e0 + threadIdx.x; e < n; e += kThreads) acc3(xp[e], mn, mx, am);
+    // the tile that holds the end, all loads first (a lane without a group reads the tile's first)
+    const uint32_t whole = (n - e0) / 4;
+    const bool one = e0 + whole * 4 + threadIdx.x < n;
+    float4 v[kRedIters];
+    const float x = xp[size_t(e0) + (one ? whole * 4 + threadIdx.x : 0u)];
+    if (whole) {
+#pragma unroll
+      for (int k = 0; k < kRedIters; k++) {
+        const uint32_t g = k * kThreads + threadIdx.x;
+        v[k] = ld4(xp + size_t(e0) + size_t(g < whole ? g : 0u) * 4);
+      }
+#pragma unroll
+      for (int k = 0; k < kRedIters; k++) acc3x4(v[k], mn, mx, am);
+    }
+    acc3(x, mn, mx, am);
   }
   uint32_t z = (am == 0.0f) ? 0u : 1u;  // 0 when this tile holds a zero
   block_reduce(mn, mx, z);
@@ -401,34 +415,34 @@ __device__ __forceinline__ uint32_t quant_unit(const float4 (&v)[UNIT / 4], floa
   return pack_codes<B, UNIT>(t);
 }
 
-// Unit u of a tensor whose end may fall inside it: element-wise from memory.
+// The elements past a tensor's last whole unit, one to a lane, so that all of them are one wait for memory (one lane that
+// went through them element by element, and byte by byte, waited for each, here and in the reductions and decoders: one tensor of
+// 2047 elements, encode and decode, 8.4 us, now 6.9; a root's pass over 24 odd-sized gradients and three messages each 22.1,
+// now 18.3).  All lanes of a wave call, `lane` is the wave's.
 template <int B, bool RANDOM, int UNIT = (8 / B > 4 ? 8 / B : 4)>
-__device__ __forceinline__ void quant_unit_ragged(const EncSeg& sg, float mn, float gi, uint32_t u,
-                                                  const uint32_t (&draw)[UNIT]) {
-  constexpr int DPB = 8 / B;
-  constexpr int BPU = UNIT / DPB;
-  const float* __restrict__ xp = sg.x;
-  uint8_t* __restrict__ pay = sg.out + 10;
-  const uint32_t n = static_cast<uint32_t>(sg.n);
-  const uint32_t nbytes = n / DPB;  // bytes the reference's transform covers
-  for (int jb = 0; jb < BPU; jb++) {
-    const uint32_t byte = u * BPU + jb;
-    const size_t e = size_t(byte) * DPB;
-    if (byte < nbytes) {
-      uint32_t qv = 0;
-      for (int j = 0; j < DPB; j++) {
-        const uint32_t t = quant_one<B, RANDOM>(xp[e + j], mn, gi, RANDOM ? draw[jb * DPB + j] : 0u);
-        qv |= t << (B * j);
-      }
-      pay[byte] = uint8_t(qv);
-    } else if (byte == nbytes && (n % DPB)) {
-      // Partial last byte: always round-to-nearest, stored at the last byte
-      // of the caller's buffer (terngrad_body.h:288-296).
-      uint32_t qv = 0;
-      for (uint32_t j = 0; j < n % DPB; j++) qv |= quant_one<B, false>(xp[e + j], mn, gi, 0u) << (B * j);
-      sg.out[sg.out_size - 1] = uint8_t(qv);
+__device__ __forceinline__ void quant_rest(const EncSeg& sg, float mn, float gi, uint32_t lane) {
+  constexpr uint32_t DPB = 8 / B;
+  const uint32_t n = static_cast<uint32_t>(sg.n), first = n / UNIT * UNIT, rest = n - first;
+  if (rest == 0) return;
+  const bool live = lane < rest;
+  const float x = sg.x[size_t(first) + (live ? lane : 0u)];
+  const uint32_t slot = lane % DPB, byte = first / DPB + lane / DPB, nbytes = n / DPB;  // bytes the reference's transform covers
+  uint32_t t = quant_one<B, false>(x, mn, gi, 0u);
+  if (RANDOM && byte < nbytes) {
+    uint32_t mul = lcg_mul(2), add = lcg_add(2);
+#pragma unroll
+    for (int j = 1; j < int(DPB); j++) {
+      mul = slot == uint32_t(j) ? lcg_mul(j + 2) : mul;
+      add = slot == uint32_t(j) ? lcg_add(j + 2) : add;
     }
+    t = quant_one<B, true>(x, mn, gi, mul * (sg.seed + byte) + add);
   }
+  uint32_t qv = live ? t << (B * slot) : 0u;
+#pragma unroll
+  for (int o = 1; o < int(DPB); o <<= 1) qv |= __shfl_xor(qv, o, kWave);
+  // A partial last byte is always rounded to nearest, and stored at the last byte of the caller's buffer
+  // (terngrad_body.h:288-296).
+  if (live && slot == 0) *(byte < nbytes ? sg.out + 10 + byte : sg.out + sg.out_size - 1) = uint8_t(qv);
 }
 
 // The BYTES packed bytes of a unit, at an address that is only known to be a byte's (the payload starts at byte 10).
@@ -464,7 +478,6 @@ __device__ __forceinline__ void quant_tile(const EncSeg& sg, const float mn, con
     }
   }
 
-  const uint32_t units_total = (n + UNIT - 1) / UNIT;
   const uint32_t tile_u0 = u0 - threadIdx.x;
   if (uint64_t(tile_u0 + kThreads * kQIters) * UNIT <= n) {
     float4 v[kQIters][UNIT / 4];
@@ -479,8 +492,8 @@ __device__ __forceinline__ void quant_tile(const EncSeg& sg, const float mn, con
     return;
   }
   // Tile holding the end of the tensor: its whole units like those above, all loads first (a lane without one reads
-  // the tile's first and stores nothing); the partial unit, if there is one, from memory element by element.  (Done
-  // element by element throughout, this workgroup waited for memory sixteen times in a row behind all others.)
+  // the tensor's first and stores nothing), and what is left behind them.  (Done element by element throughout, this workgroup
+  // waited for memory sixteen times in a row behind all others.)
   const uint32_t whole = n / UNIT;
   float4 v[kQIters][UNIT / 4];
 #pragma unroll
@@ -489,10 +502,10 @@ __device__ __forceinline__ void quant_tile(const EncSeg& sg, const float mn, con
 #pragma unroll
     for (int h = 0; h < UNIT / 4; h++) v[k][h] = whole ? ld4(xp + size_t(u < whole ? u : 0u) * UNIT + h * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  if (threadIdx.x < kWave && whole >= tile_u0 && whole - tile_u0 < uint32_t(kThreads * kQIters)) quant_rest<B, RANDOM>(sg, mn, gi, threadIdx.x);
 #pragma unroll
   for (int k = 0; k < kQIters; k++) {
     const uint32_t u = u0 + k * kThreads;
-    if (u == whole && u < units_total) quant_unit_ragged<B, RANDOM>(sg, mn, gi, u, draw);
     const uint32_t packed = quant_unit<B, RANDOM>(v[k], mn, gi, draw, kStrideBytes);
     if (u < whole) store_codes<BPU>(pay + size_t(u) * BPU, packed);
   }
@@ -585,6 +598,7 @@ __device__ __forceinline__ void small_tensor(const EncSeg& sg) {
   const float gi = inverse_gap(mn, mx, B);
   if (t == 0) write_header(sg.out, B, n, mn, mx);
   uint8_t* __restrict__ pay = sg.out + 10;
+  if (t < kWave) quant_rest<B, RANDOM>(sg, mn, gi, t);
 #pragma unroll 1
   for (uint32_t i = steps; i-- > 0;) {   // the last step's units are still in registers
     if (i + 1 < steps) load(i);
@@ -597,7 +611,6 @@ __device__ __forceinline__ void small_tensor(const EncSeg& sg) {
 #pragma unroll
     for (int k = 0; k < kSmallRows; k++) {
       const uint32_t u = u0 + k * kSmallThreads;
-      if (u == whole && whole * UNIT < n) quant_unit_ragged<B, RANDOM>(sg, mn, gi, u, draw);
       const uint32_t packed = quant_unit<B, RANDOM>(v[k], mn, gi, draw, uint32_t(kSmallThreads) * BPU);
       if (u < whole) store_codes<BPU>(pay + size_t(u) * BPU, packed);
     }
@@ -855,8 +868,10 @@ __global__ __launch_bounds__(kResThreads) void terngrad_resident_kernel(const Re
       }
     }
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0)
-    for (uint32_t e = full_units * UNIT; e < n; e++) acc_zero(xp[e], e, mn, mx, fz);
+  if (blockIdx.x == 0) {
+    const uint32_t e = full_units * UNIT + threadIdx.x;
+    if (e < n) acc_zero(xp[e], e, mn, mx, fz);
+  }
 
   mn = wave_min(mn);
   mx = wave_max(mx);
@@ -1024,15 +1039,7 @@ __global__ __launch_bounds__(kResThreads) void terngrad_resident_kernel(const Re
       for (int h = 0; h < H; h++) ring_wait<0>(v[k][h]);
   }
   // The unit that holds the end of the tensor, if the length is not a whole number of units.
-  if (blockIdx.x == 0 && threadIdx.x == 0 && full_units * UNIT < n) {
-    uint32_t d[UNIT];
-#pragma unroll
-    for (int q = 0; q < UNIT; q++) {
-      const int jb = q / DPB, j = q % DPB;
-      d[q] = lcg_mul(j + 2) * (a.seg.seed + full_units * BPU + jb) + lcg_add(j + 2);
-    }
-    quant_unit_ragged<B, RANDOM>(a.seg, mn, gi, full_units, d);
-  }
+  if (blockIdx.x == 0 && threadIdx.x < kWave) quant_rest<B, RANDOM>(a.seg, mn, gi, threadIdx.x);
   if (a.stamps) {  // uniform
     __syncthreads();
     phase_stamp(a.stamps, 3);
@@ -1144,8 +1151,7 @@ __device__ __forceinline__ void tiny_finish(const ResMultiArgs& a, int t0, int s
 #pragma unroll
         for (int h = 0; h < H; h++) acc_zero4(v[i * ROWS + k][h], (k * kWave + lane) * UNIT + h * 4, d0, d1, fz);
     }
-    if (lane == 0)
-      for (uint32_t e = full_units * UNIT; e < n; e++) acc_zero(xp[e], e, mn, mx, fz);
+    if (full_units * UNIT + lane < n) acc_zero(xp[full_units * UNIT + lane], full_units * UNIT + lane, mn, mx, fz);
     mn = wave_min(mn);
     mx = wave_max(mx);
     fz = wave_min_u32(fz);
@@ -1176,15 +1182,7 @@ __device__ __forceinline__ void tiny_finish(const ResMultiArgs& a, int t0, int s
         for (int jb = 0; jb < BPU; jb++) pay[u * BPU + jb] = uint8_t(packed >> (8 * jb));
       }
     }
-    if (lane == 0 && full_units * UNIT < n) {
-      uint32_t d[UNIT];
-#pragma unroll
-      for (int q = 0; q < UNIT; q++) {
-        const int jb = q / DPB, j = q % DPB;
-        d[q] = lcg_mul(j + 2) * (sg.seed + full_units * BPU + jb) + lcg_add(j + 2);
-      }
-      quant_unit_ragged<B, RANDOM>(sg, mn, gi, full_units, d);
-    }
+    quant_rest<B, RANDOM>(sg, mn, gi, lane);
   }
 }
 
@@ -1301,8 +1299,7 @@ __global__ __launch_bounds__(kResThreads) void terngrad_resident_multi_kernel(co
       }
     }
   }
-  if (ends_tensor && lane == 0)
-    for (uint32_t e = full_units * UNIT; e < n; e++) acc_zero(xp[e], e, mn, mx, fz);
+  if (ends_tensor && full_units * UNIT + lane < n) acc_zero(xp[full_units * UNIT + lane], full_units * UNIT + lane, mn, mx, fz);
   mn = wave_min(mn);
   mx = wave_max(mx);
   fz = wave_min_u32(fz);
@@ -1426,15 +1423,7 @@ __global__ __launch_bounds__(kResThreads) void terngrad_resident_multi_kernel(co
     }
   }
   // The unit that holds the end of the tensor, if its length is not a whole number of units.
-  if (ends_tensor && lane == 0 && full_units * UNIT < n) {
-    uint32_t d[UNIT];
-#pragma unroll
-    for (int q = 0; q < UNIT; q++) {
-      const int jb = q / DPB, j = q % DPB;
-      d[q] = lcg_mul(j + 2) * (sg.seed + full_units * BPU + jb) + lcg_add(j + 2);
-    }
-    quant_unit_ragged<B, RANDOM>(sg, mn, gi, full_units, d);
-  }
+  if (ends_tensor) quant_rest<B, RANDOM>(sg, mn, gi, lane);  // wave-uniform
   // the last of the workgroup's waves to get here leaves the reading (the waves hold pieces of different tensors
   // and lengths and no barrier joins them again)
   if (a.stamps && lane == 0)
@@ -1492,10 +1481,17 @@ __device__ __forceinline__ void decode_tile(const DecSeg& sg, float mn, float ga
     return;
   }
   // The tile that holds the end: its whole groups as above, all loads first (a lane without one reads the tensor's
-  // first and stores nothing), then the 1..3 elements that are left.
+  // first and stores nothing), and with them the 1..3 elements that are left, one to a lane.
   const uint32_t whole = cnt / 4;
-  uint32_t q[kDIters];
+  const uint32_t last = whole * 4 + threadIdx.x;  // this lane's one of them
+  const bool one = last < cnt && whole >= g0 - threadIdx.x && whole - (g0 - threadIdx.x) < uint32_t(kThreads * kDIters);
+  uint32_t q[kDIters], code = 0;
   float4 o[kDIters];
+  float old = 0.f;
+  if (one) {
+    code = pay[last / DPB];
+    if (ADD) old = op[last];
+  }
   if (whole) {
 #pragma unroll
     for (int k = 0; k < kDIters; k++) {
@@ -1512,15 +1508,9 @@ __device__ __forceinline__ void decode_tile(const DecSeg& sg, float mn, float ga
       }
     }
   }
-#pragma unroll
-  for (int k = 0; k < kDIters; k++) {
-    if (g0 + k * kThreads == whole) {
-      for (size_t i = size_t(whole) * 4; i < cnt; i++) {
-        const uint32_t c = (pay[i / DPB] >> ((i % DPB) * B)) & MASK;
-        const float v = float(int(c)) * gap + mn;
-        op[i] = ADD ? v + op[i] : v;
-      }
-    }
+  if (one) {
+    const float v = float(int((code >> ((last % DPB) * B)) & MASK)) * gap + mn;
+    op[last] = ADD ? v + old : v;
   }
 }
 
@@ -1952,11 +1942,14 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const A
   }
   if (all_cover) {
     // The sub-tile that holds the end of the tensor, every message complete.  Its whole groups are handled like
-    // the ones above, with the loads of all of a lane's groups and of up to 8 messages in flight together; only
-    // the tensor's last, partial group goes element by element.  (Done element by element for the whole
+    // the ones above, with the loads of all of a lane's groups and of up to 8 messages in flight together, and with them
+    // the tensor's last, partial group, an element to a lane.  (Done element by element for the whole
     // sub-tile, each element waited for its own loads, message after message: up to 16 x (1 + messages)
     // memory latencies in a row in ONE workgroup.  Depending on n mod 4096 that tail alone took up to 35 us and
     // made the time of a 7-message decode jump up and down with the size of the tensor.)
+    const uint32_t last = n / 4 * 4 + threadIdx.x, g_first = g0 - threadIdx.x;
+    const bool one = last < n && n / 4 - g_first < uint32_t(kThreads * kDIters);  // this lane's one of the last, partial group
+    float sum = one && need_old ? op[last] : 0.f;
     float4 acc[kDIters];
     bool live[kDIters];
 #pragma unroll
@@ -1978,16 +1971,25 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const A
             global_ptr<uint8_t> pay = as_global(s_pay[j0 + jj]);
             if (bits == 1) raw[jj][k] = (uint32_t(pay[e >> 3]) >> (e & 4)) & 0xFu;
             else if (bits == 2) raw[jj][k] = pay[e >> 2];
-            else if (bits == 4) raw[jj][k] = uint32_t(pay[e >> 1]) | (uint32_t(pay[(e >> 1) + 1]) << 8);
-            else raw[jj][k] = uint32_t(pay[e]) | (uint32_t(pay[e + 1]) << 8) | (uint32_t(pay[e + 2]) << 16) | (uint32_t(pay[e + 3]) << 24);
+            else if (bits == 4) raw[jj][k] = reinterpret_cast<global_ptr<u16u>>(pay + (e >> 1))->v;
+            else raw[jj][k] = reinterpret_cast<global_ptr<u32u>>(pay + e)->v;
           }
         }
+      uint32_t code[8];
+#pragma unroll
+      for (int jj = 0; jj < 8; jj++) {
+        code[jj] = 0;
+        if (j0 + jj < ns && one) code[jj] = as_global(s_pay[j0 + jj])[last / (8u / s_bits[j0 + jj])];
+      }
 #pragma unroll
       for (int jj = 0; jj < 8; jj++) {
         if (j0 + jj < ns) {
           const uint32_t bits = s_bits[j0 + jj];
           const float gap = s_gap[j0 + jj], mn = s_mn[j0 + jj];
           const bool add = s_add[j0 + jj] != 0;
+          const uint32_t c = (code[jj] >> (last % (8u / bits) * bits)) & ((1u << bits) - 1u);
+          const float x = float(int(c)) * gap + mn;  // terngrad_body.h:127, :158
+          sum = add ? x + sum : x;
 #pragma unroll
           for (int k = 0; k < kDIters; k++) {
             float4 v;
@@ -2007,25 +2009,7 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const A
 #pragma unroll
     for (int k = 0; k < kDIters; k++)
       if (live[k]) st4(op + size_t(g0 + k * kThreads) * 4, acc[k]);
-    // the tensor's last 1..3 elements, if this lane owns them
-#pragma unroll
-    for (int k = 0; k < kDIters; k++) {
-      const size_t e = size_t(g0 + k * kThreads) * 4;
-      if (e < n && !live[k]) {
-        float tail[3];
-        const int lim = int(n - e);
-        for (int i = 0; i < lim; i++) tail[i] = need_old ? op[e + i] : 0.f;
-        for (int j = 0; j < ns; j++) {
-          const float gap = s_gap[j], mn = s_mn[j];
-          const bool add = s_add[j] != 0;
-          for (int i = 0; i < lim; i++) {
-            const float v = float(int(code_at(s_pay[j], e + i, s_bits[j]))) * gap + mn;  // terngrad_body.h:127, :158
-            tail[i] = add ? v + tail[i] : v;
-          }
-        }
-        for (int i = 0; i < lim; i++) op[e + i] = tail[i];
-      }
-    }
+    if (one) op[last] = sum;
     continue;
   }
   // Messages that cover different numbers of elements (a clamped or malformed header): element by element.
