@@ -1,0 +1,54 @@
+"""GPU parity of the sparsifier's lists of candidates, one per 1024 elements: large values crowded into some of them, so
+that a list is full to the last place or one beyond it, and kept fractions on either side of the one up to which the
+lists are written.  Tensors settled by one workgroup, by the listing launch alone, and by a cut behind it.  Bit-exact against the
+oracle."""
+import numpy as np
+import pytest
+
+from test_gpu_gd import Gd, _check_encode
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gd(capi):
+    return Gd(capi)
+
+
+def _background(rng, n, crowd, groups):
+    """Small values everywhere and, in every `groups`-th run of 1024, `crowd` large ones."""
+    g = rng.uniform(-1e-3, 1e-3, n).astype(np.float32)
+    for start in range(0, n - 1024, 1024 * groups):
+        at = start + rng.choice(1024, crowd, replace=False)
+        g[at] = rng.choice([-1, 1], crowd) * rng.uniform(0.5, 1, crowd).astype(np.float32)
+    return g
+
+
+# 16 places in a list at a kept fraction of one in a thousand
+@pytest.mark.parametrize("crowd", [15, 16, 17, 64, 1024])
+@pytest.mark.parametrize("n,rate", [(500_000, 0.05), (1_048_576, 0.01), (3_000_001, 0.02), (17_000_003, 0.002)])
+def test_crowded_lists(gd, oracle_cpu, n, rate, crowd):
+    rng = np.random.default_rng(crowd)
+    g = _background(rng, n, crowd, 16)   # about one element in a thousand at 16 of them
+    r = rng.normal(0, 1e-4, n).astype(np.float32)
+    for seed in (1, 7 << 24):
+        _check_encode(gd, oracle_cpu, g, r.copy(), rate, 0.999, seed)
+
+
+# all large values in one list of a tensor that is otherwise flat
+@pytest.mark.parametrize("n", [1025, 4096, 70_000, 2_600_000])
+def test_one_crowded_list(gd, oracle_cpu, n):
+    rng = np.random.default_rng(n)
+    g = rng.uniform(-1e-3, 1e-3, n).astype(np.float32)
+    g[-900:] = rng.normal(0, 1, 900).astype(np.float32)
+    _check_encode(gd, oracle_cpu, g, np.zeros(n, np.float32), 0.1 if n > 5000 else 1.0, 0.999, 3)
+
+
+# lists are written up to 12 kept in 1024
+@pytest.mark.parametrize("kept", [0.0, 0.0001, 11.9 / 1024, 12.1 / 1024, 0.05])
+@pytest.mark.parametrize("n", [200_000, 900_000])
+def test_kept_fractions(gd, oracle_cpu, n, kept):
+    rng = np.random.default_rng(int(kept * 1e6) + n)
+    g, r = rng.laplace(0, 1e-3, n).astype(np.float32), rng.normal(0, 1e-4, n).astype(np.float32)
+    for seed in (5, 9 << 24):
+        _check_encode(gd, oracle_cpu, g, r.copy(), 0.02, 1 - kept, seed)

@@ -15,18 +15,19 @@
 //               passes over the fp32 bit pattern (11+11+10 bits); no sort
 //   stream      ONE pass over the tensor: r = g + r, store r, compare with the
 //               threshold, wave64 ballot -> one 64-bit word per 64 elements
-//               (bit i = element i), a popcount and the largest |r| per workgroup
+//               (bit i = element i), a popcount and the largest |r| per workgroup, and the
+//               candidates with their values in a short list per wave
 //   finish      tensors that keep up to 2560 entries: one workgroup lists the candidates, cuts
 //               them if they are too many, writes the message and clears the residual
 //   scan        larger tensors of more than 4096 workgroups: exclusive prefix of the
 //               per-workgroup counts within chunks of 4096, the chunks' totals and largest |r|
 //   expand      larger tensors: folds the totals (each workgroup for itself), reports count,
-//               threshold and largest |r| of each tensor to the host; bit words ->
-//               ascending indices at their offsets, values out, residual
-//               entries zeroed, header written
+//               threshold and largest |r| of each tensor to the host; lists (or bit words,
+//               where a list was too short) -> ascending indices at their offsets, values out,
+//               residual entries zeroed, header written
 //
 // The stream pass moves 12 bytes per element (g, r in; r out) plus 1/8 byte of
-// mask; everything else touches O(sample + selected) data.  For tensors
+// mask and 8 bytes per candidate; everything else touches O(sample + selected) data.  For tensors
 // that keep fewer than 8192 entries that is all: their cut is the device's own business.  For the others the host learns the
 // candidate counts from pinned memory while the expand launch is still running
 // (it polls the words the expand launch writes first; no wait for the stream), and only
@@ -82,7 +83,7 @@ __host__ __device__ constexpr uint32_t cdiv(uint64_t a, uint64_t b) { return sta
 
 // Where the pieces of one tensor's workspace block lie (the same arithmetic on the host and in the kernels).
 struct GdLayout {
-  size_t state, hist, samples, hitlist, masks, coarse, cnt, mx, off, ctot, cmax, coff, end;
+  size_t state, hist, samples, hitlist, masks, coarse, cnt, wcnt, mx, off, ctot, cmax, coff, end;
 };
 __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   const size_t ntiles = cdiv(n, kTile);
@@ -95,6 +96,7 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   l.masks = at;   at += align256(sizeof(uint64_t) * ntiles * kWave);      // one bit per element
   l.coarse = at;  at += align256(sizeof(uint64_t) * ntiles);              // one bit per mask word: whether it has a bit set
   l.cnt = at;     at += align256(sizeof(uint32_t) * ntiles);              // candidates per tile
+  l.wcnt = at;    at += align256(sizeof(uint64_t) * ntiles);              // candidates per wave of a tile, 16 bits each
   l.mx = at;      at += align256(sizeof(uint32_t) * ntiles);              // largest |r| per tile, as bits
   l.off = at;     at += align256(sizeof(uint32_t) * ntiles);              // exclusive prefix within the chunk
   l.ctot = at;    at += align256(sizeof(uint32_t) * kMaxChunks);
@@ -102,6 +104,19 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   l.coff = at;    at += align256(sizeof(uint32_t) * kMaxChunks);
   l.end = at;
   return l;
+}
+// Behind that block: the candidates themselves, (index, value) in ascending order, a list per wave of the pass with room
+// for this many (0: no lists, the candidates are looked up through the masks).  Twice the expected number and fourteen: a wave's
+// 1024 elements exceed that next to never unless the large ones crowd together, and then the masks serve.  The pass pays 1 %
+// for them (138 M elements: 229 us, 232 with lists); behind it the expand launch takes 9.0 us instead of 14.4, and the
+// finish 8.8 instead of 11.7 for one tensor of a million, 16.2 instead of 24.8 for ResNet-50's 161.  Up to 12 in 1024:
+// denser, the lists would be a tenth of the tensor.
+__host__ __device__ inline uint32_t list_room(uint32_t n, uint32_t limit) {
+  const float mean = float(kWaveTile) * float(limit) / float(n);
+  return mean > 12.0f ? 0u : (uint32_t(2.0f * mean) + 21u) & ~7u;
+}
+__host__ __device__ inline size_t list_bytes(uint32_t n, uint32_t limit) {
+  return align256(sizeof(uint64_t) * size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit));
 }
 // The cut path's buffers for up to `pairs` candidates: two copies of keys and indices, and the sort's counts.
 constexpr int kSortThreads = 1024;
@@ -149,6 +164,7 @@ struct GdArgs {
   int32_t margin;               // provisional path: how many times the expected number of entries the provisional
                                 // threshold lets through
   uint32_t gather;              // the pick launch gathers samples of up to this size itself
+  uint32_t listed;              // the tensor's `limit` where the segment's own is set to 0 (a second expand launch), else unused
   int32_t device_cut;           // 1: tensors that keep fewer than kCutKeep entries are cut on the device and report nothing
   int32_t tile_start[CAP + 1];  // exclusive prefix of this launch's workgroups per tensor
   GdSeg seg[CAP];
@@ -156,6 +172,7 @@ struct GdArgs {
 };
 static_assert(sizeof(GdArgs<kCapLarge>) <= 18000, "kernel-argument budget");
 
+__device__ __forceinline__ uint2* seg_list(const GdSeg& sg, const GdLayout& l) { return reinterpret_cast<uint2*>(sg.ws + l.end); }
 __device__ __forceinline__ GdState* seg_state(const GdSeg& sg) { return reinterpret_cast<GdState*>(sg.ws); }
 
 // Rank search in a descending cumulative histogram: returns the bin holding
@@ -770,7 +787,18 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t base = t * uint32_t(kTile);
   const uint32_t wbase = base + wave * uint32_t(kWaveTile);
+  // The wave's candidates are also listed as they are found, values and all: the launches behind the pass would otherwise
+  // fetch a line of r for each (see list_room).
+  const uint32_t room = a.margin < 0 ? list_room(n, sg.limit) : 0u;
+  uint2* __restrict__ list = seg_list(sg, l) + (size_t(t) * (kThreads / kWave) + wave) * room;
   uint32_t lo = 0, hi = 0, cnt = 0;
+  auto note = [&](uint64_t m, uint32_t e, float x) {  // m: the wave's candidates of 64 elements, uniform
+    if (m != 0) {
+      const uint32_t at = cnt + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+      if ((m >> lane & 1ull) && at < room) list[at] = make_uint2(e, __float_as_uint(x));
+    }
+    cnt += uint32_t(__popcll(m));
+  };
   float big = 0.0f;  // largest |x| this lane has seen
   float gv[kPerLane], rv[kPerLane];
   if (n - base >= uint32_t(kTile)) {
@@ -784,7 +812,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
       const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];  // thrust::plus<float>()(G, R), gd_body.h:121-128
       if (RESIDUAL) __builtin_nontemporal_store(x, r + size_t(wbase) + c * kWave + lane);
       const uint64_t m = __ballot((x > thr) || (x < nthr));  // gd_body.h:59-67
-      cnt += __popcll(m);
+      note(m, wbase + c * kWave + lane, x);
       big = __builtin_fmaxf(big, __builtin_fabsf(x));
       lo = lane == uint32_t(c) ? uint32_t(m) : lo;  // lane c keeps mask word c
       hi = lane == uint32_t(c) ? uint32_t(m >> 32) : hi;
@@ -802,14 +830,14 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
     for (int c = 0; c < kPerLane; c++) {
       const uint32_t e = wbase + c * kWave + lane;
       bool p = false;
+      const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];
       if (e < n) {
-        const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];
         if (RESIDUAL) r[e] = x;
         p = (x > thr) || (x < nthr);
         big = __builtin_fmaxf(big, __builtin_fabsf(x));
       }
       const uint64_t m = __ballot(p);
-      cnt += __popcll(m);
+      note(m, e, x);
       lo = lane == uint32_t(c) ? uint32_t(m) : lo;  // lane c keeps mask word c
       hi = lane == uint32_t(c) ? uint32_t(m >> 32) : hi;
     }
@@ -825,6 +853,8 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   __syncthreads();
   if (threadIdx.x == 0) {
     reinterpret_cast<uint32_t*>(sg.ws + l.cnt)[t] = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+    reinterpret_cast<uint64_t*>(sg.ws + l.wcnt)[t] =
+        uint64_t(s_cnt[0]) | (uint64_t(s_cnt[1]) << 16) | (uint64_t(s_cnt[2]) << 32) | (uint64_t(s_cnt[3]) << 48);
     reinterpret_cast<uint64_t*>(sg.ws + l.coarse)[t] =
         uint64_t(s_any[0]) | (uint64_t(s_any[1]) << 16) | (uint64_t(s_any[2]) << 32) | (uint64_t(s_any[3]) << 48);
     const uint32_t m01 = s_big[0] > s_big[1] ? s_big[0] : s_big[1], m23 = s_big[2] > s_big[3] ? s_big[2] : s_big[3];
@@ -928,10 +958,21 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t tile0 = (uint32_t(blk - a.tile_start[s]) * (kThreads / kWave) + wave) * kExpandTiles;
 
-  // the masks of this wave's tiles: requested first, used last
-  uint64_t m[kExpandTiles];
+  // The lists of this wave's tiles, four lanes to each: their first entries, whether there are as many or not, and their
+  // lengths, all requested first.
+  constexpr uint32_t kLists = kExpandTiles * (kThreads / kWave), kPer = kWave / kLists, kAhead = 2;
+  static_assert(kLists * kPer == kWave && kAhead * kPer <= 16, "lanes to a list, and entries a list has room for");
+  const uint32_t room = a.margin < 0 ? list_room(sg.n, sg.limit ? sg.limit : a.listed) : 0u;
+  const uint32_t sub = lane % kPer, mine_list = tile0 * (kThreads / kWave) + lane / kPer;
+  const bool my_tile = tile0 + lane / (kPer * (kThreads / kWave)) < ntiles;
+  const uint2* __restrict__ list = seg_list(sg, l) + size_t(mine_list) * room;
+  uint2 first[kAhead];
+  uint32_t listed = 0;
+  if (room != 0 && my_tile) {
+    listed = reinterpret_cast<const uint16_t*>(sg.ws + l.wcnt)[mine_list];
 #pragma unroll
-  for (int j = 0; j < kExpandTiles; j++) m[j] = tile0 + j < ntiles ? masks[size_t(tile0 + j) * kWave + lane] : 0ull;
+    for (uint32_t q = 0; q < kAhead; q++) first[q] = list[q * kPer + sub];
+  }
 
   __shared__ uint32_t s_sum[3][kThreads / kWave];
   uint32_t total, mm = 0;      // the tensor's candidates; its largest |r| (only the wave that reports needs it)
@@ -1041,6 +1082,48 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   if (!cut && tile0 == 0 && lane == 0) *reinterpret_cast<int32_t*>(out) = int32_t(4 + total * 8);
   if (tile0 >= ntiles) return;
 
+  const uint32_t thr_bits = st->thr_bits;
+  int32_t* __restrict__ cand = reinterpret_cast<int32_t*>(sg.cut + cl.ia);
+  uint32_t* __restrict__ keys = reinterpret_cast<uint32_t*>(sg.cut + cl.ka);
+  // For the cut launch the sign travels in the index's top bit: it then never has to read the values again.
+  const uint32_t sign = cut_here ? 0x80000000u : 0u;
+  int32_t* idx = reinterpret_cast<int32_t*>(out + 4);
+  float* val = reinterpret_cast<float*>(out + 4 + size_t(total) * 4);
+  if (room != 0 && __ballot(listed > room) == 0) {
+    // All of the wave's candidates are in its lists: the tiles follow each other, so one prefix over the lists' lengths is
+    // every list's place.
+    const uint32_t own = sub == 0 ? listed : 0u;
+    uint32_t incl = own;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t v = __shfl_up(incl, o, kWave);
+      if (lane >= uint32_t(o)) incl += v;
+    }
+    const uint32_t chunk = tile0 / kScanChunk;
+    static_assert(kScanChunk % kExpandTiles == 0, "a wave's tiles are of one chunk");
+    const uint32_t start = scanned ? __shfl((chunk & 1u) ? ex1 : ex0, int(chunk >> 1), kWave) + tile_off[tile0]
+                                   : uint32_t(__builtin_amdgcn_readlane(own_off, 0));
+    const uint32_t at = start + __shfl(incl - own, int(lane - sub), kWave);
+    auto put = [&](uint32_t place, uint2 p) {
+      if (cut) {
+        cand[place] = int32_t(p.x | (p.y & sign));
+        keys[place] = (p.y & 0x7FFFFFFFu) - thr_bits;
+      } else {
+        idx[place] = int32_t(p.x);
+        val[place] = __uint_as_float(p.y);
+        r[p.x] = 0.0f;
+      }
+    };
+#pragma unroll
+    for (uint32_t q = 0; q < kAhead; q++)
+      if (q * kPer + sub < listed) put(at + q * kPer + sub, first[q]);
+    for (uint32_t j = kAhead * kPer + sub; j < listed; j += kPer) put(at + j, list[j]);
+    return;
+  }
+  // Through the masks.
+  uint64_t m[kExpandTiles];
+#pragma unroll
+  for (int j = 0; j < kExpandTiles; j++) m[j] = tile0 + j < ntiles ? masks[size_t(tile0 + j) * kWave + lane] : 0ull;
   // first place of every tile's candidates, then of this lane's within the tile
   uint32_t pos[kExpandTiles];
 #pragma unroll
@@ -1067,11 +1150,6 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     v1[j] = m[j] ? r[e1[j]] : 0.0f;
   }
   if (cut) {
-    int32_t* __restrict__ cand = reinterpret_cast<int32_t*>(sg.cut + cl.ia);
-    uint32_t* __restrict__ keys = reinterpret_cast<uint32_t*>(sg.cut + cl.ka);
-    const uint32_t thr_bits = st->thr_bits;
-    // For the cut launch the sign travels in the index's top bit: it then never has to read the values again.
-    const uint32_t sign = cut_here ? 0x80000000u : 0u;
     // Sort key: distance of |r| above the threshold in fp32 bit patterns (same order as |r|;
     // the high digits of such keys are mostly zero, which lets the sort skip its last passes).
 #pragma unroll
@@ -1094,8 +1172,6 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     }
     return;
   }
-  int32_t* idx = reinterpret_cast<int32_t*>(out + 4);
-  float* val = reinterpret_cast<float*>(out + 4 + size_t(total) * 4);
 #pragma unroll
   for (int j = 0; j < kExpandTiles; j++) {
     if (m[j]) {
@@ -1733,8 +1809,8 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // (as many as give every lane something to do), a lane after a run of the tile's mask words, of which the tile's coarse
 // word names the few that have a bit set; lanes in order, so one prefix over the workgroup's counts puts the indices
 // in ascending order in LDS.
-// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 6.5-16 us, 10.8 on average;
-// ResNet-50's 161 tensors 58 -> 23 us, 16-36.
+// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 8.8 us on average;
+// ResNet-50's 161 tensors 58 -> 16 us.
 // Larger ones that still fit are only cut here, behind the expand launch.  All of it is queued before the host knows any
 // count.
 constexpr uint32_t kFinishKeep = 2560;
@@ -1797,6 +1873,73 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
   const uint32_t ntiles = cdiv(sg.n, kTile);
   float* __restrict__ r = sg.r;
 
+  // The pass's own lists, a few of them to a lane: where each entry of the tensor's list of candidates lies, and then the
+  // entries, each a load that depends on nothing but its place.  (Through the masks every candidate is a word of the mask and
+  // then a line of r.)
+  const uint32_t room = list_room(sg.n, keep);
+  const uint2* __restrict__ list = seg_list(sg, l);
+  bool lists = false;
+  uint32_t n = 0, pos = 0;
+  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
+  if (room != 0) {
+    constexpr uint32_t kAtOnce = 4;
+    const uint32_t nlists = ntiles * (kThreads / kWave), per = cdiv(nlists, kSortThreads), first = t * per;
+    const uint16_t* __restrict__ lengths = reinterpret_cast<const uint16_t*>(sg.ws + l.wcnt);
+    uint32_t c[kAtOnce], mine = 0;
+    bool over = false;
+    auto take = [&](uint32_t q0) {
+#pragma unroll
+      for (uint32_t q = 0; q < kAtOnce; q++) c[q] = q0 + q < per && first + q0 + q < nlists ? lengths[first + q0 + q] : 0u;
+    };
+    for (uint32_t q0 = 0; q0 < per; q0 += kAtOnce) {
+      take(q0);
+#pragma unroll
+      for (uint32_t q = 0; q < kAtOnce; q++) { mine += c[q]; over = over || c[q] > room; }
+    }
+    pos = block_prefix(mine, s_wave, n);
+    lists = !__syncthreads_or(over || n > kCutKeep);
+    if (lists) {
+      for (uint32_t q0 = 0; q0 < per; q0 += kAtOnce) {
+        if (per > kAtOnce) take(q0);
+#pragma unroll
+        for (uint32_t q = 0; q < kAtOnce; q++)
+          for (uint32_t j = 0; j < c[q]; j++) s_id[pos++] = (first + q0 + q) * room + j;
+      }
+      if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + (n > keep ? keep : n) * 8);
+      if (n == 0 || keep == 0) return;
+      __syncthreads();
+      if (n <= keep) {   // gd_body.h:193-229
+        int32_t* __restrict__ idx = reinterpret_cast<int32_t*>(sg.out + 4);
+        uint32_t* __restrict__ val = reinterpret_cast<uint32_t*>(sg.out + 4 + size_t(n) * 4);
+        for (uint32_t x0 = t; x0 < n; x0 += 3 * kSortThreads) {   // three in flight per lane
+          uint2 e[3];
+#pragma unroll
+          for (uint32_t j = 0; j < 3; j++) e[j] = list[s_id[x0 + j * kSortThreads < n ? x0 + j * kSortThreads : x0]];
+#pragma unroll
+          for (uint32_t j = 0; j < 3; j++) {
+            const uint32_t x = x0 + j * kSortThreads;
+            if (x < n) {
+              idx[x] = int32_t(e[j].x);
+              val[x] = e[j].y;
+              r[e[j].x] = 0.0f;
+            }
+          }
+        }
+        return;
+      }
+      const CutArgs f{s_stage, s_bins, s_wave, r, sg.out, n, keep, thr_bits};
+      auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
+        const uint2 e = list[s_id[x]];
+        key = (e.y & 0x7FFFFFFFu) - thr_bits;
+        id = e.x | (e.y & 0x80000000u);
+      };
+      const bool done = n <= kSortThreads ? cut_loaded<1>(f, pair) : n <= 3 * kSortThreads ? cut_loaded<3>(f, pair) : cut_loaded<8>(f, pair);
+      if (!done) cut_crowded(f);
+      return;
+    }
+    __syncthreads();
+  }
+
   // lanes per tile (a power of two, at most one per mask word), or tiles per lane
   int group = 0;   // log2
   while (group < 6 && (ntiles << (group + 1)) <= uint32_t(kSortThreads)) group++;
@@ -1817,7 +1960,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
   uint64_t c0 = tile0 < ntiles ? coarse[tile0] & range : 0ull, m0[4];
   uint32_t e0[4];
   four(tile0, c0, e0, m0);
-  uint32_t mine = 0, n;
+  uint32_t mine = 0;
   if (group == 0) {   // whole tiles: the pass has left their counts
     for (uint32_t q = 0; q < per_lane && tile0 + q < ntiles; q++) mine += reinterpret_cast<const uint32_t*>(sg.ws + l.cnt)[tile0 + q];
   } else {
@@ -1825,8 +1968,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
     for (int k = 0; k < 4; k++) mine += uint32_t(__popcll(m0[k]));
     for (uint64_t c = c0; c; c &= c - 1) mine += uint32_t(__popcll(masks[size_t(tile0) * kWave + uint32_t(__builtin_ctzll(c))]));
   }
-  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
-  uint32_t pos = block_prefix(mine, s_wave, n);
+  pos = block_prefix(mine, s_wave, n);
   const bool cut = n > keep;
   if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + (cut ? keep : n) * 8);
   if (n == 0 || keep == 0) return;
@@ -2069,6 +2211,7 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   a.margin = margin;
   a.gather = 0;
   a.device_cut = margin < 0 ? 1 : 0;
+  a.listed = 0;
   a.report = report;
   for (int i = 0; i < count; i++) a.seg[i] = plans[i].seg;
   auto tiles = [&](auto per_tensor) {
@@ -2235,7 +2378,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
     p.seg.thr_index = static_cast<uint32_t>(thr_index);
     p.seg.limit = static_cast<uint32_t>(expected);
     p.seg.cap = static_cast<uint32_t>(cap64);
-    p.ws_bytes = gd_layout(n, p.seg.sample_cnt).end;
+    p.ws_bytes = gd_layout(n, p.seg.sample_cnt).end + list_bytes(n, p.seg.limit);
     p.cut_bytes = cut_layout(cap64).end;
     p.index = i;
     ws_total += p.ws_bytes + p.cut_bytes;
@@ -2364,6 +2507,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         a.margin = -1;
         a.gather = 0;
         a.device_cut = 0;
+        a.listed = margin < 0 ? plan.seg.limit : plan.seg.n;   // the provisional path leaves no lists: no room for any
         a.report = nullptr;  // the host has its report
         a.seg[0] = plan.seg;
         a.seg[0].cut = cut;
