@@ -55,7 +55,7 @@ def test_widths_around_the_strips(psgd, m):
     _phases(psgd, [(n, m, min(2, m)) for n in (8201, 129)], m + 1)
 
 
-@pytest.mark.parametrize("n", [31, 32, 33, 255, 256, 257, 1055, 2081])
+@pytest.mark.parametrize("n", [31, 32, 33, 127, 128, 191, 192, 193, 255, 256, 257, 1055, 2081])
 def test_heights_around_the_blocks_of_rows(psgd, n):
     # blocks of 32, 64 and 128 rows dealt out to the partials of a strip, the last one not whole
     _phases(psgd, [(n, m, min(4, n)) for m in (1024, 384, 192, 70)], n)

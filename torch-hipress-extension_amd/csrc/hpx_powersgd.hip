@@ -554,9 +554,10 @@ __global__ __launch_bounds__(kOrthThreads) void psgd_orth_kernel(const Args<CAP>
 // is the A operand of MFMA t, whose block b / row-of-block i' is column
 // k0 + 16b + 4i' + t; the B operand is P[row][j] in every block.  The waves (and the rows side by side) meet
 // in LDS and the workgroup writes one partial of Q; a second kernel adds the
-// partials in a fixed order.
+// partials in a fixed order.  (Ranks up to four are held to the registers of four waves per SIMD: ResNet-50's matrices 149.7 us
+// for all three phases, 151.4 with three.)
 template <int CG, int CAP>
-__global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
+__global__ __launch_bounds__(kThreads, CG == 1 ? 4 : 1) void psgd_mtp_kernel(const Args<CAP> a) {
   const int tile = blockIdx.x;
   const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
   const Seg& sg = a.seg[s];
@@ -581,7 +582,25 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
 
   const int j = lane & 3;
   const int mine = lane / lanes;  // which of the rows side by side
-  constexpr int kRows = 8, kTail = 4;
+  constexpr int kRows = 8;
+  // K rounds' rows, summed on their own in two chains and added to what there is
+  auto add_up = [&](const auto& m4, const auto& p) {
+    constexpr int K = sizeof(m4) / sizeof(m4[0]);
+#pragma unroll
+    for (int c = 0; c < CG; c++) {
+      f32x4 sum[2][4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) sum[0][t] = sum[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < K; u++) {
+        const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
+#pragma unroll
+        for (int t = 0; t < 4; t++) sum[u & 1][t] = mfma4(v[t], p[u][c], sum[u & 1][t]);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; t++) acc[c][t] += sum[0][t] + sum[1][t];
+    }
+  };
   const int64_t block = kRows * step;
   int64_t row0 = rblk * block + wave * side;  // the first of the wave's rows in a round
   // Main loop: a block at a time, every load issued before the first use, summed on their own in two chains and added to
@@ -606,29 +625,16 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
     for (int u = 0; u < kRows; u++)
 #pragma unroll
       for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[(row0 + u * step + mine) * ld + c * 4 + j] : 0.f;
-#pragma unroll
-    for (int c = 0; c < CG; c++) {
-      f32x4 sum[2][4];
-#pragma unroll
-      for (int t = 0; t < 4; t++) sum[0][t] = sum[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int u = 0; u < kRows; u++) {
-        const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
-#pragma unroll
-        for (int t = 0; t < 4; t++) sum[u & 1][t] = mfma4(v[t], p[u][c], sum[u & 1][t]);
-      }
-#pragma unroll
-      for (int t = 0; t < 4; t++) acc[c][t] += sum[0][t] + sum[1][t];
-    }
+    add_up(m4, p);
   }
-  // The matrix's last block, where this wave's rows of it are not whole: kTail rounds' loads in flight together (one round
+  // The matrix's last block, where this wave's rows of it are not whole: all their loads in flight together (one round
   // after the other 12 of 1200 x 601 took 59.2 us for all three phases, 30 of 150 x 220 31.5; now 58.0 and 30.2).
   const int64_t after = row0 - wave * side + block;
-  for (const int64_t rend = after < n ? after : n; row0 < rend; row0 += kTail * step) {
-    float4 m4[kTail];
-    float p[kTail][CG];
+  for (const int64_t rend = after < n ? after : n; row0 < rend; row0 += kRows * step) {
+    float4 m4[kRows];
+    float p[kRows][CG];
 #pragma unroll
-    for (int u = 0; u < kTail; u++) {
+    for (int u = 0; u < kRows; u++) {
       const int64_t row = row0 + u * step + mine;
       const float* q = M + row * m + kk;
       m4[u] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -639,14 +645,7 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
 #pragma unroll
       for (int c = 0; c < CG; c++) p[u][c] = row < n && c * 4 + j < r ? P[row * ld + c * 4 + j] : 0.f;
     }
-#pragma unroll
-    for (int u = 0; u < kTail; u++) {
-      const float v[4] = {m4[u].x, m4[u].y, m4[u].z, m4[u].w};
-#pragma unroll
-      for (int c = 0; c < CG; c++)
-#pragma unroll
-        for (int t = 0; t < 4; t++) acc[c][t] = mfma4(v[t], p[u][c], acc[c][t]);
-    }
+    add_up(m4, p);
   }
   // acc[c][t][i'] in lane 4b+j  ->  Q[k0 + (16b + 4i' + t) % width][4c + j], part (16b + 4i' + t) / width of the wave
   __shared__ float s_q[kWaves][CG][4 * kWave][4];
@@ -665,12 +664,13 @@ __global__ __launch_bounds__(kThreads) void psgd_mtp_kernel(const Args<CAP> a) {
     const int c = e / (width * 4), kl = (e / 4) & (width - 1), jj = e & 3;
     const int k = k0 + kl, col = c * 4 + jj;
     if (k < m && col < r) {
-      float x = 0.f;
       static_assert(kWaves == 4, "summed in pairs");
-      for (int h = 0; h < side; h++) {
+      auto rows_beside = [&](int h) {
         const int l = h * width + kl;
-        x += (s_q[0][c][l][jj] + s_q[1][c][l][jj]) + (s_q[2][c][l][jj] + s_q[3][c][l][jj]);
-      }
+        return (s_q[0][c][l][jj] + s_q[1][c][l][jj]) + (s_q[2][c][l][jj] + s_q[3][c][l][jj]);
+      };
+      const float x = side == 1 ? rows_beside(0) : side == 2 ? rows_beside(0) + rows_beside(1)
+                                                             : (rows_beside(0) + rows_beside(1)) + (rows_beside(2) + rows_beside(3));
       part[int64_t(k) * stride + col] = x;
     }
   }
@@ -890,8 +890,14 @@ int orth_launch(const Args<CAP>& a, size_t lds, hipStream_t st) {
   return HPX_OK;
 }
 
+// A matrix of up to kQWholeRows rows takes the product in one partial, which is Q itself, by the narrowest strips: a call of such
+// matrices needs no launch to add partials up.  us of a pass: 128 x 128 22.2 -> 18.5, 30 of up to 150 x 220 36 -> 27, 10 of up to
+// 64 x 2000 32 -> 28; among taller matrices, where the launch is there anyway, 30 of up to 250 x 1220 56.4 -> 57.4, and at 256 rows
+// 10 of up to 512 x 512 37.4 -> 39.7.
+constexpr int kQWholeRows = 192;
+inline int q_lanes(int n, int m) { return n <= kQWholeRows ? 16 : strip_lanes(m); }
 // Partials of a matrix: of `rows` rows each, as many times more as strips side by side in a wave.
-inline int32_t q_parts(int n, int m, int rows) { return cdiv(n, int64_t(rows) * (kWave / strip_lanes(m))); }
+inline int32_t q_parts(int n, int m, int rows) { return cdiv(n, int64_t(rows) * (kWave / q_lanes(n, m))); }
 
 // Rows per partial: as many as leave the matrix kQTiles workgroups, since every partial is written and read back; 64 at
 // least, or 32 where 64 would leave fewer than kQTilesSmall.  Like split_rows by the matrix alone: Q is the sum of the
@@ -904,7 +910,9 @@ constexpr int kQRowsMin = 32, kQRowsMax = 512;
 // layer set, which twelve such matrices are part of, pays 4 of 1565 for their partials, and 8 if all 36 have as many.
 constexpr int64_t kQTiles = 128, kQTilesSmall = 32, kQTilesLarge = 256;
 inline int q_rows(int n, int m) {
-  auto tiles = [=](int rows) { return int64_t(cdiv(m, 4 * strip_lanes(m))) * q_parts(n, m, rows); };
+  static_assert(kQWholeRows <= 2 * kQRowsMin * (kWave / 16), "rows of one partial of the narrowest strips");
+  if (n <= kQWholeRows) return 2 * kQRowsMin;
+  auto tiles = [=](int rows) { return int64_t(cdiv(m, 4 * q_lanes(n, m))) * q_parts(n, m, rows); };
   int rows = kQRowsMax;
   const int64_t enough = int64_t(n) * m >= (1 << 24) ? kQTilesLarge : kQTiles;
   while (rows > 2 * kQRowsMin && tiles(rows) < enough) rows /= 2;
@@ -946,7 +954,7 @@ int encode2_launches(int count, int max_rank, float* partials, float* const* Ps,
       while (i < count && a.nseg < CAP) {
         const int rb = block_cols(rs[i], c0);
         if (rb == 0) { i++; continue; }
-        const int lanes = strip_lanes(ms[i]);
+        const int lanes = q_lanes(ns[i], ms[i]);
         const int rows = q_rows(ns[i], ms[i]);
         const int32_t parts = q_parts(ns[i], ms[i], rows);
         const int64_t t = int64_t(cdiv(ms[i], 4 * lanes)) * parts;
