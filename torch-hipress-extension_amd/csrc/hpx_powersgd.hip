@@ -372,38 +372,30 @@ __device__ __forceinline__ void gram_schmidt(const PView<LDS> P, double* s_red) 
   }
 }
 
-// Sums of v[0 ... V-1] over the lanes of a wave, V a power of two up to 64: at every step a lane hands on the half of
-// its values that the lanes on the other side look after, so the wave exchanges about V values in all instead of 6 V.
-// Returns the sum of v[fold_index<V>(lane)].
-template <int V, int O = kWave / 2>
-__device__ __forceinline__ double wave_fold(const double (&v)[V], int lane) {
-  if constexpr (V > 1) {
-    const bool up = (lane & O) != 0;
-    double h[V / 2];
-#pragma unroll
-    for (int k = 0; k < V / 2; k++) {
-      const double send = up ? v[k] : v[k + V / 2], keep = up ? v[k + V / 2] : v[k];
-      h[k] = keep + __shfl_xor(send, O, kWave);
-    }
-    return wave_fold<V / 2, O / 2>(h, lane);
-  } else {
-    double x = v[0];
-#pragma unroll
-    for (int o = O; o >= 1; o /= 2) x += __shfl_xor(x, o, kWave);
-    return x;
-  }
-}
-template <int V>
-__device__ __forceinline__ int fold_index(int lane) { return lane / (kWave / V); }
-
+// Row `row` of a factor of r columns, r <= C; zeros behind them and for rows past the end.
 template <int C>
 __device__ __forceinline__ void load_row(float (&x)[C], const float* P, int64_t row, int n, int r) {
-  if (C == 4 && r == 4) {
-    const float4 v = row < n ? ld4(P + row * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
-    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+  if (r == C) {
+#pragma unroll
+    for (int c = 0; c < C; c += 4) {
+      const float4 v = row < n ? ld4(P + row * C + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+      x[c] = v.x; x[c + 1] = v.y; x[c + 2] = v.z; x[c + 3] = v.w;
+    }
   } else {
 #pragma unroll
     for (int c = 0; c < C; c++) x[c] = c < r && row < n ? P[row * r + c] : 0.f;
+  }
+}
+template <int C>
+__device__ __forceinline__ void store_row(const float (&y)[C], float* P, int64_t row, int n, int r) {
+  if (row >= n) return;
+  if (r == C) {
+#pragma unroll
+    for (int c = 0; c < C; c += 4) st4(P + row * C + c, make_float4(y[c], y[c + 1], y[c + 2], y[c + 3]));
+  } else {
+#pragma unroll
+    for (int c = 0; c < C; c++)
+      if (c < r) P[row * r + c] = y[c];
   }
 }
 
@@ -411,65 +403,97 @@ __device__ __forceinline__ void load_row(float (&x)[C], const float* P, int64_t 
 // there), G = R^T R, P <- P R^-1 in fp64 with one rounding to fp32 at the end: one pass over P for the sums and one for
 // the result.  What the sums, the elimination and the product round away is at most k 2^-53 sqrt(G_ii G_jj) in the entries
 // of G and comes out multiplied by R^-1 from both sides: with s_c = sum over l of |R^-1_lc| sqrt(G_ll) the columns are
-// orthonormal to k 2^-53 s_c^2, k the length of the longest chain of sums (the n / 1024 rows of a lane, the fold over lanes
-// and waves, the elimination: 32 for all but the first).  s_c is about 1 for columns that have little to do with each other
+// orthonormal to k 2^-53 s_c^2, k the length of the longest chain of sums (the n / 256 rows of one accumulator, the fold over
+// accumulators, blocks and waves, the elimination: 36 for all but the first).  s_c is about 1 for columns that have little to do with each other
 // and grows with the product of what the columns before lose to each other, not only with each one's own loss: a chain
 // c_1 = u_1, c_k+1 = u_k + 0.05 u_k+1 of eight columns keeps every R_cc^2 above 2^-10 G_cc, and its P R^-1 is no
 // orthonormal matrix at all.  Where k s_c^2 exceeds 2^27 (2^-26 in the products of columns, a quarter of fp32's own rounding), or is no number,
 // nothing is written and the answer is false.  A column of zeros stays zero.
-// us for 36 factors of 4096 or 1024 rows and 4 columns: 38 with Gram-Schmidt, now 12; 54 factors of 64 ... 2048 rows
-// and 2 columns: 2 x 10.7, now 7.3.
+// The sums ride on v_mfma_f64_4x4x4_4b_f64, four blocks of 4 x 4 products summed over four rows each: A[blk][i][k] and
+// B[blk][k][i] are lane 16k + 4blk + i alike, so one register of sixteen rows by four columns is both operands, and D[blk][i][j]
+// (lane 16i + 4blk + j) is left to be added up over the blocks alone.  (As fp64 products in every lane the sums had to be
+// folded over 64 lanes, ten or 36 of them: for eight columns that was most of the launch.)
+// us of the launch, folded over the lanes / so: 36 factors of up to 2048 x 8 24 / 8, one of 4096 x 8 35 / 11; of 4 columns 10.5 /
+// 9.6 for one of 4096 (Gram-Schmidt: 38 for 36 of them), 11.1 / 12.9 for the 36 of the layer set; 512 x 512 of rank 4, all three
+// phases, 26.9 / 25.9.
 template <int C>
 __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
+  constexpr int H = C / 4, kBlocks = H * (H + 1) / 2;   // 4 x 4 blocks of the Gram matrix: (0, 0), and (0, 1), (1, 1)
   constexpr int kPairs = C * (C + 1) / 2;
-  constexpr int V = C <= 4 ? 16 : 64;
-  static_assert(kPairs <= V && C <= kGramCols, "pairs of columns");
-  __shared__ double s_part[kOrthWaves][V];
-  __shared__ double s_gram[V];
+  static_assert(C % 4 == 0 && C <= kGramCols, "columns in fours");
+  __shared__ double s_part[kOrthWaves][kBlocks][16];
+  __shared__ double s_gram[C][C];
   __shared__ double s_T[C][C];
   __shared__ double s_norm[C];
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  double g[V];
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  constexpr int kAcc = 4;              // independent sums
+  constexpr int kGroups = 16 / H;      // of sixteen rows, loaded together; the groups go round the waves
+  double acc[kBlocks][kAcc];
 #pragma unroll
-  for (int k = 0; k < V; k++) g[k] = 0;
-  constexpr int kRows = 16 / C;  // loaded together: one row at a time the loop is a chain of memory latencies
-  for (int64_t row0 = threadIdx.x; row0 < n; row0 += kRows * kOrthThreads) {
-    float x[kRows][C];
+  for (int k = 0; k < kBlocks; k++)
 #pragma unroll
-    for (int u = 0; u < kRows; u++) load_row<C>(x[u], P, row0 + u * kOrthThreads, n, r);
+    for (int u = 0; u < kAcc; u++) acc[k][u] = 0;
+  const int col = lane & 3;
+  for (int64_t row0 = int64_t(wave) * 16; row0 < n; row0 += kGroups * kOrthWaves * 16) {
+    float x[kGroups][H];
 #pragma unroll
-    for (int u = 0; u < kRows; u++)
+    for (int u = 0; u < kGroups; u++) {
+      const int64_t row = row0 + u * (kOrthWaves * 16) + lane / 4;
+      const float* at = P + (row < n ? row : n - 1) * r;   // (no branch between the loads)
 #pragma unroll
-      for (int c = 0; c < C; c++)
+      for (int h = 0; h < H; h++) x[u][h] = at[4 * h + col < r ? 4 * h + col : 0];
+    }
 #pragma unroll
-        for (int d = 0; d <= c; d++) g[c * (c + 1) / 2 + d] = fma(double(x[u][c]), double(x[u][d]), g[c * (c + 1) / 2 + d]);
+    for (int u = 0; u < kGroups; u++)
+#pragma unroll
+      for (int h = 0; h < H; h++)
+        x[u][h] = row0 + u * (kOrthWaves * 16) + lane / 4 < n && 4 * h + col < r ? x[u][h] : 0.f;
+#pragma unroll
+    for (int u = 0; u < kGroups; u++) {
+      if (row0 + u * (kOrthWaves * 16) >= n) break;   // wave-uniform
+      acc[0][u % kAcc] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[u][0], x[u][0], acc[0][u % kAcc], 0, 0, 0);
+      if constexpr (H == 2) {
+        acc[1][u % kAcc] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[u][0], x[u][1], acc[1][u % kAcc], 0, 0, 0);
+        acc[2][u % kAcc] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[u][1], x[u][1], acc[2][u % kAcc], 0, 0, 0);
+      }
+    }
   }
-  const int busy = n < kOrthThreads ? (n + kWave - 1) / kWave : kOrthWaves;  // waves that have a row
-  if (wave < busy) {
-    const double sum = wave_fold<V>(g, lane);
-    if (lane % (kWave / V) == 0) s_part[wave][fold_index<V>(lane)] = sum;
+#pragma unroll
+  for (int k = 0; k < kBlocks; k++) {
+    double x = (acc[k][0] + acc[k][1]) + (acc[k][2] + acc[k][3]);
+    x += __shfl_xor(x, 4, kWave);
+    x += __shfl_xor(x, 8, kWave);
+    if ((lane & 12) == 0) s_part[wave][k][lane / 16 * 4 + col] = x;   // [i][j]
   }
   __syncthreads();
-  if (threadIdx.x < V) {
-    double x = 0;
-    for (int w = 0; w < busy; w++) x += s_part[w][threadIdx.x];
-    s_gram[threadIdx.x] = x;
+  if (threadIdx.x < kBlocks * 16) {
+    const int k = threadIdx.x / 16, i = threadIdx.x / 4 % 4, j = threadIdx.x % 4;
+    double x[kOrthWaves];
+#pragma unroll
+    for (int w = 0; w < kOrthWaves; w++) x[w] = s_part[w][k][threadIdx.x % 16];
+#pragma unroll
+    for (int o = kOrthWaves / 2; o > 0; o /= 2)
+#pragma unroll
+      for (int w = 0; w < o; w++) x[w] += x[w + o];
+    const int gi = i + (k == 2 ? 4 : 0), gj = j + (k != 0 ? 4 : 0);
+    s_gram[gi][gj] = x[0];
+    s_gram[gj][gi] = x[0];
   }
   __syncthreads();
   // Cholesky's factor of G and the inverse of it by elimination on [G | I], lane j of the first wave with column j of both
   // halves.  Row k of the left half ends as R's, column l of the right half as R^-1's row l.
   if (wave == 0) {
-    const int col = lane < C ? lane : C - 1;
+    const int own = lane < C ? lane : C - 1;
     double A[C], Y[C];
 #pragma unroll
     for (int k = 0; k < C; k++) {
-      A[k] = s_gram[k >= col ? k * (k + 1) / 2 + col : col * (col + 1) / 2 + k];
-      Y[k] = k == col ? 1.0 : 0.0;
+      A[k] = s_gram[k][own];
+      Y[k] = k == own ? 1.0 : 0.0;
     }
 #pragma unroll
     for (int k = 0; k < C; k++) {
       const double d = __shfl(A[k], k, kWave);
-      const double inv = s_gram[k * (k + 1) / 2 + k] != 0 ? rsqrt(d) : 0;  // of what is not above zero: no number, or infinite
+      const double inv = s_gram[k][k] != 0 ? rsqrt(d) : 0;  // of what is not above zero: no number, or infinite
       A[k] *= inv;
       Y[k] *= inv;
 #pragma unroll
@@ -482,13 +506,13 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
     if (lane < C) {
 #pragma unroll
       for (int k = 0; k < C; k++) s_T[lane][k] = Y[k];
-      s_norm[lane] = sqrt(s_gram[lane * (lane + 1) / 2 + lane]);
+      s_norm[lane] = sqrt(s_gram[lane][lane]);
     }
   }
   __syncthreads();
   double T[kPairs];
   bool ok = true;
-  const double limit = 0x1p27 / (32 + (n - 1) / kOrthThreads + 1);
+  const double limit = 0x1p27 / (36 + (n - 1) / 256 + 1);
 #pragma unroll
   for (int c = 0; c < C; c++) {
     double s = 0;
@@ -500,20 +524,22 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
     ok = ok && s * s <= limit;
   }
   if (!ok) return false;  // the same in every thread
+  constexpr int kRows = 16 / C;  // loaded together
   for (int64_t row0 = threadIdx.x; row0 < n; row0 += kRows * kOrthThreads) {
     float x[kRows][C];
 #pragma unroll
     for (int u = 0; u < kRows; u++) load_row<C>(x[u], P, row0 + u * kOrthThreads, n, r);
 #pragma unroll
     for (int u = 0; u < kRows; u++) {
-      const int64_t row = row0 + u * kOrthThreads;
+      float out[C];
 #pragma unroll
       for (int c = 0; c < C; c++) {
         double y = 0;
 #pragma unroll
         for (int l = 0; l <= c; l++) y = fma(double(x[u][l]), T[c * (c + 1) / 2 + l], y);
-        if (c < r && row < n) P[row * r + c] = float(y);
+        out[c] = float(y);
       }
+      store_row<C>(out, P, row0 + u * kOrthThreads, n, r);
     }
   }
   return true;
