@@ -88,18 +88,19 @@ int hpx_release_stream(hpx_stream_t stream);
  *                             launch of that kind: its head stays on chip,
  *                             the rest is read twice by the same launch;
  *                             0: such tensors take the two-launch encode
- *   "gd_provisional_min_samples" a sparsifier call (hpx_gd_encode,
- *                             hpx_dgc_encode) whose tensors' samples add up to
- *                             at least this many (default -1: none) starts its
- *                             pass over the tensors from a provisional
- *                             threshold taken from the first 16384 samples and
- *                             finds the exact one afterwards among the samples
- *                             the pass marked, instead of gathering the whole
- *                             sample first; the message is the same.  Negative:
- *                             never.  Off by default: measured on a 138 M
- *                             element tensor it is 3 % slower than the gather
- *   "gd_provisional_margin"   how many times the expected number of entries
- *                             the provisional threshold lets through (default
+ *   "gd_provisional_min_samples" which tensors of a sparsifier call
+ *                             (hpx_gd_encode, hpx_dgc_encode) start their pass
+ *                             from a provisional threshold taken from the
+ *                             first samples and find the exact one afterwards
+ *                             among what the pass marked, instead of gathering
+ *                             the whole sample first; the message is the same.
+ *                             -2 (default): large ones with large samples, for
+ *                             which that is quicker (138 M elements: 337 us
+ *                             instead of 377); -1: none; otherwise all of a
+ *                             call whose samples add up to at least this many
+ *   "gd_provisional_margin"   with such a number, how many times the expected
+ *                             number of entries the provisional threshold (of
+ *                             the first 16384 samples) lets through (default
  *                             3).  A tensor whose provisional threshold turns
  *                             out not to lie below the exact one is encoded
  *                             again through the gather path (hpx_gd_fallbacks

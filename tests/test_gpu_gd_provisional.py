@@ -1,0 +1,129 @@
+"""The sparsifier's threshold without the gather of its sample: large tensors start their pass from a provisional threshold,
+and the exact one is found among the candidates, each of which works out how often it was sampled.  Message and updated
+residual are the gather path's bit for bit: at both ends of the sizes, with lists too short for their candidates,
+with equal values on either side of the threshold, zeros, infinities and NaN."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import stream_ptr
+from test_gpu_gd import Gd, _check_encode
+
+pytestmark = pytest.mark.gpu
+
+FIRST = 1 << 24   # elements from which the path is taken, with enough samples
+
+
+@pytest.fixture(scope="module")
+def gd(capi):
+    return Gd(capi)
+
+
+def _values(kind, n, gen):
+    g = torch.empty(n, device="cuda").uniform_(-1, 1, generator=gen)
+    if kind == "crowded":          # lists overflow: half of the large values within one element in a thousand
+        g *= 1e-3
+        g[n // 3:n // 3 + n // 1500] *= 4e3
+    elif kind == "sparse":         # too few non-zeros for a threshold above zero
+        g *= (torch.empty(n, device="cuda").uniform_(0, 1, generator=gen) < 2e-4)
+    elif kind == "coarse":         # many equal values, the provisional threshold among them
+        g = torch.round(g * 8) / 8
+    elif kind == "signs":          # all of one size: nothing lies above the threshold
+        g = torch.sign(g)
+    elif kind == "infinite":
+        g[::5003] = float("inf"); g[::7001] = float("-inf")
+    elif kind == "nan":            # some, so that they move the threshold's rank
+        g[::3001] = float("nan")
+    elif kind == "all_nan":        # the threshold itself is one
+        g[::400] = float("nan")
+    return g
+
+
+def _encode(gd, capi, how, tensors, residuals, rates, drops, seeds):
+    rs = [r.clone() for r in residuals]
+    gs = [g.clone() for g in tensors]
+    outs = [torch.full((4 + 8 * int(np.ceil(g.numel() * (1 - d))) + 64,), 0xEE, dtype=torch.uint8, device="cuda") for g, d in zip(gs, drops)]
+    old = capi.set_option("gd_provisional_min_samples", how)
+    L = capi.load()
+    before = L.hpx_gd_fallbacks(stream_ptr())
+    L.hpx_profile_reset(); L.hpx_profile_enable(1)
+    try:
+        gd.encode(gs, rs, outs, rates, drops, seeds)
+        torch.cuda.synchronize()
+        inverted = capi.profile_query("gd_invert_kernel")[1]
+    finally:
+        L.hpx_profile_enable(0); L.hpx_profile_reset()
+        capi.set_option("gd_provisional_min_samples", old)
+    return outs, rs, inverted, L.hpx_gd_fallbacks(stream_ptr()) - before
+
+
+def _compare(gd, capi, tensors, residuals, rates, drops, seeds, how=-2):
+    a, ra, with_inverse, fell_back = _encode(gd, capi, how, tensors, residuals, rates, drops, seeds)
+    b, rb, without, _ = _encode(gd, capi, -1, tensors, residuals, rates, drops, seeds)
+    assert without == 0
+    for i in range(len(tensors)):
+        size = int(b[i][:4].view(torch.int32)[0])
+        assert 4 <= size <= b[i].numel() - 64
+        assert torch.equal(a[i][:size], b[i][:size]), f"message {i} of {size} bytes"
+        assert (a[i][-64:] == 0xEE).all()
+        assert torch.equal(ra[i].view(torch.int32), rb[i].view(torch.int32)), f"residual {i}"
+    return with_inverse, fell_back
+
+
+@pytest.mark.parametrize("n,rate,kept,path", [(FIRST - 1, 0.05, 1e-3, False), (FIRST, 0.05, 1e-3, True), (FIRST + 4097, 0.04, 2.4e-3, True),
+                                              (FIRST + 1, 1.0, 1e-3, True), (50_000_017, 0.02, 6e-4, True), (100_000_007, 0.01, 1e-3, True),
+                                              (FIRST, 0.05, 2.6e-3, False), (FIRST, 0.05, 4e-4, False), (59_000_000, 0.01, 1e-3, False)])
+def test_sizes(gd, capi, n, rate, kept, path):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    g, r = (torch.empty(n, device="cuda").normal_(0, s, generator=gen) for s in (1e-3, 1e-4))
+    for seed in (3, (5 << 32) + 0xFFFFFF00):
+        inverted, fell_back = _compare(gd, capi, [g], [r], [rate], [1 - kept], [seed])
+        assert (inverted, fell_back) == (int(path), 0)
+
+
+@pytest.mark.parametrize("kind,fallback", [("crowded", 0), ("sparse", 0), ("coarse", 1), ("signs", 1), ("infinite", 0), ("nan", None), ("all_nan", None)])
+def test_values(gd, capi, kind, fallback):
+    n = 20_000_003
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    g, r = _values(kind, n, gen), torch.zeros(n, device="cuda")
+    inverted, fell_back = _compare(gd, capi, [g], [r], [0.05], [0.999], [11])
+    assert inverted == 1 and (fallback is None or fell_back == fallback)
+
+
+def test_beside_others(gd, capi):
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    sizes = [1000, 17_000_000, 400_000, 18_000_001, 5_000_000, FIRST - 1]
+    gs = [torch.empty(n, device="cuda").normal_(0, 1e-3, generator=gen) for n in sizes]
+    rs = [torch.empty(n, device="cuda").normal_(0, 1e-4, generator=gen) for n in sizes]
+    k = len(sizes)
+    for how in (-2, 0):   # by size; all of them, some too small to work out their samples
+        inverted, _ = _compare(gd, capi, gs, rs, [0.04] * k, [0.999] * k, list(range(k)), how)
+        assert inverted == 1
+
+
+def test_without_a_residual(capi):
+    c, L, n, rate, kept = capi, capi.load(), FIRST + 3, 0.06, 1e-3
+    g = torch.empty(n, device="cuda").normal_(0, 1e-3, generator=torch.Generator(device="cuda").manual_seed(4))
+    got = []
+    for how in (-2, -1):
+        d, out = g.clone(), torch.zeros(4 + 8 * (int(n * kept) + 1), dtype=torch.uint8, device="cuda")
+        old = c.set_option("gd_provisional_min_samples", how)
+        L.hpx_profile_reset(); L.hpx_profile_enable(1)
+        try:
+            rc = L.hpx_dgc_encode(1, c.ptr_array([d.data_ptr()]), c.i32_array([n]), c.ptr_array([out.data_ptr()]), c.f64_array([rate]),
+                                  c.f64_array([kept]), c.u64_array([9]), stream_ptr())
+            torch.cuda.synchronize()
+            assert rc == 0 and c.profile_query("gd_invert_kernel")[1] == (how == -2)
+        finally:
+            L.hpx_profile_enable(0); L.hpx_profile_reset()
+            c.set_option("gd_provisional_min_samples", old)
+        got.append((d, out))
+    size = int(got[1][1][:4].view(torch.int32)[0])
+    assert size > 4 and torch.equal(got[0][1][:size], got[1][1][:size]) and torch.equal(got[0][0], got[1][0])
+
+
+def test_against_the_oracle(gd, oracle_cpu):
+    rng = np.random.default_rng(2)
+    n = FIRST + 77
+    g, r = rng.laplace(0, 1e-3, n).astype(np.float32), rng.normal(0, 1e-4, n).astype(np.float32)
+    _check_encode(gd, oracle_cpu, g, r, 0.04, 0.999, 21 << 24)

@@ -13,6 +13,8 @@
 //               BEFORE the update (the same fp32 sum the update will store)
 //   select      exact k-th largest of the sample by three radix-histogram
 //               passes over the fp32 bit pattern (11+11+10 bits); no sort
+//   presample, pick   in place of these for tensors with large samples: a provisional threshold;
+//               behind the pass invert (or resample), exact and recount put the exact one in its place
 //   stream      ONE pass over the tensor: r = g + r, store r, compare with the
 //               threshold, wave64 ballot -> one 64-bit word per 64 elements
 //               (bit i = element i), a popcount and the largest |r| per workgroup, and the
@@ -61,14 +63,17 @@ constexpr int kCapLarge = 256;                   // tensors per launch table (17
 constexpr int kCapSmall = 4;                     // calls with a few tensors pass a table of a few hundred bytes
 
 struct GdState {
-  uint32_t hits;      // provisional path: samples found above the provisional threshold so far
   uint32_t thr_bits;  // threshold as fp32 bits (provisional path: the provisional one until the exact one is known)
   uint32_t fallback;  // provisional path: 1 when the provisional threshold turned out to lie above the exact one
   uint32_t total;     // candidates of a tensor whose cut follows on the device, left by the expand launch
-  uint32_t pad[60];
+  uint32_t pad[61];
 };
-constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold
-constexpr uint32_t kPreSamples = 16384;  // samples the provisional threshold is taken from
+constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold ...
+constexpr uint32_t kWayStep = 32;         // ... whose counters lie in lines of their own, this many words apart
+constexpr uint32_t kPreSamples = 16384;  // samples the provisional threshold is taken from where the caller gives the margin
+constexpr int64_t kProvisionalAuto = -2;  // the option that leaves the choice to provisional_pays
+constexpr int kBySpread = 1 << 20;        // the margin where the caller gives none (see pre_samples)
+constexpr uint32_t kPreExpected = 32;     // ... and how many of these samples are expected above the exact threshold
 constexpr uint32_t kFallback = 0xFFFFFFFEu;  // reported in place of a count: this tensor has to take the other path
 constexpr int kScanChunk = 4096;   // per-tile counts scanned by one workgroup
 constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
@@ -119,6 +124,12 @@ __host__ __device__ inline uint32_t list_room(uint32_t n, uint32_t limit) {
 __host__ __device__ inline size_t list_bytes(uint32_t n, uint32_t limit) {
   return align256(sizeof(uint64_t) * size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit));
 }
+// The launches behind the pass read them four lanes to a list, so that a wave has the lists of four tiles; the first entries,
+// whether there are as many or not, and the lengths are requested together.
+constexpr uint32_t kListTiles = 4, kListAhead = 2;
+constexpr uint32_t kListLanes = kWave / (kListTiles * (kThreads / kWave));
+static_assert(kListLanes * kListTiles * (kThreads / kWave) == kWave && kListAhead * kListLanes <= 16,
+              "lanes to a list, and entries a list has room for");
 // The cut path's buffers for up to `pairs` candidates: two copies of keys and indices, and the sort's counts.
 constexpr int kSortThreads = 1024;
 constexpr int kSortPer = 4;
@@ -163,7 +174,7 @@ struct GdArgs {
   int32_t nseg;
   int32_t residual;             // 0: the sparsifier without residual (dgc_body.h)
   int32_t margin;               // provisional path: how many times the expected number of entries the provisional
-                                // threshold lets through
+                                // threshold lets through, or kBySpread; negative: the gather path
   uint32_t gather;              // the pick launch gathers samples of up to this size itself
   uint32_t listed;              // the tensor's `limit` where the segment's own is set to 0 (a second expand launch), else unused
   int32_t device_cut;           // 1: tensors that keep fewer than kCutKeep entries are cut on the device and report nothing
@@ -319,16 +330,38 @@ __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<
 // The reference's threshold is the thr_index-th largest of a 1 % sample drawn at random positions: gathering it
 // costs a 128-byte line of G and one of R per sample, a fifth of the traffic of the pass over the tensor itself,
 // and it has to be finished before that pass can start.  This path starts the pass from a PROVISIONAL threshold
-// instead - taken from the first kPreSamples samples only and set low enough (`margin` times the expected
-// number of entries above it) that it all but certainly lies below the exact one - so the pass marks a superset
-// of the candidates.  Every sample whose value exceeds the provisional threshold is then one whose bit the pass
-// has set, so the exact threshold (the thr_index-th largest of ALL samples) is found among the samples whose bit is
-// set: a gather over the bit mask (1 bit per element, cache-resident) and the values of the few that hit.  A last
-// small pass clears the bits of the elements that do not exceed the exact threshold; scan and expand go on as
-// ever.  Should fewer than thr_index + 1 samples exceed the provisional threshold (it was not below the exact one,
-// or they tie), the tensor is reported as kFallback and the host sends it through the gather path, on the residual
-// the pass has already updated.
+// instead - taken from the first samples only (pre_samples) and set low enough that it all but certainly lies below the
+// exact one - so the pass lists and marks a superset of the candidates.  Every sample whose value exceeds the
+// provisional threshold is then among these, so the exact threshold (the thr_index-th largest of ALL samples) is found
+// among the candidates that are samples: by asking each of them (gd_invert_kernel), or for smaller tensors by looking
+// each sample up in the bit mask (gd_resample_kernel).  A last small launch drops the candidates that do not exceed
+// the exact threshold; scan and expand go on as ever.  Should fewer than thr_index + 1 samples exceed the provisional
+// threshold (it was not below the exact one, or they tie above zero), the tensor is reported as kFallback and the host
+// sends it through the gather path, on the residual the pass has already updated.
 //
+// How many samples the provisional threshold is taken from, and its rank among them.  Without a margin from the caller:
+// as many that kPreExpected of them should lie above the exact threshold, at a rank eight standard deviations beyond that, so
+// that the exact one lies below the provisional one in a case of 10^14.  More samples let less through and take the one
+// workgroup that ranks them longer: 138 M elements, a thousandth kept, 16, 32 and 64 expected: 348, 343 and 350 us a call.
+__host__ __device__ inline uint32_t pre_samples(uint32_t sample_cnt, uint32_t thr_index, int margin) {
+  uint64_t want = kPreSamples;
+  if (margin == kBySpread) {
+    want = (uint64_t(kPreExpected) * sample_cnt / (uint64_t(thr_index) + 1) + uint64_t(kThreads) - 1) / kThreads * kThreads;
+    want = want < kPickMax ? want : kPickMax;
+  }
+  return sample_cnt < want ? sample_cnt : uint32_t(want);
+}
+__device__ inline uint32_t pre_rank(uint32_t sample_cnt, uint32_t thr_index, int margin, uint32_t s0) {
+  uint64_t kp = 0;
+  if (margin == kBySpread) {
+    const float mean = float(thr_index + 1) * (float(s0) / float(sample_cnt));
+    kp = uint64_t(mean + 8.0f * __builtin_sqrtf(mean) + 8.0f);
+  } else if (margin > 0) {
+    kp = (uint64_t(margin) * (uint64_t(thr_index) + 1) * s0 + sample_cnt - 1) / sample_cnt + 8;
+  }
+  return kp > s0 - 1 ? s0 - 1 : uint32_t(kp);
+}
+
 // Rank `rank` (0-based from the top) of `count` keys in global memory, by one workgroup of kSelThreads lanes:
 // three histogram passes of 11 + 11 + 10 bits in LDS.  Every lane returns the key.
 __device__ __forceinline__ uint32_t select_rank(const uint32_t* __restrict__ keys, uint32_t count, uint32_t rank,
@@ -426,7 +459,7 @@ __device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[4], uin
   }
   return t;
 }
-template <int CAP>
+template <bool PROV, int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> a) {
   __shared__ uint32_t s_hist[kBins1];              // the lanes' largest keys; the histogram of the other way
   __shared__ __align__(16) uint32_t s_list[kPickAll];
@@ -435,7 +468,15 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
   const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
-  const uint32_t count = sg.sample_cnt, t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  const uint32_t count = PROV ? pre_samples(sg.sample_cnt, sg.thr_index, a.margin) : sg.sample_cnt;
+  const uint32_t rank = PROV ? pre_rank(sg.sample_cnt, sg.thr_index, a.margin, count) : sg.thr_index;
+  const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  auto settle = [&](uint32_t key) {  // one lane
+    GdState* st = seg_state(sg);
+    st->thr_bits = key;
+    if (PROV) st->fallback = 0;
+  };
+  if (PROV && t < uint32_t(kHitWays)) reinterpret_cast<uint32_t*>(sg.ws + l.hist)[t * kWayStep] = 0;
   // the lane's three largest keys
   uint32_t m1 = 0, m2 = 0, m3 = 0;
   auto take = [&](uint32_t k) {
@@ -444,7 +485,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
     m2 = m2 > u ? m2 : u;
     m3 = m3 > v ? m3 : v;
   };
-  if (count <= a.gather) {
+  if (!PROV && count <= a.gather) {
     constexpr int kOwn = (int(kPickGather) + kSelThreads - 1) / kSelThreads;
     float gv[kOwn], rv[kOwn];
 #pragma unroll
@@ -505,21 +546,21 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
     uint32_t one[1] = {q[0]};
 #pragma unroll
     for (uint32_t j = 1; j < 4; j++) one[0] = q[j] > one[0] ? q[j] : one[0];
-    const uint32_t b = count <= uint32_t(kWave) ? wave_rank<1, 0>(one, sg.thr_index, 0u)   // the sample itself
-                       : sg.thr_index < 32      ? wave_rank<1, 11>(one, sg.thr_index, 0u)
-                       : sg.thr_index < 128     ? wave_rank<4, 11>(q, sg.thr_index, 0u)
-                                                : wave_rank<kRows, 11>(k, sg.thr_index, 0u);
+    const uint32_t b = count <= uint32_t(kWave) ? wave_rank<1, 0>(one, rank, 0u)   // the sample itself
+                       : rank < 32      ? wave_rank<1, 11>(one, rank, 0u)
+                       : rank < 128     ? wave_rank<4, 11>(q, rank, 0u)
+                                                : wave_rank<kRows, 11>(k, rank, 0u);
     if (lane == 0) s_key = b;
   }
   __syncthreads();
   const uint32_t bound = s_key;
   if (count <= uint32_t(kWave)) {
-    if (t == 0) seg_state(sg)->thr_bits = bound;
+    if (t == 0) settle(bound);
     return;
   }
-  const bool bounded = sg.thr_index < uint32_t(kSelThreads) && bound != 0u;   // workgroup-uniform
+  const bool bounded = rank < uint32_t(kSelThreads) && bound != 0u;   // workgroup-uniform
   // (from 256 keys above the bound on, some lane all but certainly holds four)
-  if (bounded && sg.thr_index < 256u) {
+  if (bounded && rank < 256u) {
     if (__ballot(m1 >= bound) != 0) {   // most waves hold none
 #pragma unroll 1
       for (int j = 0; j < 3; j++) {
@@ -541,19 +582,19 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
         uint32_t found;
         if (n <= kWave) {
           const uint32_t k[1] = {lane < n ? s_list[lane] : 0u};
-          found = wave_rank<1, 0>(k, sg.thr_index, bound);
+          found = wave_rank<1, 0>(k, rank, bound);
         } else if (n <= 256) {
           uint32_t k[4];
 #pragma unroll
           for (uint32_t j = 0; j < 4; j++) k[j] = j * kWave + lane < n ? s_list[j * kWave + lane] : 0u;
-          found = wave_rank<4, 0>(k, sg.thr_index, bound);
+          found = wave_rank<4, 0>(k, rank, bound);
         } else {
           uint32_t k[kPickList / kWave];
 #pragma unroll
           for (uint32_t j = 0; j < kPickList / kWave; j++) k[j] = j * kWave + lane < n ? s_list[j * kWave + lane] : 0u;
-          found = wave_rank<kPickList / kWave, 0>(k, sg.thr_index, bound);
+          found = wave_rank<kPickList / kWave, 0>(k, rank, bound);
         }
-        if (lane == 0) seg_state(sg)->thr_bits = found;
+        if (lane == 0) settle(found);
       }
       return;
     }
@@ -604,17 +645,17 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
       uint32_t k[4];
 #pragma unroll
       for (uint32_t j = 0; j < 4; j++) k[j] = j * kSelThreads + t < n ? s_list[j * kSelThreads + t] : 0u;
-      const uint32_t found = workgroup_rank(k, sg.thr_index, bound, s_part);
-      if (t == 0) seg_state(sg)->thr_bits = found;
+      const uint32_t found = workgroup_rank(k, rank, bound, s_part);
+      if (t == 0) settle(found);
       return;
     }
   }
   __syncthreads();
-  const uint32_t exact = select_rank(samples, count, sg.thr_index, s_hist);
-  if (t == 0) seg_state(sg)->thr_bits = exact;
+  const uint32_t exact = select_rank(samples, count, rank, s_hist);
+  if (t == 0) settle(exact);
 }
 
-// The first kPreSamples samples, one per lane over many workgroups (one workgroup's gathers into arrays of
+// The first samples, one per lane over many workgroups (one workgroup's gathers into arrays of
 // hundreds of megabytes are bound by its CU's address translation: 16384 of them took it 90 us).
 template <int CAP>
 __global__ __launch_bounds__(kThreads) void gd_presample_kernel(const GdArgs<CAP> a) {
@@ -623,34 +664,11 @@ __global__ __launch_bounds__(kThreads) void gd_presample_kernel(const GdArgs<CAP
   const GdSeg& sg = a.seg[s];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
-  const uint32_t s0 = sg.sample_cnt < kPreSamples ? sg.sample_cnt : kPreSamples;
+  const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index, a.margin);
   const uint32_t x = uint32_t(tile - a.tile_start[s]) * kThreads + threadIdx.x;
   if (x < s0) {
     const uint32_t i = sample_index(sg.seed, x, sg.n);
     samples[x] = __float_as_uint(__builtin_fabsf(a.residual ? sg.g[i] + sg.r[i] : sg.g[i]));
-  }
-}
-
-// One workgroup per tensor: the provisional threshold from those samples; clears what the later phases count in.
-template <int CAP>
-__global__ __launch_bounds__(kSelThreads) void gd_provisional_kernel(const GdArgs<CAP> a) {
-  __shared__ uint32_t s_hist[kBins1];
-  const GdSeg& sg = a.seg[blockIdx.x];
-  const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
-  const uint32_t* samples = reinterpret_cast<const uint32_t*>(sg.ws + l.samples);
-  const uint32_t s0 = sg.sample_cnt < kPreSamples ? sg.sample_cnt : kPreSamples;
-  // rank of the provisional threshold among the s0 samples: `margin` times where the exact one is expected
-  uint64_t kp = 0;
-  if (a.margin > 0) kp = (uint64_t(a.margin) * (uint64_t(sg.thr_index) + 1) * s0 + sg.sample_cnt - 1) / sg.sample_cnt + 8;
-  if (kp > s0 - 1) kp = s0 - 1;
-  const uint32_t key = select_rank(samples, s0, uint32_t(kp), s_hist);
-  uint32_t* ways = reinterpret_cast<uint32_t*>(sg.ws + l.hist);
-  if (threadIdx.x < uint32_t(kHitWays)) ways[threadIdx.x] = 0;
-  if (threadIdx.x == 0) {
-    GdState* st = seg_state(sg);
-    st->thr_bits = key;
-    st->hits = 0;
-    st->fallback = 0;
   }
 }
 
@@ -671,7 +689,7 @@ __global__ __launch_bounds__(kThreads) void gd_resample_kernel(const GdArgs<CAP>
   const uint32_t blk = uint32_t(tile - a.tile_start[s]);
   const uint32_t way = blk % uint32_t(kHitWays);
   uint32_t* hits = reinterpret_cast<uint32_t*>(sg.ws + l.hitlist) + size_t(way) * hit_way_room(sg.sample_cnt);
-  uint32_t* counter = reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way;
+  uint32_t* counter = reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way * kWayStep;
   const uint32_t x = blk * kThreads + threadIdx.x;
   bool hit = false;
   uint32_t i = 0;
@@ -691,42 +709,156 @@ __global__ __launch_bounds__(kThreads) void gd_resample_kernel(const GdArgs<CAP>
   if (hit) hits[base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = __float_as_uint(__builtin_fabsf(sg.r[i]));
 }
 
-// One workgroup per tensor: the parts of the list are drawn together (into the samples' block, free by now), then
-// the exact threshold is taken from them, or the other path called for.
+// The other way round, for large tensors: no sample is looked up, each of the pass's few candidates works out how often it was
+// sampled.  Sample x is element (A (x + seed) + B mod 2^32) mod n, and A is odd: an element i is the sample of the x for
+// which that word is one of i, i + n, i + 2 n, ..., and from one of these words to the next x advances by n / A mod
+// 2^32.  2^32 / n additions and compares for each candidate, 32 for 138 M elements: for its 360 thousand candidates
+// this launch takes 7 us, the look-up of its 1.4 million samples took 13.  Four lanes to a list, as in the expand launch.
+constexpr uint32_t kInverseFrom = 1u << 24;   // elements: 256 steps a candidate
+__host__ __device__ constexpr uint32_t odd_inverse(uint32_t a) {
+  uint32_t v = a;                             // right to 3 bits; each step doubles them
+  for (int i = 0; i < 4; i++) v *= 2 - a * v;
+  return v;
+}
+constexpr uint32_t kLcgInverse = odd_inverse(lcg_mul(2));
+static_assert(kLcgInverse * lcg_mul(2) == 1u, "the multiplier has an inverse mod 2^32");
+template <int CAP>
+__global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a) {
+  const int blk = blockIdx.x;
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, blk);
+  const GdSeg& sg = a.seg[s];
+  const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
+  const uint32_t n = sg.n, ntiles = cdiv(n, kTile), lane = threadIdx.x & (kWave - 1);
+  const uint32_t own = uint32_t(blk - a.tile_start[s]);
+  const uint32_t tile0 = (own * (kThreads / kWave) + threadIdx.x / kWave) * kListTiles;
+  const uint32_t room = list_room(n, sg.limit), sub = lane % kListLanes, mine = tile0 * (kThreads / kWave) + lane / kListLanes;
+  const bool my_tile = tile0 + lane / (kListLanes * (kThreads / kWave)) < ntiles;
+  const uint2* __restrict__ list = seg_list(sg, l) + size_t(mine) * room;
+  uint2 p[kListAhead];
+  uint32_t listed = 0;
+  if (my_tile) {
+    listed = reinterpret_cast<const uint16_t*>(sg.ws + l.wcnt)[mine];
+    if (room != 0) {
+#pragma unroll
+      for (uint32_t q = 0; q < kListAhead; q++) p[q] = list[q * kListLanes + sub];
+    }
+  }
+  const uint32_t way = own % uint32_t(kHitWays), way_room = hit_way_room(sg.sample_cnt);
+  uint32_t* hits = reinterpret_cast<uint32_t*>(sg.ws + l.hitlist) + size_t(way) * way_room;
+  uint32_t* counter = reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way * kWayStep;
+  const uint32_t steps = 0xFFFFFFFFu / n, step = kLcgInverse * n, last = 0xFFFFFFFFu - steps * n;
+  auto sampled = [&](uint32_t i) {
+    uint32_t x = kLcgInverse * (i - lcg_add(2)) - sg.seed, times = 0;
+#pragma unroll 4
+    for (uint32_t m = 0; m < steps; m++, x += step) times += x < sg.sample_cnt ? 1u : 0u;
+    return times + (i <= last && x < sg.sample_cnt ? 1u : 0u);
+  };
+  auto note = [&](uint32_t times, uint32_t key) {
+    for (uint64_t m = __ballot(times != 0); m != 0; m = __ballot(times != 0)) {
+      uint32_t base = 0;
+      if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(counter, uint32_t(__popcll(m)));
+      base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+      if (times != 0) {
+        if (base < way_room) hits[base] = key; else seg_state(sg)->fallback = 1;
+        times--;
+      }
+    }
+  };
+  if (room != 0 && __ballot(listed > room) == 0) {
+    uint32_t times[kListAhead];
+#pragma unroll
+    for (uint32_t q = 0; q < kListAhead; q++) times[q] = q * kListLanes + sub < listed ? sampled(p[q].x) : 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < kListAhead; q++) note(times[q], p[q].y & 0x7FFFFFFFu);
+    for (uint32_t j = kListAhead * kListLanes; __ballot(j < listed) != 0; j += kListLanes) {
+      const bool any = j + sub < listed;
+      const uint2 e = any ? list[j + sub] : make_uint2(0, 0);
+      note(any ? sampled(e.x) : 0u, e.y & 0x7FFFFFFFu);
+    }
+    return;
+  }
+  // A list too short for its candidates: those of these tiles by the masks.
+  const uint64_t* __restrict__ masks = reinterpret_cast<const uint64_t*>(sg.ws + l.masks);
+  for (uint32_t tile = tile0; tile < tile0 + kListTiles && tile < ntiles; tile++) {
+    uint64_t m = masks[size_t(tile) * kWave + lane];
+    while (__ballot(m != 0) != 0) {
+      const uint32_t i = tile * uint32_t(kTile) + lane * kWave + uint32_t(m ? __builtin_ctzll(m) : 0);
+      const uint32_t times = m ? sampled(i) : 0u;
+      note(times, times ? __float_as_uint(sg.r[i]) & 0x7FFFFFFFu : 0u);
+      m &= m - 1;
+    }
+  }
+}
+
+// One workgroup per tensor: the parts of the list are drawn together (into LDS, or if they are too many into the samples'
+// block, free by now), then the exact threshold is taken from them, or the other path called for.
 template <int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_exact_kernel(const GdArgs<CAP> a) {
   __shared__ uint32_t s_hist[kBins1];
+  __shared__ uint32_t s_keys[kPickAll];
+  __shared__ uint32_t s_part[2][kSelThreads / kWave];
   __shared__ uint32_t s_off[kHitWays + 1];
   const GdSeg& sg = a.seg[blockIdx.x];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   GdState* st = seg_state(sg);
-  const uint32_t* ways = reinterpret_cast<const uint32_t*>(sg.ws + l.hist);
-  if (threadIdx.x == 0) {
-    uint32_t run = 0;
-    for (int w = 0; w < kHitWays; w++) { s_off[w] = run; run += ways[w]; }
-    s_off[kHitWays] = run;
+  const uint32_t prov = st->thr_bits, t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  if (st->fallback) return;   // uniform: not all that were found had room
+  static_assert(kHitWays == 2 * kWave && kHitWays * kWayStep <= uint32_t(kHistWords), "two counts a lane, in the histograms' block");
+  if (wave == 0) {
+    const uint32_t* ways = reinterpret_cast<const uint32_t*>(sg.ws + l.hist) + 2 * lane * kWayStep;
+    const uint32_t c0 = ways[0], c1 = ways[kWayStep];
+    uint32_t incl = c0 + c1;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t v = __shfl_up(incl, o, kWave);
+      if (lane >= uint32_t(o)) incl += v;
+    }
+    s_off[2 * lane] = incl - c0 - c1;
+    s_off[2 * lane + 1] = incl - c1;
+    if (lane == kWave - 1) s_off[kHitWays] = incl;
   }
   __syncthreads();
   const uint32_t found = s_off[kHitWays];
   if (found <= sg.thr_index) {
-    if (threadIdx.x == 0) st->fallback = 1;
+    // all other samples are at most the provisional threshold: nothing is less than zero, so that one is known
+    if (t == 0 && prov != 0) st->fallback = 1;
     return;
   }
   const uint32_t* parts = reinterpret_cast<const uint32_t*>(sg.ws + l.hitlist);
-  uint32_t* keys = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
+  uint32_t* keys = found <= kPickAll ? s_keys : reinterpret_cast<uint32_t*>(sg.ws + l.samples);
   const uint32_t room = hit_way_room(sg.sample_cnt);
-  for (int w = threadIdx.x / kWave; w < kHitWays; w += kSelThreads / kWave) {
-    const uint32_t c = s_off[w + 1] - s_off[w];
-    for (uint32_t k = threadIdx.x & (kWave - 1); k < c; k += kWave) keys[s_off[w] + k] = parts[size_t(w) * room + k];
+  // a wave has eight parts: the first keys of all of them are requested together
+  constexpr uint32_t kOwn = kHitWays / (kSelThreads / kWave);
+  uint32_t first[kOwn];
+#pragma unroll
+  for (uint32_t j = 0; j < kOwn; j++) {
+    const uint32_t w = j * (kSelThreads / kWave) + wave;
+    first[j] = lane < s_off[w + 1] - s_off[w] ? parts[size_t(w) * room + lane] : 0u;
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < kOwn; j++) {
+    const uint32_t w = j * (kSelThreads / kWave) + wave, c = s_off[w + 1] - s_off[w];
+    if (lane < c) keys[s_off[w] + lane] = first[j];
+    for (uint32_t k = kWave + lane; k < c; k += kWave) keys[s_off[w] + k] = parts[size_t(w) * room + k];
   }
   __syncthreads();
-  const uint32_t key = select_rank(keys, found, sg.thr_index, s_hist);
-  if (threadIdx.x == 0) st->thr_bits = key;
+  uint32_t key;
+  if (found <= kPickAll) {
+    uint32_t k[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) k[j] = j * kSelThreads + t < found ? s_keys[j * kSelThreads + t] : 0u;
+    key = workgroup_rank(k, sg.thr_index, prov, s_part);
+  } else {
+    key = select_rank(keys, found, sg.thr_index, s_hist);
+  }
+  // (a provisional threshold that is a NaN lets everything through: what is found at or below it is not all there is)
+  if (t == 0) {
+    if (key > prov) st->thr_bits = key; else st->fallback = 1;
+  }
 }
 
-// The bits of the elements that exceed the provisional threshold but not the exact one are cleared, the tiles'
-// counts corrected: a wave per tile, a mask word per lane, the value of a word's first set bit loaded for all
-// lanes together.
+// What exceeds the provisional threshold but not the exact one goes: out of the lists, in place, four lanes to each; where
+// the expand launch will look at the masks, because a list of its wave's is too short, out of those.
 template <int CAP>
 __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> a) {
   const int blk = blockIdx.x;
@@ -737,33 +869,71 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint64_t* __restrict__ masks = reinterpret_cast<uint64_t*>(sg.ws + l.masks);
   uint32_t* __restrict__ cnt = reinterpret_cast<uint32_t*>(sg.ws + l.cnt);
+  uint16_t* __restrict__ wcnt = reinterpret_cast<uint16_t*>(sg.ws + l.wcnt);
   const float* __restrict__ r = sg.r;
   const uint32_t ntiles = cdiv(sg.n, kTile);
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  const uint32_t tile = uint32_t(blk - a.tile_start[s]) * (kThreads / kWave) + threadIdx.x / kWave;
-  if (tile >= ntiles) return;
-  if (cnt[tile] == 0) return;  // wave-uniform
-  const float thr = __uint_as_float(st->thr_bits), nthr = -thr;
-  const uint64_t old = masks[size_t(tile) * kWave + lane];
-  const uint32_t e0 = tile * uint32_t(kTile) + lane * kWave;
-  uint64_t m = old, keep = 0;
-  const uint32_t b1 = m ? uint32_t(__builtin_ctzll(m)) : 0u;
-  const float v1 = m ? r[e0 + b1] : 0.0f;
-  if (m) {
-    if (v1 > thr || v1 < nthr) keep |= 1ull << b1;
-    m &= m - 1;
-  }
-  while (m) {
-    const uint32_t b = uint32_t(__builtin_ctzll(m));
-    m &= m - 1;
-    const float v = r[e0 + b];
-    if (v > thr || v < nthr) keep |= 1ull << b;
-  }
-  if (keep != old) masks[size_t(tile) * kWave + lane] = keep;
-  uint32_t c = uint32_t(__popcll(keep));
+  const uint32_t tile0 = (uint32_t(blk - a.tile_start[s]) * (kThreads / kWave) + threadIdx.x / kWave) * kListTiles;
+  const uint32_t room = list_room(sg.n, sg.limit), sub = lane % kListLanes, mine = tile0 * (kThreads / kWave) + lane / kListLanes;
+  const bool my_tile = tile0 + lane / (kListLanes * (kThreads / kWave)) < ntiles;
+  uint2* list = seg_list(sg, l) + size_t(mine) * room;
+  uint2 p[kListAhead];
+  uint32_t listed = 0;
+  if (my_tile) {
+    listed = wcnt[mine];
+    if (room != 0) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, kWave);
-  if (lane == 0) cnt[tile] = c;
+      for (uint32_t q = 0; q < kListAhead; q++) p[q] = list[q * kListLanes + sub];
+    }
+  }
+  const float thr = __uint_as_float(st->thr_bits), nthr = -thr;
+  if (room != 0 && __ballot(listed > room) == 0) {
+    uint32_t kept = 0;
+    auto keep = [&](bool any, uint2 e) {   // kept ones move down: never past a place that is still to be read
+      const float x = __uint_as_float(e.y);
+      const bool k = any && (x > thr || x < nthr);
+      const uint32_t group = uint32_t(__ballot(k) >> (lane - sub)) & ((1u << kListLanes) - 1u);
+      if (k) list[kept + uint32_t(__popc(group & ((1u << sub) - 1u)))] = e;
+      kept += uint32_t(__popc(group));
+    };
+#pragma unroll
+    for (uint32_t q = 0; q < kListAhead; q++) keep(q * kListLanes + sub < listed, p[q]);
+    for (uint32_t j = kListAhead * kListLanes; __ballot(j < listed) != 0; j += kListLanes) {
+      const bool any = j + sub < listed;
+      keep(any, any ? list[j + sub] : make_uint2(0, 0));
+    }
+    if (my_tile && sub == 0) wcnt[mine] = uint16_t(kept);
+    constexpr int kTileLanes = int(kListLanes * (kThreads / kWave));
+    uint32_t c = sub == 0 ? kept : 0u;
+#pragma unroll
+    for (int o = 1; o < kTileLanes; o <<= 1) c += __shfl_xor(c, o, kWave);
+    if (my_tile && lane % kTileLanes == 0) cnt[tile0 + lane / kTileLanes] = c;
+    return;
+  }
+  // A mask word per lane, the value of a word's first set bit loaded for all lanes together.
+  for (uint32_t tile = tile0; tile < tile0 + kListTiles && tile < ntiles; tile++) {
+    if (cnt[tile] == 0) continue;  // wave-uniform
+    const uint64_t old = masks[size_t(tile) * kWave + lane];
+    const uint32_t e0 = tile * uint32_t(kTile) + lane * kWave;
+    uint64_t m = old, keep = 0;
+    const uint32_t b1 = m ? uint32_t(__builtin_ctzll(m)) : 0u;
+    const float v1 = m ? r[e0 + b1] : 0.0f;
+    if (m) {
+      if (v1 > thr || v1 < nthr) keep |= 1ull << b1;
+      m &= m - 1;
+    }
+    while (m) {
+      const uint32_t b = uint32_t(__builtin_ctzll(m));
+      m &= m - 1;
+      const float v = r[e0 + b];
+      if (v > thr || v < nthr) keep |= 1ull << b;
+    }
+    if (keep != old) masks[size_t(tile) * kWave + lane] = keep;
+    uint32_t c = uint32_t(__popcll(keep));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, kWave);
+    if (lane == 0) cnt[tile] = c;
+  }
 }
 
 // The one pass over the tensors.  Lane l of wave w handles elements
@@ -771,7 +941,8 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
 // 64 consecutive elements in natural bit order.
 // RESIDUAL = false is the sparsifier without residual (dgc_body.h:110-117): the
 // values are G itself, nothing is added and nothing is stored (4 bytes per element).
-template <bool RESIDUAL, int CAP>
+// PROV: against the provisional threshold also a NaN is a candidate, as it is one of the largest of a sample.
+template <bool RESIDUAL, bool PROV, int CAP>
 __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a) {
   const int tile = blockIdx.x;
   const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
@@ -790,7 +961,8 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   const uint32_t wbase = base + wave * uint32_t(kWaveTile);
   // The wave's candidates are also listed as they are found, values and all: the launches behind the pass would otherwise
   // fetch a line of r for each (see list_room).
-  const uint32_t room = a.margin < 0 ? list_room(n, sg.limit) : 0u;
+  const uint32_t room = list_room(n, sg.limit);
+  auto passes = [&](float x) { return PROV ? !(__builtin_fabsf(x) <= thr) : (x > thr) || (x < nthr); };  // gd_body.h:59-67
   uint2* __restrict__ list = seg_list(sg, l) + (size_t(t) * (kThreads / kWave) + wave) * room;
   uint32_t lo = 0, hi = 0, cnt = 0;
   auto note = [&](uint64_t m, uint32_t e, float x) {  // m: the wave's candidates of 64 elements, uniform
@@ -812,7 +984,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
     for (int c = 0; c < kPerLane; c++) {
       const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];  // thrust::plus<float>()(G, R), gd_body.h:121-128
       if (RESIDUAL) __builtin_nontemporal_store(x, r + size_t(wbase) + c * kWave + lane);
-      const uint64_t m = __ballot((x > thr) || (x < nthr));  // gd_body.h:59-67
+      const uint64_t m = __ballot(passes(x));
       note(m, wbase + c * kWave + lane, x);
       big = __builtin_fmaxf(big, __builtin_fabsf(x));
       lo = lane == uint32_t(c) ? uint32_t(m) : lo;  // lane c keeps mask word c
@@ -834,7 +1006,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
       const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];
       if (e < n) {
         if (RESIDUAL) r[e] = x;
-        p = (x > thr) || (x < nthr);
+        p = passes(x);
         big = __builtin_fmaxf(big, __builtin_fabsf(x));
       }
       const uint64_t m = __ballot(p);
@@ -938,7 +1110,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_scan_kernel(const GdArgs<CAP> 
 // nothing else is touched; more than `cap` candidates do not fit those buffers
 // and the kernel does nothing for that tensor (the host then calls it again with larger ones,
 // limit = 0 and no report).
-constexpr int kExpandTiles = 4;
+constexpr int kExpandTiles = int(kListTiles);
 constexpr int kExpandPerBlock = (kThreads / kWave) * kExpandTiles;  // tiles per workgroup
 template <int CAP>
 __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a) {
@@ -959,11 +1131,9 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t tile0 = (uint32_t(blk - a.tile_start[s]) * (kThreads / kWave) + wave) * kExpandTiles;
 
-  // The lists of this wave's tiles, four lanes to each: their first entries, whether there are as many or not, and their
-  // lengths, all requested first.
-  constexpr uint32_t kLists = kExpandTiles * (kThreads / kWave), kPer = kWave / kLists, kAhead = 2;
-  static_assert(kLists * kPer == kWave && kAhead * kPer <= 16, "lanes to a list, and entries a list has room for");
-  const uint32_t room = a.margin < 0 ? list_room(sg.n, sg.limit ? sg.limit : a.listed) : 0u;
+  // The lists of this wave's tiles.
+  constexpr uint32_t kPer = kListLanes, kAhead = kListAhead;
+  const uint32_t room = list_room(sg.n, sg.limit ? sg.limit : a.listed);
   const uint32_t sub = lane % kPer, mine_list = tile0 * (kThreads / kWave) + lane / kPer;
   const bool my_tile = tile0 + lane / (kPer * (kThreads / kWave)) < ntiles;
   const uint2* __restrict__ list = seg_list(sg, l) + size_t(mine_list) * room;
@@ -2191,7 +2361,8 @@ int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
 struct Plan {
   GdSeg seg;
   size_t ws_bytes, cut_bytes;
-  int index;  // position in the call
+  int index;   // position in the call
+  int margin;  // how its threshold is found: GdArgs::margin
 };
 
 // Who settles a tensor behind the pass: one workgroup (gd_finish_kernel); the expand launch and, if it has to be cut, one
@@ -2199,6 +2370,19 @@ struct Plan {
 // many workgroups once it has heard the count.  The provisional path keeps to the last: it may have to fall back.
 bool finishes(const GdSeg& sg, int margin) { return margin < 0 && sg.limit <= kFinishKeep && cdiv(sg.n, kTile) <= kFinishTiles; }
 bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutKeep; }
+
+// Whether the provisional path is the quicker one for a tensor.  It saves the gather of the sample (two lines each, one
+// without a residual) and three of the four launches that rank it, and adds four short ones; its pass runs 8 % longer, the
+// gather's lines no longer waiting for it in the cache.  us per encode and decode, gather path -> provisional, at a sample of
+// 0.5 M: 169.6 -> 168.2; 0.6 M 192.7 -> 184.0; 0.85 M (17 M elements) 125.8 -> 113.3; 1.38 M 377 -> 337; 5 M 453 -> 280.  Encode without a residual:
+// 0.6 M 105.2 -> 108.3, 0.8 M 125.7 -> 117.1.  And by the kept fraction, which is what its own launches look at: 0.8 M
+// samples, 2 in 1000 243 -> 235, 4 in 1000 265 -> 281.
+constexpr uint32_t kProvisionalFrom = 600000, kProvisionalFromBare = 800000;   // samples
+constexpr uint32_t kProvisionalKept = 400;                                     // one in so many at most
+bool provisional_pays(const GdSeg& sg, bool residual) {
+  return sg.sample_cnt >= (residual ? kProvisionalFrom : kProvisionalFromBare) && sg.n >= kInverseFrom && sg.limit >= kCutKeep &&
+         sg.limit <= sg.n / kProvisionalKept;
+}
 
 // The phases for up to CAP tensors, no host wait.  margin < 0: the threshold from the full gathered sample
 // (for samples of up to kPickMax one workgroup each, behind a gather launch where a sample exceeds kPickGather; for
@@ -2227,10 +2411,14 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   };
   auto stream_pass = [&]() {
     const dim3 g = tiles([](const GdSeg& sg) { return cdiv(sg.n, kTile); });
-    if (residual)
-      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<true, CAP>), g, dim3(kThreads), st, a);
+    if (residual && margin < 0)
+      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<true, false, CAP>), g, dim3(kThreads), st, a);
+    else if (residual)
+      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<true, true, CAP>), g, dim3(kThreads), st, a);
+    else if (margin < 0)
+      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<false, false, CAP>), g, dim3(kThreads), st, a);
     else
-      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<false, CAP>), g, dim3(kThreads), st, a);
+      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<false, true, CAP>), g, dim3(kThreads), st, a);
   };
   dim3 grid;
   if (margin < 0) {
@@ -2246,7 +2434,7 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     });
     if (grid.x) HPX_LAUNCH("gd_sample_kernel", gd_sample_kernel<CAP>, grid, dim3(kThreads), st, a);
     grid = tiles([](const GdSeg& sg) { return sg.sample_cnt <= kPickMax ? 1u : 0u; });
-    if (grid.x) HPX_LAUNCH("gd_pick_kernel", gd_pick_kernel<CAP>, grid, dim3(kSelThreads), st, a);
+    if (grid.x) HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<false, CAP>), grid, dim3(kSelThreads), st, a);
     grid = tiles(sel_blocks);
     if (grid.x) {
       HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<1, CAP>), grid, dim3(kSelThreads), st, a);
@@ -2257,14 +2445,17 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     }
     stream_pass();
   } else {
-    grid = tiles([](const GdSeg& sg) { return cdiv(sg.sample_cnt < kPreSamples ? sg.sample_cnt : kPreSamples, kThreads); });
+    grid = tiles([margin](const GdSeg& sg) { return cdiv(pre_samples(sg.sample_cnt, sg.thr_index, margin), kThreads); });
     HPX_LAUNCH("gd_presample_kernel", gd_presample_kernel<CAP>, grid, dim3(kThreads), st, a);
-    HPX_LAUNCH("gd_provisional_kernel", gd_provisional_kernel<CAP>, dim3(uint32_t(count)), dim3(kSelThreads), st, a);
+    grid = tiles([](const GdSeg&) { return 1u; });
+    HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<true, CAP>), grid, dim3(kSelThreads), st, a);
     stream_pass();
-    grid = tiles([](const GdSeg& sg) { return cdiv(sg.sample_cnt, kThreads); });
-    HPX_LAUNCH("gd_resample_kernel", gd_resample_kernel<CAP>, grid, dim3(kThreads), st, a);
+    grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? cdiv(sg.sample_cnt, kThreads) : 0u; });
+    if (grid.x) HPX_LAUNCH("gd_resample_kernel", gd_resample_kernel<CAP>, grid, dim3(kThreads), st, a);
+    grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? 0u : cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
+    if (grid.x) HPX_LAUNCH("gd_invert_kernel", gd_invert_kernel<CAP>, grid, dim3(kThreads), st, a);
     HPX_LAUNCH("gd_exact_kernel", gd_exact_kernel<CAP>, dim3(uint32_t(count)), dim3(kSelThreads), st, a);
-    grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kThreads / kWave); });
+    grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
     HPX_LAUNCH("gd_recount_kernel", gd_recount_kernel<CAP>, grid, dim3(kThreads), st, a);
   }
   grid = tiles([](const GdSeg& sg) {
@@ -2317,9 +2508,9 @@ int poll_memory(Pending pending, const char* who, hipStream_t st) {
 // Waits until the expand launch has reported every tensor of `count` (the words are in pinned host memory and
 // the kernel writes them with system-scope stores as the first thing it does, so they arrive while the stream
 // is still busy with that launch).  A tensor that is settled on the device is not waited for.
-int wait_reports(volatile uint32_t* report, const Plan* plans, int count, int margin, hipStream_t st) {
+int wait_reports(volatile uint32_t* report, const Plan* plans, int count, hipStream_t st) {
   for (int t = 0; t < count; t++) {
-    if (cut_on_device(plans[t].seg, margin)) continue;
+    if (cut_on_device(plans[t].seg, plans[t].margin)) continue;
     volatile uint32_t* word = report + size_t(t) * kReportWords;
     auto pending = [word]() { return word[0] == kNotReported || word[1] == kNotReported || word[2] == kNotReported; };
     const int rc = poll_memory(pending, "sparsifier encode", st);
@@ -2403,12 +2594,14 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
   }
   volatile uint32_t* report = reinterpret_cast<volatile uint32_t*>(ws->pinned);
   const int total = int(plans.size());
-  // The provisional path pays where the gather of the full sample is long: from a few hundred thousand samples on.
   uint64_t all_samples = 0;
   for (const Plan& p : plans) all_samples += p.seg.sample_cnt;
   const int64_t prov_min = hpx::option(hpx::kOptGdProvisionalMinSamples);
   const int64_t prov_margin = hpx::option(hpx::kOptGdProvisionalMargin);
   const int margin = (prov_min >= 0 && all_samples >= uint64_t(prov_min) && prov_margin >= 0) ? int(prov_margin > 1000 ? 1000 : prov_margin) : -1;
+  for (Plan& p : plans) p.margin = prov_min == kProvisionalAuto ? (provisional_pays(p.seg, residuals != nullptr) ? kBySpread : -1) : margin;
+  // a launch table takes tensors of one path
+  std::stable_partition(plans.begin(), plans.end(), [](const Plan& p) { return p.margin >= 0; });
   auto reset_reports = [&](int n_) {
     for (int t = 0; t < n_; t++)
       for (int w = 0; w < 3; w++) report[size_t(t) * kReportWords + w] = kNotReported;
@@ -2417,19 +2610,20 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
   for (int first = 0; first < total; first += kMaxPerWait) {
     const int batch = total - first < kMaxPerWait ? total - first : kMaxPerWait;
     reset_reports(batch);
-    for (int k = 0; k < batch; k += kCapLarge) {
-      const int m = batch - k < kCapLarge ? batch - k : kCapLarge;
+    for (int k = 0, m; k < batch; k += m) {
+      const int how = plans[first + k].margin;
+      for (m = 1; m < kCapLarge && k + m < batch && plans[first + k + m].margin == how;) m++;
       uint32_t* rep = const_cast<uint32_t*>(report) + size_t(k) * kReportWords;
-      rc = m <= kCapSmall ? launch_phases<kCapSmall>(&plans[first + k], m, residuals != nullptr, margin, rep, st)
-                          : launch_phases<kCapLarge>(&plans[first + k], m, residuals != nullptr, margin, rep, st);
+      rc = m <= kCapSmall ? launch_phases<kCapSmall>(&plans[first + k], m, residuals != nullptr, how, rep, st)
+                          : launch_phases<kCapLarge>(&plans[first + k], m, residuals != nullptr, how, rep, st);
       if (rc != HPX_OK) return rc;
     }
-    rc = wait_reports(report, &plans[first], batch, margin, st);
+    rc = wait_reports(report, &plans[first], batch, st);
     if (rc != HPX_OK) return rc;
     // What the tensors reported, kept on the host: the pinned words serve again below.
     std::vector<uint32_t> rep_host(size_t(batch) * kReportWords);
     for (size_t w = 0; w < rep_host.size(); w++) rep_host[w] = report[w];
-    if (margin >= 0) {
+    if (plans[first].margin >= 0) {   // those come first
       // Tensors whose provisional threshold was not below the exact one: through the gather path, on the array
       // the pass has already updated (it holds G + R now: sampled and thresholded as it is, nothing added again).
       std::vector<int> fb;
@@ -2440,6 +2634,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         for (int t : fb) {
           Plan p = plans[first + t];
           p.seg.g = p.seg.r;
+          p.margin = -1;
           again.push_back(p);
         }
         ws->gd_fallbacks += fb.size();
@@ -2451,7 +2646,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
                               : launch_phases<kCapLarge>(&again[k], m, false, -1, rep, st);
           if (rc != HPX_OK) return rc;
         }
-        rc = wait_reports(report, again.data(), int(again.size()), -1, st);
+        rc = wait_reports(report, again.data(), int(again.size()), st);
         if (rc != HPX_OK) return rc;
         for (size_t j = 0; j < fb.size(); j++) {
           for (int w = 0; w < kReportWords; w++) rep_host[size_t(fb[j]) * kReportWords + w] = report[j * kReportWords + w];
@@ -2467,7 +2662,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
     for (int t = 0; t < batch; t++) {
       const GdSeg& sg = plans[first + t].seg;
       const uint32_t found = rep_host[size_t(t) * kReportWords];
-      if (cut_on_device(sg, margin) || found <= sg.limit) continue;
+      if (cut_on_device(sg, plans[first + t].margin) || found <= sg.limit) continue;
       const uint32_t thr_bits = rep_host[size_t(t) * kReportWords + 1], max_bits = rep_host[size_t(t) * kReportWords + 2];
       // keys are |r| bits minus threshold bits: the largest tells how many byte digits are in use
       const uint32_t max_key = max_bits > thr_bits ? max_bits - thr_bits : 0u;
@@ -2514,7 +2709,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         a.margin = -1;
         a.gather = 0;
         a.device_cut = 0;
-        a.listed = margin < 0 ? plan.seg.limit : plan.seg.n;   // the provisional path leaves no lists: no room for any
+        a.listed = plan.seg.limit;
         a.report = nullptr;  // the host has its report
         a.seg[0] = plan.seg;
         a.seg[0].cut = cut;
