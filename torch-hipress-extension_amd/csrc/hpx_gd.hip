@@ -426,13 +426,14 @@ __device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t
 // 161 tensors 20 -> 7 us, and 4 us less in the gather launch before it.
 constexpr uint32_t kPickList = 1024;
 constexpr uint32_t kPickAll = 4096;   // listed by a second walk over the sample where the lanes' three largest do not do
-// wave_rank over keys of the whole workgroup, four a lane: a barrier a bit.  s_part: two rows of a word per wave.
-__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[4], uint32_t rank, uint32_t floor, uint32_t (*s_part)[kSelThreads / kWave]) {
+// wave_rank over keys of the whole workgroup, R a lane: a barrier a bit.  s_part: two rows of a word per wave.
+template <int R>
+__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor, uint32_t (*s_part)[kSelThreads / kWave]) {
   constexpr int kWaves = kSelThreads / kWave;
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   uint32_t top = 0;
 #pragma unroll
-  for (int j = 0; j < 4; j++) top = key[j] > top ? key[j] : top;
+  for (int j = 0; j < R; j++) top = key[j] > top ? key[j] : top;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
   if (lane == 0) s_part[0][wave] = top;
@@ -449,7 +450,7 @@ __device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[4], uin
     const uint32_t c = t | (1u << b);
     uint32_t reach = 0;
 #pragma unroll
-    for (int j = 0; j < 4; j++) reach += uint32_t(__popcll(__ballot(key[j] >= c)));
+    for (int j = 0; j < R; j++) reach += uint32_t(__popcll(__ballot(key[j] >= c)));
     if (lane == 0) s_part[row][wave] = reach;
     __syncthreads();   // the row before it is not written again before everyone is past this one
     reach = 0;
@@ -790,66 +791,68 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
   }
 }
 
-// One workgroup per tensor: the parts of the list are drawn together (into LDS, or if they are too many into the samples'
-// block, free by now), then the exact threshold is taken from them, or the other path called for.
+// One workgroup per tensor: the exact threshold from the samples that were found, or the other path called for.  Eight lanes
+// take a part of the list, up to R keys each, and the rank is found bit by bit among the keys in registers; only if a
+// part is longer than that are they drawn together (into the samples' block, free by now) and ranked by histograms.
+// (Drawn together first: 12 thousand keys by histograms 27 us, now 18.5; 3 thousand in LDS as long as now, 10.  A histogram of the
+// keys' distance from the provisional threshold and the few keys of one bin, in place of the bits, took 2 to 4 us longer: the
+// more code of a launch of one workgroup, the more of it has to be fetched.)
+constexpr uint32_t kWayLanes = kSelThreads / kHitWays;
+template <int R>
+__device__ __forceinline__ uint32_t rank_hits(const uint32_t* __restrict__ part, uint32_t count, uint32_t rank, uint32_t floor,
+                                              uint32_t (*s_part)[kSelThreads / kWave]) {
+  uint32_t k[R];
+#pragma unroll
+  for (uint32_t j = 0; j < uint32_t(R); j++) {
+    const uint32_t at = j * kWayLanes + threadIdx.x % kWayLanes;
+    k[j] = at < count ? part[at] : 0u;
+  }
+  return workgroup_rank(k, rank, floor, s_part);
+}
 template <int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_exact_kernel(const GdArgs<CAP> a) {
   __shared__ uint32_t s_hist[kBins1];
-  __shared__ uint32_t s_keys[kPickAll];
   __shared__ uint32_t s_part[2][kSelThreads / kWave];
-  __shared__ uint32_t s_off[kHitWays + 1];
+  __shared__ uint32_t s_off[kHitWays];
   const GdSeg& sg = a.seg[blockIdx.x];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   GdState* st = seg_state(sg);
-  const uint32_t prov = st->thr_bits, t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  if (st->fallback) return;   // uniform: not all that were found had room
+  const uint32_t t = threadIdx.x, lane = t & (kWave - 1);
+  const uint32_t prov = st->thr_bits, way = t / kWayLanes, room = hit_way_room(sg.sample_cnt);
+  const uint32_t* ways = reinterpret_cast<const uint32_t*>(sg.ws + l.hist);
+  const uint32_t* parts = reinterpret_cast<const uint32_t*>(sg.ws + l.hitlist);
   static_assert(kHitWays == 2 * kWave && kHitWays * kWayStep <= uint32_t(kHistWords), "two counts a lane, in the histograms' block");
-  if (wave == 0) {
-    const uint32_t* ways = reinterpret_cast<const uint32_t*>(sg.ws + l.hist) + 2 * lane * kWayStep;
-    const uint32_t c0 = ways[0], c1 = ways[kWayStep];
-    uint32_t incl = c0 + c1;
+  const uint32_t mine = ways[way * kWayStep];
+  const uint32_t c0 = ways[2 * lane * kWayStep], c1 = ways[(2 * lane + 1) * kWayStep];   // every wave for itself
+  if (st->fallback) return;   // uniform: not all that were found had room
+  uint32_t incl = c0 + c1, most = c0 > c1 ? c0 : c1;
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t v = __shfl_up(incl, o, kWave);
-      if (lane >= uint32_t(o)) incl += v;
-    }
-    s_off[2 * lane] = incl - c0 - c1;
-    s_off[2 * lane + 1] = incl - c1;
-    if (lane == kWave - 1) s_off[kHitWays] = incl;
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t v = __shfl_up(incl, o, kWave);
+    if (lane >= uint32_t(o)) incl += v;
   }
-  __syncthreads();
-  const uint32_t found = s_off[kHitWays];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(most, o, kWave); most = v > most ? v : most; }
+  const uint32_t found = __builtin_amdgcn_readlane(incl, kWave - 1);
+  __syncthreads();   // nobody reads the state below
   if (found <= sg.thr_index) {
     // all other samples are at most the provisional threshold: nothing is less than zero, so that one is known
     if (t == 0 && prov != 0) st->fallback = 1;
     return;
   }
-  const uint32_t* parts = reinterpret_cast<const uint32_t*>(sg.ws + l.hitlist);
-  uint32_t* keys = found <= kPickAll ? s_keys : reinterpret_cast<uint32_t*>(sg.ws + l.samples);
-  const uint32_t room = hit_way_room(sg.sample_cnt);
-  // a wave has eight parts: the first keys of all of them are requested together
-  constexpr uint32_t kOwn = kHitWays / (kSelThreads / kWave);
-  uint32_t first[kOwn];
-#pragma unroll
-  for (uint32_t j = 0; j < kOwn; j++) {
-    const uint32_t w = j * (kSelThreads / kWave) + wave;
-    first[j] = lane < s_off[w + 1] - s_off[w] ? parts[size_t(w) * room + lane] : 0u;
-  }
-#pragma unroll
-  for (uint32_t j = 0; j < kOwn; j++) {
-    const uint32_t w = j * (kSelThreads / kWave) + wave, c = s_off[w + 1] - s_off[w];
-    if (lane < c) keys[s_off[w] + lane] = first[j];
-    for (uint32_t k = kWave + lane; k < c; k += kWave) keys[s_off[w] + k] = parts[size_t(w) * room + k];
-  }
-  __syncthreads();
+  const uint32_t* part = parts + size_t(way) * room;
   uint32_t key;
-  if (found <= kPickAll) {
-    uint32_t k[4];
-#pragma unroll
-    for (uint32_t j = 0; j < 4; j++) k[j] = j * kSelThreads + t < found ? s_keys[j * kSelThreads + t] : 0u;
-    key = workgroup_rank(k, sg.thr_index, prov, s_part);
+  if (most <= 8 * kWayLanes) {
+    key = rank_hits<8>(part, mine, sg.thr_index, prov, s_part);
+  } else if (most <= 32 * kWayLanes) {
+    key = rank_hits<32>(part, mine, sg.thr_index, prov, s_part);
   } else {
-    key = select_rank(keys, found, sg.thr_index, s_hist);
+    if (t < uint32_t(kWave)) { s_off[2 * lane] = incl - c0 - c1; s_off[2 * lane + 1] = incl - c1; }
+    __syncthreads();
+    uint32_t* keys = reinterpret_cast<uint32_t*>(sg.ws + l.samples) + s_off[way];
+    for (uint32_t k = t % kWayLanes; k < mine; k += kWayLanes) keys[k] = part[k];
+    __syncthreads();
+    key = select_rank(reinterpret_cast<uint32_t*>(sg.ws + l.samples), found, sg.thr_index, s_hist);
   }
   // (a provisional threshold that is a NaN lets everything through: what is found at or below it is not all there is)
   if (t == 0) {
