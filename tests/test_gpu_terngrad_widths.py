@@ -1,0 +1,55 @@
+"""GPU parity of decoding where the sizes of message and tensor do not tell the width: the decoder requests the codes of the
+width that fills the message before it has read the header, which may name another width, or fewer elements.  Bit-exact
+against the oracle."""
+import numpy as np
+import pytest
+
+from gpu_util import Terngrad, assert_bits_equal, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tg(capi):
+    return Terngrad(capi)
+
+
+def _decoded(oracle_cpu, m, out, add):
+    """What the message does to a tensor of out.size elements (the oracle writes all that the message holds)."""
+    room = np.zeros(out.size + 8 * m.size, np.float32)
+    room[:out.size] = out
+    return oracle_cpu.terngrad_decode(m, room.size, room, add)[1][:out.size]
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("n", [1, 3, 5, 2048, 4095, 4096, 4097, 9001])
+def test_messages_larger_and_smaller_than_their_codes(tg, oracle_cpu, bits, n):
+    rng = np.random.default_rng(n + bits)
+    # (min and max, as fp32, with either sign in the upper half of their words)
+    for scale in (1.0, -1.0):
+        x = (scale * np.abs(rng.normal(0, 1, n))).astype(np.float32)
+        whole = oracle_cpu.terngrad_encode(x, bits, 0, 1)[1]
+        noise = rng.integers(0, 256, 10 + n, dtype=np.uint8)
+        fills = {10 + (n * b + 7) // 8 for b in (1, 2, 4, 8)}    # where the sizes speak for some width
+        for size in sorted(fills | {whole.size + 1, whole.size + 5, whole.size - 1, 10 + n // 3} - set(range(11))):
+            m = np.concatenate([whole, noise])[:size]
+            for add in (0, 1):
+                out = rng.normal(0, 1, n).astype(np.float32)
+                d = dev(out)
+                tg.decode([dev(m)], [d], [add])
+                assert_bits_equal(host(d), _decoded(oracle_cpu, m, out, add), f"{size} bytes, add {add}")
+
+
+def test_a_list_of_mixed_fits(tg, oracle_cpu):
+    rng = np.random.default_rng(5)
+    ms, outs, adds = [], [], []
+    for i in range(40):
+        n, bits = int(rng.integers(1, 20000)), int(rng.choice([1, 2, 4, 8]))
+        m = oracle_cpu.terngrad_encode(rng.normal(0, 1, n).astype(np.float32), bits, 0, 1)[1]
+        if i % 3 == 1:
+            m = np.concatenate([m, np.zeros(int(rng.integers(1, 2 * n)), np.uint8)])
+        ms.append(m), outs.append(rng.normal(0, 1, n).astype(np.float32)), adds.append(int(i % 5 == 0))
+    ds = [dev(o) for o in outs]
+    tg.decode([dev(m) for m in ms], ds, adds)
+    for m, o, d, add in zip(ms, outs, ds, adds):
+        assert_bits_equal(host(d), _decoded(oracle_cpu, m, o, add))
