@@ -53,3 +53,35 @@ def test_a_list_of_mixed_fits(tg, oracle_cpu):
     tg.decode([dev(m) for m in ms], ds, adds)
     for m, o, d, add in zip(ms, outs, ds, adds):
         assert_bits_equal(host(d), _decoded(oracle_cpu, m, o, add))
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("n", [3, 5, 255, 4095, 4096, 4099, 9002])
+def test_several_messages_at_one_distance(tg, oracle_cpu, bits, n):
+    """A gathered buffer's slots: all as their sizes say; one of another width; one that covers fewer elements; one invalid."""
+    rng = np.random.default_rng(n * 8 + bits)
+    size = 10 + (n * bits + 7) // 8
+    for count in (2, 3, 7, 8, 9):
+        for odd in (None, "width", "tail", "invalid"):
+            for add0, skip in ((1, 0), (0, 0), (1, 1)):
+                slots = [oracle_cpu.terngrad_encode(rng.normal(0, 1, n).astype(np.float32), bits, 0, 1)[1] for _ in range(count)]
+                at = int(rng.integers(count)) if add0 else int(rng.integers(1, count))
+                if odd == "width":
+                    slots[at][0] = {1: 2, 2: 8, 4: 2, 8: 4}[bits]
+                elif odd == "tail":
+                    slots[at][1] = 255
+                elif odd == "invalid":
+                    slots[at][0] = 3
+                buf = np.zeros((count + 1) * size, np.uint8)
+                places = [j + (1 if skip and j >= count // 2 else 0) for j in range(count)]
+                for j, m in zip(places, slots):
+                    buf[j * size:(j + 1) * size] = m
+                d_buf, out = dev(buf), rng.normal(0, 1, n).astype(np.float32)
+                d = dev(out)
+                tg.decode([d_buf[j * size:(j + 1) * size] for j in places], [d] * count, [add0] + [1] * (count - 1))
+                want = out
+                for j, m in enumerate(slots):
+                    if m[0] != 3:
+                        want = _decoded(oracle_cpu, m, want, int(j > 0 or add0))
+                assert_bits_equal(host(d), want, f"{count} messages, odd one: {odd} at {at}, add0 {add0}")
+                assert (tg.status() != 0) == (odd == "invalid")

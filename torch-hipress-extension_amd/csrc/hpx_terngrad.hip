@@ -1468,6 +1468,10 @@ struct DecHead {
     if (c > sg.out_size) c = sg.out_size;
     return c > 0 ? static_cast<uint32_t>(c) : 0u;
   }
+  static __device__ __forceinline__ DecHead at(const uint8_t* in) {
+    return DecHead{as_global(reinterpret_cast<const u32u*>(in))->v, as_global(reinterpret_cast<const u32u*>(in + 4))->v,
+                   as_global(reinterpret_cast<const u16u*>(in + 8))->v};
+  }
 };
 // One tile of `cnt` elements in codes of B bits.  The codes (and old values) are requested before the header has come, of
 // which only then is seen whether it says B bits and cnt elements; if not, nothing is stored and the result is false.
@@ -1569,10 +1573,7 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_kernel(const DecArgs
   // the whole record and the place of its first tile in one round of scalar loads
   const int tile0 = a.tile_start[s];
   __asm__ volatile("" ::"s"(sg.out), "s"(sg.in), "s"(sg.out_size), "s"(sg.in_size), "s"(sg.add), "s"(sg.width), "s"(tile0));
-  DecHead head;
-  head.w0 = as_global(reinterpret_cast<const u32u*>(sg.in))->v;
-  head.w1 = as_global(reinterpret_cast<const u32u*>(sg.in + 4))->v;
-  head.w2 = as_global(reinterpret_cast<const u16u*>(sg.in + 8))->v;
+  const DecHead head = DecHead::at(sg.in);
   const uint32_t t = static_cast<uint32_t>(tile - tile0);
   const bool ss = a.stream_store != 0;
   if (decode_by_width(sg.width, sg, head, static_cast<uint32_t>(sg.out_size), t, ss)) return;
@@ -1632,7 +1633,7 @@ struct SSeg {
   int16_t nslots;
   int16_t add0;        // the first message is added to what the tensor holds
   int16_t skip;        // messages from this one on lie one distance further (the root's own slot is left out); -1: none
-  int16_t pad;
+  int16_t width;       // likely_width of the sizes
 };
 struct SArgs {
   int32_t nseg;
@@ -1654,10 +1655,11 @@ __device__ __forceinline__ MultiMsg multi_message(const MArgs& a, int s, int j) 
   const MSlot& m = a.slot[a.seg[s].first_slot + j];
   return MultiMsg{m.in, m.in_size, m.add};
 }
+__device__ __forceinline__ const uint8_t* strided_message(const SSeg& sg, int j) {
+  return sg.in0 + int64_t(j + ((sg.skip >= 0 && j >= sg.skip) ? 1 : 0)) * sg.stride;
+}
 __device__ __forceinline__ MultiMsg multi_message(const SArgs& a, int s, int j) {
-  const int skip = a.seg[s].skip;
-  return MultiMsg{a.seg[s].in0 + int64_t(j + ((skip >= 0 && j >= skip) ? 1 : 0)) * a.seg[s].stride, a.seg[s].in_size,
-                  j == 0 ? int32_t(a.seg[s].add0) : 1};
+  return MultiMsg{strided_message(a.seg[s], j), a.seg[s].in_size, j == 0 ? int32_t(a.seg[s].add0) : 1};
 }
 
 __device__ __forceinline__ uint32_t code_at(const uint8_t* __restrict__ pay, size_t i, uint32_t bits) {
@@ -1849,6 +1851,123 @@ __device__ __forceinline__ void decode_end(float* __restrict__ op, bool need_old
   for (int k = 0; k < kDIters; k++)
     if (g0 + k * kThreads < whole) st4(op + size_t(g[k]) * 4, acc[k]);
   if (one) op[last] = sum;
+}
+
+// One sub-tile of a tensor whose messages lie at one distance and fill their size with codes of B bits: their headers (one
+// to a lane), the codes of all of them and the old values are requested together, and only then is seen whether every header
+// says B bits and all n elements; if one does not, nothing is stored and the result is false.
+constexpr int kStridedMsgs = 8;
+template <int B>
+__device__ __forceinline__ bool decode_strided(const SSeg& sg, uint32_t sub) {
+  constexpr uint32_t DPB = 8 / B;
+  const uint32_t n = static_cast<uint32_t>(sg.out_size), lane = threadIdx.x & (kWave - 1);
+  const int ns = sg.nslots;
+  const bool need_old = sg.add0 != 0;
+  float* __restrict__ op = sg.out;
+  const DecHead head = DecHead::at(strided_message(sg, int(lane) < ns ? int(lane) : ns - 1));
+  const uint32_t g_first = sub * uint32_t(kThreads * kDIters);
+  const bool full = uint64_t(g_first + kThreads * kDIters) * 4 <= n;
+  // A wave's 2-bit codes of a whole sub-tile are one dword a lane and message (see decode_two_bit_whole).
+  const bool packed = B == 2 && full;
+  const uint32_t whole = n / 4, last = whole * 4 + threadIdx.x;
+  const bool one = !full && last < n && whole >= g_first && whole - g_first < uint32_t(kThreads * kDIters);  // a lane's one of the last, partial group
+  uint32_t g[kDIters];
+  float4 acc[kDIters];
+#pragma unroll
+  for (int k = 0; k < kDIters; k++) {
+    g[k] = B == 2 ? g_first + (threadIdx.x / kWave) * uint32_t(kDIters * kWave) + k * kWave + lane : g_first + k * kThreads + threadIdx.x;
+    const uint32_t at = full || g[k] < whole ? g[k] : 0u;
+    acc[k] = need_old && (full || whole) ? ld4_stream(op + size_t(at) * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  float sum = one && need_old ? op[last] : 0.f;
+  uint32_t raw[kStridedMsgs][kDIters], code[kStridedMsgs];
+#pragma unroll
+  for (int j = 0; j < kStridedMsgs; j++) {
+    if (j < ns) {
+      const uint8_t* pay = strided_message(sg, j) + 10;
+      code[j] = one ? uint32_t(as_global(pay)[last / DPB]) : 0u;
+      if (packed) {
+        raw[j][0] = as_global(reinterpret_cast<const u32u*>(pay + (g[0] - lane) + lane * 4))->v;
+      } else if (whole) {
+#pragma unroll
+        for (int k = 0; k < kDIters; k++) raw[j][k] = group_bits<B>(pay, size_t(full || g[k] < whole ? g[k] : 0u) * 4);
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  int64_t c = int64_t(sg.in_size - 10) * DPB - int64_t(head.w0 >> 8 & 0xFFu);
+  if (__ballot((head.w0 & 0xFFu) != uint32_t(B) || c < int64_t(n)) != 0) return false;
+  const float mns = __uint_as_float(head.w0 >> 16 | head.w1 << 16);
+  const float gaps = (__uint_as_float(head.w1 >> 16 | head.w2 << 16) - mns) / (float(1 << B) - 1.0f);
+#pragma unroll
+  for (int j = 0; j < kStridedMsgs; j++) {
+    if (j < ns) {
+      const float mn = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(__float_as_uint(mns), j)));
+      const float gap = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(__float_as_uint(gaps), j)));
+      const bool add = j > 0 || need_old;
+#pragma unroll
+      for (int k = 0; k < kDIters; k++) {
+        uint32_t bits = raw[j][k];
+        if (packed) bits = (uint32_t(__builtin_amdgcn_ds_bpermute(int(k * kWave + (lane / 4) * 4), int(raw[j][0]))) >> (8 * (lane & 3))) & 0xFFu;
+        const float4 v = group_values<B>(bits, gap, mn);
+        acc[k].x = add ? v.x + acc[k].x : v.x; acc[k].y = add ? v.y + acc[k].y : v.y;
+        acc[k].z = add ? v.z + acc[k].z : v.z; acc[k].w = add ? v.w + acc[k].w : v.w;
+      }
+      const float v = float(int((code[j] >> ((last % DPB) * B)) & ((1u << B) - 1u))) * gap + mn;
+      sum = add ? v + sum : v;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kDIters; k++) {
+    if (full) {
+      st4_stream(op + size_t(g[k]) * 4, acc[k]);
+      __asm__ volatile("" ::: "memory");
+    } else if (g[k] < whole) {
+      st4(op + size_t(g[k]) * 4, acc[k]);
+    }
+  }
+  if (one) op[last] = sum;
+  return true;
+}
+
+// The same sub-tile where the headers say something else than the sizes: element by element, message after message.
+__device__ __forceinline__ void decode_strided_by_header(const SSeg& sg, uint32_t sub, uint32_t* status) {
+  constexpr uint32_t kTileElements = kThreads * kDIters * 4;
+  const uint32_t n = static_cast<uint32_t>(sg.out_size), first = sub * kTileElements;
+  for (uint32_t i = threadIdx.x; i < kTileElements && first + i < n; i += kThreads) {
+    const uint32_t e = first + i;
+    float acc = sg.out[e];
+    for (int j = 0; j < sg.nslots; j++) {
+      const uint8_t* in = strided_message(sg, j);
+      const DecHead head = DecHead::at(in);
+      const uint32_t bits = head.w0 & 0xFFu;
+      if (bits != 1 && bits != 2 && bits != 4 && bits != 8) {
+        if (e == 0) atomicOr(status, 1u);
+        continue;
+      }
+      if (int64_t(e) >= int64_t(sg.in_size - 10) * int64_t(8 / bits) - int64_t(head.w0 >> 8 & 0xFFu)) continue;
+      const float mn = __uint_as_float(head.w0 >> 16 | head.w1 << 16);
+      const float gap = (__uint_as_float(head.w1 >> 16 | head.w2 << 16) - mn) / (float(1 << bits) - 1.0f);
+      const float v = float(int(code_at(in + 10, e, bits))) * gap + mn;  // terngrad_body.h:127, :158
+      acc = j > 0 || sg.add0 != 0 ? v + acc : v;
+    }
+    sg.out[e] = acc;
+  }
+}
+
+// Calls of one sub-tile to a workgroup, every message of one width by its size.  Such a launch is a chain of loads: with the
+// headers read first, through LDS, the codes behind them, and in one kernel of all widths and forms (125 KB of code, 144
+// registers; here 9 KB and 83), the launch over 24 odd-sized tensors with three 8-bit messages took 8.4 us, now 7.2, and the
+// root's pass 16.9, now 15.7.
+template <int B>
+__global__ __launch_bounds__(kThreads) void terngrad_decode_strided_kernel(const SArgs a) {
+  const int tile = blockIdx.x;
+  const int s = multi_segment(a, tile);
+  const SSeg sg = a.seg[s];
+  const int tile0 = a.tile_start[s];
+  __asm__ volatile("" ::"s"(sg.out), "s"(sg.in0), "s"(sg.stride), "s"(sg.out_size), "s"(sg.in_size), "s"(tile0));  // one round of scalar loads
+  const uint32_t sub = static_cast<uint32_t>(tile - tile0);
+  if (!decode_strided<B>(sg, sub)) decode_strided_by_header(sg, sub, a.status);
 }
 
 template <typename Args>
@@ -2538,7 +2657,8 @@ int launch_decode_multi(int count, float* const* outs, const int32_t* out_sizes,
       if (at < 0) {
         if (sa.nseg == kStrideSegs) { fits = false; break; }
         if (period == 0) index[outs[j]] = sa.nseg;
-        sa.seg[sa.nseg] = SSeg{outs[j], ins[j], 0, out_sizes[j], in_sizes[j], 1, int16_t(is_add_tos[j] != 0), -1, 0};
+        sa.seg[sa.nseg] = SSeg{outs[j], ins[j], 0, out_sizes[j], in_sizes[j], 1, int16_t(is_add_tos[j] != 0), -1,
+                               int16_t(likely_width(in_sizes[j], out_sizes[j]))};
         last[sa.nseg] = ins[j];
         sa.nseg++;
         continue;
@@ -2565,7 +2685,17 @@ int launch_decode_multi(int count, float* const* outs, const int32_t* out_sizes,
       sa.tile_start[k + 1] = int32_t(tiles);
     }
     if (fits && sa.nseg > 0) {
-      HPX_LAUNCH("terngrad_decode_multi_kernel", terngrad_decode_multi_kernel<SArgs>, dim3(sa.tile_start[sa.nseg]), dim3(kThreads), st, sa);
+      int width = sa.reps == 1 ? sa.seg[0].width : 0;
+      for (int k = 0; k < sa.nseg; k++)
+        if (sa.seg[k].width != width || sa.seg[k].nslots > kStridedMsgs) width = 0;
+      const dim3 grid(sa.tile_start[sa.nseg]);
+      switch (width) {
+        case 1: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<1>, grid, dim3(kThreads), st, sa); break;
+        case 2: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<2>, grid, dim3(kThreads), st, sa); break;
+        case 4: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<4>, grid, dim3(kThreads), st, sa); break;
+        case 8: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<8>, grid, dim3(kThreads), st, sa); break;
+        default: HPX_LAUNCH("terngrad_decode_multi_kernel", terngrad_decode_multi_kernel<SArgs>, grid, dim3(kThreads), st, sa);
+      }
       HPX_HIP(hipGetLastError());
       return HPX_OK;
     }
