@@ -127,3 +127,26 @@ def test_against_the_oracle(gd, oracle_cpu):
     n = FIRST + 77
     g, r = rng.laplace(0, 1e-3, n).astype(np.float32), rng.normal(0, 1e-4, n).astype(np.float32)
     _check_encode(gd, oracle_cpu, g, r, 0.04, 0.999, 21 << 24)
+
+
+def test_more_candidates_than_room_for_the_cut(gd, oracle_cpu, capi):
+    """Elements that are never sampled are large: the exact threshold lets five times the expected number through, and the
+    candidates are expanded a second time, into larger buffers."""
+    n, rate, seed = FIRST + 5, 0.05, 77
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    g = torch.empty(n, device="cuda").normal_(0, 1e-3, generator=gen)
+    large = torch.randint(0, n, (90_000,), device="cuda", generator=gen)
+    sampled = torch.tensor([oracle_cpu.gd_sample_index(seed, x, n) for x in range(int(np.ceil(n * rate)))], device="cuda")
+    kept = torch.zeros(n, dtype=torch.bool, device="cuda")
+    kept[sampled] = True
+    large = large[~kept[large]]
+    g[large] = torch.empty(large.numel(), device="cuda").uniform_(1, 2, generator=gen)
+    assert large.numel() > 84_000   # twice the expected number, and 65536 above it
+    assert _compare(gd, capi, [g], [torch.zeros(n, device="cuda")], [rate], [0.999], [seed]) == (1, 0)
+
+
+@pytest.mark.parametrize("n", [(1 << 28) - 3, (1 << 28) + 1])   # groups of tiles whose totals are read in one round, and in two
+def test_the_totals_of_many_groups(gd, capi, n):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    g = torch.empty(n, device="cuda").normal_(0, 1e-3, generator=gen)
+    assert _compare(gd, capi, [g], [torch.zeros(n, device="cuda")], [0.003], [0.9999], [1]) == (1, 0)

@@ -21,7 +21,7 @@
 //               candidates with their values in a short list per wave
 //   finish      tensors that keep up to 2560 entries: one workgroup lists the candidates, cuts
 //               them if they are too many, writes the message and clears the residual
-//   scan        larger tensors of more than 4096 workgroups: exclusive prefix of the
+//   scan        larger tensors of more than 4096 workgroups, but for those above: exclusive prefix of the
 //               per-workgroup counts within chunks of 4096, the chunks' totals and largest |r|
 //   expand      larger tensors: folds the totals (each workgroup for itself), reports count,
 //               threshold and largest |r| of each tensor to the host; lists (or bit words,
@@ -41,6 +41,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -77,6 +78,7 @@ constexpr uint32_t kPreExpected = 32;     // ... and how many of these samples a
 constexpr uint32_t kFallback = 0xFFFFFFFEu;  // reported in place of a count: this tensor has to take the other path
 constexpr int kScanChunk = 4096;   // per-tile counts scanned by one workgroup
 constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
+constexpr int kGroupTiles = 16;    // tiles whose candidates one workgroup of the recount and the expand launch looks after
 constexpr uint32_t kPickGather = 1536;   // a sample up to this size is gathered by the one workgroup that takes its threshold
 constexpr uint32_t kPickGatherBeside = 256;  // ... where the call has larger ones, and with them a gather launch, anyway
 constexpr uint32_t kPickMax = 65536;     // ... and up to this size its threshold is taken by one workgroup
@@ -89,7 +91,7 @@ __host__ __device__ constexpr uint32_t cdiv(uint64_t a, uint64_t b) { return sta
 
 // Where the pieces of one tensor's workspace block lie (the same arithmetic on the host and in the kernels).
 struct GdLayout {
-  size_t state, hist, samples, hitlist, masks, coarse, cnt, wcnt, mx, off, ctot, cmax, coff, end;
+  size_t state, hist, samples, hitlist, masks, coarse, cnt, wcnt, mx, off, ctot, cmax, end;
 };
 __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   const size_t ntiles = cdiv(n, kTile);
@@ -105,9 +107,9 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   l.wcnt = at;    at += align256(sizeof(uint64_t) * ntiles);              // candidates per wave of a tile, 16 bits each
   l.mx = at;      at += align256(sizeof(uint32_t) * ntiles);              // largest |r| per tile, as bits
   l.off = at;     at += align256(sizeof(uint32_t) * ntiles);              // exclusive prefix within the chunk
-  l.ctot = at;    at += align256(sizeof(uint32_t) * kMaxChunks);
-  l.cmax = at;    at += align256(sizeof(uint32_t) * kMaxChunks);
-  l.coff = at;    at += align256(sizeof(uint32_t) * kMaxChunks);
+  const size_t totals = cdiv(ntiles, kGroupTiles) > uint32_t(kMaxChunks) ? cdiv(ntiles, kGroupTiles) : size_t(kMaxChunks);
+  l.ctot = at;    at += align256(sizeof(uint32_t) * totals);              // candidates per chunk, on the provisional path per group
+  l.cmax = at;    at += align256(sizeof(uint32_t) * totals);              // largest |r| likewise
   l.end = at;
   return l;
 }
@@ -335,14 +337,14 @@ __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<
 // provisional threshold is then among these, so the exact threshold (the thr_index-th largest of ALL samples) is found
 // among the candidates that are samples: by asking each of them (gd_invert_kernel), or for smaller tensors by looking
 // each sample up in the bit mask (gd_resample_kernel).  A last small launch drops the candidates that do not exceed
-// the exact threshold; scan and expand go on as ever.  Should fewer than thr_index + 1 samples exceed the provisional
+// the exact threshold; expand goes on as ever.  Should fewer than thr_index + 1 samples exceed the provisional
 // threshold (it was not below the exact one, or they tie above zero), the tensor is reported as kFallback and the host
 // sends it through the gather path, on the residual the pass has already updated.
 //
 // How many samples the provisional threshold is taken from, and its rank among them.  Without a margin from the caller:
 // as many that kPreExpected of them should lie above the exact threshold, at a rank eight standard deviations beyond that, so
 // that the exact one lies below the provisional one in a case of 10^14.  More samples let less through and take the one
-// workgroup that ranks them longer: 138 M elements, a thousandth kept, 16, 32 and 64 expected: 348, 343 and 350 us a call.
+// workgroup that ranks them longer: 138 M elements, a thousandth kept, 16, 32 and 64 expected: 339, 335.4 and 335.4 us a call.
 __host__ __device__ inline uint32_t pre_samples(uint32_t sample_cnt, uint32_t thr_index, int margin) {
   uint64_t want = kPreSamples;
   if (margin == kBySpread) {
@@ -361,6 +363,12 @@ __device__ inline uint32_t pre_rank(uint32_t sample_cnt, uint32_t thr_index, int
   }
   return kp > s0 - 1 ? s0 - 1 : uint32_t(kp);
 }
+
+// With that choice each wave of the launch that gathers the samples leaves its kPreTop largest only.  It holds half a key above
+// the threshold at most (a rank of 86 or so among 11 thousand samples and more); one that holds more than it leaves makes the
+// provisional threshold a little lower, which it may be.
+constexpr uint32_t kPreTop = 4;
+static_assert(kPickMax / kWave * kPreTop <= 16 * kThreads, "what gd_prepick_kernel holds");
 
 // Rank `rank` (0-based from the top) of `count` keys in global memory, by one workgroup of kSelThreads lanes:
 // three histogram passes of 11 + 11 + 10 bits in LDS.  Every lane returns the key.
@@ -426,10 +434,21 @@ __device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t
 // 161 tensors 20 -> 7 us, and 4 us less in the gather launch before it.
 constexpr uint32_t kPickList = 1024;
 constexpr uint32_t kPickAll = 4096;   // listed by a second walk over the sample where the lanes' three largest do not do
-// wave_rank over keys of the whole workgroup, R a lane: a barrier a bit.  s_part: two rows of a word per wave.
-template <int R>
-__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor, uint32_t (*s_part)[kSelThreads / kWave]) {
-  constexpr int kWaves = kSelThreads / kWave;
+// The sum of a value that repeats every WAVES lanes, by rotations within the rows of 16 lanes.
+template <int WAVES>
+__device__ __forceinline__ uint32_t sum_of_waves(uint32_t v) {
+  static_assert(WAVES == 4 || WAVES == 16, "a power of two, at most a row");
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x121, 0xF, 0xF, false));
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x122, 0xF, 0xF, false));
+  if (WAVES > 4) {
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x124, 0xF, 0xF, false));
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x128, 0xF, 0xF, false));
+  }
+  return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+}
+// wave_rank over keys of a whole workgroup of WAVES waves, R a lane: a barrier a bit.  s_part: two rows of a word per wave.
+template <int R, int LO = 0, int WAVES = kSelThreads / kWave>
+__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor, uint32_t (*s_part)[WAVES]) {
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   uint32_t top = 0;
 #pragma unroll
@@ -439,24 +458,22 @@ __device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uin
   if (lane == 0) s_part[0][wave] = top;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kWaves; w++) top = s_part[0][w] > top ? s_part[0][w] : top;
+  for (int w = 0; w < WAVES; w++) top = s_part[0][w] > top ? s_part[0][w] : top;
   top = __builtin_amdgcn_readfirstlane(top);
   floor = __builtin_amdgcn_readfirstlane(floor);
   const int first = 31 - __builtin_clz((top ^ floor) | 1u);   // bits above it are common to every candidate
   uint32_t t = first < 31 ? (floor >> (first + 1)) << (first + 1) : 0u;
+  t = LO > 0 ? (t >> LO) << LO : t;
   int row = 1;
 #pragma unroll 1
-  for (int b = first < 30 ? first : 30; b >= 0; b--, row ^= 1) {
+  for (int b = first < 30 ? first : 30; b >= LO; b--, row ^= 1) {
     const uint32_t c = t | (1u << b);
     uint32_t reach = 0;
 #pragma unroll
     for (int j = 0; j < R; j++) reach += uint32_t(__popcll(__ballot(key[j] >= c)));
     if (lane == 0) s_part[row][wave] = reach;
     __syncthreads();   // the row before it is not written again before everyone is past this one
-    reach = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) reach += s_part[row][w];
-    if (reach > rank) t = c;
+    if (sum_of_waves<WAVES>(s_part[row][lane % WAVES]) > rank) t = c;
   }
   return t;
 }
@@ -667,10 +684,57 @@ __global__ __launch_bounds__(kThreads) void gd_presample_kernel(const GdArgs<CAP
   uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
   const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index, a.margin);
   const uint32_t x = uint32_t(tile - a.tile_start[s]) * kThreads + threadIdx.x;
+  uint32_t key = 0;
   if (x < s0) {
     const uint32_t i = sample_index(sg.seed, x, sg.n);
-    samples[x] = __float_as_uint(__builtin_fabsf(a.residual ? sg.g[i] + sg.r[i] : sg.g[i]));
+    key = __float_as_uint(__builtin_fabsf(a.residual ? sg.g[i] + sg.r[i] : sg.g[i]));
   }
+  if (a.margin != kBySpread) {
+    if (x < s0) samples[x] = key;
+    return;
+  }
+  const uint32_t lane = threadIdx.x & (kWave - 1), first = x - lane;
+  if (first >= s0) return;
+  uint32_t mine = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < kPreTop; j++) {
+    uint32_t top = key;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
+    if (lane == j) mine = top;
+    if (lane == uint32_t(__builtin_ctzll(__ballot(key == top)))) key = 0;
+  }
+  if (lane < kPreTop) samples[first / kWave * kPreTop + lane] = mine;
+}
+
+// The provisional threshold from what the waves of that launch have left, by one workgroup of four waves for each tensor: the
+// key of the rank wanted, cut off below ten bits of mantissa (a lower threshold will do).  Its code is short because it is
+// fetched anew in every call, and a barrier a bit is cheap among four waves: with all samples ranked by gd_pick_kernel this
+// launch took 7.3 us, and 13 in two calls of five; by sixteen waves 6.8; now 5.2 (138 M elements, 32 thousand samples).
+template <int CAP>
+__global__ __launch_bounds__(kThreads) void gd_prepick_kernel(const GdArgs<CAP> a) {
+  __shared__ uint32_t s_part[2][kThreads / kWave];
+  const GdSeg& sg = a.seg[blockIdx.x];
+  const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
+  const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index, a.margin), rank = pre_rank(sg.sample_cnt, sg.thr_index, a.margin, s0);
+  const uint32_t quads = cdiv(s0, kWave) * (kPreTop / 4), t = threadIdx.x;
+  const uint4* __restrict__ left = reinterpret_cast<const uint4*>(sg.ws + l.samples);
+  auto settle = [&](auto rounds) {
+    constexpr uint32_t kRounds = decltype(rounds)::value;
+    uint32_t key[4 * kRounds];
+#pragma unroll
+    for (uint32_t j = 0; j < kRounds; j++) {
+      const uint4 q = j * kThreads + t < quads ? left[j * kThreads + t] : make_uint4(0, 0, 0, 0);
+      key[4 * j] = q.x; key[4 * j + 1] = q.y; key[4 * j + 2] = q.z; key[4 * j + 3] = q.w;
+    }
+    if (t < uint32_t(kHitWays)) reinterpret_cast<uint32_t*>(sg.ws + l.hist)[t * kWayStep] = 0;
+    const uint32_t found = workgroup_rank<int(4 * kRounds), 13, kThreads / kWave>(key, rank, 0u, s_part);
+    if (t == 0) {
+      seg_state(sg)->thr_bits = found;
+      seg_state(sg)->fallback = 0;
+    }
+  };
+  if (quads <= 2 * kThreads) settle(std::integral_constant<uint32_t, 2>{}); else settle(std::integral_constant<uint32_t, 4>{});
 }
 
 // All samples against the bit mask the pass left: the values of those whose bit is set are listed.  The list is
@@ -868,7 +932,7 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
   const int s = find_segment<CAP>(a.tile_start, a.nseg, blk);
   const GdSeg& sg = a.seg[s];
   const GdState* st = seg_state(sg);
-  if (st->fallback) return;
+  if (st->fallback) return;   // uniform
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint64_t* __restrict__ masks = reinterpret_cast<uint64_t*>(sg.ws + l.masks);
   uint32_t* __restrict__ cnt = reinterpret_cast<uint32_t*>(sg.ws + l.cnt);
@@ -876,12 +940,15 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
   const float* __restrict__ r = sg.r;
   const uint32_t ntiles = cdiv(sg.n, kTile);
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  const uint32_t tile0 = (uint32_t(blk - a.tile_start[s]) * (kThreads / kWave) + threadIdx.x / kWave) * kListTiles;
+  const uint32_t group = uint32_t(blk - a.tile_start[s]), wave = threadIdx.x / kWave;
+  const uint32_t tile0 = (group * (kThreads / kWave) + wave) * kListTiles;
   const uint32_t room = list_room(sg.n, sg.limit), sub = lane % kListLanes, mine = tile0 * (kThreads / kWave) + lane / kListLanes;
   const bool my_tile = tile0 + lane / (kListLanes * (kThreads / kWave)) < ntiles;
   uint2* list = seg_list(sg, l) + size_t(mine) * room;
   uint2 p[kListAhead];
   uint32_t listed = 0;
+  uint32_t all = 0, big = 0;   // the wave's candidates that stay; its tiles' largest |r|
+  if (lane < kListTiles && tile0 + lane < ntiles) big = reinterpret_cast<const uint32_t*>(sg.ws + l.mx)[tile0 + lane];
   if (my_tile) {
     listed = wcnt[mine];
     if (room != 0) {
@@ -911,10 +978,11 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
 #pragma unroll
     for (int o = 1; o < kTileLanes; o <<= 1) c += __shfl_xor(c, o, kWave);
     if (my_tile && lane % kTileLanes == 0) cnt[tile0 + lane / kTileLanes] = c;
-    return;
-  }
-  // A mask word per lane, the value of a word's first set bit loaded for all lanes together.
-  for (uint32_t tile = tile0; tile < tile0 + kListTiles && tile < ntiles; tile++) {
+#pragma unroll
+    for (int o = kTileLanes; o < kWave; o <<= 1) c += __shfl_xor(c, o, kWave);
+    all = c;
+  } else for (uint32_t tile = tile0; tile < tile0 + kListTiles && tile < ntiles; tile++) {
+    // A mask word per lane, the value of a word's first set bit loaded for all lanes together.
     if (cnt[tile] == 0) continue;  // wave-uniform
     const uint64_t old = masks[size_t(tile) * kWave + lane];
     const uint32_t e0 = tile * uint32_t(kTile) + lane * kWave;
@@ -936,6 +1004,21 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, kWave);
     if (lane == 0) cnt[tile] = c;
+    all += c;
+  }
+  // The group's total and largest |r|, from which the expand launch works its places out: a scan launch before it took 6.5 us
+  // of a call with its hand-over.
+  __shared__ uint32_t s_all[kThreads / kWave], s_big[kThreads / kWave];
+#pragma unroll
+  for (int o = 1; o < int(kListTiles); o <<= 1) { const uint32_t v = __shfl_xor(big, o, kWave); big = v > big ? v : big; }
+  if (lane == 0) { s_all[wave] = all; s_big[wave] = big; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t total = 0, largest = 0;
+#pragma unroll
+    for (int w = 0; w < kThreads / kWave; w++) { total += s_all[w]; largest = s_big[w] > largest ? s_big[w] : largest; }
+    reinterpret_cast<uint32_t*>(sg.ws + l.ctot)[group] = total;
+    reinterpret_cast<uint32_t*>(sg.ws + l.cmax)[group] = largest;
   }
 }
 
@@ -1096,7 +1179,8 @@ __global__ __launch_bounds__(kSelThreads) void gd_scan_kernel(const GdArgs<CAP> 
   }
 }
 
-// Tensors of at most kScanChunk tiles (16.7 M elements) take no part in the scan launch: the expand launch's
+// Tensors of at most kScanChunk tiles (16.7 M elements), and those of the provisional path, whose recount leaves totals of 16
+// tiles each, take no part in the scan launch: the expand launch's
 // workgroups add up the counts before their tiles for themselves (at most 16 KB out of the L2), which saves
 // a launch of 3-5 us.
 //
@@ -1115,6 +1199,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_scan_kernel(const GdArgs<CAP> 
 // limit = 0 and no report).
 constexpr int kExpandTiles = int(kListTiles);
 constexpr int kExpandPerBlock = (kThreads / kWave) * kExpandTiles;  // tiles per workgroup
+static_assert(kExpandPerBlock == kGroupTiles && kExpandTiles == int(kListTiles), "the recount's groups are these workgroups' tiles");
 template <int CAP>
 __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a) {
   const int blk = blockIdx.x;
@@ -1152,7 +1237,8 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   uint32_t total, mm = 0;      // the tensor's candidates; its largest |r| (only the wave that reports needs it)
   uint32_t ex0 = 0, ex1 = 0;   // scanned tensors: exclusive prefixes of chunks 2 * lane and 2 * lane + 1
   uint32_t own_off = 0;        // the others: lane j's tile tile0 + j starts here
-  const bool scanned = nchunks > 1;
+  const bool grouped = a.margin >= 0;   // the recount has left the totals of the workgroups' tiles
+  const bool scanned = nchunks > 1 && !grouped;
   if (scanned) {
     // chunk totals, two per lane: inclusive prefix over the lanes
     const uint32_t* __restrict__ chunk_max = reinterpret_cast<const uint32_t*>(sg.ws + l.cmax);
@@ -1173,33 +1259,37 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
       for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(mm, o, kWave); mm = v > mm ? v : mm; }
     }
   } else {
-    // The counts of all tiles, four per lane and load (the array's padding may be read, not used): the total, and
-    // what lies before this workgroup's first tile.
-    const uint32_t first = uint32_t(blk - a.tile_start[s]) * kExpandPerBlock;
-    const uint4* __restrict__ cnt4 = reinterpret_cast<const uint4*>(sg.ws + l.cnt);
-    const uint4* __restrict__ mx4 = reinterpret_cast<const uint4*>(sg.ws + l.mx);
+    // The counts of all tiles, or of all groups, four per lane and load (the array's padding may be read, not used): the
+    // total, and what lies before this workgroup's first tile.
+    const uint32_t own_group = uint32_t(blk - a.tile_start[s]);
+    const uint32_t first = grouped ? own_group : own_group * kExpandPerBlock, counts = grouped ? cdiv(ntiles, kGroupTiles) : ntiles;
+    const uint4* __restrict__ cnt4 = reinterpret_cast<const uint4*>(sg.ws + (grouped ? l.ctot : l.cnt));
+    const uint4* __restrict__ mx4 = reinterpret_cast<const uint4*>(sg.ws + (grouped ? l.cmax : l.mx));
     constexpr uint32_t kSteps = kScanChunk / (4 * kThreads);
-    uint4 c[kSteps], big[kSteps];
-#pragma unroll
-    for (uint32_t q = 0; q < kSteps; q++) {
-      const uint32_t i = q * kThreads + threadIdx.x;
-      const bool any = 4 * i < ntiles;
-      c[q] = any ? cnt4[i] : make_uint4(0, 0, 0, 0);
-      big[q] = any && first == 0 ? mx4[i] : make_uint4(0, 0, 0, 0);
-    }
     const uint32_t j = tile0 + lane;
-    const uint32_t mine = lane < uint32_t(kExpandTiles) && j < ntiles ? reinterpret_cast<const uint32_t*>(cnt4)[j] : 0u;
+    const uint32_t mine = lane < uint32_t(kExpandTiles) && j < ntiles ? reinterpret_cast<const uint32_t*>(sg.ws + l.cnt)[j] : 0u;
     uint32_t all = 0, before = 0;
+#pragma unroll 1
+    for (uint32_t i0 = 0; i0 < counts; i0 += kScanChunk) {   // once, up to 2^24 elements, on the provisional path 2^28
+      uint4 c[kSteps], big[kSteps];
 #pragma unroll
-    for (uint32_t q = 0; q < kSteps; q++) {
-      const uint32_t i = 4 * (q * kThreads + threadIdx.x);
-      const uint32_t v[4] = {c[q].x, c[q].y, c[q].z, c[q].w}, b[4] = {big[q].x, big[q].y, big[q].z, big[q].w};
+      for (uint32_t q = 0; q < kSteps; q++) {
+        const uint32_t i = i0 / 4 + q * kThreads + threadIdx.x;
+        const bool any = 4 * i < counts;
+        c[q] = any ? cnt4[i] : make_uint4(0, 0, 0, 0);
+        big[q] = any && first == 0 ? mx4[i] : make_uint4(0, 0, 0, 0);
+      }
 #pragma unroll
-      for (uint32_t k = 0; k < 4; k++) {
-        const uint32_t x = i + k < ntiles ? v[k] : 0u, y = i + k < ntiles ? b[k] : 0u;
-        all += x;
-        before += i + k < first ? x : 0u;
-        mm = y > mm ? y : mm;
+      for (uint32_t q = 0; q < kSteps; q++) {
+        const uint32_t i = i0 + 4 * (q * kThreads + threadIdx.x);
+        const uint32_t v[4] = {c[q].x, c[q].y, c[q].z, c[q].w}, b[4] = {big[q].x, big[q].y, big[q].z, big[q].w};
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+          const uint32_t x = i + k < counts ? v[k] : 0u, y = i + k < counts ? b[k] : 0u;
+          all += x;
+          before += i + k < first ? x : 0u;
+          mm = y > mm ? y : mm;
+        }
       }
     }
 #pragma unroll
@@ -2390,7 +2480,7 @@ bool provisional_pays(const GdSeg& sg, bool residual) {
 // The phases for up to CAP tensors, no host wait.  margin < 0: the threshold from the full gathered sample
 // (for samples of up to kPickMax one workgroup each, behind a gather launch where a sample exceeds kPickGather; for
 // larger ones gather, three histogram passes, rank search), then the pass, and the finish or scan and expand.  A launch that no tensor of the table takes part in is left out.  margin >= 0: the provisional
-// path (above): provisional threshold, the pass, the samples against the mask, exact threshold, recount, scan, expand.
+// path (above): provisional threshold, the pass, the candidates that are samples, exact threshold, recount, expand.
 template <int CAP>
 int launch_phases(const Plan* plans, int count, bool residual, int margin, uint32_t* report, hipStream_t st) {
   GdArgs<CAP> a;
@@ -2451,7 +2541,10 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     grid = tiles([margin](const GdSeg& sg) { return cdiv(pre_samples(sg.sample_cnt, sg.thr_index, margin), kThreads); });
     HPX_LAUNCH("gd_presample_kernel", gd_presample_kernel<CAP>, grid, dim3(kThreads), st, a);
     grid = tiles([](const GdSeg&) { return 1u; });
-    HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<true, CAP>), grid, dim3(kSelThreads), st, a);
+    if (margin == kBySpread)
+      HPX_LAUNCH("gd_prepick_kernel", gd_prepick_kernel<CAP>, grid, dim3(kThreads), st, a);
+    else
+      HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<true, CAP>), grid, dim3(kSelThreads), st, a);
     stream_pass();
     grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? cdiv(sg.sample_cnt, kThreads) : 0u; });
     if (grid.x) HPX_LAUNCH("gd_resample_kernel", gd_resample_kernel<CAP>, grid, dim3(kThreads), st, a);
@@ -2461,9 +2554,9 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
     HPX_LAUNCH("gd_recount_kernel", gd_recount_kernel<CAP>, grid, dim3(kThreads), st, a);
   }
-  grid = tiles([](const GdSeg& sg) {
+  grid = tiles([margin](const GdSeg& sg) {
     const uint32_t chunks = cdiv(cdiv(sg.n, kTile), kScanChunk);
-    return chunks > 1 ? chunks : 0u;
+    return margin < 0 && chunks > 1 ? chunks : 0u;
   });
   if (grid.x) HPX_LAUNCH("gd_scan_kernel", gd_scan_kernel<CAP>, grid, dim3(kSelThreads), st, a);
   HPX_HIP(hipGetLastError());
@@ -2637,7 +2730,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         for (int t : fb) {
           Plan p = plans[first + t];
           p.seg.g = p.seg.r;
-          p.margin = -1;
+          p.margin = plans[first + t].margin = -1;
           again.push_back(p);
         }
         ws->gd_fallbacks += fb.size();
@@ -2709,7 +2802,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         GdArgs<kCapSmall> a;
         a.nseg = 1;
         a.residual = residuals != nullptr;
-        a.margin = -1;
+        a.margin = plan.margin;   // where its offsets come from
         a.gather = 0;
         a.device_cut = 0;
         a.listed = plan.seg.limit;
