@@ -72,7 +72,9 @@ def _compare(gd, capi, tensors, residuals, rates, drops, seeds, how=-2):
 
 @pytest.mark.parametrize("n,rate,kept,path", [(FIRST - 1, 0.05, 1e-3, False), (FIRST, 0.05, 1e-3, True), (FIRST + 4097, 0.04, 2.4e-3, True),
                                               (FIRST + 1, 1.0, 1e-3, True), (50_000_017, 0.02, 6e-4, True), (100_000_007, 0.01, 1e-3, True),
-                                              (FIRST, 0.05, 2.6e-3, False), (FIRST, 0.05, 4e-4, False), (59_000_000, 0.01, 1e-3, False)])
+                                              (FIRST, 0.05, 2.6e-3, True), (FIRST, 0.05, 3.4e-3, False), (FIRST, 0.05, 4e-4, False), (59_000_000, 0.01, 1e-3, False),
+                                              (24_000_000, 0.05, 3.4e-3, True), (24_000_000, 0.0416, 1.0e-2, False), (24_000_001, 0.3, 1.0e-2, True),
+                                              (100_000_007, 0.0101, 1.15e-2, True), (100_000_007, 0.0101, 1.2e-2, False), (23_999_999, 0.05, 3.4e-3, False)])
 def test_sizes(gd, capi, n, rate, kept, path):
     gen = torch.Generator(device="cuda").manual_seed(n)
     g, r = (torch.empty(n, device="cuda").normal_(0, s, generator=gen) for s in (1e-3, 1e-4))

@@ -75,6 +75,7 @@ constexpr uint32_t kPreSamples = 16384;  // samples the provisional threshold is
 constexpr int64_t kProvisionalAuto = -2;  // the option that leaves the choice to provisional_pays
 constexpr int kBySpread = 1 << 20;        // the margin where the caller gives none (see pre_samples)
 constexpr uint32_t kPreExpected = 32;     // ... and how many of these samples are expected above the exact threshold
+constexpr uint32_t kPreLeast = 32768;        // ... of at least this many
 constexpr uint32_t kFallback = 0xFFFFFFFEu;  // reported in place of a count: this tensor has to take the other path
 constexpr int kScanChunk = 4096;   // per-tile counts scanned by one workgroup
 constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
@@ -342,14 +343,14 @@ __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<
 // sends it through the gather path, on the residual the pass has already updated.
 //
 // How many samples the provisional threshold is taken from, and its rank among them.  Without a margin from the caller:
-// as many that kPreExpected of them should lie above the exact threshold, at a rank eight standard deviations beyond that, so
-// that the exact one lies below the provisional one in a case of 10^14.  More samples let less through and take the one
+// as many that kPreExpected of them should lie above the exact threshold, and kPreLeast, at a rank eight standard deviations
+// beyond that, so that the exact one lies below the provisional one in a case of 10^14.  More samples let less through and take the one
 // workgroup that ranks them longer: 138 M elements, a thousandth kept, 16, 32 and 64 expected: 339, 335.4 and 335.4 us a call.
 __host__ __device__ inline uint32_t pre_samples(uint32_t sample_cnt, uint32_t thr_index, int margin) {
   uint64_t want = kPreSamples;
   if (margin == kBySpread) {
     want = (uint64_t(kPreExpected) * sample_cnt / (uint64_t(thr_index) + 1) + uint64_t(kThreads) - 1) / kThreads * kThreads;
-    want = want < kPickMax ? want : kPickMax;
+    want = want < kPreLeast ? kPreLeast : want < kPickMax ? want : kPickMax;
   }
   return sample_cnt < want ? sample_cnt : uint32_t(want);
 }
@@ -364,9 +365,9 @@ __device__ inline uint32_t pre_rank(uint32_t sample_cnt, uint32_t thr_index, int
   return kp > s0 - 1 ? s0 - 1 : uint32_t(kp);
 }
 
-// With that choice each wave of the launch that gathers the samples leaves its kPreTop largest only.  It holds half a key above
-// the threshold at most (a rank of 86 or so among 11 thousand samples and more); one that holds more than it leaves makes the
-// provisional threshold a little lower, which it may be.
+// With that choice each wave of the launch that gathers the samples leaves its kPreTop largest only.  It holds one key above the
+// threshold at most on average (a rank of 490 or so among 32768 samples where one in a hundred is kept); one that holds more
+// than it leaves makes the provisional threshold a little lower, which it may be.
 constexpr uint32_t kPreTop = 4;
 static_assert(kPickMax / kWave * kPreTop <= 16 * kThreads, "what gd_prepick_kernel holds");
 
@@ -2465,16 +2466,21 @@ bool finishes(const GdSeg& sg, int margin) { return margin < 0 && sg.limit <= kF
 bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutKeep; }
 
 // Whether the provisional path is the quicker one for a tensor.  It saves the gather of the sample (two lines each, one
-// without a residual) and three of the four launches that rank it, and adds four short ones; its pass runs 8 % longer, the
-// gather's lines no longer waiting for it in the cache.  us per encode and decode, gather path -> provisional, at a sample of
-// 0.5 M: 169.6 -> 168.2; 0.6 M 192.7 -> 184.0; 0.85 M (17 M elements) 125.8 -> 113.3; 1.38 M 377 -> 337; 5 M 453 -> 280.  Encode without a residual:
-// 0.6 M 105.2 -> 108.3, 0.8 M 125.7 -> 117.1.  And by the kept fraction, which is what its own launches look at: 0.8 M
-// samples, 2 in 1000 243 -> 235, 4 in 1000 265 -> 281.
-constexpr uint32_t kProvisionalFrom = 600000, kProvisionalFromBare = 800000;   // samples
-constexpr uint32_t kProvisionalKept = 400;                                     // one in so many at most
+// without a residual), three of the four launches that rank it and the scan, and adds four short ones; its pass runs 8 %
+// longer, the gather's lines no longer waiting for it in the cache.  us per encode and decode, gather path -> provisional, one
+// in a thousand kept, by sample: 0.5 M 169.6 -> 168.2, 0.6 M 192.7 -> 184.0, 0.85 M (17 M elements) 125.8 -> 113.3, 1.38 M 377
+// -> 331, 5 M 453 -> 280; 3 in a thousand: 0.6 M 149.6 -> 136.1 (30 M elements) and 209 -> 196 (60 M).  Encode without a
+// residual: 0.6 M 105.2 -> 108.3, 0.8 M 125.7 -> 117.1.  Its own launches look at what is kept, and in smaller tensors longer at
+// each (gd_invert_kernel): one in a hundred, 0.6 M (31 M elements) 170.0 -> 178.5, 0.9 M 24 M elements 156.6 -> 158.4 and 90 M
+// 371 -> 360, 1.0 M 20 M elements 152 -> 155 and 50 M 250 -> 230, 1.5 M (76 M) 355 -> 311, 2.4 M (24 M) 223 -> 199, 5 M (100 M)
+// 557 -> 479; 5 in a thousand, 1.2 M 404 -> 379 (120 M).  Beyond 12 in 1024 there are no lists (list_room).
+constexpr uint32_t kProvisionalFrom = 600000, kProvisionalFromBare = 800000;   // samples ...
+constexpr uint32_t kProvisionalKept = 300;                                     // ... where one element in so many is kept at most
+constexpr uint32_t kProvisionalFromDense = 1000000, kProvisionalDense = 24000000;   // samples, and elements, where more are
 bool provisional_pays(const GdSeg& sg, bool residual) {
-  return sg.sample_cnt >= (residual ? kProvisionalFrom : kProvisionalFromBare) && sg.n >= kInverseFrom && sg.limit >= kCutKeep &&
-         sg.limit <= sg.n / kProvisionalKept;
+  if (sg.n < kInverseFrom || sg.limit < kCutKeep || list_room(sg.n, sg.limit) == 0) return false;
+  if (sg.limit <= sg.n / kProvisionalKept) return sg.sample_cnt >= (residual ? kProvisionalFrom : kProvisionalFromBare);
+  return residual && sg.n >= kProvisionalDense && sg.sample_cnt >= kProvisionalFromDense;
 }
 
 // The phases for up to CAP tensors, no host wait.  margin < 0: the threshold from the full gathered sample
