@@ -630,9 +630,9 @@ def x_terngrad_sizes(torch, np, capi, L, stream, gen, res):
     res["terngrad_102M"] = dict(big, algorithmic_bytes=8.5 * 102_760_448, workload="VGG-16 fc6, 2-bit, stochastic rounding, encode + decode(write)")
 
 
-GD_KERNELS = ["gd_sample_kernel", "gd_select_kernel", "gd_threshold_kernel", "gd_presample_kernel", "gd_pick_kernel", "gd_stream_kernel",
-              "gd_resample_kernel", "gd_invert_kernel", "gd_exact_kernel", "gd_recount_kernel", "gd_scan_kernel",
-              "gd_expand_kernel", "gd_sort_count_kernel", "gd_sort_pass_kernel", "gd_gather_kernel"]
+GD_KERNELS = ["gd_sample_kernel", "gd_select_kernel", "gd_threshold_kernel", "gd_presample_kernel", "gd_prepick_kernel", "gd_pick_kernel",
+              "gd_stream_kernel", "gd_resample_kernel", "gd_invert_kernel", "gd_exact_kernel", "gd_recount_kernel", "gd_scan_kernel",
+              "gd_expand_kernel", "gd_sort_count_kernel", "gd_sort_pass_kernel"]
 
 
 def x_dgc(torch, np, capi, L, stream, gen, res):
@@ -670,9 +670,9 @@ def x_dgc(torch, np, capi, L, stream, gen, res):
         r.copy_(r0)
         scrub.sum()
         kts = kernel_times(torch, capi, gd, GD_KERNELS, reps=1)
-        cut = kts["gd_gather_kernel"] is not None
+        cut = kts["gd_sort_pass_kernel"] is not None
         per_seed.append({"seed": seed, "encode_ms": round(float(np.median(times[2:])) * 1e3, 4), "selected": k, "cut": cut})
-        if kt is None or (cut and kt["gd_gather_kernel"] is None):
+        if kt is None or (cut and kt["gd_sort_pass_kernel"] is None):
             kt = kts
     sec = float(np.mean([p["encode_ms"] for p in per_seed])) * 1e-3
     dout = torch.zeros(n, device="cuda")

@@ -52,3 +52,18 @@ def test_kept_fractions(gd, oracle_cpu, n, kept):
     g, r = rng.laplace(0, 1e-3, n).astype(np.float32), rng.normal(0, 1e-4, n).astype(np.float32)
     for seed in (5, 9 << 24):
         _check_encode(gd, oracle_cpu, g, r.copy(), 0.02, 1 - kept, seed)
+
+
+@pytest.mark.parametrize("n,kept", [(900_001, 1e-2), (2_500_000, 1e-2), (9_000_001, 2e-3)])   # beyond what one workgroup cuts
+def test_a_cut_by_the_sort_keeps_the_signs(gd, oracle_cpu, n, kept):
+    """The sort's last pass writes the message from keys and indices alone: both signs, equal magnitudes, infinities."""
+    rng = np.random.default_rng(n)
+    cuts = 0
+    for seed in range(1 << 24, 6 << 24, 1 << 24):
+        g, r = rng.laplace(0, 1e-3, n).astype(np.float32), rng.normal(0, 1e-4, n).astype(np.float32)
+        g[::1009] = 0.5 * rng.choice([-1, 1], g[::1009].size).astype(np.float32)
+        r[::1009] = 0.0
+        g[n // 2], g[n // 2 + 1] = np.inf, -np.inf
+        info = _check_encode(gd, oracle_cpu, g, r, 0.02, 1 - kept, seed)[2]
+        cuts += info["candidates"] > info["kept"]
+    assert cuts > 0

@@ -1350,8 +1350,8 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   const uint32_t thr_bits = st->thr_bits;
   int32_t* __restrict__ cand = reinterpret_cast<int32_t*>(sg.cut + cl.ia);
   uint32_t* __restrict__ keys = reinterpret_cast<uint32_t*>(sg.cut + cl.ka);
-  // For the cut launch the sign travels in the index's top bit: it then never has to read the values again.
-  const uint32_t sign = cut_here ? 0x80000000u : 0u;
+  // In a cut the sign travels in the index's top bit: no launch then has to read the values again.
+  const uint32_t sign = 0x80000000u;
   int32_t* idx = reinterpret_cast<int32_t*>(out + 4);
   float* val = reinterpret_cast<float*>(out + 4 + size_t(total) * 4);
   if (room != 0 && __ballot(listed > room) == 0) {
@@ -1464,7 +1464,7 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
 // gives, take three passes instead of four), descending (bin = BINS - 1 - digit).
 // A pass is a count launch and a scatter launch over tiles of 4096 pairs
 // (1024 lanes x 4), counts[tile * BINS + bin]; the last pass writes
-// the message's index block instead of a sorted list.  All tensors of a call that
+// the message instead of a sorted list.  All tensors of a call that
 // have to be cut share these launches (a table of tensors in the kernel arguments);
 // the number of passes is that of the tensor with the largest key (a pass over a
 // digit that is zero in every key of a tensor leaves that tensor's order as it is).
@@ -1474,16 +1474,25 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
 // which costs more than the launches saved.)  (Counting a pass's digits where its
 // input is written, with global atomics, saves the count launches but was five
 // times slower: some 10^5 scattered atomics cost more than the launches.)
-struct SortSeg {           // one tensor that is being cut; 64 bytes
-  uint32_t* keys[2];       // the pass with parity p reads keys[p], idx[p] and writes keys[1 - p], idx[1 - p]
-  int32_t* idx[2];
-  uint32_t* counts;        // [tile][bins] of the current pass
-  uint8_t* msg;            // the message: its index block gets the first `keep` indices from the last pass
-  float* r;                // values are read from here, and cleared
+struct SortSeg {           // one tensor that is being cut; 40 bytes
+  uint8_t* cut;            // its buffers, cut_layout(cap): the pass with parity p reads one copy of keys and indices and writes the other
+  uint8_t* msg;            // the message, which the last pass writes
+  float* r;                // the entries that are sent are cleared here
   uint32_t n;              // candidates
   uint32_t keep;           // `expected`
+  uint32_t cap;
+  uint32_t thr_bits;       // a candidate's key is |r| less this, as bits
 };
-static_assert(sizeof(SortSeg) == 64, "segment record");
+static_assert(sizeof(SortSeg) == 40, "segment record");
+__device__ __forceinline__ uint32_t* sort_keys(const SortSeg& sg, const CutLayout& c, int parity) {
+  return reinterpret_cast<uint32_t*>(sg.cut + (parity ? c.kb : c.ka));
+}
+__device__ __forceinline__ int32_t* sort_ids(const SortSeg& sg, const CutLayout& c, int parity) {
+  return reinterpret_cast<int32_t*>(sg.cut + (parity ? c.ib : c.ia));
+}
+__device__ __forceinline__ uint32_t* sort_counts(const SortSeg& sg, const CutLayout& c) {   // [tile][bins] of the current pass
+  return reinterpret_cast<uint32_t*>(sg.cut + c.sc);
+}
 template <int CAP>
 struct SortArgs {
   int32_t nseg;
@@ -1494,29 +1503,6 @@ struct SortArgs {
   SortSeg seg[CAP];
 };
 static_assert(sizeof(SortArgs<kCapLarge>) <= 18000, "kernel-argument budget");
-
-// generate_S_value, gd_body.h:80-99, plus the header (gd_body.h:193-201), for
-// messages whose k indices are already in place (the cut path).  A launch of its
-// own with one lane per entry: done by the few workgroups of the last sort pass
-// these random accesses to r took three times as long.  tile_start counts blocks of
-// kThreads entries here.
-template <int CAP>
-__global__ __launch_bounds__(kThreads) void gd_gather_kernel(const SortArgs<CAP> a) {
-  const int blk = blockIdx.x;
-  const int s = find_segment<CAP>(a.tile_start, a.nseg, blk);
-  uint8_t* __restrict__ out = a.seg[s].msg;
-  float* __restrict__ r = a.seg[s].r;
-  const uint32_t k = a.seg[s].keep;
-  const int32_t* idx = reinterpret_cast<const int32_t*>(out + 4);
-  float* val = reinterpret_cast<float*>(out + 4 + size_t(k) * 4);
-  const uint32_t x = uint32_t(blk - a.tile_start[s]) * kThreads + threadIdx.x;
-  if (x == 0) *reinterpret_cast<int32_t*>(out) = int32_t(4 + k * 8);
-  if (x < k) {
-    const int32_t i = idx[x];
-    val[x] = r[i];
-    r[i] = 0.0f;
-  }
-}
 
 // Lanes of the wave whose `bin` equals this lane's, among the lanes in `live`.
 template <int BITS>
@@ -1538,11 +1524,13 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_count_kernel(const SortA
   constexpr uint32_t BINS = 1u << BITS;
   const int tile = blockIdx.x;
   const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
-  const uint32_t* __restrict__ keys = a.seg[s].keys[a.parity];
-  const uint32_t n = a.seg[s].n;
+  const SortSeg& sg = a.seg[s];
+  const CutLayout cl = cut_layout(sg.cap);
+  const uint32_t* __restrict__ keys = sort_keys(sg, cl, a.parity);
+  const uint32_t n = sg.n;
   const int shift = a.shift;
   const uint32_t ltile = uint32_t(tile - a.tile_start[s]);
-  uint32_t* __restrict__ counts = a.seg[s].counts;
+  uint32_t* __restrict__ counts = sort_counts(sg, cl);
   __shared__ uint32_t s_hist[BINS];
   const uint32_t t = threadIdx.x;
   const uint32_t lane = t & (kWave - 1);
@@ -1593,12 +1581,26 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
   const uint32_t n = sg.n;
   const uint32_t blk = uint32_t(gtile - a.tile_start[sgi]);                         // this tensor's tile ...
   const uint32_t nblk = uint32_t(a.tile_start[sgi + 1] - a.tile_start[sgi]);       // ... of so many
-  const uint32_t* __restrict__ keys_in = sg.keys[a.parity];
-  const int32_t* __restrict__ idx_in = sg.idx[a.parity];
-  uint32_t* __restrict__ keys_out = sg.keys[1 - a.parity];
-  int32_t* __restrict__ idx_out = sg.idx[1 - a.parity];
-  const uint32_t* __restrict__ counts = sg.counts;
+  const CutLayout cl = cut_layout(sg.cap);
+  const uint32_t* __restrict__ keys_in = sort_keys(sg, cl, a.parity);
+  const int32_t* __restrict__ idx_in = sort_ids(sg, cl, a.parity);
+  uint32_t* __restrict__ keys_out = sort_keys(sg, cl, 1 - a.parity);
+  int32_t* __restrict__ idx_out = sort_ids(sg, cl, 1 - a.parity);
+  const uint32_t* __restrict__ counts = sort_counts(sg, cl);
+  // The last pass writes the message (generate_S_value, gd_body.h:80-99, and the header, :193-201): a pair is all of an
+  // entry, its value the key above the threshold and the sign in the index's top bit, so nothing of r is read, and its
+  // clearing is a store that nobody waits for.  (A launch behind it that looked the values up: 9 us for 138 thousand
+  // entries of 138 M elements, 42 for 760 thousand of 76 M; the last pass takes 6 and 24 longer.)
   uint8_t* __restrict__ msg = a.last ? sg.msg : nullptr;
+  const uint32_t keep = sg.keep, thr_bits = sg.thr_bits;
+  float* __restrict__ r = sg.r;
+  auto send = [&](uint32_t slot, uint32_t k, uint32_t i) {
+    const uint32_t at = i & 0x7FFFFFFFu;
+    reinterpret_cast<uint32_t*>(msg + 4)[slot] = at;
+    reinterpret_cast<uint32_t*>(msg + 4 + size_t(keep) * 4)[slot] = (k + thr_bits) | (i & 0x80000000u);
+    r[at] = 0.0f;
+  };
+  if (msg && blk == 0 && t == 0) *reinterpret_cast<int32_t*>(msg) = int32_t(4 + keep * 8);
   const uint32_t b0 = blk * uint32_t(kSortTile);
   const uint32_t x0 = b0 + wave * uint32_t(kSortPer * kWave) + lane;
   uint32_t key[kSortPer];
@@ -1662,7 +1664,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
 #pragma unroll
       for (int j = 0; j < kSortPer; j++) {
         const uint32_t x = x0 + j * kWave;
-        if (x < n && x < sg.keep) reinterpret_cast<int32_t*>(msg + 4)[x] = id[j];
+        if (x < n && x < keep) send(x, key[j], uint32_t(id[j]));
       }
       return;
     }
@@ -1729,8 +1731,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
       const uint32_t b = (BINS - 1) - ((k >> a.shift) & (BINS - 1));
       const uint32_t slot = s_slot[b] + (p - s_first[b]);
       if (msg) {
-        // last pass: the indices that survive the cut go straight into the message
-        if (slot < sg.keep) reinterpret_cast<int32_t*>(msg + 4)[slot] = i;
+        if (slot < keep) send(slot, k, uint32_t(i));
       } else {
         keys_out[slot] = k;
         idx_out[slot] = i;
@@ -2403,6 +2404,7 @@ int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
 struct CutJob {
   SortSeg seg;
   int bits;  // significant bits of its largest key (at least 1)
+  int plan;  // the tensor's place among the call's plans
 };
 
 // The sort's launches for digits of BITS bits: `passes` x (count launch, scatter launch), lowest digit first, the
@@ -2425,8 +2427,7 @@ int sort_passes(SortArgs<CAP>& a, int passes, hipStream_t st) {
 }
 
 // The cut path for up to CAP tensors: the sort over all of them (as many digits as the largest key of any of
-// them has; digits of 9 bits where that takes fewer passes than bytes), then one gather launch that adds values
-// and headers and clears the residual entries.
+// them has; digits of 9 bits where that takes fewer passes than bytes), whose last pass writes the messages.
 template <int CAP>
 int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
   SortArgs<CAP> a;
@@ -2441,12 +2442,6 @@ int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
   const int bytes = (bits + 7) / 8, nines = (bits + 8) / 9;
   const int rc = nines < bytes ? sort_passes<CAP, 9>(a, nines, st) : sort_passes<CAP, 8>(a, bytes, st);
   if (rc != HPX_OK) return rc;
-  for (int i = 0; i < count; i++) {
-    const uint32_t k = jobs[i].seg.keep;
-    a.tile_start[i + 1] = a.tile_start[i] + int32_t(cdiv(k > 0 ? k : 1, kThreads));
-  }
-  HPX_LAUNCH("gd_gather_kernel", gd_gather_kernel<CAP>, dim3(uint32_t(a.tile_start[count])), dim3(kThreads), st, a);
-  HPX_HIP(hipGetLastError());
   return HPX_OK;
 }
 
@@ -2774,18 +2769,13 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
       job.seg.r = sg.r;
       job.seg.n = found;
       job.seg.keep = sg.limit;
-      job.seg.counts = nullptr;
+      job.seg.thr_bits = thr_bits;
+      job.seg.cut = sg.cut;
+      job.seg.cap = sg.cap;
+      job.plan = first + t;
       if (found > sg.cap) {
         overflow.push_back(int(jobs.size()));
         aux_need += cut_layout(found).end;
-        job.seg.keys[0] = reinterpret_cast<uint32_t*>(uintptr_t(first + t));  // the plan, until the block exists
-      } else {
-        const CutLayout cl = cut_layout(sg.cap);
-        job.seg.keys[0] = reinterpret_cast<uint32_t*>(sg.cut + cl.ka);
-        job.seg.keys[1] = reinterpret_cast<uint32_t*>(sg.cut + cl.kb);
-        job.seg.idx[0] = reinterpret_cast<int32_t*>(sg.cut + cl.ia);
-        job.seg.idx[1] = reinterpret_cast<int32_t*>(sg.cut + cl.ib);
-        job.seg.counts = reinterpret_cast<uint32_t*>(sg.cut + cl.sc);
       }
       jobs.push_back(job);
     }
@@ -2796,15 +2786,10 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
       size_t at = 0;
       for (int j : overflow) {
         CutJob& job = jobs[j];
-        const Plan& plan = plans[size_t(reinterpret_cast<uintptr_t>(job.seg.keys[0]))];
-        const CutLayout cl = cut_layout(job.seg.n);
-        uint8_t* cut = ws->aux + at;
-        at += cl.end;
-        job.seg.keys[0] = reinterpret_cast<uint32_t*>(cut + cl.ka);
-        job.seg.keys[1] = reinterpret_cast<uint32_t*>(cut + cl.kb);
-        job.seg.idx[0] = reinterpret_cast<int32_t*>(cut + cl.ia);
-        job.seg.idx[1] = reinterpret_cast<int32_t*>(cut + cl.ib);
-        job.seg.counts = reinterpret_cast<uint32_t*>(cut + cl.sc);
+        const Plan& plan = plans[job.plan];
+        job.seg.cut = ws->aux + at;
+        job.seg.cap = job.seg.n;
+        at += cut_layout(job.seg.n).end;
         GdArgs<kCapSmall> a;
         a.nseg = 1;
         a.residual = residuals != nullptr;
@@ -2814,7 +2799,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         a.listed = plan.seg.limit;
         a.report = nullptr;  // the host has its report
         a.seg[0] = plan.seg;
-        a.seg[0].cut = cut;
+        a.seg[0].cut = job.seg.cut;
         a.seg[0].cap = job.seg.n;
         a.seg[0].limit = 0u;
         a.tile_start[0] = 0;
