@@ -532,3 +532,31 @@ def test_batches_one_after_the_other_share_their_staging_memory(hp):
         used.append(torch.cuda.mem_get_info()[0])
     assert used[0] - used[-1] <= 2 << 20, used
     assert hp.error_count() == 0, hp.last_error()
+
+
+def test_large_graddrop_tasks_of_one_batch_share_one_workspace(hp, oracle_cpu):
+    # Queued together (the worker is busy with the first one), large tasks are encoded one call after the other.
+    n, sr, dr_ = 34_000_000, 0.002, 0.9999
+    fixed = 4 + int(2 * np.ceil(n * (1 - dr_))) * 4
+    gs = [torch.randn(n, device="cuda") * 1e-3 for _ in range(5)]
+    rs = [torch.zeros(n, device="cuda") for _ in gs]
+    Cs = [_host_buf(fixed, 1) for _ in gs]
+    items = [(f"w{k}", g, r, torch.zeros(fixed, dtype=torch.uint8, device="cuda"), c, 0, 10) for k, (g, r, c) in enumerate(zip(gs, rs, Cs))]
+    torch.cuda.synchronize()
+    assert hp.init("graddrop", {"sample_rate": sr, "drop_ratio": dr_, "seed": 1}, 0, 0, 2)
+    free = torch.cuda.mem_get_info()[0]
+    assert hp.submit_task(*items[0])
+    _collect(hp, 10, ["w0"])
+    one = free - torch.cuda.mem_get_info()[0]
+    rs[0].zero_()
+    torch.cuda.synchronize()
+    for it in items:
+        assert hp.submit_task(*it)
+    _collect(hp, 10, [it[0] for it in items])
+    assert one > 0 and free - torch.cuda.mem_get_info()[0] <= one + (2 << 20), one
+    for g, r, c in zip(gs, rs, Cs):
+        want_r = np.zeros(n, np.float32)
+        msg, _ = oracle_cpu.gd_encode(host(g), want_r, sr, dr_, 1)
+        assert_bits_equal(c.numpy()[:msg.size], msg, "message")
+        assert_bits_equal(host(r), want_r, "residual")
+    assert hp.error_count() == 0, hp.last_error()

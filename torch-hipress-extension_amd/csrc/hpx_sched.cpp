@@ -319,6 +319,7 @@ hipEvent_t mark(Worker& w, hipStream_t st) {
 }
 
 // ---- the three quantiser / sparsifier algorithms ---------------------------------
+constexpr int64_t kGdRunElements = int64_t(1) << 25;   // of these a pass alone takes 60 us, several times a call's host wait
 void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch, bool one_lane) {
   // GradDrop stays on one lane too: its encode's workspace grows with the tensors (20 MB for 60 M elements), and a second
   // one would buy little, with messages a thousandth of the tensor.
@@ -348,7 +349,8 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
   // Transfers and codec calls are cut into runs so that the PCIe transfer of one run overlaps the kernels of
   // the next (a 200-tensor TBQ bucket spends 2.5 times as long on the link as in its encode kernel).
   // GradDrop messages are tiny and its encode has a large fixed cost per call, so a GradDrop batch stays
-  // one run.
+  // one run, up to kGdRunElements: its workspace grows with the tensors of a call (24 MB for 60 M elements), and how many
+  // large ones fall into a batch is a matter of when the worker looks.
   const bool one_run = p.alg == kGraddrop;
   auto next_run_bytes = [one_run](int64_t b) {
     if (one_run) return INT64_MAX;
@@ -486,8 +488,10 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
       std::vector<const Task*> run;
       int64_t bytes = 0;
       pipe_bytes = next_run_bytes(pipe_bytes);
-      while (i < ts.size() && bytes < pipe_bytes) {
+      int64_t elements = 0;
+      while (i < ts.size() && bytes < pipe_bytes && !(one_run && elements >= kGdRunElements)) {
         bytes += message_bytes(p, ts[i]->t);
+        elements += ts[i]->t.tensor_numel;
         run.push_back(ts[i++]);
       }
       const bool alone = i == ts.size() && run.size() == ts.size() && w.in_flight.size() == 1;
