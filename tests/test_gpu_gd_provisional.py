@@ -2,6 +2,8 @@
 and the exact one is found among the candidates, each of which works out how often it was sampled.  Message and updated
 residual are the gather path's bit for bit: at both ends of the sizes, with lists too short for their candidates,
 with equal values on either side of the threshold, zeros, infinities and NaN."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -24,6 +26,11 @@ def _values(kind, n, gen):
     if kind == "crowded":          # lists overflow: half of the large values within one element in a thousand
         g *= 1e-3
         g[n // 3:n // 3 + n // 1500] *= 4e3
+    elif kind == "rows":           # an embedding's gradient: one row of 1024 in fifty, or in 666, and nothing else
+        rows = n // 1024
+        on = torch.rand(rows, device="cuda", generator=gen) < (1 / 50 if n % 2 else 1 / 666)
+        g[:rows * 1024].view(rows, 1024).mul_(on[:, None])
+        g[rows * 1024:] = 0
     elif kind == "sparse":         # too few non-zeros for a threshold above zero
         g *= (torch.empty(n, device="cuda").uniform_(0, 1, generator=gen) < 2e-4)
     elif kind == "coarse":         # many equal values, the provisional threshold among them
@@ -83,13 +90,40 @@ def test_sizes(gd, capi, n, rate, kept, path):
         assert (inverted, fell_back) == (int(path), 0)
 
 
-@pytest.mark.parametrize("kind,fallback", [("crowded", 0), ("sparse", 0), ("coarse", 1), ("signs", 1), ("infinite", 0), ("nan", None), ("all_nan", None)])
+@pytest.mark.parametrize("kind,fallback", [("crowded", 0), ("rows", 0), ("sparse", 0), ("coarse", 1), ("signs", 1), ("infinite", 0), ("nan", None), ("all_nan", None)])
 def test_values(gd, capi, kind, fallback):
     n = 20_000_003
     gen = torch.Generator(device="cuda").manual_seed(7)
     g, r = _values(kind, n, gen), torch.zeros(n, device="cuda")
     inverted, fell_back = _compare(gd, capi, [g], [r], [0.05], [0.999], [11])
     assert inverted == 1 and (fallback is None or fell_back == fallback)
+
+
+def _us(gd, capi, how, g, rate, drop):
+    """Least time of a call, from its start until the GPU has finished."""
+    r, out = torch.zeros_like(g), torch.empty(4 + 8 * int(np.ceil(g.numel() * (1 - drop))), dtype=torch.uint8, device="cuda")
+    old, least = capi.set_option("gd_provisional_min_samples", how), float("inf")
+    try:
+        for seed in range(9):
+            r.zero_()
+            torch.cuda.synchronize()
+            start = time.perf_counter()
+            gd.encode([g], [r], [out], [rate], [drop], [seed])
+            torch.cuda.synchronize()
+            least = min(least, (time.perf_counter() - start) * 1e6)
+    finally:
+        capi.set_option("gd_provisional_min_samples", old)
+    return least
+
+
+@pytest.mark.parametrize("kind", ["crowded", "rows"])
+@pytest.mark.parametrize("n,rate", [(FIRST, 0.05), (FIRST + 1, 0.05), (60_000_000, 0.02), (60_000_001, 0.02)])
+def test_large_values_that_lie_together_take_no_longer(gd, capi, kind, n, rate):
+    """The path is there because it is quicker: it has to be for these tensors as well, whose candidates crowd into few of
+    the lists.  A quarter more than the gather path is allowed for the noise of two runs."""
+    g = _values(kind, n, torch.Generator(device="cuda").manual_seed(n))
+    provisional, gather = (_us(gd, capi, how, g, rate, 0.999) for how in (-2, -1))
+    assert provisional <= 1.25 * gather, (provisional, gather)
 
 
 def test_beside_others(gd, capi):

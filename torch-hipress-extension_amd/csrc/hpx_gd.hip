@@ -14,7 +14,7 @@
 //   select      exact k-th largest of the sample by three radix-histogram
 //               passes over the fp32 bit pattern (11+11+10 bits); no sort
 //   presample, pick   in place of these for tensors with large samples: a provisional threshold;
-//               behind the pass invert (or resample), exact and recount put the exact one in its place
+//               behind the pass invert, exact and recount put the exact one in its place
 //   stream      ONE pass over the tensor: r = g + r, store r, compare with the
 //               threshold, wave64 ballot -> one 64-bit word per 64 elements
 //               (bit i = element i), a popcount and the largest |r| per workgroup, and the
@@ -67,7 +67,8 @@ struct GdState {
   uint32_t thr_bits;  // threshold as fp32 bits (provisional path: the provisional one until the exact one is known)
   uint32_t fallback;  // provisional path: 1 when the provisional threshold turned out to lie above the exact one
   uint32_t total;     // candidates of a tensor whose cut follows on the device, left by the expand launch
-  uint32_t pad[61];
+  uint32_t crowded;   // provisional path: 1 when a wave of the pass found more candidates than its list has room for
+  uint32_t pad[60];
 };
 constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold ...
 constexpr uint32_t kWayStep = 32;         // ... whose counters lie in lines of their own, this many words apart
@@ -101,7 +102,7 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   l.state = at;   at += align256(sizeof(GdState));
   l.hist = at;    at += align256(sizeof(uint32_t) * kHistWords);
   l.samples = at; at += align256(sizeof(uint32_t) * size_t(sample_cnt));
-  l.hitlist = at; at += align256(sizeof(uint32_t) * (size_t(sample_cnt) + size_t(256) * 128));  // provisional path, see gd_resample_kernel
+  l.hitlist = at; at += align256(sizeof(uint32_t) * (size_t(sample_cnt) + size_t(256) * 128));  // provisional path, see hit_way_room
   l.masks = at;   at += align256(sizeof(uint64_t) * ntiles * kWave);      // one bit per element
   l.coarse = at;  at += align256(sizeof(uint64_t) * ntiles);              // one bit per mask word: whether it has a bit set
   l.cnt = at;     at += align256(sizeof(uint32_t) * ntiles);              // candidates per tile
@@ -336,8 +337,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<
 // instead - taken from the first samples only (pre_samples) and set low enough that it all but certainly lies below the
 // exact one - so the pass lists and marks a superset of the candidates.  Every sample whose value exceeds the
 // provisional threshold is then among these, so the exact threshold (the thr_index-th largest of ALL samples) is found
-// among the candidates that are samples: by asking each of them (gd_invert_kernel), or for smaller tensors by looking
-// each sample up in the bit mask (gd_resample_kernel).  A last small launch drops the candidates that do not exceed
+// among the candidates that are samples (gd_invert_kernel).  A last small launch drops the candidates that do not exceed
 // the exact threshold; expand goes on as ever.  Should fewer than thr_index + 1 samples exceed the provisional
 // threshold (it was not below the exact one, or they tie above zero), the tensor is reported as kFallback and the host
 // sends it through the gather path, on the residual the pass has already updated.
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
   auto settle = [&](uint32_t key) {  // one lane
     GdState* st = seg_state(sg);
     st->thr_bits = key;
-    if (PROV) st->fallback = 0;
+    if (PROV) st->fallback = st->crowded = 0;
   };
   if (PROV && t < uint32_t(kHitWays)) reinterpret_cast<uint32_t*>(sg.ws + l.hist)[t * kWayStep] = 0;
   // the lane's three largest keys
@@ -732,54 +732,25 @@ __global__ __launch_bounds__(kThreads) void gd_prepick_kernel(const GdArgs<CAP> 
     const uint32_t found = workgroup_rank<int(4 * kRounds), 13, kThreads / kWave>(key, rank, 0u, s_part);
     if (t == 0) {
       seg_state(sg)->thr_bits = found;
-      seg_state(sg)->fallback = 0;
+      seg_state(sg)->fallback = seg_state(sg)->crowded = 0;
     }
   };
   if (quads <= 2 * kThreads) settle(std::integral_constant<uint32_t, 2>{}); else settle(std::integral_constant<uint32_t, 4>{});
 }
 
-// All samples against the bit mask the pass left: the values of those whose bit is set are listed.  The list is
-// kept in kHitWays parts, workgroup b appending to part b % kHitWays (one counter for all would take the few
-// thousand appends one after the other, 37 ns each); a part has room for every sample its workgroups look at.
-__host__ __device__ inline uint32_t hit_way_room(uint32_t sample_cnt) {
-  const uint32_t blocks = cdiv(sample_cnt, kThreads);
-  return cdiv(blocks, kHitWays) * uint32_t(kThreads);
-}
-template <int CAP>
-__global__ __launch_bounds__(kThreads) void gd_resample_kernel(const GdArgs<CAP> a) {
-  const int tile = blockIdx.x;
-  const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
-  const GdSeg& sg = a.seg[s];
-  const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
-  const uint64_t* __restrict__ masks = reinterpret_cast<const uint64_t*>(sg.ws + l.masks);
-  const uint32_t blk = uint32_t(tile - a.tile_start[s]);
-  const uint32_t way = blk % uint32_t(kHitWays);
-  uint32_t* hits = reinterpret_cast<uint32_t*>(sg.ws + l.hitlist) + size_t(way) * hit_way_room(sg.sample_cnt);
-  uint32_t* counter = reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way * kWayStep;
-  const uint32_t x = blk * kThreads + threadIdx.x;
-  bool hit = false;
-  uint32_t i = 0;
-  if (x < sg.sample_cnt) {
-    i = sample_index(sg.seed, x, sg.n);
-    // first whether the element's mask word has any bit at all (one bit per word: the whole map stays in cache),
-    // and only then the word itself
-    const uint64_t* __restrict__ coarse = reinterpret_cast<const uint64_t*>(sg.ws + l.coarse);
-    if ((coarse[i >> 12] >> ((i >> 6) & 63u)) & 1ull) hit = (masks[i >> 6] >> (i & 63u)) & 1ull;
-  }
-  const uint64_t m = __ballot(hit);
-  if (m == 0) return;
-  const uint32_t lane = threadIdx.x & (kWave - 1);
-  uint32_t base = 0;
-  if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(counter, uint32_t(__popcll(m)));
-  base = __shfl(base, __builtin_ctzll(m), kWave);
-  if (hit) hits[base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = __float_as_uint(__builtin_fabsf(sg.r[i]));
-}
-
-// The other way round, for large tensors: no sample is looked up, each of the pass's few candidates works out how often it was
+// The candidates that are samples, listed with their values, in one of two ways.
+//
+// Large tensors look no sample up: each of the pass's few candidates works out how often it was
 // sampled.  Sample x is element (A (x + seed) + B mod 2^32) mod n, and A is odd: an element i is the sample of the x for
 // which that word is one of i, i + n, i + 2 n, ..., and from one of these words to the next x advances by n / A mod
 // 2^32.  2^32 / n additions and compares for each candidate, 32 for 138 M elements: for its 360 thousand candidates
 // this launch takes 7 us, the look-up of its 1.4 million samples took 13.  Four lanes to a list, as in the expand launch.
+//
+// Where a list was too short for its candidates (the large values lie together: whole rows of an embedding's gradient),
+// and in small tensors, where a candidate's steps are many, every sample is looked up in the bit mask instead.  That is the
+// same work wherever the candidates lie.  When a wave walked the masks of such tiles instead, thousands of candidates of 2^32 / n
+// steps each, this launch took 782 us for 17 M elements, half of the large ones among them within one element in 1500, and
+// 271 for 138 M; now 12 and 14.5.  The whole call: 927 -> 150 and 792 -> 518 us, 150 and 556 through the gather path.
 constexpr uint32_t kInverseFrom = 1u << 24;   // elements: 256 steps a candidate
 __host__ __device__ constexpr uint32_t odd_inverse(uint32_t a) {
   uint32_t v = a;                             // right to 3 bits; each step doubles them
@@ -788,6 +759,14 @@ __host__ __device__ constexpr uint32_t odd_inverse(uint32_t a) {
 }
 constexpr uint32_t kLcgInverse = odd_inverse(lcg_mul(2));
 static_assert(kLcgInverse * lcg_mul(2) == 1u, "the multiplier has an inverse mod 2^32");
+// What is found goes to one of kHitWays parts of a list (one counter for all would take the few thousand appends one after
+// the other, 37 ns each): samples 256 b to 256 b + 255 to part b % kHitWays, which has room for all of them, or the candidates of
+// workgroup b.
+__host__ __device__ inline uint32_t hit_way_room(uint32_t sample_cnt) {
+  const uint32_t blocks = cdiv(sample_cnt, kThreads);
+  return cdiv(blocks, kHitWays) * uint32_t(kThreads);
+}
+constexpr int kLook = 4;   // blocks of samples a workgroup looks up together, so that their loads are in flight together
 template <int CAP>
 __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a) {
   const int blk = blockIdx.x;
@@ -802,16 +781,55 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
   const uint2* __restrict__ list = seg_list(sg, l) + size_t(mine) * room;
   uint2 p[kListAhead];
   uint32_t listed = 0;
-  if (my_tile) {
+  if (n >= kInverseFrom && my_tile) {
     listed = reinterpret_cast<const uint16_t*>(sg.ws + l.wcnt)[mine];
     if (room != 0) {
 #pragma unroll
       for (uint32_t q = 0; q < kListAhead; q++) p[q] = list[q * kListLanes + sub];
     }
   }
-  const uint32_t way = own % uint32_t(kHitWays), way_room = hit_way_room(sg.sample_cnt);
-  uint32_t* hits = reinterpret_cast<uint32_t*>(sg.ws + l.hitlist) + size_t(way) * way_room;
-  uint32_t* counter = reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way * kWayStep;
+  const uint32_t way_room = hit_way_room(sg.sample_cnt);
+  auto append = [&](uint32_t way, bool hit, uint32_t key) {   // by all lanes
+    const uint64_t m = __ballot(hit);
+    if (m == 0) return;
+    uint32_t base = 0;
+    if (lane == uint32_t(__builtin_ctzll(m)))
+      base = atomicAdd(reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way * kWayStep, uint32_t(__popcll(m)));
+    base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+    if (!hit) return;
+    if (base < way_room) reinterpret_cast<uint32_t*>(sg.ws + l.hitlist)[size_t(way) * way_room + base] = key;
+    else seg_state(sg)->fallback = 1;
+  };
+  if (n < kInverseFrom || seg_state(sg)->crowded) {   // uniform
+    const uint64_t* __restrict__ masks = reinterpret_cast<const uint64_t*>(sg.ws + l.masks);
+    const uint64_t* __restrict__ coarse = reinterpret_cast<const uint64_t*>(sg.ws + l.coarse);
+    const uint32_t blocks = cdiv(sg.sample_cnt, kThreads), groups = uint32_t(a.tile_start[s + 1] - a.tile_start[s]);
+#pragma unroll 1
+    for (uint32_t b = own; b < blocks; b += kLook * groups) {
+      uint32_t i[kLook], key[kLook];
+      uint64_t c[kLook], m[kLook];
+      bool hit[kLook];
+      // first whether the element's mask word has any bit at all (one bit per word: the whole map stays in cache),
+      // and only then the word itself, and the value
+#pragma unroll
+      for (uint32_t q = 0; q < uint32_t(kLook); q++) {
+        const uint64_t x = (uint64_t(b) + uint64_t(q) * groups) * kThreads + threadIdx.x;
+        hit[q] = x < sg.sample_cnt;
+        i[q] = sample_index(sg.seed, uint32_t(x), n);
+        c[q] = hit[q] ? coarse[i[q] >> 12] : 0ull;
+      }
+#pragma unroll
+      for (int q = 0; q < kLook; q++) m[q] = (c[q] >> ((i[q] >> 6) & 63u)) & 1ull ? masks[i[q] >> 6] : 0ull;
+#pragma unroll
+      for (int q = 0; q < kLook; q++) {
+        hit[q] = (m[q] >> (i[q] & 63u)) & 1ull;
+        key[q] = hit[q] ? __float_as_uint(sg.r[i[q]]) & 0x7FFFFFFFu : 0u;
+      }
+#pragma unroll
+      for (int q = 0; q < kLook; q++) append((b + uint32_t(q) * groups) % uint32_t(kHitWays), hit[q], key[q]);
+    }
+    return;
+  }
   const uint32_t steps = 0xFFFFFFFFu / n, step = kLcgInverse * n, last = 0xFFFFFFFFu - steps * n;
   auto sampled = [&](uint32_t i) {
     uint32_t x = kLcgInverse * (i - lcg_add(2)) - sg.seed, times = 0;
@@ -820,39 +838,17 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
     return times + (i <= last && x < sg.sample_cnt ? 1u : 0u);
   };
   auto note = [&](uint32_t times, uint32_t key) {
-    for (uint64_t m = __ballot(times != 0); m != 0; m = __ballot(times != 0)) {
-      uint32_t base = 0;
-      if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(counter, uint32_t(__popcll(m)));
-      base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
-      if (times != 0) {
-        if (base < way_room) hits[base] = key; else seg_state(sg)->fallback = 1;
-        times--;
-      }
-    }
+    for (; __ballot(times != 0) != 0; times -= times != 0 ? 1u : 0u) append(own % uint32_t(kHitWays), times != 0, key);
   };
-  if (room != 0 && __ballot(listed > room) == 0) {
-    uint32_t times[kListAhead];
+  uint32_t times[kListAhead];
 #pragma unroll
-    for (uint32_t q = 0; q < kListAhead; q++) times[q] = q * kListLanes + sub < listed ? sampled(p[q].x) : 0u;
+  for (uint32_t q = 0; q < kListAhead; q++) times[q] = q * kListLanes + sub < listed ? sampled(p[q].x) : 0u;
 #pragma unroll
-    for (uint32_t q = 0; q < kListAhead; q++) note(times[q], p[q].y & 0x7FFFFFFFu);
-    for (uint32_t j = kListAhead * kListLanes; __ballot(j < listed) != 0; j += kListLanes) {
-      const bool any = j + sub < listed;
-      const uint2 e = any ? list[j + sub] : make_uint2(0, 0);
-      note(any ? sampled(e.x) : 0u, e.y & 0x7FFFFFFFu);
-    }
-    return;
-  }
-  // A list too short for its candidates: those of these tiles by the masks.
-  const uint64_t* __restrict__ masks = reinterpret_cast<const uint64_t*>(sg.ws + l.masks);
-  for (uint32_t tile = tile0; tile < tile0 + kListTiles && tile < ntiles; tile++) {
-    uint64_t m = masks[size_t(tile) * kWave + lane];
-    while (__ballot(m != 0) != 0) {
-      const uint32_t i = tile * uint32_t(kTile) + lane * kWave + uint32_t(m ? __builtin_ctzll(m) : 0);
-      const uint32_t times = m ? sampled(i) : 0u;
-      note(times, times ? __float_as_uint(sg.r[i]) & 0x7FFFFFFFu : 0u);
-      m &= m - 1;
-    }
+  for (uint32_t q = 0; q < kListAhead; q++) note(times[q], p[q].y & 0x7FFFFFFFu);
+  for (uint32_t j = kListAhead * kListLanes; __ballot(j < listed) != 0; j += kListLanes) {
+    const bool any = j + sub < listed;
+    const uint2 e = any ? list[j + sub] : make_uint2(0, 0);
+    note(any ? sampled(e.x) : 0u, e.y & 0x7FFFFFFFu);
   }
 }
 
@@ -925,6 +921,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_exact_kernel(const GdArgs<CAP>
   }
 }
 
+constexpr int kRecountWords = 32;
 // What exceeds the provisional threshold but not the exact one goes: out of the lists, in place, four lanes to each; where
 // the expand launch will look at the masks, because a list of its wave's is too short, out of those.
 template <int CAP>
@@ -982,30 +979,49 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
 #pragma unroll
     for (int o = kTileLanes; o < kWave; o <<= 1) c += __shfl_xor(c, o, kWave);
     all = c;
-  } else for (uint32_t tile = tile0; tile < tile0 + kListTiles && tile < ntiles; tile++) {
-    // A mask word per lane, the value of a word's first set bit loaded for all lanes together.
-    if (cnt[tile] == 0) continue;  // wave-uniform
-    const uint64_t old = masks[size_t(tile) * kWave + lane];
-    const uint32_t e0 = tile * uint32_t(kTile) + lane * kWave;
-    uint64_t m = old, keep = 0;
-    const uint32_t b1 = m ? uint32_t(__builtin_ctzll(m)) : 0u;
-    const float v1 = m ? r[e0 + b1] : 0.0f;
-    if (m) {
-      if (v1 > thr || v1 < nthr) keep |= 1ull << b1;
-      m &= m - 1;
-    }
-    while (m) {
-      const uint32_t b = uint32_t(__builtin_ctzll(m));
-      m &= m - 1;
-      const float v = r[e0 + b];
-      if (v > thr || v < nthr) keep |= 1ull << b;
-    }
-    if (keep != old) masks[size_t(tile) * kWave + lane] = keep;
-    uint32_t c = uint32_t(__popcll(keep));
+  } else {
+    // A mask word per lane; then its 64 elements lane by lane, kRecountWords words' values requested together: a tile full
+    // of candidates takes two rounds (with each lane walking its own word's bits this launch took 29 us for the 17 M elements
+    // of gd_invert_kernel's comment, now 23.5; 47.5 and 32 for its 138 M).
+    uint64_t word[kListTiles];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, kWave);
-    if (lane == 0) cnt[tile] = c;
-    all += c;
+    for (uint32_t j = 0; j < kListTiles; j++) word[j] = tile0 + j < ntiles ? masks[size_t(tile0 + j) * kWave + lane] : 0ull;
+#pragma unroll 1
+    for (uint32_t j = 0; j < kListTiles; j++) {
+      const uint32_t tile = tile0 + j;
+      const uint64_t old = j == 0 ? word[0] : j == 1 ? word[1] : j == 2 ? word[2] : word[3];
+      static_assert(kListTiles == 4, "the words above");
+      auto bit = [&](uint32_t w) {   // whether the lane's element of word w is a candidate
+        const uint64_t m = uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(old)), int(w)))) |
+                           uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(old >> 32)), int(w)))) << 32;
+        return ((m >> lane) & 1ull) != 0;
+      };
+      uint64_t keep = 0, left = __ballot(old != 0);
+      if (left == 0) continue;   // wave-uniform
+      do {
+        uint64_t now = left;
+        float v[kRecountWords];
+#pragma unroll
+        for (int q = 0; q < kRecountWords; q++) {   // no branches, so that nothing is waited for in between
+          const uint32_t w = left ? uint32_t(__builtin_ctzll(left)) : 0u;
+          v[q] = left != 0 && bit(w) ? r[tile * uint32_t(kTile) + w * kWave + lane] : 0.0f;
+          left &= left - 1;   // 0 stays 0
+        }
+#pragma unroll
+        for (int q = 0; q < kRecountWords; q++) {
+          const uint32_t w = now ? uint32_t(__builtin_ctzll(now)) : uint32_t(kWave);
+          const uint64_t k = __ballot(v[q] > thr || v[q] < nthr);   // a threshold is not negative: zero does not pass
+          keep = lane == w ? k : keep;
+          now &= now - 1;
+        }
+      } while (left);
+      if (keep != old) masks[size_t(tile) * kWave + lane] = keep;
+      uint32_t c = uint32_t(__popcll(keep));
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, kWave);
+      if (lane == 0) cnt[tile] = c;
+      all += c;
+    }
   }
   // The group's total and largest |r|, from which the expand launch works its places out: a scan launch before it took 6.5 us
   // of a call with its hand-over.
@@ -1103,6 +1119,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
     }
   }
   if (lane < kPerLane) masks[(size_t(wbase) >> 6) + lane] = (uint64_t(hi) << 32) | lo;
+  if (PROV && cnt > room && lane == 0) seg_state(sg)->crowded = 1;   // all of them store the same
   // which of the wave's sixteen mask words have a bit set (lanes beyond the sixteenth hold zeros)
   const uint32_t any16 = uint32_t(__ballot((lo | hi) != 0u));
   uint32_t bigb = __float_as_uint(big);  // non-negative floats order like their bit patterns; a NaN is not an input
@@ -2547,10 +2564,8 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     else
       HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<true, CAP>), grid, dim3(kSelThreads), st, a);
     stream_pass();
-    grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? cdiv(sg.sample_cnt, kThreads) : 0u; });
-    if (grid.x) HPX_LAUNCH("gd_resample_kernel", gd_resample_kernel<CAP>, grid, dim3(kThreads), st, a);
-    grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? 0u : cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
-    if (grid.x) HPX_LAUNCH("gd_invert_kernel", gd_invert_kernel<CAP>, grid, dim3(kThreads), st, a);
+    grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? cdiv(sg.sample_cnt, kThreads) : cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
+    HPX_LAUNCH("gd_invert_kernel", gd_invert_kernel<CAP>, grid, dim3(kThreads), st, a);
     HPX_LAUNCH("gd_exact_kernel", gd_exact_kernel<CAP>, dim3(uint32_t(count)), dim3(kSelThreads), st, a);
     grid = tiles([](const GdSeg& sg) { return cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
     HPX_LAUNCH("gd_recount_kernel", gd_recount_kernel<CAP>, grid, dim3(kThreads), st, a);
