@@ -37,6 +37,13 @@ def _values(kind, n, gen):
         g = torch.round(g * 8) / 8
     elif kind == "signs":          # all of one size: nothing lies above the threshold
         g = torch.sign(g)
+    elif kind == "scaled":         # the same of a size with all its bits, some of them zero
+        g = torch.sign(g) * 0.0123
+        g[::7] = 0
+    elif kind in ("astride", "edge", "short"):   # one element in 500 of one size, some larger: fewer than are kept, as many, more
+        u = torch.empty(n, device="cuda").uniform_(0, 1, generator=gen)
+        share = {"astride": 6e-4, "edge": 1e-3, "short": 1.25e-3}[kind]
+        g = torch.where(u < share, 2 + g, torch.where(u < share + 2e-3, torch.sign(g) * 0.77, 0.5 * g))
     elif kind == "infinite":
         g[::5003] = float("inf"); g[::7001] = float("-inf")
     elif kind == "nan":            # some, so that they move the threshold's rank
@@ -90,13 +97,15 @@ def test_sizes(gd, capi, n, rate, kept, path):
         assert (inverted, fell_back) == (int(path), 0)
 
 
-@pytest.mark.parametrize("kind,fallback", [("crowded", 0), ("rows", 0), ("sparse", 0), ("coarse", 1), ("signs", 1), ("infinite", 0), ("nan", None), ("all_nan", None)])
+@pytest.mark.parametrize("kind,fallback", [("crowded", 0), ("rows", 0), ("sparse", 0), ("coarse", 0), ("signs", 0), ("scaled", 0), ("astride", 0), ("edge", 0),
+                                           ("short", 0), ("infinite", 0), ("nan", None), ("all_nan", None)])
 def test_values(gd, capi, kind, fallback):
     n = 20_000_003
     gen = torch.Generator(device="cuda").manual_seed(7)
     g, r = _values(kind, n, gen), torch.zeros(n, device="cuda")
-    inverted, fell_back = _compare(gd, capi, [g], [r], [0.05], [0.999], [11])
-    assert inverted == 1 and (fallback is None or fell_back == fallback)
+    for seed in (11, 12, 13):
+        inverted, fell_back = _compare(gd, capi, [g], [r], [0.05], [0.999], [seed])
+        assert inverted == 1 and (fallback is None or fell_back == fallback)
 
 
 def _us(gd, capi, how, g, rate, drop):
@@ -116,11 +125,11 @@ def _us(gd, capi, how, g, rate, drop):
     return least
 
 
-@pytest.mark.parametrize("kind", ["crowded", "rows"])
+@pytest.mark.parametrize("kind", ["crowded", "rows", "coarse", "signs", "scaled", "astride"])
 @pytest.mark.parametrize("n,rate", [(FIRST, 0.05), (FIRST + 1, 0.05), (60_000_000, 0.02), (60_000_001, 0.02)])
-def test_large_values_that_lie_together_take_no_longer(gd, capi, kind, n, rate):
+def test_crowds_and_equal_values_take_no_longer(gd, capi, kind, n, rate):
     """The path is there because it is quicker: it has to be for these tensors as well, whose candidates crowd into few of
-    the lists.  A quarter more than the gather path is allowed for the noise of two runs."""
+    the lists, or whose threshold is a value that many elements share.  A quarter more than the gather path is allowed for the noise of two runs."""
     g = _values(kind, n, torch.Generator(device="cuda").manual_seed(n))
     provisional, gather = (_us(gd, capi, how, g, rate, 0.999) for how in (-2, -1))
     assert provisional <= 1.25 * gather, (provisional, gather)

@@ -63,12 +63,13 @@ constexpr int kHistWords = kBins1 + kBins2 + kBins3;
 constexpr int kCapLarge = 256;                   // tensors per launch table (17 KiB of kernel arguments)
 constexpr int kCapSmall = 4;                     // calls with a few tensors pass a table of a few hundred bytes
 
-struct GdState {
+struct alignas(16) GdState {
   uint32_t thr_bits;  // threshold as fp32 bits (provisional path: the provisional one until the exact one is known)
   uint32_t fallback;  // provisional path: 1 when the provisional threshold turned out to lie above the exact one
+  uint32_t crowded;   // ... 1 when a wave of the pass found more candidates than its list has room for
+  uint32_t ties;      // ... and 1 when the provisional threshold is a value that many samples share
   uint32_t total;     // candidates of a tensor whose cut follows on the device, left by the expand launch
-  uint32_t crowded;   // provisional path: 1 when a wave of the pass found more candidates than its list has room for
-  uint32_t pad[60];
+  uint32_t pad[59];
 };
 constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold ...
 constexpr uint32_t kWayStep = 32;         // ... whose counters lie in lines of their own, this many words apart
@@ -338,9 +339,20 @@ __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<
 // exact one - so the pass lists and marks a superset of the candidates.  Every sample whose value exceeds the
 // provisional threshold is then among these, so the exact threshold (the thr_index-th largest of ALL samples) is found
 // among the candidates that are samples (gd_invert_kernel).  A last small launch drops the candidates that do not exceed
-// the exact threshold; expand goes on as ever.  Should fewer than thr_index + 1 samples exceed the provisional
-// threshold (it was not below the exact one, or they tie above zero), the tensor is reported as kFallback and the host
-// sends it through the gather path, on the residual the pass has already updated.
+// the exact threshold; expand goes on as ever.
+//
+// Values that many elements share (signs, a few levels: gradients that were quantised) may leave the two thresholds equal.  A
+// provisional threshold with too many equal samples about it is therefore that value itself, to the last bit (gd_prepick_kernel),
+// so that the elements that share it are no candidates, and where so few samples lie above it that it may be the exact one the
+// samples equal to it are counted behind the pass (gd_invert_kernel reads all of them, a line of r each): with those above it they
+// say that it is.  (Cut off below ten bits as ever it let the sharing elements through, every element of a tensor of signs
+// of size 0.0123, or where those bits are zero did not lie below the exact one and the tensor was encoded again.  us per call at 17 M /
+// 60 M / 138 M elements: signs of size 0.0123 3494 / 892 / 1130, now 96 / 174 / 340, signs of size 1 170 / 276 / 494, now 97 / 174 / 342;
+// through the gather path 142 / 240 / 427.)
+//
+// Should fewer than thr_index + 1 samples reach the provisional threshold (it lies above the exact one), or should it be a NaN,
+// the tensor is reported as kFallback and the host sends it through the gather path, on the residual the pass has already
+// updated.
 //
 // How many samples the provisional threshold is taken from, and its rank among them.  Without a margin from the caller:
 // as many that kPreExpected of them should lie above the exact threshold, and kPreLeast, at a rank eight standard deviations
@@ -363,6 +375,11 @@ __device__ inline uint32_t pre_rank(uint32_t sample_cnt, uint32_t thr_index, int
     kp = (uint64_t(margin) * (uint64_t(thr_index) + 1) * s0 + sample_cnt - 1) / sample_cnt + 8;
   }
   return kp > s0 - 1 ? s0 - 1 : uint32_t(kp);
+}
+
+// How far the number of samples above a threshold strays: four standard deviations, half the provisional threshold's distance.
+__device__ inline uint32_t pre_slack(uint32_t sample_cnt, uint32_t thr_index, uint32_t s0) {
+  return uint32_t(4.0f * __builtin_sqrtf(float(thr_index + 1) * (float(s0) / float(sample_cnt))) + 4.0f);
 }
 
 // With that choice each wave of the launch that gathers the samples leaves its kPreTop largest only.  It holds one key above the
@@ -448,8 +465,11 @@ __device__ __forceinline__ uint32_t sum_of_waves(uint32_t v) {
   return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
 }
 // wave_rank over keys of a whole workgroup of WAVES waves, R a lane: a barrier a bit.  s_part: two rows of a word per wave.
-template <int R, int LO = 0, int WAVES = kSelThreads / kWave>
-__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor, uint32_t (*s_part)[WAVES]) {
+// `stop` is asked before each bit whether the bits so far will do: with how many keys reach what they give (zeros for the rest),
+// and how many reach the next such value; on return `above` is the latter.
+template <int R, int WAVES, typename Stop>
+__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor, uint32_t (*s_part)[WAVES],
+                                                   uint32_t& above, Stop stop) {
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   uint32_t top = 0;
 #pragma unroll
@@ -464,19 +484,27 @@ __device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uin
   floor = __builtin_amdgcn_readfirstlane(floor);
   const int first = 31 - __builtin_clz((top ^ floor) | 1u);   // bits above it are common to every candidate
   uint32_t t = first < 31 ? (floor >> (first + 1)) << (first + 1) : 0u;
-  t = LO > 0 ? (t >> LO) << LO : t;
+  uint32_t least = R * WAVES * kWave;   // keys that reach t
+  above = 0;
   int row = 1;
 #pragma unroll 1
-  for (int b = first < 30 ? first : 30; b >= LO; b--, row ^= 1) {
+  for (int b = first < 30 ? first : 30; b >= 0; b--, row ^= 1) {
+    if (stop(b, least, above)) break;
     const uint32_t c = t | (1u << b);
     uint32_t reach = 0;
 #pragma unroll
     for (int j = 0; j < R; j++) reach += uint32_t(__popcll(__ballot(key[j] >= c)));
     if (lane == 0) s_part[row][wave] = reach;
     __syncthreads();   // the row before it is not written again before everyone is past this one
-    if (sum_of_waves<WAVES>(s_part[row][lane % WAVES]) > rank) t = c;
+    reach = sum_of_waves<WAVES>(s_part[row][lane % WAVES]);
+    if (reach > rank) { t = c; least = reach; } else above = reach;   // the last that failed is t and one more in the last place
   }
   return t;
+}
+template <int R, int WAVES = kSelThreads / kWave>
+__device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uint32_t rank, uint32_t floor, uint32_t (*s_part)[WAVES]) {
+  uint32_t above;
+  return workgroup_rank(key, rank, floor, s_part, above, [](int, uint32_t, uint32_t) { return false; });
 }
 template <bool PROV, int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> a) {
@@ -493,9 +521,9 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
   auto settle = [&](uint32_t key) {  // one lane
     GdState* st = seg_state(sg);
     st->thr_bits = key;
-    if (PROV) st->fallback = st->crowded = 0;
+    if (PROV) st->fallback = st->crowded = st->ties = 0;
   };
-  if (PROV && t < uint32_t(kHitWays)) reinterpret_cast<uint32_t*>(sg.ws + l.hist)[t * kWayStep] = 0;
+  if (PROV && t < uint32_t(kHitWays)) *reinterpret_cast<uint2*>(sg.ws + l.hist + t * kWayStep * sizeof(uint32_t)) = make_uint2(0, 0);
   // the lane's three largest keys
   uint32_t m1 = 0, m2 = 0, m3 = 0;
   auto take = [&](uint32_t k) {
@@ -709,15 +737,18 @@ __global__ __launch_bounds__(kThreads) void gd_presample_kernel(const GdArgs<CAP
 }
 
 // The provisional threshold from what the waves of that launch have left, by one workgroup of four waves for each tensor: the
-// key of the rank wanted, cut off below ten bits of mantissa (a lower threshold will do).  Its code is short because it is
+// key of the rank wanted, cut off below ten bits of mantissa (a lower threshold will do) unless a crowd of keys shares these,
+// too many for all of them to lie above the exact threshold by chance: then to the last bit.  Its code is short because it is
 // fetched anew in every call, and a barrier a bit is cheap among four waves: with all samples ranked by gd_pick_kernel this
-// launch took 7.3 us, and 13 in two calls of five; by sixteen waves 6.8; now 5.2 (138 M elements, 32 thousand samples).
+// launch took 7.3 us, and 13 in two calls of five; by sixteen waves 6.8; now 5.2, and 5.6 since it looks for
+// crowds (138 M elements, 32 thousand samples).
 template <int CAP>
 __global__ __launch_bounds__(kThreads) void gd_prepick_kernel(const GdArgs<CAP> a) {
   __shared__ uint32_t s_part[2][kThreads / kWave];
   const GdSeg& sg = a.seg[blockIdx.x];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index, a.margin), rank = pre_rank(sg.sample_cnt, sg.thr_index, a.margin, s0);
+  const uint32_t slack = pre_slack(sg.sample_cnt, sg.thr_index, s0);
   const uint32_t quads = cdiv(s0, kWave) * (kPreTop / 4), t = threadIdx.x;
   const uint4* __restrict__ left = reinterpret_cast<const uint4*>(sg.ws + l.samples);
   auto settle = [&](auto rounds) {
@@ -728,11 +759,17 @@ __global__ __launch_bounds__(kThreads) void gd_prepick_kernel(const GdArgs<CAP> 
       const uint4 q = j * kThreads + t < quads ? left[j * kThreads + t] : make_uint4(0, 0, 0, 0);
       key[4 * j] = q.x; key[4 * j + 1] = q.y; key[4 * j + 2] = q.z; key[4 * j + 3] = q.w;
     }
-    if (t < uint32_t(kHitWays)) reinterpret_cast<uint32_t*>(sg.ws + l.hist)[t * kWayStep] = 0;
-    const uint32_t found = workgroup_rank<int(4 * kRounds), 13, kThreads / kWave>(key, rank, 0u, s_part);
+    if (t < uint32_t(kHitWays)) *reinterpret_cast<uint2*>(sg.ws + l.hist + t * kWayStep * sizeof(uint32_t)) = make_uint2(0, 0);
+    uint32_t above;
+    const uint32_t found = workgroup_rank(key, rank, 0u, s_part, above,
+                                          [=](int b, uint32_t least, uint32_t above) { return b == 12 && least - above <= slack; });
     if (t == 0) {
-      seg_state(sg)->thr_bits = found;
-      seg_state(sg)->fallback = seg_state(sg)->crowded = 0;
+      GdState* st = seg_state(sg);
+      st->thr_bits = found;
+      st->fallback = found > 0x7F800000u ? 1u : 0u;   // a NaN: every element would be a candidate, and which of them are above it?
+      st->crowded = 0;
+      // so few samples above it that it may be the exact one; zero need not be counted, nothing lies below it
+      st->ties = found != 0 && float(above) < float(sg.thr_index + 1) * (float(s0) / float(sg.sample_cnt)) + float(slack) ? 1u : 0u;
     }
   };
   if (quads <= 2 * kThreads) settle(std::integral_constant<uint32_t, 2>{}); else settle(std::integral_constant<uint32_t, 4>{});
@@ -774,6 +811,7 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
   const GdSeg& sg = a.seg[s];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   const uint32_t n = sg.n, ntiles = cdiv(n, kTile), lane = threadIdx.x & (kWave - 1);
+  const uint4 st = *reinterpret_cast<const uint4*>(seg_state(sg));   // GdState's first four words, uniform
   const uint32_t own = uint32_t(blk - a.tile_start[s]);
   const uint32_t tile0 = (own * (kThreads / kWave) + threadIdx.x / kWave) * kListTiles;
   const uint32_t room = list_room(n, sg.limit), sub = lane % kListLanes, mine = tile0 * (kThreads / kWave) + lane / kListLanes;
@@ -800,10 +838,36 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
     if (base < way_room) reinterpret_cast<uint32_t*>(sg.ws + l.hitlist)[size_t(way) * way_room + base] = key;
     else seg_state(sg)->fallback = 1;
   };
-  if (n < kInverseFrom || seg_state(sg)->crowded) {   // uniform
+  if (st.y) return;   // fallback: a NaN, or noted by a wave before; what is listed will not be used
+  const uint32_t blocks = cdiv(sg.sample_cnt, kThreads), groups = uint32_t(a.tile_start[s + 1] - a.tile_start[s]);
+  if (st.w) {   // ties
+    const uint32_t thr_bits = st.x;
+    const float thr = __uint_as_float(thr_bits);
+    uint32_t equal = 0;   // the wave's
+#pragma unroll 1
+    for (uint32_t b = own; b < blocks; b += kLook * groups) {
+      float v[kLook];
+      bool any[kLook];
+#pragma unroll
+      for (uint32_t q = 0; q < uint32_t(kLook); q++) {
+        const uint64_t x = (uint64_t(b) + uint64_t(q) * groups) * kThreads + threadIdx.x;
+        any[q] = x < sg.sample_cnt;
+        v[q] = any[q] ? sg.r[sample_index(sg.seed, uint32_t(x), n)] : 0.0f;
+      }
+#pragma unroll
+      for (int q = 0; q < kLook; q++) {
+        const uint32_t key = __float_as_uint(v[q]) & 0x7FFFFFFFu;
+        equal += uint32_t(__popcll(__ballot(any[q] && key == thr_bits)));
+        append((b + uint32_t(q) * groups) % uint32_t(kHitWays), any[q] && !(__builtin_fabsf(v[q]) <= thr), key);
+      }
+    }
+    if (lane == 0 && equal != 0)
+      atomicAdd(reinterpret_cast<uint32_t*>(sg.ws + l.hist) + own % uint32_t(kHitWays) * kWayStep + 1, equal);
+    return;
+  }
+  if (n < kInverseFrom || st.z) {   // crowded
     const uint64_t* __restrict__ masks = reinterpret_cast<const uint64_t*>(sg.ws + l.masks);
     const uint64_t* __restrict__ coarse = reinterpret_cast<const uint64_t*>(sg.ws + l.coarse);
-    const uint32_t blocks = cdiv(sg.sample_cnt, kThreads), groups = uint32_t(a.tile_start[s + 1] - a.tile_start[s]);
 #pragma unroll 1
     for (uint32_t b = own; b < blocks; b += kLook * groups) {
       uint32_t i[kLook], key[kLook];
@@ -897,8 +961,13 @@ __global__ __launch_bounds__(kSelThreads) void gd_exact_kernel(const GdArgs<CAP>
   const uint32_t found = __builtin_amdgcn_readlane(incl, kWave - 1);
   __syncthreads();   // nobody reads the state below
   if (found <= sg.thr_index) {
-    // all other samples are at most the provisional threshold: nothing is less than zero, so that one is known
-    if (t == 0 && prov != 0) st->fallback = 1;
+    // all other samples are at most the provisional threshold: it is the exact one if enough of them are equal to it (nothing is
+    // less than zero, so that one is known)
+    uint32_t equal = 0;
+    if (st->ties) equal = ways[2 * lane * kWayStep + 1] + ways[(2 * lane + 1) * kWayStep + 1];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) equal += __shfl_xor(equal, o, kWave);
+    if (t == 0 && prov != 0 && found + equal <= sg.thr_index) st->fallback = 1;
     return;
   }
   const uint32_t* part = parts + size_t(way) * room;
