@@ -95,16 +95,17 @@ int hpx_release_stream(hpx_stream_t stream);
  *                             among what the pass marked, instead of gathering
  *                             the whole sample first; the message is the same.
  *                             -2 (default): large ones with large samples, for
- *                             which that is quicker (138 M elements: 337 us
+ *                             which that is quicker (138 M elements: 331 us
  *                             instead of 377); -1: none; otherwise all of a
  *                             call whose samples add up to at least this many
  *   "gd_provisional_margin"   with such a number, how many times the expected
  *                             number of entries the provisional threshold (of
- *                             the first 16384 samples) lets through (default
- *                             3).  A tensor whose provisional threshold turns
- *                             out not to lie below the exact one is encoded
- *                             again through the gather path (hpx_gd_fallbacks
- *                             counts them); 0 all but forces that
+ *                             the first samples, 32768 or more) lets through
+ *                             (default 3).  A tensor whose provisional
+ *                             threshold turns out to lie above the exact one
+ *                             is encoded again through the gather path
+ *                             (hpx_gd_fallbacks counts them); 0 all but forces
+ *                             that
  *   "clock_seed"              what an encoder uses when it is called with
  *                             seeds == NULL; negative (default): the wall
  *                             clock, as the reference's bodies
@@ -327,8 +328,8 @@ int hpx_gd_decode(int count, const uint8_t* const* ins, const int32_t* in_sizes,
                   const int32_t* is_add_tos, hpx_stream_t stream);
 
 /* Diagnostic: tensors of sparsifier calls on `stream` so far whose provisional
- * threshold was not below the exact one and that were therefore encoded through
- * the gather path after all (see "gd_provisional_margin"). */
+ * threshold lay above the exact one, or was a NaN, and that were therefore
+ * encoded through the gather path after all (see "gd_provisional_margin"). */
 int64_t hpx_gd_fallbacks(hpx_stream_t stream);
 
 /* ---- DGC without residual --------------------------------------------------

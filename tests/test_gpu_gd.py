@@ -44,9 +44,10 @@ def gd(capi):
 @pytest.fixture(autouse=True, scope="module", params=["gather", "provisional", "provisional_fall_back"])
 def threshold_path(request, capi):
     """Every test of this module runs three times: with the threshold taken from the gathered sample before the
-    pass; with the pass started from a provisional threshold and the exact one found afterwards (an option, off by
-    default); and with the provisional threshold put at the top of its
-    samples, so that it lies above the exact one and every tensor falls back to the gather path after the pass has
+    pass; with the pass started from a provisional threshold and the exact one found afterwards, as large tensors do by
+    themselves, through the same launches (here tensors of every size, with the provisional threshold's rank by an option; with
+    the rank that large tensors choose: test_gpu_gd_provisional.py); and with the provisional threshold put at the top of
+    its samples, so that it lies above the exact one and every tensor falls back to the gather path after the pass has
     updated the residual.  The messages are the same bit for bit."""
     mode = request.param
     old = [capi.set_option("gd_provisional_min_samples", -1 if mode == "gather" else 0),
@@ -66,16 +67,16 @@ def test_the_path_under_test_is_the_one_that_runs(gd, oracle_cpu, capi, threshol
     L.hpx_profile_reset(); L.hpx_profile_enable(1)
     try:
         _check_encode(gd, oracle_cpu, g, r0, 0.01, 0.999, 5)
-        launched = {k: capi.profile_query(k)[1] for k in ("gd_sample_kernel", "gd_presample_kernel", "gd_recount_kernel")}
+        launched = {k: capi.profile_query(k)[1] for k in ("gd_sample_kernel", "gd_prepick_kernel", "gd_recount_kernel")}
     finally:
         L.hpx_profile_enable(0); L.hpx_profile_reset()
     fell_back = L.hpx_gd_fallbacks(stream_ptr()) - before
     if threshold_path == "gather":
-        assert launched == {"gd_sample_kernel": 1, "gd_presample_kernel": 0, "gd_recount_kernel": 0} and fell_back == 0
+        assert launched == {"gd_sample_kernel": 1, "gd_prepick_kernel": 0, "gd_recount_kernel": 0} and fell_back == 0
     elif threshold_path == "provisional":
-        assert launched == {"gd_sample_kernel": 0, "gd_presample_kernel": 1, "gd_recount_kernel": 1} and fell_back == 0
+        assert launched == {"gd_sample_kernel": 0, "gd_prepick_kernel": 1, "gd_recount_kernel": 1} and fell_back == 0
     else:
-        assert launched == {"gd_sample_kernel": 1, "gd_presample_kernel": 1, "gd_recount_kernel": 1} and fell_back == 1
+        assert launched == {"gd_sample_kernel": 1, "gd_prepick_kernel": 1, "gd_recount_kernel": 1} and fell_back == 1
 
 
 _BRANCHES = set()

@@ -113,7 +113,7 @@ struct Workspace {
   CompletionLog<ResidentRec, ResidentMark> resident_log;
   uint32_t* done = nullptr;  // kBarMaxWorkgroups words, see ensure_barrier
   uint64_t repaired = 0;  // tensors encoded again after an expired barrier, ever
-  uint64_t gd_fallbacks = 0;  // sparsifier tensors whose provisional threshold was not below the exact one, ever
+  uint64_t gd_fallbacks = 0;  // sparsifier tensors whose provisional threshold lay above the exact one, ever
 };
 constexpr size_t kStateWords = 4096;       // 16 KiB
 constexpr size_t kStatusWord = kStateWords - 16;  // sticky flags live here

@@ -13,7 +13,7 @@
 //               BEFORE the update (the same fp32 sum the update will store)
 //   select      exact k-th largest of the sample by three radix-histogram
 //               passes over the fp32 bit pattern (11+11+10 bits); no sort
-//   presample, pick   in place of these for tensors with large samples: a provisional threshold;
+//   presample, prepick   in place of these for tensors with large samples: a provisional threshold;
 //               behind the pass invert, exact and recount put the exact one in its place
 //   stream      ONE pass over the tensor: r = g + r, store r, compare with the
 //               threshold, wave64 ballot -> one 64-bit word per 64 elements
@@ -73,11 +73,10 @@ struct alignas(16) GdState {
 };
 constexpr int kHitWays = 128;             // parts of the list of samples above the provisional threshold ...
 constexpr uint32_t kWayStep = 32;         // ... whose counters lie in lines of their own, this many words apart
-constexpr uint32_t kPreSamples = 16384;  // samples the provisional threshold is taken from where the caller gives the margin
 constexpr int64_t kProvisionalAuto = -2;  // the option that leaves the choice to provisional_pays
 constexpr int kBySpread = 1 << 20;        // the margin where the caller gives none (see pre_samples)
-constexpr uint32_t kPreExpected = 32;     // ... and how many of these samples are expected above the exact threshold
-constexpr uint32_t kPreLeast = 32768;        // ... of at least this many
+constexpr uint32_t kPreExpected = 32;     // how many of the samples the provisional threshold is taken from are expected above the exact one
+constexpr uint32_t kPreLeast = 32768;     // ... of at least this many samples
 constexpr uint32_t kFallback = 0xFFFFFFFEu;  // reported in place of a count: this tensor has to take the other path
 constexpr int kScanChunk = 4096;   // per-tile counts scanned by one workgroup
 constexpr int kMaxChunks = 128;    // 2^31 elements / kTile / kScanChunk
@@ -354,16 +353,14 @@ __global__ __launch_bounds__(kSelThreads) void gd_threshold_kernel(const GdArgs<
 // the tensor is reported as kFallback and the host sends it through the gather path, on the residual the pass has already
 // updated.
 //
-// How many samples the provisional threshold is taken from, and its rank among them.  Without a margin from the caller:
-// as many that kPreExpected of them should lie above the exact threshold, and kPreLeast, at a rank eight standard deviations
-// beyond that, so that the exact one lies below the provisional one in a case of 10^14.  More samples let less through and take the one
-// workgroup that ranks them longer: 138 M elements, a thousandth kept, 16, 32 and 64 expected: 339, 335.4 and 335.4 us a call.
-__host__ __device__ inline uint32_t pre_samples(uint32_t sample_cnt, uint32_t thr_index, int margin) {
-  uint64_t want = kPreSamples;
-  if (margin == kBySpread) {
-    want = (uint64_t(kPreExpected) * sample_cnt / (uint64_t(thr_index) + 1) + uint64_t(kThreads) - 1) / kThreads * kThreads;
-    want = want < kPreLeast ? kPreLeast : want < kPickMax ? want : kPickMax;
-  }
+// How many samples the provisional threshold is taken from, and its rank among them: as many that kPreExpected of them should lie
+// above the exact threshold, and kPreLeast, at a rank eight standard deviations beyond that, so that the exact one lies below the
+// provisional one in a case of 10^14.  More samples let less through and take the one workgroup that ranks them longer: 138 M
+// elements, a thousandth kept, 16, 32 and 64 expected: 339, 335.4 and 335.4 us a call.  A margin from the caller gives the rank
+// in its place, as that many times the number expected.
+__host__ __device__ inline uint32_t pre_samples(uint32_t sample_cnt, uint32_t thr_index) {
+  uint64_t want = (uint64_t(kPreExpected) * sample_cnt / (uint64_t(thr_index) + 1) + uint64_t(kThreads) - 1) / kThreads * kThreads;
+  want = want < kPreLeast ? kPreLeast : want < kPickMax ? want : kPickMax;
   return sample_cnt < want ? sample_cnt : uint32_t(want);
 }
 __device__ inline uint32_t pre_rank(uint32_t sample_cnt, uint32_t thr_index, int margin, uint32_t s0) {
@@ -376,15 +373,15 @@ __device__ inline uint32_t pre_rank(uint32_t sample_cnt, uint32_t thr_index, int
   }
   return kp > s0 - 1 ? s0 - 1 : uint32_t(kp);
 }
-
 // How far the number of samples above a threshold strays: four standard deviations, half the provisional threshold's distance.
 __device__ inline uint32_t pre_slack(uint32_t sample_cnt, uint32_t thr_index, uint32_t s0) {
   return uint32_t(4.0f * __builtin_sqrtf(float(thr_index + 1) * (float(s0) / float(sample_cnt))) + 4.0f);
 }
 
-// With that choice each wave of the launch that gathers the samples leaves its kPreTop largest only.  It holds one key above the
+// Each wave of the launch that gathers the samples leaves its kPreTop largest only.  It holds one key above the
 // threshold at most on average (a rank of 490 or so among 32768 samples where one in a hundred is kept); one that holds more
-// than it leaves makes the provisional threshold a little lower, which it may be.
+// than it leaves makes the provisional threshold a little lower, which it may be (down to zero where the caller has a tensor
+// take this path that keeps one element in ten).
 constexpr uint32_t kPreTop = 4;
 static_assert(kPickMax / kWave * kPreTop <= 16 * kThreads, "what gd_prepick_kernel holds");
 
@@ -506,7 +503,7 @@ __device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uin
   uint32_t above;
   return workgroup_rank(key, rank, floor, s_part, above, [](int, uint32_t, uint32_t) { return false; });
 }
-template <bool PROV, int CAP>
+template <int CAP>
 __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> a) {
   __shared__ uint32_t s_hist[kBins1];              // the lanes' largest keys; the histogram of the other way
   __shared__ __align__(16) uint32_t s_list[kPickAll];
@@ -515,15 +512,9 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
   const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
-  const uint32_t count = PROV ? pre_samples(sg.sample_cnt, sg.thr_index, a.margin) : sg.sample_cnt;
-  const uint32_t rank = PROV ? pre_rank(sg.sample_cnt, sg.thr_index, a.margin, count) : sg.thr_index;
+  const uint32_t count = sg.sample_cnt, rank = sg.thr_index;
   const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  auto settle = [&](uint32_t key) {  // one lane
-    GdState* st = seg_state(sg);
-    st->thr_bits = key;
-    if (PROV) st->fallback = st->crowded = st->ties = 0;
-  };
-  if (PROV && t < uint32_t(kHitWays)) *reinterpret_cast<uint2*>(sg.ws + l.hist + t * kWayStep * sizeof(uint32_t)) = make_uint2(0, 0);
+  auto settle = [&](uint32_t key) { seg_state(sg)->thr_bits = key; };  // one lane
   // the lane's three largest keys
   uint32_t m1 = 0, m2 = 0, m3 = 0;
   auto take = [&](uint32_t k) {
@@ -532,7 +523,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
     m2 = m2 > u ? m2 : u;
     m3 = m3 > v ? m3 : v;
   };
-  if (!PROV && count <= a.gather) {
+  if (count <= a.gather) {
     constexpr int kOwn = (int(kPickGather) + kSelThreads - 1) / kSelThreads;
     float gv[kOwn], rv[kOwn];
 #pragma unroll
@@ -711,16 +702,12 @@ __global__ __launch_bounds__(kThreads) void gd_presample_kernel(const GdArgs<CAP
   const GdSeg& sg = a.seg[s];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
   uint32_t* samples = reinterpret_cast<uint32_t*>(sg.ws + l.samples);
-  const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index, a.margin);
+  const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index);
   const uint32_t x = uint32_t(tile - a.tile_start[s]) * kThreads + threadIdx.x;
   uint32_t key = 0;
   if (x < s0) {
     const uint32_t i = sample_index(sg.seed, x, sg.n);
     key = __float_as_uint(__builtin_fabsf(a.residual ? sg.g[i] + sg.r[i] : sg.g[i]));
-  }
-  if (a.margin != kBySpread) {
-    if (x < s0) samples[x] = key;
-    return;
   }
   const uint32_t lane = threadIdx.x & (kWave - 1), first = x - lane;
   if (first >= s0) return;
@@ -747,7 +734,7 @@ __global__ __launch_bounds__(kThreads) void gd_prepick_kernel(const GdArgs<CAP> 
   __shared__ uint32_t s_part[2][kThreads / kWave];
   const GdSeg& sg = a.seg[blockIdx.x];
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
-  const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index, a.margin), rank = pre_rank(sg.sample_cnt, sg.thr_index, a.margin, s0);
+  const uint32_t s0 = pre_samples(sg.sample_cnt, sg.thr_index), rank = pre_rank(sg.sample_cnt, sg.thr_index, a.margin, s0);
   const uint32_t slack = pre_slack(sg.sample_cnt, sg.thr_index, s0);
   const uint32_t quads = cdiv(s0, kWave) * (kPreTop / 4), t = threadIdx.x;
   const uint4* __restrict__ left = reinterpret_cast<const uint4*>(sg.ws + l.samples);
@@ -1407,7 +1394,7 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     }
   }
   if (a.margin >= 0 && st->fallback) {
-    // the provisional threshold was not below the exact one: nothing of what the masks hold may be used
+    // the provisional threshold lies above the exact one: nothing of what the masks hold may be used
     if (tile0 == 0 && a.report != nullptr && lane == 0) {
       uint32_t* rep = a.report + size_t(s) * kReportWords;
       __hip_atomic_store(rep + 0, kFallback, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -2614,7 +2601,7 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     });
     if (grid.x) HPX_LAUNCH("gd_sample_kernel", gd_sample_kernel<CAP>, grid, dim3(kThreads), st, a);
     grid = tiles([](const GdSeg& sg) { return sg.sample_cnt <= kPickMax ? 1u : 0u; });
-    if (grid.x) HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<false, CAP>), grid, dim3(kSelThreads), st, a);
+    if (grid.x) HPX_LAUNCH("gd_pick_kernel", gd_pick_kernel<CAP>, grid, dim3(kSelThreads), st, a);
     grid = tiles(sel_blocks);
     if (grid.x) {
       HPX_LAUNCH("gd_select_kernel", (gd_select_kernel<1, CAP>), grid, dim3(kSelThreads), st, a);
@@ -2625,13 +2612,9 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     }
     stream_pass();
   } else {
-    grid = tiles([margin](const GdSeg& sg) { return cdiv(pre_samples(sg.sample_cnt, sg.thr_index, margin), kThreads); });
+    grid = tiles([](const GdSeg& sg) { return cdiv(pre_samples(sg.sample_cnt, sg.thr_index), kThreads); });
     HPX_LAUNCH("gd_presample_kernel", gd_presample_kernel<CAP>, grid, dim3(kThreads), st, a);
-    grid = tiles([](const GdSeg&) { return 1u; });
-    if (margin == kBySpread)
-      HPX_LAUNCH("gd_prepick_kernel", gd_prepick_kernel<CAP>, grid, dim3(kThreads), st, a);
-    else
-      HPX_LAUNCH("gd_pick_kernel", (gd_pick_kernel<true, CAP>), grid, dim3(kSelThreads), st, a);
+    HPX_LAUNCH("gd_prepick_kernel", gd_prepick_kernel<CAP>, dim3(uint32_t(count)), dim3(kThreads), st, a);
     stream_pass();
     grid = tiles([](const GdSeg& sg) { return sg.n < kInverseFrom ? cdiv(sg.sample_cnt, kThreads) : cdiv(cdiv(sg.n, kTile), kExpandPerBlock); });
     HPX_LAUNCH("gd_invert_kernel", gd_invert_kernel<CAP>, grid, dim3(kThreads), st, a);
@@ -2805,7 +2788,7 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
     std::vector<uint32_t> rep_host(size_t(batch) * kReportWords);
     for (size_t w = 0; w < rep_host.size(); w++) rep_host[w] = report[w];
     if (plans[first].margin >= 0) {   // those come first
-      // Tensors whose provisional threshold was not below the exact one: through the gather path, on the array
+      // Tensors whose provisional threshold lies above the exact one: through the gather path, on the array
       // the pass has already updated (it holds G + R now: sampled and thresholded as it is, nothing added again).
       std::vector<int> fb;
       for (int t = 0; t < batch; t++)
