@@ -76,6 +76,39 @@ def test_ranks_around_the_gram_matrix(psgd, r):
     _phases(psgd, [(n, 70, r) for n in (r, 63, 1025, 4100)], r)
 
 
+@pytest.mark.parametrize("n", [4, 63, 64, 65, 1023, 1024, 1025, 4095, 4096, 4097, 5121, 8193])
+def test_heights_of_four_columns(psgd, n):
+    # a row to a lane: around whole waves, the rows that a workgroup holds, and those it reads twice
+    _phases(psgd, [(n, 70, 4), (n, 9, 4)], n)
+
+
+def test_four_columns_take_less_than_eight(psgd, capi):
+    """The launch that orthonormalises 36 factors, right behind the one that has written them: half the columns are half the
+    bytes and a third of the products: with what every launch takes, less than 0.7 of the time."""
+    L = capi.load()
+
+    def us(r):
+        shapes = [(8192, 64)] * 36
+        gen = torch.Generator(device="cuda").manual_seed(r)
+        G, R, M = ([torch.empty(n, m, device="cuda").normal_(0, 1, generator=gen) for n, m in shapes] for _ in range(3))
+        Q = [torch.empty(m, r, device="cuda").normal_(0, 1, generator=gen) for n, m in shapes]
+        P = [torch.empty(n, r, device="cuda") for n, m in shapes]
+        times = []
+        for _ in range(12):
+            L.hpx_profile_reset(); L.hpx_profile_enable(1)
+            try:
+                psgd.encode1(G, R, Q, M, P)
+                psgd.encode2(P, M, Q)
+                torch.cuda.synchronize()
+                times.append(capi.profile_query("psgd_orth_kernel")[0] * 1e3)
+            finally:
+                L.hpx_profile_enable(0); L.hpx_profile_reset()
+        return sorted(times)[len(times) // 2]
+
+    four, eight = us(4), us(8)
+    assert four < 0.7 * eight, (four, eight)
+
+
 @pytest.mark.parametrize("r", [2, 4, 8])
 def test_columns_that_depend_on_each_other(psgd, r):
     # The last column is the first plus `eps` of something else: with eps 1e-2 the Gram matrix

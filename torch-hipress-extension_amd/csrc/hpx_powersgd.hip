@@ -413,9 +413,24 @@ __device__ __forceinline__ void store_row(const float (&y)[C], float* P, int64_t
 // B[blk][k][i] are lane 16k + 4blk + i alike, so one register of sixteen rows by four columns is both operands, and D[blk][i][j]
 // (lane 16i + 4blk + j) is left to be added up over the blocks alone.  (As fp64 products in every lane the sums had to be
 // folded over 64 lanes, ten or 36 of them: for eight columns that was most of the launch.)
-// us of the launch, folded over the lanes / so: 36 factors of up to 2048 x 8 24 / 8, one of 4096 x 8 35 / 11; of 4 columns 10.5 /
-// 9.6 for one of 4096 (Gram-Schmidt: 38 for 36 of them), 11.1 / 12.9 for the 36 of the layer set; 512 x 512 of rank 4, all three
-// phases, 26.9 / 25.9.
+// Up to four columns are loaded a row to a lane and turned round within four lanes: with an element to a lane, as of more
+// columns, a wave made four times as many requests.  What a thread has loaded it still holds when the result is worked out, its
+// rows being the same, in factors of up to 4096 rows.
+// us of the launch, folded over the lanes / an element to a lane / so: 36 factors of 2048 x 8 23.5 / 8.3, one of 30000 x 8 164 / 61;
+// the 36 of the layer set (4 columns) 10.5 / 13.1 / 5.6, 36 of 8192 x 4 18.3 / 23.6 / 9.4, of 8192 x 2 11.3 / 23.5 / 9.9, of 4096 x 3
+// 9.2 / 14.2 / 6.0, one of 30000 x 4 47 / 56 / 24; 512 x 512 of rank 4, all three phases, 27.7 / 26.2 / 25.3.
+__device__ __forceinline__ float quad_xor(float x, int one_or_two) {   // of the lane across, within four
+  return __int_as_float(one_or_two == 1 ? __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xF, 0xF, false)
+                                        : __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xF, 0xF, false));
+}
+// Four rows, one to a lane of each four, to four registers of one row each with a column to a lane.
+__device__ __forceinline__ float4 quad_transpose(float4 v, int lane) {
+  const bool odd = lane & 1, high = lane & 2;
+  const float a = quad_xor(odd ? v.x : v.y, 1), b = quad_xor(odd ? v.z : v.w, 1);
+  const float x = odd ? a : v.x, y = odd ? v.y : a, z = odd ? b : v.z, w = odd ? v.w : b;
+  const float c = quad_xor(high ? x : z, 2), d = quad_xor(high ? y : w, 2);
+  return make_float4(high ? c : x, high ? d : y, high ? z : c, high ? w : d);
+}
 template <int C>
 __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
   constexpr int H = C / 4, kBlocks = H * (H + 1) / 2;   // 4 x 4 blocks of the Gram matrix: (0, 0), and (0, 1), (1, 1)
@@ -434,7 +449,43 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
 #pragma unroll
     for (int u = 0; u < kAcc; u++) acc[k][u] = 0;
   const int col = lane & 3;
-  for (int64_t row0 = int64_t(wave) * 16; row0 < n; row0 += kGroups * kOrthWaves * 16) {
+  constexpr int kRows = 16 / C;  // loaded together, a row to a lane
+  float own[kRows][C];           // up to four columns: the thread's rows, all of them where held
+  bool held = false;
+  if constexpr (C == 4) {
+    held = n <= kRows * kOrthThreads;
+    auto sums = [&](auto columns) {
+      constexpr int R = decltype(columns)::value;
+      for (int64_t row0 = int64_t(wave) * kWave; row0 < n; row0 += kRows * kOrthThreads) {
+#pragma unroll
+        for (int u = 0; u < kRows; u++) {
+          const int64_t row = row0 + u * kOrthThreads + lane;
+          const float* at = P + (row < n ? row : n - 1) * R;   // (no branch between the loads)
+          if constexpr (R == C) {
+            const float4 v = ld4(at);
+            own[u][0] = v.x; own[u][1] = v.y; own[u][2] = v.z; own[u][3] = v.w;
+          } else {
+#pragma unroll
+            for (int c = 0; c < C; c++) own[u][c] = c < R ? at[c] : 0.f;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kRows; u++) {
+#pragma unroll
+          for (int c = 0; c < R; c++) own[u][c] = row0 + u * kOrthThreads + lane < n ? own[u][c] : 0.f;
+          const float4 t = quad_transpose(make_float4(own[u][0], own[u][1], own[u][2], own[u][3]), lane);
+          acc[0][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.x, t.x, acc[0][0], 0, 0, 0);
+          acc[0][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.y, t.y, acc[0][1], 0, 0, 0);
+          acc[0][2] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.z, t.z, acc[0][2], 0, 0, 0);
+          acc[0][3] = __builtin_amdgcn_mfma_f64_4x4x4f64(t.w, t.w, acc[0][3], 0, 0, 0);
+        }
+      }
+    };
+    if (r == 4) sums(std::integral_constant<int, 4>{});
+    else if (r == 3) sums(std::integral_constant<int, 3>{});
+    else if (r == 2) sums(std::integral_constant<int, 2>{});
+    else sums(std::integral_constant<int, 1>{});
+  } else for (int64_t row0 = int64_t(wave) * 16; row0 < n; row0 += kGroups * kOrthWaves * 16) {
     float x[kGroups][H];
 #pragma unroll
     for (int u = 0; u < kGroups; u++) {
@@ -524,11 +575,17 @@ __device__ __forceinline__ bool gram_orth(float* __restrict__ P, int n, int r) {
     ok = ok && s * s <= limit;
   }
   if (!ok) return false;  // the same in every thread
-  constexpr int kRows = 16 / C;  // loaded together
   for (int64_t row0 = threadIdx.x; row0 < n; row0 += kRows * kOrthThreads) {
     float x[kRows][C];
 #pragma unroll
-    for (int u = 0; u < kRows; u++) load_row<C>(x[u], P, row0 + u * kOrthThreads, n, r);
+    for (int u = 0; u < kRows; u++) {
+      if (held) {
+#pragma unroll
+        for (int c = 0; c < C; c++) x[u][c] = own[u][c];
+      } else {
+        load_row<C>(x[u], P, row0 + u * kOrthThreads, n, r);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < kRows; u++) {
       float out[C];
