@@ -85,3 +85,31 @@ def test_several_messages_at_one_distance(tg, oracle_cpu, bits, n):
                         want = _decoded(oracle_cpu, m, want, int(j > 0 or add0))
                 assert_bits_equal(host(d), want, f"{count} messages, odd one: {odd} at {at}, add0 {add0}")
                 assert (tg.status() != 0) == (odd == "invalid")
+
+
+@pytest.mark.parametrize("odd", ["width", "tail", "invalid"])
+@pytest.mark.parametrize("count, apart, n", [(8, False, 4099), (9, False, 4099), (3, True, 4099), (2, False, 1024 * 2 * 4096 + 3)])
+def test_a_first_message_that_does_not_cover_what_it_overwrites(tg, oracle_cpu, odd, count, apart, n):
+    """What it leaves is the tensor's own, under the messages added behind it: in the kernel for up to eight messages of one
+    width, in that for more, for messages at no one distance, and for tensors of several sub-tiles to a workgroup."""
+    rng = np.random.default_rng(count + n)
+    slots = [oracle_cpu.terngrad_encode(rng.normal(0, 1, n).astype(np.float32), 2, 0, 1)[1] for _ in range(count)]
+    if odd == "width":
+        slots[0][0] = 4    # half of the elements
+    elif odd == "tail":
+        slots[0][1] = 255
+    else:
+        slots[0][0] = 3
+    size, out = slots[0].size, rng.normal(0, 1, n).astype(np.float32)
+    at = [j * size + (j * j if apart else 0) for j in range(count)]
+    buf = np.zeros(at[-1] + size, np.uint8)
+    for a, m in zip(at, slots):
+        buf[a:a + size] = m
+    d_buf, d = dev(buf), dev(out)
+    tg.decode([d_buf[a:a + size] for a in at], [d] * count, [0] + [1] * (count - 1))
+    want = out
+    for j, m in enumerate(slots):
+        if m[0] != 3:
+            want = _decoded(oracle_cpu, m, want, int(j > 0))
+    assert_bits_equal(host(d), want, odd)
+    assert (tg.status() != 0) == (odd == "invalid")

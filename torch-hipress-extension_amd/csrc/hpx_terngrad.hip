@@ -2219,14 +2219,15 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const A
     if (one) op[last] = sum;
     continue;
   }
-  // Messages that cover different numbers of elements (a clamped or malformed header): element by element.
+  // Messages that cover different numbers of elements (a clamped or malformed header): element by element, and from what the
+  // tensor holds: an element that the first message does not cover keeps that under those added to it.
   for (int k = 0; k < kDIters; k++) {
     const size_t e = size_t(g0 + k * kThreads) * 4;
     if (e >= n) break;
     const int lim = (n - e >= 4) ? 4 : int(n - e);
     for (int i = 0; i < lim; i++) {
-      float acc = need_old ? op[e + i] : 0.f;
-      bool touched = need_old;
+      float acc = op[e + i];
+      bool touched = false;
       for (int j = 0; j < ns; j++) {
         if (e + i < s_cnt[j]) {
           const float v = float(int(code_at(s_pay[j], e + i, s_bits[j]))) * s_gap[j] + s_mn[j];  // terngrad_body.h:127, :158
