@@ -560,3 +560,35 @@ def test_large_graddrop_tasks_of_one_batch_share_one_workspace(hp, oracle_cpu):
         assert_bits_equal(c.numpy()[:msg.size], msg, "message")
         assert_bits_equal(host(r), want_r, "residual")
     assert hp.error_count() == 0, hp.last_error()
+
+
+def test_a_large_graddrop_task_behind_small_ones_has_a_call_of_its_own(hp, oracle_cpu):
+    # Queued together, smaller tasks in front of a large one take no more memory than the large one alone.
+    sr, dr_ = 0.002, 0.9999
+    ns = {"large": 34_000_000, "small": 20_000_000}
+    items, want = [], []
+    for k, kind in enumerate(["large", "small", "large", "small", "large"]):
+        n = ns[kind]
+        g, r = torch.randn(n, device="cuda") * 1e-3, torch.zeros(n, device="cuda")
+        fixed = 4 + int(2 * np.ceil(n * (1 - dr_))) * 4
+        c = _host_buf(fixed, 1)
+        items.append((f"w{k}", g, r, torch.zeros(fixed, dtype=torch.uint8, device="cuda"), c, 0, 10))
+        want.append((g, r, c))
+    torch.cuda.synchronize()
+    assert hp.init("graddrop", {"sample_rate": sr, "drop_ratio": dr_, "seed": 1}, 0, 0, 2)
+    free = torch.cuda.mem_get_info()[0]
+    assert hp.submit_task(*items[0])
+    _collect(hp, 10, ["w0"])
+    one = free - torch.cuda.mem_get_info()[0]
+    want[0][1].zero_()
+    torch.cuda.synchronize()
+    for it in items:
+        assert hp.submit_task(*it)
+    _collect(hp, 10, [it[0] for it in items])
+    assert one > 0 and free - torch.cuda.mem_get_info()[0] <= one + (2 << 20), one
+    for g, r, c in want[:3]:
+        want_r = np.zeros(g.numel(), np.float32)
+        msg, _ = oracle_cpu.gd_encode(host(g), want_r, sr, dr_, 1)
+        assert_bits_equal(c.numpy()[:msg.size], msg, "message")
+        assert_bits_equal(host(r), want_r, "residual")
+    assert hp.error_count() == 0, hp.last_error()

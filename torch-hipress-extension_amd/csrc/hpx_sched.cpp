@@ -349,8 +349,8 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
   // Transfers and codec calls are cut into runs so that the PCIe transfer of one run overlaps the kernels of
   // the next (a 200-tensor TBQ bucket spends 2.5 times as long on the link as in its encode kernel).
   // GradDrop messages are tiny and its encode has a large fixed cost per call, so a GradDrop batch stays
-  // one run, up to kGdRunElements: its workspace grows with the tensors of a call (24 MB for 60 M elements), and how many
-  // large ones fall into a batch is a matter of when the worker looks.
+  // one run, up to kGdRunElements (a larger task is a run of its own): its workspace grows with the tensors of a call (24 MB for
+  // 60 M elements), and how many large ones fall into a batch, and behind which, is a matter of when the worker looks.
   const bool one_run = p.alg == kGraddrop;
   auto next_run_bytes = [one_run](int64_t b) {
     if (one_run) return INT64_MAX;
@@ -489,7 +489,8 @@ void run_codec_batch(Worker& w, const Params& p, const std::vector<Task>& batch,
       int64_t bytes = 0;
       pipe_bytes = next_run_bytes(pipe_bytes);
       int64_t elements = 0;
-      while (i < ts.size() && bytes < pipe_bytes && !(one_run && elements >= kGdRunElements)) {
+      auto fits = [&](int64_t n) { return !one_run || run.empty() || elements + n <= kGdRunElements; };
+      while (i < ts.size() && bytes < pipe_bytes && fits(ts[i]->t.tensor_numel)) {
         bytes += message_bytes(p, ts[i]->t);
         elements += ts[i]->t.tensor_numel;
         run.push_back(ts[i++]);
