@@ -1,10 +1,12 @@
 """GPU parity of the sparsifier's lists of candidates, one per 1024 elements: large values crowded into some of them, so
 that a list is full to the last place or one beyond it, and kept fractions on either side of the one up to which the
-lists are written.  Tensors settled by one workgroup, by the listing launch alone, and by a cut behind it.  Bit-exact against the
-oracle."""
+lists are written; numbers kept on either side of the one from which they are.  Tensors settled by one workgroup, by the
+listing launch alone, and by a cut behind it.  Bit-exact against the oracle."""
 import numpy as np
 import pytest
+import torch
 
+from gpu_util import assert_bits_equal, dev, host
 from test_gpu_gd import Gd, _check_encode
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +54,26 @@ def test_kept_fractions(gd, oracle_cpu, n, kept):
     g, r = rng.laplace(0, 1e-3, n).astype(np.float32), rng.normal(0, 1e-4, n).astype(np.float32)
     for seed in (5, 9 << 24):
         _check_encode(gd, oracle_cpu, g, r.copy(), 0.02, 1 - kept, seed)
+
+
+# and from 400 kept on, and one in 6144 elements; in a call of both kinds each tensor goes by its own number
+@pytest.mark.parametrize("n,kept", [(40_000, (398, 399, 400, 401, 20)), (405_505, (399, 400, 401, 1024)), (500 * 6144, (498, 499, 500, 501)),
+                                    (500 * 6144 + 1, (500, 501))])
+def test_on_either_side_of_the_least_number_kept(gd, oracle_cpu, n, kept):
+    rng = np.random.default_rng(n)
+    gs = [rng.laplace(0, 1e-3, n).astype(np.float32) for _ in kept]
+    rs = [rng.normal(0, 1e-4, n).astype(np.float32) for _ in kept]
+    drops = [1 - (k - 0.5) / n for k in kept]
+    for seed in (5, 9 << 24):
+        for g, r, d in zip(gs, rs, drops):
+            _check_encode(gd, oracle_cpu, g, r.copy(), 0.05, d, seed)
+        d_r, outs = [dev(r) for r in rs], [torch.zeros(4 + 8 * k, dtype=torch.uint8, device="cuda") for k in kept]
+        gd.encode([dev(g) for g in gs], d_r, outs, [0.05] * len(kept), drops, [seed] * len(kept))
+        for g, r, d, got_r, out in zip(gs, rs, drops, d_r, outs):
+            want_r = r.copy()
+            msg = oracle_cpu.gd_encode(g, want_r, 0.05, d, seed)[0]
+            assert_bits_equal(host(out)[:msg.size], msg, "message")
+            assert_bits_equal(host(got_r), want_r, "residual")
 
 
 @pytest.mark.parametrize("n,kept", [(900_001, 1e-2), (2_500_000, 1e-2), (9_000_001, 2e-3)])   # beyond what one workgroup cuts

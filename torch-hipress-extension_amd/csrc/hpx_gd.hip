@@ -117,11 +117,24 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
 }
 // Behind that block: the candidates themselves, (index, value) in ascending order, a list per wave of the pass with room
 // for this many (0: no lists, the candidates are looked up through the masks).  Twice the expected number and fourteen: a wave's
-// 1024 elements exceed that next to never unless the large ones crowd together, and then the masks serve.  The pass pays 1 %
-// for them (138 M elements: 229 us, 232 with lists); behind it the expand launch takes 9.0 us instead of 14.4, and the
-// finish 8.8 instead of 11.7 for one tensor of a million, 16.2 instead of 24.8 for ResNet-50's 161.  Up to 12 in 1024:
-// denser, the lists would be a tenth of the tensor.
+// 1024 elements exceed that next to never unless the large ones crowd together, and then the masks serve.  The pass pays
+// for them (138 M elements 229 -> 232 us, ResNet-50's 161 tensors 46.7 -> 48.4, one of a million 4.3 -> 5.1); behind it the
+// expand launch takes 9.0 us instead of 14.4 (138 M), and the finish 8.8 instead of 11.7 for the million, 16.2 instead of 24.8 for
+// ResNet-50's 161.  Up to 12 in 1024: denser, the lists would be a tenth of the tensor.
+// Of the tensors that one workgroup settles (gd_finish_kernel) those with few candidates to a list have none either: the masks are
+// as quick there, or quicker, and the pass is without the lists' code and stores.  us per encode and decode of one tensor,
+// lists / masks: 20 thousand elements, 20 kept 23.3 / 21.7; 80 thousand, 80 kept 25.2 / 23.6; 120 thousand, 120 kept 28.2 / 27.7;
+// 32 thousand, 320 kept 25.8 / 24.9; 400 thousand, 400 kept 30.8 / 30.8; 50 thousand, 500 kept 27.1 / 26.9; 80 thousand, 800 kept
+// 28.6 / 29.0; 1 M, 1049 kept 32.7 / 34.9; 4 M, 400, 700 and 1200 kept 38.1 / 37.6, 39.3 / 39.4 and 41.4 / 42.9; 8 M, 700, 1200 and 2400
+// kept 61.9 / 60.6, 63.5 / 63.6 and 67.1 / 70.7; 16 M, 400 and 2400 kept 87.1 / 77.5 and 93.9 / 89.2; 30 tensors of 150 thousand elements
+// together, one in a hundred kept, 31.9 / 30.0.
+constexpr uint32_t kFinishKeep = 2560;         // what one workgroup settles: entries kept ...
+constexpr uint32_t kFinishTiles = kScanChunk;  // ... and tiles
+constexpr uint32_t kListFrom = 400;            // with lists from so many kept ...
+constexpr uint32_t kListShare = 6;             // ... and one for so many lists
+__host__ __device__ inline bool one_workgroup(uint32_t n, uint32_t limit) { return limit <= kFinishKeep && cdiv(n, kTile) <= kFinishTiles; }
 __host__ __device__ inline uint32_t list_room(uint32_t n, uint32_t limit) {
+  if (one_workgroup(n, limit) && (limit < kListFrom || limit * (kListShare * uint32_t(kWaveTile)) < n)) return 0;
   const float mean = float(kWaveTile) * float(limit) / float(n);
   return mean > 12.0f ? 0u : (uint32_t(2.0f * mean) + 21u) & ~7u;
 }
@@ -1101,7 +1114,8 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
 // RESIDUAL = false is the sparsifier without residual (dgc_body.h:110-117): the
 // values are G itself, nothing is added and nothing is stored (4 bytes per element).
 // PROV: against the provisional threshold also a NaN is a candidate, as it is one of the largest of a sample.
-template <bool RESIDUAL, bool PROV, int CAP>
+// LISTS: some tensor of the launch may have lists.
+template <bool RESIDUAL, bool PROV, bool LISTS, int CAP>
 __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a) {
   const int tile = blockIdx.x;
   const int s = find_segment<CAP>(a.tile_start, a.nseg, tile);
@@ -1125,7 +1139,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   uint2* __restrict__ list = seg_list(sg, l) + (size_t(t) * (kThreads / kWave) + wave) * room;
   uint32_t lo = 0, hi = 0, cnt = 0;
   auto note = [&](uint64_t m, uint32_t e, float x) {  // m: the wave's candidates of 64 elements, uniform
-    if (m != 0) {
+    if (LISTS && m != 0) {
       const uint32_t at = cnt + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
       if ((m >> lane & 1ull) && at < room) list[at] = make_uint2(e, __float_as_uint(x));
     }
@@ -1186,7 +1200,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   __syncthreads();
   if (threadIdx.x == 0) {
     reinterpret_cast<uint32_t*>(sg.ws + l.cnt)[t] = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-    reinterpret_cast<uint64_t*>(sg.ws + l.wcnt)[t] =
+    if (LISTS) reinterpret_cast<uint64_t*>(sg.ws + l.wcnt)[t] =
         uint64_t(s_cnt[0]) | (uint64_t(s_cnt[1]) << 16) | (uint64_t(s_cnt[2]) << 32) | (uint64_t(s_cnt[3]) << 48);
     reinterpret_cast<uint64_t*>(sg.ws + l.coarse)[t] =
         uint64_t(s_any[0]) | (uint64_t(s_any[1]) << 16) | (uint64_t(s_any[2]) << 32) | (uint64_t(s_any[3]) << 48);
@@ -2152,8 +2166,6 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // ResNet-50's 161 tensors 58 -> 16 us.
 // Larger ones that still fit are only cut here, behind the expand launch.  All of it is queued before the host knows any
 // count.
-constexpr uint32_t kFinishKeep = 2560;
-constexpr uint32_t kFinishTiles = kScanChunk;
 // The cut of the tensors that keep between kFinishKeep and kCutKeep entries, whose candidates and keys the expand
 // launch has listed (or, where they are too many for the list or for LDS, are found again in the mask).
 __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, uint32_t* s_bins, uint32_t* s_wave) {
@@ -2200,7 +2212,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
   uint32_t* s_key = s_stage;
   uint32_t* s_id = s_stage + kCutLds;
   const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
-  if (sg.limit > kFinishKeep || cdiv(sg.n, kTile) > kFinishTiles) {
+  if (!one_workgroup(sg.n, sg.limit)) {
     cut_listed(sg, s_stage, s_bins, s_wave);
     return;
   }
@@ -2530,7 +2542,7 @@ struct Plan {
 // Who settles a tensor behind the pass: one workgroup (gd_finish_kernel); the expand launch and, if it has to be cut, one
 // workgroup (the same launch: its LDS holds what is kept); or the expand launch and the host, which queues the sort of
 // many workgroups once it has heard the count.  The provisional path keeps to the last: it may have to fall back.
-bool finishes(const GdSeg& sg, int margin) { return margin < 0 && sg.limit <= kFinishKeep && cdiv(sg.n, kTile) <= kFinishTiles; }
+bool finishes(const GdSeg& sg, int margin) { return margin < 0 && one_workgroup(sg.n, sg.limit); }
 bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutKeep; }
 
 // Whether the provisional path is the quicker one for a tensor.  It saves the gather of the sample (two lines each, one
@@ -2578,14 +2590,12 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   };
   auto stream_pass = [&]() {
     const dim3 g = tiles([](const GdSeg& sg) { return cdiv(sg.n, kTile); });
-    if (residual && margin < 0)
-      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<true, false, CAP>), g, dim3(kThreads), st, a);
-    else if (residual)
-      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<true, true, CAP>), g, dim3(kThreads), st, a);
-    else if (margin < 0)
-      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<false, false, CAP>), g, dim3(kThreads), st, a);
-    else
-      HPX_LAUNCH("gd_stream_kernel", (gd_stream_kernel<false, true, CAP>), g, dim3(kThreads), st, a);
+    bool lists = false;
+    for (int i = 0; i < count; i++) lists = lists || list_room(a.seg[i].n, a.seg[i].limit) != 0;
+    auto pass = [&](auto kernel) { HPX_LAUNCH("gd_stream_kernel", kernel, g, dim3(kThreads), st, a); };
+    if (margin >= 0) pass(residual ? gd_stream_kernel<true, true, true, CAP> : gd_stream_kernel<false, true, true, CAP>);
+    else if (lists) pass(residual ? gd_stream_kernel<true, false, true, CAP> : gd_stream_kernel<false, false, true, CAP>);
+    else pass(residual ? gd_stream_kernel<true, false, false, CAP> : gd_stream_kernel<false, false, false, CAP>);
   };
   dim3 grid;
   if (margin < 0) {
