@@ -61,6 +61,13 @@ def test_heights_around_the_blocks_of_rows(psgd, n):
     _phases(psgd, [(n, m, min(4, n)) for m in (1024, 384, 192, 70)], n)
 
 
+@pytest.mark.parametrize("n", [129, 130, 143, 144, 145, 160, 177, 190, 191, 192])
+def test_heights_of_a_block_and_up_to_half_of_another(psgd, n):
+    # one partial whose loads are all in flight together, by itself and beside matrices that have several
+    _phases(psgd, [(n, m, r) for m in (61, 64, 130, 511) for r in (1, 4, 7)], n)
+    _phases(psgd, [(n, 301, 4), (515, 301, 4), (128, 301, 4), (193, 301, 4)], n + 1)
+
+
 @pytest.mark.parametrize("n,m", [(4095, 4096), (4097, 4096), (5001, 3500)])
 def test_matrices_around_the_larger_number_of_partials(psgd, n, m):
     _phases(psgd, [(n, m, 4)], n + m)

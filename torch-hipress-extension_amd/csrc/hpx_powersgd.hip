@@ -68,7 +68,7 @@ struct Seg {
   int32_t part_off;    // encode2: offset (in floats / 4) of this matrix's partials
   int32_t ld;          // row stride of P and Q (the full rank; r is the width of the block of columns at hand)
   int32_t mode;        // kFromM | kOntoM | kKeepGrad, for the passes of a rank above 16
-  int32_t split;       // encode1: waves that share four rows.  encode2, decode: strip_lanes
+  int32_t split;       // encode1: waves that share four rows.  encode2: q_lanes.  decode: strip_lanes
   int32_t rows;        // encode2: rows folded into one partial of Q (of a strip 256 columns wide)
 };
 constexpr int32_t kFromM = 1;    // encode1: M has been stored by an earlier pass: read it instead of grad + residual
@@ -629,7 +629,7 @@ __global__ __launch_bounds__(kOrthThreads) void psgd_orth_kernel(const Args<CAP>
 }
 
 // ---- encode2, step 2: Q = M^T P ------------------------------------------------
-// A workgroup takes a strip of columns (256, or 128 or 64 with two or four rows side by side in a wave: strip_lanes)
+// A workgroup takes a strip of columns (256, or 128 or 64 with two or four rows side by side in a wave: q_lanes)
 // and sg.rows rows of it (two or four times that), in blocks of 32 rows (64, 128) that the workgroups of a strip take in
 // turn: what is being read at any time is one stretch of the matrix, not a place every sg.rows rows (the layer set 210 us
 // with each workgroup's rows in one piece, 188 so).  The rows of a block go round the waves.  Per row a
@@ -686,48 +686,70 @@ __global__ __launch_bounds__(kThreads, CG == 1 ? 4 : 1) void psgd_mtp_kernel(con
   };
   const int64_t block = kRows * step;
   int64_t row0 = rblk * block + wave * side;  // the first of the wave's rows in a round
-  // Main loop: a block at a time, every load issued before the first use, summed on their own in two chains and added to
-  // what there is (one chain of fp32 sums down all rows of a partial of 512 left Q half as far again from the exact product;
-  // two chains of four instead of one of eight 8.24e-8 of its norm for 4096 x 4096 and 7.5e-8 for 200 x 600, from
-  // 8.46e-8 and 7.7e-8).  Only the lane that holds the row's end and those past it take the element-wise way.
-  for (; row0 + (kRows - 1) * step + side <= n; row0 += parts * block) {
-    float4 m4[kRows];
-    float p[kRows][CG];
-    const float* Mp = M + (row0 + mine) * m + kk;
+  // Rounds `from` ... `from` + K - 1 of the rows from row0 on; every load is issued before the first use, and only the lane that
+  // holds the row's end and those past it take the element-wise way.  WHOLE: all of these rows are the matrix's.
+  auto load = [&](auto whole, int64_t row0, int from, auto& m4, auto& p) {
+    constexpr bool WHOLE = decltype(whole)::value;
+    constexpr int K = sizeof(m4) / sizeof(m4[0]);
+    auto row_of = [&](int u) {
+      const int64_t row = row0 + (from + u) * step + mine;
+      return WHOLE || row < n ? row : int64_t(n) - 1;
+    };
     if (kk + 4 <= m) {
 #pragma unroll
-      for (int u = 0; u < kRows; u++) m4[u] = ld4_stream(Mp + int64_t(u) * step * m);
+      for (int u = 0; u < K; u++) m4[u] = ld4_stream(M + row_of(u) * m + kk);
     } else {
 #pragma unroll
-      for (int u = 0; u < kRows; u++) {
-        const float* q = Mp + int64_t(u) * step * m;
+      for (int u = 0; u < K; u++) {
+        const float* q = M + row_of(u) * m + kk;
         m4[u] = make_float4(kk < m ? q[0] : 0.f, kk + 1 < m ? q[1] : 0.f, kk + 2 < m ? q[2] : 0.f, 0.f);
       }
     }
 #pragma unroll
-    for (int u = 0; u < kRows; u++)
+    for (int u = 0; u < K; u++)
 #pragma unroll
-      for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[(row0 + u * step + mine) * ld + c * 4 + j] : 0.f;
+      for (int c = 0; c < CG; c++) p[u][c] = (c * 4 + j) < r ? P[row_of(u) * ld + c * 4 + j] : 0.f;
+  };
+  auto clear_past = [&](int64_t row0, int from, auto& m4) {
+    constexpr int K = sizeof(m4) / sizeof(m4[0]);
+#pragma unroll
+    for (int u = 0; u < K; u++) {
+      const bool any = row0 + (from + u) * step + mine < n;
+      m4[u] = make_float4(any ? m4[u].x : 0.f, any ? m4[u].y : 0.f, any ? m4[u].z : 0.f, any ? m4[u].w : 0.f);
+    }
+  };
+  constexpr auto kWhole = std::true_type{};
+  constexpr auto kRagged = std::false_type{};
+  if (parts == 1 && n > block && n <= block + kRows / 2 * step) {
+    // One partial of a block and at most half of another: both are loaded together (one after the other 192 x 192 20.4 us for
+    // all three phases, 30 of up to 250 x 1220 56.5; now 19.6 and 55.3).
+    float4 m4[kRows], rest4[kRows / 2];
+    float p[kRows][CG], rest_p[kRows / 2][CG];
+    load(kWhole, row0, 0, m4, p);
+    load(kRagged, row0, kRows, rest4, rest_p);
+    add_up(m4, p);
+    clear_past(row0, kRows, rest4);
+    add_up(rest4, rest_p);
+    row0 = n;
+  }
+  // Main loop: a block at a time, summed on their own in two chains and added to
+  // what there is (one chain of fp32 sums down all rows of a partial of 512 left Q half as far again from the exact product;
+  // two chains of four instead of one of eight 8.24e-8 of its norm for 4096 x 4096 and 7.5e-8 for 200 x 600, from
+  // 8.46e-8 and 7.7e-8).
+  for (; row0 + (kRows - 1) * step + side <= n; row0 += parts * block) {
+    float4 m4[kRows];
+    float p[kRows][CG];
+    load(kWhole, row0, 0, m4, p);
     add_up(m4, p);
   }
-  // The matrix's last block, where this wave's rows of it are not whole: all their loads in flight together (one round
-  // after the other 12 of 1200 x 601 took 59.2 us for all three phases, 30 of 150 x 220 31.5; now 58.0 and 30.2).
+  // The matrix's last block, where this wave's rows of it are not whole: all their loads in flight together, no branch between
+  // them (one round after the other 12 of 1200 x 601 took 57.7 us for all three phases, together with a branch each 56.5, now 55.2).
   const int64_t after = row0 - wave * side + block;
   for (const int64_t rend = after < n ? after : n; row0 < rend; row0 += kRows * step) {
     float4 m4[kRows];
     float p[kRows][CG];
-#pragma unroll
-    for (int u = 0; u < kRows; u++) {
-      const int64_t row = row0 + u * step + mine;
-      const float* q = M + row * m + kk;
-      m4[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (row < n) {
-        if (kk + 4 <= m) m4[u] = ld4_stream(q);
-        else m4[u] = make_float4(kk < m ? q[0] : 0.f, kk + 1 < m ? q[1] : 0.f, kk + 2 < m ? q[2] : 0.f, 0.f);
-      }
-#pragma unroll
-      for (int c = 0; c < CG; c++) p[u][c] = row < n && c * 4 + j < r ? P[row * ld + c * 4 + j] : 0.f;
-    }
+    load(kRagged, row0, 0, m4, p);
+    clear_past(row0, 0, m4);
     add_up(m4, p);
   }
   // acc[c][t][i'] in lane 4b+j  ->  Q[k0 + (16b + 4i' + t) % width][4c + j], part (16b + 4i' + t) / width of the wave
@@ -973,10 +995,12 @@ int orth_launch(const Args<CAP>& a, size_t lds, hipStream_t st) {
   return HPX_OK;
 }
 
-// A matrix of up to kQWholeRows rows takes the product in one partial, which is Q itself, by the narrowest strips: a call of such
-// matrices needs no launch to add partials up.  us of a pass: 128 x 128 22.2 -> 18.5, 30 of up to 150 x 220 36 -> 27, 10 of up to
-// 64 x 2000 32 -> 28; among taller matrices, where the launch is there anyway, 30 of up to 250 x 1220 56.4 -> 57.4, and at 256 rows
-// 10 of up to 512 x 512 37.4 -> 39.7.
+// A matrix of up to kQWholeRows rows, one block and a half of the narrowest strips, takes the product in one partial, which is Q
+// itself: a call of such matrices needs no launch to add partials up.  us of a pass, by the strips of other matrices / so:
+// 128 x 128 20.3 / 17.5, 192 x 192 23.1 / 19.6, 190 x 4000 34.5 / 30.0, 30 of up to 150 x 220 29.5 / 25.4, of up to 190 x 800
+// 42.8 / 39.4, 10 of up to 64 x 2000 30.8 / 25.8; among taller matrices, where the launch is there anyway, 30 of up to 250 x 1220
+// 54.8 / 55.3, of up to 400 x 600 47.2 / 47.2, of up to 600 x 300 44.5 / 45.4, 12 of up to 256 x 2000 42.6 / 43.2 (56.5, 48.8, 45.8
+// and 44.5 with the half block loaded behind the block), 10 of up to 512 x 512 36.5 / 35.7; at 256 rows these 39.7.
 constexpr int kQWholeRows = 192;
 inline int q_lanes(int n, int m) { return n <= kQWholeRows ? 16 : strip_lanes(m); }
 // Partials of a matrix: of `rows` rows each, as many times more as strips side by side in a wave.
@@ -986,11 +1010,13 @@ inline int32_t q_parts(int n, int m, int rows) { return cdiv(n, int64_t(rows) * 
 // least, or 32 where 64 would leave fewer than kQTilesSmall.  Like split_rows by the matrix alone: Q is the sum of the
 // partials, and what a matrix's Q is must not depend on what else is in the call.  A pass over all three phases in us, with the rows
 // chosen so that the call had 1024 workgroups / with this rule / with at most 256 rows: layer set of 36 matrices 1566 /
-// 1574 / 1588, 4096 x 4096 alone 116 / 127 / 119, 4 of 2000 x 1000 74 / 70 / 70, ResNet-50's 54 157.6 / 157.5 / 157.5
+// 1574 / 1588, 4 of 2000 x 1000 74 / 70 / 70, ResNet-50's 54 157.6 / 157.5 / 157.5
 // (with 32 rows for all of those 160.5); with kQTiles 64 and 32 4096 x 1024 alone is at 59 and 68 instead of 56.
 constexpr int kQRowsMin = 32, kQRowsMax = 512;
-// A matrix of 2^24 elements and more is given kQTilesLarge: 4096 x 4096 alone 127 us with 128 workgroups, 119 with 256; the
-// layer set, which twelve such matrices are part of, pays 4 of 1565 for their partials, and 8 if all 36 have as many.
+// A matrix of 2^24 elements and more is given kQTilesLarge workgroups.  us of a pass with 128 / 256: 4096 x 4096 alone 113.1 / 107.2, of
+// rank 8 152 / 142.5, 16384 x 1024 131 / 126.5, 5000 x 3500 166 / 157, 30000 x 600 184 / 177, 4 of 4100 x 4099 285 / 273; from 2^25
+// elements 512 rows a partial leave as many anyway; the layer set, which twelve such matrices are part of, pays 2.5 of
+// 1550 for their partials.
 constexpr int64_t kQTiles = 128, kQTilesSmall = 32, kQTilesLarge = 256;
 inline int q_rows(int n, int m) {
   static_assert(kQWholeRows <= 2 * kQRowsMin * (kWave / 16), "rows of one partial of the narrowest strips");
