@@ -1132,7 +1132,8 @@ int decode_launches(int count, int max_rank, const float* const* Ps, const float
       if (a.nseg == 0) continue;
       // One read and three writes per element: held to two workgroups per CU (LDS the kernel never touches,
       // hpx_common.h), the 36 matrices of the configuration decode in 765 us instead of 784 with three or four (a
-      // pass over three such sets of buffers in turn).
+      // pass over three such sets of buffers in turn; 755 in another process, with buffers at other addresses, and a launch
+      // between 744 and 831).
       PSGD_LAUNCH_CG_LDS(psgd_decode_kernel, cg, a.tile_start[a.nseg], hpx::kWriteStreamPadLds2, st, a);
       HPX_HIP(hipGetLastError());
     }
