@@ -207,7 +207,7 @@ constexpr size_t kStreamStoreMaxBytes = size_t(1) << 62;
 // A write stream of streaming stores runs faster with few workgroups per CU (their stores then reach memory as a
 // compact front): launches of the write-mode decoders ask for this much LDS they never touch, which holds a CU to
 // three (52 KiB) or four (40 KiB) workgroups of 256 lanes.  TBQ decode of 110 M elements: 73 -> 62 us at three
-// (66 at four, 80 at two); TernGrad decode: 73 -> 65 us at four (72 at three).  Kernels that also read what they
+// (66 at four, 80 at two); TernGrad's line lies in hpx_terngrad.hip.  Kernels that also read what they
 // write (the add-mode decoders, the encoders' in-place residual update, GradDrop's stream pass) gain nothing.
 constexpr int kWriteStreamPadLds2 = 64 * 1024;  // two per CU: the PowerSGD decode (one read, three writes: 792 -> 755 us)
 constexpr int kWriteStreamPadLds3 = 52 * 1024;

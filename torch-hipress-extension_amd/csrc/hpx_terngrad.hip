@@ -2544,6 +2544,12 @@ int launch_encode(int count, const float* const* ins, const int32_t* in_sizes, u
   return HPX_OK;
 }
 
+// Output of a call from which its write-mode decode is held to three workgroups per CU, to four below.  us per encode and decode at
+// two / three / four / five: 2 bits, one tensor of 25.6 M elements 44.5 / 42.8 / 42.7 / 42.8, of 30 M 52.6 / 50.5 / 50.6 / 50.6, of 40 M
+// 69.4 / 67.5 / 67.9 / 67.8, of 95.5 M 175.5 / 172.0 / 173.9 / 175.1, 110 M in 200 tensors 207 / 195 / 204 / 206; 8 bits, 110 M in
+// 20 tensors 234 / 226.7 / 225.9 / 224.9; ResNet-50's 161 tensors at three / four 47.8 / 47.4.  (The workgroups ask for their codes
+// with the header.  When they waited for it first their stores were further apart, and four were best: the 200 tensors 197.)
+constexpr size_t kThreePerCuFrom = size_t(128) << 20;
 template <int CAP>
 int launch_decode(int count, float* const* outs, const int32_t* out_sizes, const uint8_t* const* ins,
                   const int32_t* in_sizes, const int32_t* is_add_tos, uint32_t* status, hipStream_t st) {
@@ -2572,8 +2578,8 @@ int launch_decode(int count, float* const* outs, const int32_t* out_sizes, const
       i++;
     }
     if (a.nseg == 0) continue;
-    // write mode throughout: a pure write stream, held to four workgroups per CU (hpx_common.h)
-    const int pad = (a.stream_store && !any_add) ? hpx::kWriteStreamPadLds4 : 0;
+    // write mode throughout: a pure write stream, held to few workgroups per CU (hpx_common.h)
+    const int pad = !a.stream_store || any_add ? 0 : out_bytes < kThreePerCuFrom ? hpx::kWriteStreamPadLds4 : hpx::kWriteStreamPadLds3;
     HPX_LAUNCH_LDS("terngrad_decode_kernel", hpx::g_prof_on, terngrad_decode_kernel<CAP>, dim3(a.tile_start[a.nseg]), dim3(kThreads), pad, st, a);
     HPX_HIP(hipGetLastError());
   }
