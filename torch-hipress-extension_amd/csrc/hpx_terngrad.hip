@@ -1755,6 +1755,12 @@ __device__ __forceinline__ uint32_t decode_two_bit_whole(float* __restrict__ op,
   return nfull;
 }
 
+// A pointer that all lanes hold alike, in scalar registers: what is loaded through it takes one register of offset.
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(v)))), hi = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(v >> 32))));
+  return reinterpret_cast<const uint8_t*>(uint64_t(hi) << 32 | lo);
+}
 // NS (at most 4) messages of one width folded into the groups `g` of a sub-tile: the loads of all of them and of the lane's
 // groups in flight together.  END: the sub-tile that holds the end of the tensor; `one`: the lane also has element `last` of the
 // partial group there.
@@ -1765,10 +1771,10 @@ __device__ __forceinline__ void fold_messages(float4 (&acc)[kDIters], const uint
   uint32_t raw[NS][kDIters], code[NS];
 #pragma unroll
   for (int j = 0; j < NS; j++) {
-    global_ptr<uint8_t> pay = as_global(s_pay[j0 + j]);
+    global_ptr<uint8_t> pay = as_global(uniform_ptr(s_pay[j0 + j]));
 #pragma unroll
     for (int k = 0; k < kDIters; k++) {
-      const size_t e = size_t(g[k]) * 4;
+      const uint32_t e = g[k] * 4u;
       if (B == 1) raw[j][k] = (uint32_t(pay[e >> 3]) >> (e & 4)) & 0xFu;
       else if (B == 2) raw[j][k] = pay[e >> 2];
       else if (B == 4) raw[j][k] = reinterpret_cast<global_ptr<u16u>>(pay + (e >> 1))->v;
@@ -1971,7 +1977,7 @@ __global__ __launch_bounds__(kThreads) void terngrad_decode_strided_kernel(const
 }
 
 template <typename Args>
-__global__ __launch_bounds__(kThreads) void terngrad_decode_multi_kernel(const Args a) {
+__global__ __launch_bounds__(kThreads, 4) void terngrad_decode_multi_kernel(const Args a) {
   __shared__ float s_mn[kMultiSlotsPerSeg], s_gap[kMultiSlotsPerSeg];
   __shared__ uint32_t s_cnt[kMultiSlotsPerSeg], s_bits[kMultiSlotsPerSeg];
   __shared__ int32_t s_add[kMultiSlotsPerSeg];
