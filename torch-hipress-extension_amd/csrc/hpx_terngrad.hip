@@ -2707,7 +2707,15 @@ int launch_decode_multi(int count, float* const* outs, const int32_t* out_sizes,
         case 2: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<2>, grid, dim3(kThreads), st, sa); break;
         case 4: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<4>, grid, dim3(kThreads), st, sa); break;
         case 8: HPX_LAUNCH("terngrad_decode_strided_kernel", terngrad_decode_strided_kernel<8>, grid, dim3(kThreads), st, sa); break;
-        default: HPX_LAUNCH("terngrad_decode_multi_kernel", terngrad_decode_multi_kernel<SArgs>, grid, dim3(kThreads), st, sa);
+        default: {
+          // Of a little more than four workgroups per CU the last few would run with the chip to themselves: held to three per CU (LDS
+          // that the kernel never touches) they are spread better.  us of a root's pass at four / three: 17.5 M elements with seven
+          // 2-bit messages 56.3 / 54.1, 20 M 59.7 / 58.3, 20 M in 30 tensors with three of 8 bits 70.1 / 67.0, in one 63.6 / 64.2; beyond,
+          // 22.5 M of 2 bits 64.2 / 66.7, 25.6 M of 4 bits in 30 tensors 95.0 / 104.2.
+          const bool few_more = sa.reps == kMultiRep && grid.x > kMultiFull && grid.x <= kMultiFull * 5 / 4;
+          HPX_LAUNCH_LDS("terngrad_decode_multi_kernel", hpx::g_prof_on, terngrad_decode_multi_kernel<SArgs>, grid, dim3(kThreads),
+                         few_more ? hpx::kWriteStreamPadLds3 - 2048 : 0, st, sa);  // less than 2 KiB of its own
+        }
       }
       HPX_HIP(hipGetLastError());
       return HPX_OK;
