@@ -82,8 +82,7 @@ __global__ __launch_bounds__(kThreads) void ecq_max_kernel(const EcqArgs a) {
     for (uint32_t e = e0 + threadIdx.x; e < n; e += kThreads) m = __builtin_fmaxf(m, gh_of(a.g[e], a.h[e], a.alpha));
   }
   uint32_t mb = __float_as_uint(m);  // non-negative floats order like their bit patterns
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(mb, o, kWave); mb = v > mb ? v : mb; }
+  mb = wave_max_u32(mb);
   __shared__ uint32_t s_m[kThreads / kWave];
   if ((threadIdx.x & (kWave - 1)) == 0) s_m[threadIdx.x / kWave] = mb;
   __syncthreads();
@@ -130,8 +129,7 @@ __global__ __launch_bounds__(kThreads) void ecq_quant_kernel(const EcqArgs a) {
   if (threadIdx.x < kWave) {
     uint32_t v = 0;
     for (int w = threadIdx.x; w < kWays; w += kWave) { const uint32_t t = a.ways[w]; v = t > v ? t : v; }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { const uint32_t t = __shfl_xor(v, o, kWave); v = t > v ? t : v; }
+    v = wave_max_u32(v);
     if (threadIdx.x == 0) s_max = v;
   }
   __syncthreads();

@@ -226,12 +226,7 @@ __device__ __forceinline__ void find_digit(const uint32_t* __restrict__ hist, ui
   // Inclusive prefix over the threads in order: within each wave by shuffles, then the sixteen wave totals
   // (three workgroup barriers in all; a workgroup-wide scan through LDS, ten rounds of two barriers each, was
   // most of the time of the launches that call this).
-  uint32_t incl = sum;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t v = __shfl_up(incl, o, kWave);
-    if (lane >= uint32_t(o)) incl += v;
-  }
+  const uint32_t incl = wave_prefix_u32(sum);
   if (lane == kWave - 1) s_wave[wave] = incl;
   if (t == 0) { s_res[0] = 0; s_res[1] = 0; }
   __syncthreads();
@@ -432,8 +427,7 @@ __device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t
   uint32_t top = 0;
 #pragma unroll
   for (int j = 0; j < R; j++) top = key[j] > top ? key[j] : top;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
+  top = wave_max_u32(top);
   top = __builtin_amdgcn_readfirstlane(top);
   floor = __builtin_amdgcn_readfirstlane(floor);
   const int first = 31 - __builtin_clz((top ^ floor) | 1u);   // bits above it are common to every candidate
@@ -463,6 +457,14 @@ __device__ __forceinline__ uint32_t wave_rank(const uint32_t (&key)[R], uint32_t
 // 161 tensors 20 -> 7 us, and 4 us less in the gather launch before it.
 constexpr uint32_t kPickList = 1024;
 constexpr uint32_t kPickAll = 4096;   // listed by a second walk over the sample where the lanes' three largest do not do
+// The sum over each row of 16 lanes, in all of its lanes.
+__device__ __forceinline__ uint32_t row_sum(uint32_t v) {
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x121, 0xF, 0xF, false));   // row_ror:1
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x122, 0xF, 0xF, false));
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x124, 0xF, 0xF, false));
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x128, 0xF, 0xF, false));
+  return v;
+}
 // The sum of a value that repeats every WAVES lanes, by rotations within the rows of 16 lanes.
 template <int WAVES>
 __device__ __forceinline__ uint32_t sum_of_waves(uint32_t v) {
@@ -485,8 +487,7 @@ __device__ __forceinline__ uint32_t workgroup_rank(const uint32_t (&key)[R], uin
   uint32_t top = 0;
 #pragma unroll
   for (int j = 0; j < R; j++) top = key[j] > top ? key[j] : top;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
+  top = wave_max_u32(top);
   if (lane == 0) s_part[0][wave] = top;
   __syncthreads();
 #pragma unroll
@@ -621,7 +622,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_pick_kernel(const GdArgs<CAP> 
         if (m == 0) break;
         uint32_t base = 0;
         if (lane == uint32_t(__builtin_ctzll(m))) base = atomicAdd(&s_n, uint32_t(__popcll(m)));
-        base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+        base = uint32_t(__builtin_amdgcn_readlane(int(base), __builtin_ctzll(m))) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
         if (in && base < kPickList) s_list[base] = m1;
         m1 = m2; m2 = m3;
         if (j == 2 && __ballot(in) != 0 && lane == 0) atomicAdd(&s_n, kPickList);   // a lane may hold a fourth: not all are listed
@@ -729,8 +730,7 @@ __global__ __launch_bounds__(kThreads) void gd_presample_kernel(const GdArgs<CAP
 #pragma unroll
   for (uint32_t j = 0; j < kPreTop; j++) {
     uint32_t top = key;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(top, o, kWave); top = v > top ? v : top; }
+    top = wave_max_u32(top);
     if (lane == j) mine = top;
     if (lane == uint32_t(__builtin_ctzll(__ballot(key == top)))) key = 0;
   }
@@ -834,7 +834,7 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
     uint32_t base = 0;
     if (lane == uint32_t(__builtin_ctzll(m)))
       base = atomicAdd(reinterpret_cast<uint32_t*>(sg.ws + l.hist) + way * kWayStep, uint32_t(__popcll(m)));
-    base = __shfl(base, __builtin_ctzll(m), kWave) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+    base = uint32_t(__builtin_amdgcn_readlane(int(base), __builtin_ctzll(m))) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
     if (!hit) return;
     if (base < way_room) reinterpret_cast<uint32_t*>(sg.ws + l.hitlist)[size_t(way) * way_room + base] = key;
     else seg_state(sg)->fallback = 1;
@@ -951,14 +951,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_exact_kernel(const GdArgs<CAP>
   const uint32_t mine = ways[way * kWayStep];
   const uint32_t c0 = ways[2 * lane * kWayStep], c1 = ways[(2 * lane + 1) * kWayStep];   // every wave for itself
   if (st->fallback) return;   // uniform: not all that were found had room
-  uint32_t incl = c0 + c1, most = c0 > c1 ? c0 : c1;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t v = __shfl_up(incl, o, kWave);
-    if (lane >= uint32_t(o)) incl += v;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(most, o, kWave); most = v > most ? v : most; }
+  const uint32_t incl = wave_prefix_u32(c0 + c1), most = wave_max_u32(c0 > c1 ? c0 : c1);
   const uint32_t found = __builtin_amdgcn_readlane(incl, kWave - 1);
   __syncthreads();   // nobody reads the state below
   if (found <= sg.thr_index) {
@@ -966,8 +959,7 @@ __global__ __launch_bounds__(kSelThreads) void gd_exact_kernel(const GdArgs<CAP>
     // less than zero, so that one is known)
     uint32_t equal = 0;
     if (st->ties) equal = ways[2 * lane * kWayStep + 1] + ways[(2 * lane + 1) * kWayStep + 1];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) equal += __shfl_xor(equal, o, kWave);
+    equal = wave_sum_u32(equal);
     if (t == 0 && prov != 0 && found + equal <= sg.thr_index) st->fallback = 1;
     return;
   }
@@ -1042,13 +1034,11 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
     }
     if (my_tile && sub == 0) wcnt[mine] = uint16_t(kept);
     constexpr int kTileLanes = int(kListLanes * (kThreads / kWave));
-    uint32_t c = sub == 0 ? kept : 0u;
-#pragma unroll
-    for (int o = 1; o < kTileLanes; o <<= 1) c += __shfl_xor(c, o, kWave);
-    if (my_tile && lane % kTileLanes == 0) cnt[tile0 + lane / kTileLanes] = c;
-#pragma unroll
-    for (int o = kTileLanes; o < kWave; o <<= 1) c += __shfl_xor(c, o, kWave);
-    all = c;
+    const uint32_t c = sub == 0 ? kept : 0u;
+    static_assert(kTileLanes == 16, "a tile's lists are a row of lanes");
+    const uint32_t tile_cnt = row_sum(c);
+    if (my_tile && lane % kTileLanes == 0) cnt[tile0 + lane / kTileLanes] = tile_cnt;
+    all = wave_sum_u32(c);
   } else {
     // A mask word per lane; then its 64 elements lane by lane, kRecountWords words' values requested together: a tile full
     // of candidates takes two rounds (with each lane walking its own word's bits this launch took 29 us for the 17 M elements
@@ -1087,8 +1077,7 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
       } while (left);
       if (keep != old) masks[size_t(tile) * kWave + lane] = keep;
       uint32_t c = uint32_t(__popcll(keep));
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, kWave);
+      c = wave_sum_u32(c);
       if (lane == 0) cnt[tile] = c;
       all += c;
     }
@@ -1096,8 +1085,7 @@ __global__ __launch_bounds__(kThreads) void gd_recount_kernel(const GdArgs<CAP> 
   // The group's total and largest |r|, from which the expand launch works its places out: a scan launch before it took 6.5 us
   // of a call with its hand-over.
   __shared__ uint32_t s_all[kThreads / kWave], s_big[kThreads / kWave];
-#pragma unroll
-  for (int o = 1; o < int(kListTiles); o <<= 1) { const uint32_t v = __shfl_xor(big, o, kWave); big = v > big ? v : big; }
+  big = wave_max_u32(big);   // zero in the other lanes
   if (lane == 0) { s_all[wave] = all; s_big[wave] = big; }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1194,8 +1182,7 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   // which of the wave's sixteen mask words have a bit set (lanes beyond the sixteenth hold zeros)
   const uint32_t any16 = uint32_t(__ballot((lo | hi) != 0u));
   uint32_t bigb = __float_as_uint(big);  // non-negative floats order like their bit patterns; a NaN is not an input
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(bigb, o, kWave); bigb = v > bigb ? v : bigb; }
+  bigb = wave_max_u32(bigb);
   __shared__ uint32_t s_cnt[kThreads / kWave], s_big[kThreads / kWave], s_any[kThreads / kWave];
   if (lane == 0) { s_cnt[wave] = cnt; s_big[wave] = bigb; s_any[wave] = any16; }
   __syncthreads();
@@ -1238,14 +1225,8 @@ __global__ __launch_bounds__(kSelThreads) void gd_scan_kernel(const GdArgs<CAP> 
     big = m > big ? m : big;
   }
   const uint32_t sum = c[0] + c[1] + c[2] + c[3];
-  uint32_t incl = sum;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t v = __shfl_up(incl, o, kWave);
-    if (lane >= uint32_t(o)) incl += v;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(big, o, kWave); big = v > big ? v : big; }
+  const uint32_t incl = wave_prefix_u32(sum);
+  big = wave_max_u32(big);
   if (lane == kWave - 1) { s_wave[wave] = incl; s_wmax[wave] = big; }
   __syncthreads();
   uint32_t before = 0, all = 0, allmax = 0;
@@ -1332,20 +1313,14 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     // chunk totals, two per lane: inclusive prefix over the lanes
     const uint32_t* __restrict__ chunk_max = reinterpret_cast<const uint32_t*>(sg.ws + l.cmax);
     const uint32_t a0 = 2 * lane < nchunks ? chunk_tot[2 * lane] : 0u, a1 = 2 * lane + 1 < nchunks ? chunk_tot[2 * lane + 1] : 0u;
-    uint32_t inc2 = a0 + a1;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t v = __shfl_up(inc2, o, kWave);
-      if (lane >= uint32_t(o)) inc2 += v;
-    }
+    const uint32_t inc2 = wave_prefix_u32(a0 + a1);
     total = __builtin_amdgcn_readlane(inc2, kWave - 1);
     ex0 = inc2 - a0 - a1;
     ex1 = ex0 + a0;
     if (tile0 == 0) {
       const uint32_t m0 = 2 * lane < nchunks ? chunk_max[2 * lane] : 0u, m1 = 2 * lane + 1 < nchunks ? chunk_max[2 * lane + 1] : 0u;
       mm = m0 > m1 ? m0 : m1;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(mm, o, kWave); mm = v > mm ? v : mm; }
+      mm = wave_max_u32(mm);
     }
   } else {
     // The counts of all tiles, or of all groups, four per lane and load (the array's padding may be read, not used): the
@@ -1381,19 +1356,10 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
         }
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      all += __shfl_xor(all, o, kWave);
-      before += __shfl_xor(before, o, kWave);
-      const uint32_t v = __shfl_xor(mm, o, kWave);
-      mm = v > mm ? v : mm;
-    }
-    uint32_t incl = mine;
-#pragma unroll
-    for (int o = 1; o < kExpandTiles; o <<= 1) {
-      const uint32_t v = __shfl_up(incl, o, kWave);
-      if (lane >= uint32_t(o)) incl += v;
-    }
+    all = wave_sum_u32(all);
+    before = wave_sum_u32(before);
+    mm = wave_max_u32(mm);
+    const uint32_t incl = wave_prefix_u32(mine);
     const uint32_t own = __builtin_amdgcn_readlane(incl, kExpandTiles - 1);  // this wave's candidates
     __shared__ uint32_t s_own[kThreads / kWave];
     if (lane == 0) { s_sum[0][wave] = all; s_sum[1][wave] = before; s_sum[2][wave] = mm; s_own[wave] = own; }
@@ -1446,17 +1412,13 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
     // All of the wave's candidates are in its lists: the tiles follow each other, so one prefix over the lists' lengths is
     // every list's place.
     const uint32_t own = sub == 0 ? listed : 0u;
-    uint32_t incl = own;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t v = __shfl_up(incl, o, kWave);
-      if (lane >= uint32_t(o)) incl += v;
-    }
+    const uint32_t incl = wave_prefix_u32(own);
     const uint32_t chunk = tile0 / kScanChunk;
     static_assert(kScanChunk % kExpandTiles == 0, "a wave's tiles are of one chunk");
-    const uint32_t start = scanned ? __shfl((chunk & 1u) ? ex1 : ex0, int(chunk >> 1), kWave) + tile_off[tile0]
+    const uint32_t start = scanned ? uint32_t(__builtin_amdgcn_readlane(int((chunk & 1u) ? ex1 : ex0), int(chunk >> 1))) + tile_off[tile0]
                                    : uint32_t(__builtin_amdgcn_readlane(own_off, 0));
-    const uint32_t at = start + __shfl(incl - own, int(lane - sub), kWave);
+    static_assert(kPer == 4, "a list's lanes are a quad");
+    const uint32_t at = start + uint32_t(__builtin_amdgcn_update_dpp(0, int(incl - own), 0x00, 0xF, 0xF, false));   // of the quad's first lane
     auto put = [&](uint32_t place, uint2 p) {
       if (cut) {
         cand[place] = int32_t(p.x | (p.y & sign));
@@ -1483,15 +1445,10 @@ __global__ __launch_bounds__(kThreads) void gd_expand_kernel(const GdArgs<CAP> a
   for (int j = 0; j < kExpandTiles; j++) {
     const uint32_t tile = tile0 + j < ntiles ? tile0 + j : ntiles - 1;
     const uint32_t chunk = tile / kScanChunk;
-    const uint32_t start = scanned ? __shfl((chunk & 1u) ? ex1 : ex0, int(chunk >> 1), kWave) + tile_off[tile]
+    const uint32_t start = scanned ? uint32_t(__builtin_amdgcn_readlane(int((chunk & 1u) ? ex1 : ex0), int(chunk >> 1))) + tile_off[tile]
                                    : uint32_t(__builtin_amdgcn_readlane(own_off, j));
     const uint32_t c = __popcll(m[j]);
-    uint32_t incl = c;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t v = __shfl_up(incl, o, kWave);
-      if (lane >= uint32_t(o)) incl += v;
-    }
+    const uint32_t incl = wave_prefix_u32(c);
     pos[j] = start + incl - c;
   }
   // The first candidate of each of the lane's 64-element groups: their values are loaded together.
@@ -1778,12 +1735,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
 
   // Exclusive scans over the bins, of the global totals and of this tile's
   // counts: within each of the first BINS / 64 waves, then across them.
-  uint32_t incl_g = total, incl_l = mine;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t vg = __shfl_up(incl_g, o, kWave), vl = __shfl_up(incl_l, o, kWave);
-    if (lane >= uint32_t(o)) { incl_g += vg; incl_l += vl; }
-  }
+  const uint32_t incl_g = wave_prefix_u32(total), incl_l = wave_prefix_u32(mine);
   if (t < BINS && lane == kWave - 1) { s_part[wave] = incl_g; s_part[kBinWaves + wave] = incl_l; }
   __syncthreads();  // also: every wave's row of s_cnt is complete
   if (t < BINS) {
@@ -1831,12 +1783,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
 // Exclusive prefix of `v` over the workgroup's lanes in order; `total` is the sum.  s_wave: a word per wave.
 __device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* s_wave, uint32_t& total) {
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  uint32_t incl = v;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t u = __shfl_up(incl, o, kWave);
-    if (lane >= uint32_t(o)) incl += u;
-  }
+  const uint32_t incl = wave_prefix_u32(v);
   if (lane == kWave - 1) s_wave[wave] = incl;
   __syncthreads();
   uint32_t before = 0;
@@ -2070,8 +2017,7 @@ __device__ __forceinline__ void cut_crowded(const CutArgs& f) {
     key[j] = live ? s_key[x] : 0u;
     big = key[j] > big ? key[j] : big;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { const uint32_t v = __shfl_xor(big, o, kWave); big = v > big ? v : big; }
+  big = wave_max_u32(big);
   if (lane == 0) s_max[wave] = big;
   __syncthreads();   // also: every pair has been read
 #pragma unroll
@@ -2106,12 +2052,7 @@ __device__ __forceinline__ void cut_crowded(const CutArgs& f) {
 #pragma unroll
       for (int w = 0; w < kSortWaves; w++) { c[w] = s_cnt[w][t]; mine += c[w]; }
     }
-    uint32_t incl = mine;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t v = __shfl_up(incl, o, kWave);
-      if (lane >= uint32_t(o)) incl += v;
-    }
+    const uint32_t incl = wave_prefix_u32(mine);
     if (t < BINS && lane == kWave - 1) s_part[wave] = incl;
     __syncthreads();
     if (t < BINS) {

@@ -109,34 +109,11 @@ struct DecArgs {
 };
 static_assert(sizeof(EncArgs<kCapLarge>) <= 9600 && sizeof(DecArgs<kCapLarge>) <= 9600, "kernel-argument budget");
 
-// Reductions over the 64 lanes of a wave through the lane-permuting forms of the move instruction (no LDS
-// round trips): within quads, within rows of 16, then row 0 into row 1 and row 2 into row 3, then rows 0-1
-// into rows 2-3; lane 63 holds the result and hands it to every lane.
-template <typename T, typename Op>
-__device__ __forceinline__ T wave_reduce(T v, Op op) {
-  static_assert(sizeof(T) == 4, "32-bit values");
-  auto perm = [](T x, auto ctrl, auto rows) {
-    const int xi = __builtin_bit_cast(int, x);
-    // lanes whose row is not named keep their own value
-    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(xi, xi, decltype(ctrl)::value, decltype(rows)::value, 0xF, false));
-  };
-  using std::integral_constant;
-  v = op(v, perm(v, integral_constant<int, 0xB1>{}, integral_constant<int, 0xF>{}));   // quad_perm [1,0,3,2]
-  v = op(v, perm(v, integral_constant<int, 0x4E>{}, integral_constant<int, 0xF>{}));   // quad_perm [2,3,0,1]
-  v = op(v, perm(v, integral_constant<int, 0x141>{}, integral_constant<int, 0xF>{}));  // row_half_mirror
-  v = op(v, perm(v, integral_constant<int, 0x140>{}, integral_constant<int, 0xF>{}));  // row_mirror
-  v = op(v, perm(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{}));  // row_bcast:15 into rows 1 and 3
-  v = op(v, perm(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{}));  // row_bcast:31 into rows 2 and 3
-  return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
 __device__ __forceinline__ float wave_min(float v) {
   return wave_reduce(v, [](float a, float b) { return b < a ? b : a; });
 }
 __device__ __forceinline__ float wave_max(float v) {
   return wave_reduce(v, [](float a, float b) { return b > a ? b : a; });
-}
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-  return wave_reduce(v, [](uint32_t a, uint32_t b) { return b < a ? b : a; });
 }
 
 // Block-wide (min, max, min-u32) over 4 waves.  Result valid in every thread.
