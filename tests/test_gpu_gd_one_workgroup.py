@@ -64,6 +64,24 @@ def test_cut_far_beyond_what_is_kept(gd, oracle_cpu, n, sr, dr):
     assert cut
 
 
+# one to eight pairs a lane, the most that are sorted, and one more, which the masks find; all from the pass's lists, whose entries
+# the pass has cleared in the residual: the dropped ones have to be back
+@pytest.mark.parametrize("found", [1049, 1050, 2048, 2049, 3072, 3073, 8192, 8193])
+@pytest.mark.parametrize("levels", [0, 300])
+def test_cut_of_listed_candidates(gd, oracle_cpu, found, levels):
+    n, seen = 1 << 20, 0
+    rng = np.random.default_rng(found)
+    r = np.zeros(n, np.float32)
+    at = (np.arange(found) * (n // found) + rng.integers(0, n // found, found)).astype(np.int64)
+    size = rng.uniform(0.5, 1, found) if levels == 0 else rng.integers(1, levels, found) / levels
+    r[at] = rng.choice([-1, 1], found) * size
+    for seed in range(3):
+        _, _, info = _check_encode(gd, oracle_cpu, np.zeros(n, np.float32), r.copy(), 3 / n, 1 - 1048.5 / n, seed << 24)
+        assert info["kept"] <= 1049
+        seen += info["candidates"] == found   # three samples of a million: all but always zeros
+    assert seen
+
+
 def _messages(rng, sizes, ks):
     out = []
     for n, k in zip(sizes, ks):

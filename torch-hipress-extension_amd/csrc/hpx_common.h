@@ -304,19 +304,20 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
   return wave_reduce(v, [](uint32_t a, uint32_t b) { return a + b; });
 }
-// Inclusive prefix sum over the lanes of a wave, all of them active, the same way: within rows of 16 by shifts of 1, 2, 4
-// and 8 lanes, then each row's last lane into the row behind it, and lane 31 into rows 2 and 3.
+// Inclusive prefix sum over the lanes of a row of 16, by shifts of 1, 2, 4 and 8 lanes (zero where there is no such lane).
+__device__ __forceinline__ uint32_t row_prefix_u32(uint32_t v) {
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x111, 0xF, 0xF, false));   // row_shr:1
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x112, 0xF, 0xF, false));
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x114, 0xF, 0xF, false));
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x118, 0xF, 0xF, false));
+  return v;
+}
+// Inclusive prefix sum over the lanes of a wave, all of them active: within rows of 16, then each row's last lane into the
+// row behind it, and lane 31 into rows 2 and 3.
 __device__ __forceinline__ uint32_t wave_prefix_u32(uint32_t v) {
-  auto from = [](uint32_t x, auto ctrl, auto rows) {   // zero where there is no such lane
-    return uint32_t(__builtin_amdgcn_update_dpp(0, int(x), decltype(ctrl)::value, decltype(rows)::value, 0xF, false));
-  };
-  using std::integral_constant;
-  v += from(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});   // row_shr:1
-  v += from(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
-  v += from(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
-  v += from(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
-  v += from(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});   // row_bcast:15 into rows 1 and 3
-  v += from(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});   // row_bcast:31 into rows 2 and 3
+  v = row_prefix_u32(v);
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x142, 0xA, 0xF, false));   // row_bcast:15 into rows 1 and 3
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x143, 0xC, 0xF, false));   // row_bcast:31 into rows 2 and 3
   return v;
 }
 

@@ -120,8 +120,8 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
 // 1024 elements exceed that next to never unless the large ones crowd together, and then the masks serve (of one million, half of the
 // large ones within one element in 1500: 49.3 us, 50.9 since there are lists to look at first).  The pass pays
 // for them (138 M elements 229 -> 232 us, ResNet-50's 161 tensors 46.7 -> 48.4, one of a million 4.3 -> 5.1); behind it the
-// expand launch takes 9.0 us instead of 14.4 (138 M), and the finish 8.8 instead of 11.7 for the million, 16.2 instead of 24.8 for
-// ResNet-50's 161.  Up to 12 in 1024: denser, the lists would be a tenth of the tensor.
+// expand launch takes 9.0 us instead of 14.4 (138 M), and the finish took 8.8 instead of 11.7 for the million, 16.2 instead of 24.8 for
+// ResNet-50's 161 (6.1 and 10.3 since).  Up to 12 in 1024: denser, the lists would be a tenth of the tensor.
 // Of the tensors that one workgroup settles (gd_finish_kernel) those with few candidates to a list have none either: the masks are
 // as quick there, or quicker, and the pass is without the lists' code and stores.  us per encode and decode of one tensor,
 // lists / masks: 20 thousand elements, 20 kept 23.3 / 21.7; 80 thousand, 80 kept 25.2 / 23.6; 120 thousand, 120 kept 28.2 / 27.7;
@@ -139,6 +139,11 @@ __host__ __device__ inline uint32_t list_room(uint32_t n, uint32_t limit) {
   const float mean = float(kWaveTile) * float(limit) / float(n);
   return mean > 12.0f ? 0u : (uint32_t(2.0f * mean) + 21u) & ~7u;
 }
+// Whether the pass leaves zeros in the residual where it lists a candidate's value.  Of a tensor that one workgroup settles nearly all
+// candidates are kept, and that workgroup wrote to as many lines of r, at about 700 a microsecond for one CU (ResNet-50's 161
+// tensors 16.2 us for that launch, 14.5 with this and the message written in order, the pass as long as before); it puts back
+// the few that a cut drops, and all of them where the lists turn out too short (gd_finish_kernel).
+__host__ __device__ inline bool clears_listed(uint32_t n, uint32_t limit) { return one_workgroup(n, limit) && list_room(n, limit) != 0; }
 __host__ __device__ inline size_t list_bytes(uint32_t n, uint32_t limit) {
   return align256(sizeof(uint64_t) * size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit));
 }
@@ -1127,12 +1132,19 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
   auto passes = [&](float x) { return PROV ? !(__builtin_fabsf(x) <= thr) : (x > thr) || (x < nthr); };  // gd_body.h:59-67
   uint2* __restrict__ list = seg_list(sg, l) + (size_t(t) * (kThreads / kWave) + wave) * room;
   uint32_t lo = 0, hi = 0, cnt = 0;
-  auto note = [&](uint64_t m, uint32_t e, float x) {  // m: the wave's candidates of 64 elements, uniform
+  const bool clears = LISTS && RESIDUAL && !PROV && clears_listed(n, sg.limit);
+  // m: the wave's candidates of 64 elements, uniform; the result is what the element leaves in r
+  auto note = [&](uint64_t m, uint32_t e, float x) {
+    float left = x;
     if (LISTS && m != 0) {
       const uint32_t at = cnt + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
-      if ((m >> lane & 1ull) && at < room) list[at] = make_uint2(e, __float_as_uint(x));
+      if ((m >> lane & 1ull) && at < room) {
+        list[at] = make_uint2(e, __float_as_uint(x));
+        if (clears) left = 0.0f;
+      }
     }
     cnt += uint32_t(__popcll(m));
+    return left;
   };
   float big = 0.0f;  // largest |x| this lane has seen
   float gv[kPerLane], rv[kPerLane];
@@ -1145,9 +1157,9 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
 #pragma unroll
     for (int c = 0; c < kPerLane; c++) {
       const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];  // thrust::plus<float>()(G, R), gd_body.h:121-128
-      if (RESIDUAL) __builtin_nontemporal_store(x, r + size_t(wbase) + c * kWave + lane);
       const uint64_t m = __ballot(passes(x));
-      note(m, wbase + c * kWave + lane, x);
+      const float left = note(m, wbase + c * kWave + lane, x);
+      if (RESIDUAL) __builtin_nontemporal_store(left, r + size_t(wbase) + c * kWave + lane);
       big = __builtin_fmaxf(big, __builtin_fabsf(x));
       lo = lane == uint32_t(c) ? uint32_t(m) : lo;  // lane c keeps mask word c
       hi = lane == uint32_t(c) ? uint32_t(m >> 32) : hi;
@@ -1167,12 +1179,12 @@ __global__ __launch_bounds__(kThreads) void gd_stream_kernel(const GdArgs<CAP> a
       bool p = false;
       const float x = RESIDUAL ? gv[c] + rv[c] : gv[c];
       if (e < n) {
-        if (RESIDUAL) r[e] = x;
         p = passes(x);
         big = __builtin_fmaxf(big, __builtin_fabsf(x));
       }
       const uint64_t m = __ballot(p);
-      note(m, e, x);
+      const float left = note(m, e, x);
+      if (RESIDUAL && e < n) r[e] = left;
       lo = lane == uint32_t(c) ? uint32_t(m) : lo;  // lane c keeps mask word c
       hi = lane == uint32_t(c) ? uint32_t(m >> 32) : hi;
     }
@@ -1780,22 +1792,37 @@ __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortAr
   }
 }
 
+// The sixteen waves' sums, folded: what lies before this wave's, and all of them.  A row of lanes reads them and shifts them
+// through itself.  (Sixteen waves on one CU: an instruction of each takes a SIMD sixteen cycles, so a hundred and fifty take a
+// microsecond.  Every wave walking the sixteen words took sixty.)
+__device__ __forceinline__ uint32_t before_wave(uint32_t sum_of_lane, uint32_t& total) {
+  static_assert(kSortWaves == 16, "a row of lanes");
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
+  const uint32_t incl = row_prefix_u32(sum_of_lane);
+  total = uint32_t(__builtin_amdgcn_readlane(int(incl), 15));
+  return uint32_t(__builtin_amdgcn_readlane(int(incl - sum_of_lane), wave));
+}
 // Exclusive prefix of `v` over the workgroup's lanes in order; `total` is the sum.  s_wave: a word per wave.
 __device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* s_wave, uint32_t& total) {
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const uint32_t incl = wave_prefix_u32(v);
   if (lane == kWave - 1) s_wave[wave] = incl;
   __syncthreads();
-  uint32_t before = 0;
-  total = 0;
-#pragma unroll
-  for (uint32_t w = 0; w < uint32_t(kSortWaves); w++) {
-    const uint32_t c = s_wave[w];
-    before += w < wave ? c : 0u;
-    total += c;
-  }
+  const uint32_t before = before_wave(s_wave[lane & 15], total);
   __syncthreads();
   return before + incl - v;
+}
+// The same with one barrier, for words of `s_wave` that nobody uses again before the next one; `any`: whether some lane's flag
+// is set (a wave's sum is below 2^31).
+__device__ __forceinline__ uint32_t block_prefix_once(uint32_t v, bool flag, uint32_t* s_wave, uint32_t& total, bool& any) {
+  const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const uint32_t incl = wave_prefix_u32(v);
+  const uint32_t marked = __ballot(flag) != 0 ? 0x80000000u : 0u;
+  if (lane == kWave - 1) s_wave[wave] = incl | marked;
+  __syncthreads();
+  const uint32_t c = s_wave[lane & 15];
+  any = __ballot((c >> 31) != 0) != 0;
+  return before_wave(c & 0x7FFFFFFFu, total) + incl - v;
 }
 
 // The `keep` largest |r| among the elements whose mask bit is set, in ascending index order, to LDS (keys as
@@ -1855,43 +1882,74 @@ __device__ __forceinline__ void top_of_masks(const uint64_t* __restrict__ masks,
 }
 
 // The cut by one workgroup, of up to kCutKeep candidates (listed ones: kCutLds, cut_wide).  What bounds it is the chain of workgroup-wide steps, so the sort
-// has as few as possible: the keys (distance of |r| above the threshold in bit patterns) go into 4096 bins by exponent
-// and seven further bits of the distance as a float - fine where keys crowd just above the threshold, however far the
-// largest lies - the bins are laid out one after the other, and a key's place is its bin's first place plus the number
+// has as few as possible: the keys (distance of |r| above the threshold in bit patterns) go into 8192 bins by exponent
+// and eight further bits of the distance as a float - fine where keys crowd just above the threshold, however far the
+// largest lies (4096 bins: 0.8 and 1.2 us longer over the comparisons within them, for 1049 and 2360 kept) - the bins are laid out one after the other, and a key's place is its bin's first place plus the number
 // of keys of the bin that come before it (larger, or equal with a smaller index).  Where a bin is crowded all the same
 // (many equal values) the keys take a stable LSD sort by byte digits, pairs in registers between the passes and in
 // LDS for the exchange.  The code is instantiated for the number of pairs per lane: unrolled for the
 // most a workgroup can hold it was three times as long, and a launch of one workgroup per tensor meets a cold
 // instruction cache.
-constexpr uint32_t kCutBins = 4096;
+constexpr uint32_t kCutBins = 8192;
+constexpr uint32_t kBinWords = kCutBins / 2;   // 16 bits each: there are at most kCutLds keys
 constexpr uint32_t kCutCrowd = 128;   // keys of one bin from which the digit sort is the quicker one
 struct CutArgs {
   uint32_t* stage;   // LDS: 2 * kCutLds words
-  uint32_t* bins;    // LDS: kCutBins + 4 words, the first kCutBins zero
-  uint32_t* wave;    // LDS: a word per wave
+  uint32_t* bins;    // LDS: kBinWords + 4 words, the first kBinWords zero
+  uint32_t* wave;    // LDS: a word per wave, of the cut's own
   float* r;
   uint8_t* out;
   uint32_t n, keep, thr_bits;
-  __device__ __forceinline__ void put(uint32_t place, uint32_t key, uint32_t id) const {   // an entry of the message
-    const uint32_t i = id & 0x7FFFFFFFu;
-    reinterpret_cast<int32_t*>(out + 4)[place] = int32_t(i);
-    reinterpret_cast<uint32_t*>(out + 4 + size_t(keep) * 4)[place] = (key + thr_bits) | (id & 0x80000000u);
-    r[i] = 0.0f;
+  bool cleared;      // r holds zeros at the candidates: the dropped ones go back.  Else their values: the kept ones are cleared
+  __device__ __forceinline__ uint32_t value(uint32_t key, uint32_t id) const { return (key + thr_bits) | (id & 0x80000000u); }
+  __device__ __forceinline__ void entry(uint32_t place, uint32_t key, uint32_t id) const {   // of the message
+    reinterpret_cast<uint32_t*>(out + 4)[place] = id & 0x7FFFFFFFu;
+    reinterpret_cast<uint32_t*>(out + 4 + size_t(keep) * 4)[place] = value(key, id);
+  }
+  __device__ __forceinline__ void residual(uint32_t place, uint32_t key, uint32_t id) const {
+    if (cleared != (place < keep)) r[id & 0x7FFFFFFFu] = cleared ? __uint_as_float(value(key, id)) : 0.0f;
+  }
+  __device__ __forceinline__ void put(uint32_t place, uint32_t key, uint32_t id) const {
+    if (place < keep) entry(place, key, id);
+    residual(place, key, id);
   }
 };
 
-__device__ __forceinline__ uint32_t cut_bin(uint32_t key) { return kCutBins - 1 - ((__float_as_uint(float(key)) >> 16) - (127u << 7)); }
+__device__ __forceinline__ uint32_t cut_bin(uint32_t key) { return kCutBins - 1 - ((__float_as_uint(float(key)) >> 15) - (127u << 8)); }
+// One more at a bin's count (or its next place); what was there before.
+__device__ __forceinline__ uint32_t bin_step(const CutArgs& f, uint32_t bin) {
+  const uint32_t shift = (bin & 1u) * 16u;
+  return (atomicAdd(&f.bins[bin >> 1], 1u << shift) >> shift) & 0xFFFFu;
+}
+__device__ __forceinline__ uint32_t bin_at(const CutArgs& f, uint32_t bin) { return reinterpret_cast<const uint16_t*>(f.bins)[bin]; }
 // From the counts of the bins to their first places, in place (all lanes, behind the barrier that follows the counting).
 // False: some bin is crowded, and the counts are still there.
 __device__ __forceinline__ bool bins_laid_out(const CutArgs& f) {
   const uint32_t t = threadIdx.x;
+  static_assert(kBinWords == 4 * kSortThreads && kCutLds < 65536, "four words to a lane, places of 16 bits");
   const uint4 c = reinterpret_cast<const uint4*>(f.bins)[t];
-  const uint32_t c01 = c.x > c.y ? c.x : c.y, c23 = c.z > c.w ? c.z : c.w;
+  const uint32_t word[4] = {c.x, c.y, c.z, c.w};
+  uint32_t sum = 0, most = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t a = word[k] & 0xFFFFu, b = word[k] >> 16;
+    sum += a + b;
+    most = a > most ? a : most;
+    most = b > most ? b : most;
+  }
   uint32_t total;
-  const uint32_t first = block_prefix(c.x + c.y + c.z + c.w, f.wave, total);
-  if (__syncthreads_or((c01 > c23 ? c01 : c23) > kCutCrowd)) return false;
-  reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
-  if (t == 0) f.bins[kCutBins] = total;
+  bool crowded;
+  uint32_t at = block_prefix_once(sum, most > kCutCrowd, f.wave, total, crowded);
+  if (crowded) return false;
+  uint32_t first[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t a = word[k] & 0xFFFFu, b = word[k] >> 16;
+    first[k] = at | ((at + a) << 16);
+    at += a + b;
+  }
+  reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(first[0], first[1], first[2], first[3]);
+  if (t == 0) f.bins[kBinWords] = total;
   __syncthreads();
   return true;
 }
@@ -1905,46 +1963,66 @@ __device__ __forceinline__ void stage_pairs(const CutArgs& f, const uint32_t (&k
   __syncthreads();
 }
 
+// A pair as one number, larger for what comes first: the key, then the smaller index (the sign in the last bit).
+__device__ __forceinline__ uint64_t ranked(uint32_t key, uint32_t id) { return (uint64_t(key) << 32) | ~((id << 1) | (id >> 31)); }
+__device__ __forceinline__ uint32_t ranked_key(uint64_t p) { return uint32_t(p >> 32); }
+__device__ __forceinline__ uint32_t ranked_id(uint64_t p) { const uint32_t x = ~uint32_t(p); return (x >> 1) | (x << 31); }
+
 // n pairs, lane t with those at t, t + 1024 ... (in ascending index order; the sign in the index's top bit).  False: some
 // bin is crowded, nothing has been written, and the pairs are in LDS, [kCutLds] keys and then [kCutLds] indices.
 template <int PER>
 __device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER]) {
   const uint32_t t = threadIdx.x, n = f.n;
-  uint2* s_pair = reinterpret_cast<uint2*>(f.stage);
-  uint32_t* s_bins = f.bins;
+  uint64_t* s_pair = reinterpret_cast<uint64_t*>(f.stage);
   uint32_t bin[PER], slot[PER];
 #pragma unroll
   for (int j = 0; j < PER; j++) {
     const bool live = uint32_t(j) * kSortThreads + t < n;
     bin[j] = live ? cut_bin(key[j]) : 0u;
-    slot[j] = live ? atomicAdd(&s_bins[bin[j]], 1u) : 0u;
+    slot[j] = live ? bin_step(f, bin[j]) : 0u;
   }
   __syncthreads();
   if (!bins_laid_out(f)) {
     stage_pairs<PER>(f, key, id);
     return false;
   }
-  uint32_t lo[PER], hi[PER], place[PER], longest = 0;
+  uint64_t own[PER];
+  uint32_t lo[PER], len[PER], place[PER], longest = 0;
 #pragma unroll
   for (int j = 0; j < PER; j++) {
     const bool live = uint32_t(j) * kSortThreads + t < n;
-    place[j] = lo[j] = live ? s_bins[bin[j]] : 0u;
-    hi[j] = live ? s_bins[bin[j] + 1] : 0u;
-    longest = hi[j] - lo[j] > longest ? hi[j] - lo[j] : longest;
-    if (live) s_pair[lo[j] + slot[j]] = make_uint2(key[j], id[j]);
+    own[j] = ranked(key[j], id[j]);
+    place[j] = lo[j] = live ? bin_at(f, bin[j]) : 0u;
+    len[j] = live ? bin_at(f, bin[j] + 1) - lo[j] : 0u;
+    slot[j] += lo[j];
+    longest = len[j] > longest ? len[j] : longest;
+    if (live) s_pair[slot[j]] = own[j];
   }
   __syncthreads();
+#pragma unroll 1
   for (uint32_t q = 0; q < longest; q++) {   // the lane's pairs side by side: their LDS reads overlap
-    uint2 k[PER];
+    uint64_t k[PER];
 #pragma unroll
-    for (int j = 0; j < PER; j++) k[j] = s_pair[lo[j] + q < hi[j] ? lo[j] + q : lo[j]];
+    for (int j = 0; j < PER; j++) k[j] = s_pair[q < len[j] ? lo[j] + q : slot[j]];   // (a pair is not larger than itself)
 #pragma unroll
-    for (int j = 0; j < PER; j++)
-      place[j] += lo[j] + q < hi[j] && (k[j].x > key[j] || (k[j].x == key[j] && (k[j].y << 1) < (id[j] << 1))) ? 1u : 0u;
+    for (int j = 0; j < PER; j++) place[j] += k[j] > own[j] ? 1u : 0u;
   }
+  // The entries in order, by way of LDS behind the pairs: a lane's own go to places all over the message, a line each of the
+  // indices and of the values.
+  static_assert(PER * kSortThreads <= int(kCutLds) / 2, "pairs and entries side by side");
+  uint64_t* s_entry = s_pair + PER * kSortThreads;
 #pragma unroll
   for (int j = 0; j < PER; j++)
-    if (lo[j] < hi[j] && place[j] < f.keep) f.put(place[j], key[j], id[j]);
+    if (len[j] != 0) {
+      s_entry[place[j]] = own[j];
+      f.residual(place[j], key[j], id[j]);
+    }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const uint32_t x = uint32_t(j) * kSortThreads + t;
+    if (x < f.keep) f.entry(x, ranked_key(s_entry[x]), ranked_id(s_entry[x]));
+  }
   return true;
 }
 
@@ -1954,7 +2032,7 @@ __device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&k
 __device__ __forceinline__ bool cut_wide(const CutArgs& f, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cand) {
   constexpr uint32_t kAtOnce = 4;
   const uint32_t t = threadIdx.x, n = f.n;
-  uint2* s_pair = reinterpret_cast<uint2*>(f.stage);
+  uint64_t* s_pair = reinterpret_cast<uint64_t*>(f.stage);
 #pragma unroll 1
   for (uint32_t x0 = t; x0 < n; x0 += kAtOnce * kSortThreads) {
     uint32_t key[kAtOnce];
@@ -1962,7 +2040,7 @@ __device__ __forceinline__ bool cut_wide(const CutArgs& f, const uint32_t* __res
     for (uint32_t j = 0; j < kAtOnce; j++) key[j] = x0 + j * kSortThreads < n ? keys[x0 + j * kSortThreads] : 0u;
 #pragma unroll
     for (uint32_t j = 0; j < kAtOnce; j++)
-      if (x0 + j * kSortThreads < n) atomicAdd(&f.bins[cut_bin(key[j])], 1u);
+      if (x0 + j * kSortThreads < n) bin_step(f, cut_bin(key[j]));
   }
   __syncthreads();
   if (!bins_laid_out(f)) return false;
@@ -1976,20 +2054,17 @@ __device__ __forceinline__ bool cut_wide(const CutArgs& f, const uint32_t* __res
     }
 #pragma unroll
     for (uint32_t j = 0; j < kAtOnce; j++)
-      if (x0 + j * kSortThreads < n) s_pair[atomicAdd(&f.bins[cut_bin(pair[j].x)], 1u)] = pair[j];
+      if (x0 + j * kSortThreads < n) s_pair[bin_step(f, cut_bin(pair[j].x))] = ranked(pair[j].x, pair[j].y);
   }
-  __syncthreads();   // a bin's word is now the place behind its last pair
+  __syncthreads();   // at a bin there is now the place behind its last pair
 #pragma unroll 1
   for (uint32_t x = t; x < n; x += kSortThreads) {
-    const uint2 own = s_pair[x];
-    const uint32_t b = cut_bin(own.x), lo = b ? f.bins[b - 1] : 0u, hi = f.bins[b];
+    const uint64_t own = s_pair[x];
+    const uint32_t b = cut_bin(ranked_key(own)), lo = b ? bin_at(f, b - 1) : 0u, hi = bin_at(f, b);
     uint32_t place = lo;
 #pragma unroll 4
-    for (uint32_t q = lo; q < hi; q++) {
-      const uint2 k = s_pair[q];
-      place += k.x > own.x || (k.x == own.x && (k.y << 1) < (own.y << 1)) ? 1u : 0u;
-    }
-    if (place < f.keep) f.put(place, own.x, own.y);
+    for (uint32_t q = lo; q < hi; q++) place += s_pair[q] > own ? 1u : 0u;
+    f.put(place, ranked_key(own), ranked_id(own));
   }
   return true;
 }
@@ -1999,12 +2074,12 @@ __device__ __forceinline__ void cut_crowded(const CutArgs& f) {
   constexpr uint32_t BINS = 256, kBinWaves = BINS / kWave;
   constexpr int kPer = int(kCutKeep) / kSortThreads;
   __shared__ uint32_t s_part[kBinWaves], s_max[kSortWaves];
-  static_assert(kCutBins >= kSortWaves * BINS, "one block for both");
+  static_assert(kBinWords >= kSortWaves * BINS, "one block for both");
   uint32_t (*s_cnt)[BINS] = reinterpret_cast<uint32_t (*)[BINS]>(f.bins);
   uint32_t* s_key = f.stage;
   uint32_t* s_id = f.stage + kCutLds;
   const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t / kWave);
-  const uint32_t n = f.n, keep = f.keep;
+  const uint32_t n = f.n;
   // pairs in order, the same number of rounds of 64 per wave for every wave
   const uint32_t per = cdiv(n, kSortThreads);
   const uint32_t x0 = wave * per * kWave + lane;
@@ -2082,7 +2157,7 @@ __device__ __forceinline__ void cut_crowded(const CutArgs& f) {
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
     const uint32_t p = uint32_t(j) * kSortThreads + t;
-    if (p < keep) f.put(p, s_key[p], s_id[p]);
+    if (p < n) f.put(p, s_key[p], s_id[p]);
   }
 }
 // Pairs from wherever `pair(x, key, id)` finds them.
@@ -2104,13 +2179,15 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // (as many as give every lane something to do), a lane after a run of the tile's mask words, of which the tile's coarse
 // word names the few that have a bit set; lanes in order, so one prefix over the workgroup's counts puts the indices
 // in ascending order in LDS.
-// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 8.8 us on average;
-// ResNet-50's 161 tensors 58 -> 16 us.
+// One tensor of 1 M: scan, expand and the cut's seven launches 36 us with the host's turn-around -> 6.1 us on average;
+// ResNet-50's 161 tensors 58 -> 10.3 us.  What bounds it is instructions (before_wave) and lines (list_room): from the kernel's
+// start, us, for a cut of 2481 to 2360, lengths 1.6, their prefix 2.1, places in LDS 3.9, entries 6.3, counted into bins 6.6, laid out
+// 8.0, compared 9.5, written 11 (before: 1.8, 2.5, 4.5, 6.7, 7.5, 9.2, 12.5, 14.5); a cut of 1230 to 1049 8 (before 10).
 // Larger ones that still fit are only cut here, behind the expand launch.  All of it is queued before the host knows any
 // count.
 // The cut of the tensors that keep between kFinishKeep and kCutKeep entries, whose candidates and keys the expand
 // launch has listed (or, where they are too many for the list or for LDS, are found again in the mask).
-__device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, uint32_t* s_bins, uint32_t* s_wave) {
+__device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, uint32_t* s_bins, uint32_t* s_wave, uint32_t* s_cut_wave) {
   const uint32_t found = seg_state(sg)->total, keep = sg.limit, thr_bits = seg_state(sg)->thr_bits;
   if (found <= keep) return;
   const uint32_t t = threadIdx.x;
@@ -2125,7 +2202,7 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
   };
   if (found <= sg.cap && found > kCutKeep && found <= kCutLds) {
     clear_bins();
-    if (cut_wide(CutArgs{s_stage, s_bins, s_wave, sg.r, sg.out, found, keep, thr_bits}, keys, cand)) return;
+    if (cut_wide(CutArgs{s_stage, s_bins, s_cut_wave, sg.r, sg.out, found, keep, thr_bits, false}, keys, cand)) return;
     __syncthreads();
   }
   const bool listed = found <= sg.cap && found <= kCutKeep;
@@ -2134,7 +2211,7 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
     top_of_masks(reinterpret_cast<const uint64_t*>(sg.ws + l.masks), sg.r, sg.n, keep, thr_bits, s_bins, s_wave, s_stage, s_stage + kCutLds);
   }
   clear_bins();
-  const CutArgs f{s_stage, s_bins, s_wave, sg.r, sg.out, listed ? found : keep, keep, thr_bits};
+  const CutArgs f{s_stage, s_bins, s_cut_wave, sg.r, sg.out, listed ? found : keep, keep, thr_bits, false};
   bool done;
   if (listed) {
     auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) { key = keys[x]; id = cand[x]; };
@@ -2148,14 +2225,14 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
 template <int CAP>
 __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CAP> a) {
   extern __shared__ uint32_t s_stage[];          // [kCutLds] keys, then [kCutLds] indices; or pairs of them
-  __shared__ __align__(16) uint32_t s_bins[kCutBins + 4];   // counts, then first places; the rank search's histogram; the digit sort's counts
-  __shared__ uint32_t s_wave[kSortWaves];
-  static_assert(kCutBins >= uint32_t(kBins1), "one block for both");
+  __shared__ __align__(16) uint32_t s_bins[kBinWords + 4];   // counts, then first places; the rank search's histogram; the digit sort's counts
+  __shared__ uint32_t s_wave[kSortWaves], s_cut_wave[kSortWaves];
+  static_assert(kBinWords >= uint32_t(kBins1), "one block for both");
   uint32_t* s_key = s_stage;
   uint32_t* s_id = s_stage + kCutLds;
   const GdSeg& sg = a.seg[find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x)];
   if (!one_workgroup(sg.n, sg.limit)) {
-    cut_listed(sg, s_stage, s_bins, s_wave);
+    cut_listed(sg, s_stage, s_bins, s_wave, s_cut_wave);
     return;
   }
   const GdLayout l = gd_layout(sg.n, sg.sample_cnt);
@@ -2168,8 +2245,10 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
 
   // The pass's own lists, a few of them to a lane: where each entry of the tensor's list of candidates lies, and then the
   // entries, each a load that depends on nothing but its place.  (Through the masks every candidate is a word of the mask and
-  // then a line of r.)
+  // then a line of r.  Each list's first entries requested along with its length, six to a lane: as many requests as there are
+  // lists, times three, which one CU takes 3 us over for 2304 of them.)
   const uint32_t room = list_room(sg.n, keep);
+  const bool cleared = a.residual != 0 && clears_listed(sg.n, keep);
   const uint2* __restrict__ list = seg_list(sg, l);
   bool lists = false;
   uint32_t n = 0, pos = 0;
@@ -2189,8 +2268,9 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
 #pragma unroll
       for (uint32_t q = 0; q < kAtOnce; q++) { mine += c[q]; over = over || c[q] > room; }
     }
-    pos = block_prefix(mine, s_wave, n);
-    lists = !__syncthreads_or(over || n > kCutKeep);
+    bool some_over;
+    pos = block_prefix_once(mine, over, s_wave, n, some_over);
+    lists = !some_over && n <= kCutKeep;
     if (lists) {
       for (uint32_t q0 = 0; q0 < per; q0 += kAtOnce) {
         if (per > kAtOnce) take(q0);
@@ -2214,21 +2294,34 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
             if (x < n) {
               idx[x] = int32_t(e[j].x);
               val[x] = e[j].y;
-              r[e[j].x] = 0.0f;
+              if (!cleared) r[e[j].x] = 0.0f;
             }
           }
         }
         return;
       }
-      const CutArgs f{s_stage, s_bins, s_wave, r, sg.out, n, keep, thr_bits};
+      const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, cleared};
       auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
         const uint2 e = list[s_id[x]];
         key = (e.y & 0x7FFFFFFFu) - thr_bits;
         id = e.x | (e.y & 0x80000000u);
       };
-      const bool done = n <= kSortThreads ? cut_loaded<1>(f, pair) : n <= 3 * kSortThreads ? cut_loaded<3>(f, pair) : cut_loaded<8>(f, pair);
+      const bool done = n <= kSortThreads       ? cut_loaded<1>(f, pair)
+                        : n <= 2 * kSortThreads ? cut_loaded<2>(f, pair)
+                        : n <= 3 * kSortThreads ? cut_loaded<3>(f, pair)
+                                                : cut_loaded<8>(f, pair);
       if (!done) cut_crowded(f);
       return;
+    }
+    // Too many for a list, or for the workgroup: the masks name them, and their values are looked up in r.
+    if (cleared) {
+      for (uint32_t q = first; q < first + per && q < nlists; q++) {
+        const uint32_t in_list = lengths[q] < room ? lengths[q] : room;
+        for (uint32_t j = 0; j < in_list; j++) {
+          const uint2 e = list[size_t(q) * room + j];
+          r[e.x] = __uint_as_float(e.y);
+        }
+      }
     }
     __syncthreads();
   }
@@ -2308,7 +2401,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
     }
     return;
   }
-  const CutArgs f{s_stage, s_bins, s_wave, r, sg.out, n, keep, thr_bits};
+  const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, false};
   auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
     id = s_id[x];
     const uint32_t v = __float_as_uint(r[id & 0x7FFFFFFFu]);
