@@ -1,0 +1,65 @@
+"""GPU parity of the sparsifier's cut in one launch (gd_order_kernel), tensors that keep 8192 entries and more, at the sizes and
+kinds of values where it can go wrong: the fewest and the most candidates it takes and one more, few distinct values (bins that
+are crowded), one value that more share than a window holds (the digit sort behind it), all candidates side by side, and
+several tensors in a call.  Bit-exact against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import assert_bits_equal, dev, host
+from test_gpu_gd import Gd, _check_encode
+
+pytestmark = pytest.mark.gpu
+MOST = 224 * 1024
+
+
+@pytest.fixture(scope="module")
+def gd(capi):
+    return Gd(capi)
+
+
+def _candidates(rng, n, found, kind):
+    """A residual of zeros but for `found` elements."""
+    r = np.zeros(n, np.float32)
+    at = np.arange(n - found, n) if kind == "together" else np.sort(rng.choice(n, found, replace=False))
+    x = rng.laplace(0, 1e-3, found)
+    x = np.where(np.abs(x) < 1e-6, 1e-6, x).astype(np.float32)
+    if kind == "bf16":
+        x = (x.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    if kind == "shared":   # more than half of them, between larger and smaller ones
+        share = rng.random(found) < 0.6
+        x[share] = np.float32(1e-3) * rng.choice([-1, 1], int(share.sum())).astype(np.float32)
+    if kind == "equal":
+        x[:] = np.float32(0.25) * rng.choice([-1, 1], found).astype(np.float32)
+    r[at] = x
+    return r
+
+
+@pytest.mark.parametrize("kind", ["spread", "together", "bf16", "shared", "equal"])
+@pytest.mark.parametrize("found,keep", [(8193, 8192), (9217, 8200), (16_385, 12_000), (60_001, 59_000), (MOST - 3, 100_000), (MOST, MOST - 1),
+                                        (MOST + 1, MOST - 5)])
+def test_cut_of_many(gd, oracle_cpu, found, keep, kind):
+    n, seen = 8 * found + 3, 0
+    rng = np.random.default_rng(found)
+    r = _candidates(rng, n, found, kind)
+    for seed in range(3):
+        _, _, info = _check_encode(gd, oracle_cpu, np.zeros(n, np.float32), r.copy(), 1 / n, 1 - (keep - 0.5) / n, seed << 24)
+        seen += info["candidates"] == found   # the one sample is a zero
+    assert seen
+
+
+def test_several_tensors(gd, oracle_cpu):
+    rng = np.random.default_rng(1)
+    found, keep, kinds = (9000, 30_000, 20_000, 12_345), (8500, 20_000, 19_999, 8192), ("spread", "equal", "bf16", "together")
+    rs = [_candidates(rng, 40 * f, f, k) for f, k in zip(found, kinds)]
+    drops = [1 - (k - 0.5) / r.size for k, r in zip(keep, rs)]
+    rates = [1 / r.size for r in rs]
+    for seed in (0, 5 << 24):
+        gs, d_r = [torch.zeros(r.size, device="cuda") for r in rs], [dev(r) for r in rs]
+        outs = [torch.zeros(4 + 8 * k, dtype=torch.uint8, device="cuda") for k in keep]
+        gd.encode(gs, d_r, outs, rates, drops, [seed] * len(rs))
+        for r, rate, d, got_r, out in zip(rs, rates, drops, d_r, outs):
+            want_r = r.copy()
+            msg = oracle_cpu.gd_encode(np.zeros(r.size, np.float32), want_r, rate, d, seed)[0]
+            assert_bits_equal(host(out)[:msg.size], msg, "message")
+            assert_bits_equal(host(got_r), want_r, "residual")

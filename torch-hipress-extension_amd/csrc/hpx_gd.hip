@@ -1556,6 +1556,7 @@ struct SortArgs {
   int32_t shift;
   int32_t parity;
   int32_t last;            // this pass writes the messages
+  uint32_t* told;          // pinned host memory: a word for each window of gd_order_kernel
   int32_t tile_start[CAP + 1];
   SortSeg seg[CAP];
 };
@@ -1623,7 +1624,7 @@ template <int CAP, int BITS>
 __global__ __launch_bounds__(kSortThreads) void gd_sort_pass_kernel(const SortArgs<CAP> a) {
   constexpr uint32_t BINS = 1u << BITS;
   constexpr uint32_t kBinWaves = BINS / kWave;    // waves whose lanes each look after one bin
-  extern __shared__ uint32_t s_stage[];          // [kSortTile] keys, then [kSortTile] indices
+  extern __shared__ __align__(16) uint32_t s_stage[];          // [kSortTile] keys, then [kSortTile] indices
   __shared__ uint32_t s_cnt[kSortWaves][BINS];   // per wave: pairs per bin, then the wave's first place per bin
   __shared__ uint32_t s_first[BINS];             // first place of the bin within the tile
   __shared__ uint32_t s_slot[BINS];              // first global slot of the bin's pairs of this tile
@@ -1901,10 +1902,11 @@ struct CutArgs {
   uint8_t* out;
   uint32_t n, keep, thr_bits;
   bool cleared;      // r holds zeros at the candidates: the dropped ones go back.  Else their values: the kept ones are cleared
+  uint32_t first, all;   // place in the message of the largest pair at hand, and entries of the message
   __device__ __forceinline__ uint32_t value(uint32_t key, uint32_t id) const { return (key + thr_bits) | (id & 0x80000000u); }
   __device__ __forceinline__ void entry(uint32_t place, uint32_t key, uint32_t id) const {   // of the message
-    reinterpret_cast<uint32_t*>(out + 4)[place] = id & 0x7FFFFFFFu;
-    reinterpret_cast<uint32_t*>(out + 4 + size_t(keep) * 4)[place] = value(key, id);
+    reinterpret_cast<uint32_t*>(out + 4)[first + place] = id & 0x7FFFFFFFu;
+    reinterpret_cast<uint32_t*>(out + 4 + size_t(all) * 4)[first + place] = value(key, id);
   }
   __device__ __forceinline__ void residual(uint32_t place, uint32_t key, uint32_t id) const {
     if (cleared != (place < keep)) r[id & 0x7FFFFFFFu] = cleared ? __uint_as_float(value(key, id)) : 0.0f;
@@ -1970,8 +1972,10 @@ __device__ __forceinline__ uint32_t ranked_id(uint64_t p) { const uint32_t x = ~
 
 // n pairs, lane t with those at t, t + 1024 ... (in ascending index order; the sign in the index's top bit).  False: some
 // bin is crowded, nothing has been written, and the pairs are in LDS, [kCutLds] keys and then [kCutLds] indices.
-template <int PER>
-__device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER]) {
+// `placed` is called by every lane once it is known that no bin is.
+struct Nothing { __device__ __forceinline__ void operator()() const {} };
+template <int PER, typename Placed = Nothing>
+__device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER], Placed placed = {}) {
   const uint32_t t = threadIdx.x, n = f.n;
   uint64_t* s_pair = reinterpret_cast<uint64_t*>(f.stage);
   uint32_t bin[PER], slot[PER];
@@ -1986,6 +1990,7 @@ __device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&k
     stage_pairs<PER>(f, key, id);
     return false;
   }
+  placed();
   uint64_t own[PER];
   uint32_t lo[PER], len[PER], place[PER], longest = 0;
 #pragma unroll
@@ -2172,6 +2177,188 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
   return cut_by_bins<PER>(f, key, id);
 }
 
+// The cut of a tensor that keeps kCutKeep entries and more, in one launch.  A workgroup takes a window of the keys, from one
+// quantile of them to the next, about kWindow pairs: the windows' bounds come from kWindowSample of the keys, one out of so
+// many, which every workgroup ranks for itself; then it reads all the keys, counts those above its window, which is the
+// place of its largest in the message, collects its own in LDS and places them as a workgroup does that has them all.  What
+// bounds it is instructions, of that walk over all keys by each and of the largest window (1024 pairs on average 27 us for 138
+// thousand, 2048 40, with 1024 keys to take the bounds from 33).  The digit sort's six launches took 44 and more: us per
+// encode with a cut, sort -> windows, 10 thousand kept of 1 M 62.6 -> 44.5 and of 10 M 92 -> 74.5, 20 thousand 119.5 -> 102,
+// 60 thousand 201 -> 184, 120 thousand 104 -> 91 (12 M), 138 thousand 361 -> 345, 200 thousand 137.5 -> 127; 400 thousand
+// 205 -> 233, which is why kOrderMax lies between; bf16 values 62.6 -> 51 (1 M) and 366 -> 351 (138 M).
+// Where a window would have more pairs than fit (a value that thousands share) it says so, and the host, which waits for a word of
+// every window, queues the digit sort behind it, which writes the message anew: that detour takes 14 us (20 M elements, 30 thousand of one
+// size 109 -> 122).
+constexpr uint32_t kWindow = 1024, kWindowSample = 512;
+constexpr uint32_t kOrderMax = 224 * 1024;   // candidates
+constexpr uint32_t kWindowFits = 1u, kWindowFails = 2u;
+// False: a bin is crowded (many equal keys), nothing has been written, and the pairs are in LDS as cut_crowded takes them, in the
+// order of the candidates.  That order comes from bins of the places among those, so wide that no more than kWideBin can share one.
+template <int PER, typename Placed>
+__device__ __forceinline__ bool window_by_bins(const CutArgs& f, uint32_t below, const uint32_t* s_found,
+                                               const uint32_t* __restrict__ keys, const int32_t* __restrict__ ids, Placed placed) {
+  constexpr uint32_t kWideBin = (kOrderMax + kCutBins - 1) / kCutBins;
+  static_assert(kWideBin <= kCutCrowd, "no bin of places is crowded");
+  const uint32_t t = threadIdx.x;
+  uint32_t key[PER], id[PER], at[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const uint32_t x = uint32_t(j) * kSortThreads + t;
+    at[j] = s_found[x < f.n ? x : f.n - 1];
+    key[j] = keys[at[j]] - below;
+    id[j] = uint32_t(ids[at[j]]);
+  }
+  if (cut_by_bins<PER>(f, key, id, placed)) return true;
+  reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
+  uint32_t slot[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++) slot[j] = uint32_t(j) * kSortThreads + t < f.n ? bin_step(f, at[j] / kWideBin) : 0u;
+  __syncthreads();
+  bins_laid_out(f);
+  uint32_t* s_at = f.stage + kCutLds + kCutKeep;
+#pragma unroll
+  for (int j = 0; j < PER; j++)
+    if (uint32_t(j) * kSortThreads + t < f.n) s_at[bin_at(f, at[j] / kWideBin) + slot[j]] = at[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    if (uint32_t(j) * kSortThreads + t >= f.n) continue;
+    const uint32_t lo = bin_at(f, at[j] / kWideBin), hi = bin_at(f, at[j] / kWideBin + 1);
+    uint32_t place = lo;
+#pragma unroll 1
+    for (uint32_t q = lo; q < hi; q++) place += s_at[q] < at[j] ? 1u : 0u;
+    f.stage[place] = key[j];
+    f.stage[kCutLds + place] = id[j];
+  }
+  __syncthreads();
+  return false;
+}
+template <int CAP>
+__global__ __launch_bounds__(kSortThreads) void gd_order_kernel(const SortArgs<CAP> a) {
+  // (Aligned by name: behind an odd number of words the pairs' 64-bit accesses took this launch from 27 to 42 us.)
+  extern __shared__ __align__(16) uint32_t s_stage[];   // 2 * kCutLds words: where the window's keys lie, a list per wave and then all of them; the pairs
+  __shared__ __align__(16) uint32_t s_bins[kBinWords + 4];
+  __shared__ uint32_t s_wave[kSortWaves], s_cut_wave[kSortWaves], s_bound[2], s_heavy;
+  const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int s = find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x);
+  const SortSeg& sg = a.seg[s];
+  const uint32_t window = uint32_t(int(blockIdx.x) - a.tile_start[s]), windows = uint32_t(a.tile_start[s + 1] - a.tile_start[s]);
+  const CutLayout cl = cut_layout(sg.cap);
+  const uint32_t* __restrict__ keys = sort_keys(sg, cl, 0);
+  const uint32_t n = sg.n, keep = sg.keep;
+  auto tell = [&](uint32_t what) {
+    if (t == 0) __hip_atomic_store(a.told + blockIdx.x, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
+  if (wave < 3) {   // (the others too: 4 us more, a request for each of their keys)
+    constexpr uint32_t kOwn = kWindowSample / kWave;
+    uint32_t key[kOwn];
+#pragma unroll
+    for (uint32_t j = 0; j < kOwn; j++) key[j] = keys[uint32_t(uint64_t(j * kWave + lane) * n / kWindowSample)];
+    if (wave < 2) {   // one wave for each bound
+      const uint32_t w = window + wave;
+      uint32_t bound = w == 0 ? 0xFFFFFFFFu : 1u;   // keys are at least 1
+      if (w > 0 && w < windows) {
+        bound = wave_rank<int(kOwn), 0>(key, uint32_t(uint64_t(w) * kWindowSample / windows), 0u);
+        bound = bound > 1u ? bound : 1u;
+      }
+      if (lane == 0) s_bound[wave] = bound;
+    } else {          // ... and one looks how often some of the sample come up in it
+      uint32_t most = 0;
+#pragma unroll 1
+      for (int p = 0; p < kWave; p += 4) {
+        const uint32_t probe = uint32_t(__builtin_amdgcn_readlane(int(key[0]), p));
+        uint32_t equal = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kOwn; j++) equal += uint32_t(__popcll(__ballot(key[j] == probe)));
+        most = equal > most ? equal : most;
+      }
+      if (lane == 0) s_heavy = uint64_t(most) * n > uint64_t(kCutKeep) * kWindowSample ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+  if (s_heavy != 0) {   // some window would not hold it
+    tell(kWindowFails);
+    return;
+  }
+  const uint32_t hi = s_bound[0], lo = s_bound[1], below = lo - 1;
+  if (window == 0 && t == 0) *reinterpret_cast<int32_t*>(sg.msg) = int32_t(4 + keep * 8);
+  if (hi == lo) {   // its quantiles are one value, the lower bound of the window before it
+    tell(kWindowFits);
+    return;
+  }
+  // A lane marks those of its sixteen keys that are in the window, and the wave then lists the marked ones, one of each lane at
+  // a time: no branch on the way (with one at every key the walk over 138 thousand took 20 us).
+  constexpr uint32_t kListOf = kCutLds / kSortWaves;   // a wave's list, next to sixteen times what it finds on average
+  uint32_t* s_list = s_stage + wave * kListOf;
+  uint32_t above = 0, mine = 0;                         // of the wave
+  constexpr uint32_t kAtOnce = 4;
+  const uint4* __restrict__ quads = reinterpret_cast<const uint4*>(keys);
+  const uint32_t last = (n - 1) / 4, span = hi - lo;
+#pragma unroll 1
+  for (uint32_t q0 = 0; q0 <= last; q0 += kAtOnce * kSortThreads) {
+    uint4 k[kAtOnce];
+    uint32_t marks = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kAtOnce; j++) {
+      const uint32_t q = q0 + j * kSortThreads + t;
+      k[j] = quads[q < last ? q : last];
+    }
+    const bool ends = q0 + kAtOnce * kSortThreads > last;   // uniform
+#pragma unroll
+    for (uint32_t j = 0; j < kAtOnce; j++) {
+      const uint32_t x = 4 * (q0 + j * kSortThreads + t);
+      uint32_t v[4] = {k[j].x, k[j].y, k[j].z, k[j].w};
+      if (ends) {   // zeros are below every window
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) v[i] = x + i < n ? v[i] : 0u;
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) {
+        above += uint32_t(__popcll(__ballot(v[i] >= hi)));
+        marks |= v[i] - lo < span ? 1u << (4 * j + i) : 0u;
+      }
+    }
+#pragma unroll 1
+    for (uint64_t some = __ballot(marks != 0); some != 0; some = __ballot(marks != 0)) {
+      const uint32_t at = mine + __builtin_amdgcn_mbcnt_hi(uint32_t(some >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(some), 0u));
+      const uint32_t i = marks ? uint32_t(__builtin_ctz(marks)) : 0u;
+      if (marks != 0 && at < kListOf) s_list[at] = 4 * (q0 + i / 4 * kSortThreads + t) + i % 4;
+      marks &= marks - 1;   // 0 stays 0
+      mine += uint32_t(__popcll(some));
+    }
+  }
+  if (lane == 0) { s_wave[wave] = above; s_cut_wave[wave] = mine; }
+  __syncthreads();
+  uint32_t first, found;
+  before_wave(s_wave[lane & 15], first);
+  const uint32_t in_wave = s_cut_wave[lane & 15], start = before_wave(in_wave, found);
+  const bool long_list = __ballot(in_wave > kListOf) != 0;
+  if (found == 0 || first >= keep) {   // nothing of it is sent
+    tell(kWindowFits);
+    return;
+  }
+  if (long_list || found > kCutKeep) {
+    tell(kWindowFails);
+    return;
+  }
+  uint32_t* s_found = s_stage + kCutLds;
+  for (uint32_t i = lane; i < mine; i += kWave) s_found[start + i] = s_list[i];
+  __syncthreads();
+  const uint32_t kept = keep - first < found ? keep - first : found;
+  const CutArgs f{s_stage, s_bins, s_cut_wave, sg.r, sg.msg, found, kept, sg.thr_bits + below, false, first, keep};
+  const int32_t* __restrict__ ids = sort_ids(sg, cl, 0);
+  auto placed = [&]() { tell(kWindowFits); };
+  const bool done = found <= 2 * kSortThreads   ? window_by_bins<2>(f, below, s_found, keys, ids, placed)
+                    : found <= 3 * kSortThreads ? window_by_bins<3>(f, below, s_found, keys, ids, placed)
+                    : found <= 4 * kSortThreads ? window_by_bins<4>(f, below, s_found, keys, ids, placed)
+                                                : window_by_bins<8>(f, below, s_found, keys, ids, placed);
+  if (done) return;
+  tell(kWindowFits);
+  cut_crowded(f);
+}
+
 // What is left to do for a tensor that keeps at most kFinishKeep entries once the pass has marked its candidates,
 // by one workgroup in one launch: list them, cut them if there are too many, write the message and clear the
 // residual.  (Beyond that the values' random reads and the clearing's random writes, at about 700 lines a
@@ -2202,7 +2389,7 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
   };
   if (found <= sg.cap && found > kCutKeep && found <= kCutLds) {
     clear_bins();
-    if (cut_wide(CutArgs{s_stage, s_bins, s_cut_wave, sg.r, sg.out, found, keep, thr_bits, false}, keys, cand)) return;
+    if (cut_wide(CutArgs{s_stage, s_bins, s_cut_wave, sg.r, sg.out, found, keep, thr_bits, false, 0, keep}, keys, cand)) return;
     __syncthreads();
   }
   const bool listed = found <= sg.cap && found <= kCutKeep;
@@ -2211,7 +2398,7 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
     top_of_masks(reinterpret_cast<const uint64_t*>(sg.ws + l.masks), sg.r, sg.n, keep, thr_bits, s_bins, s_wave, s_stage, s_stage + kCutLds);
   }
   clear_bins();
-  const CutArgs f{s_stage, s_bins, s_cut_wave, sg.r, sg.out, listed ? found : keep, keep, thr_bits, false};
+  const CutArgs f{s_stage, s_bins, s_cut_wave, sg.r, sg.out, listed ? found : keep, keep, thr_bits, false, 0, keep};
   bool done;
   if (listed) {
     auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) { key = keys[x]; id = cand[x]; };
@@ -2224,7 +2411,7 @@ __device__ __forceinline__ void cut_listed(const GdSeg& sg, uint32_t* s_stage, u
 
 template <int CAP>
 __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CAP> a) {
-  extern __shared__ uint32_t s_stage[];          // [kCutLds] keys, then [kCutLds] indices; or pairs of them
+  extern __shared__ __align__(16) uint32_t s_stage[];          // [kCutLds] keys, then [kCutLds] indices; or pairs of them
   __shared__ __align__(16) uint32_t s_bins[kBinWords + 4];   // counts, then first places; the rank search's histogram; the digit sort's counts
   __shared__ uint32_t s_wave[kSortWaves], s_cut_wave[kSortWaves];
   static_assert(kBinWords >= uint32_t(kBins1), "one block for both");
@@ -2300,7 +2487,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
         }
         return;
       }
-      const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, cleared};
+      const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, cleared, 0, keep};
       auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
         const uint2 e = list[s_id[x]];
         key = (e.y & 0x7FFFFFFFu) - thr_bits;
@@ -2401,7 +2588,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
     }
     return;
   }
-  const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, false};
+  const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, false, 0, keep};
   auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
     id = s_id[x];
     const uint32_t v = __float_as_uint(r[id & 0x7FFFFFFFu]);
@@ -2546,11 +2733,12 @@ int sort_passes(SortArgs<CAP>& a, int passes, hipStream_t st) {
   return HPX_OK;
 }
 
-// The cut path for up to CAP tensors: the sort over all of them (as many digits as the largest key of any of
+// The cut path of what gd_order_kernel does not take, for up to CAP tensors: the sort over all of them (as many digits as the largest key of any of
 // them has; digits of 9 bits where that takes fewer passes than bytes), whose last pass writes the messages.
 template <int CAP>
 int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
   SortArgs<CAP> a;
+  a.told = nullptr;
   a.nseg = count;
   int bits = 1;
   a.tile_start[0] = 0;
@@ -2565,6 +2753,26 @@ int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
   return HPX_OK;
 }
 
+// The cut path in one launch, a word of `told` for each of the windows (cleared by the caller).
+template <int CAP>
+int launch_order(const CutJob* jobs, int count, uint32_t* told, hipStream_t st) {
+  SortArgs<CAP> a;
+  a.nseg = count;
+  a.shift = a.parity = a.last = 0;
+  a.told = told;
+  a.tile_start[0] = 0;
+  for (int i = 0; i < count; i++) {
+    a.seg[i] = jobs[i].seg;
+    a.tile_start[i + 1] = a.tile_start[i] + int32_t(cdiv(jobs[i].seg.n, kWindow));
+  }
+  constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));
+  static std::atomic<uint64_t> attr_done{0};
+  if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_order_kernel<CAP>), kStageBytes, attr_done)) return rc;
+  HPX_LAUNCH_LDS("gd_order_kernel", hpx::g_prof_on, gd_order_kernel<CAP>, dim3(uint32_t(a.tile_start[count])), dim3(kSortThreads), kStageBytes, st, a);
+  HPX_HIP(hipGetLastError());
+  return HPX_OK;
+}
+
 // What the host works out per tensor before anything is launched (size arithmetic of gd_body.h:112-115, :153;
 // dgc_body.h:79-80, :103).
 struct Plan {
@@ -2574,8 +2782,8 @@ struct Plan {
 };
 
 // Who settles a tensor behind the pass: one workgroup (gd_finish_kernel); the expand launch and, if it has to be cut, one
-// workgroup (the same launch: its LDS holds what is kept); or the expand launch and the host, which queues the sort of
-// many workgroups once it has heard the count.  The provisional path keeps to the last: it may have to fall back.
+// workgroup (the same launch: its LDS holds what is kept); or the expand launch and the host, which queues the cut by
+// many workgroups (gd_order_kernel, or the digit sort) once it has heard the count.  The provisional path keeps to the last: it may have to fall back.
 bool finishes(const GdSeg& sg, int margin) { return margin < 0 && one_workgroup(sg.n, sg.limit); }
 bool cut_on_device(const GdSeg& sg, int margin) { return margin < 0 && sg.limit < kCutKeep; }
 
@@ -2739,6 +2947,36 @@ int wait_word(volatile unsigned long long* word, hipStream_t st) {
     hpx::set_error("sparsifier decode: the headers were not reported");
     return HPX_ERR_HIP;
   }
+  return HPX_OK;
+}
+
+// Orders and cuts the tensors of `jobs` in one launch, where it can: those that are left to do go to the front of `jobs`.
+int order_in_windows(std::vector<CutJob>& jobs, volatile uint32_t* told, hipStream_t st) {
+  int windows = 0;
+  for (const CutJob& job : jobs) {
+    if (job.seg.n < kWindowSample || job.seg.n > kOrderMax) return HPX_OK;
+    windows += int(cdiv(job.seg.n, kWindow));
+  }
+  if (jobs.empty() || jobs.size() > size_t(kCapLarge) || size_t(windows) > hpx::kPinnedFlagOffset / sizeof(uint32_t)) return HPX_OK;
+  for (int w = 0; w < windows; w++) told[w] = 0;
+  __atomic_thread_fence(__ATOMIC_RELEASE);
+  const int count = int(jobs.size());
+  uint32_t* words = const_cast<uint32_t*>(told);
+  int rc = count <= kCapSmall ? launch_order<kCapSmall>(jobs.data(), count, words, st) : launch_order<kCapLarge>(jobs.data(), count, words, st);
+  if (rc != HPX_OK) return rc;
+  std::vector<CutJob> left;
+  int w = 0;
+  for (const CutJob& job : jobs) {
+    bool fails = false;
+    for (const int end = w + int(cdiv(job.seg.n, kWindow)); w < end; w++) {
+      volatile uint32_t* word = told + w;
+      rc = poll_memory([word]() { return *word == 0; }, "sparsifier encode", st);
+      if (rc != HPX_OK) return rc;
+      fails = fails || *word != kWindowFits;
+    }
+    if (fails) left.push_back(job);
+  }
+  jobs.swap(left);
   return HPX_OK;
 }
 
@@ -2918,6 +3156,8 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         HPX_HIP(hipGetLastError());
       }
     }
+    rc = order_in_windows(jobs, report, st);
+    if (rc != HPX_OK) return rc;
     for (size_t k = 0; k < jobs.size(); k += kCapLarge) {
       const int m = int(jobs.size() - k < size_t(kCapLarge) ? jobs.size() - k : size_t(kCapLarge));
       rc = m <= kCapSmall ? sort_and_cut<kCapSmall>(&jobs[k], m, st) : sort_and_cut<kCapLarge>(&jobs[k], m, st);
