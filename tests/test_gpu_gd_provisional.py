@@ -108,6 +108,17 @@ def test_values(gd, capi, kind, fallback):
         assert inverted == 1 and (fallback is None or fell_back == fallback)
 
 
+@pytest.mark.parametrize("step", [1e-4, 0.01, 0.04, 0.05, 0.06, 0.2, 1.0])   # equal hits from a few to hundreds: a bin that one wave ranks, or not
+def test_equal_hits(gd, capi, step):
+    n = FIRST
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    u = torch.empty(n, device="cuda").uniform_(-0.5, 0.5, generator=gen)
+    g = torch.round(-torch.log1p(-2 * u.abs().clamp(max=0.4999999)) * u.sign() / step) * step
+    for seed in (1, 9 << 24):
+        inverted, _ = _compare(gd, capi, [g], [torch.zeros(n, device="cuda")], [0.05], [0.999], [seed])
+        assert inverted == 1
+
+
 def _us(gd, capi, how, g, rate, drop):
     """Least time of a call, from its start until the GPU has finished."""
     r, out = torch.zeros_like(g), torch.empty(4 + 8 * int(np.ceil(g.numel() * (1 - drop))), dtype=torch.uint8, device="cuda")
