@@ -2221,8 +2221,8 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // quantile of them to the next, about kWindow pairs: the windows' bounds come from kWindowSample of the keys, one out of so
 // many, which every workgroup ranks for itself; then it reads all the keys, counts those above its window, which is the
 // place of its largest in the message, collects its own in LDS and places them as a workgroup does that has them all.  What
-// bounds it is instructions, of that walk over all keys by each and of the largest window (1024 pairs on average 27 us for 138
-// thousand, 2048 40, with 1024 keys to take the bounds from 33).  The digit sort's six launches took 44 and more: us per
+// bounds it is instructions, of that walk over all keys by each and of the largest window (138 thousand 26 us with windows of
+// 1024 pairs on average, 31 with 1536; 10 thousand 11.8).  The digit sort's six launches took 44 and more: us per
 // encode with a cut, sort -> windows, 10 thousand kept of 1 M 62.6 -> 44.5 and of 10 M 92 -> 74.5, 20 thousand 119.5 -> 102,
 // 60 thousand 201 -> 184, 120 thousand 104 -> 91 (12 M), 138 thousand 361 -> 345, 200 thousand 137.5 -> 127; 400 thousand
 // 205 -> 233, which is why kOrderMax lies between; bf16 values 62.6 -> 51 (1 M) and 366 -> 351 (138 M).
