@@ -1,7 +1,8 @@
 """GPU parity of the sparsifier's cut in one launch (gd_order_kernel), tensors that keep 8192 entries and more, at the sizes and
 kinds of values where it can go wrong: the fewest and the most candidates it takes and one more, few distinct values (bins that
-are crowded), one value that more share than a window holds (the digit sort behind it), all candidates side by side, and
-several tensors in a call.  Bit-exact against the oracle."""
+are crowded), one value that more share than a window holds, all candidates side by side, and
+several tensors in a call; values that the launch's own sample of the keys misses, and places that one wave reads.  Bit-exact
+against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -43,8 +44,63 @@ def test_cut_of_many(gd, oracle_cpu, found, keep, kind):
     rng = np.random.default_rng(found)
     r = _candidates(rng, n, found, kind)
     for seed in range(3):
-        _, _, info = _check_encode(gd, oracle_cpu, np.zeros(n, np.float32), r.copy(), 1 / n, 1 - (keep - 0.5) / n, seed << 24)
-        seen += info["candidates"] == found   # the one sample is a zero
+        gd.L.hpx_profile_reset(); gd.L.hpx_profile_enable(1)
+        try:
+            _, _, info = _check_encode(gd, oracle_cpu, np.zeros(n, np.float32), r.copy(), 1 / n, 1 - (keep - 0.5) / n, seed << 24)
+            order, sort = [gd.c.profile_query(k)[1] for k in ("gd_order_kernel", "gd_sort_pass_kernel")]
+        finally:
+            gd.L.hpx_profile_enable(0); gd.L.hpx_profile_reset()
+        if info["candidates"] == found:   # the one sample is a zero
+            seen += 1
+            assert order == (1 if found <= MOST else 0) and (sort > 0) == (found > MOST)
+    assert seen
+
+
+def _by_place(found, kind, rng):
+    """Candidates by their place among the candidates, with values that the windows' bounds say nothing of: the launch takes those
+    from one candidate of each stretch of found/512."""
+    x = rng.laplace(0, 1e-3, found)
+    x = np.where(np.abs(x) < 1e-6, 1e-6, x).astype(np.float32)
+    unseen = np.ones(found, bool)
+    at = np.arange(512, dtype=np.int64)
+    unseen[at * found // 512 + (((at * 0x9E3779B1 & 0xFFFFFFFF) >> 16) * (found // 512) >> 16)] = False
+    sign = rng.choice([-1, 1], found).astype(np.float32)
+    if kind == "equal":    # more of one value than a window holds, and of its neighbours
+        x[unseen] = (np.float32(1e-3) * sign)[unseen]
+        x[np.flatnonzero(unseen)[::5]] = np.nextafter(np.float32(1e-3), np.float32(1))
+    if kind == "near":     # as many that differ in the last bits
+        x[unseen] = (rng.permutation(found).astype(np.uint32) + np.float32(1e-3).view(np.uint32)).view(np.float32)[unseen] * sign[unseen]
+    if kind == "mixed":
+        some = np.flatnonzero(unseen)
+        x[some[: some.size // 3]] = 1e-3
+        x[some[some.size // 3: some.size // 2]] *= np.float32(1e-3)
+        x[some[-9000:]] = 0.25
+    if kind == "late":     # a third of them at the end, of one value
+        x[-(found // 3):] = -1e-3
+    if kind == "one_wave":  # the largest where one wave of a workgroup reads
+        one = np.arange(found) // 256 % 16 == 0
+        x[one] = (rng.uniform(0.5, 1, found).astype(np.float32) * sign)[one]
+    return x
+
+
+@pytest.mark.parametrize("kind", ["equal", "near", "mixed", "late", "one_wave"])
+@pytest.mark.parametrize("found,keep", [(20_001, 19_990), (60_002, 30_000), (60_002, 60_001), (MOST, 210_000)])
+def test_one_launch_settles_it(gd, oracle_cpu, found, keep, kind):
+    n = 3 * found
+    rng = np.random.default_rng(found + keep)
+    r = np.zeros(n, np.float32)
+    r[np.sort(rng.choice(n - 1, found, replace=False)) + 1] = _by_place(found, kind, rng)
+    seen = 0
+    for seed in range(4):
+        gd.L.hpx_profile_reset(); gd.L.hpx_profile_enable(1)
+        try:
+            _, _, info = _check_encode(gd, oracle_cpu, np.zeros(n, np.float32), r.copy(), 1 / n, 1 - (keep - 0.5) / n, seed << 24)
+            order, sort = [gd.c.profile_query(k)[1] for k in ("gd_order_kernel", "gd_sort_pass_kernel")]
+        finally:
+            gd.L.hpx_profile_enable(0); gd.L.hpx_profile_reset()
+        if info["candidates"] == found:   # the one sample is a zero
+            seen += 1
+            assert (order, sort) == (1, 0)
     assert seen
 
 

@@ -1596,7 +1596,6 @@ struct SortArgs {
   int32_t shift;
   int32_t parity;
   int32_t last;            // this pass writes the messages
-  uint32_t* told;          // pinned host memory: a word for each window of gd_order_kernel
   int32_t tile_start[CAP + 1];
   SortSeg seg[CAP];
 };
@@ -2012,10 +2011,8 @@ __device__ __forceinline__ uint32_t ranked_id(uint64_t p) { const uint32_t x = ~
 
 // n pairs, lane t with those at t, t + 1024 ... (in ascending index order; the sign in the index's top bit).  False: some
 // bin is crowded, nothing has been written, and the pairs are in LDS, [kCutLds] keys and then [kCutLds] indices.
-// `placed` is called by every lane once it is known that no bin is.
-struct Nothing { __device__ __forceinline__ void operator()() const {} };
-template <int PER, typename Placed = Nothing>
-__device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER], Placed placed = {}) {
+template <int PER>
+__device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&key)[PER], const uint32_t (&id)[PER]) {
   const uint32_t t = threadIdx.x, n = f.n;
   uint64_t* s_pair = reinterpret_cast<uint64_t*>(f.stage);
   uint32_t bin[PER], slot[PER];
@@ -2030,7 +2027,6 @@ __device__ __forceinline__ bool cut_by_bins(const CutArgs& f, const uint32_t (&k
     stage_pairs<PER>(f, key, id);
     return false;
   }
-  placed();
   uint64_t own[PER];
   uint32_t lo[PER], len[PER], place[PER], longest = 0;
 #pragma unroll
@@ -2219,24 +2215,28 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 
 // The cut of a tensor that keeps kCutKeep entries and more, in one launch.  A workgroup takes a window of the keys, from one
 // quantile of them to the next, about kWindow pairs: the windows' bounds come from kWindowSample of the keys, one out of so
-// many, which every workgroup ranks for itself; then it reads all the keys, counts those above its window, which is the
+// many, which a wave for each bound ranks; then it reads all the keys, counts those above its window, which is the
 // place of its largest in the message, collects its own in LDS and places them as a workgroup does that has them all.  What
 // bounds it is instructions, of that walk over all keys by each and of the largest window (138 thousand 26 us with windows of
 // 1024 pairs on average, 31 with 1536; 10 thousand 11.8).  The digit sort's six launches took 44 and more: us per
 // encode with a cut, sort -> windows, 10 thousand kept of 1 M 62.6 -> 44.5 and of 10 M 92 -> 74.5, 20 thousand 119.5 -> 102,
 // 60 thousand 201 -> 184, 120 thousand 104 -> 91 (12 M), 138 thousand 361 -> 345, 200 thousand 137.5 -> 127; 400 thousand
 // 205 -> 233, which is why kOrderMax lies between; bf16 values 62.6 -> 51 (1 M) and 366 -> 351 (138 M).
-// Where a window would have more pairs than fit (a value that thousands share) it says so, and the host, which waits for a word of
-// every window, queues the digit sort behind it, which writes the message anew: that detour takes 14 us (20 M elements, 30 thousand of one
-// size 109 -> 122).
+// A value that thousands share is several quantiles, and the windows between two of these share its candidates by their places
+// (order_ties).  What does not fit all the same - the sample is one of many, and one wave may read most of a window - goes part
+// by part (next_part).  So all of it is settled here, and the host, which queues the launch, does not wait for it.  us per encode of
+// tensors with zeros around their candidates, sort -> windows: 100 thousand candidates 107 -> 77, with a tenth of them equal 112 -> 77,
+// all of them 99 -> 72; 16 thousand with six in ten equal 103 -> 73; 220 thousand with the last three in ten equal 209 -> 183; the
+// largest of 220 thousand where one wave reads 115 -> 117.  (Windows that left such tensors to a sort queued behind them, the host waiting
+// for their word: 127, 118, 119, 248 and 153; and 60 instead of 20 until the call returned.)  Part by part is no more than a way out:
+// 100 thousand candidates laid around the sample, on purpose, so that one window has nearly all: 1.4 ms.
 constexpr uint32_t kWindow = 1024, kWindowSample = 512;
 constexpr uint32_t kOrderMax = 224 * 1024;   // candidates
-constexpr uint32_t kWindowFits = 1u, kWindowFails = 2u;
 // False: a bin is crowded (many equal keys), nothing has been written, and the pairs are in LDS as cut_crowded takes them, in the
 // order of the candidates.  That order comes from bins of the places among those, so wide that no more than kWideBin can share one.
-template <int PER, typename Placed>
+template <int PER>
 __device__ __forceinline__ bool window_by_bins(const CutArgs& f, uint32_t below, const uint32_t* s_found,
-                                               const uint32_t* __restrict__ keys, const int32_t* __restrict__ ids, Placed placed) {
+                                               const uint32_t* __restrict__ keys, const int32_t* __restrict__ ids) {
   constexpr uint32_t kWideBin = (kOrderMax + kCutBins - 1) / kCutBins;
   static_assert(kWideBin <= kCutCrowd, "no bin of places is crowded");
   const uint32_t t = threadIdx.x;
@@ -2248,7 +2248,7 @@ __device__ __forceinline__ bool window_by_bins(const CutArgs& f, uint32_t below,
     key[j] = keys[at[j]] - below;
     id[j] = uint32_t(ids[at[j]]);
   }
-  if (cut_by_bins<PER>(f, key, id, placed)) return true;
+  if (cut_by_bins<PER>(f, key, id)) return true;
   reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(0, 0, 0, 0);
   __syncthreads();
   uint32_t slot[PER];
@@ -2274,12 +2274,128 @@ __device__ __forceinline__ bool window_by_bins(const CutArgs& f, uint32_t below,
   __syncthreads();
   return false;
 }
+// The candidates whose key is `v`, of the part-th of `parts` stretches of the keys, in their order to their places in the message.
+// (`f`: with all of the message's entries.)  Gives how many candidates come before the stretch's first and how many there are.
+__device__ __forceinline__ void order_ties(const CutArgs& f, const uint32_t* __restrict__ keys, const int32_t* __restrict__ ids, uint32_t v,
+                                           uint32_t part, uint32_t parts, uint32_t& before, uint32_t& found) {
+  const uint32_t t = threadIdx.x, quads = (f.n + 3) / 4;
+  const uint32_t from = quads * part / parts, to = quads * (part + 1) / parts;
+  const uint4* __restrict__ quad = reinterpret_cast<const uint4*>(keys);
+  auto take = [&](uint32_t q, uint32_t (&k)[4]) {   // zeros behind the last one: no key is
+    const uint4 x = quad[q];
+    k[0] = x.x; k[1] = x.y; k[2] = x.z; k[3] = x.w;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) k[i] = 4 * q + i < f.n ? k[i] : 0u;
+  };
+  uint32_t mine = 0;
+#pragma unroll 4
+  for (uint32_t q = t; q < quads; q += kSortThreads) {
+    uint32_t k[4];
+    take(q, k);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) mine += k[i] > v || (q < from && k[i] == v) ? 1u : 0u;
+  }
+  found = 0;
+  block_prefix(mine, f.wave, before);
+  for (uint32_t q0 = from; q0 < to && before + found < f.keep; q0 += kSortThreads) {
+    uint32_t k[4] = {0, 0, 0, 0};
+    if (q0 + t < to) take(q0 + t, k);
+    mine = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) mine += k[i] == v ? 1u : 0u;
+    uint32_t all;
+    uint32_t place = before + found + block_prefix(mine, f.wave, all);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++)
+      if (k[i] == v) f.put(place++, v, uint32_t(ids[4 * (q0 + t) + i]));
+    found += all;
+  }
+}
+// Of the `left` keys in [lo, top), the largest, kPart of them at most: where they lie to s_found, how many of them there are as the
+// result (0: none are left), the least key that is theirs to `bottom`.  Where not all of them fit: bins of 1 << shift keys each,
+// larger ones first, as many from the front as hold no more than fit; if the first one does not, its keys in finer ones, down to
+// one value, whose candidates go to the message at once.
+constexpr uint32_t kPart = 4096;
+__device__ __forceinline__ uint32_t next_part(const CutArgs& f, const uint32_t* __restrict__ keys, const int32_t* __restrict__ ids, uint32_t lo,
+                                              uint32_t& top, uint32_t& bottom, uint32_t& first, uint32_t& left, uint32_t* s_found,
+                                              uint32_t* s_cut) {
+  const uint32_t t = threadIdx.x;
+  auto walk = [&](auto key_at) {   // (a place behind the last key: zero, below all that is asked for)
+    const uint4* __restrict__ quad = reinterpret_cast<const uint4*>(keys);
+    const uint32_t quads = (f.n + 3) / 4;
+#pragma unroll 4
+    for (uint32_t q = t; q < quads; q += kSortThreads) {
+      const uint4 x = quad[q];
+      const uint32_t k[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) key_at(4 * q + i < f.n ? k[i] : 0u, 4 * q + i);
+    }
+  };
+  bottom = lo;
+#pragma unroll 1
+  while (left > 0 && first < f.keep) {
+    uint32_t count = left;
+    if (t == 0) s_cut[2] = 0;
+    if (left > kPart) {
+      const uint32_t span = top - bottom, wide = 32 - uint32_t(__builtin_clz(span)), shift = wide > 12 ? wide - 12 : 0u;
+      static_assert(kBinWords == 1u << 12 && kBinWords == 4 * kSortThreads, "four bins to a lane");
+      reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(0, 0, 0, 0);
+      __syncthreads();
+      walk([&](uint32_t k, uint32_t) {
+        const uint32_t d = top - 1 - k;
+        if (d < span) atomicAdd(&f.bins[d >> shift], 1u);
+      });
+      __syncthreads();
+      const uint4 c = reinterpret_cast<const uint4*>(f.bins)[t];
+      const uint32_t bin[4] = {c.x, c.y, c.z, c.w};
+      uint32_t total;
+      uint32_t at = block_prefix(c.x + c.y + c.z + c.w, f.wave, total);
+      if (t == 0) { s_cut[0] = kBinWords; s_cut[1] = total; }
+      __syncthreads();
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) {   // the bin that no longer fits, if there is one, and how many keys lie before it
+        if (at <= kPart && at + bin[i] > kPart) { s_cut[0] = 4 * t + i; s_cut[1] = at; }
+        at += bin[i];
+      }
+      __syncthreads();
+      const uint32_t bins = s_cut[0];
+      count = s_cut[1];
+      if (bins == 0 && shift > 0) {
+        bottom = top - (1u << shift);   // there are more bins than that one
+        continue;
+      }
+      if (bins == 0) {
+        uint32_t before, found;
+        order_ties(f, keys, ids, top - 1, 0, 1, before, found);
+        first += found;   // (not all of them where the message ends there)
+        left -= found;
+        top -= 1;
+        bottom = lo;
+        continue;
+      }
+      if (bins < kBinWords) bottom = top - (bins << shift);
+      if (count == 0) {
+        top = bottom;
+        bottom = lo;
+        continue;
+      }
+    }
+    reinterpret_cast<uint4*>(f.bins)[t] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    walk([&](uint32_t k, uint32_t x) {
+      if (k >= bottom && k < top) s_found[atomicAdd(&s_cut[2], 1u)] = x;
+    });
+    __syncthreads();
+    return count;
+  }
+  return 0;
+}
 template <int CAP>
 __global__ __launch_bounds__(kSortThreads) void gd_order_kernel(const SortArgs<CAP> a) {
   // (Aligned by name: behind an odd number of words the pairs' 64-bit accesses took this launch from 27 to 42 us.)
   extern __shared__ __align__(16) uint32_t s_stage[];   // 2 * kCutLds words: where the window's keys lie, a list per wave and then all of them; the pairs
   __shared__ __align__(16) uint32_t s_bins[kBinWords + 4];
-  __shared__ uint32_t s_wave[kSortWaves], s_cut_wave[kSortWaves], s_bound[2], s_heavy;
+  __shared__ uint32_t s_wave[kSortWaves], s_cut_wave[kSortWaves], s_bound[3], s_cut[3];
   const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int s = find_segment<CAP>(a.tile_start, a.nseg, blockIdx.x);
   const SortSeg& sg = a.seg[s];
@@ -2287,46 +2403,50 @@ __global__ __launch_bounds__(kSortThreads) void gd_order_kernel(const SortArgs<C
   const CutLayout cl = cut_layout(sg.cap);
   const uint32_t* __restrict__ keys = sort_keys(sg, cl, 0);
   const uint32_t n = sg.n, keep = sg.keep;
-  auto tell = [&](uint32_t what) {
-    if (t == 0) __hip_atomic_store(a.told + blockIdx.x, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  const int32_t* __restrict__ ids = sort_ids(sg, cl, 0);
+  constexpr uint32_t kOwn = kWindowSample / kWave;
+  auto sample = [&](uint32_t (&key)[kOwn]) {   // one of each stretch, anywhere in it: no regular order of the values passes between them
+#pragma unroll
+    for (uint32_t j = 0; j < kOwn; j++) {
+      const uint32_t x = j * kWave + lane;
+      key[j] = keys[uint32_t(uint64_t(x) * n / kWindowSample) + (((x * 0x9E3779B1u) >> 16) * (n / kWindowSample) >> 16)];
+    }
   };
   reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
-  if (wave < 3) {   // (the others too: 4 us more, a request for each of their keys)
-    constexpr uint32_t kOwn = kWindowSample / kWave;
+  if (wave < 3) {   // one for each bound, and for the lower one of the window below (the other waves too: 4 us more, a request for each of their keys)
     uint32_t key[kOwn];
-#pragma unroll
-    for (uint32_t j = 0; j < kOwn; j++) key[j] = keys[uint32_t(uint64_t(j * kWave + lane) * n / kWindowSample)];
-    if (wave < 2) {   // one wave for each bound
-      const uint32_t w = window + wave;
-      uint32_t bound = w == 0 ? 0xFFFFFFFFu : 1u;   // keys are at least 1
-      if (w > 0 && w < windows) {
-        bound = wave_rank<int(kOwn), 0>(key, uint32_t(uint64_t(w) * kWindowSample / windows), 0u);
-        bound = bound > 1u ? bound : 1u;
-      }
-      if (lane == 0) s_bound[wave] = bound;
-    } else {          // ... and one looks how often some of the sample come up in it
-      uint32_t most = 0;
-#pragma unroll 1
-      for (int p = 0; p < kWave; p += 4) {
-        const uint32_t probe = uint32_t(__builtin_amdgcn_readlane(int(key[0]), p));
-        uint32_t equal = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < kOwn; j++) equal += uint32_t(__popcll(__ballot(key[j] == probe)));
-        most = equal > most ? equal : most;
-      }
-      if (lane == 0) s_heavy = uint64_t(most) * n > uint64_t(kCutKeep) * kWindowSample ? 1u : 0u;
+    sample(key);
+    const uint32_t w = window + wave;
+    uint32_t bound = w == 0 ? 0xFFFFFFFFu : w == windows ? 1u : 0u;   // keys are at least 1
+    if (w > 0 && w < windows) {
+      bound = wave_rank<int(kOwn), 0>(key, uint32_t(uint64_t(w) * kWindowSample / windows), 0u);
+      bound = bound > 1u ? bound : 1u;
     }
+    if (lane == 0) s_bound[wave] = bound;
   }
   __syncthreads();
-  if (s_heavy != 0) {   // some window would not hold it
-    tell(kWindowFails);
+  const uint32_t hi = s_bound[0];
+  uint32_t lo = s_bound[1];
+  if (window == 0 && t == 0) *reinterpret_cast<int32_t*>(sg.msg) = int32_t(4 + keep * 8);
+  const CutArgs whole{s_stage, s_bins, s_wave, sg.r, sg.msg, n, keep, sg.thr_bits, false, 0, keep};
+  if (hi == lo) {   // its quantiles are one value, so are those of the windows from `from` to `to`
+    uint32_t key[kOwn], above = 0, reach = 0;
+    sample(key);
+#pragma unroll
+    for (uint32_t j = 0; j < kOwn; j++) {
+      above += uint32_t(__popcll(__ballot(key[j] > lo)));
+      reach += uint32_t(__popcll(__ballot(key[j] >= lo)));
+    }
+    uint32_t from = cdiv(above * windows, kWindowSample), to = cdiv(reach * windows, kWindowSample) - 1;
+    from = from > 1u ? from : 1u;
+    to = lo == 1u ? windows : to < windows - 1 ? to : windows - 1;
+    uint32_t before, found;
+    order_ties(whole, keys, ids, lo, window - from, to - from, before, found);
     return;
   }
-  const uint32_t hi = s_bound[0], lo = s_bound[1], below = lo - 1;
-  if (window == 0 && t == 0) *reinterpret_cast<int32_t*>(sg.msg) = int32_t(4 + keep * 8);
-  if (hi == lo) {   // its quantiles are one value, the lower bound of the window before it
-    tell(kWindowFits);
-    return;
+  if (lo == s_bound[2]) {   // the windows below see to that value
+    lo++;
+    if (hi == lo) return;
   }
   // A lane marks those of its sixteen keys that are in the window, and the wave then lists the marked ones, one of each lane at
   // a time: no branch on the way (with one at every key the walk over 138 thousand took 20 us).
@@ -2374,29 +2494,37 @@ __global__ __launch_bounds__(kSortThreads) void gd_order_kernel(const SortArgs<C
   uint32_t first, found;
   before_wave(s_wave[lane & 15], first);
   const uint32_t in_wave = s_cut_wave[lane & 15], start = before_wave(in_wave, found);
-  const bool long_list = __ballot(in_wave > kListOf) != 0;
-  if (found == 0 || first >= keep) {   // nothing of it is sent
-    tell(kWindowFits);
-    return;
-  }
-  if (long_list || found > kCutKeep) {
-    tell(kWindowFails);
-    return;
-  }
+  const bool fits = __ballot(in_wave > kListOf) == 0 && found <= kCutKeep;
+  if (found == 0 || first >= keep) return;   // nothing of it is sent
   uint32_t* s_found = s_stage + kCutLds;
-  for (uint32_t i = lane; i < mine; i += kWave) s_found[start + i] = s_list[i];
-  __syncthreads();
-  const uint32_t kept = keep - first < found ? keep - first : found;
-  const CutArgs f{s_stage, s_bins, s_cut_wave, sg.r, sg.msg, found, kept, sg.thr_bits + below, false, first, keep};
-  const int32_t* __restrict__ ids = sort_ids(sg, cl, 0);
-  auto placed = [&]() { tell(kWindowFits); };
-  const bool done = found <= 2 * kSortThreads   ? window_by_bins<2>(f, below, s_found, keys, ids, placed)
-                    : found <= 3 * kSortThreads ? window_by_bins<3>(f, below, s_found, keys, ids, placed)
-                    : found <= 4 * kSortThreads ? window_by_bins<4>(f, below, s_found, keys, ids, placed)
-                                                : window_by_bins<8>(f, below, s_found, keys, ids, placed);
-  if (done) return;
-  tell(kWindowFits);
-  cut_crowded(f);
+  auto pairs = [&](uint32_t below, uint32_t count) {
+    const uint32_t kept = keep - first < count ? keep - first : count;
+    return CutArgs{s_stage, s_bins, s_cut_wave, sg.r, sg.msg, count, kept, sg.thr_bits + below, false, first, keep};
+  };
+  if (fits) {
+    for (uint32_t i = lane; i < mine; i += kWave) s_found[start + i] = s_list[i];
+    __syncthreads();
+    const uint32_t below = lo - 1;
+    const CutArgs f = pairs(below, found);
+    const bool done = found <= 2 * kSortThreads   ? window_by_bins<2>(f, below, s_found, keys, ids)
+                      : found <= 3 * kSortThreads ? window_by_bins<3>(f, below, s_found, keys, ids)
+                      : found <= 4 * kSortThreads ? window_by_bins<4>(f, below, s_found, keys, ids)
+                                                  : window_by_bins<8>(f, below, s_found, keys, ids);
+    if (!done) cut_crowded(f);
+    return;
+  }
+  uint32_t top = hi, bottom;
+#pragma unroll 1
+  for (;;) {
+    __syncthreads();
+    const uint32_t count = next_part(whole, keys, ids, lo, top, bottom, first, found, s_found, s_cut);
+    if (count == 0) return;
+    const CutArgs f = pairs(bottom - 1, count);
+    if (!window_by_bins<int(kPart) / kSortThreads>(f, bottom - 1, s_found, keys, ids)) cut_crowded(f);
+    first += count;
+    found -= count;
+    top = bottom;
+  }
 }
 
 // What is left to do for a tensor that keeps at most kFinishKeep entries once the pass has marked its candidates,
@@ -2778,7 +2906,6 @@ int sort_passes(SortArgs<CAP>& a, int passes, hipStream_t st) {
 template <int CAP>
 int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
   SortArgs<CAP> a;
-  a.told = nullptr;
   a.nseg = count;
   int bits = 1;
   a.tile_start[0] = 0;
@@ -2793,13 +2920,12 @@ int sort_and_cut(const CutJob* jobs, int count, hipStream_t st) {
   return HPX_OK;
 }
 
-// The cut path in one launch, a word of `told` for each of the windows (cleared by the caller).
+// The cut path in one launch.
 template <int CAP>
-int launch_order(const CutJob* jobs, int count, uint32_t* told, hipStream_t st) {
+int launch_order(const CutJob* jobs, int count, hipStream_t st) {
   SortArgs<CAP> a;
   a.nseg = count;
   a.shift = a.parity = a.last = 0;
-  a.told = told;
   a.tile_start[0] = 0;
   for (int i = 0; i < count; i++) {
     a.seg[i] = jobs[i].seg;
@@ -2990,34 +3116,11 @@ int wait_word(volatile unsigned long long* word, hipStream_t st) {
   return HPX_OK;
 }
 
-// Orders and cuts the tensors of `jobs` in one launch, where it can: those that are left to do go to the front of `jobs`.
-int order_in_windows(std::vector<CutJob>& jobs, volatile uint32_t* told, hipStream_t st) {
-  int windows = 0;
-  for (const CutJob& job : jobs) {
-    if (job.seg.n < kWindowSample || job.seg.n > kOrderMax) return HPX_OK;
-    windows += int(cdiv(job.seg.n, kWindow));
-  }
-  if (jobs.empty() || jobs.size() > size_t(kCapLarge) || size_t(windows) > hpx::kPinnedFlagOffset / sizeof(uint32_t)) return HPX_OK;
-  for (int w = 0; w < windows; w++) told[w] = 0;
-  __atomic_thread_fence(__ATOMIC_RELEASE);
-  const int count = int(jobs.size());
-  uint32_t* words = const_cast<uint32_t*>(told);
-  int rc = count <= kCapSmall ? launch_order<kCapSmall>(jobs.data(), count, words, st) : launch_order<kCapLarge>(jobs.data(), count, words, st);
-  if (rc != HPX_OK) return rc;
-  std::vector<CutJob> left;
-  int w = 0;
-  for (const CutJob& job : jobs) {
-    bool fails = false;
-    for (const int end = w + int(cdiv(job.seg.n, kWindow)); w < end; w++) {
-      volatile uint32_t* word = told + w;
-      rc = poll_memory([word]() { return *word == 0; }, "sparsifier encode", st);
-      if (rc != HPX_OK) return rc;
-      fails = fails || *word != kWindowFits;
-    }
-    if (fails) left.push_back(job);
-  }
-  jobs.swap(left);
-  return HPX_OK;
+// Whether the windows are quicker than the digit sort for what a call has to cut.
+bool windows_pay(const std::vector<CutJob>& jobs) {
+  for (const CutJob& job : jobs)
+    if (job.seg.n < kWindowSample || job.seg.n > kOrderMax) return false;
+  return true;
 }
 
 constexpr int kMaxPerWait = int((hpx::kPinnedFlagOffset) / (kReportWords * sizeof(uint32_t)));  // tensors whose reports fit the pinned block
@@ -3196,11 +3299,11 @@ int gd_encode_batch(int count, float* const* grads, const int32_t* Ns, float* co
         HPX_HIP(hipGetLastError());
       }
     }
-    rc = order_in_windows(jobs, report, st);
-    if (rc != HPX_OK) return rc;
+    const bool windows = windows_pay(jobs);
     for (size_t k = 0; k < jobs.size(); k += kCapLarge) {
       const int m = int(jobs.size() - k < size_t(kCapLarge) ? jobs.size() - k : size_t(kCapLarge));
-      rc = m <= kCapSmall ? sort_and_cut<kCapSmall>(&jobs[k], m, st) : sort_and_cut<kCapLarge>(&jobs[k], m, st);
+      if (windows) rc = m <= kCapSmall ? launch_order<kCapSmall>(&jobs[k], m, st) : launch_order<kCapLarge>(&jobs[k], m, st);
+      else rc = m <= kCapSmall ? sort_and_cut<kCapSmall>(&jobs[k], m, st) : sort_and_cut<kCapLarge>(&jobs[k], m, st);
       if (rc != HPX_OK) return rc;
     }
   }
