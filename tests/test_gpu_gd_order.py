@@ -119,3 +119,47 @@ def test_several_tensors(gd, oracle_cpu):
             msg = oracle_cpu.gd_encode(np.zeros(r.size, np.float32), want_r, rate, d, seed)[0]
             assert_bits_equal(host(out)[:msg.size], msg, "message")
             assert_bits_equal(host(got_r), want_r, "residual")
+
+
+def _encode_call(gd, oracle_cpu, rs, keep, seed):
+    """One call, checked; how many of its tensors were cut, and the launches of (windows, sort)."""
+    gs, d_r = [torch.zeros(r.size, device="cuda") for r in rs], [dev(r) for r in rs]
+    outs = [torch.zeros(4 + 8 * k, dtype=torch.uint8, device="cuda") for k in keep]
+    drops, rates = [1 - (k - 0.5) / r.size for k, r in zip(keep, rs)], [1 / r.size for r in rs]
+    gd.L.hpx_profile_reset(); gd.L.hpx_profile_enable(1)
+    try:
+        gd.encode(gs, d_r, outs, rates, drops, [seed] * len(rs))
+        torch.cuda.synchronize()
+        launches = tuple(int(gd.c.profile_query(k)[1]) for k in ("gd_order_kernel", "gd_sort_pass_kernel"))
+    finally:
+        gd.L.hpx_profile_enable(0); gd.L.hpx_profile_reset()
+    cut = []
+    for r, rate, d, got_r, out in zip(rs, rates, drops, d_r, outs):
+        want_r = r.copy()
+        msg, info = oracle_cpu.gd_encode(np.zeros(r.size, np.float32), want_r, rate, d, seed)
+        assert_bits_equal(host(out)[:msg.size], msg, "message")
+        assert_bits_equal(host(got_r), want_r, "residual")
+        if info["candidates"] > info["kept"]:
+            cut.append(info["candidates"])
+    return cut, launches
+
+
+# tensors of a call on either side of where the sort is the quicker one for all of them: by the keys that the windows read in
+# all, by their number, by one tensor; more tensors than a small launch table holds, more windows than CUs
+@pytest.mark.parametrize("found", [(60_000,) * 6, (9500,) * 40, (MOST, MOST), (150_000,) * 5, (9300,) * 190, (MOST + 1, 20_000, 9000),
+                                   (100_000, 20_000, 8193, 8200, 30_000)])
+def test_one_way_for_a_call(gd, oracle_cpu, found):
+    rng = np.random.default_rng(len(found))
+    kinds = ["spread", "bf16", "shared"]
+    rs = [_candidates(rng, 4 * f, f, kinds[i % 3]) for i, f in enumerate(found)]
+    keep = [max(8192, f - 500 - i) for i, f in enumerate(found)]
+    ways = set()
+    for seed in (3, 9 << 24):
+        cut, (order, sort) = _encode_call(gd, oracle_cpu, rs, keep, seed)
+        windows = [-(-c // 1024) for c in cut]
+        if not cut:
+            continue
+        pays = max(cut) <= MOST and sum(windows) <= 7 * 256 and sum(w * c for w, c in zip(windows, cut)) <= 90 << 20
+        assert (order, sort > 0) == ((1, False) if pays else (0, True))
+        ways.add(pays)
+    assert ways

@@ -2231,7 +2231,7 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // for their word: 127, 118, 119, 248 and 153; and 60 instead of 20 until the call returned.)  Part by part is no more than a way out:
 // 100 thousand candidates laid around the sample, on purpose, so that one window has nearly all: 1.4 ms.
 constexpr uint32_t kWindow = 1024, kWindowSample = 512;
-constexpr uint32_t kOrderMax = 224 * 1024;   // candidates
+constexpr uint32_t kOrderMax = 224 * 1024;   // candidates of one tensor; for all of a call: windows_pay
 // False: a bin is crowded (many equal keys), nothing has been written, and the pairs are in LDS as cut_crowded takes them, in the
 // order of the candidates.  That order comes from bins of the places among those, so wide that no more than kWideBin can share one.
 template <int PER>
@@ -3116,11 +3116,27 @@ int wait_word(volatile unsigned long long* word, hipStream_t st) {
   return HPX_OK;
 }
 
-// Whether the windows are quicker than the digit sort for what a call has to cut.
+// Whether the windows are quicker than the digit sort for what a call has to cut, all of it one way or the other.  The sort shares
+// its launches among the tensors; the windows queue up, one for each CU at a time, and each reads all the keys of its tensor.  us per
+// encode of tensors with zeros around their candidates, sort / windows (keys read in all by the windows; their number):
+//   4 tensors of 130 thousand candidates 117 / 105 (66 M; 508), 5 of 120 thousand 124 / 122 (71 M; 590), 12 of 90 thousand 173 / 173 (95 M; 1056),
+//   2 of 220 thousand 118 / 119 (95 M; 430), 4 of 160 thousand 123 / 130 (101 M), 5 of 150 thousand 133 / 144 (110 M),
+//   10 of 220 thousand 221 / 312;
+//   100 of 9 thousand 168 / 147 (900), 50 of 30 thousand 204 / 190 (1500), 200 of 9 thousand 245 / 240 (1800), 100 of 20 thousand 243 / 256 (2000),
+//   200 of 12 thousand 299 / 311 (2400).
+// Where one tensor has to be sorted, or has hardly any candidates, the others go with it: one of 240 thousand and five of 50 thousand 124, with these
+// in windows 138; one of 300 thousand and five of 10 thousand 124 and 147.
+constexpr uint64_t kOrderKeys = 90u << 20;        // read by the windows of a call ...
+constexpr uint32_t kOrderWindows = 7 * 256;       // ... and how many of them
 bool windows_pay(const std::vector<CutJob>& jobs) {
-  for (const CutJob& job : jobs)
+  uint64_t keys = 0, windows = 0;
+  for (const CutJob& job : jobs) {
     if (job.seg.n < kWindowSample || job.seg.n > kOrderMax) return false;
-  return true;
+    const uint64_t w = cdiv(job.seg.n, kWindow);
+    windows += w;
+    keys += w * job.seg.n;
+  }
+  return keys <= kOrderKeys && windows <= kOrderWindows;
 }
 
 constexpr int kMaxPerWait = int((hpx::kPinnedFlagOffset) / (kReportWords * sizeof(uint32_t)));  // tensors whose reports fit the pinned block
