@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from gpu_util import assert_bits_equal, dev, host
-from test_gpu_gd import Gd, _check_encode
+from test_gpu_gd import Gd, _check_encode, _dgc_encode
 
 pytestmark = pytest.mark.gpu
 
@@ -35,6 +35,31 @@ def test_crowded_lists(gd, oracle_cpu, n, rate, crowd):
     r = rng.normal(0, 1e-4, n).astype(np.float32)
     for seed in (1, 7 << 24):
         _check_encode(gd, oracle_cpu, g, r.copy(), rate, 0.999, seed)
+
+
+# several lists of one wave's lanes too short at once, more than it takes at a time, by one and by many; in the last list too, which
+# ends inside a mask word; sent as they are and cut; more candidates than one workgroup sorts; with a residual and without
+@pytest.mark.parametrize("n,kept,crowd,groups", [(200_003, 2000, 41, 5), (200_003, 2000, 47, 5), (200_003, 2000, 45, 1), (200_003, 1000, 1024, 60),
+                                                 (1_000_001, 2300, 25, 12), (1_000_001, 2300, 200, 90), (5_000_001, 1400, 17, 61),
+                                                 (9_000_001, 2500, 17, 40), (200_003, 2500, 60, 1)])
+def test_several_lists_too_short(gd, oracle_cpu, n, kept, crowd, groups):
+    rng = np.random.default_rng(n + crowd)
+    g = np.zeros(n, np.float32)
+    last = (n - 1) // 1024 * 1024
+    for start in list(range(0, last, 1024 * groups)) + [last]:
+        at = start + rng.choice(min(1024, n - start), min(crowd, n - start), replace=False)
+        g[at] = rng.choice([-1, 1], at.size) * rng.integers(1, 1000, at.size).astype(np.float32)
+    rate, drop = 1 / n, 1 - (kept - 0.5) / n
+    found, seen = np.count_nonzero(g), 0
+    for seed in range(3):
+        _, _, info = _check_encode(gd, oracle_cpu, g, np.zeros(n, np.float32), rate, drop, seed << 24)
+        seen += info["candidates"] == found   # the one sample is a zero
+        dg, out, want = dev(g), torch.zeros(4 + 8 * kept, dtype=torch.uint8, device="cuda"), g.copy()
+        _dgc_encode(gd, dg, out, rate, (kept - 0.5) / n, seed << 24)
+        msg, _ = oracle_cpu.dgc_encode(want, rate, (kept - 0.5) / n, seed << 24)
+        assert_bits_equal(host(out)[:msg.size], msg, "message without a residual")
+        assert_bits_equal(host(dg), want, "gradient")
+    assert seen
 
 
 # all large values in one list of a tensor that is otherwise flat

@@ -117,8 +117,7 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
 }
 // Behind that block: the candidates themselves, (index, value) in ascending order, a list per wave of the pass with room
 // for this many (0: no lists, the candidates are looked up through the masks).  Twice the expected number and fourteen: a wave's
-// 1024 elements exceed that next to never unless the large ones crowd together, and then the masks serve (of one million, half of the
-// large ones within one element in 1500: 49.3 us, 50.9 since there are lists to look at first).  The pass pays
+// 1024 elements exceed that next to never unless the large ones crowd together, and then the masks name the others.  The pass pays
 // for them (138 M elements 229 -> 232 us, ResNet-50's 161 tensors 46.7 -> 48.4, one of a million 4.3 -> 5.1); behind it the
 // expand launch takes 9.0 us instead of 14.4 (138 M), and the finish took 8.8 instead of 11.7 for the million, 16.2 instead of 24.8 for
 // ResNet-50's 161 (6.1 and 10.3 since).  Up to 12 in 1024: denser, the lists would be a tenth of the tensor.
@@ -142,10 +141,11 @@ __host__ __device__ inline uint32_t list_room(uint32_t n, uint32_t limit) {
 // Whether the pass leaves zeros in the residual where it lists a candidate's value.  Of a tensor that one workgroup settles nearly all
 // candidates are kept, and that workgroup wrote to as many lines of r, at about 700 a microsecond for one CU (ResNet-50's 161
 // tensors 16.2 us for that launch, 14.5 with this and the message written in order, the pass as long as before); it puts back
-// the few that a cut drops, and all of them where the lists turn out too short (gd_finish_kernel).
+// the few that a cut drops, and all of them where it cannot take them from the lists (gd_finish_kernel).
 __host__ __device__ inline bool clears_listed(uint32_t n, uint32_t limit) { return one_workgroup(n, limit) && list_room(n, limit) != 0; }
 __host__ __device__ inline size_t list_bytes(uint32_t n, uint32_t limit) {
-  return align256(sizeof(uint64_t) * size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit));
+  const size_t lists = size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit);
+  return align256(sizeof(uint64_t) * (lists + (clears_listed(n, limit) ? kCutKeep : 0u)));   // behind them what has no room in its list
 }
 // The launches behind the pass read them four lanes to a list, so that a wave has the lists of four tiles; the first entries,
 // whether there are as many or not, and the lengths are requested together.
@@ -2604,8 +2604,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
   // lists, times three, which one CU takes 3 us over for 2304 of them.)
   const uint32_t room = list_room(sg.n, keep);
   const bool cleared = a.residual != 0 && clears_listed(sg.n, keep);
-  const uint2* __restrict__ list = seg_list(sg, l);
-  bool lists = false;
+  uint2* list = seg_list(sg, l);
   uint32_t n = 0, pos = 0;
   reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
   if (room != 0) {
@@ -2625,13 +2624,51 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
     }
     bool some_over;
     pos = block_prefix_once(mine, over, s_wave, n, some_over);
-    lists = !some_over && n <= kCutKeep;
-    if (lists) {
+    if (n <= kCutKeep) {
+      uint32_t start = pos;
       for (uint32_t q0 = 0; q0 < per; q0 += kAtOnce) {
         if (per > kAtOnce) take(q0);
 #pragma unroll
-        for (uint32_t q = 0; q < kAtOnce; q++)
-          for (uint32_t j = 0; j < c[q]; j++) s_id[pos++] = (first + q0 + q) * room + j;
+        for (uint32_t q = 0; q < kAtOnce; q++) {
+          for (uint32_t j = 0; j < (c[q] < room ? c[q] : room); j++) s_id[pos + j] = (first + q0 + q) * room + j;
+          pos += c[q];
+        }
+      }
+      // What has no room in its list the masks name; its values get places behind all lists.  (All candidates through the masks as soon as
+      // one list is too short: one million, half of its large values within 1 in 1500, 60 us per encode, now 34; 2.4 M with 37
+      // lists of 2400 too short by four 59, and 65 with what the pass had cleared put back first, now 55; with 146 such lists 53, now 49.)
+      if (some_over) {
+        // by their element and a mark; a row of lanes to a list, a word of the mask to a lane
+        static_assert(kWaveTile / kWave == 16, "a row of words");
+        const uint32_t lane = t & (kWave - 1), row = lane / 16;
+#pragma unroll 1
+        for (uint32_t q = first; q < first + per; q++) {
+          const uint32_t found = q < nlists ? lengths[q] : 0u;
+#pragma unroll 1
+          for (uint64_t some = __ballot(found > room); some != 0;) {
+            uint32_t of = kWave;   // whose list it is
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++) {
+              if (row == k && some != 0) of = uint32_t(__builtin_ctzll(some));
+              some &= some - 1;   // 0 stays 0
+            }
+            const uint32_t which = __shfl(q, int(of), kWave), at = __shfl(start, int(of), kWave);
+            const uint64_t m = of < uint32_t(kWave) ? masks[size_t(which) * 16 + lane % 16] : 0ull;
+            const uint32_t c = uint32_t(__popcll(m));
+            uint32_t before = row_prefix_u32(c) - c;
+            for (uint64_t x = m; x; x &= x - 1, before++)
+              if (before >= room) s_id[at + before] = 0x80000000u | (which * uint32_t(kWaveTile) + lane % 16 * kWave + uint32_t(__builtin_ctzll(x)));
+          }
+          start += found;
+        }
+        __syncthreads();
+        for (uint32_t x = t; x < n; x += kSortThreads) {
+          if (!(s_id[x] >> 31)) continue;
+          const uint32_t i = s_id[x] & 0x7FFFFFFFu;
+          list[nlists * room + x] = make_uint2(i, __float_as_uint(r[i]));
+          if (cleared) r[i] = 0.0f;
+          s_id[x] = nlists * room + x;
+        }
       }
       if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + (n > keep ? keep : n) * 8);
       if (n == 0 || keep == 0) return;
@@ -2668,7 +2705,8 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
       if (!done) cut_crowded(f);
       return;
     }
-    // Too many for a list, or for the workgroup: the masks name them, and their values are looked up in r.
+    // Too many for the workgroup: the masks name them, and their values are looked up in r.  (8500 to 16 thousand candidates of a million that
+    // keeps 1049 146 to 182 us per encode; 148 to 176 when the pass cleared nothing.)
     if (cleared) {
       for (uint32_t q = first; q < first + per && q < nlists; q++) {
         const uint32_t in_list = lengths[q] < room ? lengths[q] : room;
