@@ -3043,6 +3043,10 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     else if (lists) pass(residual ? gd_stream_kernel<true, false, true, CAP> : gd_stream_kernel<false, false, true, CAP>);
     else pass(residual ? gd_stream_kernel<true, false, false, CAP> : gd_stream_kernel<false, false, false, CAP>);
   };
+  // Before anything is launched: the pass leaves zeros in the residual for what the finish sends (clears_listed).
+  constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));
+  static std::atomic<uint64_t> attr_done{0};
+  if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_finish_kernel<CAP>), kStageBytes, attr_done)) return rc;
   dim3 grid;
   if (margin < 0) {
     // One workgroup's gathers of a sample take as long as a launch that spreads them at about kPickGather samples;
@@ -3090,9 +3094,6 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
   if (grid.x) HPX_LAUNCH("gd_expand_kernel", gd_expand_kernel<CAP>, grid, dim3(kThreads), st, a);
   grid = tiles([margin](const GdSeg& sg) { return finishes(sg, margin) || cut_on_device(sg, margin) ? 1u : 0u; });
   if (grid.x) {
-    constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));
-    static std::atomic<uint64_t> attr_done{0};
-    if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_finish_kernel<CAP>), kStageBytes, attr_done)) return rc;
     HPX_LAUNCH_LDS("gd_finish_kernel", hpx::g_prof_on, gd_finish_kernel<CAP>, grid, dim3(kSortThreads), kStageBytes, st, a);
   }
   HPX_HIP(hipGetLastError());
