@@ -632,7 +632,8 @@ def x_terngrad_sizes(torch, np, capi, L, stream, gen, res):
 
 GD_KERNELS = ["gd_sample_kernel", "gd_select_kernel", "gd_threshold_kernel", "gd_presample_kernel", "gd_prepick_kernel", "gd_pick_kernel",
               "gd_stream_kernel", "gd_invert_kernel", "gd_exact_kernel", "gd_recount_kernel", "gd_scan_kernel",
-              "gd_expand_kernel", "gd_sort_count_kernel", "gd_sort_pass_kernel"]
+              "gd_expand_kernel", "gd_finish_kernel", "gd_order_kernel", "gd_sort_count_kernel", "gd_sort_pass_kernel"]
+GD_CUT_KERNELS = ["gd_order_kernel", "gd_sort_pass_kernel"]   # one of them in a call that cuts
 
 
 def x_dgc(torch, np, capi, L, stream, gen, res):
@@ -672,7 +673,7 @@ def x_dgc(torch, np, capi, L, stream, gen, res):
         kts = kernel_times(torch, capi, gd, GD_KERNELS, reps=1)
         cut = k == int(np.ceil(n * (1 - 0.999)))   # of the calls timed; those profiled go on from the residual they leave
         per_seed.append({"seed": seed, "encode_ms": round(float(np.median(times[2:])) * 1e3, 4), "selected": k, "cut": cut})
-        if kt is None or (kt["gd_sort_pass_kernel"] is None and kts["gd_sort_pass_kernel"] is not None):
+        if kt is None or (not any(kt[k_] for k_ in GD_CUT_KERNELS) and any(kts[k_] for k_ in GD_CUT_KERNELS)):
             kt = kts
     sec = float(np.mean([p["encode_ms"] for p in per_seed])) * 1e-3
     dout = torch.zeros(n, device="cuda")
