@@ -101,9 +101,10 @@ def test_on_either_side_of_the_least_number_kept(gd, oracle_cpu, n, kept):
             assert_bits_equal(host(got_r), want_r, "residual")
 
 
-@pytest.mark.parametrize("n,kept", [(900_001, 1e-2), (2_500_000, 1e-2), (9_000_001, 2e-3)])   # beyond what one workgroup cuts
+# beyond what one workgroup cuts: in windows, and beyond their 224 thousand candidates by the sort
+@pytest.mark.parametrize("n,kept", [(900_001, 1e-2), (2_500_000, 1e-2), (9_000_001, 2e-3), (3_000_000, 8e-2)])
 def test_a_cut_by_the_sort_keeps_the_signs(gd, oracle_cpu, n, kept):
-    """The sort's last pass writes the message from keys and indices alone: both signs, equal magnitudes, infinities."""
+    """The message is written from keys and indices alone: both signs, equal magnitudes, infinities."""
     rng = np.random.default_rng(n)
     cuts = 0
     for seed in range(1 << 24, 6 << 24, 1 << 24):
@@ -111,6 +112,13 @@ def test_a_cut_by_the_sort_keeps_the_signs(gd, oracle_cpu, n, kept):
         g[::1009] = 0.5 * rng.choice([-1, 1], g[::1009].size).astype(np.float32)
         r[::1009] = 0.0
         g[n // 2], g[n // 2 + 1] = np.inf, -np.inf
-        info = _check_encode(gd, oracle_cpu, g, r, 0.02, 1 - kept, seed)[2]
-        cuts += info["candidates"] > info["kept"]
+        gd.L.hpx_profile_reset(); gd.L.hpx_profile_enable(1)
+        try:
+            info = _check_encode(gd, oracle_cpu, g, r, 0.02, 1 - kept, seed)[2]
+            by = [gd.c.profile_query(k)[1] > 0 for k in ("gd_order_kernel", "gd_sort_pass_kernel")]
+        finally:
+            gd.L.hpx_profile_enable(0); gd.L.hpx_profile_reset()
+        if info["candidates"] > info["kept"]:
+            cuts += 1
+            assert by == [info["candidates"] <= 224 * 1024, info["candidates"] > 224 * 1024]
     assert cuts > 0

@@ -163,3 +163,18 @@ def test_one_way_for_a_call(gd, oracle_cpu, found):
         assert (order, sort > 0) == ((1, False) if pays else (0, True))
         ways.add(pays)
     assert ways
+
+
+# the sort's tiles of 4096, of which one lane adds up 40, in a call that a larger tensor sends there
+@pytest.mark.parametrize("found", [39 * 4096, 40 * 4096 - 1, 40 * 4096, 40 * 4096 + 1, 41 * 4096 + 5])
+def test_sort_beside_a_larger_one(gd, oracle_cpu, found):
+    rng = np.random.default_rng(found)
+    both = (found, MOST + 100)
+    rs = [_candidates(rng, 2 * f, f, "spread") for f in both]
+    seen = 0
+    for seed in range(8):
+        cut, (order, sort) = _encode_call(gd, oracle_cpu, rs, [f - 4000 for f in both], seed << 24)
+        if cut == list(both):
+            seen += 1
+            assert order == 0 and sort > 0
+    assert seen
