@@ -77,13 +77,18 @@ def _by_place(found, kind, rng):
         x[some[-9000:]] = 0.25
     if kind == "late":     # a third of them at the end, of one value
         x[-(found // 3):] = -1e-3
+    if kind == "levels":   # as many of each as one to three windows hold
+        x = ((rng.integers(0, max(2, found // 2500), found) + 1) * np.float32(1e-3) * sign).astype(np.float32)
+    if kind == "tiny":     # distances of one, two and three, next to a few large ones
+        x = (rng.integers(1, 4, found).astype(np.uint32)).view(np.float32) * sign
+        x[::5000] = 1.0
     if kind == "one_wave":  # the largest where one wave of a workgroup reads
         one = np.arange(found) // 256 % 16 == 0
         x[one] = (rng.uniform(0.5, 1, found).astype(np.float32) * sign)[one]
     return x
 
 
-@pytest.mark.parametrize("kind", ["equal", "near", "mixed", "late", "one_wave"])
+@pytest.mark.parametrize("kind", ["equal", "near", "mixed", "late", "levels", "tiny", "one_wave"])
 @pytest.mark.parametrize("found,keep", [(20_001, 19_990), (60_002, 30_000), (60_002, 60_001), (MOST, 210_000)])
 def test_one_launch_settles_it(gd, oracle_cpu, found, keep, kind):
     n = 3 * found

@@ -2231,6 +2231,8 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // for their word: 127, 118, 119, 248 and 153; and 60 instead of 20 until the call returned.)  Part by part is no more than a way out:
 // 100 thousand candidates laid around the sample, on purpose, so that one window has nearly all: 1.4 ms.
 constexpr uint32_t kWindow = 1024, kWindowSample = 512;
+constexpr uint32_t kShared = 2;   // windows that share a value; if there were fewer of them, it goes with the window above (one by
+                                  // itself walked all the keys for it: 200 thousand candidates of 64 values 141 us per encode, now 93; sort 103)
 constexpr uint32_t kOrderMax = 224 * 1024;   // candidates of one tensor; for all of a call: windows_pay
 // False: a bin is crowded (many equal keys), nothing has been written, and the pairs are in LDS as cut_crowded takes them, in the
 // order of the candidates.  That order comes from bins of the places among those, so wide that no more than kWideBin can share one.
@@ -2297,17 +2299,24 @@ __device__ __forceinline__ void order_ties(const CutArgs& f, const uint32_t* __r
   }
   found = 0;
   block_prefix(mine, f.wave, before);
-  for (uint32_t q0 = from; q0 < to && before + found < f.keep; q0 += kSortThreads) {
-    uint32_t k[4] = {0, 0, 0, 0};
-    if (q0 + t < to) take(q0 + t, k);
-    mine = 0;
+  // Four quads to a lane of a stretch that has so many (one: 57 us for 200 thousand keys in one stretch, each round waits for its keys).
+  constexpr uint32_t kAtOnce = 4;
+  const uint32_t per = cdiv(to - from, kSortThreads) < kAtOnce ? cdiv(to - from, kSortThreads) : kAtOnce;
+#pragma unroll 1
+  for (uint32_t q0 = from; q0 < to && before + found < f.keep; q0 += per * kSortThreads) {
+    const uint32_t q = q0 + per * t;
+    uint32_t marks = 0;
 #pragma unroll
-    for (uint32_t i = 0; i < 4; i++) mine += k[i] == v ? 1u : 0u;
+    for (uint32_t j = 0; j < kAtOnce; j++) {
+      const bool in = j < per && q + j < to;
+      uint32_t k[4];
+      take(in ? q + j : from, k);
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) marks |= in && k[i] == v ? 1u << (4 * j + i) : 0u;
+    }
     uint32_t all;
-    uint32_t place = before + found + block_prefix(mine, f.wave, all);
-#pragma unroll
-    for (uint32_t i = 0; i < 4; i++)
-      if (k[i] == v) f.put(place++, v, uint32_t(ids[4 * (q0 + t) + i]));
+    uint32_t place = before + found + block_prefix(uint32_t(__builtin_popcount(marks)), f.wave, all);
+    for (; marks != 0; marks &= marks - 1) f.put(place++, v, uint32_t(ids[4 * q + uint32_t(__builtin_ctz(marks))]));
     found += all;
   }
 }
@@ -2413,15 +2422,24 @@ __global__ __launch_bounds__(kSortThreads) void gd_order_kernel(const SortArgs<C
     }
   };
   reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
-  if (wave < 3) {   // one for each bound, and for the lower one of the window below (the other waves too: 4 us more, a request for each of their keys)
+  // The last window bound that a value reaches: those between its first one and that one are its own.
+  auto last_bound = [&](const uint32_t (&key)[kOwn], uint32_t v) {
+    uint32_t reach = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kOwn; j++) reach += uint32_t(__popcll(__ballot(key[j] >= v)));
+    const uint32_t to = cdiv(reach * windows, kWindowSample) - 1;
+    return v == 1u ? windows : to < windows - 1 ? to : windows - 1;
+  };
+  if (wave < 3) {   // one for each bound, and one looks how far the lower one reaches (the others too: 4 us more, a request for each of their keys)
     uint32_t key[kOwn];
     sample(key);
-    const uint32_t w = window + wave;
-    uint32_t bound = w == 0 ? 0xFFFFFFFFu : w == windows ? 1u : 0u;   // keys are at least 1
+    const uint32_t w = window + (wave > 0 ? 1u : 0u);
+    uint32_t bound = w == 0 ? 0xFFFFFFFFu : 1u;   // keys are at least 1
     if (w > 0 && w < windows) {
       bound = wave_rank<int(kOwn), 0>(key, uint32_t(uint64_t(w) * kWindowSample / windows), 0u);
       bound = bound > 1u ? bound : 1u;
     }
+    if (wave == 2) bound = last_bound(key, bound);
     if (lane == 0) s_bound[wave] = bound;
   }
   __syncthreads();
@@ -2429,22 +2447,19 @@ __global__ __launch_bounds__(kSortThreads) void gd_order_kernel(const SortArgs<C
   uint32_t lo = s_bound[1];
   if (window == 0 && t == 0) *reinterpret_cast<int32_t*>(sg.msg) = int32_t(4 + keep * 8);
   const CutArgs whole{s_stage, s_bins, s_wave, sg.r, sg.msg, n, keep, sg.thr_bits, false, 0, keep};
-  if (hi == lo) {   // its quantiles are one value, so are those of the windows from `from` to `to`
-    uint32_t key[kOwn], above = 0, reach = 0;
+  if (hi == lo) {   // its quantiles are one value
+    uint32_t key[kOwn], above = 0;
     sample(key);
 #pragma unroll
-    for (uint32_t j = 0; j < kOwn; j++) {
-      above += uint32_t(__popcll(__ballot(key[j] > lo)));
-      reach += uint32_t(__popcll(__ballot(key[j] >= lo)));
-    }
-    uint32_t from = cdiv(above * windows, kWindowSample), to = cdiv(reach * windows, kWindowSample) - 1;
+    for (uint32_t j = 0; j < kOwn; j++) above += uint32_t(__popcll(__ballot(key[j] > lo)));
+    uint32_t from = cdiv(above * windows, kWindowSample);
     from = from > 1u ? from : 1u;
-    to = lo == 1u ? windows : to < windows - 1 ? to : windows - 1;
+    const uint32_t to = s_bound[2];
     uint32_t before, found;
-    order_ties(whole, keys, ids, lo, window - from, to - from, before, found);
+    if (to - from >= kShared) order_ties(whole, keys, ids, lo, window - from, to - from, before, found);
     return;
   }
-  if (lo == s_bound[2]) {   // the windows below see to that value
+  if (s_bound[2] - (window + 1) >= kShared) {   // the windows below see to that value
     lo++;
     if (hi == lo) return;
   }
