@@ -2640,19 +2640,23 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
     bool some_over;
     pos = block_prefix_once(mine, over, s_wave, n, some_over);
     if (n <= kCutKeep) {
-      uint32_t start = pos;
-      for (uint32_t q0 = 0; q0 < per; q0 += kAtOnce) {
-        if (per > kAtOnce) take(q0);
+      if (!some_over) {
+        for (uint32_t q0 = 0; q0 < per; q0 += kAtOnce) {
+          if (per > kAtOnce) take(q0);
 #pragma unroll
-        for (uint32_t q = 0; q < kAtOnce; q++) {
-          for (uint32_t j = 0; j < (c[q] < room ? c[q] : room); j++) s_id[pos + j] = (first + q0 + q) * room + j;
-          pos += c[q];
+          for (uint32_t q = 0; q < kAtOnce; q++)
+            for (uint32_t j = 0; j < c[q]; j++) s_id[pos++] = (first + q0 + q) * room + j;
         }
-      }
-      // What has no room in its list the masks name; its values get places behind all lists.  (All candidates through the masks as soon as
-      // one list is too short: one million, half of its large values within 1 in 1500, 60 us per encode, now 34; 2.4 M with 37
-      // lists of 2400 too short by four 59, and 65 with what the pass had cleared put back first, now 55; with 146 such lists 53, now 49.)
-      if (some_over) {
+      } else {
+        // What has no room in its list the masks name; its values get places behind all lists.  (All candidates through the masks as soon as
+        // one list is too short: one million, half of its large values within 1 in 1500, 60 us per encode, now 34; 2.4 M with 37
+        // lists of 2400 too short by four 59, and 65 with what the pass had cleared put back first, now 55; with 146 such lists 53, now 49.)
+        for (uint32_t q = first; q < first + per && q < nlists; q++) {
+          const uint32_t found = lengths[q];
+          for (uint32_t j = 0; j < found && j < room; j++) s_id[pos + j] = q * room + j;
+          pos += found;
+        }
+        uint32_t start = pos - mine;
         // by their element and a mark; a row of lanes to a list, a word of the mask to a lane
         static_assert(kWaveTile / kWave == 16, "a row of words");
         const uint32_t lane = t & (kWave - 1), row = lane / 16;
@@ -3058,10 +3062,7 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
     else if (lists) pass(residual ? gd_stream_kernel<true, false, true, CAP> : gd_stream_kernel<false, false, true, CAP>);
     else pass(residual ? gd_stream_kernel<true, false, false, CAP> : gd_stream_kernel<false, false, false, CAP>);
   };
-  // Before anything is launched: the pass leaves zeros in the residual for what the finish sends (clears_listed).
-  constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));
-  static std::atomic<uint64_t> attr_done{0};
-  if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_finish_kernel<CAP>), kStageBytes, attr_done)) return rc;
+  constexpr int kStageBytes = 2 * int(kCutLds) * int(sizeof(uint32_t));   // of the finish
   dim3 grid;
   if (margin < 0) {
     // One workgroup's gathers of a sample take as long as a launch that spreads them at about kPickGather samples;
@@ -3085,6 +3086,9 @@ int launch_phases(const Plan* plans, int count, bool residual, int margin, uint3
       grid = tiles([](const GdSeg& sg) { return sg.sample_cnt <= kPickMax ? 0u : 1u; });
       HPX_LAUNCH("gd_threshold_kernel", gd_threshold_kernel<CAP>, grid, dim3(kSelThreads), st, a);
     }
+    // Before the pass, which leaves zeros in the residual for what the finish sends (clears_listed); behind the first launches, which it need not hold up.
+    static std::atomic<uint64_t> attr_done{0};
+    if (const int rc = allow_lds(reinterpret_cast<const void*>(&gd_finish_kernel<CAP>), kStageBytes, attr_done)) return rc;
     stream_pass();
   } else {
     grid = tiles([](const GdSeg& sg) { return cdiv(pre_samples(sg.sample_cnt, sg.thr_index), kThreads); });
