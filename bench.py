@@ -639,7 +639,7 @@ GD_CUT_KERNELS = ["gd_order_kernel", "gd_sort_pass_kernel"]   # one of them in a
 def x_dgc(torch, np, capi, L, stream, gen, res):
     # ---- DGC / GradDrop top-0.1 %: 138,357,544 elements --------------------------------------
     n = N_DGC
-    # A generator of its own: which seeds below have to sort and cut depends on the gradient drawn here (each does
+    # A generator of its own: which seeds below have to cut depends on the gradient drawn here (each does
     # with probability about one half), and the section's mean should not move with what other sections drew before it.
     gen = torch.Generator(device="cuda").manual_seed(138_357_544)
     u = torch.rand(n, device="cuda", generator=gen) - 0.5

@@ -306,8 +306,8 @@ int hpx_terngrad_decode_status(hpx_stream_t stream);
  * scheduler does (hp_cuda.cpp:284-301).  The reference waits for the stream
  * three times per tensor; this call never waits for the stream: it polls
  * pinned host words in which a kernel reports the candidate count of every
- * tensor (while later kernels are still running), queues the sort-and-cut for
- * the tensors that overshoot and returns; results are stream-ordered.  Because
+ * tensor (while later kernels are still running), queues the cut of the
+ * tensors that overshoot and returns; results are stream-ordered.  Because
  * of that dependence on the host it returns -3 on a stream that is being
  * captured into a graph; so do hpx_gd_decode and the two DGC calls.
  * A tensor whose parameters make no sense (threshold index outside the sample)

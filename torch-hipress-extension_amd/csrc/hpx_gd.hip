@@ -20,7 +20,8 @@
 //               (bit i = element i), a popcount and the largest |r| per workgroup, and the
 //               candidates with their values in a short list per wave
 //   finish      tensors that keep up to 2560 entries: one workgroup lists the candidates, cuts
-//               them if they are too many, writes the message and clears the residual
+//               them if they are too many and writes the message; the residual is cleared by the pass
+//               where it lists a candidate (what a cut drops goes back), else here
 //   scan        larger tensors of more than 4096 workgroups, but for those above: exclusive prefix of the
 //               per-workgroup counts within chunks of 4096, the chunks' totals and largest |r|
 //   expand      larger tensors: folds the totals (each workgroup for itself), reports count,
@@ -33,10 +34,11 @@
 // that keep fewer than 8192 entries that is all: their cut is the device's own business.  For the others the host learns the
 // candidate counts from pinned memory while the expand launch is still running
 // (it polls the words the expand launch writes first; no wait for the stream), and only
-// for tensors with more than `expected` candidates queues the cut: a stable LSD
-// radix sort by |r| (ties keep ascending index) over as many byte digits as the
+// for tensors with more than `expected` candidates queues the cut, largest |r| first, ties in
+// ascending index: one launch of many workgroups, each with a window of the keys, or beyond
+// what that is good for (windows_pay) a stable LSD radix sort over as many byte digits as the
 // largest key has, whose last pass writes the message.  The expand launch has
-// by then left the candidates and their keys where the sort wants them.
+// by then left the candidates and their keys where both want them.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -228,7 +230,7 @@ __device__ __forceinline__ void find_digit(const uint32_t* __restrict__ hist, ui
     h[j] = hist[BINS - 1 - (t * PER + j)];
     sum += h[j];
   }
-  // Inclusive prefix over the threads in order: within each wave by shuffles, then the sixteen wave totals
+  // Inclusive prefix over the threads in order: within each wave by lane permutes, then the sixteen wave totals
   // (three workgroup barriers in all; a workgroup-wide scan through LDS, ten rounds of two barriers each, was
   // most of the time of the launches that call this).
   const uint32_t incl = wave_prefix_u32(sum);
@@ -923,11 +925,9 @@ __global__ __launch_bounds__(kThreads) void gd_invert_kernel(const GdArgs<CAP> a
 }
 
 // One workgroup per tensor: the exact threshold from the samples that were found, or the other path called for.  Eight lanes
-// take a part of the list, up to R keys each, and the rank is found bit by bit among the keys in registers; only if a
+// take a part of the list, up to R keys each, and the rank is found among the keys in registers (rank_hits); only if a
 // part is longer than that are they drawn together (into the samples' block, free by now) and ranked by histograms.
-// (Drawn together first: 12 thousand keys by histograms 27 us, now 18.5; 3 thousand in LDS as long as now, 10.  A histogram of the
-// keys' distance from the provisional threshold and the few keys of one bin, in place of the bits, took 2 to 4 us longer: the
-// more code of a launch of one workgroup, the more of it has to be fetched.)
+// (Drawn together first, then the bits tried one by one: 12 thousand keys 27 us, 18.5 from the registers.)
 constexpr uint32_t kWayLanes = kSelThreads / kHitWays;
 // The hits' distances from the provisional threshold go into 2048 bins by exponent and six further bits, larger ones first, as
 // a cut's do (cut_bin); the bin that the rank falls into holds a handful, and one wave finds the key among them.  Where it holds
@@ -2225,8 +2225,8 @@ __device__ __forceinline__ bool cut_loaded(const CutArgs& f, F pair) {
 // A value that thousands share is several quantiles, and the windows between two of these share its candidates by their places
 // (order_ties).  What does not fit all the same - the sample is one of many, and one wave may read most of a window - goes part
 // by part (next_part).  So all of it is settled here, and the host, which queues the launch, does not wait for it.  us per encode of
-// tensors with zeros around their candidates, sort -> windows: 100 thousand candidates 107 -> 77, with a tenth of them equal 112 -> 77,
-// all of them 99 -> 72; 16 thousand with six in ten equal 103 -> 73; 220 thousand with the last three in ten equal 209 -> 183; the
+// tensors with zeros around their candidates, sort -> windows: 100 thousand candidates 107 -> 77, with a tenth of them equal 112 -> 78,
+// all of them 99 -> 74; 16 thousand with six in ten equal 103 -> 74; 220 thousand with the last three in ten equal 209 -> 184; the
 // largest of 220 thousand where one wave reads 115 -> 117.  (Windows that left such tensors to a sort queued behind them, the host waiting
 // for their word: 127, 118, 119, 248 and 153; and 60 instead of 20 until the call returned.)  Part by part is no more than a way out:
 // 100 thousand candidates laid around the sample, on purpose, so that one window has nearly all: 1.4 ms.
