@@ -93,6 +93,7 @@ constexpr uint32_t kCutLds = 16384;      // ... by one workgroup, which sorts up
 __host__ __device__ constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 __host__ __device__ constexpr uint32_t cdiv(uint64_t a, uint64_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
 
+constexpr uint32_t kHitExtra = 256 * 128;
 // Where the pieces of one tensor's workspace block lie (the same arithmetic on the host and in the kernels).
 struct GdLayout {
   size_t state, hist, samples, hitlist, masks, coarse, cnt, wcnt, mx, off, ctot, cmax, end;
@@ -104,7 +105,7 @@ __host__ __device__ inline GdLayout gd_layout(uint32_t n, uint32_t sample_cnt) {
   l.state = at;   at += align256(sizeof(GdState));
   l.hist = at;    at += align256(sizeof(uint32_t) * kHistWords);
   l.samples = at; at += align256(sizeof(uint32_t) * size_t(sample_cnt));
-  l.hitlist = at; at += align256(sizeof(uint32_t) * (size_t(sample_cnt) + size_t(256) * 128));  // provisional path, see hit_way_room
+  l.hitlist = at; at += align256(sizeof(uint32_t) * (size_t(sample_cnt) + size_t(kHitExtra)));  // provisional path, see hit_way_room; the finish
   l.masks = at;   at += align256(sizeof(uint64_t) * ntiles * kWave);      // one bit per element
   l.coarse = at;  at += align256(sizeof(uint64_t) * ntiles);              // one bit per mask word: whether it has a bit set
   l.cnt = at;     at += align256(sizeof(uint32_t) * ntiles);              // candidates per tile
@@ -146,8 +147,7 @@ __host__ __device__ inline uint32_t list_room(uint32_t n, uint32_t limit) {
 // the few that a cut drops, and all of them where it cannot take them from the lists (gd_finish_kernel).
 __host__ __device__ inline bool clears_listed(uint32_t n, uint32_t limit) { return one_workgroup(n, limit) && list_room(n, limit) != 0; }
 __host__ __device__ inline size_t list_bytes(uint32_t n, uint32_t limit) {
-  const size_t lists = size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit);
-  return align256(sizeof(uint64_t) * (lists + (clears_listed(n, limit) ? kCutKeep : 0u)));   // behind them what has no room in its list
+  return align256(sizeof(uint64_t) * size_t(cdiv(n, kTile)) * (kThreads / kWave) * list_room(n, limit));
 }
 // The launches behind the pass read them four lanes to a list, so that a wave has the lists of four tiles; the first entries,
 // whether there are as many or not, and the lengths are requested together.
@@ -2619,7 +2619,10 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
   // lists, times three, which one CU takes 3 us over for 2304 of them.)
   const uint32_t room = list_room(sg.n, keep);
   const bool cleared = a.residual != 0 && clears_listed(sg.n, keep);
-  uint2* list = seg_list(sg, l);
+  uint2* entries = reinterpret_cast<uint2*>(sg.ws + l.hitlist);   // what has no room in the lists, from `lists0` on the lists
+  const uint2* __restrict__ list = seg_list(sg, l);
+  const uint32_t lists0 = uint32_t((l.end - l.hitlist) / sizeof(uint2));   // (below 2^31 at any size of sample)
+  static_assert(sizeof(uint32_t) * kHitExtra >= sizeof(uint2) * kCutKeep, "which the provisional path's block holds");
   uint32_t n = 0, pos = 0;
   reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0, 0, 0, 0);
   if (room != 0) {
@@ -2645,15 +2648,15 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
           if (per > kAtOnce) take(q0);
 #pragma unroll
           for (uint32_t q = 0; q < kAtOnce; q++)
-            for (uint32_t j = 0; j < c[q]; j++) s_id[pos++] = (first + q0 + q) * room + j;
+            for (uint32_t j = 0; j < c[q]; j++) s_id[pos++] = lists0 + (first + q0 + q) * room + j;
         }
       } else {
-        // What has no room in its list the masks name; its values get places behind all lists.  (All candidates through the masks as soon as
+        // What has no room in its list the masks name; its values get places in a block that is free here.  (All candidates through the masks as soon as
         // one list is too short: one million, half of its large values within 1 in 1500, 60 us per encode, now 34; 2.4 M with 37
         // lists of 2400 too short by four 59, and 65 with what the pass had cleared put back first, now 55; with 146 such lists 53, now 49.)
         for (uint32_t q = first; q < first + per && q < nlists; q++) {
           const uint32_t found = lengths[q];
-          for (uint32_t j = 0; j < found && j < room; j++) s_id[pos + j] = q * room + j;
+          for (uint32_t j = 0; j < found && j < room; j++) s_id[pos + j] = lists0 + q * room + j;
           pos += found;
         }
         uint32_t start = pos - mine;
@@ -2684,9 +2687,9 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
         for (uint32_t x = t; x < n; x += kSortThreads) {
           if (!(s_id[x] >> 31)) continue;
           const uint32_t i = s_id[x] & 0x7FFFFFFFu;
-          list[nlists * room + x] = make_uint2(i, __float_as_uint(r[i]));
+          entries[x] = make_uint2(i, __float_as_uint(r[i]));
           if (cleared) r[i] = 0.0f;
-          s_id[x] = nlists * room + x;
+          s_id[x] = x;
         }
       }
       if (t == 0) *reinterpret_cast<int32_t*>(sg.out) = int32_t(4 + (n > keep ? keep : n) * 8);
@@ -2698,7 +2701,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
         for (uint32_t x0 = t; x0 < n; x0 += 3 * kSortThreads) {   // three in flight per lane
           uint2 e[3];
 #pragma unroll
-          for (uint32_t j = 0; j < 3; j++) e[j] = list[s_id[x0 + j * kSortThreads < n ? x0 + j * kSortThreads : x0]];
+          for (uint32_t j = 0; j < 3; j++) e[j] = entries[s_id[x0 + j * kSortThreads < n ? x0 + j * kSortThreads : x0]];
 #pragma unroll
           for (uint32_t j = 0; j < 3; j++) {
             const uint32_t x = x0 + j * kSortThreads;
@@ -2713,7 +2716,7 @@ __global__ __launch_bounds__(kSortThreads) void gd_finish_kernel(const GdArgs<CA
       }
       const CutArgs f{s_stage, s_bins, s_cut_wave, r, sg.out, n, keep, thr_bits, cleared, 0, keep};
       auto pair = [=](uint32_t x, uint32_t& key, uint32_t& id) {
-        const uint2 e = list[s_id[x]];
+        const uint2 e = entries[s_id[x]];
         key = (e.y & 0x7FFFFFFFu) - thr_bits;
         id = e.x | (e.y & 0x80000000u);
       };
